@@ -831,7 +831,7 @@ int rlt_sac_polyak_list(rlt_rocm_device* device, const float* const* sources, fl
         P.n = n - base < MAX_POLYAK ? n - base : MAX_POLYAK; P.polyak = polyak;
         uint32_t largest = 0;
         for (int i = 0; i < P.n; i++) { P.source[i] = sources[base + i]; P.target[i] = targets[base + i]; P.count[i] = counts[base + i]; largest = counts[base + i] > largest ? counts[base + i] : largest; }
-        const int parts = (int)((largest + 2047) / 2048);
+        const int parts = (int)((largest + 511) / 512);
         hipLaunchKernelGGL(polyak_list_kernel, dim3(P.n * (parts < 1 ? 1 : parts)), dim3(256), 0, device->stream, P);
         int rc = rlt_launch_status(device);
         if (rc) return rc;
