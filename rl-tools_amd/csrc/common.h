@@ -6,6 +6,7 @@
 #include "../../include/rlt_rocm.h"
 
 constexpr int RLT_SIDE_STREAMS = 2;
+constexpr size_t RLT_ADAM_TICKETS_OFFSET = 8192, RLT_COUNTERS_BYTES = 16384;
 struct rlt_rocm_device {
     int hip_device;
     hipStream_t own_stream;
@@ -18,7 +19,7 @@ struct rlt_rocm_device {
     void* pad_scratch;           // a second grow-only buffer: zero-padded copies of narrow networks (pad.hip)
     size_t pad_scratch_bytes;
     void* copy_scratch; size_t copy_scratch_bytes;      // weight copies in consumption order of the MLP calls on sixteen-row tiles: not the handle's scratch buffer, which callers of forward() / evaluate() may hold across the call
-    void* counters;              // 8 KiB, zero between launches: [0,256) ticket counters, [256,..) per-workgroup partial sums
+    void* counters;              // RLT_COUNTERS_BYTES, zero between launches: [0,256) ticket counters, [256,4096) per-workgroup partial sums, [4096,8192) words of the XCD groups, the fault flag and the stream offset, then the optimisers' tickets
     unsigned* fault;             // [0]: set by a persistent kernel that gave up waiting for another workgroup; read back by check_status
     int fault_armed;             // a kernel that can set it was launched since the last check
     int xcd_stride;              // workgroups b and b + xcd_stride run on the same XCD (0: not established; consecutive workgroups go round the XCDs)
@@ -60,7 +61,7 @@ int rlt_side_join(rlt_rocm_device* device);
 
 // Grow-only scratch owned by the device handle.
 int rlt_scratch(rlt_rocm_device* device, size_t bytes, void** out);
-// 8 KiB of zero-initialised device memory for last-workgroup-done tickets and per-workgroup partials.
+// RLT_COUNTERS_BYTES of zero-initialised device memory for last-workgroup-done tickets and per-workgroup partials.
 int rlt_counters(rlt_rocm_device* device, void** out);
 // Returns hipGetLastError() folded into the return convention; called after every launch.
 int rlt_launch_status(rlt_rocm_device* device);

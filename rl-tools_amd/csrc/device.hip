@@ -154,10 +154,10 @@ int rlt_rocm_init(int hip_device_index, rlt_rocm_device** out_device) {
     e = hipStreamCreate(&device->own_stream);   // default priority
     if (e != hipSuccess) { delete device; return (int)e; }
     device->stream = device->own_stream;
-    e = hipMalloc(&device->counters, 8192);
-    if (e == hipSuccess) e = hipMemset(device->counters, 0, 8192);
+    e = hipMalloc(&device->counters, RLT_COUNTERS_BYTES);
+    if (e == hipSuccess) e = hipMemset(device->counters, 0, RLT_COUNTERS_BYTES);
     if (e != hipSuccess) { (void)hipStreamDestroy(device->own_stream); delete device; return (int)e; }
-    device->fault = (unsigned*)((char*)device->counters + 8192 - 64);   // the last 64 bytes of the block are never used as counters
+    device->fault = (unsigned*)((char*)device->counters + 8192 - 64);   // these 64 bytes are never used as counters
     device->stream_offset = (uint64_t*)((char*)device->counters + 8192 - 128);      // zero: stream numbers mean what the caller passes
     // Dispatch order over the XCDs: probe twice with 64 workgroups; if workgroup b always shares its XCD with b + 8 (and with no
     // workgroup in between), persistent kernels may place a small grid on one XCD by using every 8th workgroup of a larger one.

@@ -16,7 +16,7 @@ struct AdamLaunch {
     rlt_adam_parameters p;
     float polyak;
     uint32_t* age;
-    uint32_t* done_counter;      // zero between launches
+    uint32_t* tickets;           // zero between launches: TICKET_LEAVES words a cache line apart, then the root (see last_through())
     float* block_partials;       // [gridDim.x] sums of squared gradients
     float* out_sq_norm;          // optional
     int increment_age;
@@ -32,6 +32,25 @@ struct AdamLaunch {
     float* extra_out; uint32_t extra_offset; float extra_scale;      // optional: one more sum of the blocks, stored scaled (not a gradient)
     uint32_t vec_end;            // elements [0, vec_end) can be stepped four at a time (16-byte loads of the blocks, moments and values): see vector_end()
 };
+
+// The last workgroup through a launch advances the optimiser's age, which every workgroup reads. Nothing else passes between the workgroups (unless the squared norm is
+// asked for), so the ticket needs no fence: a workgroup's reads of the age have returned before its ticket is drawn. The tickets are two levels deep because atomics
+// on one word are served one after the other, about 80 ns each across the XCDs. At 72 k parameters the launch took 23 us with 281 workgroups on one word, 10.4 us
+// with them behind a device-wide fence each (which writes the XCD's L2 back), and takes 6.1 us with sixteen leaves in lines of their own, no fence and four elements
+// per thread. Drawing the ticket before the elements are stepped, so that its answer travels meanwhile, was no faster (6.0 us; 8.0 instead of 6.9 us with sixteen
+// blocks per element): the workgroup then waits for the age before anything else.
+constexpr uint32_t TICKET_LEAVES = 16, TICKET_STRIDE = 32;      // words
+constexpr size_t TICKET_BYTES = (TICKET_LEAVES + 1) * TICKET_STRIDE * sizeof(uint32_t);
+__device__ __forceinline__ bool last_through(uint32_t* tickets, uint32_t block, uint32_t n_blocks) {
+    const uint32_t leaf = block % TICKET_LEAVES, in_leaf = (n_blocks - leaf + TICKET_LEAVES - 1) / TICKET_LEAVES, leaves = min(n_blocks, TICKET_LEAVES);
+    uint32_t* const word = tickets + leaf * TICKET_STRIDE;
+    uint32_t* const root = tickets + TICKET_LEAVES * TICKET_STRIDE;
+    if (__hip_atomic_fetch_add(word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != in_leaf - 1) return false;
+    __hip_atomic_store(word, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__hip_atomic_fetch_add(root, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != leaves - 1) return false;
+    __hip_atomic_store(root, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return true;
+}
 
 // sum over the blocks of one element, every load in flight at once where there are at most 16 blocks
 __device__ __forceinline__ float sum_of_blocks(const float* __restrict__ p, int groups, int stride) {
@@ -95,7 +114,7 @@ __device__ __forceinline__ void adam_body(const AdamLaunch& a, uint32_t block, u
             __syncthreads();
         }
     } else {
-    // at most 16 blocks, four neighbouring elements per thread: every load is 16 bytes per lane (the same sums in the same order per element)
+    // four neighbouring elements per thread, from their gradient or from at most 16 blocks: every load is 16 bytes per lane (the same sums in the same order per element)
     typedef float f4 __attribute__((ext_vector_type(4)));
     for (uint32_t i = (block * blockDim.x + threadIdx.x) * 4u; i < a.vec_end; i += n_blocks * blockDim.x * 4u) {
         int ti = 0;
@@ -106,35 +125,38 @@ __device__ __forceinline__ void adam_body(const AdamLaunch& a, uint32_t block, u
         f4 m = *reinterpret_cast<const f4*>(T.first_moment + j), v = *reinterpret_cast<const f4*>(T.second_moment + j), param = *reinterpret_cast<const f4*>(T.parameters + j);
         f4 target = {0.f, 0.f, 0.f, 0.f};
         if (T.polyak_target) target = *reinterpret_cast<const f4*>(T.polyak_target + j);
-        const float* __restrict__ p = a.source + a.source_offset[ti] + j;
-        const int per = (a.groups + 3) / 4;
-        f4 blk[16];
-#pragma unroll
-        for (int qi = 0; qi < 4; qi++)
-#pragma unroll
-            for (int u = 0; u < 4; u++) blk[4 * qi + u] = *reinterpret_cast<const f4*>(p + (size_t)min(qi * per + u, a.groups - 1) * a.block_stride);
-        __builtin_amdgcn_sched_barrier(0);
-        f4 q[4];
-#pragma unroll
-        for (int qi = 0; qi < 4; qi++) {
-            const int g0 = qi * per, g1 = min(a.groups, g0 + per);
-            f4 sum = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int u = 0; u < 4; u++) if (u < per && g0 + u < g1) sum += blk[4 * qi + u];
-            q[qi] = sum;
-        }
-        const f4 total4 = (q[0] + q[1]) + (q[2] + q[3]);
         f4 g;
+        if (a.source) {
+            const float* __restrict__ p = a.source + a.source_offset[ti] + j;
+            const int per = (a.groups + 3) / 4;
+            f4 blk[16];
+#pragma unroll
+            for (int qi = 0; qi < 4; qi++)
+#pragma unroll
+                for (int u = 0; u < 4; u++) blk[4 * qi + u] = *reinterpret_cast<const f4*>(p + (size_t)min(qi * per + u, a.groups - 1) * a.block_stride);
+            __builtin_amdgcn_sched_barrier(0);
+            f4 q[4];
+#pragma unroll
+            for (int qi = 0; qi < 4; qi++) {
+                const int g0 = qi * per, g1 = min(a.groups, g0 + per);
+                f4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int u = 0; u < 4; u++) if (u < per && g0 + u < g1) sum += blk[4 * qi + u];
+                q[qi] = sum;
+            }
+            const f4 total4 = (q[0] + q[1]) + (q[2] + q[3]);
+#pragma unroll
+            for (int c = 0; c < 4; c++) g[c] = rlt_scaled_sum(total4[c], a.source_scale[ti], a.source_add[ti]);
+        } else g = *reinterpret_cast<const f4*>(T.gradient + j);
 #pragma unroll
         for (int c = 0; c < 4; c++) {
-            g[c] = rlt_scaled_sum(total4[c], a.source_scale[ti], a.source_add[ti]);
             sq += g[c] * g[c];
             float mc = m[c], vc = v[c], pc = param[c];
             rlt_adam_values(a.p, T.flags, g[c], bc1, bc2, mc, vc, pc);
             m[c] = mc; v[c] = vc; param[c] = pc;
             if (T.polyak_target) target[c] = rlt_polyak_value(a.polyak, target[c], pc);
         }
-        *reinterpret_cast<f4*>(T.gradient + j) = g;
+        if (a.source) *reinterpret_cast<f4*>(T.gradient + j) = g;
         *reinterpret_cast<f4*>(T.first_moment + j) = m; *reinterpret_cast<f4*>(T.second_moment + j) = v; *reinterpret_cast<f4*>(T.parameters + j) = param;
         if (T.polyak_target) *reinterpret_cast<f4*>(T.polyak_target + j) = target;
     }
@@ -159,28 +181,27 @@ __device__ __forceinline__ void adam_body(const AdamLaunch& a, uint32_t block, u
     }
     }
     if (a.extra_out && block == n_blocks - 1 && threadIdx.x == blockDim.x - 1) *a.extra_out = sum_of_blocks(a.source + a.extra_offset, a.groups, a.block_stride) * a.extra_scale;
-    // gradient norm + age increment: the last workgroup to finish has seen every other one read `age`
+    if (!a.out_sq_norm) {
+        asm volatile("" :: "v"(bc1), "v"(bc2));      // every thread has read the age ...
+        rlt_lds_barrier();                           // ... before the workgroup's ticket is drawn; its stores may still be on their way
+        if (threadIdx.x == 0 && last_through(a.tickets, block, n_blocks) && a.increment_age) *a.age = age + 1;
+        return;
+    }
+    // the squared norm: the last workgroup adds the others' sums up, which a fence on both sides of the ticket makes visible to it
     __shared__ float partial[4];
-    __shared__ bool last;
     sq = rlt_wave_sum(sq);
     if ((threadIdx.x & 63) == 0) partial[threadIdx.x >> 6] = sq;
     __syncthreads();
     if (threadIdx.x == 0) {
         a.block_partials[block] = partial[0] + partial[1] + partial[2] + partial[3];
         __threadfence();
-        uint32_t ticket = atomicAdd(a.done_counter, 1u);
-        last = (ticket == n_blocks - 1);
-    }
-    __syncthreads();
-    if (last && threadIdx.x == 0) {
-        __threadfence();
-        if (a.out_sq_norm) {
+        if (last_through(a.tickets, block, n_blocks)) {
+            __threadfence();
             float s = a.accumulate_norm ? *a.out_sq_norm : 0.0f;
             for (uint32_t b = 0; b < n_blocks; b++) s += ((volatile float*)a.block_partials)[b];
             *a.out_sq_norm = s;
+            if (a.increment_age) *a.age = age + 1;
         }
-        if (a.increment_age) *a.age = age + 1;
-        *a.done_counter = 0;
     }
 }
 
@@ -212,7 +233,31 @@ __global__ __launch_bounds__(256) void polyak_kernel(const float* __restrict__ s
 
 }  // namespace
 
-// Layout of the device handle's scratch for this file: [0,256) the done counter, [256, ...) block partials.
+// how far the elements can be stepped four at a time: up to the first tensor whose start, pointers or place in the blocks is not a multiple of 16 bytes, or that
+// ends off one (then its last one to three elements and everything behind them are stepped one by one)
+static uint32_t vector_end(const AdamLaunch& a) {
+    auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
+    if (a.source && (a.groups > 16 || a.block_stride % 4 != 0 || !aligned(a.source))) return 0;
+    uint32_t end = 0;
+    for (int i = 0; i < a.n; i++) {
+        const rlt_adam_tensor& T = a.t[i];
+        if (a.prefix[i] % 4 != 0 || (a.source && a.source_offset[i] % 4 != 0) || !aligned(T.parameters) || !aligned(T.gradient) || !aligned(T.first_moment) || !aligned(T.second_moment) ||
+            (T.polyak_target && !aligned(T.polyak_target))) break;
+        end = a.prefix[i] + (T.count & ~3u);
+        if (T.count % 4 != 0) break;
+    }
+    return end;
+}
+// workgroups for an optimiser of `total` elements: 64 elements per workgroup pass on the many-block path, 256 threads of four elements each where those apply
+static uint32_t blocks_for(const AdamLaunch& a, uint32_t total, const rlt_adam_source* source) {
+    if (source && source->groups > 16) return (total + 63) / 64;
+    const uint32_t threads = a.vec_end / 4 > total - a.vec_end ? a.vec_end / 4 : total - a.vec_end;
+    return (threads + 255) / 256;
+}
+
+// Place in the device handle's counters block: [256, 4096) the workgroups' sums for the squared norm, the tickets of up to two optimisers from RLT_ADAM_TICKETS_OFFSET on.
+static uint32_t* tickets_of(void* counters, int k) { return (uint32_t*)((char*)counters + RLT_ADAM_TICKETS_OFFSET + k * TICKET_BYTES); }
+static_assert(RLT_ADAM_TICKETS_OFFSET + 2 * TICKET_BYTES <= RLT_COUNTERS_BYTES, "the tickets fit the counters block");
 static int adam_launch(rlt_rocm_device* device, const rlt_adam_tensor* tensors, int n_tensors, const rlt_adam_parameters* p, uint32_t* age,
                        float polyak, float* out_sq_norm, bool reset) {
     void* counters = nullptr;
@@ -230,10 +275,11 @@ static int adam_launch(rlt_rocm_device* device, const rlt_adam_tensor* tensors, 
         for (int i = a.n; i <= MAX_T; i++) a.prefix[i] = total;
         if (p) a.p = *p;
         a.polyak = polyak; a.age = age;
-        a.done_counter = (uint32_t*)counters; a.block_partials = (float*)((char*)counters + 256);
+        a.tickets = tickets_of(counters, 0); a.block_partials = (float*)((char*)counters + 256);
         a.out_sq_norm = out_sq_norm; a.accumulate_norm = base > 0;
         a.increment_age = (base + MAX_T >= n_tensors);
-        int blocks = (int)((total + 255) / 256); if (blocks > 960) blocks = 960; if (blocks < 1) blocks = 1;
+        if (!reset) a.vec_end = vector_end(a);
+        int blocks = (int)blocks_for(a, total, nullptr); if (blocks > 960) blocks = 960; if (blocks < 1) blocks = 1;
         if (reset) hipLaunchKernelGGL(adam_reset_kernel, dim3(blocks), dim3(256), 0, device->stream, a);
         else hipLaunchKernelGGL(adam_kernel, dim3(blocks), dim3(256), 0, device->stream, a);
         if ((rc = rlt_launch_status(device))) return rc;
@@ -241,35 +287,12 @@ static int adam_launch(rlt_rocm_device* device, const rlt_adam_tensor* tensors, 
     return 0;
 }
 
-// how far the elements can be stepped four at a time: up to the first tensor whose start, pointers or place in the blocks is not a multiple of 16 bytes, or that
-// ends off one (then its last one to three elements and everything behind them are stepped one by one)
-static uint32_t vector_end(const AdamLaunch& a) {
-    auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
-    if (!a.source || a.groups > 16 || a.block_stride % 4 != 0 || !aligned(a.source)) return 0;
-    uint32_t end = 0;
-    for (int i = 0; i < a.n; i++) {
-        const rlt_adam_tensor& T = a.t[i];
-        if (a.prefix[i] % 4 != 0 || a.source_offset[i] % 4 != 0 || !aligned(T.parameters) || !aligned(T.gradient) || !aligned(T.first_moment) || !aligned(T.second_moment) ||
-            (T.polyak_target && !aligned(T.polyak_target))) break;
-        end = a.prefix[i] + (T.count & ~3u);
-        if (T.count % 4 != 0) break;
-    }
-    return end;
-}
 static void set_source(AdamLaunch& a, const rlt_adam_source* source) {
     if (!source) return;
     a.source = source->partial; a.groups = source->groups; a.block_stride = source->block_stride;
     for (int i = 0; i < a.n; i++) { a.source_offset[i] = source->offsets[i]; a.source_scale[i] = source->scales[i]; a.source_add[i] = source->adds ? source->adds[i] : 0.0f; }
     a.extra_out = source->extra_out; a.extra_offset = source->extra_offset; a.extra_scale = source->extra_scale;
-    a.vec_end = vector_end(a);
 }
-// workgroups for an optimiser of `total` elements: 64 elements per workgroup pass on the many-block path, 256 threads of four elements each where those apply
-static uint32_t blocks_for(const AdamLaunch& a, uint32_t total, const rlt_adam_source* source) {
-    if (source && source->groups > 16) return (total + 63) / 64;
-    const uint32_t threads = a.vec_end / 4 > total - a.vec_end ? a.vec_end / 4 : total - a.vec_end;
-    return (threads + 255) / 256;
-}
-
 int rlt_adam_step_from_partials(rlt_rocm_device* device, const rlt_adam_tensor* tensors, int n, const rlt_adam_parameters* parameters, uint32_t* age, const rlt_adam_source* source, float polyak) {
     RLT_REQUIRE(tensors && n > 0 && n <= MAX_T && parameters && age && source && source->partial && source->groups > 0);
     void* counters = nullptr;
@@ -285,9 +308,10 @@ int rlt_adam_step_from_partials(rlt_rocm_device* device, const rlt_adam_tensor* 
     }
     for (int i = n; i <= MAX_T; i++) a.prefix[i] = total;
     a.p = *parameters; a.age = age; a.polyak = polyak;
-    a.done_counter = (uint32_t*)counters; a.block_partials = (float*)((char*)counters + 256);
+    a.tickets = tickets_of(counters, 0); a.block_partials = (float*)((char*)counters + 256);
     a.increment_age = 1;
     set_source(a, source);
+    a.vec_end = vector_end(a);
     int blocks = (int)blocks_for(a, total, source); if (blocks > 960) blocks = 960; if (blocks < 1) blocks = 1;
     hipLaunchKernelGGL(adam_kernel, dim3(blocks), dim3(256), 0, device->stream, a);
     return rlt_launch_status(device);
@@ -320,11 +344,12 @@ int rlt_adam_step_pair(rlt_rocm_device* device, const rlt_adam_tensor* tensors_a
         for (int i = a.n; i <= MAX_T; i++) a.prefix[i] = total;
         a.p = k ? *parameters_b : *parameters_a;
         a.age = k ? age_b : age_a; a.polyak = polyak;
-        // the second optimiser's ticket counter and partial sums sit in their own part of the counters block
-        a.done_counter = (uint32_t*)((char*)counters + (k ? 64 : 0)); a.block_partials = (float*)((char*)counters + 256) + (k ? 480 : 0);
+        // the second optimiser's tickets and partial sums sit in their own part of the counters block
+        a.tickets = tickets_of(counters, k); a.block_partials = (float*)((char*)counters + 256) + (k ? 480 : 0);
         a.increment_age = 1;
         const rlt_adam_source* source = k ? source_b : source_a;
         set_source(a, source);
+        a.vec_end = vector_end(a);
         blocks[k] = blocks_for(a, total, source); if (blocks[k] > 480) blocks[k] = 480; if (blocks[k] < 1) blocks[k] = 1;
     }
     hipLaunchKernelGGL(adam_pair_kernel, dim3(blocks[0] + blocks[1]), dim3(256), 0, device->stream, L[0], L[1], blocks[0]);

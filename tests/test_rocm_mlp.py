@@ -252,3 +252,34 @@ def test_zero_gradient_of_tensors_that_lie_apart(rocm, n_layers):
     for at, size in offsets:
         want[at:at + size] = 0.0
     assert np.array_equal(buffer.numpy(), want)
+
+
+# one workgroup; the last one partly filled; sixteen and seventeen workgroups (every leaf of the tickets, one with a second member); more tensors than a launch takes;
+# a start off 16 bytes and counts that are no multiple of four (the elements behind them are stepped one by one)
+@pytest.mark.parametrize("counts,shift", [([1], 0), ([3, 1021], 0), ([16 * 1024], 0), ([16 * 1024 + 4], 0), ([5, 70000, 7], 1), ([4100] * 13 + [2], 0), ([1100000], 0)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_adam_step_at_the_edges_of_its_launch(oracle, rocm, counts, shift, norm):
+    rng = np.random.default_rng(sum(counts))
+    n, steps = sum(counts), 3
+    p, m, v = (rng.standard_normal(n + shift).astype(np.float32) for _ in range(3))
+    v = np.abs(v)
+    g = rng.standard_normal((steps, n + shift)).astype(np.float32)
+    par = capi.adam_parameters()
+    res = []
+    for b in (oracle, rocm):
+        arrays = [b.array(a) for a in (p, g[0], m, v)]
+        age, sq = b.array(np.array([1], np.uint32)), b.zeros((1,))
+        tensors, o = [], shift
+        for c in counts:
+            tensors.append(capi.AdamTensor(*[a.offset(o) for a in arrays], None, c, 1))
+            o += c
+        tensors = (capi.AdamTensor * len(tensors))(*tensors)
+        for k in range(steps):
+            arrays[1].upload(g[k])
+            b.call("adam_step", tensors, len(counts), C.byref(par), age.ptr, 0.0, sq.ptr if norm else None)
+            b.sync()
+        assert age.numpy()[0] == 1 + steps
+        res.append([a.numpy() for a in arrays] + ([sq.numpy()] if norm else []))
+    # an element's step is a dozen roundings of 6e-8; the norm's summands are positive, so that their sum is off by no more than their roundings
+    for r, ref in zip(res[1], res[0]):
+        assert rel_err(r, ref) <= 1e-6 if ref.size > 1 else rel_err(r, ref) <= 1e-5
