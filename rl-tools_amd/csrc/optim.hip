@@ -16,7 +16,7 @@ struct AdamLaunch {
     rlt_adam_parameters p;
     float polyak;
     uint32_t* age;
-    uint32_t* tickets;           // zero between launches: TICKET_LEAVES words a cache line apart, then the root (see last_through())
+    uint32_t* tickets;           // zero between launches: TICKET_LEAVES words a cache line apart, then the root (rlt_last_through)
     float* block_partials;       // [gridDim.x] sums of squared gradients
     float* out_sq_norm;          // optional
     int increment_age;
@@ -32,25 +32,6 @@ struct AdamLaunch {
     float* extra_out; uint32_t extra_offset; float extra_scale;      // optional: one more sum of the blocks, stored scaled (not a gradient)
     uint32_t vec_end;            // elements [0, vec_end) can be stepped four at a time (16-byte loads of the blocks, moments and values): see vector_end()
 };
-
-// The last workgroup through a launch advances the optimiser's age, which every workgroup reads. Nothing else passes between the workgroups (unless the squared norm is
-// asked for), so the ticket needs no fence: a workgroup's reads of the age have returned before its ticket is drawn. The tickets are two levels deep because atomics
-// on one word are served one after the other, about 80 ns each across the XCDs. At 72 k parameters the launch took 23 us with 281 workgroups on one word, 10.4 us
-// with them behind a device-wide fence each (which writes the XCD's L2 back), and takes 6.1 us with sixteen leaves in lines of their own, no fence and four elements
-// per thread. Drawing the ticket before the elements are stepped, so that its answer travels meanwhile, was no faster (6.0 us; 8.0 instead of 6.9 us with sixteen
-// blocks per element): the workgroup then waits for the age before anything else.
-constexpr uint32_t TICKET_LEAVES = 16, TICKET_STRIDE = 32;      // words
-constexpr size_t TICKET_BYTES = (TICKET_LEAVES + 1) * TICKET_STRIDE * sizeof(uint32_t);
-__device__ __forceinline__ bool last_through(uint32_t* tickets, uint32_t block, uint32_t n_blocks) {
-    const uint32_t leaf = block % TICKET_LEAVES, in_leaf = (n_blocks - leaf + TICKET_LEAVES - 1) / TICKET_LEAVES, leaves = min(n_blocks, TICKET_LEAVES);
-    uint32_t* const word = tickets + leaf * TICKET_STRIDE;
-    uint32_t* const root = tickets + TICKET_LEAVES * TICKET_STRIDE;
-    if (__hip_atomic_fetch_add(word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != in_leaf - 1) return false;
-    __hip_atomic_store(word, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (__hip_atomic_fetch_add(root, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != leaves - 1) return false;
-    __hip_atomic_store(root, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return true;
-}
 
 // sum over the blocks of one element, every load in flight at once where there are at most 16 blocks
 __device__ __forceinline__ float sum_of_blocks(const float* __restrict__ p, int groups, int stride) {
@@ -184,7 +165,7 @@ __device__ __forceinline__ void adam_body(const AdamLaunch& a, uint32_t block, u
     if (!a.out_sq_norm) {
         asm volatile("" :: "v"(bc1), "v"(bc2));      // every thread has read the age ...
         rlt_lds_barrier();                           // ... before the workgroup's ticket is drawn; its stores may still be on their way
-        if (threadIdx.x == 0 && last_through(a.tickets, block, n_blocks) && a.increment_age) *a.age = age + 1;
+        if (threadIdx.x == 0 && rlt_last_through(a.tickets, block, n_blocks) && a.increment_age) *a.age = age + 1;
         return;
     }
     // the squared norm: the last workgroup adds the others' sums up, which a fence on both sides of the ticket makes visible to it
@@ -195,7 +176,7 @@ __device__ __forceinline__ void adam_body(const AdamLaunch& a, uint32_t block, u
     if (threadIdx.x == 0) {
         a.block_partials[block] = partial[0] + partial[1] + partial[2] + partial[3];
         __threadfence();
-        if (last_through(a.tickets, block, n_blocks)) {
+        if (rlt_last_through(a.tickets, block, n_blocks)) {
             __threadfence();
             float s = a.accumulate_norm ? *a.out_sq_norm : 0.0f;
             for (uint32_t b = 0; b < n_blocks; b++) s += ((volatile float*)a.block_partials)[b];
@@ -255,9 +236,7 @@ static uint32_t blocks_for(const AdamLaunch& a, uint32_t total, const rlt_adam_s
     return (threads + 255) / 256;
 }
 
-// Place in the device handle's counters block: [256, 4096) the workgroups' sums for the squared norm, the tickets of up to two optimisers from RLT_ADAM_TICKETS_OFFSET on.
-static uint32_t* tickets_of(void* counters, int k) { return (uint32_t*)((char*)counters + RLT_ADAM_TICKETS_OFFSET + k * TICKET_BYTES); }
-static_assert(RLT_ADAM_TICKETS_OFFSET + 2 * TICKET_BYTES <= RLT_COUNTERS_BYTES, "the tickets fit the counters block");
+// [256, 4096) of the device handle's counters block hold the workgroups' sums for the squared norm
 static int adam_launch(rlt_rocm_device* device, const rlt_adam_tensor* tensors, int n_tensors, const rlt_adam_parameters* p, uint32_t* age,
                        float polyak, float* out_sq_norm, bool reset) {
     void* counters = nullptr;
@@ -275,7 +254,7 @@ static int adam_launch(rlt_rocm_device* device, const rlt_adam_tensor* tensors, 
         for (int i = a.n; i <= MAX_T; i++) a.prefix[i] = total;
         if (p) a.p = *p;
         a.polyak = polyak; a.age = age;
-        a.tickets = tickets_of(counters, 0); a.block_partials = (float*)((char*)counters + 256);
+        a.tickets = rlt_tickets_of(counters, 0); a.block_partials = (float*)((char*)counters + 256);
         a.out_sq_norm = out_sq_norm; a.accumulate_norm = base > 0;
         a.increment_age = (base + MAX_T >= n_tensors);
         if (!reset) a.vec_end = vector_end(a);
@@ -308,7 +287,7 @@ int rlt_adam_step_from_partials(rlt_rocm_device* device, const rlt_adam_tensor* 
     }
     for (int i = n; i <= MAX_T; i++) a.prefix[i] = total;
     a.p = *parameters; a.age = age; a.polyak = polyak;
-    a.tickets = tickets_of(counters, 0); a.block_partials = (float*)((char*)counters + 256);
+    a.tickets = rlt_tickets_of(counters, 0); a.block_partials = (float*)((char*)counters + 256);
     a.increment_age = 1;
     set_source(a, source);
     a.vec_end = vector_end(a);
@@ -345,7 +324,7 @@ int rlt_adam_step_pair(rlt_rocm_device* device, const rlt_adam_tensor* tensors_a
         a.p = k ? *parameters_b : *parameters_a;
         a.age = k ? age_b : age_a; a.polyak = polyak;
         // the second optimiser's tickets and partial sums sit in their own part of the counters block
-        a.tickets = tickets_of(counters, k); a.block_partials = (float*)((char*)counters + 256) + (k ? 480 : 0);
+        a.tickets = rlt_tickets_of(counters, k); a.block_partials = (float*)((char*)counters + 256) + (k ? 480 : 0);
         a.increment_age = 1;
         const rlt_adam_source* source = k ? source_b : source_a;
         set_source(a, source);

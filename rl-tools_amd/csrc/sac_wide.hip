@@ -4,41 +4,46 @@
 // reference: rl/algorithms/sac/operations_generic.h:243-337 (train_critic), :395-468 (train_actor),
 //            nn/layers/sample_and_squash/operations_generic.h:148-398, nn_models/mlp/operations_generic.h:128-260.
 //
-// A workgroup of sixteen wavefronts takes 16 rows of the batch through every pass of the update, one network after the other:
-//   critic update   actor on the next observations -> squashed sample and its log-probability -> target critic 0, target critic 1 on
-//                   [next observation | sample] -> TD target -> trained critic forward on the current rows -> MSE gradient -> backward
-//   actor update    actor forward -> squashed sample -> critic 0, then critic 1: forward and the gradient of -value / batch with respect
-//                   to the action -> gradient of the smaller value per row -> sample_and_squash backward (entropy term, log_alpha
-//                   gradient) -> actor backward
+// A workgroup of sixteen wavefronts takes 16 rows of the batch through the passes that depend on each other; passes that do not depend on each other have workgroups
+// of their own (a role each), which hand over a few values per row through memory:
+//   critic update   target roles: actor on the next observations -> squashed sample and its log-probability -> one target critic on [next observation | sample];
+//                   critic roles: trained critic forward on the current rows -> (wait for the targets' values) -> TD target -> MSE gradient -> backward
+//   actor update    a role per critic: actor forward -> squashed sample -> critic forward and the gradient of -value / batch with respect to the action; critic 0's goes on
+//                   (with critic 1's values): gradient of the smaller value per row -> sample_and_squash backward (entropy term, log_alpha gradient) -> actor backward
 // The same kernel runs TD3's two updates (rl/algorithms/td3/operations_generic.h:170-281; actors obs -> h -> h -> act with a tanh output followed by the
-// td3_sampling layer): the critic update with the target actor, the smoothing noise on the next action and no entropy term, the actor update through critic 0 only.
+// td3_sampling layer): the critic update with the target actor, the smoothing noise on the next action and no entropy term (each critic's targets are formed with
+// sampling noise of its own, so each has its own pair of target roles), the actor update through critic 0 only.
 // Wavefront w owns hidden units 16 w .. 16 w + 15 of every layer: it computes that tile of the 16 x h activations from the whole previous
 // layer (LDS, behind a workgroup barrier), contributes the units' share of the output layer's reduction (the partial tiles are added in
-// wavefront order), and in the backward pass owns the same units' pre-activation gradients and their rows of dW1, dW2 and columns of dW3.
-// Weights are read from memory (L2) straight into the B operands of v_mfma_f32_16x16x4_f32 when a layer needs them, the second
-// layer's first half a layer ahead; hidden widths that are no multiple of 16 are completed with zero operands. The reduction index of a
-// 16-deep chunk is dealt to the four lane groups as k = 16 j + 4 g + i for the i-th of four instructions, so that activations (LDS) and
-// weights (memory) are both read 16 bytes at a time.
-// A workgroup writes one block of partial sums of the trained network's gradients [dW1 | db1 | dW2 | db2 | dW3 | db3 | extra]; the
-// optimiser's launch adds the blocks up over the whole chip (one compute unit draws about 4 GB/s from memory and 20 GB/s from L2 with loads
-// of this kind: read by the update's own sixteen workgroups, the 4.4 MB of blocks at width 256 took 70 us; spread over all compute units, 10).
-// Bound: per workgroup, a 16 x 256 x 256 layer is 2.1 MFLOP = 3.4 us of one compute unit's matrix pipeline, and an update has six or seven
-// of them; a batch of 256 is sixteen workgroups (thirty-two where both critics share the launch).
+// wavefront order), and in the backward pass owns the same units' pre-activation gradients.
+// Weights are read from memory (L2) straight into the B operands of v_mfma_f32_16x16x4_f32, the next pass's while this one runs; hidden widths that are no multiple
+// of 16 are completed with zero operands. The reduction index of a 16-deep chunk is dealt to the four lane groups as k = 16 j + 4 g + i for the i-th of four
+// instructions, so that activations (LDS) and weights (memory) are both read 16 bytes at a time.
+// The trained network's activations and pre-activation gradients go to memory (4 KB per row at width 256); the weight gradients and the optimisers' steps are the next
+// launch (batch_gradient.hip). Before, a workgroup ended with its sixteen rows' weight gradients (6.5 us on the matrix pipe at width 256) and a block of partial sums
+// that the optimisers' launch added up, and took all passes one after the other. At width 256, batch 256 (kernel and optimisers' launch; before / now): SAC critics
+// 55.7 + 10.6 / 26.0 + 8.2 us, SAC actor 65.6 + 10.6 / 33.9 + 8.2 us; TD3 critics (27 + 8 inputs) 61.1 + 11.9 / 28.1 + 8.0 us, TD3 actor 50.5 + 8.4 / 35.9 + 8.0 us.
+// Bound: per workgroup, a 16 x 256 x 256 layer is 2.1 MFLOP = 4 us of one compute unit's matrix pipeline, and the longest chain has three of them (critic update)
+// or four (actor update); the trips to memory at the start (3 us) and for the values handed over (2 us) come on top.
 #include "sac_update.h"
 #include "optim.h"
 #include "rng.h"
 #include "sac_heads.h"
+#include "batch_gradient.h"
 
 namespace {
 using namespace rlt_sac;
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) floatx4* lptr4;
+constexpr int FEW = 4;      // first-layer chunks that leave registers for a whole pass's operands at once
 constexpr int ROWS = 16, MAX_H = 256, WAVES = MAX_H / 16, THREADS = 64 * WAVES, S = MAX_H + 4, MAX_D = 128, SXS = MAX_D + 4, MAX_ACT = 8, MAX_OUT = 16, D3S = MAX_OUT + 1,
-              N_EXTRA = 16, MISC = 64, YP = ROWS * D3S;
+              MISC = 64, YP = ROWS * D3S;
 enum { MODE_CRITIC = 0, MODE_ACTOR = 1, MODE_TD3_CRITIC = 2, MODE_TD3_ACTOR = 3 };      // SAC's two updates, TD3's two updates
 
-// W2f / W2b: copies of the second layer's weights in the order the wavefronts consume them (wide_prepare_kernel): 16 bytes per lane, a wavefront's load 1 KB in a row
-struct WNet { const float *W1, *b1, *W2, *b2, *W3, *b3; int in, hid, out, act_h, vec1, vec2, vec3; const float *W2f, *W2b; };      // vecN: the rows of WN can be read 16 bytes at a time
+// W1f, W2f, W2b: copies of the weights in the order the wavefronts consume them (wide_prepare_kernel)
+struct WNet { const float *W1, *b1, *W2, *b2, *W3, *b3; int in, hid, out, act_h, vec3; const float *W1f, *W2f, *W2b; };      // vec3: the rows of W3 can be read 16 bytes at a time
+struct Trained { float *h1, *h2, *d1, *d2, *d3; };      // [batch][hid] each, d3 [batch][MAX_OUT]
+constexpr int EXCHANGE = ROWS * (1 + MAX_ACT), LOG_PROB_SLOT = 4;      // words per tile: critic update [slot][row] (slot = 2 set + target, then the log-probabilities), actor update [row] values, then [row][action]
 struct WideArgs {
     WNet actor, critic[2], target[2];
     const float* batch_base;               // [2][batch][obs + act]: current rows, then next rows
@@ -52,46 +57,33 @@ struct WideArgs {
     rlt_sas_parameters sas;
     float gamma;
     int batch, obs, act;
-    float* partial; int count;             // per workgroup and trained network: count floats (the optimiser's launch adds the blocks up)
+    int groups, roles, n_critics, by_xcd;   // row tiles, workgroups per tile, critics trained by the launch; by_xcd: workgroups of a role lie on as few XCDs as possible (each has its own L2)
+    Trained trained[2];                    // where the trained networks' activations and gradients go
+    float* extra;                          // actor update: [groups] the tiles' shares of the log_alpha gradient
+    uint64_t* exchange; unsigned max_poll; unsigned* fault;      // [groups][EXCHANGE] values handed from role to role: the value in the low word, a tag in the high one, zero before the launch
     float* out_log_probabilities; float* out_target_action_value; float* out_actions; float* out_pre_squashing;
     // TD3 (rl/algorithms/td3/operations_generic.h:170-281): `actor` is the target actor in the critic update and has `act` outputs; they pass tanh and the
     // td3_sampling layer (sac_heads.h); the critic update adds target_noise [batch][act] (already clamped) to the next action; the actor update goes through critic[0] only
     float sampling_std; int ignore_termination; const float* target_noise; float* out_pre_clip;
-    const float* noise_second;             // TD3 critic update of both critics in one launch: the sampling noise of the second (blockIdx.y = 1), each critic's targets being formed with its own
-    int packed;                            // every 8th workgroup of an 8 x larger grid works: all of them on one XCD
+    const float* noise_second;             // TD3 critic update of both critics in one launch: the sampling noise of the second, each critic's targets being formed with its own
 };
 
 __device__ __forceinline__ floatx4 mfma16(float a, float b, floatx4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 template <int ACT_H> __device__ __forceinline__ float act_hidden(float x, int f) { return rlt_act(x, ACT_H >= 0 ? ACT_H : f); }
 template <int ACT_H> __device__ __forceinline__ float dact_hidden(float o, int f) { return rlt_dact_from_output(o, ACT_H >= 0 ? ACT_H : f); }
 
-// B operands of one layer for this lane's output column n: W[n][16 j + 4 g ... + 3] for chunks j0 <= j < j0 + JN; zero beyond the layer's shape
+// The loads of operands are unconditional, from addresses clamped into the arrays: a load that some wavefronts skip makes the compiler wait for every load in flight before
+// the first value requested ahead of it is used (4 us at the start of a launch: the input rows, requested first, were waited for together with all weights). What lies
+// beyond a layer's shape is masked where it is used.
+// Weights are read from copies laid out in consumption order: [wavefront's 16 units][16-deep chunk j][lane][4] -- lane (c, g) finds W[16 w + c][16 j + 4 g ... + 3]
+// (forward copies of the first and second layers) or W[16 j + 4 g ... + 3][16 w + c] (backward copy of the second), zero beyond the layer's shape, and a wavefront's
+// load is 1 KB of consecutive addresses. Straight from W a lane's 16 bytes lie a row apart from its neighbour's: 64 lines per load, which the compute unit's address
+// pipeline takes 64 cycles for; first layers whose rows are no multiple of 16 bytes (17 or 35 inputs) take four such loads per chunk, 5 us at the start of a launch.
 template <int JN>
-__device__ __forceinline__ void load_rows(const float* __restrict__ W, int K, int N, bool vec, int n, int g, int j0, floatx4 (&b)[JN]) {
-    const bool n_ok = n < N;
-    const float* row = W + (size_t)(n_ok ? n : 0) * K;
+__device__ __forceinline__ void load_swizzled(const float* __restrict__ copy, int tiles, int wave, int lane, int j0, floatx4 (&b)[JN]) {      // tiles: chunks of the copy
+    const float* const mine = copy + ((size_t)wave * tiles * 64 + lane) * 4;
 #pragma unroll
-    for (int j = 0; j < JN; j++) {
-        const int k = 16 * (j0 + j) + 4 * g;
-        floatx4 v = {0.f, 0.f, 0.f, 0.f};
-        if (n_ok && k < K) {
-            if (vec) v = *reinterpret_cast<const floatx4*>(row + k);      // K is a multiple of 4 here
-            else { v[0] = row[k]; if (k + 1 < K) v[1] = row[k + 1]; if (k + 2 < K) v[2] = row[k + 2]; if (k + 3 < K) v[3] = row[k + 3]; }
-        }
-        b[j] = v;
-    }
-}
-// The same operands from a copy laid out in consumption order: [wavefront's 16 units][16-deep chunk j][lane][4] -- lane (c, g) finds W[16 w + c][16 j + 4 g ... + 3]
-// (forward copy) or W[16 j + 4 g ... + 3][16 w + c] (backward copy), zero beyond the layer's shape, and a wavefront's load is 1 KB of consecutive addresses. Straight from
-// W a lane's 16 bytes lie a row (1 KB) apart from its neighbour's: 64 lines per load, which the compute unit's address pipeline takes 64 cycles for.
-template <int JN>
-__device__ __forceinline__ void load_swizzled(const float* __restrict__ copy, int tiles, int wave, int lane, int j0, floatx4 (&b)[JN]) {
-#pragma unroll
-    for (int j = 0; j < JN; j++) {
-        floatx4 v = {0.f, 0.f, 0.f, 0.f};
-        if (j0 + j < tiles) v = *reinterpret_cast<const floatx4*>(copy + ((size_t)(wave * tiles + j0 + j) * 64 + lane) * 4);
-        b[j] = v;
-    }
+    for (int j = 0; j < JN; j++) b[j] = *reinterpret_cast<const floatx4*>(mine + (size_t)min(j0 + j, tiles - 1) * 256);      // chunks beyond the width are not used
 }
 // acc += in[rows][16 (j0 + j) + ...] * b[j], the workgroup's 16 rows against this lane's column
 template <int JN>
@@ -117,29 +109,31 @@ __device__ unsigned long long rlt_wide_ticks[2][32];
 // A wavefront's weight operands of one network: its 16 units' rows of W1 and W2 (the B operands of layers 1 and 2), row c of W3 for its 16 units, its lane's biases
 template <int NT1C>
 struct Operands { floatx4 w1[NT1C], w2a[8], w2b[8], w3; float b1, b2; };
-__device__ __forceinline__ floatx4 load_w3(const WNet& N, int wave, int c, int g) {
-    floatx4 w3 = {0.f, 0.f, 0.f, 0.f};
-    if (c < N.out) {      // row c of W3 (c < out), this wavefront's 16 units
-        const int k = 16 * wave + 4 * g;
-        const float* row = N.W3 + (size_t)c * N.hid;
-        if (N.vec3 && k + 3 < N.hid) w3 = *reinterpret_cast<const floatx4*>(row + k);
-        else { if (k < N.hid) w3[0] = row[k]; if (k + 1 < N.hid) w3[1] = row[k + 1]; if (k + 2 < N.hid) w3[2] = row[k + 2]; if (k + 3 < N.hid) w3[3] = row[k + 3]; }
+__device__ __forceinline__ floatx4 load_w3(const WNet& N, int wave, int c, int g) {      // row c of W3 (c < out), this wavefront's 16 units
+    floatx4 w3;
+    const int k = 16 * wave + 4 * g;
+    const float* row = N.W3 + (size_t)min(c, N.out - 1) * N.hid;
+    if (N.vec3) w3 = *reinterpret_cast<const floatx4*>(row + min(k, N.hid - 4));      // hid is a multiple of 4 here
+    else {
+#pragma unroll
+        for (int i = 0; i < 4; i++) w3[i] = row[min(k + i, N.hid - 1)];
     }
     return w3;
+}
+__device__ __forceinline__ void mask_w3(const WNet& N, int wave, int c, int g, floatx4& w3) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) if (c >= N.out || 16 * wave + 4 * g + i >= N.hid) w3[i] = 0.f;
 }
 // everything of network N that forward3 reads from memory, requested at once (few first-layer operands leave room for the whole second layer; otherwise its second
 // half is requested after the first layer has run)
 template <int NT1C>
 __device__ __forceinline__ void load_operands(const WNet& N, int wave, int c, int g, Operands<NT1C>& W) {
-    const int n = 16 * wave + c;
-    if (wave < ((N.hid + 15) >> 4)) {
-        load_rows<NT1C>(N.W1, N.in, N.hid, N.vec1, n, g, 0, W.w1);
-        const int tiles = (N.hid + 15) >> 4, lane = c + 16 * g;
-        load_swizzled<8>(N.W2f, tiles, wave, lane, 0, W.w2a);
-        if (NT1C <= 2) load_swizzled<8>(N.W2f, tiles, wave, lane, 8, W.w2b);
-        W.b1 = n < N.hid ? N.b1[n] : 0.f; W.b2 = n < N.hid ? N.b2[n] : 0.f;
-        W.w3 = load_w3(N, wave, c, g);
-    }
+    const int n = 16 * wave + c, tiles = (N.hid + 15) >> 4, lane = c + 16 * g;
+    load_swizzled<NT1C>(N.W1f, (N.in + 15) >> 4, wave, lane, 0, W.w1);
+    W.b1 = N.b1[min(n, N.hid - 1)]; W.b2 = N.b2[min(n, N.hid - 1)];
+    load_swizzled<8>(N.W2f, tiles, wave, lane, 0, W.w2a);
+    if (NT1C <= FEW) load_swizzled<8>(N.W2f, tiles, wave, lane, 8, W.w2b);
+    W.w3 = load_w3(N, wave, c, g);
 }
 
 // The three layers of network N on the workgroup's rows x [16][xstride]: this wavefront's tile of h1 and h2 (after the activation) into
@@ -150,296 +144,360 @@ __device__ __forceinline__ void load_operands(const WNet& N, int wave, int c, in
 // took as long as the layers' arithmetic when they were requested at the start of each pass.
 // First layers of more than two chunks fill too many registers for that: then only the second layer's first half (and the small operands) are requested ahead, the
 // first layer's own operands at the start of the pass (W1_READY = false) and the second half after the first layer, as before.
-template <int ACT_H, int NT1C, bool PREFETCH, bool W1_READY>
-__device__ __forceinline__ void forward3(const WNet& N, Operands<NT1C>& W, const WNet& next, lptr x, int xstride, lptr h1, lptr h2, lptr yp, int wave, int c, int g, int tick = -1) {
-#ifdef RLT_WIDE_PROFILE
-#define FT(i) do { if (tick >= 0 && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) rlt_wide_ticks[0][tick + i] = wall_clock64(); } while (0)
-#else
-#define FT(i) do {} while (0)
-#endif
-    const int HID = N.hid, n = 16 * wave + c, tiles = (HID + 15) >> 4;
-    const bool on = wave < tiles, n_ok = n < HID;
-    const int n_next = 16 * wave + c;
-    const bool next_on = PREFETCH && wave < ((next.hid + 15) >> 4);
-    const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
-    if (on) {
-        if (!W1_READY) load_rows<NT1C>(N.W1, N.in, HID, N.vec1, n, g, 0, W.w1);
-        floatx4 a0 = zero4, a1 = zero4;
-        FT(0);
-        chunks<NT1C>(a0, a1, x, xstride, c, g, 0, (N.in + 15) >> 4, W.w1);
-        FT(1);
-        const floatx4 acc = a0 + a1;
+// KEEP: the hidden layers' pre-activations and outputs are also stored to memory, rows [row0, row0 + 16) of [batch x hid] arrays (forward() of a network keeps them)
+struct KeepArgs { float* pre[2]; float* out[2]; int row0, batch; };
+template <int ACT_H, bool KEEP>
+__device__ __forceinline__ void place_hidden(const WNet& N, const floatx4& acc, float bias, lptr h, int n, int g, const KeepArgs* keep, int layer) {
+    const bool n_ok = n < N.hid;
 #pragma unroll
-        for (int v = 0; v < 4; v++) h1[(4 * g + v) * S + n] = n_ok ? act_hidden<ACT_H>(acc[v] + W.b1, N.act_h) : 0.f;
-        if (NT1C > 2) load_swizzled<8>(N.W2f, tiles, wave, c + 16 * g, 8, W.w2b);
+    for (int v = 0; v < 4; v++) {
+        const float pre = acc[v] + bias, o = act_hidden<ACT_H>(pre, N.act_h);
+        h[(4 * g + v) * S + n] = n_ok ? o : 0.f;
+        if (KEEP && n_ok && keep->row0 + 4 * g + v < keep->batch) {
+            const size_t at = (size_t)(keep->row0 + 4 * g + v) * N.hid + n;
+            if (keep->pre[layer]) keep->pre[layer][at] = pre;
+            if (keep->out[layer]) keep->out[layer][at] = o;
+        }
     }
-    if (next_on) {
-        if (NT1C <= 2) load_rows<NT1C>(next.W1, next.in, next.hid, next.vec1, n_next, g, 0, W.w1);
-        W.b1 = n_next < next.hid ? next.b1[n_next] : 0.f;
+}
+template <int ACT_H, int NT1C, bool PREFETCH, bool W1_READY, bool KEEP = false>
+__device__ __forceinline__ void forward3(const WNet& N, Operands<NT1C>& W, const WNet& next, lptr x, int xstride, lptr h1, lptr h2, lptr yp, int wave, int c, int g, const KeepArgs* keep = nullptr) {
+    const int n = 16 * wave + c, tiles = (N.hid + 15) >> 4, lane = c + 16 * g, next_tiles = (next.hid + 15) >> 4;
+    const bool on = wave < tiles;
+    const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
+    if (!W1_READY) load_swizzled<NT1C>(N.W1f, (N.in + 15) >> 4, wave, lane, 0, W.w1);
+    if (on) {
+        floatx4 a0 = zero4, a1 = zero4;
+        chunks<NT1C>(a0, a1, x, xstride, c, g, 0, (N.in + 15) >> 4, W.w1);
+        place_hidden<ACT_H, KEEP>(N, a0 + a1, W.b1, h1, n, g, keep, 0);
     }
-    FT(2);
+    if (NT1C > FEW) load_swizzled<8>(N.W2f, tiles, wave, lane, 8, W.w2b);
+    if (PREFETCH) {
+        if (NT1C <= FEW) load_swizzled<NT1C>(next.W1f, (next.in + 15) >> 4, wave, lane, 0, W.w1);
+        W.b1 = next.b1[min(n, next.hid - 1)];
+    }
     rlt_lds_barrier();
-    FT(3);
     {
         floatx4 a0 = zero4, a1 = zero4;
         if (on) chunks<8>(a0, a1, h1, S, c, g, 0, tiles, W.w2a);
-        if (next_on) load_swizzled<8>(next.W2f, (next.hid + 15) >> 4, wave, c + 16 * g, 0, W.w2a);
-        FT(4);
+        if (PREFETCH) load_swizzled<8>(next.W2f, next_tiles, wave, lane, 0, W.w2a);
         if (on) chunks<8>(a0, a1, h1, S, c, g, 8, tiles, W.w2b);
-        if (next_on && NT1C <= 2) load_swizzled<8>(next.W2f, (next.hid + 15) >> 4, wave, c + 16 * g, 8, W.w2b);
-        FT(5);
-        if (on) {
-            const floatx4 acc = a0 + a1;
-#pragma unroll
-            for (int v = 0; v < 4; v++) h2[(4 * g + v) * S + n] = n_ok ? act_hidden<ACT_H>(acc[v] + W.b2, N.act_h) : 0.f;
-        }
-        if (next_on) W.b2 = n_next < next.hid ? next.b2[n_next] : 0.f;
+        if (PREFETCH && NT1C <= FEW) load_swizzled<8>(next.W2f, next_tiles, wave, lane, 8, W.w2b);
+        if (on) place_hidden<ACT_H, KEEP>(N, a0 + a1, W.b2, h2, n, g, keep, 1);
+        if (PREFETCH) W.b2 = next.b2[min(n, next.hid - 1)];
     }
-    FT(6);
     rlt_lds_barrier();
-    FT(7);
     if (on) {
+        mask_w3(N, wave, c, g, W.w3);
         const floatx4 a = *(lptr4)(h2 + c * S + 16 * wave + 4 * g);
         floatx4 y = zero4;
         y = mfma16(a[0], W.w3[0], y); y = mfma16(a[1], W.w3[1], y); y = mfma16(a[2], W.w3[2], y); y = mfma16(a[3], W.w3[3], y);
 #pragma unroll
         for (int v = 0; v < 4; v++) yp[(wave * ROWS + 4 * g + v) * D3S + c] = y[v];
     }
-    if (next_on) W.w3 = load_w3(next, wave, c, g);
-    rlt_lds_barrier();
-}
-// The same three layers for a pass that requests its own operands when it starts (the actor update: its passes are separated by the head and the critics' backward
-// passes, which need the registers)
-// KEEP: the hidden layers' pre-activations and outputs are also stored to memory, rows [row0, row0 + 16) of [batch x hid] arrays (forward() of a network keeps them)
-struct KeepArgs { float* pre[2]; float* out[2]; int row0, batch; };
-template <int ACT_H, int NT1C, bool KEEP = false>
-__device__ __forceinline__ void forward3_own_loads(const WNet& N, lptr x, int xstride, lptr h1, lptr h2, lptr yp, int wave, int c, int g, const KeepArgs* keep = nullptr) {
-    const int HID = N.hid, n = 16 * wave + c, tiles = (HID + 15) >> 4;
-    const bool on = wave < tiles, n_ok = n < HID;
-    const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
-    floatx4 w2a[8], w2b[8], w3 = zero4;
-    float b1 = 0.f, b2 = 0.f;
-    if (on) {
-        floatx4 w1[NT1C];
-        load_rows<NT1C>(N.W1, N.in, HID, N.vec1, n, g, 0, w1);
-        load_swizzled<8>(N.W2f, tiles, wave, c + 16 * g, 0, w2a);      // on their way while the first layer runs
-        if (NT1C <= 2) load_swizzled<8>(N.W2f, tiles, wave, c + 16 * g, 8, w2b);      // few first-layer operands: room for the whole second layer at once
-        if (n_ok) { b1 = N.b1[n]; b2 = N.b2[n]; }
-        // the output layer's operands: row c of W3 (c < out), this wavefront's 16 units
-        if (c < N.out) {
-            const int k = 16 * wave + 4 * g;
-            const float* row = N.W3 + (size_t)c * HID;
-            if (N.vec3 && k + 3 < HID) w3 = *reinterpret_cast<const floatx4*>(row + k);
-            else { if (k < HID) w3[0] = row[k]; if (k + 1 < HID) w3[1] = row[k + 1]; if (k + 2 < HID) w3[2] = row[k + 2]; if (k + 3 < HID) w3[3] = row[k + 3]; }
-        }
-        floatx4 a0 = zero4, a1 = zero4;
-        chunks<NT1C>(a0, a1, x, xstride, c, g, 0, (N.in + 15) >> 4, w1);
-        const floatx4 acc = a0 + a1;
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const float pre = acc[v] + b1, o = act_hidden<ACT_H>(pre, N.act_h);
-            h1[(4 * g + v) * S + n] = n_ok ? o : 0.f;
-            if (KEEP && n_ok && keep->row0 + 4 * g + v < keep->batch) {
-                const size_t at = (size_t)(keep->row0 + 4 * g + v) * HID + n;
-                if (keep->pre[0]) keep->pre[0][at] = pre;
-                if (keep->out[0]) keep->out[0][at] = o;
-            }
-        }
-        if (NT1C > 2) load_swizzled<8>(N.W2f, tiles, wave, c + 16 * g, 8, w2b);
-    }
-    rlt_lds_barrier();
-    if (on) {
-        floatx4 a0 = zero4, a1 = zero4;
-        chunks<8>(a0, a1, h1, S, c, g, 0, tiles, w2a);
-        chunks<8>(a0, a1, h1, S, c, g, 8, tiles, w2b);
-        const floatx4 acc = a0 + a1;
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const float pre = acc[v] + b2, o = act_hidden<ACT_H>(pre, N.act_h);
-            h2[(4 * g + v) * S + n] = n_ok ? o : 0.f;
-            if (KEEP && n_ok && keep->row0 + 4 * g + v < keep->batch) {
-                const size_t at = (size_t)(keep->row0 + 4 * g + v) * HID + n;
-                if (keep->pre[1]) keep->pre[1][at] = pre;
-                if (keep->out[1]) keep->out[1][at] = o;
-            }
-        }
-    }
-    rlt_lds_barrier();
-    if (on) {
-        const floatx4 a = *(lptr4)(h2 + c * S + 16 * wave + 4 * g);
-        floatx4 y = zero4;
-        y = mfma16(a[0], w3[0], y); y = mfma16(a[1], w3[1], y); y = mfma16(a[2], w3[2], y); y = mfma16(a[3], w3[3], y);
-#pragma unroll
-        for (int v = 0; v < 4; v++) yp[(wave * ROWS + 4 * g + v) * D3S + c] = y[v];
-    }
+    if (PREFETCH) W.w3 = load_w3(next, wave, c, g);
     rlt_lds_barrier();
 }
 // the sums of the partial tiles, in wavefront order: element v of lane (c, g) belongs to row 4 g + v, column c
 __device__ __forceinline__ floatx4 output_tile(lptr yp, int tiles, int c, int g) {
     floatx4 y = {0.f, 0.f, 0.f, 0.f};
-    for (int w = 0; w < tiles; w++)
 #pragma unroll
-        for (int v = 0; v < 4; v++) y[v] += yp[(w * ROWS + 4 * g + v) * D3S + c];
+    for (int w0 = 0; w0 < WAVES; w0 += 4) {      // four tiles' reads in flight together; tiles beyond the width's are never written
+        float p[4][4];
+#pragma unroll
+        for (int w = 0; w < 4; w++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) p[w][v] = yp[((w0 + w) * ROWS + 4 * g + v) * D3S + c];
+#pragma unroll
+        for (int w = 0; w < 4; w++)
+            if (w0 + w < tiles)
+#pragma unroll
+                for (int v = 0; v < 4; v++) y[v] += p[w][v];
+    }
     return y;
 }
 
-// this wavefront's tile of d_pre2 = (d_pre3 W3) f'(h2) into g2 (may be h2 itself); returns the lane's share of its unit's column sum
+// column n of W3 for this lane's share of the reduction over the outputs, and the second layer's backward copy: the operands of a backward pass, requested ahead of it
+struct BackOperands { float w3[MAX_OUT / 4]; floatx4 w2[MAX_H / 16]; };
+__device__ __forceinline__ void load_back_operands(const WNet& N, int wave, int c, int g, BackOperands& W) {
+    const int n = 16 * wave + c, tiles = (N.hid + 15) >> 4;
+#pragma unroll
+    for (int ks = 0; ks < MAX_OUT / 4; ks++) W.w3[ks] = N.W3[(size_t)min(4 * ks + g, N.out - 1) * N.hid + min(n, N.hid - 1)];
+    load_swizzled<MAX_H / 16>(N.W2b, tiles, wave, c + 16 * g, 0, W.w2);
+}
+// this wavefront's tile of d_pre2 = (d_pre3 W3) f'(h2) into g2 (may be h2 itself)
 template <int ACT_H>
-__device__ __forceinline__ float backward_layer3(const WNet& N, lptr d3, lptr h2, lptr g2, int wave, int c, int g) {
+__device__ __forceinline__ void backward_layer3(const WNet& N, const BackOperands& W, lptr d3, lptr h2, lptr g2, int wave, int c, int g) {
     const int n = 16 * wave + c;
     const bool n_ok = n < N.hid;
     floatx4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int ks = 0; ks < MAX_OUT / 4; ks++) {
-        const int o = 4 * ks + g;
-        const float w = (o < N.out && n_ok) ? N.W3[(size_t)o * N.hid + n] : 0.f;
-        acc = mfma16(d3[c * D3S + 4 * ks + g], w, acc);      // columns of d_pre3 beyond the output width are zero
-    }
-    float sum = 0.f;
+    for (int ks = 0; ks < MAX_OUT / 4; ks++) acc = mfma16(d3[c * D3S + 4 * ks + g], 4 * ks + g < N.out ? W.w3[ks] : 0.f, acc);      // columns of d_pre3 beyond the output width are zero
 #pragma unroll
     for (int v = 0; v < 4; v++) {
         const int idx = (4 * g + v) * S + n;
-        const float dp = n_ok ? acc[v] * dact_hidden<ACT_H>(h2[idx], N.act_h) : 0.f;
-        g2[idx] = dp; sum += dp;
+        g2[idx] = n_ok ? acc[v] * dact_hidden<ACT_H>(h2[idx], N.act_h) : 0.f;
     }
-    return sum;
 }
-// this wavefront's tile of d_pre1 = (d_pre2 W2) f'(h1) into p1 (may be h1 itself); returns the lane's share of its unit's column sum
+// this wavefront's tile of d_pre1 = (d_pre2 W2) f'(h1) into p1 (may be h1 itself)
 template <int ACT_H>
-__device__ __forceinline__ float backward_layer2(const WNet& N, lptr g2, lptr h1, lptr p1, int wave, int c, int g) {
-    const int HID = N.hid, n = 16 * wave + c, tiles = (HID + 15) >> 4;
-    const bool n_ok = n < HID;
+__device__ __forceinline__ void backward_layer2(const WNet& N, const BackOperands& W, lptr g2, lptr h1, lptr p1, int wave, int c, int g) {
+    const int n = 16 * wave + c, tiles = (N.hid + 15) >> 4;
+    const bool n_ok = n < N.hid;
     const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
     floatx4 a0 = zero4, a1 = zero4;
-#pragma unroll 1
-    for (int j0 = 0; j0 < tiles; j0 += 4) {
-        floatx4 b[4];
-        load_swizzled<4>(N.W2b, tiles, wave, c + 16 * g, j0, b);      // W2[16 j + 4 g + i][n]
-        chunks<4>(a0, a1, g2, S, c, g, j0, tiles, b);
-    }
+    chunks<MAX_H / 16>(a0, a1, g2, S, c, g, 0, tiles, W.w2);
     const floatx4 acc = a0 + a1;
-    float sum = 0.f;
 #pragma unroll
     for (int v = 0; v < 4; v++) {
         const int idx = (4 * g + v) * S + n;
-        const float dp = n_ok ? acc[v] * dact_hidden<ACT_H>(h1[idx], N.act_h) : 0.f;
-        p1[idx] = dp; sum += dp;
+        p1[idx] = n_ok ? acc[v] * dact_hidden<ACT_H>(h1[idx], N.act_h) : 0.f;
     }
-    return sum;
 }
-
-// The copies of the second layers' weights that load_swizzled reads, made anew before every update (the optimisers change the weights between them): thread t of
-// block (x, job) writes the 16 bytes of lane t % 64 of one (wavefront, chunk) pair. Forward copies read 16 consecutive bytes of a row of W2, backward copies four
-// values a row apart (the 16 lanes of a group read 64 consecutive bytes each time).
-constexpr int PREP_JOBS = 8;
-struct PrepArgs { const float* W2[PREP_JOBS]; float* dst[PREP_JOBS]; int hid[PREP_JOBS]; int backward[PREP_JOBS]; };
+// The workgroup's 16 rows of an array between memory and LDS: wavefront w takes row w, all of a lane's loads are on their way before the first is written (a loop that
+// writes each element before the next load cost 3.8 us at the start of a launch, three trips to memory one after the other; and the operands' wait with it). Columns from `cols` on are zero.
+template <int N>
+__device__ __forceinline__ void request_row(const float* row, int cols, int lane, float (&v)[N]) {
+#pragma unroll
+    for (int u = 0; u < N; u++) v[u] = row[min(64 * u + lane, cols - 1)];
+}
+template <int N>
+__device__ __forceinline__ void place_row(lptr to, bool ok, int cols, int end, int lane, const float (&v)[N]) {
+#pragma unroll
+    for (int u = 0; u < N; u++) if (64 * u + lane < end) to[64 * u + lane] = ok && 64 * u + lane < cols ? v[u] : 0.f;
+}
+__device__ __forceinline__ void store_rows(lptr from, float* to, int hid, int row0, int batch, int wave, int lane) {
+    if (row0 + wave >= batch) return;
+    float* const row = to + (size_t)(row0 + wave) * hid;
+    for (int n = lane; n < hid; n += 64) row[n] = from[wave * S + n];
+}
+// A value handed from one workgroup to another of the same launch: one 8-byte store that carries its own tag, so that nothing has to be ordered around it. The wait is
+// bounded (rlt_rocm_set_wait_limit); a workgroup that gives up sets the fault word and goes on with zero, and the update's results are void.
+__device__ __forceinline__ void hand_over(uint64_t* word, float value) {
+    __hip_atomic_store(word, (1ull << 32) | (uint64_t)__float_as_uint(value), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <int N>
+__device__ __forceinline__ void take_over(uint64_t* const (&word)[N], float (&value)[N], unsigned max_poll, unsigned* fault) {
+    for (unsigned tries = 0;;) {
+        bool all = true;
+        uint64_t w[N];
+#pragma unroll
+        for (int i = 0; i < N; i++) w[i] = __hip_atomic_load(word[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);      // one trip for all of them
+#pragma unroll
+        for (int i = 0; i < N; i++) { all = all && (w[i] >> 32) != 0; value[i] = __uint_as_float((uint32_t)w[i]); }
+        if (all) return;
+        if (++tries >= max_poll) { __hip_atomic_store(fault, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); return; }
+        __builtin_amdgcn_s_sleep(1);
+    }
+}
+// The copies of the weights that load_swizzled reads, made anew before every update (the optimisers change the weights between them): thread t of block (x, job) writes
+// the 16 bytes of lane t % 64 of one (wavefront, chunk) pair, for all sixteen wavefronts whatever the width (those beyond it find zeros). Forward copies read 16
+// consecutive bytes of a row, backward copies four values a row apart (the 16 lanes of a group read 64 consecutive bytes each time).
+constexpr int PREP_JOBS = 12;
+struct PrepArgs {
+    const float* W[PREP_JOBS]; float* dst[PREP_JOBS]; int units[PREP_JOBS], depth[PREP_JOBS], backward[PREP_JOBS];      // W [units][depth], or for a backward copy [depth][units]
+    uint64_t* clear; int n_clear;                      // words that the next launch wants zero
+    uint32_t* age[3]; uint32_t* age_before;            // optimiser ages that are advanced, their values before that left in age_before (read by the optimisers' launch)
+};
+size_t copy_floats(int depth) { return (size_t)WAVES * ((depth + 15) >> 4) * 256; }
 __global__ __launch_bounds__(256) void wide_prepare_kernel(PrepArgs P) {
-    const int job = blockIdx.y, HID = P.hid[job], tiles = (HID + 15) >> 4;
+    const int job = blockIdx.y, units = P.units[job], depth = P.depth[job], chunks = (depth + 15) >> 4;
     const int t = blockIdx.x * 256 + threadIdx.x;
-    if (t >= tiles * tiles * 64) return;
-    const int lane = t & 63, pair = t >> 6, w = pair / tiles, j = pair - w * tiles, c = lane & 15, g = lane >> 4;
+    for (int i = (blockIdx.y * gridDim.x + blockIdx.x) * 256 + threadIdx.x; i < P.n_clear; i += gridDim.x * gridDim.y * 256) P.clear[i] = 0;
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 3 && P.age_before) {
+        uint32_t* const age = threadIdx.x == 0 ? P.age[0] : threadIdx.x == 1 ? P.age[1] : P.age[2];
+        if (age) { const uint32_t before = *age; P.age_before[threadIdx.x] = before; *age = before + 1; }
+    }
+    if (t >= WAVES * chunks * 64) return;
+    const int lane = t & 63, pair = t >> 6, w = pair / chunks, j = pair - w * chunks, c = lane & 15, g = lane >> 4;
     const int n = 16 * w + c, k = 16 * j + 4 * g;
-    const float* W = P.W2[job];
+    const float* W = P.W[job];
     floatx4 v = {0.f, 0.f, 0.f, 0.f};
-    if (n < HID) {
+    if (n < units) {
 #pragma unroll
         for (int i = 0; i < 4; i++)
-            if (k + i < HID) v[i] = P.backward[job] ? W[(size_t)(k + i) * HID + n] : W[(size_t)n * HID + k + i];
+            if (k + i < depth) v[i] = P.backward[job] ? W[(size_t)(k + i) * units + n] : W[(size_t)n * depth + k + i];
     }
     *reinterpret_cast<floatx4*>(P.dst[job] + (size_t)t * 4) = v;
 }
+// The copies of a launch: asked for one by one (a copy that is asked for again is shared), then made by one launch.
+struct Copies {
+    PrepArgs args = {}; int jobs = 0, blocks = 1; float* next;
+    explicit Copies(float* memory) : next(memory) {}
+    const float* copy(const float* W, int units, int depth, bool backward) {
+        for (int q = 0; q < jobs; q++) if (args.W[q] == W && args.backward[q] == (int)backward) return args.dst[q];
+        args.W[jobs] = W; args.dst[jobs] = next; args.units[jobs] = units; args.depth[jobs] = depth; args.backward[jobs] = backward;
+        next += copy_floats(depth);
+        const int b = rlt_div_up(WAVES * ((depth + 15) >> 4) * 64, 256);
+        if (b > blocks) blocks = b;
+        return args.dst[jobs++];
+    }
+    void forward(WNet& N) { N.W1f = copy(N.W1, N.hid, N.in, false); N.W2f = copy(N.W2, N.hid, N.hid, false); }
+    void backward(WNet& N) { N.W2b = copy(N.W2, N.hid, N.hid, true); }
+    int launch(rlt_rocm_device* device) {
+        hipLaunchKernelGGL(wide_prepare_kernel, dim3(blocks, jobs), dim3(256), 0, device->stream, args);
+        return rlt_launch_status(device);
+    }
+};
+constexpr size_t MAX_COPY_FLOATS = (size_t)WAVES * (MAX_H / 16) * 256, MAX_W1_COPY_FLOATS = (size_t)WAVES * (MAX_D / 16) * 256;
 
 template <int MODE, int ACT_H, int NT1C>
 __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
     constexpr bool CRITIC = MODE == MODE_CRITIC || MODE == MODE_TD3_CRITIC, TD3 = MODE == MODE_TD3_CRITIC || MODE == MODE_TD3_ACTOR;
     extern __shared__ __attribute__((aligned(16))) float lds_wide[];
-    if (A.packed && (blockIdx.x & 7)) return;
-    const int gi = A.packed ? blockIdx.x >> 3 : blockIdx.x, G = A.packed ? gridDim.x >> 3 : gridDim.x;
-    const int y = CRITIC ? blockIdx.y : 0;
+    const int G = A.groups;
+    const int place = A.by_xcd ? (int)((blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3)) : (int)blockIdx.x;
+    if (place >= A.roles * G) return;
+    const int role = place / G, gi = place - role * G;
     const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const bool scalar_wave = wave == 0;
     const int OBS = A.obs, ACT = A.act, D = OBS + ACT, B = A.batch;
-    const lptr xa = (lptr)lds_wide, xb = xa + ROWS * SXS, h1 = xb + ROWS * SXS, h2 = h1 + ROWS * S, ta = h2 + ROWS * S, tb = ta + ROWS * S,
+    const lptr xa = (lptr)lds_wide, h1 = xa + ROWS * SXS, h2 = h1 + ROWS * S, ta = h2 + ROWS * S, tb = ta + ROWS * S,
                d3 = tb + ROWS * S, d3c = d3 + ROWS * D3S, da = d3c + ROWS * D3S, yp = da + 2 * ROWS * D3S, misc = yp + WAVES * YP;
     const int row0 = gi * ROWS;
     const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
-    const WNet trained = CRITIC ? (y ? A.critic[1] : A.critic[0]) : A.actor;      // by value: an index into the kernel's argument would keep all of it in private memory
-    const int HID = trained.hid, tiles = (HID + 15) >> 4;
-    const bool on = wave < tiles;
+    uint64_t* const exchange = A.exchange + (size_t)gi * EXCHANGE;
+    const bool row_ok = row0 + c < B;
+    // critic update: target roles [set][target critic] first, then a role per trained critic; actor update: critic 1's role (SAC), then the role that goes on with the actor
+    const int n_target_roles = CRITIC ? 2 * (TD3 ? A.n_critics : 1) : 0;
+    const bool target_role = CRITIC && role < n_target_roles;
+    const int set = target_role ? role >> 1 : 0;
 
-    // the input tiles: xa = next rows (critic update) or current rows (actor update; the actor reads its observation columns), xb = current rows
-    for (int e = threadIdx.x; e < ROWS * SXS; e += THREADS) {
-        const int r = e / SXS, k = e % SXS;
-        const bool ok = row0 + r < B && k < D;
-        const float* cur = A.batch_base + (size_t)min(row0 + r, B - 1) * D + min(k, D - 1);
-        if (CRITIC) { xa[e] = ok ? cur[(size_t)B * D] : 0.f; xb[e] = ok ? cur[0] : 0.f; }
-        else xa[e] = (ok && k < OBS) ? cur[0] : 0.f;
+    RLT_TICK(0);
+    // the input rows: next rows for the target roles, else the current ones (the actor reads their observation columns, zero beyond them until the sample is in place)
+    float in_row[3];
+    request_row(A.batch_base + (target_role ? (size_t)B * D : 0) + (size_t)min(row0 + wave, B - 1) * D, CRITIC ? D : OBS, lane, in_row);
+    if (CRITIC && !target_role) {
+        // ---- a trained critic
+        const int y = role - n_target_roles;
+        const WNet trained = y ? A.critic[1] : A.critic[0];      // by value: an index into the kernel's argument would keep all of it in private memory
+        const Trained T = y ? A.trained[1] : A.trained[0];
+        const int HID = trained.hid, tiles = (HID + 15) >> 4;
+        Operands<NT1C> W;
+        load_operands<NT1C>(trained, wave, c, g, W);
+        place_row(xa + wave * SXS, row0 + wave < B, CRITIC ? D : OBS, SXS, lane, in_row);
+        float reward[4] = {0.f, 0.f, 0.f, 0.f}, alpha = 0.f, b3 = 0.f;
+        bool terminated[4] = {false, false, false, false};
+        if (scalar_wave) {
+            b3 = trained.b3[0];
+            if (!TD3) alpha = expf(*A.log_alpha);
+#pragma unroll
+            for (int v = 0; v < 4; v++) { const int row = min(row0 + 4 * g + v, B - 1); reward[v] = A.rewards[row]; terminated[v] = A.terminated[row] != 0; }
+        }
+        rlt_lds_barrier();      // the input rows are in place
+        RLT_TICK(1);
+        forward3<ACT_H, NT1C, false, true>(trained, W, trained, xa, SXS, h1, h2, yp, wave, c, g);
+        RLT_TICK(2);
+        BackOperands K;
+        load_back_operands(trained, wave, c, g, K);      // on their way while the targets' values are waited for
+        store_rows(h1, T.h1, HID, row0, B, wave, lane);
+        store_rows(h2, T.h2, HID, row0, B, wave, lane);
+        if (scalar_wave) {
+            // TD target of rows 4 g + v (meaningful in the lanes c == 0, which hold output 0), MSE gradient at the critic's pre-activation:
+            // loss weight batch * 0.5 / n with n = batch rows (no masks), times the MSE gradient's 2 / batch (rl/algorithms/sac/operations_generic.h:298-316)
+            const floatx4 yc = output_tile(yp, tiles, c, g);
+            // (TD3: loss weight batch / n, rl/algorithms/td3/operations_generic.h:200-212)
+            const float loss_weight = TD3 ? (float)B / (float)B : (1.0f / (float)B) * ((float)B * 0.5f);
+            const float constant = 2.0f / (float)B * loss_weight;
+            uint64_t* const slot = exchange + (TD3 ? 2 * y : 0) * ROWS;
+            uint64_t* word[TD3 ? 8 : 12];
+            float value[TD3 ? 8 : 12];
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                word[v] = slot + 4 * g + v; word[4 + v] = slot + ROWS + 4 * g + v;
+                if (!TD3) word[(TD3 ? 0 : 8) + v] = exchange + LOG_PROB_SLOT * ROWS + 4 * g + v;
+            }
+            take_over(word, value, A.max_poll, A.fault);
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int row = 4 * g + v;
+                const float q_min = fminf(value[v], value[4 + v]);
+                const float min_q = TD3 ? q_min : q_min - alpha * value[(TD3 ? 0 : 8) + v];
+                const float future = (terminated[v] && !(TD3 && A.ignore_termination)) ? 0.0f : A.gamma * min_q;
+                const float y_target = reward[v] + future;
+                const bool ok = c == 0 && row0 + row < B;
+                // (SAC's critics share their targets; TD3's are formed with each critic's own sampling noise: the last critic's stay, as after two calls)
+                if (A.out_target_action_value && ok && y == (TD3 ? A.n_critics - 1 : 0)) A.out_target_action_value[row0 + row] = y_target;
+                const float diff = (yc[v] + b3) - y_target;
+                const float dp = ok ? diff * constant : 0.f;
+                d3[row * D3S + c] = dp;
+                if (row0 + row < B) T.d3[(size_t)(row0 + row) * MAX_OUT + c] = dp;
+            }
+        }
+        rlt_lds_barrier();      // d_pre3 is in place
+        RLT_TICK(3);
+        if (wave < tiles) backward_layer3<ACT_H>(trained, K, d3, h2, ta, wave, c, g);
+        rlt_lds_barrier();      // every wavefront's tile of d_pre2 is in place
+        store_rows(ta, T.d2, HID, row0, B, wave, lane);
+        if (wave < tiles) backward_layer2<ACT_H>(trained, K, ta, h1, tb, wave, c, g);
+        rlt_lds_barrier();
+        store_rows(tb, T.d1, HID, row0, B, wave, lane);
+        RLT_TICK(4);
+        return;
     }
-    float noise[2] = {0.f, 0.f}, target_noise[2] = {0.f, 0.f}, reward[4] = {0.f, 0.f, 0.f, 0.f}, alpha = 0.f, s3 = 0.f, extra = 0.f;
-    bool terminated[4] = {false, false, false, false};
+
+    // ---- target roles and the actor update: the actor (critic update: on the next observations; actor update: on the observations)
+    const int critic_index = target_role ? (role & 1) : (role == A.roles - 1 ? 0 : 1);
+    const bool owner = !CRITIC && critic_index == 0;
+    const bool writes = target_role ? role == 0 : owner;      // of the roles that compute the same sample, the one that stores what is asked for
+    const WNet Q = CRITIC ? (critic_index ? A.target[1] : A.target[0]) : (critic_index ? A.critic[1] : A.critic[0]);
+    Operands<NT1C> W;
+    load_operands<NT1C>(A.actor, wave, c, g, W);      // on their way while the input rows are written
+    place_row(xa + wave * SXS, row0 + wave < B, CRITIC ? D : OBS, SXS, lane, in_row);
+    float noise[2] = {0.f, 0.f}, target_noise[2] = {0.f, 0.f}, alpha = 0.f, actor_b3 = 0.f, q_b3 = 0.f;
     if (scalar_wave) {
+        actor_b3 = c < A.actor.out ? A.actor.b3[c] : 0.f; q_b3 = Q.b3[0];
         if (!TD3) alpha = expf(*A.log_alpha);
         if (MODE == MODE_TD3_CRITIC) {
 #pragma unroll
             for (int j = 0; j < 2; j++) {
-                if (g + 4 * j < ACT && row0 + c < B) {
+                if (g + 4 * j < ACT && row_ok) {
                     const size_t i = (size_t)(row0 + c) * ACT + g + 4 * j;
                     if (A.target_noise) target_noise[j] = A.target_noise[i];
                     else {
                         const float scaled = rlt_randn_element(A.noise_seed, A.target_noise_stream + *A.stream_offset, i) * A.target_noise_std + 0.0f;
                         target_noise[j] = clampf(scaled, -A.target_noise_clip, A.target_noise_clip);
-                        if (y == 0) A.out_target_noise[i] = target_noise[j];
+                        if (writes) A.out_target_noise[i] = target_noise[j];
                     }
                 }
             }
         }
 #pragma unroll
         for (int j = 0; j < 2; j++) {
-            if (g + 4 * j < ACT && row0 + c < B) {
+            if (g + 4 * j < ACT && row_ok) {
                 const size_t i = (size_t)(row0 + c) * ACT + g + 4 * j;
-                const float* const given = (MODE == MODE_TD3_CRITIC && y) ? A.noise_second : A.noise;
-                noise[j] = given ? given[i] : rlt_randn_element(A.noise_seed, ((MODE == MODE_TD3_CRITIC && y) ? A.noise_stream_second : A.noise_stream) + *A.stream_offset, i);
-                if (A.out_noise && y == 0) A.out_noise[i] = noise[j];
+                const float* const given = (MODE == MODE_TD3_CRITIC && set) ? A.noise_second : A.noise;
+                noise[j] = given ? given[i] : rlt_randn_element(A.noise_seed, ((MODE == MODE_TD3_CRITIC && set) ? A.noise_stream_second : A.noise_stream) + *A.stream_offset, i);
+                if (A.out_noise && writes) A.out_noise[i] = noise[j];
             }
-        }
-        if (CRITIC) {
-#pragma unroll
-            for (int v = 0; v < 4; v++) { const int row = min(row0 + 4 * g + v, B - 1); reward[v] = A.rewards[row]; terminated[v] = A.terminated[row] != 0; }
         }
     }
     HeadItem item[2];
-    const bool row_ok = row0 + c < B;
-    Operands<NT1C> W;
-    if (CRITIC) load_operands<NT1C>(A.actor, wave, c, g, W);      // on their way while the input tiles are written
-    RLT_TICK(0);
-    rlt_lds_barrier();      // the input tiles are in place
-    RLT_TICK(1);
-
-    // the actor (critic update: on the next observations; actor update: on the observations, activations kept for its backward pass)
-    if (CRITIC) forward3<ACT_H, NT1C, true, true>(A.actor, W, A.target[0], xa, SXS, ta, tb, yp, wave, c, g);
-    else forward3_own_loads<ACT_H, NT1C>(A.actor, xa, SXS, h1, h2, yp, wave, c, g);
-    RLT_TICK(2);
+    RLT_TICK(13);
+    rlt_lds_barrier();      // the input rows are in place
+    RLT_TICK(5);
+    forward3<ACT_H, NT1C, true, true>(A.actor, W, Q, xa, SXS, h1, h2, yp, wave, c, g);
+    RLT_TICK(6);
     if (scalar_wave) {
         const floatx4 out = output_tile(yp, (A.actor.hid + 15) >> 4, c, g);
-        const float b3 = c < A.actor.out ? A.actor.b3[c] : 0.f;
 #pragma unroll
-        for (int v = 0; v < 4; v++) d3[(4 * g + v) * D3S + c] = c < A.actor.out ? out[v] + b3 : 0.f;
+        for (int v = 0; v < 4; v++) d3[(4 * g + v) * D3S + c] = c < A.actor.out ? out[v] + actor_b3 : 0.f;
         wave_sync();
         float log_prob = 0.f;
         if (TD3) td3_head_forward(OBS, ACT, A.sampling_std, d3, D3S, xa, SXS, noise, target_noise, CRITIC, c, g, item);
         else log_prob = head_forward(A.sas, OBS, ACT, d3, D3S, xa, SXS, noise, c, g, item);
         if (TD3) {
-            if (!CRITIC && row_ok && A.out_pre_clip) {
+            if (owner && row_ok && A.out_pre_clip) {
 #pragma unroll
                 for (int j = 0; j < 2; j++)
                     if (g + 4 * j < ACT) A.out_pre_clip[(size_t)(row0 + c) * ACT + g + 4 * j] = item[j].sample;
             }
-        } else if (g == 0) {
-            if (CRITIC) misc[c] = log_prob;
+        } else if (g == 0 && writes) {
+            if (CRITIC) hand_over(exchange + LOG_PROB_SLOT * ROWS + c, log_prob);
             if (A.out_log_probabilities && row_ok) A.out_log_probabilities[row0 + c] = log_prob;
         }
-        if (!TD3 && !CRITIC && row_ok) {
+        if (!TD3 && owner && row_ok) {
 #pragma unroll
             for (int j = 0; j < 2; j++)
                 if (g + 4 * j < ACT) {
@@ -449,213 +507,132 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
         }
     }
     rlt_lds_barrier();      // the action columns of xa are in place
-    RLT_TICK(3);
-
+    RLT_TICK(7);
+    forward3<ACT_H, NT1C, false, NT1C <= FEW>(Q, W, Q, xa, SXS, ta, tb, yp, wave, c, g);
+    RLT_TICK(8);
+    const int qtiles = (Q.hid + 15) >> 4;
     if (CRITIC) {
-        // both target critics on [next observation | sampled action], then the trained critic on the current rows
-        floatx4 q_next[2];
+        if (scalar_wave && c == 0) {
+            const floatx4 q = output_tile(yp, qtiles, c, g);
 #pragma unroll
-        for (int k = 0; k < 2; k++) {
-            const WNet T = k ? A.target[1] : A.target[0];
-            const WNet after = k ? trained : A.target[1];
-            forward3<ACT_H, NT1C, true, NT1C <= 2>(T, W, after, xa, SXS, ta, tb, yp, wave, c, g, k == 0 && CRITIC ? 20 : -1);
-            RLT_TICK(4 + k);
-            if (scalar_wave) { q_next[k] = output_tile(yp, (T.hid + 15) >> 4, c, g); const float b3 = T.b3[0]; for (int v = 0; v < 4; v++) q_next[k][v] += b3; }
+            for (int v = 0; v < 4; v++) hand_over(exchange + (2 * set + critic_index) * ROWS + 4 * g + v, q[v] + q_b3);
         }
-        forward3<ACT_H, NT1C, false, NT1C <= 2>(trained, W, trained, xb, SXS, h1, h2, yp, wave, c, g);
-        RLT_TICK(6);
-        if (scalar_wave) {
-            // TD target of rows 4 g + v (meaningful in the lanes c == 0, which hold output 0), MSE gradient at the critic's pre-activation:
-            // loss weight batch * 0.5 / n with n = batch rows (no masks), times the MSE gradient's 2 / batch (rl/algorithms/sac/operations_generic.h:298-316)
-            const floatx4 yc = output_tile(yp, tiles, c, g);
-            const float b3 = trained.b3[0];
-            // (TD3: loss weight batch / n, rl/algorithms/td3/operations_generic.h:200-212)
-            const float loss_weight = TD3 ? (float)B / (float)B : (1.0f / (float)B) * ((float)B * 0.5f);
-            const float constant = 2.0f / (float)B * loss_weight;
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const float q_min = fminf(q_next[0][v], q_next[1][v]);
-                const float min_q = TD3 ? q_min : q_min - alpha * misc[4 * g + v];
-                const float future = (terminated[v] && !(TD3 && A.ignore_termination)) ? 0.0f : A.gamma * min_q;
-                const float y_target = reward[v] + future;
-                const bool ok = c == 0 && row0 + 4 * g + v < B;
-                // (SAC's critics share their targets; TD3's are formed with each critic's own sampling noise: the last critic's stay, as after two calls)
-                if (A.out_target_action_value && ok && y == (TD3 ? (int)gridDim.y - 1 : 0)) A.out_target_action_value[row0 + 4 * g + v] = y_target;
-                const float diff = (yc[v] + b3) - y_target;
-                const float dp = ok ? diff * constant : 0.f;
-                if (ok) extra += diff * diff;
-                s3 += dp;
-                d3[(4 * g + v) * D3S + c] = dp;
-            }
-        }
-        rlt_lds_barrier();      // d_pre3 is in place
-        RLT_TICK(7);
-    } else {
-        // each critic (TD3: critic 0 only, rl/algorithms/td3/operations_generic.h:260): value on [observation | sampled action], then the gradient of -value / batch
-        // with respect to the action
-        const float loss_weight = (1.0f / (float)B) * -1.0f;       // rl/algorithms/sac/operations_generic.h:437-453 with n = batch rows
-#pragma unroll 1
-        for (int k = 0; k < (TD3 ? 1 : 2); k++) {
-            const WNet C = k ? A.critic[1] : A.critic[0];
-            const int ctiles = (C.hid + 15) >> 4;
-            forward3_own_loads<ACT_H, NT1C>(C, xa, SXS, ta, tb, yp, wave, c, g);
-            RLT_TICK(4 + 4 * k);
-            if (scalar_wave) {
-                const floatx4 out = output_tile(yp, ctiles, c, g);
-                const float b3 = C.b3[0];
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    if (c == 0) misc[16 * k + 4 * g + v] = out[v] + b3;
-                    d3c[(4 * g + v) * D3S + c] = (c == 0 && row0 + 4 * g + v < B) ? loss_weight : 0.f;
-                }
-            }
-            rlt_lds_barrier();
-            if (wave < ctiles) backward_layer3<ACT_H>(C, d3c, tb, tb, wave, c, g);
-            rlt_lds_barrier();
-            RLT_TICK(5 + 4 * k);
-            if (wave < ctiles) {
-                backward_layer2<ACT_H>(C, tb, ta, ta, wave, c, g);
-                wave_sync();
-                // d value / d action = the action columns of d_pre1 W1: this wavefront's units' share of the reduction
-                floatx4 acc = zero4;
-                const floatx4 a = *(lptr4)(ta + c * S + 16 * wave + 4 * g);
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int unit = 16 * wave + 4 * g + i;
-                    const float w = (c < ACT && unit < C.hid) ? C.W1[(size_t)unit * D + OBS + c] : 0.f;
-                    acc = mfma16(a[i], w, acc);
-                }
-#pragma unroll
-                for (int v = 0; v < 4; v++) yp[(wave * ROWS + 4 * g + v) * D3S + c] = acc[v];
-            }
-            rlt_lds_barrier();
-            RLT_TICK(6 + 4 * k);
-            if (scalar_wave) {
-                const floatx4 out = output_tile(yp, ctiles, c, g);
-#pragma unroll
-                for (int v = 0; v < 4; v++) da[(k * ROWS + 4 * g + v) * D3S + c] = out[v];
-            }
-        }
-        if (scalar_wave) {
-            // sample_and_squash backward on the gradient of the smaller value; TD3: the td3_sampling layer's backward (zero where the sample was clamped,
-            // nn/layers/td3_sampling/operations_generic.h:139-163) and the derivative of the actor's tanh output
-            wave_sync();
-            const lptr dak = da + ((TD3 || misc[c] < misc[16 + c]) ? 0 : 1) * ROWS * D3S + c * D3S;
-#pragma unroll
-            for (int v = 0; v < 4; v++) d3[(4 * g + v) * D3S + c] = 0.f;
-            wave_sync();
-            const float alpha_over_b = alpha / (float)B;
-            float entropy = 0.f;
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const int a = g + 4 * j;
-                if (a < ACT) {
-                    if (TD3) {
-                        const float d_mean = (item[j].sample < -1.0f || item[j].sample > 1.0f) ? 0.0f : dak[a];
-                        if (row_ok) d3[c * D3S + a] = d_mean * (1.0f - item[j].mean * item[j].mean);
-                        continue;
-                    }
-                    float d_mu, d_ls;
-                    head_backward(A.sas, item[j], dak[a], alpha_over_b, d_mu, d_ls, entropy);
-                    if (row_ok) { d3[c * D3S + a] = d_mu; d3[c * D3S + ACT + a] = d_ls; }
-                }
-            }
-            entropy = groups_sum(entropy);
-            // d log_alpha: sum over the rows of alpha (entropy - target entropy), divided by the batch size by the reduction
-            const float per_row = (g == 0 && row_ok) ? alpha * (entropy - A.sas.target_entropy) : 0.f;
-            const float tile_sum = row16_sum(per_row);
-            if (lane == 0) extra += tile_sum;
-            wave_sync();
-#pragma unroll
-            for (int v = 0; v < 4; v++) s3 += d3[(4 * g + v) * D3S + c];
-        }
-        rlt_lds_barrier();      // d_pre3 is in place
-        RLT_TICK(12);
+        return;
     }
 
-    // backward pass of the trained network with its weight gradients over the workgroup's 16 rows; h1, h2: its hidden activations,
-    // d3: the gradient at its last pre-activation; ta receives d_pre2, tb receives d_pre1
-    float* dst = A.partial + ((size_t)y * G + gi) * A.count;
-    const int IN = trained.in, OUT = trained.out, NT1 = (IN + 15) >> 4;
-    const int o_b1 = HID * IN, o_w2 = o_b1 + HID, o_b2 = o_w2 + HID * HID, o_w3 = o_b2 + HID, o_b3 = o_w3 + OUT * HID, o_ex = o_b3 + OUT;
-    const lptr xt = CRITIC ? xb : xa;
-    const int n = 16 * wave + c;
-    const bool n_ok = n < HID;
-    float s2 = 0.f;
-    if (on) {
-        floatx4 aW3 = zero4;
+    // ---- actor update: the gradient of -value / batch with respect to the action (TD3: critic 0 only, rl/algorithms/td3/operations_generic.h:260)
+    const float loss_weight = (1.0f / (float)B) * -1.0f;       // rl/algorithms/sac/operations_generic.h:437-453 with n = batch rows
+    BackOperands K;
+    load_back_operands(Q, wave, c, g, K);
+    float w1[4];
 #pragma unroll
-        for (int ks = 0; ks < ROWS / 4; ks++) aW3 = mfma16(d3[(4 * ks + g) * D3S + c], h2[(4 * ks + g) * S + n], aW3);
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-            if (4 * g + v < OUT && n_ok) dst[o_w3 + (4 * g + v) * HID + n] = aW3[v];
-        s2 = backward_layer3<ACT_H>(trained, d3, h2, ta, wave, c, g);
-    }
-    rlt_lds_barrier();      // every wavefront's tile of d_pre2 is in place
-    RLT_TICK(13);
-    if (on) {
-        {   // dW2: this wavefront's units' rows
-            float a[4];
-#pragma unroll
-            for (int ks = 0; ks < 4; ks++) a[ks] = ta[(4 * ks + g) * S + n];
-#pragma unroll 4
-            for (int nt = 0; nt < tiles; nt++) {
-                floatx4 acc = zero4;
-#pragma unroll
-                for (int ks = 0; ks < 4; ks++) acc = mfma16(a[ks], h1[(4 * ks + g) * S + 16 * nt + c], acc);
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const int m = 16 * wave + 4 * g + v;
-                    if (m < HID && 16 * nt + c < HID) dst[o_w2 + (size_t)m * HID + 16 * nt + c] = acc[v];
-                }
-            }
-        }
-        RLT_TICK(14);
-        float s1 = backward_layer2<ACT_H>(trained, ta, h1, tb, wave, c, g);
-        RLT_TICK(15);
-        wave_sync();            // dW1's rows are this wavefront's own tile of d_pre1
-        {
-            float a[4];
-#pragma unroll
-            for (int ks = 0; ks < 4; ks++) a[ks] = tb[(4 * ks + g) * S + n];
-#pragma unroll 2
-            for (int nt = 0; nt < NT1; nt++) {
-                floatx4 acc = zero4;
-#pragma unroll
-                for (int ks = 0; ks < 4; ks++) acc = mfma16(a[ks], xt[(4 * ks + g) * SXS + 16 * nt + c], acc);
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const int m = 16 * wave + 4 * g + v;
-                    if (m < HID && 16 * nt + c < IN) dst[(size_t)m * IN + 16 * nt + c] = acc[v];
-                }
-            }
-        }
-        s1 = groups_sum(s1); s2 = groups_sum(s2);
-        if (g == 0 && n_ok) { dst[o_b1 + n] = s1; dst[o_b2 + n] = s2; }
-    }
+    for (int i = 0; i < 4; i++) { const int unit = 16 * wave + 4 * g + i; w1[i] = (c < ACT && unit < Q.hid) ? Q.W1[(size_t)unit * D + OBS + c] : 0.f; }
     if (scalar_wave) {
-        s3 = groups_sum(s3); extra = groups_sum(extra);
-        if (g == 0) {
-            if (c < OUT) dst[o_b3 + c] = s3;
-            dst[o_ex + c] = extra;
+        const floatx4 out = output_tile(yp, qtiles, c, g);
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            if (c == 0) misc[4 * g + v] = out[v] + q_b3;
+            d3c[(4 * g + v) * D3S + c] = (c == 0 && row0 + 4 * g + v < B) ? loss_weight : 0.f;
         }
     }
-    RLT_TICK(16);
+    rlt_lds_barrier();
+    if (wave < qtiles) backward_layer3<ACT_H>(Q, K, d3c, tb, tb, wave, c, g);
+    rlt_lds_barrier();
+    RLT_TICK(9);
+    if (wave < qtiles) {
+        backward_layer2<ACT_H>(Q, K, tb, ta, ta, wave, c, g);
+        wave_sync();
+        // d value / d action = the action columns of d_pre1 W1: this wavefront's units' share of the reduction
+        floatx4 acc = zero4;
+        const floatx4 a = *(lptr4)(ta + c * S + 16 * wave + 4 * g);
+#pragma unroll
+        for (int i = 0; i < 4; i++) acc = mfma16(a[i], w1[i], acc);
+#pragma unroll
+        for (int v = 0; v < 4; v++) yp[(wave * ROWS + 4 * g + v) * D3S + c] = acc[v];
+    }
+    rlt_lds_barrier();
+    RLT_TICK(10);
+    if (!owner) {
+        if (scalar_wave) {
+            const floatx4 out = output_tile(yp, qtiles, c, g);
+#pragma unroll
+            for (int v = 0; v < 4; v++) if (c < ACT) hand_over(exchange + ROWS + (4 * g + v) * MAX_ACT + c, out[v]);
+            if (g == 0) hand_over(exchange + c, misc[c]);
+        }
+        return;
+    }
+    const WNet trained = A.actor;
+    const Trained T = A.trained[0];
+    const int HID = trained.hid, tiles = (HID + 15) >> 4;
+    load_back_operands(trained, wave, c, g, K);
+    store_rows(h1, T.h1, HID, row0, B, wave, lane);
+    store_rows(h2, T.h2, HID, row0, B, wave, lane);
+    if (scalar_wave) {
+        // sample_and_squash backward on the gradient of the smaller value; TD3: the td3_sampling layer's backward (zero where the sample was clamped,
+        // nn/layers/td3_sampling/operations_generic.h:139-163) and the derivative of the actor's tanh output
+        const floatx4 out = output_tile(yp, qtiles, c, g);
+#pragma unroll
+        for (int v = 0; v < 4; v++) { da[(4 * g + v) * D3S + c] = out[v]; d3[(4 * g + v) * D3S + c] = 0.f; }
+        bool first = true;
+        if (!TD3) {
+            uint64_t* const mine = exchange + ROWS + c * MAX_ACT;
+            uint64_t* const word[3] = {exchange + c, mine + min(g, ACT - 1), mine + min(g + 4, ACT - 1)};
+            float value[3];
+            take_over(word, value, A.max_poll, A.fault);
+            first = misc[c] < value[0];
+#pragma unroll
+            for (int j = 0; j < 2; j++) if (g + 4 * j < ACT) da[(ROWS + c) * D3S + g + 4 * j] = value[1 + j];
+        }
+        wave_sync();
+        const lptr dak = da + (first ? 0 : 1) * ROWS * D3S + c * D3S;
+        const float alpha_over_b = alpha / (float)B;
+        float entropy = 0.f;
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int a = g + 4 * j;
+            if (a < ACT) {
+                if (TD3) {
+                    const float d_mean = (item[j].sample < -1.0f || item[j].sample > 1.0f) ? 0.0f : dak[a];
+                    if (row_ok) d3[c * D3S + a] = d_mean * (1.0f - item[j].mean * item[j].mean);
+                    continue;
+                }
+                float d_mu, d_ls;
+                head_backward(A.sas, item[j], dak[a], alpha_over_b, d_mu, d_ls, entropy);
+                if (row_ok) { d3[c * D3S + a] = d_mu; d3[c * D3S + ACT + a] = d_ls; }
+            }
+        }
+        entropy = groups_sum(entropy);
+        // d log_alpha: sum over the rows of alpha (entropy - target entropy), divided by the batch size by the optimiser
+        const float per_row = (g == 0 && row_ok) ? alpha * (entropy - A.sas.target_entropy) : 0.f;
+        const float tile_sum = row16_sum(per_row);
+        wave_sync();
+#pragma unroll
+        for (int v = 0; v < 4; v++) if (row0 + 4 * g + v < B) T.d3[(size_t)(row0 + 4 * g + v) * MAX_OUT + c] = d3[(4 * g + v) * D3S + c];
+        if (lane == 0 && A.extra) A.extra[gi] = tile_sum;
+    }
+    rlt_lds_barrier();      // d_pre3 is in place
+    RLT_TICK(11);
+    if (wave < tiles) backward_layer3<ACT_H>(trained, K, d3, h2, ta, wave, c, g);
+    rlt_lds_barrier();      // every wavefront's tile of d_pre2 is in place
+    store_rows(ta, T.d2, HID, row0, B, wave, lane);
+    if (wave < tiles) backward_layer2<ACT_H>(trained, K, ta, h1, tb, wave, c, g);
+    rlt_lds_barrier();
+    store_rows(tb, T.d1, HID, row0, B, wave, lane);
+    RLT_TICK(12);
 }
 
-constexpr size_t LDS_FLOATS = (size_t)2 * ROWS * SXS + 4 * ROWS * S + 4 * ROWS * D3S + WAVES * YP + MISC;
+constexpr size_t LDS_FLOATS = (size_t)ROWS * SXS + 4 * ROWS * S + 4 * ROWS * D3S + WAVES * YP + MISC;
 
 // ---- Forward and backward pass of one three-layer network over a few thousand rows at most, on the same machinery (nn_models/mlp/operations_generic.h:103-204: forward, the
-// loss gradient given or formed from a target as the MSE's, backward with weight gradients): a workgroup takes 16 rows through the three layers and back, the activations
-// never leave LDS, and writes one block of partial sums [dW1 | db1 | dW2 | db2 | dW3 | db3]; mlp_wide_reduce_kernel adds the blocks up in workgroup order onto the layers'
-// gradients. Where a batch is too small to fill the chip with the 64-row tiles of the one-pass kernel for large batches (mlp_fused.hip: 4,096 rows are 64 tiles for 256
+// loss gradient given or formed from a target as the MSE's, backward with weight gradients): a workgroup takes 16 rows through the three layers and back and leaves
+// activations and pre-activation gradients in memory; the weight gradients over the whole batch are the next launch (batch_gradient.hip). Where a batch is too small to fill the chip with the 64-row tiles of the one-pass kernel for large batches (mlp_fused.hip: 4,096 rows are 64 tiles for 256
 // compute units, and a tile takes its 74 us whatever the batch), sixteen-row tiles are a launch of 256 workgroups.
 struct MlpWideArgs {
     WNet net;
     const float* x; int ldx; float* y; int ldy;
     const float* d_output; int ldd; const float* target; int ldt; float mse_scale;
     int batch;
-    float* partial; int count;
+    Trained kept;                              // MLP_FORWARD_BACKWARD: hidden activations; both: the gradients at the hidden pre-activations (and, unless the caller's array serves, the last)
     const float* out1; const float* out2;      // MLP_BACKWARD: the outputs of layers 1 and 2 that a forward() left in memory, [batch x hid] each; d_output is then the gradient at the last pre-activations
     float* keep_pre[3]; float* keep_out[3]; int act3;      // MLP_FORWARD: every layer's pre-activations and outputs as forward() keeps them (each may be NULL); the last layer's activation
 };
@@ -667,32 +644,37 @@ __global__ __launch_bounds__(THREADS) void mlp_wide_kernel(MlpWideArgs A) {
     const int gi = blockIdx.x;
     const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const lptr xa = (lptr)lds_wide, h1 = xa + 2 * ROWS * SXS, h2 = h1 + ROWS * S, ta = h2 + ROWS * S, tb = ta + ROWS * S, d3 = tb + ROWS * S, yp = d3 + 4 * ROWS * D3S;
+    const lptr xa = (lptr)lds_wide, h1 = xa + ROWS * SXS, h2 = h1 + ROWS * S, ta = h2 + ROWS * S, tb = ta + ROWS * S, d3 = tb + ROWS * S, yp = d3 + 4 * ROWS * D3S;
     const WNet N = A.net;
     const int B = A.batch, IN = N.in, HID = N.hid, OUT = N.out, tiles = (HID + 15) >> 4, row0 = gi * ROWS;
     const bool on = wave < tiles;
     const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
-    for (int e = threadIdx.x; e < ROWS * SXS; e += THREADS) {
-        const int r = e / SXS, k = e % SXS;
-        xa[e] = (row0 + r < B && k < IN) ? A.x[(size_t)(row0 + r) * A.ldx + k] : 0.f;
-    }
+    const bool my_row = row0 + wave < B;
+    const size_t row_at = min(row0 + wave, B - 1);
+    Operands<NT1C> W;
+    BackOperands K;
+    float b3 = 0.f;
     if (BACKWARD_ONLY) {
         // the hidden activations come back from memory (zero beyond the batch and beyond the width, up to the multiple of 16 that the tiles run to)
-        const int HP = 16 * tiles;
-        for (int e = threadIdx.x; e < ROWS * HP; e += THREADS) {
-            const int r = e / HP, k = e - r * HP;
-            const bool ok = row0 + r < B && k < HID;
-            h1[r * S + k] = ok ? A.out1[(size_t)(row0 + r) * HID + k] : 0.f;
-            h2[r * S + k] = ok ? A.out2[(size_t)(row0 + r) * HID + k] : 0.f;
-        }
+        float v1[4], v2[4];
+        request_row(A.out1 + row_at * HID, HID, lane, v1);
+        request_row(A.out2 + row_at * HID, HID, lane, v2);
+        load_back_operands(N, wave, c, g, K);
+        place_row(h1 + wave * S, my_row, HID, 16 * tiles, lane, v1);
+        place_row(h2 + wave * S, my_row, HID, 16 * tiles, lane, v2);
+    } else {
+        float v[3];
+        request_row(A.x + row_at * A.ldx, IN, lane, v);
+        load_operands<NT1C>(N, wave, c, g, W);
+        b3 = N.b3[min(c, OUT - 1)];
+        place_row(xa + wave * SXS, my_row, IN, SXS, lane, v);
     }
     rlt_lds_barrier();
     if (PASS == MLP_FORWARD) {
         const KeepArgs keep = {{A.keep_pre[0], A.keep_pre[1]}, {A.keep_out[0], A.keep_out[1]}, row0, B};
-        forward3_own_loads<ACT_H, NT1C, true>(N, xa, SXS, h1, h2, yp, wave, c, g, &keep);
+        forward3<ACT_H, NT1C, false, true, true>(N, W, N, xa, SXS, h1, h2, yp, wave, c, g, &keep);
         if (wave == 0) {
             const floatx4 out = output_tile(yp, tiles, c, g);
-            const float b3 = c < OUT ? N.b3[c] : 0.f;
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 const int row = row0 + 4 * g + v;
@@ -707,22 +689,23 @@ __global__ __launch_bounds__(THREADS) void mlp_wide_kernel(MlpWideArgs A) {
         }
         return;
     }
-    if (PASS == MLP_FORWARD_BACKWARD) forward3_own_loads<ACT_H, NT1C>(N, xa, SXS, h1, h2, yp, wave, c, g);
-    float s3 = 0.f;
+    if (PASS == MLP_FORWARD_BACKWARD) {
+        forward3<ACT_H, NT1C, false, true>(N, W, N, xa, SXS, h1, h2, yp, wave, c, g);
+        load_back_operands(N, wave, c, g, K);
+        store_rows(h1, A.kept.h1, HID, row0, B, wave, lane);
+        store_rows(h2, A.kept.h2, HID, row0, B, wave, lane);
+    }
     if (BACKWARD_ONLY) {
         if (wave == 0) {
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 const int row = row0 + 4 * g + v;
-                const float d = (c < OUT && row < B) ? A.d_output[(size_t)row * A.ldd + c] : 0.f;
-                d3[(4 * g + v) * D3S + c] = d;
-                s3 += d;
+                d3[(4 * g + v) * D3S + c] = (c < OUT && row < B) ? A.d_output[(size_t)row * A.ldd + c] : 0.f;
             }
         }
     } else if (wave == 0) {
         // lane (c, g): output column c of rows 4 g + v; the gradient at the output (the last layer has no activation): given, or the MSE's against the target
         const floatx4 out = output_tile(yp, tiles, c, g);
-        const float b3 = c < OUT ? N.b3[c] : 0.f;
 #pragma unroll
         for (int v = 0; v < 4; v++) {
             const int row = row0 + 4 * g + v;
@@ -732,88 +715,16 @@ __global__ __launch_bounds__(THREADS) void mlp_wide_kernel(MlpWideArgs A) {
             float d = 0.f;
             if (ok) d = A.target ? (yv - A.target[(size_t)row * A.ldt + c]) * A.mse_scale : A.d_output[(size_t)row * A.ldd + c];
             d3[(4 * g + v) * D3S + c] = d;
-            s3 += d;
+            if (row < B) A.kept.d3[(size_t)row * MAX_OUT + c] = d;
         }
     }
     rlt_lds_barrier();      // d_pre3 is in place
-    // backward pass with the weight gradients over the workgroup's 16 rows: ta receives d_pre2, tb receives d_pre1
-    float* dst = A.partial + (size_t)gi * A.count;
-    const int NT1 = (IN + 15) >> 4;
-    const int o_b1 = HID * IN, o_w2 = o_b1 + HID, o_b2 = o_w2 + HID * HID, o_w3 = o_b2 + HID, o_b3 = o_w3 + OUT * HID;
-    const int n = 16 * wave + c;
-    const bool n_ok = n < HID;
-    float s2 = 0.f;
-    if (on) {
-        floatx4 aW3 = zero4;
-#pragma unroll
-        for (int ks = 0; ks < ROWS / 4; ks++) aW3 = mfma16(d3[(4 * ks + g) * D3S + c], h2[(4 * ks + g) * S + n], aW3);
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-            if (4 * g + v < OUT && n_ok) dst[o_w3 + (4 * g + v) * HID + n] = aW3[v];
-        s2 = backward_layer3<ACT_H>(N, d3, h2, ta, wave, c, g);
-    }
+    if (on) backward_layer3<ACT_H>(N, K, d3, h2, ta, wave, c, g);
     rlt_lds_barrier();      // every wavefront's tile of d_pre2 is in place
-    if (on) {
-        {   // dW2: this wavefront's units' rows
-            float a[4];
-#pragma unroll
-            for (int ks = 0; ks < 4; ks++) a[ks] = ta[(4 * ks + g) * S + n];
-#pragma unroll 4
-            for (int nt = 0; nt < tiles; nt++) {
-                floatx4 acc = zero4;
-#pragma unroll
-                for (int ks = 0; ks < 4; ks++) acc = mfma16(a[ks], h1[(4 * ks + g) * S + 16 * nt + c], acc);
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const int m = 16 * wave + 4 * g + v;
-                    if (m < HID && 16 * nt + c < HID) dst[o_w2 + (size_t)m * HID + 16 * nt + c] = acc[v];
-                }
-            }
-        }
-        float s1 = backward_layer2<ACT_H>(N, ta, h1, tb, wave, c, g);
-        wave_sync();            // dW1's rows are this wavefront's own tile of d_pre1
-        {
-            float a[4];
-#pragma unroll
-            for (int ks = 0; ks < 4; ks++) a[ks] = tb[(4 * ks + g) * S + n];
-#pragma unroll 2
-            for (int nt = 0; nt < NT1; nt++) {
-                floatx4 acc = zero4;
-#pragma unroll
-                for (int ks = 0; ks < 4; ks++) acc = mfma16(a[ks], xa[(4 * ks + g) * SXS + 16 * nt + c], acc);
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const int m = 16 * wave + 4 * g + v;
-                    if (m < HID && 16 * nt + c < IN) dst[(size_t)m * IN + 16 * nt + c] = acc[v];
-                }
-            }
-        }
-        s1 = groups_sum(s1); s2 = groups_sum(s2);
-        if (g == 0 && n_ok) { dst[o_b1 + n] = s1; dst[o_b2 + n] = s2; }
-    }
-    if (wave == 0) {
-        s3 = groups_sum(s3);
-        if (g == 0 && c < OUT) dst[o_b3 + c] = s3;
-    }
-}
-// gradient[e] += the sum over the workgroups' blocks of element e, in workgroup order; thread = one element, sixteen blocks' loads in flight
-struct WideReduceArgs { const float* partial; int blocks, count, total; float* dst[6]; int end[6]; };
-__global__ __launch_bounds__(256) void mlp_wide_reduce_kernel(WideReduceArgs R) {
-    const int e = blockIdx.x * 256 + threadIdx.x;
-    if (e >= R.total) return;
-    float sum = 0.f;
-    for (int b0 = 0; b0 < R.blocks; b0 += 16) {
-        float v[16];
-#pragma unroll
-        for (int u = 0; u < 16; u++) v[u] = b0 + u < R.blocks ? R.partial[(size_t)(b0 + u) * R.count + e] : 0.f;
-#pragma unroll
-        for (int u = 0; u < 16; u++) sum += v[u];
-    }
-    int k = 0, begin = 0;
-#pragma unroll
-    for (int q = 0; q < 5; q++) if (e >= R.end[q]) { k = q + 1; begin = R.end[q]; }
-    float* const dst = k == 0 ? R.dst[0] : k == 1 ? R.dst[1] : k == 2 ? R.dst[2] : k == 3 ? R.dst[3] : k == 4 ? R.dst[4] : R.dst[5];
-    dst[e - begin] += sum;
+    store_rows(ta, A.kept.d2, HID, row0, B, wave, lane);
+    if (on) backward_layer2<ACT_H>(N, K, ta, h1, tb, wave, c, g);
+    rlt_lds_barrier();
+    store_rows(tb, A.kept.d1, HID, row0, B, wave, lane);
 }
 
 bool hidden_ok(int a) { return a == RLT_ACT_RELU || a == RLT_ACT_TANH || a == RLT_ACT_FAST_TANH || a == RLT_ACT_SIGMOID; }
@@ -828,40 +739,15 @@ bool aligned16(const float* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) =
 WNet net_of(const rlt_dense_layer* L) {
     const int in = L[0].in_dim, hid = L[0].out_dim;
     return {L[0].weights, L[0].biases, L[1].weights, L[1].biases, L[2].weights, L[2].biases, in, hid, L[2].out_dim, L[0].activation,
-            in % 4 == 0 && aligned16(L[0].weights), hid % 4 == 0 && aligned16(L[1].weights), hid % 4 == 0 && aligned16(L[2].weights)};
+            hid % 4 == 0 && aligned16(L[2].weights)};
 }
-int partial_count(int in, int hid, int out) { return hid * in + hid + hid * hid + hid + out * hid + out + N_EXTRA; }
-
-// where each Adam tensor's gradient lies in a block of partial sums (a tensor may span several of the network's six gradient buffers
-// where those follow each other in memory); false unless the tensors cover the six buffers exactly
-bool map_gradients(const rlt_dense_layer* L, const rlt_adam_tensor* T, int n, uint32_t* offsets, int* first_segment, int* n_segments) {
-    if (!T || n < 1 || n > RLT_TAIL_TENSORS) return false;
-    const int hid = L[0].out_dim;
-    const float* seg[6] = {L[0].d_weights, L[0].d_biases, L[1].d_weights, L[1].d_biases, L[2].d_weights, L[2].d_biases};
-    const uint32_t size[6] = {(uint32_t)(hid * L[0].in_dim), (uint32_t)hid, (uint32_t)(hid * hid), (uint32_t)hid, (uint32_t)(L[2].out_dim * hid), (uint32_t)L[2].out_dim};
-    uint32_t off[6], covered = 0;
-    for (int k = 0, o = 0; k < 6; o += size[k], k++) off[k] = o;
-    for (int i = 0; i < n; i++) {
-        int s = 0;
-        while (s < 6 && seg[s] != T[i].gradient) s++;
-        if (s == 6 || T[i].polyak_target) return false;
-        uint32_t cnt = 0; int k = s;
-        for (; k < 6 && cnt < T[i].count && seg[k] == seg[s] + cnt; k++) {
-            if (covered & (1u << k)) return false;
-            covered |= 1u << k; cnt += size[k];
-        }
-        if (cnt != T[i].count) return false;
-        offsets[i] = off[s]; first_segment[i] = s; n_segments[i] = k - s;
-    }
-    return covered == 63u;
-}
-float* parameter_segments(const rlt_dense_layer* L, int first, int count) {
-    const int hid = L[0].out_dim;
-    float* seg[6] = {L[0].weights, L[0].biases, L[1].weights, L[1].biases, L[2].weights, L[2].biases};
-    const uint32_t size[6] = {(uint32_t)(hid * L[0].in_dim), (uint32_t)hid, (uint32_t)(hid * hid), (uint32_t)hid, (uint32_t)(L[2].out_dim * hid), (uint32_t)L[2].out_dim};
-    uint32_t cnt = 0;
-    for (int k = first; k < first + count; k++) { if (seg[k] != seg[first] + cnt) return nullptr; cnt += size[k]; }
-    return seg[first];
+// the network's six gradient buffers as segments [dW1, db1, dW2, db2, dW3, db3], and the parameters that they belong to
+struct Segments { float* gradient[6]; float* parameter[6]; uint32_t size[6]; };
+Segments segments_of(const rlt_dense_layer* L) {
+    const uint32_t hid = L[0].out_dim;
+    return {{L[0].d_weights, L[0].d_biases, L[1].d_weights, L[1].d_biases, L[2].d_weights, L[2].d_biases},
+            {L[0].weights, L[0].biases, L[1].weights, L[1].biases, L[2].weights, L[2].biases},
+            {hid * L[0].in_dim, hid, hid * hid, hid, L[2].out_dim * hid, (uint32_t)L[2].out_dim}};
 }
 
 struct Optimiser {
@@ -870,75 +756,91 @@ struct Optimiser {
     const rlt_dense_layer* soft_target;
 };
 
-// The optimisers' steps, as one launch after the update kernel that adds up the workgroups' blocks itself (16 blocks of 68 k floats at
-// width 256: read through one compute unit each, as the update kernel's own last step, that costs 70 us; spread over the chip 10): both
-// critics' optimisers share it, and a tensor's soft update of its target rides along where the layouts correspond.
-struct Step { rlt_adam_tensor tensors[RLT_TAIL_TENSORS]; uint32_t offsets[RLT_TAIL_TENSORS]; float scales[RLT_TAIL_TENSORS]; bool targets_fused; };
-bool describe_step(const Optimiser& O, Step& S) {
-    int first[RLT_TAIL_TENSORS], count[RLT_TAIL_TENSORS];
-    if (!map_gradients(O.trained, O.tensors, O.n_tensors, S.offsets, first, count)) return false;
-    S.targets_fused = O.soft_target != nullptr;
+// What the gradients' launch needs of a trained network and its optimiser. A tensor of the optimiser may span several segments where those follow each other in memory;
+// false unless the tensors cover the six segments exactly. The soft update of the target rides along where the tensors' parameters are the network's own.
+bool describe(const Optimiser& O, rlt_gradient_net& N, bool* targets_fused) {
+    const Segments s = segments_of(O.trained);
+    if (!O.tensors || O.n_tensors < 1 || O.n_tensors > RLT_TAIL_TENSORS) return false;
+    const Segments soft = O.soft_target ? segments_of(O.soft_target) : Segments{};
+    uint32_t covered = 0;
+    *targets_fused = O.soft_target != nullptr;
     for (int i = 0; i < O.n_tensors; i++) {
-        S.tensors[i] = O.tensors[i]; S.scales[i] = 1.0f;
-        if (O.soft_target && (parameter_segments(O.trained, first[i], count[i]) != O.tensors[i].parameters || !(S.tensors[i].polyak_target = parameter_segments(O.soft_target, first[i], count[i])))) S.targets_fused = false;
+        const rlt_adam_tensor& T = O.tensors[i];
+        if (T.polyak_target || !T.parameters || !T.gradient || !T.first_moment || !T.second_moment) return false;
+        int k = 0;
+        while (k < 6 && s.gradient[k] != T.gradient) k++;
+        uint32_t at = 0;
+        for (; k < 6 && at < T.count && s.gradient[k] == T.gradient + at; k++) {
+            if (covered & (1u << k)) return false;
+            covered |= 1u << k;
+            N.gradient[k] = s.gradient[k]; N.parameter[k] = T.parameters + at; N.first_moment[k] = T.first_moment + at; N.second_moment[k] = T.second_moment + at; N.flags[k] = T.flags;
+            N.target[k] = soft.parameter[k];
+            if (N.parameter[k] != s.parameter[k]) *targets_fused = false;
+            at += s.size[k];
+        }
+        if (at != T.count) return false;
     }
-    if (!S.targets_fused) for (int i = 0; i < O.n_tensors; i++) S.tensors[i].polyak_target = nullptr;
-    return true;
+    N.in = O.trained[0].in_dim; N.hid = O.trained[0].out_dim; N.out = O.trained[2].out_dim;
+    N.step = 1; N.adam = *O.parameters;
+    return covered == 63u;
 }
-
-// false: the agent's Adam tensors are not its networks' gradient buffers; the caller takes the per-operation path
-bool steps_describable(const Optimiser* opts, int n_opts) {
-    Step S;
-    for (int k = 0; k < n_opts; k++) {
-        if (!describe_step(opts[k], S)) return false;
-        if (opts[k].second && (opts[k].second->polyak_target || !opts[k].second->parameters || !opts[k].second->gradient || !opts[k].second->first_moment || !opts[k].second->second_moment)) return false;
-    }
-    return true;
+// room for a batch's activations and gradients of a trained network; floats
+size_t trained_floats(int hid, int batch) { return (((size_t)hid * batch * 4 + (size_t)MAX_OUT * batch) + 63) & ~(size_t)63; }
+Trained place_trained(float* base, int hid, int batch) {
+    const size_t n = (size_t)hid * batch;
+    return {base, base + n, base + 2 * n, base + 3 * n, base + 4 * n};
 }
+void set_rows(rlt_gradient_net& N, const Trained& T, const float* x, int ldx) { N.x = x; N.ldx = ldx; N.h1 = T.h1; N.h2 = T.h2; N.d1 = T.d1; N.d2 = T.d2; N.d3 = T.d3; N.ld3 = MAX_OUT; }
 
 template <int MODE>
 int launch_wide(rlt_rocm_device* device, WideArgs& a, int groups, const Optimiser* opts, int n_opts, float polyak, bool* targets_done) {
-    const rlt_dense_layer* trained = opts[0].trained;
-    if (!steps_describable(opts, n_opts)) return RLT_E_UNSUPPORTED;
-    const int exact_count = partial_count(trained[0].in_dim, trained[0].out_dim, trained[2].out_dim);
-    a.count = (exact_count + 63) & ~63;      // blocks start on 256-byte boundaries: the optimisers' launch reads them 16 bytes per lane
-    // the copies of the second layers' weights: forward copies of every network that runs forward, backward copies of those whose second layer is also walked backwards
-    WNet* forward_nets[5]; WNet* backward_nets[3];
-    int n_forward = 0, n_backward = 0;
-    forward_nets[n_forward++] = &a.actor;
-    for (int k = 0; k < 2; k++) forward_nets[n_forward++] = &a.critic[k];
+    rlt_gradient_net net[2] = {};
+    bool fused[2] = {false, false};
+    for (int k = 0; k < n_opts; k++) {      // the agent's Adam tensors are not its networks' gradient buffers: the caller takes the per-operation path
+        if (!describe(opts[k], net[k], &fused[k])) return RLT_E_UNSUPPORTED;
+        if (opts[k].second && (opts[k].second->polyak_target || !opts[k].second->parameters || !opts[k].second->gradient || !opts[k].second->first_moment || !opts[k].second->second_moment)) return RLT_E_UNSUPPORTED;
+    }
+    const bool fuse_targets = targets_done && n_opts == 2 && fused[0] && fused[1];
+    if (targets_done) *targets_done = fuse_targets;
+    if (!fuse_targets) for (int k = 0; k < n_opts; k++) for (int q = 0; q < 6; q++) net[k].target[q] = nullptr;
     constexpr bool CRITIC_UPDATE = MODE == MODE_CRITIC || MODE == MODE_TD3_CRITIC;
-    if (CRITIC_UPDATE) for (int k = 0; k < 2; k++) forward_nets[n_forward++] = &a.target[k];
-    for (int k = 0; k < 2; k++) backward_nets[n_backward++] = &a.critic[k];
-    if (!CRITIC_UPDATE) backward_nets[n_backward++] = &a.actor;
-    const size_t copy_floats = (size_t)256 * WAVES * WAVES;      // [16 wavefronts][16 chunks][64 lanes][4] at width 256
-    const size_t partial_bytes = ((size_t)n_opts * groups * a.count * sizeof(float) + 255) & ~(size_t)255;
+    const size_t copies_floats = 5 * (MAX_COPY_FLOATS + MAX_W1_COPY_FLOATS) + 3 * MAX_COPY_FLOATS;
+    const size_t trained_each = trained_floats(net[0].hid, a.batch), exchange_words = (size_t)groups * EXCHANGE, extra_floats = (size_t)(groups + 63) & ~(size_t)63,
+                 partial_floats = (rlt_batch_gradients_partial_floats(net, n_opts, a.batch) + 63) & ~(size_t)63;
     void* scratch = nullptr;
-    int rc = rlt_scratch(device, partial_bytes + (size_t)PREP_JOBS * copy_floats * sizeof(float), &scratch);
+    int rc = rlt_scratch(device, (copies_floats + n_opts * trained_each + extra_floats + partial_floats) * sizeof(float) + exchange_words * sizeof(uint64_t) + 256, &scratch);
     if (rc) return rc;
-    a.partial = (float*)scratch;
-    {
-        PrepArgs P = {};
-        float* copies = (float*)((char*)scratch + partial_bytes);
-        int jobs = 0, max_tiles = 1;
-        auto job = [&](WNet* net, bool backward) {
-            for (int q = 0; q < jobs; q++)      // networks given twice (one critic trained alone) share a copy
-                if (P.W2[q] == net->W2 && P.backward[q] == (backward ? 1 : 0)) { (backward ? net->W2b : net->W2f) = P.dst[q]; return; }
-            P.W2[jobs] = net->W2; P.dst[jobs] = copies + (size_t)jobs * copy_floats; P.hid[jobs] = net->hid; P.backward[jobs] = backward ? 1 : 0;
-            (backward ? net->W2b : net->W2f) = P.dst[jobs];
-            const int tiles = (net->hid + 15) >> 4;
-            if (tiles > max_tiles) max_tiles = tiles;
-            jobs++;
-        };
-        for (int q = 0; q < n_forward; q++) job(forward_nets[q], false);
-        for (int q = 0; q < n_backward; q++) job(backward_nets[q], true);
-        hipLaunchKernelGGL(wide_prepare_kernel, dim3(rlt_div_up(max_tiles * max_tiles * 64, 256), jobs), dim3(256), 0, device->stream, P);
-        if ((rc = rlt_launch_status(device))) return rc;
+    float* const rows = (float*)scratch + copies_floats; float* const extra = rows + n_opts * trained_each;
+    for (int k = 0; k < n_opts; k++) {
+        a.trained[k] = place_trained(rows + k * trained_each, net[k].hid, a.batch);
+        set_rows(net[k], a.trained[k], a.batch_base, a.obs + a.act);
+    }
+    a.extra = opts[0].second ? extra : nullptr;
+    float* const partial = extra + extra_floats;
+    a.exchange = (uint64_t*)(partial + partial_floats);
+    uint32_t* const age_before = (uint32_t*)(a.exchange + exchange_words);
+    for (int k = 0; k < n_opts; k++) net[k].age = age_before + k;
+    a.max_poll = device->wait_limit; a.fault = device->fault;
+    device->fault_armed = 1;
+    {   // every network runs forward; the critics (their targets' own weights are another matter) and in the actor update the actor are also walked backwards
+        Copies copies((float*)scratch);
+        copies.forward(a.actor);
+        for (int k = 0; k < 2; k++) { copies.forward(a.critic[k]); copies.backward(a.critic[k]); if (CRITIC_UPDATE) copies.forward(a.target[k]); }
+        if (!CRITIC_UPDATE) copies.backward(a.actor);
+        copies.args.clear = a.exchange; copies.args.n_clear = (int)exchange_words;
+        for (int k = 0; k < n_opts; k++) copies.args.age[k] = opts[k].age;
+        copies.args.age[2] = opts[0].second ? opts[0].second_age : nullptr; copies.args.age_before = age_before;
+        if ((rc = copies.launch(device))) return rc;
     }
     a.stream_offset = device->stream_offset;
-    a.packed = device->update_one_xcd && device->xcd_stride == 8 && n_opts * groups <= 32 ? 1 : 0;
+    a.groups = groups; a.n_critics = n_opts;
+    a.roles = MODE == MODE_CRITIC ? 2 + n_opts : MODE == MODE_TD3_CRITIC ? 3 * n_opts : MODE == MODE_ACTOR ? 2 : 1;
+    // A workgroup waits for others of its tile only, and all are resident where there is a compute unit for each: then a role's workgroups are kept on neighbouring
+    // positions of the XCDs' round (workgroup b runs on XCD b % 8), so that few XCDs read a network's weights. Larger grids are numbered role by role, so that whoever
+    // is waited for was dispatched before whoever waits.
+    a.by_xcd = device->update_one_xcd && device->xcd_stride == 8 && a.roles * groups <= device->compute_units;
     const size_t lds_bytes = LDS_FLOATS * sizeof(float);
-    const dim3 grid(a.packed ? 8 * groups : groups, n_opts);
+    const dim3 grid(a.by_xcd ? 8 * rlt_div_up(a.roles * groups, 8) : a.roles * groups);
 #define RLT_LAUNCH_WIDE(ACT, NT)                                                                                                                          \
     do {                                                                                                                                                  \
         RLT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(sac_wide_kernel<MODE, ACT, NT>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes)); \
@@ -946,30 +848,17 @@ int launch_wide(rlt_rocm_device* device, WideArgs& a, int groups, const Optimise
     } while (0)
     int act = a.actor.act_h;
     for (int k = 0; k < 2; k++) if (a.critic[k].act_h != act || a.target[k].act_h != act) act = -1;
-    // first layers of at most 32 inputs (two 16-deep chunks) leave registers for all of a pass's weights at once
-    if (a.obs + a.act <= 32) {
-        if (act == RLT_ACT_RELU) RLT_LAUNCH_WIDE(RLT_ACT_RELU, 2); else if (act == RLT_ACT_FAST_TANH) RLT_LAUNCH_WIDE(RLT_ACT_FAST_TANH, 2); else RLT_LAUNCH_WIDE(-1, 2);
-    } else {
-        if (act == RLT_ACT_RELU) RLT_LAUNCH_WIDE(RLT_ACT_RELU, MAX_D / 16); else if (act == RLT_ACT_FAST_TANH) RLT_LAUNCH_WIDE(RLT_ACT_FAST_TANH, MAX_D / 16); else RLT_LAUNCH_WIDE(-1, MAX_D / 16);
-    }
+#define RLT_LAUNCH_WIDE_ACT(NT) do { if (act == RLT_ACT_RELU) RLT_LAUNCH_WIDE(RLT_ACT_RELU, NT); else if (act == RLT_ACT_FAST_TANH) RLT_LAUNCH_WIDE(RLT_ACT_FAST_TANH, NT); else RLT_LAUNCH_WIDE(-1, NT); } while (0)
+    // the first layer's chunks that the code is unrolled for: up to 64 inputs they leave registers for all of a pass's weights at once
+    if (a.obs + a.act <= 32) RLT_LAUNCH_WIDE_ACT(2); else if (a.obs + a.act <= 64) RLT_LAUNCH_WIDE_ACT(4); else RLT_LAUNCH_WIDE_ACT(MAX_D / 16);
+#undef RLT_LAUNCH_WIDE_ACT
 #undef RLT_LAUNCH_WIDE
     if ((rc = rlt_launch_status(device))) return rc;
-    Step S[2];
-    rlt_adam_source source[2];
-    for (int k = 0; k < n_opts; k++) {
-        describe_step(opts[k], S[k]);
-        source[k] = {a.partial + (size_t)k * groups * a.count, groups, a.count, S[k].offsets, S[k].scales};
-    }
-    if (targets_done) *targets_done = n_opts == 2 && S[0].targets_fused && S[1].targets_fused;
-    if (targets_done && !*targets_done) for (int k = 0; k < n_opts; k++) for (int i = 0; i < opts[k].n_tensors; i++) S[k].tensors[i].polyak_target = nullptr;
-    if (n_opts == 2)
-        return rlt_adam_step_pair(device, S[0].tensors, opts[0].n_tensors, opts[0].parameters, opts[0].age, S[1].tensors, opts[1].n_tensors, opts[1].parameters, opts[1].age, &source[0], &source[1], polyak);
     if (opts[0].second) {
-        const uint32_t second_offset = (uint32_t)(exact_count - N_EXTRA);
-        const rlt_adam_source second_source = {a.partial, groups, a.count, &second_offset, &opts[0].second_scale};
-        return rlt_adam_step_pair(device, S[0].tensors, opts[0].n_tensors, opts[0].parameters, opts[0].age, opts[0].second, 1, opts[0].second_parameters, opts[0].second_age, &source[0], &second_source);
+        const rlt_gradient_scalar scalar = {a.extra, groups, opts[0].second_scale, *opts[0].second, *opts[0].second_parameters, age_before + 2};
+        return rlt_batch_gradients(device, net, n_opts, a.batch, polyak, &scalar, partial);
     }
-    return rlt_adam_step_from_partials(device, S[0].tensors, opts[0].n_tensors, opts[0].parameters, opts[0].age, &source[0]);
+    return rlt_batch_gradients(device, net, n_opts, a.batch, polyak, nullptr, partial);
 }
 
 void set_noise(WideArgs& a, const rlt_update_noise& N) { a.noise = N.values; a.noise_seed = N.seed; a.noise_stream = N.stream; a.out_noise = N.values ? nullptr : N.drawn; }
@@ -1113,35 +1002,30 @@ static int mlp_wide_launch(rlt_rocm_device* device, const rlt_dense_layer* L, in
     if (forward_only) for (int l = 0; l < 3; l++) { a.keep_pre[l] = L[l].pre_activations; a.keep_out[l] = L[l].output; }
     a.act3 = L[2].activation;
     const int IN = L[0].in_dim, OUT = L[2].out_dim, groups = rlt_div_up(batch, ROWS);
-    const int exact = hid * IN + hid + hid * hid + hid + OUT * hid + OUT;
-    a.count = (exact + 63) & ~63;
-    const size_t copy_floats = (size_t)256 * WAVES * WAVES;
-    const size_t partial_bytes = forward_only ? 0 : ((size_t)groups * a.count * sizeof(float) + 255) & ~(size_t)255;
-    void* scratch = nullptr;
     int rc = 0;
+    rlt_gradient_net net = {};
+    net.in = IN; net.hid = hid; net.out = OUT;
+    float* partial = nullptr;
     if (!forward_only) {
-        if ((rc = rlt_scratch(device, partial_bytes, &scratch))) return rc;
-        a.partial = (float*)scratch;
+        void* scratch = nullptr;
+        if ((rc = rlt_scratch(device, (trained_floats(hid, batch) + rlt_batch_gradients_partial_floats(&net, 1, batch)) * sizeof(float), &scratch))) return rc;
+        a.kept = place_trained((float*)scratch, hid, batch);
+        partial = (float*)scratch + trained_floats(hid, batch);
+        set_rows(net, a.kept, x, ldx);
     }
     // the weight copies have a buffer of their own: forward() and evaluate() have never touched the handle's scratch buffer at these batch sizes, and callers hold data there across them
-    if (device->copy_scratch_bytes < 2 * copy_floats * sizeof(float)) {
+    constexpr size_t COPY_BYTES = (2 * MAX_COPY_FLOATS + MAX_W1_COPY_FLOATS) * sizeof(float);
+    if (device->copy_scratch_bytes < COPY_BYTES) {
         if (device->capturing) return RLT_E_CAPTURING;
         if (device->copy_scratch) RLT_HIP(hipFree(device->copy_scratch));
         device->copy_scratch = nullptr; device->copy_scratch_bytes = 0;
-        RLT_HIP(hipMalloc(&device->copy_scratch, 2 * copy_floats * sizeof(float)));
-        device->copy_scratch_bytes = 2 * copy_floats * sizeof(float);
+        RLT_HIP(hipMalloc(&device->copy_scratch, COPY_BYTES));
+        device->copy_scratch_bytes = COPY_BYTES;
     }
-    {
-        // the second layer's weights in the order the wavefronts consume them: the copy for d_pre2 W2, and for the forward pass the one for h1 W2^T
-        PrepArgs P = {};
-        float* copies = (float*)device->copy_scratch;
-        const int jobs = pass == MLP_FORWARD_BACKWARD ? 2 : 1;
-        for (int q = 0; q < jobs; q++) { P.W2[q] = a.net.W2; P.dst[q] = copies + (size_t)q * copy_floats; P.hid[q] = hid; P.backward[q] = (q == 0 && !forward_only) ? 1 : 0; }
-        a.net.W2b = forward_only ? nullptr : P.dst[0]; a.net.W2f = forward_only ? P.dst[0] : (backward_only ? nullptr : P.dst[1]);
-        const int tiles = (hid + 15) >> 4;
-        hipLaunchKernelGGL(wide_prepare_kernel, dim3(rlt_div_up(tiles * tiles * 64, 256), jobs), dim3(256), 0, device->stream, P);
-        if ((rc = rlt_launch_status(device))) return rc;
-    }
+    Copies copies((float*)device->copy_scratch);
+    if (!backward_only) copies.forward(a.net);
+    if (!forward_only) copies.backward(a.net);
+    if ((rc = copies.launch(device))) return rc;
     const size_t lds_bytes = LDS_FLOATS * sizeof(float);
 #define RLT_LAUNCH_MLP_WIDE(ACT, NT, BWD)                                                                                                                   \
     do {                                                                                                                                                    \
@@ -1152,6 +1036,7 @@ static int mlp_wide_launch(rlt_rocm_device* device, const rlt_dense_layer* L, in
 #define RLT_LAUNCH_MLP_WIDE_PASS(P)                                                                                                       \
     do {                                                                                                                                  \
         if (IN <= 32) { if (relu) RLT_LAUNCH_MLP_WIDE(RLT_ACT_RELU, 2, P); else RLT_LAUNCH_MLP_WIDE(-1, 2, P); }                          \
+        else if (IN <= 64) { if (relu) RLT_LAUNCH_MLP_WIDE(RLT_ACT_RELU, 4, P); else RLT_LAUNCH_MLP_WIDE(-1, 4, P); }                     \
         else { if (relu) RLT_LAUNCH_MLP_WIDE(RLT_ACT_RELU, MAX_D / 16, P); else RLT_LAUNCH_MLP_WIDE(-1, MAX_D / 16, P); }                  \
     } while (0)
     if (backward_only) RLT_LAUNCH_MLP_WIDE_PASS(MLP_BACKWARD); else if (forward_only) RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD); else RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD_BACKWARD);
@@ -1159,13 +1044,10 @@ static int mlp_wide_launch(rlt_rocm_device* device, const rlt_dense_layer* L, in
 #undef RLT_LAUNCH_MLP_WIDE
     if ((rc = rlt_launch_status(device))) return rc;
     if (forward_only) return 0;
-    WideReduceArgs R = {};
-    R.partial = a.partial; R.blocks = groups; R.count = a.count; R.total = exact;
-    float* const dst[6] = {L[0].d_weights, L[0].d_biases, L[1].d_weights, L[1].d_biases, L[2].d_weights, L[2].d_biases};
-    const int size[6] = {hid * IN, hid, hid * hid, hid, OUT * hid, OUT};
-    for (int k = 0, end = 0; k < 6; k++) { end += size[k]; R.dst[k] = dst[k]; R.end[k] = end; }
-    hipLaunchKernelGGL(mlp_wide_reduce_kernel, dim3(rlt_div_up(exact, 256)), dim3(256), 0, device->stream, R);
-    return rlt_launch_status(device);
+    const Segments seg = segments_of(L);
+    for (int k = 0; k < 6; k++) net.gradient[k] = seg.gradient[k];
+    if (backward_only) { net.h1 = L[0].output; net.h2 = L[1].output; net.d3 = d_output; net.ld3 = ldd; }
+    return rlt_batch_gradients(device, &net, 1, batch, 0.0f, nullptr, partial);
 }
 int rlt_mlp_wide_forward_backward(rlt_rocm_device* device, const rlt_dense_layer* L, int n_layers, const float* x, int ldx, float* y, int ldy,
                                   const float* d_output, int ldd, const float* target, int ldt, float mse_scale, int batch) {

@@ -1,5 +1,5 @@
 """Parity of the forward + backward call on sixteen-row tiles (three-layer networks of hidden width up to 256 over at most 4,096 rows: mlp_wide_kernel, a workgroup of
-sixteen wavefronts per tile, the workgroups' partial gradient sums added up by a second launch) with the CPU checker and with the library's other paths for the same
+sixteen wavefronts per tile, the weight gradients over the whole batch by a second launch) with the CPU checker and with the library's other paths for the same
 call (RLT_MLP_WIDE=0), through the C ABI.
 
 fp32 tolerance: 1e-5 relative to the largest magnitude of the tensor compared (the contraction order differs from the checker's)."""
@@ -37,6 +37,9 @@ CASES = [
     (300, 35, 256, 1, "relu", True),         # a critic of the Ant's width (27 + 8 inputs): the first layer in more than two chunks
     (100, 128, 200, 16, "fast_tanh", False), # the widest input and output, a hidden width that is no multiple of 16
     (2048, 1, 16, 2, "sigmoid", False),      # the narrowest
+    (512, 64, 33, 6, "tanh", False),         # the most rows that one workgroup of the gradients' launch takes; two columns of the second tile of 32
+    (513, 65, 256, 2, "tanh", True),         # ... and one more: two groups of workgroups share the batch; the first layer in five chunks
+    (2051, 17, 250, 3, "tanh", False),       # eight groups
 ]
 
 

@@ -138,6 +138,13 @@ def test_wider_agents_match_the_checker_on_both_paths(oracle, rocm, batch, obs, 
     assert moved.max() > 1e-4 and results["one_launch"]["ages"].tolist() == [1 + steps] * 4
 
 
+# the batch shared out to two, four and four groups of workgroups by the gradients' launch (beyond 512, 1,024 rows); 4 x 128 workgroups of the update kernel, more than compute units
+@pytest.mark.parametrize("batch,hidden", [(513, 256), (1025, 40), (2048, 72)])
+def test_wider_agents_at_large_batches(oracle, rocm, batch, hidden):
+    test_wider_agents_match_the_checker_on_both_paths(oracle, rocm, batch, 9, 2, hidden, "tanh")
+
+
+
 def test_agents_outside_the_fused_shapes_take_the_per_operation_path(oracle, rocm):
     """an agent with sequence masks: same entry points, same results as the checker"""
     batch, obs, act = 64, 3, 1

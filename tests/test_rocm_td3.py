@@ -167,6 +167,12 @@ def test_wider_agents_match_the_checker_on_both_paths(oracle, rocm, batch, obs, 
     fused_against_checker_and_per_operation(oracle, rocm, batch, obs, act, hidden_act, hidden)
 
 
+# the batch shared out by the gradients' launch (beyond 512 rows); 6 x 128 workgroups of the update kernel for both critics, more than compute units
+@pytest.mark.parametrize("batch,hidden", [(513, 256), (2048, 40)])
+def test_wider_agents_at_large_batches(oracle, rocm, batch, hidden):
+    fused_against_checker_and_per_operation(oracle, rocm, batch, 9, 2, "tanh", hidden)
+
+
 def fused_against_checker_and_per_operation(oracle, rocm, batch, obs, act, hidden_act, hidden):
     rng = np.random.default_rng(batch * 7 + obs)
     D = obs + act
