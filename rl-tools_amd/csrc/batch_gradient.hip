@@ -12,17 +12,16 @@
 // then the loads of the operands from L2: each row of a network is read by its 8 to 16 column tiles.
 #include "batch_gradient.h"
 #include "optim.h"
+#include "batch_tile.h"
 
 namespace {
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-constexpr int WAVES = 4, THREADS = 64 * WAVES, TN = 32, CHUNK = 8, SPLIT_ROWS = 512, MAX_SPLITS = 8;      // tile of a gradient; steps of four rows whose operands are requested together
+using namespace rlt_batch;
+constexpr int WAVES = 4, THREADS = 64 * WAVES, SPLIT_ROWS = 512, MAX_SPLITS = 8;
 struct GradientLaunch {
     rlt_gradient_net net[2]; int blocks0, batch, splits, total0, total; float polyak;      // total0, total: gradient elements of the first network, of both
     rlt_gradient_scalar scalar; int has_scalar;
     float* partial;      // splits > 1: [splits][total] sums, the networks' elements one after the other, segments in order
 };
-
-__device__ __forceinline__ float groups_sum(float v) { asm volatile("" : "+v"(v)); v += __shfl_xor(v, 16, 64); v += __shfl_xor(v, 32, 64); return v; }
 
 __host__ __device__ inline int segment_size(const rlt_gradient_net& N, int k) { return k == 0 ? N.hid * N.in : k == 2 ? N.hid * N.hid : k == 4 ? N.out * N.hid : k == 5 ? N.out : N.hid; }
 
@@ -60,9 +59,8 @@ __device__ __forceinline__ void finish_scalar(const rlt_gradient_scalar& Z, int 
 // eight times the workgroups (four loads for four matrix instructions instead of three for two)
 template <bool SPLIT>
 __global__ __launch_bounds__(THREADS) void batch_gradient_kernel(GradientLaunch K) {
-    constexpr int TM = SPLIT ? 32 : 16, MT_TILES = TM / 16, PER_THREAD = TM * TN / THREADS;
-    __shared__ float part[WAVES][TM][TN + 1];
-    __shared__ float part_bias[WAVES][TM];
+    constexpr int TM = SPLIT ? 32 : 16, PER_THREAD = TM * TN / THREADS;
+    __shared__ Parts<WAVES, TM / 16> P;
     const int split = SPLIT ? blockIdx.x % K.splits : 0, block = SPLIT ? blockIdx.x / K.splits : blockIdx.x;      // splits divide 8: a split's workgroups lie on 8 / splits XCDs
     const int y = block >= K.blocks0 ? 1 : 0;
     const rlt_gradient_net& N = y ? K.net[1] : K.net[0];
@@ -75,28 +73,9 @@ __global__ __launch_bounds__(THREADS) void batch_gradient_kernel(GradientLaunch 
     else if ((t -= MT * N2) < MT * N1) { segment = 0; tiles = N1; a = N.d1; lda = N.hid; rows = N.hid; b = N.x; ldb = N.ldx; cols = N.in; }
     else { t -= MT * N1; segment = 4; tiles = N2; a = N.d3; lda = N.ld3; rows = N.out; b = N.h2; ldb = N.hid; cols = N.hid; }
     const int mt = t / tiles, nt = t - mt * tiles;
-    const int n0 = TN * nt + r, n1 = n0 + 16;
-    const bool n0_ok = n0 < cols, n1_ok = n1 < cols;
-    const float* pa[MT_TILES]; bool m_ok[MT_TILES];
-#pragma unroll
-    for (int q = 0; q < MT_TILES; q++) { const int m = TM * mt + 16 * q + r; m_ok[q] = m < rows; pa[q] = a + (m_ok[q] ? m : 0); }
-    const float* pb0 = b + (n0_ok ? n0 : 0); const float* pb1 = b + (n1_ok ? n1 : 0);
     // this wavefront's rows of the batch
     const int shares = SPLIT ? WAVES * K.splits : WAVES, per = ((B + shares - 1) / shares + 3) & ~3, k0 = (WAVES * split + wave) * per, k1 = min(B, k0 + per);
-    float va[MT_TILES][CHUNK], v0[CHUNK], v1[CHUNK];
-    auto request = [&](int kb) {
-#pragma unroll
-        for (int s = 0; s < CHUNK; s++) {
-            const int k = kb + 4 * s + g, kc = min(k, B - 1);
-#pragma unroll
-            for (int q = 0; q < MT_TILES; q++) { va[q][s] = pa[q][(size_t)kc * lda]; if (k >= k1 || !m_ok[q]) va[q][s] = 0.f; }
-            v0[s] = pb0[(size_t)kc * ldb]; v1[s] = pb1[(size_t)kc * ldb];
-            if (!n0_ok) v0[s] = 0.f;
-            if (!n1_ok) v1[s] = 0.f;
-        }
-    };
-    if (k0 < k1) request(k0);
-    // what the step needs of this thread's elements travels with the operands
+    // what the step needs of this thread's elements travels before the operands
     Held held[PER_THREAD];
     float bc1 = 0.f, bc2 = 0.f;
     if (!SPLIT) {
@@ -107,35 +86,10 @@ __global__ __launch_bounds__(THREADS) void batch_gradient_kernel(GradientLaunch 
         }
         if (N.step) rlt_adam_bias_corrections(N.adam, *N.age, bc1, bc2);
     }
-    floatx4 c0[MT_TILES], c1[MT_TILES];
-    float bias[MT_TILES];
-#pragma unroll
-    for (int q = 0; q < MT_TILES; q++) { c0[q] = c1[q] = floatx4{0.f, 0.f, 0.f, 0.f}; bias[q] = 0.f; }
-    for (int kb = k0; kb < k1; kb += 4 * CHUNK) {
-        float xa[MT_TILES][CHUNK], x0[CHUNK], x1[CHUNK];
-#pragma unroll
-        for (int s = 0; s < CHUNK; s++) {
-            x0[s] = v0[s]; x1[s] = v1[s];
-#pragma unroll
-            for (int q = 0; q < MT_TILES; q++) xa[q][s] = va[q][s];
-        }
-        if (kb + 4 * CHUNK < k1) request(kb + 4 * CHUNK);
-#pragma unroll
-        for (int s = 0; s < CHUNK; s++)
-#pragma unroll
-            for (int q = 0; q < MT_TILES; q++) {
-                c0[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[q][s], x0[s], c0[q], 0, 0, 0);
-                c1[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[q][s], x1[s], c1[q], 0, 0, 0);
-                bias[q] += xa[q][s];
-            }
-    }
-#pragma unroll
-    for (int q = 0; q < MT_TILES; q++) {
-#pragma unroll
-        for (int v = 0; v < 4; v++) { part[wave][16 * q + 4 * g + v][r] = c0[q][v]; part[wave][16 * q + 4 * g + v][16 + r] = c1[q][v]; }
-        bias[q] = groups_sum(bias[q]);
-        if (g == 0) part_bias[wave][16 * q + r] = bias[q];
-    }
+    floatx4 c[TM / 16][2];
+    float bias[TM / 16];
+    tile_product<TM / 16>(a, lda, rows, TM * mt, b, ldb, cols, TN * nt, B, k0, k1, r, g, c, bias);
+    place_parts(P, wave, r, g, c, bias);
     rlt_lds_barrier();
     size_t first = SPLIT ? (size_t)split * K.total + (y ? K.total0 : 0) : 0;      // where this segment's sums of this split lie
     if (SPLIT) for (int k = 0; k < segment; k++) first += segment_size(N, k);
@@ -143,7 +97,7 @@ __global__ __launch_bounds__(THREADS) void batch_gradient_kernel(GradientLaunch 
     for (int u = 0; u < PER_THREAD; u++) {
         const int e = threadIdx.x + u * THREADS, em = e / TN, en = e % TN;
         if (TM * mt + em < rows && TN * nt + en < cols) {
-            const float sum = (part[0][em][en] + part[1][em][en]) + (part[2][em][en] + part[3][em][en]);
+            const float sum = (P.tile[0][em][en] + P.tile[1][em][en]) + (P.tile[2][em][en] + P.tile[3][em][en]);
             const size_t at = (size_t)(TM * mt + em) * cols + TN * nt + en;
             if (SPLIT) K.partial[first + at] = sum;
             else finish(N, segment, at, sum, held[u], bc1, bc2, K.polyak);
@@ -152,7 +106,7 @@ __global__ __launch_bounds__(THREADS) void batch_gradient_kernel(GradientLaunch 
     // the layer's bias gradient: column sums of the left operand, by the workgroups of the first column tile
     if (nt == 0 && threadIdx.x < TM && TM * mt + (int)threadIdx.x < rows) {
         const int at = TM * mt + threadIdx.x;
-        const float sum = (part_bias[0][threadIdx.x] + part_bias[1][threadIdx.x]) + (part_bias[2][threadIdx.x] + part_bias[3][threadIdx.x]);
+        const float sum = (P.bias[0][threadIdx.x] + P.bias[1][threadIdx.x]) + (P.bias[2][threadIdx.x] + P.bias[3][threadIdx.x]);
         if (SPLIT) K.partial[first + (size_t)rows * cols + at] = sum;
         else finish(N, segment + 1, at, sum, hold(N, segment + 1, at), bc1, bc2, K.polyak);
     }

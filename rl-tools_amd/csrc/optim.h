@@ -9,11 +9,11 @@
 // extra_out (optional): one more sum of the blocks, at extra_offset, times extra_scale, stored there (a loss that the kernel summed per block).
 struct rlt_adam_source { const float* partial; int groups, block_stride; const uint32_t* offsets; const float* scales; const float* adds; float* extra_out; uint32_t extra_offset; float extra_scale; };
 
-// rlt_rocm_adam_step for at most 12 tensors whose gradients are blocks of partial sums
+// rlt_rocm_adam_step for at most 16 tensors whose gradients are blocks of partial sums
 int rlt_adam_step_from_partials(rlt_rocm_device* device, const rlt_adam_tensor* tensors, int n, const rlt_adam_parameters* parameters, uint32_t* age, const rlt_adam_source* source,
                                 float polyak = 0.0f);
 
-// rlt_rocm_adam_step for two optimisers (each with its own tensors, parameters and age) in one launch; each list at most 12 tensors
+// rlt_rocm_adam_step for two optimisers (each with its own tensors, parameters and age) in one launch; each list at most 16 tensors
 // where a source is given
 int rlt_adam_step_pair(rlt_rocm_device* device, const rlt_adam_tensor* tensors_a, int n_a, const rlt_adam_parameters* parameters_a, uint32_t* age_a,
                        const rlt_adam_tensor* tensors_b, int n_b, const rlt_adam_parameters* parameters_b, uint32_t* age_b,

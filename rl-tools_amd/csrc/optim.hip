@@ -8,7 +8,7 @@
 
 namespace {
 
-constexpr int MAX_T = 12;
+constexpr int MAX_T = 16;
 struct AdamLaunch {
     rlt_adam_tensor t[MAX_T];
     uint32_t prefix[MAX_T + 1];

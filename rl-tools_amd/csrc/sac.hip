@@ -3,6 +3,8 @@
 // reference: nn/layers/sample_and_squash/operations_generic.h:148-398 (CUDA :17-115),
 //            rl/algorithms/sac/operations_generic.h:133-527 (CUDA :12-128), nn/loss_functions/mse/operations_generic.h:9-97,
 //            random/operations_generic.h:72-105.
+#include "seq_stack.h"
+#include "optim.h"
 #include "common.h"
 #include "sac_update.h"
 #include "mlp_rows.h"
@@ -440,6 +442,54 @@ size_t rlt_rocm_sac_sequence_workspace_bytes(const rlt_sac_sequence_agent* A) {
     return 3 * sequence_pass_workspace_bytes(A, T, B) + ((sizeof(float) * (size_t)A->batch.sequence_length * B + 255) & ~(size_t)255);
 }
 
+// Agents whose networks are the reference's recurrent approximators (seq_stack.hip): a launch takes every layer of a pass, and the passes that do not depend on each other
+// share one. The trained critics' loss gradients and backward passes follow, then their optimisers in one launch.
+static bool sequence_agent_stacked(const rlt_sac_sequence_agent* A) {
+    const int T = A->batch.sequence_length + 1;
+    if (!rlt_seq_stack_supported(A->actor, A->n_actor_layers, T)) return false;
+    for (int k = 0; k < 2; k++)
+        if (!rlt_seq_stack_supported(A->critics[k], A->n_critic_layers, T) || !rlt_seq_stack_supported(A->critics_target[k], A->n_critic_layers, T)) return false;
+    return true;
+}
+static int stacked_train_critics(rlt_rocm_device* device, const rlt_sac_sequence_agent* A, int ci, int count, const float* action_noise) {
+    const rlt_sequence_batch& K = A->batch;
+    const int S = K.sequence_length, B = K.batch, OBS = A->observation_dim, ACT = A->action_dim, D = OBS + ACT;
+    const int first = A->include_first_step_in_targets ? 1 : 0, T = S + first, next_offset = first ? 0 : 1;
+    const size_t ws_bytes = sequence_pass_workspace_bytes(A, S + 1, B);
+    const float* base_next = K.observations_actions_base + (size_t)next_offset * B * D;
+    const uint8_t* next_reset = K.next_reset_base + (size_t)next_offset * B;
+    const uint8_t* next_final = K.next_final_step_mask_base + (size_t)next_offset * B;
+    rlt_stack_forward forward[3];
+    for (int k = 0; k < count; k++) forward[k] = {A->critics[ci + k], K.observations_actions_base, D, K.reset, S, B, nullptr};
+    forward[count] = {A->actor, base_next, D, next_reset, T, B, nullptr};
+    int rc;
+    if ((rc = rlt_seq_stack_forward(device, forward, count + 1))) return rc;
+    float* next_actions = A->next_state_action_value_input + OBS;
+    if ((rc = rlt_rocm_sas_forward(device, &A->sas, seq_output(A->actor, A->n_actor_layers), 2 * ACT, action_noise, ACT, next_actions, D, nullptr, 0,
+                                   A->next_log_probabilities, T * B, ACT))) return rc;
+    if ((rc = rlt_rocm_mask_copy(device, base_next + OBS, D, next_actions, D, next_final, 1, T * B, ACT))) return rc;
+    if ((rc = copy2d(device, base_next, D, A->next_state_action_value_input, D, T * B, OBS))) return rc;
+    const rlt_stack_forward targets[2] = {{A->critics_target[0], A->next_state_action_value_input, D, next_reset, T, B, A->next_q[0]},
+                                          {A->critics_target[1], A->next_state_action_value_input, D, next_reset, T, B, A->next_q[1]}};
+    if ((rc = rlt_seq_stack_forward(device, targets, 2))) return rc;
+    if ((rc = rlt_rocm_sac_target_action_values(device, A->next_q[0] + first * B, A->next_q[1] + first * B, K.rewards, K.terminated, A->next_log_probabilities,
+                                               A->log_alpha.parameters, A->gamma, 0, A->target_action_value, S * B))) return rc;
+    rlt_stack_backward backward[2];
+    for (int k = 0; k < count; k++) {
+        // the last critic's loss gradient goes to the agent's buffer (where two calls leave it), the other's to the end of the workspace
+        float* const d_output = k == count - 1 ? A->d_output : (float*)((char*)A->workspace + 3 * ws_bytes);
+        hipLaunchKernelGGL(sac_d_output_kernel, dim3(1), dim3(1024), 0, device->stream, seq_output(A->critics[ci + k], A->n_critic_layers), (const float*)A->target_action_value,
+                           (const uint8_t*)K.final_step_mask, d_output, S * B, 0);
+        if ((rc = rlt_launch_status(device))) return rc;
+        backward[k] = {A->critics[ci + k], K.observations_actions_base, D, d_output, nullptr, K.reset, S, B, 1, 1, (char*)A->workspace + k * ws_bytes};
+    }
+    if ((rc = rlt_seq_stack_backward(device, backward, count))) return rc;
+    if (count == 2)
+        return rlt_adam_step_pair(device, A->critic_adam_tensors[0], A->n_critic_adam_tensors, &A->critic_adam, A->critic_age[0], A->critic_adam_tensors[1], A->n_critic_adam_tensors,
+                                  &A->critic_adam, A->critic_age[1]);
+    return rlt_rocm_adam_step(device, A->critic_adam_tensors[ci], A->n_critic_adam_tensors, &A->critic_adam, A->critic_age[ci], 0.0f, nullptr);
+}
+
 // rl/algorithms/sac/operations_generic.h:243-337 on a sequence batch, one launch per reference operation
 int rlt_rocm_sac_sequence_train_critic(rlt_rocm_device* device, const rlt_sac_sequence_agent* A, int ci, const float* action_noise) {
     if (!device) return RLT_E_NOT_INITIALISED;
@@ -449,6 +499,7 @@ int rlt_rocm_sac_sequence_train_critic(rlt_rocm_device* device, const rlt_sac_se
     const int S = K.sequence_length, B = K.batch, OBS = A->observation_dim, ACT = A->action_dim, D = OBS + ACT;
     const int first = A->include_first_step_in_targets ? 1 : 0, T = S + first, next_offset = first ? 0 : 1;   // off_policy_runner/operations_generic.h:85-92
     const rlt_seq_layer* critic = A->critics[ci];
+    if (sequence_agent_stacked(A)) return stacked_train_critics(device, A, ci, 1, action_noise);
     // two halves of the workspace: passes that do not depend on each other run at the same time, one on the handle's side stream -- the trained critic's forward
     // pass next to the actor's on the next rows, then the second target critic next to the first (each recurrence fills a twentieth of the chip)
     const size_t ws_bytes = sequence_pass_workspace_bytes(A, S + 1, B);
@@ -503,6 +554,7 @@ int rlt_rocm_sac_sequence_train_critics(rlt_rocm_device* device, const rlt_sac_s
     const int first = A->include_first_step_in_targets ? 1 : 0, T = S + first, next_offset = first ? 0 : 1;
     const size_t ws_bytes = sequence_pass_workspace_bytes(A, S + 1, B);
     void* ws = A->workspace; void* ws_side = (char*)A->workspace + ws_bytes; void* ws_second = (char*)A->workspace + 2 * ws_bytes;
+    if (sequence_agent_stacked(A)) return stacked_train_critics(device, A, 0, 2, action_noise);
     float* d_output_first = (float*)((char*)A->workspace + 3 * ws_bytes);      // critic 0's loss gradient; critic 1's goes to the agent's buffer, where two single calls leave it
     const bool overlap = S >= 48;      // short sequences: a pass is shorter than the two events that fork and join a stream cost on the host
     int rc;
@@ -558,7 +610,7 @@ int rlt_rocm_sac_sequence_train_critics(rlt_rocm_device* device, const rlt_sac_s
 int rlt_rocm_sac_sequence_update_critic_targets(rlt_rocm_device* device, const rlt_sac_sequence_agent* A) {
     if (!device) return RLT_E_NOT_INITIALISED;
     RLT_REQUIRE(sequence_agent_ok(A) && A->n_critic_layers <= RLT_SEQ_MAX_LAYERS);
-    // every tensor of both target critics in one launch per sixteen tensors
+    // every tensor of both target critics in one launch per 32 tensors
     const float* sources[2 * 5 * RLT_SEQ_MAX_LAYERS]; float* targets[2 * 5 * RLT_SEQ_MAX_LAYERS]; uint32_t counts[2 * 5 * RLT_SEQ_MAX_LAYERS];
     int n = 0;
     auto pair = [&](const float* source, float* target, size_t count) { sources[n] = source; targets[n] = target; counts[n++] = (uint32_t)count; };
@@ -589,9 +641,10 @@ int rlt_rocm_sac_sequence_train_actor(rlt_rocm_device* device, const rlt_sac_seq
     const int S = K.sequence_length, B = K.batch, OBS = A->observation_dim, ACT = A->action_dim, D = OBS + ACT, R = S * B;
     const size_t ws_bytes = sequence_pass_workspace_bytes(A, S + 1, B);
     void* ws = A->workspace; void* ws_side = (char*)A->workspace + ws_bytes;
-    const bool overlap = S >= 48;      // short sequences: a pass is shorter than the two events that fork and join a stream cost on the host
+    const bool stacked = sequence_agent_stacked(A);
+    const bool overlap = S >= 48 && !stacked;      // short sequences: a pass is shorter than the two events that fork and join a stream cost on the host
     int rc;
-    if ((rc = rlt_rocm_seq_zero_gradient(device, A->actor, A->n_actor_layers))) return rc;                                                  // :414
+    if (!stacked && (rc = rlt_rocm_seq_zero_gradient(device, A->actor, A->n_actor_layers))) return rc;                                      // :414
     if ((rc = rlt_rocm_fill_f32(device, A->log_alpha.gradient, 1, 1, 1, 0.0f))) return rc;
     const float* obs = K.observations_actions_base;
     if ((rc = rlt_rocm_seq_forward(device, A->actor, A->n_actor_layers, obs, D, K.reset, S, B, ws, ws_bytes))) return rc;                   // :427
@@ -609,7 +662,15 @@ int rlt_rocm_sac_sequence_train_actor(rlt_rocm_device* device, const rlt_sac_seq
     if ((rc = rlt_launch_status(device))) return rc;
     // the inner layers of backward_input run without the reset mode (nn_models/sequential/operations_generic.h:399-407); the critics'
     // output layer has no activation function, so d_output survives the calls unchanged (both read it)
-    for (int k = 1; k >= 0; k--) {
+    if (stacked) {
+        rlt_stack_forward forward[2]; rlt_stack_backward backward[2];
+        for (int k = 0; k < 2; k++) {
+            forward[k] = {A->critics[k], A->state_action_value_input, D, K.reset, S, B, nullptr};
+            backward[k] = {A->critics[k], nullptr, 0, A->d_output, A->d_critic_input[k], nullptr, S, B, 0, 0, nullptr};
+        }
+        if ((rc = rlt_seq_stack_forward(device, forward, 2)) || (rc = rlt_seq_stack_backward(device, backward, 2))) return rc;
+    }
+    for (int k = 1; k >= 0 && !stacked; k--) {
         const bool side = k == 1 && overlap && rlt_side_begin(device);
         void* w = side ? ws_side : ws;
         rc = rlt_rocm_seq_forward(device, A->critics[k], A->n_critic_layers, A->state_action_value_input, D, K.reset, S, B, w, ws_bytes);
@@ -623,6 +684,11 @@ int rlt_rocm_sac_sequence_train_actor(rlt_rocm_device* device, const rlt_sac_seq
     if ((rc = rlt_rocm_mask_zero(device, A->d_actor_output_squashing, ACT, K.final_step_mask, 1, R, ACT))) return rc;                       // :461-463
     if ((rc = sas_backward_impl(device, &A->sas, actor_out, 2 * ACT, action_noise, ACT, A->actor_actions, ACT, A->actor_pre_squashing, ACT, A->d_actor_output_squashing, ACT,
                                 A->d_actor_output, 2 * ACT, A->log_alpha.parameters, A->log_alpha.gradient, K.reset, R, ACT))) return rc;   // :464
+    if (stacked) {
+        const rlt_stack_backward backward = {A->actor, obs, D, A->d_actor_output, nullptr, K.reset, S, B, 1, 1, ws};
+        if ((rc = rlt_seq_stack_backward(device, &backward, 1))) return rc;
+        return rlt_adam_step_pair(device, A->actor_adam_tensors, A->n_actor_adam_tensors, &A->actor_adam, A->actor_age, &A->log_alpha, 1, &A->alpha_adam, A->alpha_age);
+    }
     if ((rc = rlt_rocm_seq_backward(device, A->actor, A->n_actor_layers, obs, D, A->d_actor_output, nullptr, K.reset, S, B, 1, 0, ws, ws_bytes))) return rc;
     if ((rc = rlt_rocm_adam_step(device, A->actor_adam_tensors, A->n_actor_adam_tensors, &A->actor_adam, A->actor_age, 0.0f, nullptr))) return rc;   // :465
     return rlt_rocm_adam_step(device, &A->log_alpha, 1, &A->alpha_adam, A->alpha_age, 0.0f, nullptr);                                      // :466

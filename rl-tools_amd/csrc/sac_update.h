@@ -22,7 +22,7 @@ int rlt_sac_update_critics(rlt_rocm_device* device, const rlt_sac_agent* agent, 
 bool rlt_sac_wide_supported(const rlt_rocm_device* device, const rlt_sac_agent* agent);
 int rlt_sac_wide_update_critics(rlt_rocm_device* device, const rlt_sac_agent* agent, int first, int count, const rlt_update_noise& noise, bool update_targets);
 int rlt_sac_wide_update_actor(rlt_rocm_device* device, const rlt_sac_agent* agent, const rlt_update_noise& noise);
-// target[i] = polyak * target[i] + (1 - polyak) * source[i] for a list of tensors, one launch per 16 tensors
+// target[i] = polyak * target[i] + (1 - polyak) * source[i] for a list of tensors, one launch per 32 tensors
 int rlt_sac_polyak_list(rlt_rocm_device* device, const float* const* sources, float* const* targets, const uint32_t* counts, int n, float polyak);
 
 // The same for TD3 (rl/algorithms/td3/operations_generic.h:170-281): actors obs -> 64 -> 64 -> act with a tanh output followed by the

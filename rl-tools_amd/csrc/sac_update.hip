@@ -544,8 +544,8 @@ __global__ __launch_bounds__(THREADS) void sac_update_kernel(UpdateArgs A) {
     rlt_optimiser_tail<THREADS>(&((const RLT_CONSTANT UpdateArgs*)__builtin_amdgcn_kernarg_segment_ptr())->tail, y, g, G, (__attribute__((address_space(3))) int*)(misc + 48));
 }
 
-// soft update of up to 16 tensors in one launch (utils/polyak/operations_generic.h:11-27): workgroup b serves tensor b % n
-constexpr int MAX_POLYAK = 16;
+// soft update of up to 32 tensors in one launch (utils/polyak/operations_generic.h:11-27): workgroup b serves tensor b % n
+constexpr int MAX_POLYAK = 32;
 struct PolyakList { const float* source[MAX_POLYAK]; float* target[MAX_POLYAK]; uint32_t count[MAX_POLYAK]; int n; float polyak; };
 __global__ __launch_bounds__(256) void polyak_list_kernel(PolyakList P) {
     const int t = blockIdx.x % P.n, part = blockIdx.x / P.n, parts = gridDim.x / P.n;

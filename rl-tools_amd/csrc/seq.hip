@@ -4,6 +4,7 @@
 #include "common.h"
 #include "gemm.h"
 #include "mlp_rows.h"
+#include "seq_stack.h"
 #include <algorithm>
 
 namespace {
@@ -100,7 +101,8 @@ extern "C" {
 
 size_t rlt_rocm_seq_workspace_bytes(const rlt_seq_layer* layers, int n, int steps, int batch) {
     if (!layers || n <= 0 || steps <= 0 || batch <= 0) return 0;
-    return 2 * align256((size_t)steps * batch * max_width(layers, n) * sizeof(float)) + gru_bytes(layers, n, steps, batch) + 256;
+    const size_t by_layer = 2 * align256((size_t)steps * batch * max_width(layers, n) * sizeof(float)) + gru_bytes(layers, n, steps, batch) + 256;
+    return rlt_seq_stack_supported(layers, n, 1) ? std::max(by_layer, rlt_seq_stack_workspace_bytes(layers, steps, batch) + 256) : by_layer;
 }
 
 int rlt_rocm_seq_forward(rlt_rocm_device* device, const rlt_seq_layer* layers, int n, const float* x, int ldx, const uint8_t* reset, int steps, int batch,
@@ -109,6 +111,10 @@ int rlt_rocm_seq_forward(rlt_rocm_device* device, const rlt_seq_layer* layers, i
     RLT_REQUIRE(layers_ok(layers, n) && x && steps > 0 && batch > 0 && ldx >= layer_in(layers[0]));
     Workspace W;
     RLT_REQUIRE(carve(layers, n, steps, batch, workspace, workspace_bytes, &W));
+    if (rlt_seq_stack_supported(layers, n, steps)) {
+        const rlt_stack_forward pass = {layers, x, ldx, reset, steps, batch, nullptr};
+        return rlt_seq_stack_forward(device, &pass, 1);
+    }
     const float* in = x; int ld = ldx, rc;
     for (int l = 0; l < n; l++) {
         const rlt_seq_layer& L = layers[l];
@@ -132,6 +138,10 @@ int rlt_rocm_seq_backward(rlt_rocm_device* device, const rlt_seq_layer* layers, 
     const int rows = steps * batch;
     // backward and backward_full hand the mode to every layer; backward_input hands it on only when the model has a single layer
     const uint8_t* reset_here = (want_w || reset_in_backward_input || n == 1) ? reset : nullptr;
+    if (rlt_seq_stack_supported(layers, n, steps) && (want_w || d_input)) {
+        const rlt_stack_backward pass = {layers, x, ldx, d_output, d_input, reset_here, steps, batch, want_w, 0, (void*)(((uintptr_t)workspace + 255) & ~(uintptr_t)255)};
+        return rlt_seq_stack_backward(device, &pass, 1);
+    }
     float* d_cur = d_output; int which = 0, rc;
     for (int l = n - 1; l >= 0; l--) {
         const rlt_seq_layer& L = layers[l];

@@ -150,7 +150,7 @@ bool agent_ok(const rlt_td3_agent* A) {
            A->workspace && A->actor[A->n_actor_layers - 1].out_dim == A->action_dim && A->critics[0][0].in_dim == A->observation_dim + A->action_dim;
 }
 
-// the soft update of a network's tensors, sixteen to a launch (a launch per tensor: 27 us for the Ant actor's six, together 4.4)
+// the soft update of a network's tensors, 32 to a launch (a launch per tensor: 27 us for the Ant actor's six, together 4.4)
 int polyak_mlp(rlt_rocm_device* device, const rlt_dense_layer* source, const rlt_dense_layer* target, int n, float polyak) {
     RLT_REQUIRE(n <= 32);
     const float* sources[64]; float* targets[64]; uint32_t counts[64];
