@@ -1,37 +1,40 @@
 // Passes of the reference's recurrent approximators (rl/algorithms/sac/loop/core/approximators_gru.h:13-74: dense, GRU, GRU, dense) over a batch of sequences, all
 // layers in one launch (nn_models/sequential/operations_generic.h:277-428, nn/layers/gru/operations_generic.h:231-341, :594-795).
 //
-// Batch rows are independent, layers depend on each other only step by step: a workgroup carries ONE batch row, its five wavefronts are the stages of a pipeline, and a
-// stage works on the step behind the previous stage's (one workgroup barrier per tick orders LDS only; the slots between two stages are double-buffered by the step's
-// parity). Forward: dense layer and first input projection | first recurrence | second input projection | second recurrence | output layer; backward, from the last
-// step on: output layer and second recurrence | its input gradient | first recurrence | its input gradient and the dense layer's | the input's gradient.
-// Within a stage lane (u, p) owns hidden unit u and a share p of the reduction index (half of it at width 32, a quarter at 16), with its 3 H / (64 / H) weights in
-// registers; the vector of the step arrives through LDS (16-byte broadcast reads) and the shares are added with v_permlane32_swap / v_permlane16_swap.
+// Batch rows are independent, layers depend on each other only step by step: a workgroup carries ONE batch row, its wavefronts are the stages of a pipeline, and a
+// stage works a step or two behind the previous stage (one workgroup barrier per tick orders LDS only; the slots between two stages are double-buffered). Forward: dense
+// layer and first input projection | first recurrence | second input projection | second recurrence | output layer; backward, from the last step on: output layer |
+// second recurrence | its input gradient | first recurrence | its input gradient and the dense layer's | the input's gradient.
 // Weight gradients are contractions over all steps and rows, done afterwards for all layers by one launch on the matrix cores (and a second that adds the shares of the
 // rows up).
-// Bound: the chain of dependent steps, TODO us per step at width 32 (a launch per layer and direction with a row per 32 lanes took 0.58 us per step, one layer
-// after the other, plus a launch per dense layer, projection and gradient: TODO). Workgroups of up to three models share a launch.
+// Bound: the instructions of a recurrence's step. A wavefront is alone on its SIMD and issues one instruction every four to five cycles whatever it is (vector, scalar,
+// wait), so a step takes its instruction count: about 115 at width 32, 48 of them the products. Hence the forms below: values exchanged between lanes instead of through
+// LDS, the r gate in one half of the lanes while z is in the other, stores and LDS writes by all lanes of a unit rather than under an exec mask, addresses moved on
+// instead of formed, loops unrolled to the slots' parity. TODO us per step at width 32 (TODO backward); a launch per layer with a row per 32 lanes took 0.58 us per step,
+// one layer after the other, plus launches for the dense layers, projections and gradients.
 #include "seq_stack.h"
 #include "gemm.h"
 #include "batch_tile.h"
+#include <utility>
 
 namespace {
 typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
-constexpr int MAX_IN = 16, MAX_OUT = 16, STAGES = 5, THREADS = 64 * STAGES, MAX_PASSES = 3;
+constexpr int MAX_IN = 16, MAX_OUT = 16, FORWARD_STAGES = 5, BACKWARD_STAGES = 6, MAX_PASSES = 3;
 constexpr size_t LDS_LIMIT = 48 * 1024;      // three to four workgroups per compute unit
 
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+__device__ __forceinline__ void swap32(float& a, float& b) {      // the upper half of a's lanes against the lower half of b's
+    const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false); a = __uint_as_float(s[0]); b = __uint_as_float(s[1]);
 }
-// the sum of x over the lanes of one unit (lanes 64 / PARTS apart); every one of them receives it
+__device__ __forceinline__ void swap16(float& a, float& b) {      // the odd rows of sixteen lanes of a against the even rows of b
+    const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false); a = __uint_as_float(s[0]); b = __uint_as_float(s[1]);
+}
+// the sum of x over the lanes of one unit (64 / PARTS apart); every one of them receives it
 template <int PARTS>
 __device__ __forceinline__ float sum_parts(float x) {
-    if (PARTS == 4) { const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false); x = __uint_as_float(s[0]) + __uint_as_float(s[1]); }
-    const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+    float y = x;
+    if (PARTS == 4) { swap16(x, y); x += y; y = x; }
+    swap32(x, y);
+    return x + y;
 }
 // The reference's rational tanh (math/operations_generic.h:247-255) with the quotient from v_rcp_f32 and two corrections (the divisor lies in [27, 108]: no scaling is
 // needed, and the result is within one rounding of the quotient)
@@ -46,59 +49,96 @@ __device__ __forceinline__ float fast_tanh(float x) {
 template <bool FAST> __device__ __forceinline__ float gate_sigmoid(float x) { return FAST ? 0.5f * fast_tanh(0.5f * x) + 0.5f : 1.0f / (1.0f + expf(-x)); }
 template <bool FAST> __device__ __forceinline__ float gate_tanh(float x) { return FAST ? fast_tanh(x) : tanhf(x); }
 
-// rows u, H + u, 2H + u of a [3H x H] matrix (or, transposed, its columns u of the three blocks), this lane's share of the reduction index
-template <int H>
-struct Weights3 { float w[3][H * H / 64]; };
+// Products of a vector with rows (or columns) of a recurrence's weights: every lane of a unit holds the unit's value, and a multiply-add whose first operand carries the
+// row_newbcast control takes it from one lane of each row of sixteen lanes. At width 32 the rows hold units 0-15, 16-31, 0-15, 16-31: after an exchange the first two
+// have units 0-15 in their lanes and the last two units 16-31, each row forms its units' three sums over that half of the reduction index, and the halves meet across the
+// rows. At width 16 the rows of lanes are the three gates (and nothing): each forms its gate's sums over all sixteen units.
+// (The control in the multiply-add itself: left to the compiler, each broadcast is an instruction of its own. The data of such an operand must have been written two wait
+// states before it is read: wait_for_dpp() stands between.)
+__device__ __forceinline__ void wait_for_dpp(float& x) { asm volatile("s_nop 1" : "+v"(x)); }
+template <int K> __device__ __forceinline__ void broadcast_fma(float& acc, float x, float w) {
+    if (K < 0) return;
+    asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(x), "v"(w), "n"(K < 0 ? 0 : K));
+}
+__device__ __forceinline__ float broadcast_first(float x, float w) { float acc; asm("v_mul_f32_dpp %0, %1, %2 row_newbcast:0 row_mask:0xf bank_mask:0xf" : "=v"(acc) : "v"(x), "v"(w)); return acc; }
+// a lane's weights of a [3H x H] matrix: width 32: rows (or columns) u of the three blocks, half p of the reduction index; width 16: row (column) u of block p
+template <int H> struct Weights3 { float w[H == 32 ? 3 : 1][16]; };
 template <int H>
 __device__ __forceinline__ void load_rows3(const float* W, int u, int p, Weights3<H>& R) {
-    constexpr int KP = H * H / 64;
 #pragma unroll
-    for (int k = 0; k < 3; k++)
+    for (int k = 0; k < (H == 32 ? 3 : 1); k++) {
+        const float* from = H == 32 ? W + (size_t)(k * H + u) * H + p * 16 : W + (size_t)(min(p, 2) * H + u) * H;
 #pragma unroll
-        for (int q = 0; q < KP; q += 4) {
+        for (int q = 0; q < 16; q += 4) {
             floatx4 v;
-            __builtin_memcpy(&v, W + (size_t)(k * H + u) * H + p * KP + q, sizeof v);      // 16 bytes at a time, whatever the tensor's alignment
+            __builtin_memcpy(&v, from + q, sizeof v);      // 16 bytes at a time, whatever the tensor's alignment
             R.w[k][q] = v[0]; R.w[k][q + 1] = v[1]; R.w[k][q + 2] = v[2]; R.w[k][q + 3] = v[3];
         }
+    }
 }
 template <int H>
 __device__ __forceinline__ void load_columns3(const float* W, int u, int p, Weights3<H>& R) {
-    constexpr int KP = H * H / 64;
 #pragma unroll
-    for (int k = 0; k < 3; k++)
+    for (int k = 0; k < (H == 32 ? 3 : 1); k++)
 #pragma unroll
-        for (int q = 0; q < KP; q++) R.w[k][q] = W[(size_t)(k * H + p * KP + q) * H + u];
+        for (int q = 0; q < 16; q++) R.w[k][q] = H == 32 ? W[(size_t)(k * H + p * 16 + q) * H + u] : (p < 3 ? W[(size_t)(p * H + q) * H + u] : 0.f);
 }
-// the three products of a vector v (LDS, H values) with rows u of the three blocks
-template <int H>
-__device__ __forceinline__ void products3(const Weights3<H>& R, const float* v, int p, float (&out)[3]) {
-    constexpr int KP = H * H / 64, PARTS = 64 / H;
-    float acc[3] = {0.f, 0.f, 0.f};
-    floatx4 x[KP / 4];
-#pragma unroll
-    for (int q = 0; q < KP / 4; q++) x[q] = reinterpret_cast<const floatx4*>(v + p * KP)[q];
-#pragma unroll
-    for (int q = 0; q < KP; q++)
-#pragma unroll
-        for (int k = 0; k < 3; k++) acc[k] += x[q / 4][q % 4] * R.w[k][q];
-#pragma unroll
-    for (int k = 0; k < 3; k++) out[k] = sum_parts<PARTS>(acc[k]);
+__device__ __forceinline__ float half_in_rows(float v, int p) { float w = v; swap16(v, w); return p ? w : v; }
+template <int H, int... Q>
+__device__ __forceinline__ void multiply(const Weights3<H>& R, float x, float y, float z, float (&acc)[3], std::integer_sequence<int, Q...>) {
+    wait_for_dpp(x);
+    if (H == 32) {
+        acc[0] = broadcast_first(x, R.w[0][0]); acc[1] = broadcast_first(y, R.w[H == 32 ? 1 : 0][0]); acc[2] = broadcast_first(z, R.w[H == 32 ? 2 : 0][0]);
+        ((broadcast_fma<Q + 1>(acc[0], x, R.w[0][Q + 1]), broadcast_fma<Q + 1>(acc[1], y, R.w[H == 32 ? 1 : 0][Q + 1]), broadcast_fma<Q + 1>(acc[2], z, R.w[H == 32 ? 2 : 0][Q + 1])), ...);
+    } else {
+        acc[0] = broadcast_first(x, R.w[0][0]); acc[1] = 0.f; acc[2] = 0.f;
+        (broadcast_fma<Q + 1>(acc[(Q + 1) % 3], x, R.w[0][Q + 1]), ...);
+        acc[0] += acc[1] + acc[2];
+    }
 }
-// the sum over three vectors (LDS, 3 x H values) of their products with columns u of the three blocks
+// The products of a vector (element u in the lanes of unit u) with rows u of the three blocks. rz: the first block's in the lanes with p = 0, the second's where p = 1
+// (width 16: also the third's where p = 2); n: the third's in every lane.
 template <int H>
-__device__ __forceinline__ float product_sum3(const Weights3<H>& R, const float* v, int p) {
-    constexpr int KP = H * H / 64, PARTS = 64 / H;
-    float acc[3] = {0.f, 0.f, 0.f};
-    floatx4 x[3][KP / 4];
-#pragma unroll
-    for (int k = 0; k < 3; k++)
-#pragma unroll
-        for (int q = 0; q < KP / 4; q++) x[k][q] = reinterpret_cast<const floatx4*>(v + k * H + p * KP)[q];
-#pragma unroll
-    for (int q = 0; q < KP; q++)
-#pragma unroll
-        for (int k = 0; k < 3; k++) acc[k] += x[k][q / 4][q % 4] * R.w[k][q];
-    return sum_parts<PARTS>(acc[0] + (acc[1] + acc[2]));
+__device__ __forceinline__ void products3(const Weights3<H>& R, float v, int p, float& rz, float& n) {
+    float acc[3];
+    const float x = H == 32 ? half_in_rows(v, p) : v;
+    multiply<H>(R, x, x, x, acc, std::make_integer_sequence<int, 15>{});
+    if (H == 32) {
+        swap32(acc[0], acc[1]);
+        rz = acc[0] + acc[1];
+        n = sum_parts<2>(acc[2]);
+    } else {
+        float a = acc[0], b = acc[0];
+        rz = acc[0];
+        swap16(a, b); b = a; swap32(a, b);
+        n = b;
+    }
+}
+// the sum over three vectors of their products with columns u of the three blocks, in every lane of the unit
+template <int H>
+__device__ __forceinline__ float product_sum3(const Weights3<H>& R, float x, float y, float z, int p) {
+    float acc[3];
+    if (H == 32) {
+        x = half_in_rows(x, p); y = half_in_rows(y, p); z = half_in_rows(z, p);
+        wait_for_dpp(y); wait_for_dpp(z);
+        multiply<H>(R, x, y, z, acc, std::make_integer_sequence<int, 15>{});
+        return sum_parts<2>(acc[0] + (acc[1] + acc[2]));
+    }
+    multiply<H>(R, p == 0 ? x : p == 1 ? y : z, 0.f, 0.f, acc, std::make_integer_sequence<int, 15>{});
+    return sum_parts<4>(acc[0]);
+}
+
+// A stage: `before` ticks until its first step is there, one per step, `after` ticks for the stages behind it. The steps are unrolled U at a time with their number in the
+// group as a constant (slots and queues are indexed by it).
+template <class F, int... D>
+__device__ __forceinline__ void stage_group(int i, int S, F& step, std::integer_sequence<int, D...>) {
+    ((i + D < S ? (step(std::integral_constant<int, D>{}, i + D), rlt_lds_barrier()) : (void)0), ...);
+}
+template <int U, class F>
+__device__ __forceinline__ void stage(int S, int before, int after, F&& step) {
+    for (int k = 0; k < before; k++) rlt_lds_barrier();
+    for (int i = 0; i < S; i += U) stage_group(i, S, step, std::make_integer_sequence<int, U>{});
+    for (int k = 0; k < after; k++) rlt_lds_barrier();
 }
 
 struct Gru { const float *W_i, *b_i, *W_h, *b_h, *h0; float *post, *npp, *out; };
@@ -108,60 +148,58 @@ struct Forward {
 };
 struct ForwardLaunch { Forward pass[MAX_PASSES]; int n; };
 
-// LDS of a workgroup: the row's inputs (rows of four floats' multiples) and reset flags, then the slots between the stages
-template <int H> struct ForwardSlots { float dense[H], own[2][H], p1[2][3 * H], h1[2][H], p2[2][3 * H], h2[2][H]; };
+// LDS of a workgroup: the slots between the stages, then the row's inputs (rows of four floats' multiples) and reset flags. A projection's slot: what the r and z gates
+// and then the n gate receive (width 16: a fourth row that nobody reads).
+template <int H> struct ForwardSlots { float p1[2][4 * H], h1[2][H], p2[2][4 * H], h2[2][H]; };
 
-template <int H, bool FAST>
-__device__ __forceinline__ void recurrence(const Forward& P, int layer, int lag, const float (*in)[3 * H], float* own, float (*out)[H], const uint8_t* flags, int b, int lane) {
-    constexpr int PARTS = 64 / H;
-    const Gru& G = P.g[layer];
-    const int u = lane & (H - 1), p = lane / H, S = P.S;
-    Weights3<H> R;
-    load_rows3<H>(G.W_h, u, p, R);
-    const float br = G.b_h[u], bz = G.b_h[H + u], bn = G.b_h[2 * H + u], h0 = G.h0[u];
-    float h = h0;
-    if (p == 0) own[u] = h0;
-    for (int tick = 0; tick < S + STAGES - 1; tick++) {
-        const int t = tick - lag;
-        if (t >= 0 && t < S) {
-            const float* x = in[t & 1];
-            const float xr = x[u], xz = x[H + u], xn = x[2 * H + u];
-            float a[3];
-            products3<H>(R, own, p, a);
-            const float an = bn + a[2];
-            const float r = gate_sigmoid<FAST>(xr + (br + a[0])), z = gate_sigmoid<FAST>(xz + (bz + a[1]));
-            const float n = gate_tanh<FAST>(xn + an * r);
-            h = (1.0f - z) * n + z * h;
-            const size_t at = (size_t)t * P.B + b;
-            // what a restart at the next step takes in place of this step's state
-            const bool restart = t + 1 < S && flags[t + 1];
-            const float out_h = h;
-            if (restart) h = h0;
-            wave_sync();
-            if (p == 0) { out[t & 1][u] = out_h; own[u] = h; }
-            wave_sync();
-            float* const post = G.post + at * 3 * H;
-            if (p < 2) { post[p * H + u] = p ? z : r; (p ? G.npp + at * H : post + 2 * H)[u] = p ? an : n; }
-            if (p == PARTS - 1) G.out[at * H + u] = out_h;
-        }
-        rlt_lds_barrier();
-    }
+// the input projection of one step into a slot; the biases of the hidden path's r and z gates ride along
+template <int H> struct Projection { Weights3<H> R; float brz, bn; };
+template <int H>
+__device__ __forceinline__ void load_projection(const Gru& G, int u, int p, Projection<H>& J) {
+    load_rows3<H>(G.W_i, u, p, J.R);
+    J.brz = p < 2 ? G.b_i[p * H + u] + G.b_h[p * H + u] : 0.f; J.bn = G.b_i[2 * H + u];
 }
 template <int H>
-__device__ __forceinline__ void projection(const Gru& G, int S, int lag, const float (*in)[H], float (*out)[3 * H], int lane) {
+__device__ __forceinline__ void project(const Projection<H>& J, float v, int u, int p, float* slot) {
+    float rz, n;
+    products3<H>(J.R, v, p, rz, n);
+    slot[p * H + u] = rz + J.brz;      // width 16: the third row is overwritten by the next line, the fourth is nobody's
+    slot[2 * H + u] = n + J.bn;
+}
+template <int H, bool FAST>
+__device__ __forceinline__ void recurrence(const Forward& P, int layer, int lag, const float (*in)[4 * H], float (*out)[H], const uint8_t* flags, int b, int lane) {
+    constexpr int PARTS = 64 / H;
+    const Gru& G = P.g[layer];
     const int u = lane & (H - 1), p = lane / H;
     Weights3<H> R;
-    load_rows3<H>(G.W_i, u, p, R);
-    const float br = G.b_i[u], bz = G.b_i[H + u], bn = G.b_i[2 * H + u];
-    for (int tick = 0; tick < S + STAGES - 1; tick++) {
-        const int t = tick - lag;
-        if (t >= 0 && t < S) {
-            float a[3];
-            products3<H>(R, in[t & 1], p, a);
-            if (p == 0) { float* o = out[t & 1]; o[u] = br + a[0]; o[H + u] = bz + a[1]; o[2 * H + u] = bn + a[2]; }
-        }
-        rlt_lds_barrier();
-    }
+    load_rows3<H>(G.W_h, u, p, R);
+    const float bn = G.b_h[2 * H + u], h0 = G.h0[u];
+    // where a lane stores what it keeps of a step, moved on from step to step. Width 32: r / z, then n / the n gate's hidden part in the two halves; width 16: one of the
+    // four in each row of lanes. The output by all lanes of a unit.
+    const size_t stride = (size_t)P.B * H;
+    float* const post = G.post + (size_t)b * 3 * H + u; float* const npp = G.npp + (size_t)b * H + u;
+    float* keep1 = PARTS == 2 ? post + p * H : p < 3 ? post + p * H : npp; float* keep2 = p ? npp : post + 2 * H; float* keep3 = G.out + (size_t)b * H + u;
+    const size_t stride1 = PARTS == 2 || p < 3 ? 3 * stride : stride, stride2 = p ? stride : 3 * stride;
+    float h = h0;
+    stage<2>(P.S, lag, FORWARD_STAGES - 1 - lag, [&](auto d, int t) {
+        constexpr int PAR = decltype(d)::value & 1;
+        const float x = in[PAR][PARTS == 2 ? p * H + u : min(p, 1) * H + u], xn = in[PAR][2 * H + u];
+        const bool restart = flags[t + 1];      // the next step starts from the initial state (the flags end with one more entry)
+        float rz, n_hidden;
+        products3<H>(R, h, p, rz, n_hidden);
+        const float an = n_hidden + bn, s = gate_sigmoid<FAST>(x + rz);
+        float r = s, z = s;
+        if (PARTS == 2) swap32(r, z);
+        else { swap16(r, z); float r2 = r, z2 = z; swap32(r, r2); swap32(z, z2); }
+        const float n = gate_tanh<FAST>(xn + an * r);
+        const float o = n + z * (h - n);
+        h = restart ? h0 : o;
+        out[PAR][u] = o;
+        if (PARTS == 2) { *keep1 = s; *keep2 = p ? an : n; keep2 += stride2; }
+        else *keep1 = p < 2 ? s : p == 2 ? n : an;
+        *keep3 = o;
+        keep1 += stride1; keep3 += stride;
+    });
 }
 template <int H, bool FAST>
 __device__ __forceinline__ void forward_row(const Forward& P, int b, char* lds) {
@@ -169,8 +207,8 @@ __device__ __forceinline__ void forward_row(const Forward& P, int b, char* lds) 
     ForwardSlots<H>& L = *reinterpret_cast<ForwardSlots<H>*>(lds);
     float* const xs = reinterpret_cast<float*>(lds + ((sizeof(ForwardSlots<H>) + 15) & ~(size_t)15));
     uint8_t* const flags = reinterpret_cast<uint8_t*>(xs + (size_t)S * in4);
-    for (int i = threadIdx.x; i < S * in4; i += THREADS) { const int t = i / in4, k = i - t * in4; xs[i] = k < P.in ? P.x[((size_t)t * P.B + b) * P.ldx + k] : 0.f; }
-    for (int t = threadIdx.x; t < S; t += THREADS) flags[t] = t == 0 || (P.reset && P.reset[(size_t)t * P.B + b]);
+    for (int i = threadIdx.x; i < S * in4; i += 64 * FORWARD_STAGES) { const int t = i / in4, k = i - t * in4; xs[i] = k < P.in ? P.x[((size_t)t * P.B + b) * P.ldx + k] : 0.f; }
+    for (int t = threadIdx.x; t <= S; t += 64 * FORWARD_STAGES) flags[t] = t == 0 || (t < S && P.reset && P.reset[(size_t)t * P.B + b]);
     rlt_lds_barrier();
     if (wave == 0) {
         // the dense layer and the first recurrence's input projection
@@ -178,31 +216,32 @@ __device__ __forceinline__ void forward_row(const Forward& P, int b, char* lds) 
 #pragma unroll
         for (int k = 0; k < MAX_IN; k++) w0[k] = k < P.in ? P.W0[(size_t)u * P.in + k] : 0.f;
         const float b0 = P.b0[u];
-        Weights3<H> R;
-        load_rows3<H>(P.g[0].W_i, u, p, R);
-        const float br = P.g[0].b_i[u], bz = P.g[0].b_i[H + u], bn = P.g[0].b_i[2 * H + u];
-        for (int t = 0; t < S + STAGES - 1; t++) {
-            if (t < S) {
-                float acc = b0;
-                const floatx4* x = reinterpret_cast<const floatx4*>(xs + (size_t)t * in4);
+        Projection<H> J;
+        load_projection<H>(P.g[0], u, p, J);
+        float* keep = ((p & 1) ? P.out0 : P.pre0) + (size_t)b * H + u;
+        const size_t stride = (size_t)P.B * H;
+        const int in = P.in, act0 = P.act0;
+        const float* row = xs;
+        stage<2>(S, 0, FORWARD_STAGES - 1, [&](auto d, int) {
+            float acc = b0;
+            const floatx4* x = reinterpret_cast<const floatx4*>(row);
 #pragma unroll
-                for (int q = 0; q < MAX_IN / 4; q++)
-                    if (4 * q < P.in) { const floatx4 v = x[q]; acc += v[0] * w0[4 * q]; acc += v[1] * w0[4 * q + 1]; acc += v[2] * w0[4 * q + 2]; acc += v[3] * w0[4 * q + 3]; }
-                const float o = rlt_act(acc, P.act0);
-                if (p < 2) (p ? P.out0 : P.pre0)[((size_t)t * P.B + b) * H + u] = p ? o : acc;
-                if (p == 0) L.dense[u] = o;
-                wave_sync();
-                float a[3];
-                products3<H>(R, L.dense, p, a);
-                wave_sync();
-                if (p == 0) { float* d = L.p1[t & 1]; d[u] = br + a[0]; d[H + u] = bz + a[1]; d[2 * H + u] = bn + a[2]; }
-            }
-            rlt_lds_barrier();
-        }
+            for (int q = 0; q < MAX_IN / 4; q++)
+                if (q == 0 || 4 * q < in) { const floatx4 v = x[q]; acc += v[0] * w0[4 * q]; acc += v[1] * w0[4 * q + 1]; acc += v[2] * w0[4 * q + 2]; acc += v[3] * w0[4 * q + 3]; }
+            row += in4;
+            const float o = rlt_act(acc, act0);
+            *keep = (p & 1) ? o : acc;
+            keep += stride;
+            project<H>(J, o, u, p, L.p1[decltype(d)::value & 1]);
+        });
     }
-    else if (wave == 1) recurrence<H, FAST>(P, 0, 1, L.p1, L.own[0], L.h1, flags, b, lane);
-    else if (wave == 2) projection<H>(P.g[1], S, 2, L.h1, L.p2, lane);
-    else if (wave == 3) recurrence<H, FAST>(P, 1, 3, L.p2, L.own[1], L.h2, flags, b, lane);
+    else if (wave == 1) recurrence<H, FAST>(P, 0, 1, L.p1, L.h1, flags, b, lane);
+    else if (wave == 2) {
+        Projection<H> J;
+        load_projection<H>(P.g[1], u, p, J);
+        stage<2>(S, 2, 2, [&](auto d, int) { project<H>(J, L.h1[decltype(d)::value & 1][u], u, p, L.p2[decltype(d)::value & 1]); });
+    }
+    else if (wave == 3) recurrence<H, FAST>(P, 1, 3, L.p2, L.h2, flags, b, lane);
     else {
         // the output layer: lane = output, all of the reduction
         float w3[H];
@@ -210,22 +249,21 @@ __device__ __forceinline__ void forward_row(const Forward& P, int b, char* lds) 
 #pragma unroll
         for (int k = 0; k < H; k++) w3[k] = P.W3[(size_t)o * H + k];
         const float b3 = P.b3[o];
-        for (int tick = 0; tick < S + STAGES - 1; tick++) {
-            const int t = tick - 4;
-            if (t >= 0) {
-                const floatx4* h = reinterpret_cast<const floatx4*>(L.h2[t & 1]);
-                float a0 = b3, a1 = 0.f, a2 = 0.f, a3 = 0.f;
+        // (without a third place the second is written twice)
+        float* pre3 = P.pre3 + (size_t)b * P.out + o; float* out3 = P.out3 + (size_t)b * P.out + o; float* also = P.also ? P.also + (size_t)b * P.out + o : out3;
+        const size_t stride = (size_t)P.B * P.out;
+        stage<2>(S, 4, 0, [&](auto d, int) {
+            const floatx4* h = reinterpret_cast<const floatx4*>(L.h2[decltype(d)::value & 1]);
+            float a0 = b3, a1 = 0.f, a2 = 0.f, a3 = 0.f;
 #pragma unroll
-                for (int q = 0; q < H / 4; q++) { const floatx4 v = h[q]; a0 += v[0] * w3[4 * q]; a1 += v[1] * w3[4 * q + 1]; a2 += v[2] * w3[4 * q + 2]; a3 += v[3] * w3[4 * q + 3]; }
-                const float y = (a0 + a1) + (a2 + a3);
-                const size_t at = ((size_t)t * P.B + b) * P.out + lane;
-                if (lane < P.out) { P.pre3[at] = y; P.out3[at] = y; if (P.also) P.also[at] = y; }
-            }
-            rlt_lds_barrier();
-        }
+            for (int q = 0; q < H / 4; q++) { const floatx4 v = h[q]; a0 += v[0] * w3[4 * q]; a1 += v[1] * w3[4 * q + 1]; a2 += v[2] * w3[4 * q + 2]; a3 += v[3] * w3[4 * q + 3]; }
+            const float y = (a0 + a1) + (a2 + a3);
+            *pre3 = y; *out3 = y; *also = y;
+            pre3 += stride; out3 += stride; also += stride;
+        });
     }
 }
-__global__ __launch_bounds__(THREADS) void seq_stack_forward_kernel(ForwardLaunch K) {
+__global__ __launch_bounds__(64 * FORWARD_STAGES) void seq_stack_forward_kernel(ForwardLaunch K) {
     extern __shared__ __attribute__((aligned(16))) char lds_stack[];
     int k = 0;
     if (K.n > 1 && (int)blockIdx.x >= K.pass[1].first_block) k = 1;
@@ -242,120 +280,115 @@ struct Backward {
     GruBack g[2]; const float *W0, *pre0, *W3, *d_output; float *d_pre0, *d_input; const uint8_t* reset; int in, out, act0, S, B, H, want_w, first_block;
 };
 struct BackwardLaunch { Backward pass[MAX_PASSES]; int n; };
-template <int H> struct BackwardSlots { float own[2][3 * H], g2[2][3 * H], dy1[2][H], g1[2][3 * H], dp0[2][H]; };
+template <int H> struct BackwardSlots { float dy2[2][H], g2[2][3 * H], dy1[2][H], g1[2][3 * H], dp0[2][H]; };
+constexpr int AHEAD = 6;      // steps ahead of its use that a saved value is requested (a load takes several steps)
 
-template <int H, bool TOP>
-__device__ __forceinline__ void recurrence_back(const Backward& P, int layer, int lag, const float* d_out, const float (*dy)[H], float* own, float (*g)[3 * H], const uint8_t* flags, int b, int lane) {
-    constexpr int PARTS = 64 / H, DEPTH = 4;
+// A recurrence's way back, step i of S (from the last on). dy: the gradient at its output from the stage above, held in a register from the tick before.
+template <int H>
+__device__ __forceinline__ void recurrence_back(const Backward& P, int layer, int lag, const float (*dy)[H], float (*g)[3 * H], const uint8_t* flags, int b, int lane) {
     const GruBack& G = P.g[layer];
     const int u = lane & (H - 1), p = lane / H, S = P.S;
     Weights3<H> R;
     load_columns3<H>(G.W_h, u, p, R);
     const float h0 = G.h0[u];
-    float w3[TOP ? MAX_OUT : 1];
-    if (TOP) {
-#pragma unroll
-        for (int o = 0; o < MAX_OUT; o++) w3[o] = o < P.out ? P.W3[(size_t)o * H + u] : 0.f;
-    }
-    // a step's saved values, requested DEPTH steps ahead (a load takes longer than a step); the lanes of a unit load different ones and exchange them
-    struct Saved { float rz, nn, hp; };
-    auto request = [&](int t) {
-        const size_t at = (size_t)(t > 0 ? t : 0) * P.B + b, before = (size_t)(t > 1 ? t - 1 : 0) * P.B + b;
-        Saved v;
-        v.rz = G.post[at * 3 * H + (p & 1) * H + u]; v.nn = ((p & 1) ? G.npp + at * H : G.post + at * 3 * H + 2 * H)[u]; v.hp = G.out[before * H + u];
-        return v;
+    const size_t stride = (size_t)P.B * H, last = (size_t)(S - 1) * stride + (size_t)b * H;      // the row's last step in an array of H columns
+    const float* post = G.post + 3 * last + u; const float* npp = G.npp + last + u; const float* state = G.out + last + u;
+    struct Saved { float r, z, n, npp, hp; };
+    Saved queue[AHEAD];
+    auto request = [&](int i, Saved& v) {      // step i's values; the state is the one before the step (the first step takes the initial one)
+        if (i >= S) return;
+        if (i + 1 < S) state -= stride;
+        v.r = post[0]; v.z = post[H]; v.n = post[2 * H]; v.npp = *npp; v.hp = *state;
+        post -= 3 * stride; npp -= stride;
     };
-    Saved queue[DEPTH];
 #pragma unroll
-    for (int d = 0; d < DEPTH; d++) queue[d] = request(S - 1 - d);
-    float carry = 0.f, db_hn = 0.f;
-    for (int tick = 0; tick < S + STAGES - 1; tick++) {
-        const int t = S - 1 - (tick - lag);
-        if (t >= 0 && t < S) {
-            const Saved cur = queue[0];
-#pragma unroll
-            for (int d = 0; d + 1 < DEPTH; d++) queue[d] = queue[d + 1];
-            queue[DEPTH - 1] = request(t - DEPTH);
-            float r, z, n, npp;
-            if (PARTS == 2) {
-                const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(cur.rz), __float_as_uint(cur.rz), false, false), c = __builtin_amdgcn_permlane32_swap(__float_as_uint(cur.nn), __float_as_uint(cur.nn), false, false);
-                r = __uint_as_float(a[0]); z = __uint_as_float(a[1]); n = __uint_as_float(c[0]); npp = __uint_as_float(c[1]);
-            } else {
-                const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(cur.rz), __float_as_uint(cur.rz), false, false), c = __builtin_amdgcn_permlane16_swap(__float_as_uint(cur.nn), __float_as_uint(cur.nn), false, false);
-                r = __uint_as_float(a[0]); z = __uint_as_float(a[1]); n = __uint_as_float(c[0]); npp = __uint_as_float(c[1]);
-            }
-            float dh = carry;
-            if (TOP) {
-                const float* d = d_out + (size_t)t * P.out;
-                float s = 0.f;
-#pragma unroll
-                for (int o = 0; o < MAX_OUT; o++) if (o < P.out) s += d[o] * w3[o];
-                dh += s;
-            } else dh += dy[t & 1][u];
-            const bool from_initial = flags[t];
-            const float hp = from_initial ? h0 : cur.hp;
-            const float gz = dh * (hp - n) * z * (1.0f - z);
-            const float gn = dh * (1.0f - z) * (1.0f - n * n);
-            const float gr = gn * npp * r * (1.0f - r);
-            const float gnr = gn * r;
-            if (p == 0) { own[u] = gr; own[H + u] = gz; own[2 * H + u] = gnr; float* s = g[t & 1]; s[u] = gr; s[H + u] = gz; s[2 * H + u] = gn; }
-            wave_sync();
-            const float sum = product_sum3<H>(R, own, p);
-            wave_sync();
-            carry = from_initial ? 0.f : dh * z + sum;
-            if (P.want_w) {
-                const size_t at = (size_t)t * P.B + b;
-                if (p < 2) { G.g[at * 3 * H + p * H + u] = p ? gz : gr; (p ? G.gnr + at * H : G.g + at * 3 * H + 2 * H)[u] = p ? gnr : gn; }
-                if (p == PARTS - 1) G.hp[at * H + u] = hp;
-                // the reference drops reset samples (t > 0) from the b_hn gradient (their buffer rows are zeroed before that sum, gru/operations_generic.h:716-749)
-                if (!(t > 0 && from_initial)) db_hn += gnr;
-            }
+    for (int d = 0; d < AHEAD; d++) request(d, queue[d]);
+    const bool want_w = P.want_w;
+    float* to_g = want_w ? G.g + 3 * last + u : nullptr; float* to_gnr = want_w ? G.gnr + last + u : nullptr; float* to_hp = want_w ? G.hp + last + u : nullptr;
+    float carry = 0.f, db_hn = 0.f, above = 0.f;
+    for (int k = 0; k < lag - 1; k++) rlt_lds_barrier();
+    above = dy[0][u];
+    rlt_lds_barrier();
+    stage<AHEAD>(S, 0, BACKWARD_STAGES + 1 - lag, [&](auto d, int i) {
+        constexpr int N = decltype(d)::value;
+        const Saved v = queue[N];
+        request(i + AHEAD, queue[N]);
+        const float dh = above + carry;
+        above = dy[(N + 1) & 1][u];      // the next step's
+        const bool from_initial = flags[i];
+        const float hp = from_initial ? h0 : v.hp, t = dh * (1.0f - v.z);
+        const float gz = t * (hp - v.n) * v.z;
+        const float gn = t * (1.0f - v.n * v.n);
+        const float gr = gn * v.npp * v.r * (1.0f - v.r);
+        const float gnr = gn * v.r;
+        g[N & 1][u] = gr; g[N & 1][H + u] = gz; g[N & 1][2 * H + u] = gn;
+        const float sum = product_sum3<H>(R, gr, gz, gnr, p);
+        carry = from_initial ? 0.f : dh * v.z + sum;
+        if (want_w) {
+            to_g[0] = gr; to_g[H] = gz; to_g[2 * H] = gn; *to_gnr = gnr; *to_hp = hp;
+            to_g -= 3 * stride; to_gnr -= stride; to_hp -= stride;
+            // the reference drops reset samples from the b_hn gradient, but for the sequence's first step (their buffer rows are zeroed before that sum, gru/operations_generic.h:716-749)
+            db_hn += from_initial && i + 1 < S ? 0.f : gnr;
         }
-        rlt_lds_barrier();
-    }
-    if (P.want_w && p == 0) G.db_hn[(size_t)b * H + u] = db_hn;
+    });
+    if (want_w && p == 0) G.db_hn[(size_t)b * H + u] = db_hn;
 }
 template <int H>
 __device__ __forceinline__ void backward_row(const Backward& P, int b, char* lds) {
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), u = lane & (H - 1), p = lane / H, S = P.S;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), u = lane & (H - 1), p = lane / H, S = P.S, out4 = (P.out + 3) & ~3;
     BackwardSlots<H>& L = *reinterpret_cast<BackwardSlots<H>*>(lds);
+    // the loss gradient and the reset flags, from the last step on
     float* const ds = reinterpret_cast<float*>(lds + ((sizeof(BackwardSlots<H>) + 15) & ~(size_t)15));
-    uint8_t* const flags = reinterpret_cast<uint8_t*>(ds + (size_t)S * P.out);
-    for (int i = threadIdx.x; i < S * P.out; i += THREADS) { const int t = i / P.out; ds[i] = P.d_output[((size_t)t * P.B + b) * P.out + (i - t * P.out)]; }
-    for (int t = threadIdx.x; t < S; t += THREADS) flags[t] = t == 0 || (P.reset && P.reset[(size_t)t * P.B + b]);
+    uint8_t* const flags = reinterpret_cast<uint8_t*>(ds + (size_t)S * out4);
+    for (int e = threadIdx.x; e < S * out4; e += 64 * BACKWARD_STAGES) { const int i = e / out4, o = e - i * out4; ds[e] = o < P.out ? P.d_output[((size_t)(S - 1 - i) * P.B + b) * P.out + o] : 0.f; }
+    for (int i = threadIdx.x; i < S; i += 64 * BACKWARD_STAGES) flags[i] = i == S - 1 || (P.reset && P.reset[(size_t)(S - 1 - i) * P.B + b]);
     rlt_lds_barrier();
-    if (wave == 0) recurrence_back<H, true>(P, 1, 0, ds, nullptr, L.own[1], L.g2, flags, b, lane);
-    else if (wave == 1) {
+    // ticks behind the first stage: 2 (second recurrence), 3, 5 (first recurrence), 6, 7
+    if (wave == 0) {
+        float w3[MAX_OUT];
+#pragma unroll
+        for (int o = 0; o < MAX_OUT; o++) w3[o] = o < P.out ? P.W3[(size_t)o * H + u] : 0.f;
+        const int out = P.out;
+        const float* row = ds;
+        stage<2>(S, 0, BACKWARD_STAGES + 1, [&](auto d, int) {
+            const floatx4* x = reinterpret_cast<const floatx4*>(row);
+            float s = 0.f;
+#pragma unroll
+            for (int q = 0; q < MAX_OUT / 4; q++)
+                if (q == 0 || 4 * q < out) { const floatx4 v = x[q]; s += v[0] * w3[4 * q]; s += v[1] * w3[4 * q + 1]; s += v[2] * w3[4 * q + 2]; s += v[3] * w3[4 * q + 3]; }
+            row += out4;
+            L.dy2[decltype(d)::value & 1][u] = s;
+        });
+    }
+    else if (wave == 1) recurrence_back<H>(P, 1, 2, L.dy2, L.g2, flags, b, lane);
+    else if (wave == 2) {
         Weights3<H> R;
         load_columns3<H>(P.g[1].W_i, u, p, R);
-        for (int tick = 0; tick < S + STAGES - 1; tick++) {
-            const int t = S - 1 - (tick - 1);
-            if (t >= 0 && t < S) { const float d = product_sum3<H>(R, L.g2[t & 1], p); if (p == 0) L.dy1[t & 1][u] = d; }
-            rlt_lds_barrier();
-        }
+        stage<2>(S, 3, 4, [&](auto d, int) {
+            constexpr int PAR = decltype(d)::value & 1;
+            L.dy1[PAR][u] = product_sum3<H>(R, L.g2[PAR][u], L.g2[PAR][H + u], L.g2[PAR][2 * H + u], p);
+        });
     }
-    else if (wave == 2) recurrence_back<H, false>(P, 0, 2, nullptr, L.dy1, L.own[0], L.g1, flags, b, lane);
-    else if (wave == 3) {
+    else if (wave == 3) recurrence_back<H>(P, 0, 5, L.dy1, L.g1, flags, b, lane);
+    else if (wave == 4) {
         Weights3<H> R;
         load_columns3<H>(P.g[0].W_i, u, p, R);
-        constexpr int DEPTH = 4;
-        float queue[DEPTH];
-        auto request = [&](int t) { return P.pre0[((size_t)(t > 0 ? t : 0) * P.B + b) * H + u]; };
+        float queue[AHEAD];
+        const size_t stride = (size_t)P.B * H, last = (size_t)(S - 1) * stride + (size_t)b * H + u;
+        const float* from = P.pre0 + last;
+        float* to = P.want_w ? P.d_pre0 + last : nullptr;
+        const int act0 = P.act0;
+        auto request = [&](int i, float& v) { if (i < S) { v = *from; from -= stride; } };
 #pragma unroll
-        for (int d = 0; d < DEPTH; d++) queue[d] = request(S - 1 - d);
-        for (int tick = 0; tick < S + STAGES - 1; tick++) {
-            const int t = S - 1 - (tick - 3);
-            if (t >= 0 && t < S) {
-                const float pre = queue[0];
-#pragma unroll
-                for (int d = 0; d + 1 < DEPTH; d++) queue[d] = queue[d + 1];
-                queue[DEPTH - 1] = request(t - DEPTH);
-                const float d = product_sum3<H>(R, L.g1[t & 1], p) * rlt_dact(pre, P.act0);
-                if (p == 0) L.dp0[t & 1][u] = d;
-                if (p == 0 && P.want_w) P.d_pre0[((size_t)t * P.B + b) * H + u] = d;
-            }
-            rlt_lds_barrier();
-        }
+        for (int d = 0; d < AHEAD; d++) request(d, queue[d]);
+        stage<AHEAD>(S, 6, 1, [&](auto d, int i) {
+            constexpr int N = decltype(d)::value, PAR = N & 1;
+            const float pre = queue[N];
+            request(i + AHEAD, queue[N]);
+            const float v = product_sum3<H>(R, L.g1[PAR][u], L.g1[PAR][H + u], L.g1[PAR][2 * H + u], p) * rlt_dact(pre, act0);
+            L.dp0[PAR][u] = v;
+            if (to) { *to = v; to -= stride; }
+        });
     } else {
         float w0[H];
         const int k = min(lane, P.in - 1);
@@ -363,20 +396,20 @@ __device__ __forceinline__ void backward_row(const Backward& P, int b, char* lds
 #pragma unroll
             for (int j = 0; j < H; j++) w0[j] = P.W0[(size_t)j * P.in + k];
         }
-        for (int tick = 0; tick < S + STAGES - 1; tick++) {
-            const int t = S - 1 - (tick - 4);
-            if (P.d_input && t >= 0 && t < S) {
-                const floatx4* d = reinterpret_cast<const floatx4*>(L.dp0[t & 1]);
-                float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
+        const size_t stride = (size_t)P.B * P.in;
+        float* to = P.d_input ? P.d_input + (size_t)(S - 1) * stride + (size_t)b * P.in + k : nullptr;
+        stage<2>(S, 7, 0, [&](auto dd, int) {
+            if (!to) return;
+            const floatx4* d = reinterpret_cast<const floatx4*>(L.dp0[decltype(dd)::value & 1]);
+            float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
 #pragma unroll
-                for (int q = 0; q < H / 4; q++) { const floatx4 v = d[q]; a0 += v[0] * w0[4 * q]; a1 += v[1] * w0[4 * q + 1]; a2 += v[2] * w0[4 * q + 2]; a3 += v[3] * w0[4 * q + 3]; }
-                if (lane < P.in) P.d_input[((size_t)t * P.B + b) * P.in + lane] = (a0 + a1) + (a2 + a3);
-            }
-            rlt_lds_barrier();
-        }
+            for (int q = 0; q < H / 4; q++) { const floatx4 v = d[q]; a0 += v[0] * w0[4 * q]; a1 += v[1] * w0[4 * q + 1]; a2 += v[2] * w0[4 * q + 2]; a3 += v[3] * w0[4 * q + 3]; }
+            *to = (a0 + a1) + (a2 + a3);
+            to -= stride;
+        });
     }
 }
-__global__ __launch_bounds__(THREADS) void seq_stack_backward_kernel(BackwardLaunch K) {
+__global__ __launch_bounds__(64 * BACKWARD_STAGES) void seq_stack_backward_kernel(BackwardLaunch K) {
     extern __shared__ __attribute__((aligned(16))) char lds_stack[];
     int k = 0;
     if (K.n > 1 && (int)blockIdx.x >= K.pass[1].first_block) k = 1;
@@ -440,8 +473,8 @@ __global__ __launch_bounds__(256) void seq_gradient_finish_kernel(JobLaunch K) {
 }
 
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
-size_t forward_lds(int H, int in, int S) { return (H == 32 ? sizeof(ForwardSlots<32>) : sizeof(ForwardSlots<16>)) + 16 + (size_t)S * ((in + 3) & ~3) * sizeof(float) + S; }
-size_t backward_lds(int H, int out, int S) { return (H == 32 ? sizeof(BackwardSlots<32>) : sizeof(BackwardSlots<16>)) + 16 + (size_t)S * out * sizeof(float) + S; }
+size_t forward_lds(int H, int in, int S) { return (H == 32 ? sizeof(ForwardSlots<32>) : sizeof(ForwardSlots<16>)) + 16 + (size_t)S * ((in + 3) & ~3) * sizeof(float) + S + 1; }
+size_t backward_lds(int H, int out, int S) { return (H == 32 ? sizeof(BackwardSlots<32>) : sizeof(BackwardSlots<16>)) + 16 + (size_t)S * ((out + 3) & ~3) * sizeof(float) + S; }
 }  // namespace
 
 bool rlt_seq_stack_supported(const rlt_seq_layer* L, int n, int steps) {
@@ -478,7 +511,7 @@ int rlt_seq_stack_forward(rlt_rocm_device* device, const rlt_stack_forward* pass
         const size_t need = forward_lds(P.H, P.in, P.S);
         lds = need > lds ? need : lds;
     }
-    hipLaunchKernelGGL(seq_stack_forward_kernel, dim3(blocks), dim3(THREADS), lds, device->stream, K);
+    hipLaunchKernelGGL(seq_stack_forward_kernel, dim3(blocks), dim3(64 * FORWARD_STAGES), lds, device->stream, K);
     return rlt_launch_status(device);
 }
 
@@ -537,7 +570,7 @@ int rlt_seq_stack_backward(rlt_rocm_device* device, const rlt_stack_backward* pa
         if ((rc = rlt_scratch(device, (size_t)SPLITS * J.elements * sizeof(float), &scratch))) return rc;
         J.partial = (float*)scratch;
     }
-    hipLaunchKernelGGL(seq_stack_backward_kernel, dim3(blocks), dim3(THREADS), lds, device->stream, K);
+    hipLaunchKernelGGL(seq_stack_backward_kernel, dim3(blocks), dim3(64 * BACKWARD_STAGES), lds, device->stream, K);
     if ((rc = rlt_launch_status(device)) || !J.n) return rc;
     hipLaunchKernelGGL(seq_gradient_kernel, dim3(job_blocks * SPLITS), dim3(64 * WAVES), 0, device->stream, J);
     if ((rc = rlt_launch_status(device))) return rc;
