@@ -54,8 +54,10 @@ template <bool FAST> __device__ __forceinline__ float gate_tanh(float x) { retur
 // have units 0-15 in their lanes and the last two units 16-31, each row forms its units' three sums over that half of the reduction index, and the halves meet across the
 // rows. At width 16 the rows of lanes are the three gates (and nothing): each forms its gate's sums over all sixteen units.
 // (The control in the multiply-add itself: left to the compiler, each broadcast is an instruction of its own. The data of such an operand must have been written two wait
-// states before it is read: wait_for_dpp() stands between.)
+// states before it is read, which the compiler does not see to inside an asm statement: wait_for_dpp() stands between, and what it has passed is all that is multiplied.
+// tests/test_dpp_wait_states.py looks the built instructions over.)
 __device__ __forceinline__ void wait_for_dpp(float& x) { asm volatile("s_nop 1" : "+v"(x)); }
+__device__ __forceinline__ void wait_for_dpp(float& x, float& y, float& z) { asm volatile("s_nop 1" : "+v"(x), "+v"(y), "+v"(z)); }
 template <int K> __device__ __forceinline__ void broadcast_fma(float& acc, float x, float w) {
     if (K < 0) return;
     asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(x), "v"(w), "n"(K < 0 ? 0 : K));
@@ -84,9 +86,9 @@ __device__ __forceinline__ void load_columns3(const float* W, int u, int p, Weig
         for (int q = 0; q < 16; q++) R.w[k][q] = H == 32 ? W[(size_t)(k * H + p * 16 + q) * H + u] : (p < 3 ? W[(size_t)(p * H + q) * H + u] : 0.f);
 }
 __device__ __forceinline__ float half_in_rows(float v, int p) { float w = v; swap16(v, w); return p ? w : v; }
+// (x, y, z have passed wait_for_dpp)
 template <int H, int... Q>
-__device__ __forceinline__ void multiply(const Weights3<H>& R, float x, float y, float z, float (&acc)[3], std::integer_sequence<int, Q...>) {
-    wait_for_dpp(x);
+__device__ __forceinline__ void multiply(const Weights3<H>& R, const float& x, const float& y, const float& z, float (&acc)[3], std::integer_sequence<int, Q...>) {
     if (H == 32) {
         acc[0] = broadcast_first(x, R.w[0][0]); acc[1] = broadcast_first(y, R.w[H == 32 ? 1 : 0][0]); acc[2] = broadcast_first(z, R.w[H == 32 ? 2 : 0][0]);
         ((broadcast_fma<Q + 1>(acc[0], x, R.w[0][Q + 1]), broadcast_fma<Q + 1>(acc[1], y, R.w[H == 32 ? 1 : 0][Q + 1]), broadcast_fma<Q + 1>(acc[2], z, R.w[H == 32 ? 2 : 0][Q + 1])), ...);
@@ -101,7 +103,8 @@ __device__ __forceinline__ void multiply(const Weights3<H>& R, float x, float y,
 template <int H>
 __device__ __forceinline__ void products3(const Weights3<H>& R, float v, int p, float& rz, float& n) {
     float acc[3];
-    const float x = H == 32 ? half_in_rows(v, p) : v;
+    float x = H == 32 ? half_in_rows(v, p) : v;
+    wait_for_dpp(x);
     multiply<H>(R, x, x, x, acc, std::make_integer_sequence<int, 15>{});
     if (H == 32) {
         swap32(acc[0], acc[1]);
@@ -120,11 +123,13 @@ __device__ __forceinline__ float product_sum3(const Weights3<H>& R, float x, flo
     float acc[3];
     if (H == 32) {
         x = half_in_rows(x, p); y = half_in_rows(y, p); z = half_in_rows(z, p);
-        wait_for_dpp(y); wait_for_dpp(z);
+        wait_for_dpp(x, y, z);
         multiply<H>(R, x, y, z, acc, std::make_integer_sequence<int, 15>{});
         return sum_parts<2>(acc[0] + (acc[1] + acc[2]));
     }
-    multiply<H>(R, p == 0 ? x : p == 1 ? y : z, 0.f, 0.f, acc, std::make_integer_sequence<int, 15>{});
+    float own = p == 0 ? x : p == 1 ? y : z;
+    wait_for_dpp(own);
+    multiply<H>(R, own, own, own, acc, std::make_integer_sequence<int, 15>{});
     return sum_parts<4>(acc[0]);
 }
 
