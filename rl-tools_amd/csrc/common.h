@@ -112,9 +112,12 @@ __device__ __forceinline__ float rlt_dact_from_output(float o, int f) {
 }
 
 // Workgroup barrier that orders LDS traffic only. __syncthreads() also waits for every global load and store the wavefront has in
-// flight, which defeats prefetching across a barrier; kernels whose wavefronts exchange data through LDS alone use this one.
+// flight, which defeats prefetching across a barrier; kernels whose wavefronts exchange data through LDS alone use this one. The wait for this wavefront's LDS
+// operations is written out: the compiler drops the one that the fence stands for where the barrier opens a loop and nothing is outstanding on the way into it, although
+// the loop's own writes are on the way round (tests/test_barrier_waits.py).
 __device__ __forceinline__ void rlt_lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_waitcnt(0xC07F);      // lgkmcnt(0)
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }

@@ -12,6 +12,7 @@
 //     gradients and d_input are then three contractions over sequence*batch rows.
 #include "common.h"
 #include "gemm.h"
+#include <utility>
 
 namespace {
 
@@ -276,171 +277,205 @@ __global__ __launch_bounds__(GRU_THREADS) void gru_backward_reg_kernel(GruArgs A
 }
 
 // ---- hidden width 64: the recurrence on the matrix cores -------------------------------------------------------------------------
-// A workgroup of four wavefronts carries FOUR batch rows through the sequence; W_h stays in registers as the B operand of
-// v_mfma_f32_4x4x1_16b_f32 (16 blocks of a 4 x 1 by 1 x 4 product: lane 4 blk + i supplies A[i], lane 4 blk + j supplies B[j], register i of
-// lane 4 blk + j receives D[i][j]; with the broadcast control set to 16 blocks every block takes its A from the block the instruction names,
-// so one register of previous hidden states feeds 16 reduction steps). The four rows are the A side (i = row), a block is one hidden unit and
-// its four columns are that unit's r, z and n gates (the fourth is idle): 64 instructions of 8 cycles replace the 192 multiply-adds and 64
-// lane reads per lane of the vector version, and a step takes about half its time at any batch size (the chain of dependent steps, not the
-// arithmetic, bounds both).
-// The gates at this width on the hardware's exponential and reciprocal (v_exp_f32, v_rcp_f32: 1 ulp each; absolute error of a gate below 3e-7, an order
-// below the tolerance the layer is held to): the library routines cost 500 cycles of every step's 1,900, these 300.
-__device__ __forceinline__ float hw_sigmoid(float x) { return __frcp_rn(1.0f + __expf(-x)); }
-__device__ __forceinline__ float hw_tanh(float x) { return 1.0f - 2.0f * __frcp_rn(__expf(2.0f * x) + 1.0f); }
+// A workgroup of four wavefronts carries FOUR batch rows through the sequence; wavefront w owns hidden units 16 w ... 16 w + 15, W_h stays in
+// registers as the B operand of v_mfma_f32_4x4x1_16b_f32 (16 blocks of a 4 x 1 by 1 x 4 product: lane 4 blk + i supplies A[i], lane 4 blk + j
+// supplies B[j], register i of lane 4 blk + j receives D[i][j]; with the broadcast control set to 4 blocks every block of a group of four takes
+// its A from the group's block that the instruction names). The four rows are the A side. Block 4 kg + cg takes columns 4 cg ... 4 cg + 3 of the
+// wavefront's sixteen and quarter kg of the reduction, so all four columns of every block work: 48 instructions of 8 cycles for the 4 x 192 x 64
+// products (with a block per unit and its gates as columns the fourth column is idle: 64). The quarters' sums meet in three lane exchanges and
+// three additions that leave row kg in the lanes of group kg: lane = (row, unit) finishes its unit with no trip through LDS.
+//
+// Bound: the chain of a step -- barrier and one 16-byte LDS read (the state, in the order of the A operand), the matrix instructions, the lane
+// exchanges, the gates -- at any batch size up to one workgroup per compute unit. What a step reads from memory is requested D steps ahead into
+// registers that the unrolled loop names: as a queue whose entries move up, the compiler waits for every step's own request (and all stores
+// before it) at that step's end. 64 steps at batch 64: forward 50.4 -> 35.9 us, backward 52.7 -> 35.3 us (batch 1,024: 56.4 -> 41.4 and 56.1 -> 43.8).
+//
+// The gates at this width on the hardware's exponential and reciprocal (v_exp_f32, v_rcp_f32: 1 ulp each; the reciprocal corrected by one
+// Newton step; absolute error of a gate below 3e-7, an order below the tolerance the layer is held to): the library routines cost 500 cycles of
+// a step, these 150.
+__device__ __forceinline__ float corrected_rcp(float d) {      // 1 / d for d >= 1; infinite d gives 0, a NaN stays one
+    const float q = __builtin_amdgcn_rcpf(d), better = fmaf(fmaf(-d, q, 1.0f), q, q);
+    return d == INFINITY ? 0.0f : better;
+}
+__device__ __forceinline__ float hw_sigmoid(float x) { return corrected_rcp(1.0f + __expf(-x)); }
+__device__ __forceinline__ float hw_tanh(float x) { return fmaf(-2.0f, corrected_rcp(__expf(2.0f * x) + 1.0f), 1.0f); }
 typedef float gru_floatx4 __attribute__((ext_vector_type(4)));
 constexpr int GM_ROWS = 4;
-template <int ABID> __device__ __forceinline__ gru_floatx4 mfma4(float a, float b, gru_floatx4 c) { return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 4, ABID, 0); }
-// 16 reduction steps: A register `a` holds, in block blk, the four rows' values of reduction index base + blk
-__device__ __forceinline__ void mfma4_16(float a, const float* w, gru_floatx4& c0, gru_floatx4& c1, gru_floatx4& c2, gru_floatx4& c3) {
-    c0 = mfma4<0>(a, w[0], c0); c1 = mfma4<1>(a, w[1], c1); c2 = mfma4<2>(a, w[2], c2); c3 = mfma4<3>(a, w[3], c3);
-    c0 = mfma4<4>(a, w[4], c0); c1 = mfma4<5>(a, w[5], c1); c2 = mfma4<6>(a, w[6], c2); c3 = mfma4<7>(a, w[7], c3);
-    c0 = mfma4<8>(a, w[8], c0); c1 = mfma4<9>(a, w[9], c1); c2 = mfma4<10>(a, w[10], c2); c3 = mfma4<11>(a, w[11], c3);
-    c0 = mfma4<12>(a, w[12], c0); c1 = mfma4<13>(a, w[13], c1); c2 = mfma4<14>(a, w[14], c2); c3 = mfma4<15>(a, w[15], c3);
+template <int ABID> __device__ __forceinline__ gru_floatx4 mfma4(float a, float b, gru_floatx4 c) { return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 2, ABID, 0); }
+// The four quarters of the reduction added up: c[row] of a lane in group kg (lanes 16 kg ...) is row `row`'s sum over quarter kg; the result is row kg's sum over all of them
+__device__ __forceinline__ float sum_quarters(gru_floatx4 c) {
+    auto across = [](float a, float b, auto swap) { const auto s = swap(__float_as_uint(a), __float_as_uint(b)); return __uint_as_float(s[0]) + __uint_as_float(s[1]); };
+    auto swap32 = [](unsigned a, unsigned b) { return __builtin_amdgcn_permlane32_swap(a, b, false, false); };
+    auto swap16 = [](unsigned a, unsigned b) { return __builtin_amdgcn_permlane16_swap(a, b, false, false); };
+    return across(across(c[0], c[2], swap32), across(c[1], c[3], swap32), swap16);
+}
+// The steps of a sequence in groups of D whose members know their number in the group (a queue's entries are indexed by it). Whole groups are straight-line code: with an
+// exit before every step the compiler waits for all requests where the paths meet. For the same reason everything requested before the loop is waited for in front of it: the
+// first step of a group then waits for its own values, requested D steps before, and not for the last ones.
+template <class F, int... K> __device__ __forceinline__ void gru_whole_group(int first, F& step, std::integer_sequence<int, K...>) { (step(std::integral_constant<int, K>{}, first + K), ...); }
+template <class F, int... K> __device__ __forceinline__ void gru_rest(int first, int S, F& step, std::integer_sequence<int, K...>) { ((first + K < S ? step(std::integral_constant<int, K>{}, first + K) : (void)0), ...); }
+template <int D, class F>
+__device__ __forceinline__ void gru_steps(int S, F&& step) {
+    int i = 0;
+    __builtin_amdgcn_s_waitcnt(0x0F70);      // vmcnt(0)
+    for (; i + D <= S; i += D) gru_whole_group(i, step, std::make_integer_sequence<int, D>{});
+    gru_rest(i, S, step, std::make_integer_sequence<int, D - 1>{});
 }
 
-// Wavefront w owns hidden units 16 w ... 16 w + 15. hs (two copies, by the parity of the step) holds the previous hidden state of the four rows,
-// unit-major: hs[unit * 4 + row]. One workgroup barrier per step; the pre-activations pass from the matrix layout (lane = unit, gate; register =
-// row) to the lane that finishes (row, unit) through a slot of LDS private to the wavefront.
-template <bool FAST>
-__global__ __launch_bounds__(256) void gru_forward_mfma_kernel(GruArgs A) {
-    constexpr int H = 64;
-    __shared__ __align__(16) float hs[2][H * GM_ROWS];
-    __shared__ __align__(16) float xw[4][GM_ROWS * 64];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, blk = lane >> 2, j = lane & 3;
-    // B operand: column j of block blk = gate j of unit 16 w + blk, one register per reduction index
-    float wb[H];
-    {
-        const float4* src = reinterpret_cast<const float4*>(A.L.weights_hidden + ((size_t)(j < 3 ? j : 0) * H + 16 * w + blk) * H);
+// Reset flags of 64 consecutive steps from `first` on, as a mask in every lane of the row's group (bit i: step first + i starts an episode); steps from S on: no. A wavefront
+// reads a step per lane: a byte load per step would hold the recurrence up for its widening.
+__device__ __forceinline__ uint64_t gru_reset_flags(const uint8_t* reset, int first, int S, int B, int b0, int kg) {
+    if (!reset) return 0;
+    const int t = first + (int)(threadIdx.x & 63);
+    uint64_t mask = 0;
 #pragma unroll
-        for (int q = 0; q < H / 4; q++) {
-            const float4 v = src[q];
-            wb[4 * q] = j < 3 ? v.x : 0.f; wb[4 * q + 1] = j < 3 ? v.y : 0.f; wb[4 * q + 2] = j < 3 ? v.z : 0.f; wb[4 * q + 3] = j < 3 ? v.w : 0.f;
-        }
+    for (int r = 0; r < GM_ROWS; r++) {
+        const uint64_t row = __ballot(t < S && reset[(size_t)min(t, S - 1) * B + min(b0 + r, B - 1)] != 0);
+        mask = kg == r ? row : mask;
     }
-    // the lane that finishes (row, unit)
-    const int row_local = lane >> 4, u = 16 * w + (lane & 15);
-    const int b_raw = blockIdx.x * GM_ROWS + row_local;
-    const bool live = b_raw < A.B;
-    const int b = live ? b_raw : A.B - 1;      // rows beyond the batch read the last row and store nothing
+    return mask;
+}
+__device__ __forceinline__ float& gru_at(float* base, unsigned bytes) { return *reinterpret_cast<float*>(reinterpret_cast<char*>(base) + bytes); }
+
+// hs (two copies, by the parity of the step): the previous hidden state of the four rows in the order of the A operand: group kg's lane (cg, row) reads
+// units 16 kg + 4 s + cg, s = 0 ... 3, in one 16-byte read. One workgroup barrier per step. Lane = (row kg, unit) finishes its unit; rows beyond the batch repeat the last
+// row (the same wavefront's lanes hold it: they read, compute and store the same values). Memory is addressed by pointers of the workgroup that move from step to step and
+// the lane's place within four rows.
+template <bool FAST>
+__global__ __launch_bounds__(256, 2) void gru_forward_mfma_kernel(GruArgs A) {
+    constexpr int H = 64, D = 4;
+    __shared__ __align__(16) float hs[2][H * GM_ROWS];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kg = lane >> 4, c16 = lane & 15, u = 16 * w + c16;
+    // B operand: column c16 (unit u) of gate g, reduction index 16 kg + 4 s + abid = 16 kg + k
+    float wb[3][16];
+#pragma unroll
+    for (int g = 0; g < 3; g++) {
+        const float4* src = reinterpret_cast<const float4*>(A.L.weights_hidden + (size_t)(g * H + u) * H + 16 * kg);
+#pragma unroll
+        for (int q = 0; q < 4; q++) { const float4 v = src[q]; wb[g][4 * q] = v.x; wb[g][4 * q + 1] = v.y; wb[g][4 * q + 2] = v.z; wb[g][4 * q + 3] = v.w; }
+    }
+    const int b0 = blockIdx.x * GM_ROWS, row = min(kg, A.B - 1 - b0);
+    const unsigned at = (row * H + u) * sizeof(float), at3 = (row * 3 * H + u) * sizeof(float);
     const float bhr = A.L.biases_hidden[u], bhz = A.L.biases_hidden[H + u], bhn = A.L.biases_hidden[2 * H + u];
     const float h0 = A.L.initial_hidden_state[u];
-    const size_t stride = (size_t)A.B * 3 * H;
-    // The inputs W_i x + b_i (and the reset flag) of step t + D are requested during step t and wait in a queue: consecutive steps lie 12 H B bytes
-    // apart, and a load takes longer than a step.
-    constexpr int D = 4;
-    struct In { float r, z, n; int rs; };
-    auto request = [&](int t) {
-        const int tc = t < A.S ? t : A.S - 1;       // the last steps request the last one again: no branch around the loads
-        const float* p = A.L.post_activation + (size_t)tc * stride + (size_t)b * 3 * H;
-        In v; v.r = p[u]; v.z = p[H + u]; v.n = p[2 * H + u]; v.rs = A.reset ? A.reset[(size_t)tc * A.B + b] : 0;
-        return v;
+    const size_t stride = (size_t)A.B * H;
+    float* post = A.L.post_activation + (size_t)b0 * 3 * H; float* npp = A.L.n_pre_pre_activation + (size_t)b0 * H; float* out = A.L.output + (size_t)b0 * H;
+    struct In { float r, z, n; };
+    float* in = post;
+    auto request = [&](int t, In& v) {      // in the order of the steps; the last steps request the last one again: no branch around the loads
+        v.r = gru_at(in, at3); v.z = gru_at(in + H, at3); v.n = gru_at(in + 2 * H, at3);
+        in += t + 1 < A.S ? 3 * stride : 0;
     };
     In q[D];
 #pragma unroll
-    for (int d = 0; d < D; d++) q[d] = request(d);
+    for (int d = 0; d < D; d++) request(d, q[d]);
+    const int place = ((4 * w + (c16 & 3)) * 4 + kg) * 4 + (c16 >> 2);      // this (row, unit) in hs
     float h = h0;
-    hs[0][u * GM_ROWS + row_local] = h;
-    for (int t = 0; t < A.S; t++) {
-        rlt_lds_barrier();
-        const float* hp = hs[t & 1];
-        const float a0 = hp[lane], a1 = hp[64 + lane], a2 = hp[128 + lane], a3 = hp[192 + lane];
-        const In far = request(t + D);
-        gru_floatx4 c0 = {0.f, 0.f, 0.f, 0.f}, c1 = c0, c2 = c0, c3 = c0;
-        mfma4_16(a0, wb, c0, c1, c2, c3); mfma4_16(a1, wb + 16, c0, c1, c2, c3); mfma4_16(a2, wb + 32, c0, c1, c2, c3); mfma4_16(a3, wb + 48, c0, c1, c2, c3);
-        const gru_floatx4 c = (c0 + c1) + (c2 + c3);
-        float* x = xw[w];
-        x[lane] = c[0]; x[64 + lane] = c[1]; x[128 + lane] = c[2]; x[192 + lane] = c[3];      // x[(row * 16 + unit) * 4 + gate]
-        wave_sync();
-        const float4 pre = *reinterpret_cast<const float4*>(x + 4 * lane);
-        wave_sync();
-        const float ar = bhr + pre.x, az = bhz + pre.y, an = bhn + pre.z;
-        const float r = FAST ? gate_sigmoid(q[0].r + ar, 1) : hw_sigmoid(q[0].r + ar), z = FAST ? gate_sigmoid(q[0].z + az, 1) : hw_sigmoid(q[0].z + az);
-        const float n = FAST ? gate_tanh(q[0].n + an * r, 1) : hw_tanh(q[0].n + an * r);
-        h = (1.0f - z) * n + z * h;
-        if (live) {
-            float* po = A.L.post_activation + (size_t)t * stride + (size_t)b * 3 * H;
-            po[u] = r; po[H + u] = z; po[2 * H + u] = n;
-            const size_t at = ((size_t)t * A.B + b) * H + u;
-            A.L.n_pre_pre_activation[at] = an;
-            A.L.output[at] = h;
-        }
-        if (t + 1 < A.S && q[1].rs) h = h0;       // the next step starts an episode
-        hs[(t + 1) & 1][u * GM_ROWS + row_local] = h;
-#pragma unroll
-        for (int d = 0; d + 1 < D; d++) q[d] = q[d + 1];
-        q[D - 1] = far;
+    hs[0][place] = h;
+    for (int first = 0; first < A.S; first += 64) {
+        uint64_t flags = gru_reset_flags(A.reset, first + 1, A.S, A.B, b0, kg);      // of the steps after these
+        gru_steps<D>(min(64, A.S - first), [&](auto number, int i) {
+            constexpr int N = decltype(number)::value;
+            __builtin_amdgcn_sched_barrier(0);      // later steps' values are not touched (and waited for) before their step
+            rlt_lds_barrier();
+            const float4 a = *reinterpret_cast<const float4*>(&hs[N & 1][4 * lane]);
+            const float xr = q[N].r + bhr, xz = q[N].z + bhz, xn = q[N].n;
+            gru_floatx4 cr = {0.f, 0.f, 0.f, 0.f}, cz = cr, cn = cr;
+#define RLT_GRU_STEPS(X, s) \
+            cr = mfma4<0>(X, wb[0][4 * s], cr); cn = mfma4<0>(X, wb[2][4 * s], cn); cz = mfma4<0>(X, wb[1][4 * s], cz); \
+            cr = mfma4<1>(X, wb[0][4 * s + 1], cr); cn = mfma4<1>(X, wb[2][4 * s + 1], cn); cz = mfma4<1>(X, wb[1][4 * s + 1], cz); \
+            cr = mfma4<2>(X, wb[0][4 * s + 2], cr); cn = mfma4<2>(X, wb[2][4 * s + 2], cn); cz = mfma4<2>(X, wb[1][4 * s + 2], cz); \
+            cr = mfma4<3>(X, wb[0][4 * s + 3], cr); cn = mfma4<3>(X, wb[2][4 * s + 3], cn); cz = mfma4<3>(X, wb[1][4 * s + 3], cz);
+            RLT_GRU_STEPS(a.x, 0) RLT_GRU_STEPS(a.y, 1) RLT_GRU_STEPS(a.z, 2) RLT_GRU_STEPS(a.w, 3)
+#undef RLT_GRU_STEPS
+            const float ar = xr + sum_quarters(cr), an = bhn + sum_quarters(cn), az = xz + sum_quarters(cz);
+            const float r = FAST ? gate_sigmoid(ar, 1) : hw_sigmoid(ar), z = FAST ? gate_sigmoid(az, 1) : hw_sigmoid(az);
+            const float n = FAST ? gate_tanh(xn + an * r, 1) : hw_tanh(xn + an * r);
+            const float o = (1.0f - z) * n + z * h;
+            h = flags & 1 ? h0 : o;       // the next step starts an episode
+            flags >>= 1;
+            hs[(N + 1) & 1][place] = h;
+            gru_at(post, at3) = r; gru_at(post + H, at3) = z; gru_at(post + 2 * H, at3) = n; gru_at(npp, at) = an; gru_at(out, at) = o;
+            post += 3 * stride; npp += stride; out += stride;
+            request(first + i + D, q[N]);      // behind the last use of the entry: before it, the loop would start with copies of all entries, and with waits for them
+        });
     }
 }
 
-// Reverse pass. The gate gradients of the four rows are the A side, the reduction runs over the 192 (gate, unit) pairs -- a quarter per
-// wavefront, whose B operands are rows 48 w ... 48 w + 47 of W_h (lane = column: coalesced) -- and the four partial sums of d h_prev meet in
-// LDS. Thread (w, lane) finishes (row w, unit lane): its loads and stores are whole rows. Two workgroup barriers per step.
-__global__ __launch_bounds__(256) void gru_backward_mfma_kernel(GruArgs A) {
-    constexpr int H = 64, GS = 3 * H + 16;      // row stride of the gate gradients in LDS: rows 16 banks apart
-    __shared__ float gs[GM_ROWS * GS];
-    __shared__ float part[4][GM_ROWS * 64];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, blk = lane >> 2, i = lane & 3;
+// Reverse pass: the gate gradients of the four rows are the A side (192 reduction indices, quarter kg = the 48 of wavefront kg's units), a wavefront forms d h_prev of
+// its sixteen units. gs (two copies, by the parity of the step): lane (kg, cg, row) of the A operand reads its twelve values in three 16-byte reads (neighbours lie 12
+// floats apart: no two of a group share a bank). One workgroup barrier per step; lane = (row, unit) and addresses as in the forward pass.
+__global__ __launch_bounds__(256, 2) void gru_backward_mfma_kernel(GruArgs A) {
+    constexpr int H = 64, D = 4;
+    __shared__ __align__(16) float gs[2][3 * H * GM_ROWS];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kg = lane >> 4, c16 = lane & 15, u = 16 * w + c16, S = A.S;
+    // B operand: column u, reduction index (gate s >> 2, unit 16 kg + 4 (s & 3) + abid)
     float wb[48];
 #pragma unroll
-    for (int k = 0; k < 48; k++) wb[k] = A.L.weights_hidden[(size_t)(48 * w + k) * H + lane];
-    const int b_raw = blockIdx.x * GM_ROWS + w;
-    const bool live = b_raw < A.B;
-    const int b = live ? b_raw : A.B - 1;
-    const int u = lane;
+    for (int s = 0; s < 12; s++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) wb[4 * s + k] = A.L.weights_hidden[(size_t)((s >> 2) * H + 16 * kg + 4 * (s & 3) + k) * H + u];
+    const int b0 = blockIdx.x * GM_ROWS, row = min(kg, A.B - 1 - b0);
+    const unsigned at = (row * H + u) * sizeof(float), at3 = (row * 3 * H + u) * sizeof(float);
     const float h0 = A.L.initial_hidden_state[u];
-    float carry = 0.f, db_hn = 0.f;
-    struct Saved { float r, z, n, npp, dy, hp; int rs; };
-    auto request = [&](int t) {
-        const size_t a = (size_t)(t > 0 ? t : 0) * A.B + b;
-        Saved v;
-        v.r = A.L.post_activation[a * 3 * H + u]; v.z = A.L.post_activation[a * 3 * H + H + u]; v.n = A.L.post_activation[a * 3 * H + 2 * H + u];
-        v.npp = A.L.n_pre_pre_activation[a * H + u]; v.dy = A.d_output[a * H + u];
-        v.hp = A.L.output[((size_t)(t > 1 ? t - 1 : 0) * A.B + b) * H + u];
-        v.rs = A.reset ? A.reset[a] : 0;
-        return v;
+    const size_t stride = (size_t)A.B * H, last = (size_t)(S - 1) * stride + (size_t)b0 * H;
+    struct Saved { float r, z, n, npp, dy, hp; };
+    float *post = A.L.post_activation + 3 * last, *npp = A.L.n_pre_pre_activation + last, *dy = A.d_output + last, *state = A.L.output + last;
+    auto request = [&](int i, Saved& v) {      // i-th step from the end; steps before the first read the first again; the state is the one before the step (the first step's is not used)
+        const size_t on = i + 1 < S ? stride : 0;
+        state -= on;
+        v.r = gru_at(post, at3); v.z = gru_at(post + H, at3); v.n = gru_at(post + 2 * H, at3); v.npp = gru_at(npp, at); v.dy = gru_at(dy, at); v.hp = gru_at(state, at);
+        post -= 3 * on; npp -= on; dy -= on;
     };
-    // a step's saved values are requested D steps ahead (a load takes longer than a step); steps before the first read the first again
-    constexpr int D = 3;
     Saved q[D];
 #pragma unroll
-    for (int d = 0; d < D; d++) q[d] = request(A.S - 1 - d);
-    for (int t = A.S - 1; t >= 0; t--) {
-        const size_t at = (size_t)t * A.B + b;
-        const Saved far = request(t - D);
-        const Saved cur = q[0];
-        const bool from_initial = t == 0 || cur.rs;
-        const float hp = from_initial ? h0 : cur.hp;
-        const float dh = cur.dy + carry;
-        const float gz = dh * (hp - cur.n) * cur.z * (1.0f - cur.z);
-        const float gn = dh * (1.0f - cur.z) * (1.0f - cur.n * cur.n);
-        const float gr = gn * cur.npp * cur.r * (1.0f - cur.r);
-        const float gnr = gn * cur.r;
-        if (live) {
-            A.d_output[at * H + u] = dh;
-            float* bi = A.buffer_input + at * 3 * H; float* bh = A.buffer_hidden + at * 3 * H;
-            bi[u] = gr; bi[H + u] = gz; bi[2 * H + u] = gn;
-            bh[u] = gr; bh[H + u] = gz; bh[2 * H + u] = gnr;
-            A.h_previous[at * H + u] = hp;
-        }
-        // the reference drops reset samples (t > 0) from the b_hn gradient (their buffer rows are zeroed before that sum, :716-749)
-        if (!(t > 0 && from_initial)) db_hn += gnr;
-        gs[w * GS + u] = gr; gs[w * GS + H + u] = gz; gs[w * GS + 2 * H + u] = gnr;
-        rlt_lds_barrier();
-        const float* ga = gs + i * GS + 48 * w + blk;
-        const float a0 = ga[0], a1 = ga[16], a2 = ga[32];
-        gru_floatx4 c0 = {0.f, 0.f, 0.f, 0.f}, c1 = c0, c2 = c0, c3 = c0;
-        mfma4_16(a0, wb, c0, c1, c2, c3); mfma4_16(a1, wb + 16, c0, c1, c2, c3); mfma4_16(a2, wb + 32, c0, c1, c2, c3);
-        const gru_floatx4 c = (c0 + c1) + (c2 + c3);
-        float* pw = part[w];
-        pw[lane] = c[0]; pw[64 + lane] = c[1]; pw[128 + lane] = c[2]; pw[192 + lane] = c[3];      // part[w][row * 64 + column]
-        rlt_lds_barrier();
-        const float sum = (part[0][w * 64 + u] + part[1][w * 64 + u]) + (part[2][w * 64 + u] + part[3][w * 64 + u]);
-        carry = from_initial ? 0.f : dh * cur.z + sum;
-#pragma unroll
-        for (int d = 0; d + 1 < D; d++) q[d] = q[d + 1];
-        q[D - 1] = far;
+    for (int d = 0; d < D; d++) request(d, q[d]);
+    float *to_dy = A.d_output + last, *to_hp = A.h_previous + last, *bi = A.buffer_input + 3 * last, *bh = A.buffer_hidden + 3 * last;
+    const int place = ((4 * w + (c16 & 3)) * 4 + kg) * 12 + (c16 >> 2);      // the r gate of this (row, unit) in gs; z and n four and eight on
+    float carry = 0.f, db_hn = 0.f;
+    for (int back = 0; back < S; back += 64) {
+        const int steps = min(64, S - back);
+        const uint64_t flags = gru_reset_flags(A.reset, S - back - steps, S, A.B, b0, kg);      // bit of step t = S - 1 - back - i: steps - 1 - i
+        uint64_t high = flags << (64 - steps);
+        gru_steps<D>(steps, [&](auto number, int i) {
+            constexpr int N = decltype(number)::value;
+            __builtin_amdgcn_sched_barrier(0);
+            const Saved cur = q[N];
+            const bool first = back + i + 1 == S, from_initial = first || (high >> 63);
+            high <<= 1;
+            const float hp = from_initial ? h0 : cur.hp;
+            const float dh = cur.dy + carry;
+            const float gz = dh * (hp - cur.n) * cur.z * (1.0f - cur.z);
+            const float gn = dh * (1.0f - cur.z) * (1.0f - cur.n * cur.n);
+            const float gr = gn * cur.npp * cur.r * (1.0f - cur.r);
+            const float gnr = gn * cur.r;
+            float through = dh * cur.z;
+            asm volatile("" : "+v"(through));      // (not formed below by a multiply-add that would keep the entry's z)
+            request(back + i + D, q[N]);      // behind the last use of the entry: before it, the loop would start with copies of all entries, and with waits for them
+            float* g = &gs[N & 1][place];
+            g[0] = gr; g[4] = gz; g[8] = gnr;
+            rlt_lds_barrier();
+            const float4* ga = reinterpret_cast<const float4*>(&gs[N & 1][12 * lane]);
+            const float4 a0 = ga[0], a1 = ga[1], a2 = ga[2];
+            gru_at(to_dy, at) = dh; gru_at(to_hp, at) = hp;
+            gru_at(bi, at3) = gr; gru_at(bi + H, at3) = gz; gru_at(bi + 2 * H, at3) = gn;
+            gru_at(bh, at3) = gr; gru_at(bh + H, at3) = gz; gru_at(bh + 2 * H, at3) = gnr;
+            to_dy -= stride; to_hp -= stride; bi -= 3 * stride; bh -= 3 * stride;
+            // the reference drops reset samples (t > 0) from the b_hn gradient (their buffer rows are zeroed before that sum, :716-749)
+            db_hn += first || !from_initial ? gnr : 0.f;
+            gru_floatx4 c0 = {0.f, 0.f, 0.f, 0.f}, c1 = c0, c2 = c0;
+#define RLT_GRU_STEPS(X, k) \
+            c0 = mfma4<0>(a0.X, wb[4 * k], c0); c1 = mfma4<0>(a1.X, wb[16 + 4 * k], c1); c2 = mfma4<0>(a2.X, wb[32 + 4 * k], c2); \
+            c0 = mfma4<1>(a0.X, wb[4 * k + 1], c0); c1 = mfma4<1>(a1.X, wb[16 + 4 * k + 1], c1); c2 = mfma4<1>(a2.X, wb[32 + 4 * k + 1], c2); \
+            c0 = mfma4<2>(a0.X, wb[4 * k + 2], c0); c1 = mfma4<2>(a1.X, wb[16 + 4 * k + 2], c1); c2 = mfma4<2>(a2.X, wb[32 + 4 * k + 2], c2); \
+            c0 = mfma4<3>(a0.X, wb[4 * k + 3], c0); c1 = mfma4<3>(a1.X, wb[16 + 4 * k + 3], c1); c2 = mfma4<3>(a2.X, wb[32 + 4 * k + 3], c2);
+            RLT_GRU_STEPS(x, 0) RLT_GRU_STEPS(y, 1) RLT_GRU_STEPS(z, 2) RLT_GRU_STEPS(w, 3)
+#undef RLT_GRU_STEPS
+            const float sum = sum_quarters(c0 + (c1 + c2));
+            carry = from_initial ? 0.f : through + sum;
+        });
     }
-    if (live && A.db_hn_partial) A.db_hn_partial[(size_t)b * H + u] = db_hn;
+    if (A.db_hn_partial) gru_at(A.db_hn_partial + (size_t)b0 * H, at) = db_hn;
 }
 
 // db_h[n part] += sum over batch rows of the per-row sums, db_h[r, z parts] = db_i[r, z parts] (the reference copies, :679-681).
