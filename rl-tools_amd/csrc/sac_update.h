@@ -54,3 +54,5 @@ int rlt_mlp_wide_backward(rlt_rocm_device* device, const rlt_dense_layer* layers
 // forward() alone, storing every layer's pre-activations and outputs (those of the layers that have the buffers) where `keep` is set, and the network's output into y
 // (optional, leading dimension ldy); any output activation
 int rlt_mlp_wide_forward(rlt_rocm_device* device, const rlt_dense_layer* layers, int n_layers, const float* x, int ldx, float* y, int ldy, int batch, bool keep);
+// allocates the buffer of these calls' weight copies (once per handle; not while a graph is recorded)
+int rlt_mlp_wide_reserve(rlt_rocm_device* device);

@@ -982,6 +982,19 @@ int rlt_td3_wide_update_actor(rlt_rocm_device* device, const rlt_td3_agent* A, c
 }
 
 
+// The weight copies of the calls below have a buffer of their own: forward() and evaluate() have never touched the handle's scratch buffer at these batch sizes, and callers hold
+// data there across them. RLT_E_CAPTURING: not there yet, and the stream records a graph.
+int rlt_mlp_wide_reserve(rlt_rocm_device* device) {
+    constexpr size_t COPY_BYTES = (2 * MAX_COPY_FLOATS + MAX_W1_COPY_FLOATS) * sizeof(float);
+    if (device->copy_scratch_bytes >= COPY_BYTES) return 0;
+    if (device->capturing) return RLT_E_CAPTURING;
+    if (device->copy_scratch) RLT_HIP(hipFree(device->copy_scratch));
+    device->copy_scratch = nullptr; device->copy_scratch_bytes = 0;
+    RLT_HIP(hipMalloc(&device->copy_scratch, COPY_BYTES));
+    device->copy_scratch_bytes = COPY_BYTES;
+    return 0;
+}
+
 // ---- forward + backward of a three-layer network on sixteen-row tiles (see mlp_wide_kernel), or the backward pass alone from the outputs that a forward() left in
 // the layers; RLT_E_UNSUPPORTED: the caller takes another path
 static int mlp_wide_launch(rlt_rocm_device* device, const rlt_dense_layer* L, int n_layers, const float* x, int ldx, float* y, int ldy,
@@ -1013,15 +1026,7 @@ static int mlp_wide_launch(rlt_rocm_device* device, const rlt_dense_layer* L, in
         partial = (float*)scratch + trained_floats(hid, batch);
         set_rows(net, a.kept, x, ldx);
     }
-    // the weight copies have a buffer of their own: forward() and evaluate() have never touched the handle's scratch buffer at these batch sizes, and callers hold data there across them
-    constexpr size_t COPY_BYTES = (2 * MAX_COPY_FLOATS + MAX_W1_COPY_FLOATS) * sizeof(float);
-    if (device->copy_scratch_bytes < COPY_BYTES) {
-        if (device->capturing) return RLT_E_CAPTURING;
-        if (device->copy_scratch) RLT_HIP(hipFree(device->copy_scratch));
-        device->copy_scratch = nullptr; device->copy_scratch_bytes = 0;
-        RLT_HIP(hipMalloc(&device->copy_scratch, COPY_BYTES));
-        device->copy_scratch_bytes = COPY_BYTES;
-    }
+    if ((rc = rlt_mlp_wide_reserve(device))) return rc;
     Copies copies((float*)device->copy_scratch);
     if (!backward_only) copies.forward(a.net);
     if (!forward_only) copies.backward(a.net);
