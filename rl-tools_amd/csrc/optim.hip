@@ -9,9 +9,14 @@
 namespace {
 
 constexpr int MAX_T = 16;
+constexpr uint32_t MAX_BLOCKS = 960 - MAX_T;      // rounding up per tensor included, the workgroups' sums for the squared norm fit the counters block
 struct AdamLaunch {
     rlt_adam_tensor t[MAX_T];
-    uint32_t prefix[MAX_T + 1];
+    // Workgroups [first_block[i], first_block[i + 1]) step tensor i, span[i] elements each: the tensor is the same for a whole workgroup and its pointers arrive with scalar loads.
+    // (As a list of elements that each lane searched for its own, every launch made another trip to the argument segment before it could ask for data: 7.4 instead of 5.6 us
+    // at 72 k parameters in six tensors.)
+    uint32_t first_block[MAX_T + 1], span[MAX_T];
+    uint32_t vec;                // bit i: tensor i is stepped four elements at a time (16-byte loads of the blocks, moments and values), but for its last one to three
     int n;
     rlt_adam_parameters p;
     float polyak;
@@ -30,8 +35,15 @@ struct AdamLaunch {
     uint32_t source_offset[MAX_T];
     float source_scale[MAX_T], source_add[MAX_T];
     float* extra_out; uint32_t extra_offset; float extra_scale;      // optional: one more sum of the blocks, stored scaled (not a gradient)
-    uint32_t vec_end;            // elements [0, vec_end) can be stepped four at a time (16-byte loads of the blocks, moments and values): see vector_end()
 };
+
+// the workgroup's tensor (the same for all of its lanes)
+__device__ __forceinline__ int tensor_of(const AdamLaunch& a, uint32_t block) {
+    int ti = 0;
+#pragma unroll
+    for (int k = 1; k < MAX_T; k++) ti += (k < a.n && block >= a.first_block[k]) ? 1 : 0;
+    return __builtin_amdgcn_readfirstlane(ti);
+}
 
 // sum over the blocks of one element, every load in flight at once where there are at most 16 blocks
 __device__ __forceinline__ float sum_of_blocks(const float* __restrict__ p, int groups, int stride) {
@@ -47,7 +59,11 @@ __device__ __forceinline__ void adam_body(const AdamLaunch& a, uint32_t block, u
     // bias corrections from the un-incremented age (adam/operations_generic.h:49-58)
     float bc1, bc2;
     rlt_adam_bias_corrections(a.p, age, bc1, bc2);
-    const uint32_t total = a.prefix[a.n];
+    const int ti = tensor_of(a, block);
+    const rlt_adam_tensor T = a.t[ti];
+    const uint32_t begin = (block - a.first_block[ti]) * a.span[ti], end = begin + min(a.span[ti], T.count - begin);
+    const float* __restrict__ const source = a.source + a.source_offset[ti];
+    const float scale = a.source_scale[ti], add = a.source_add[ti];
     float sq = 0.0f;
     if (a.source && a.groups > 16) {
         // many blocks: 64 elements per pass of a workgroup, four threads per element each add up a quarter of the blocks (the order of
@@ -55,15 +71,10 @@ __device__ __forceinline__ void adam_body(const AdamLaunch& a, uint32_t block, u
         __shared__ float quarter[4][64];
         const uint32_t el = threadIdx.x & 63u, qtr = threadIdx.x >> 6;
         const int per = (a.groups + 3) / 4, g0 = qtr * per, g1 = min(a.groups, g0 + per);
-        for (uint32_t base = block * 64u; base < total; base += n_blocks * 64u) {
-            const uint32_t i = min(base + el, total - 1u);
-            int ti = 0;
-#pragma unroll
-            for (int k = 1; k < MAX_T; k++) ti += (k < a.n && i >= a.prefix[k]) ? 1 : 0;
-            const uint32_t j = i - a.prefix[ti];
-            const float* __restrict__ p = a.source + a.source_offset[ti] + j;
+        for (uint32_t base = begin; base < end; base += 64u) {
+            const uint32_t j = min(base + el, end - 1u);
+            const float* __restrict__ p = source + j;
             // the element's moments and value travel while the blocks are added up
-            const rlt_adam_tensor& T = a.t[ti];
             float m = 0.f, v2 = 0.f, param = 0.f, target = 0.f;
             if (qtr == 0) { m = T.first_moment[j]; v2 = T.second_moment[j]; param = T.parameters[j]; if (T.polyak_target) target = T.polyak_target[j]; }
             float s = 0.f;
@@ -84,8 +95,8 @@ __device__ __forceinline__ void adam_body(const AdamLaunch& a, uint32_t block, u
             }
             quarter[qtr][el] = s;
             __syncthreads();
-            if (qtr == 0 && base + el < total) {
-                const float g = rlt_scaled_sum((quarter[0][el] + quarter[1][el]) + (quarter[2][el] + quarter[3][el]), a.source_scale[ti], a.source_add[ti]);
+            if (qtr == 0 && base + el < end) {
+                const float g = rlt_scaled_sum((quarter[0][el] + quarter[1][el]) + (quarter[2][el] + quarter[3][el]), scale, add);
                 T.gradient[j] = g;
                 sq += g * g;
                 rlt_adam_values(a.p, T.flags, g, bc1, bc2, m, v2, param);
@@ -97,18 +108,14 @@ __device__ __forceinline__ void adam_body(const AdamLaunch& a, uint32_t block, u
     } else {
     // four neighbouring elements per thread, from their gradient or from at most 16 blocks: every load is 16 bytes per lane (the same sums in the same order per element)
     typedef float f4 __attribute__((ext_vector_type(4)));
-    for (uint32_t i = (block * blockDim.x + threadIdx.x) * 4u; i < a.vec_end; i += n_blocks * blockDim.x * 4u) {
-        int ti = 0;
-#pragma unroll
-        for (int k = 1; k < MAX_T; k++) ti += (k < a.n && i >= a.prefix[k]) ? 1 : 0;
-        const rlt_adam_tensor& T = a.t[ti];
-        const uint32_t j = i - a.prefix[ti];
+    const uint32_t vec_end = (a.vec >> ti & 1u) ? end & ~3u : begin;
+    for (uint32_t j = begin + threadIdx.x * 4u; j < vec_end; j += 1024u) {
         f4 m = *reinterpret_cast<const f4*>(T.first_moment + j), v = *reinterpret_cast<const f4*>(T.second_moment + j), param = *reinterpret_cast<const f4*>(T.parameters + j);
         f4 target = {0.f, 0.f, 0.f, 0.f};
         if (T.polyak_target) target = *reinterpret_cast<const f4*>(T.polyak_target + j);
         f4 g;
         if (a.source) {
-            const float* __restrict__ p = a.source + a.source_offset[ti] + j;
+            const float* __restrict__ p = source + j;
             const int per = (a.groups + 3) / 4;
             f4 blk[16];
 #pragma unroll
@@ -127,7 +134,7 @@ __device__ __forceinline__ void adam_body(const AdamLaunch& a, uint32_t block, u
             }
             const f4 total4 = (q[0] + q[1]) + (q[2] + q[3]);
 #pragma unroll
-            for (int c = 0; c < 4; c++) g[c] = rlt_scaled_sum(total4[c], a.source_scale[ti], a.source_add[ti]);
+            for (int c = 0; c < 4; c++) g[c] = rlt_scaled_sum(total4[c], scale, add);
         } else g = *reinterpret_cast<const f4*>(T.gradient + j);
 #pragma unroll
         for (int c = 0; c < 4; c++) {
@@ -141,18 +148,13 @@ __device__ __forceinline__ void adam_body(const AdamLaunch& a, uint32_t block, u
         *reinterpret_cast<f4*>(T.first_moment + j) = m; *reinterpret_cast<f4*>(T.second_moment + j) = v; *reinterpret_cast<f4*>(T.parameters + j) = param;
         if (T.polyak_target) *reinterpret_cast<f4*>(T.polyak_target + j) = target;
     }
-    for (uint32_t i = a.vec_end + block * blockDim.x + threadIdx.x; i < total; i += n_blocks * blockDim.x) {
-        int ti = 0;
-#pragma unroll
-        for (int k = 1; k < MAX_T; k++) ti += (k < a.n && i >= a.prefix[k]) ? 1 : 0;
-        const rlt_adam_tensor& T = a.t[ti];
-        const uint32_t j = i - a.prefix[ti];
+    for (uint32_t j = vec_end + threadIdx.x; j < end; j += 256u) {
         // the element's moments, value and target travel together with its gradient (or the blocks that add up to it)
         float m = T.first_moment[j], v = T.second_moment[j], param = T.parameters[j];
         const float target = T.polyak_target ? T.polyak_target[j] : 0.f;
         float g;
         if (a.source) {
-            g = rlt_scaled_sum(sum_of_blocks(a.source + a.source_offset[ti] + j, a.groups, a.block_stride), a.source_scale[ti], a.source_add[ti]);
+            g = rlt_scaled_sum(sum_of_blocks(source + j, a.groups, a.block_stride), scale, add);
             T.gradient[j] = g;
         } else g = T.gradient[j];
         sq += g * g;
@@ -194,14 +196,10 @@ __global__ __launch_bounds__(256) void adam_pair_kernel(AdamLaunch a, AdamLaunch
 }
 
 __global__ __launch_bounds__(256) void adam_reset_kernel(AdamLaunch a) {
-    const uint32_t total = a.prefix[a.n];
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x) {
-        int ti = 0;
-#pragma unroll
-        for (int k = 1; k < MAX_T; k++) ti += (k < a.n && i >= a.prefix[k]) ? 1 : 0;
-        const uint32_t j = i - a.prefix[ti];
-        a.t[ti].first_moment[j] = 0.0f; a.t[ti].second_moment[j] = 0.0f;
-    }
+    const int ti = tensor_of(a, blockIdx.x);
+    const rlt_adam_tensor T = a.t[ti];
+    const uint32_t begin = (blockIdx.x - a.first_block[ti]) * a.span[ti], end = begin + min(a.span[ti], T.count - begin);
+    for (uint32_t j = begin + threadIdx.x; j < end; j += blockDim.x) { T.first_moment[j] = 0.0f; T.second_moment[j] = 0.0f; }
     if (a.increment_age && blockIdx.x == 0 && threadIdx.x == 0) *a.age = 1;
 }
 
@@ -214,26 +212,51 @@ __global__ __launch_bounds__(256) void polyak_kernel(const float* __restrict__ s
 
 }  // namespace
 
-// how far the elements can be stepped four at a time: up to the first tensor whose start, pointers or place in the blocks is not a multiple of 16 bytes, or that
-// ends off one (then its last one to three elements and everything behind them are stepped one by one)
-static uint32_t vector_end(const AdamLaunch& a) {
+// Tensors that follow each other in every array (and in the blocks of partial sums) and are stepped alike are one: a network laid out as an arena of parameters, gradients and
+// moments is a single tensor, with one ragged end instead of one per layer.
+static void join_neighbours(AdamLaunch& a) {
+    const uint32_t flags = (a.p.enable_weight_decay ? 1u : 0u) | (a.p.enable_bias_lr_factor ? 2u : 0u);      // those that make a difference
+    int n = 0;
+    for (int i = 1; i < a.n; i++) {
+        rlt_adam_tensor& T = a.t[n];
+        const rlt_adam_tensor& U = a.t[i];
+        bool follows = T.parameters + T.count == U.parameters && T.gradient + T.count == U.gradient && T.first_moment + T.count == U.first_moment &&
+                       T.second_moment + T.count == U.second_moment && (T.polyak_target ? T.polyak_target + T.count == U.polyak_target : !U.polyak_target) &&
+                       ((T.flags ^ U.flags) & flags) == 0;
+        if (a.source)
+            follows = follows && a.source_offset[n] + T.count == a.source_offset[i] && a.source_scale[n] == a.source_scale[i] && a.source_add[n] == a.source_add[i];
+        if (follows) { T.count += U.count; continue; }
+        n++;
+        a.t[n] = U;
+        a.source_offset[n] = a.source_offset[i]; a.source_scale[n] = a.source_scale[i]; a.source_add[n] = a.source_add[i];
+    }
+    a.n = n + 1;
+}
+// Deals the tensors out to at most about `most` workgroups and returns their number: 64 elements per workgroup pass where many blocks are added up, four per thread
+// where pointers, place in the blocks and block size are multiples of 16 bytes, one otherwise.
+static uint32_t deal_out(AdamLaunch& a, uint32_t most) {
     auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
-    if (a.source && (a.groups > 16 || a.block_stride % 4 != 0 || !aligned(a.source))) return 0;
-    uint32_t end = 0;
+    const bool many = a.source && a.groups > 16;
+    const bool source_ok = !a.source || (a.block_stride % 4 == 0 && aligned(a.source));
+    uint64_t passes = 0;
+    a.vec = 0;
     for (int i = 0; i < a.n; i++) {
         const rlt_adam_tensor& T = a.t[i];
-        if (a.prefix[i] % 4 != 0 || (a.source && a.source_offset[i] % 4 != 0) || !aligned(T.parameters) || !aligned(T.gradient) || !aligned(T.first_moment) || !aligned(T.second_moment) ||
-            (T.polyak_target && !aligned(T.polyak_target))) break;
-        end = a.prefix[i] + (T.count & ~3u);
-        if (T.count % 4 != 0) break;
+        const bool vec = !many && source_ok && (!a.source || a.source_offset[i] % 4 == 0) && aligned(T.parameters) && aligned(T.gradient) && aligned(T.first_moment) &&
+                         aligned(T.second_moment) && (!T.polyak_target || aligned(T.polyak_target));
+        if (vec) a.vec |= 1u << i;
+        a.span[i] = many ? 64u : vec ? 1024u : 256u;
+        passes += (T.count + (uint64_t)a.span[i] - 1) / a.span[i];
     }
-    return end;
-}
-// workgroups for an optimiser of `total` elements: 64 elements per workgroup pass on the many-block path, 256 threads of four elements each where those apply
-static uint32_t blocks_for(const AdamLaunch& a, uint32_t total, const rlt_adam_source* source) {
-    if (source && source->groups > 16) return (total + 63) / 64;
-    const uint32_t threads = a.vec_end / 4 > total - a.vec_end ? a.vec_end / 4 : total - a.vec_end;
-    return (threads + 255) / 256;
+    const uint32_t rounds = (uint32_t)((passes + most - 1) / most);
+    uint32_t blocks = 0;
+    for (int i = 0; i < a.n; i++) {
+        a.first_block[i] = blocks;
+        if (rounds > 1) a.span[i] *= rounds;
+        blocks += (uint32_t)((a.t[i].count + (uint64_t)a.span[i] - 1) / a.span[i]);
+    }
+    for (int i = a.n; i <= MAX_T; i++) a.first_block[i] = blocks;
+    return blocks;
 }
 
 // [256, 4096) of the device handle's counters block hold the workgroups' sums for the squared norm
@@ -245,20 +268,18 @@ static int adam_launch(rlt_rocm_device* device, const rlt_adam_tensor* tensors, 
     for (int base = 0; base < n_tensors; base += MAX_T) {
         AdamLaunch a = {};
         a.n = n_tensors - base < MAX_T ? n_tensors - base : MAX_T;
-        uint32_t total = 0;
         for (int i = 0; i < a.n; i++) {
             const rlt_adam_tensor& T = tensors[base + i];
             if (!T.first_moment || !T.second_moment || (!reset && (!T.parameters || !T.gradient)) || T.count == 0) return RLT_E_INVALID_ARGUMENT;
-            a.t[i] = T; a.prefix[i] = total; total += T.count;
+            a.t[i] = T;
         }
-        for (int i = a.n; i <= MAX_T; i++) a.prefix[i] = total;
         if (p) a.p = *p;
         a.polyak = polyak; a.age = age;
         a.tickets = rlt_tickets_of(counters, 0); a.block_partials = (float*)((char*)counters + 256);
         a.out_sq_norm = out_sq_norm; a.accumulate_norm = base > 0;
         a.increment_age = (base + MAX_T >= n_tensors);
-        if (!reset) a.vec_end = vector_end(a);
-        int blocks = (int)blocks_for(a, total, nullptr); if (blocks > 960) blocks = 960; if (blocks < 1) blocks = 1;
+        if (!reset) join_neighbours(a);
+        const uint32_t blocks = deal_out(a, MAX_BLOCKS);
         if (reset) hipLaunchKernelGGL(adam_reset_kernel, dim3(blocks), dim3(256), 0, device->stream, a);
         else hipLaunchKernelGGL(adam_kernel, dim3(blocks), dim3(256), 0, device->stream, a);
         if ((rc = rlt_launch_status(device))) return rc;
@@ -279,19 +300,17 @@ int rlt_adam_step_from_partials(rlt_rocm_device* device, const rlt_adam_tensor* 
     if (rc) return rc;
     AdamLaunch a = {};
     a.n = n;
-    uint32_t total = 0;
     for (int i = 0; i < n; i++) {
         const rlt_adam_tensor& T = tensors[i];
         if (!T.first_moment || !T.second_moment || !T.parameters || !T.gradient || T.count == 0) return RLT_E_INVALID_ARGUMENT;
-        a.t[i] = T; a.prefix[i] = total; total += T.count;
+        a.t[i] = T;
     }
-    for (int i = n; i <= MAX_T; i++) a.prefix[i] = total;
     a.p = *parameters; a.age = age; a.polyak = polyak;
     a.tickets = rlt_tickets_of(counters, 0); a.block_partials = (float*)((char*)counters + 256);
     a.increment_age = 1;
     set_source(a, source);
-    a.vec_end = vector_end(a);
-    int blocks = (int)blocks_for(a, total, source); if (blocks > 960) blocks = 960; if (blocks < 1) blocks = 1;
+    join_neighbours(a);
+    const uint32_t blocks = deal_out(a, MAX_BLOCKS);
     hipLaunchKernelGGL(adam_kernel, dim3(blocks), dim3(256), 0, device->stream, a);
     return rlt_launch_status(device);
 }
@@ -314,13 +333,11 @@ int rlt_adam_step_pair(rlt_rocm_device* device, const rlt_adam_tensor* tensors_a
         AdamLaunch& a = L[k];
         const rlt_adam_tensor* tensors = k ? tensors_b : tensors_a;
         a.n = k ? n_b : n_a;
-        uint32_t total = 0;
         for (int i = 0; i < a.n; i++) {
             const rlt_adam_tensor& T = tensors[i];
             if (!T.first_moment || !T.second_moment || !T.parameters || !T.gradient || T.count == 0) return RLT_E_INVALID_ARGUMENT;
-            a.t[i] = T; a.prefix[i] = total; total += T.count;
+            a.t[i] = T;
         }
-        for (int i = a.n; i <= MAX_T; i++) a.prefix[i] = total;
         a.p = k ? *parameters_b : *parameters_a;
         a.age = k ? age_b : age_a; a.polyak = polyak;
         // the second optimiser's tickets and partial sums sit in their own part of the counters block
@@ -328,8 +345,8 @@ int rlt_adam_step_pair(rlt_rocm_device* device, const rlt_adam_tensor* tensors_a
         a.increment_age = 1;
         const rlt_adam_source* source = k ? source_b : source_a;
         set_source(a, source);
-        a.vec_end = vector_end(a);
-        blocks[k] = blocks_for(a, total, source); if (blocks[k] > 480) blocks[k] = 480; if (blocks[k] < 1) blocks[k] = 1;
+        join_neighbours(a);
+        blocks[k] = deal_out(a, MAX_BLOCKS / 2);
     }
     hipLaunchKernelGGL(adam_pair_kernel, dim3(blocks[0] + blocks[1]), dim3(256), 0, device->stream, L[0], L[1], blocks[0]);
     return rlt_launch_status(device);
