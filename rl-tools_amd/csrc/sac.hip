@@ -20,20 +20,36 @@ __device__ __forceinline__ float normal_log_prob(float mean, float log_std, floa
     return neg_log_sqrt_2pi - log_std - 0.5f * z * z;
 }
 
+// one action: sampled, squashed; returns its log-probability
+__device__ __forceinline__ float sas_forward_element(const rlt_sas_parameters& p, float mean, float log_std_raw, const float* noise, float& sample, float& action) {
+    const float log_std = clampf(log_std_raw, p.log_std_lower_bound, p.log_std_upper_bound), sd = expf(log_std);
+    sample = noise ? mean + *noise * sd : mean;
+    action = tanhf(sample);
+    return normal_log_prob(mean, log_std, sd, sample) - logf(1.0f - action * action + p.log_probability_epsilon);
+}
+// the gradients at one action's mean and log standard deviation from the gradient at the action; returns the action's log-probability
+__device__ __forceinline__ float sas_backward_element(const rlt_sas_parameters& p, float action, float d_action, float eps, float mu, float log_std_raw, float sample,
+                                                      float alpha_over_b, float& d_mu, float& d_ls) {
+    const float g = d_action * (1.0f - action * action);
+    const float log_std = clampf(log_std_raw, p.log_std_lower_bound, p.log_std_upper_bound), sd = expf(log_std);
+    const float z = (sample - mu) / sd;
+    const float dlp_dmean = z / sd, dlp_dsample = -z / sd, dlp_dlogstd = z * z - 1.0f;
+    d_mu = g + alpha_over_b * (dlp_dmean + dlp_dsample + 2.0f * action);
+    d_ls = sd * (g * eps) + alpha_over_b * (dlp_dlogstd + dlp_dsample * eps * sd + 2.0f * action * eps * sd);
+    if (log_std_raw < p.log_std_lower_bound || log_std_raw > p.log_std_upper_bound) d_ls = 0.0f;
+    return normal_log_prob(mu, log_std, sd, sample) - logf(1.0f - action * action + p.log_probability_epsilon);
+}
+
 __global__ __launch_bounds__(256) void sas_forward_kernel(rlt_sas_parameters p, const float* __restrict__ input, int ldin, const float* __restrict__ noise, int ldn,
                                                           float* __restrict__ actions, int lda, float* __restrict__ pre_squashing, int ldp,
                                                           float* __restrict__ log_probabilities, int batch, int dim) {
     for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < batch; r += gridDim.x * blockDim.x) {
         float log_prob = 0.0f;
         for (int c = 0; c < dim; c++) {
-            float mean = input[(size_t)r * ldin + c];
-            float log_std = clampf(input[(size_t)r * ldin + dim + c], p.log_std_lower_bound, p.log_std_upper_bound);
-            float sd = expf(log_std);
-            float sample = noise ? mean + noise[(size_t)r * ldn + c] * sd : mean;
+            float sample, a;
+            log_prob += sas_forward_element(p, input[(size_t)r * ldin + c], input[(size_t)r * ldin + dim + c], noise ? noise + (size_t)r * ldn + c : nullptr, sample, a);
             if (pre_squashing) pre_squashing[(size_t)r * ldp + c] = sample;
-            float a = tanhf(sample);
             actions[(size_t)r * lda + c] = a;
-            log_prob += normal_log_prob(mean, log_std, sd, sample) - logf(1.0f - a * a + p.log_probability_epsilon);
         }
         log_probabilities[r] = log_prob;
     }
@@ -53,23 +69,11 @@ __global__ __launch_bounds__(1024) void sas_backward_kernel(rlt_sas_parameters p
     for (int b = threadIdx.x; b < batch; b += blockDim.x) {
         float entropy = 0.0f;
         for (int a = 0; a < dim; a++) {
-            float action = actions[(size_t)b * lda + a];
-            float g = d_output[(size_t)b * lddo + a] * (1.0f - action * action);
-            float eps = noise[(size_t)b * ldn + a];
-            float log_std_raw = input[(size_t)b * ldin + dim + a];
-            float log_std = clampf(log_std_raw, p.log_std_lower_bound, p.log_std_upper_bound);
-            float sd = expf(log_std);
-            float mu = input[(size_t)b * ldin + a];
-            float sample = pre_squashing[(size_t)b * ldp + a];
-            float z = (sample - mu) / sd;
-            float dlp_dmean = z / sd, dlp_dsample = -z / sd, dlp_dlogstd = z * z - 1.0f;
-            float d_mu = g + alpha_over_b * (dlp_dmean + dlp_dsample + 2.0f * action);
-            float d_ls = sd * (g * eps) + alpha_over_b * (dlp_dlogstd + dlp_dsample * eps * sd + 2.0f * action * eps * sd);
-            if (log_std_raw < p.log_std_lower_bound || log_std_raw > p.log_std_upper_bound) d_ls = 0.0f;
+            float d_mu, d_ls;
+            entropy -= sas_backward_element(p, actions[(size_t)b * lda + a], d_output[(size_t)b * lddo + a], noise[(size_t)b * ldn + a], input[(size_t)b * ldin + a],
+                                            input[(size_t)b * ldin + dim + a], pre_squashing[(size_t)b * ldp + a], alpha_over_b, d_mu, d_ls);
             d_input[(size_t)b * lddi + a] = d_mu;
             d_input[(size_t)b * lddi + dim + a] = d_ls;
-            float lp = normal_log_prob(mu, log_std, sd, sample) - logf(1.0f - action * action + p.log_probability_epsilon);
-            entropy -= lp;
         }
         acc += alpha * (entropy - p.target_entropy);
         nreset += reset ? (float)(reset[b] != 0) : 1.0f;
@@ -84,14 +88,17 @@ __global__ __launch_bounds__(1024) void sas_backward_kernel(rlt_sas_parameters p
     }
 }
 
+__device__ __forceinline__ float target_value(float q1, float q2, float reward, bool terminated, float next_log_prob, float alpha, float gamma) {
+    const float min_q = fminf(q1, q2) - alpha * next_log_prob;
+    const float future = !terminated ? gamma * min_q : 0.0f;
+    return reward + future;
+}
 __global__ __launch_bounds__(256) void target_q_kernel(const float* __restrict__ q1, const float* __restrict__ q2, const float* __restrict__ rewards,
                                                        const uint8_t* __restrict__ terminated, const float* __restrict__ next_log_probs,
                                                        const float* __restrict__ log_alpha, float gamma, int ignore_termination, float* __restrict__ target, int batch) {
     const float alpha = expf(*log_alpha);
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < batch; i += gridDim.x * blockDim.x) {
-        float min_q = fminf(q1[i], q2[i]) - alpha * next_log_probs[i];
-        float future = (ignore_termination || !terminated[i]) ? gamma * min_q : 0.0f;
-        target[i] = rewards[i] + future;
+        target[i] = target_value(q1[i], q2[i], rewards[i], !ignore_termination && terminated[i], next_log_probs[i], alpha, gamma);
     }
 }
 __global__ __launch_bounds__(256) void min_q_kernel(const float* __restrict__ q1, const float* __restrict__ q2, const float* __restrict__ d1, const float* __restrict__ d2,
@@ -169,6 +176,131 @@ __global__ __launch_bounds__(1024) void sac_d_output_kernel(const float* __restr
         d[i] = m ? v : 0.0f;
     }
 }
+
+// ---- The steps between the passes of a sequence update, over S x B rows of one time step each. What bounds them is the launch (4.5 us each while the values are a few hundred
+// kilobytes) and, where a sum over the rows is wanted, that one workgroup cannot ask for them all at once (9 and 15 us at 10,000 rows): each step is one launch of a row
+// per thread, and the sums are formed per workgroup (the number of masked rows by every workgroup for itself, the entropy term's partial sums by the last one through).
+
+// rows whose mask is set (all without one), the same in every thread of a workgroup of 256
+__device__ __forceinline__ float count_rows(const uint8_t* __restrict__ mask, int rows) {
+    if (!mask) return (float)rows;
+    __shared__ int partial[4];
+    int n = 0, head = (int)((4 - (reinterpret_cast<uintptr_t>(mask) & 3)) & 3);      // bytes before the first whole word
+    if (head > rows) head = rows;
+    const int words = (rows - head) / 4, tail = head + 4 * words;
+    const uint32_t* w = reinterpret_cast<const uint32_t*>(mask + head);
+    for (int i0 = threadIdx.x; i0 < words; i0 += 256 * 8) {
+        uint32_t v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) { const int i = i0 + 256 * u; v[u] = i < words ? w[i] : 0u; }
+#pragma unroll
+        for (int u = 0; u < 8; u++) n += __popc((((v[u] & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | v[u]) & 0x80808080u);
+    }
+    if ((int)threadIdx.x < head) n += mask[threadIdx.x] != 0;
+    if ((int)threadIdx.x < rows - tail) n += mask[tail + threadIdx.x] != 0;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
+    if ((threadIdx.x & 63) == 0) partial[threadIdx.x >> 6] = n;
+    __syncthreads();
+    return (float)(partial[0] + partial[1] + partial[2] + partial[3]);
+}
+
+// The critics' input rows: observations and, where the row's step is a final one, the policy's action, elsewhere the action taken (sac/operations_generic.h:266-278, 427-431).
+// The actor's update also keeps the actions and their samples, and has the gradient at the critics' outputs filled in (:437-453).
+struct SequenceActions {
+    rlt_sas_parameters sas; const float* policy; const float* noise; const float* base; const uint8_t* final_step;
+    float* critic_input; float* log_probabilities; float* actions; float* pre_squashing; float* d_output;      // the last three may be NULL
+    int rows, obs, act;
+};
+__global__ __launch_bounds__(256) void sequence_actions_kernel(SequenceActions A) {
+    const int D = A.obs + A.act;
+    const float d = A.d_output ? (1.0f / count_rows(A.final_step, A.rows)) * -1.0f : 0.0f;
+    for (int r = blockIdx.x * 256 + threadIdx.x; r < A.rows; r += gridDim.x * 256) {
+        const bool last = A.final_step[r] != 0;
+        const float* base = A.base + (size_t)r * D;
+        float* row = A.critic_input + (size_t)r * D;
+        float log_probability = 0.0f;
+        for (int c = 0; c < A.act; c++) {
+            float sample, action;
+            const float* policy = A.policy + (size_t)r * 2 * A.act;
+            log_probability += sas_forward_element(A.sas, policy[c], policy[A.act + c], A.noise + (size_t)r * A.act + c, sample, action);
+            row[A.obs + c] = last ? action : base[A.obs + c];
+            if (A.actions) { A.actions[(size_t)r * A.act + c] = action; A.pre_squashing[(size_t)r * A.act + c] = sample; }
+        }
+        A.log_probabilities[r] = log_probability;
+        for (int c = 0; c < A.obs; c++) row[c] = base[c];
+        if (A.d_output) A.d_output[r] = last ? d : 0.0f;
+    }
+}
+
+// the target values and, for one or two critics, the gradient at the output (:144-154, 289-316)
+struct SequenceTargets {
+    const float* next_q[2]; const float* rewards; const uint8_t* terminated; const float* next_log_probabilities; const float* log_alpha; const uint8_t* final_step;
+    const float* q[2]; float* d_output[2]; float* target; float gamma; int rows, count;
+};
+__global__ __launch_bounds__(256) void sequence_targets_kernel(SequenceTargets A) {
+    const float alpha = expf(*A.log_alpha);
+    const float constant = 2.0f / (float)A.rows * ((1.0f / count_rows(A.final_step, A.rows)) * ((float)A.rows * 0.5f));
+    for (int r = blockIdx.x * 256 + threadIdx.x; r < A.rows; r += gridDim.x * 256) {
+        const float target = target_value(A.next_q[0][r], A.next_q[1][r], A.rewards[r], A.terminated[r] != 0, A.next_log_probabilities[r], alpha, A.gamma);
+        A.target[r] = target;
+        const bool last = A.final_step[r] != 0;
+        for (int k = 0; k < A.count; k++) A.d_output[k][r] = last ? (A.q[k][r] - target) * constant : 0.0f;
+    }
+}
+
+// the gradient at the policy's action from the critic that values it lower (zero where the row's step is not a final one), through the squashed sample to the policy's outputs,
+// and d log_alpha (:456-464)
+struct SequenceActorGradient {
+    rlt_sas_parameters sas; const float* q[2]; const float* d_critic_input[2]; const uint8_t* final_step; const uint8_t* reset;
+    const float* policy; const float* noise; const float* actions; const float* pre_squashing; const float* log_alpha;
+    float* d_action; float* d_policy; float* d_log_alpha; float* partial; uint32_t* tickets;
+    int rows, obs, act;
+};
+__global__ __launch_bounds__(256) void sequence_actor_gradient_kernel(SequenceActorGradient A) {
+    __shared__ float sums[2][4];
+    const int D = A.obs + A.act;
+    const float alpha = expf(*A.log_alpha), alpha_over_b = alpha / (float)A.rows;
+    float acc = 0.0f, resets = 0.0f;
+    for (int r = blockIdx.x * 256 + threadIdx.x; r < A.rows; r += gridDim.x * 256) {
+        const float* d = (A.q[0][r] < A.q[1][r] ? A.d_critic_input[0] : A.d_critic_input[1]) + (size_t)r * D + A.obs;
+        const bool last = A.final_step[r] != 0;
+        float entropy = 0.0f;
+        for (int c = 0; c < A.act; c++) {
+            const size_t i = (size_t)r * A.act + c;
+            const float* policy = A.policy + (size_t)r * 2 * A.act;
+            const float d_action = last ? d[c] : 0.0f;
+            A.d_action[i] = d_action;
+            float d_mu, d_ls;
+            entropy -= sas_backward_element(A.sas, A.actions[i], d_action, A.noise[i], policy[c], policy[A.act + c], A.pre_squashing[i], alpha_over_b, d_mu, d_ls);
+            A.d_policy[(size_t)r * 2 * A.act + c] = d_mu;
+            A.d_policy[(size_t)r * 2 * A.act + A.act + c] = d_ls;
+        }
+        acc += alpha * (entropy - A.sas.target_entropy);
+        resets += (float)(A.reset[r] != 0);
+    }
+    acc = rlt_wave_sum(acc); resets = rlt_wave_sum(resets);
+    if ((threadIdx.x & 63) == 0) { sums[0][threadIdx.x >> 6] = acc; sums[1][threadIdx.x >> 6] = resets; }
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        bool last = false;
+        if (threadIdx.x == 0) {
+            A.partial[2 * blockIdx.x] = (sums[0][0] + sums[0][1]) + (sums[0][2] + sums[0][3]);
+            A.partial[2 * blockIdx.x + 1] = (sums[1][0] + sums[1][1]) + (sums[1][2] + sums[1][3]);
+            __threadfence();
+            last = rlt_last_through(A.tickets, blockIdx.x, gridDim.x);
+        }
+        if (__any(last)) {      // this workgroup's first wavefront sees what every other one has written
+            __threadfence();
+            float s = 0.0f, n = 0.0f;
+            for (uint32_t b = threadIdx.x; b < gridDim.x; b += 64) { s += ((volatile float*)A.partial)[2 * b]; n += ((volatile float*)A.partial)[2 * b + 1]; }
+            s = rlt_wave_sum(s); n = rlt_wave_sum(n);
+            if (threadIdx.x == 0) *A.d_log_alpha = s / n;
+        }
+    }
+}
+constexpr int MAX_PARTIALS = 448;      // workgroups whose two sums fit the counters block
+int sequence_grid(int rows) { const int b = (rows + 255) / 256; return b > MAX_PARTIALS ? MAX_PARTIALS : b; }
 
 int grid1(int n) { int b = (n + 255) / 256; return b > 1024 ? 1024 : (b < 1 ? 1 : b); }
 
@@ -451,6 +583,26 @@ static bool sequence_agent_stacked(const rlt_sac_sequence_agent* A) {
         if (!rlt_seq_stack_supported(A->critics[k], A->n_critic_layers, T) || !rlt_seq_stack_supported(A->critics_target[k], A->n_critic_layers, T)) return false;
     return true;
 }
+static int sequence_next_actions(rlt_rocm_device* device, const rlt_sac_sequence_agent* A, const float* base_next, const uint8_t* next_final, int rows, const float* action_noise) {
+    SequenceActions a = {};
+    a.sas = A->sas; a.policy = seq_output(A->actor, A->n_actor_layers); a.noise = action_noise; a.base = base_next; a.final_step = next_final;
+    a.critic_input = A->next_state_action_value_input; a.log_probabilities = A->next_log_probabilities;
+    a.rows = rows; a.obs = A->observation_dim; a.act = A->action_dim;
+    hipLaunchKernelGGL(sequence_actions_kernel, dim3(sequence_grid(rows)), dim3(256), 0, device->stream, a);
+    return rlt_launch_status(device);
+}
+// target values, and the loss gradients of critics ci ... ci + count - 1 into d_output[k]; `offset`: where in the next values the first step's lies
+static int sequence_targets(rlt_rocm_device* device, const rlt_sac_sequence_agent* A, int ci, int count, int offset, float* const (&d_output)[2]) {
+    const rlt_sequence_batch& K = A->batch;
+    SequenceTargets a = {};
+    for (int k = 0; k < 2; k++) a.next_q[k] = A->next_q[k] + offset;
+    for (int k = 0; k < count; k++) { a.q[k] = seq_output(A->critics[ci + k], A->n_critic_layers); a.d_output[k] = d_output[k]; }
+    a.rewards = K.rewards; a.terminated = K.terminated; a.next_log_probabilities = A->next_log_probabilities; a.log_alpha = A->log_alpha.parameters;
+    a.final_step = K.final_step_mask; a.target = A->target_action_value; a.gamma = A->gamma; a.rows = K.sequence_length * K.batch; a.count = count;
+    hipLaunchKernelGGL(sequence_targets_kernel, dim3(sequence_grid(a.rows)), dim3(256), 0, device->stream, a);
+    return rlt_launch_status(device);
+}
+
 static int stacked_train_critics(rlt_rocm_device* device, const rlt_sac_sequence_agent* A, int ci, int count, const float* action_noise) {
     const rlt_sequence_batch& K = A->batch;
     const int S = K.sequence_length, B = K.batch, OBS = A->observation_dim, ACT = A->action_dim, D = OBS + ACT;
@@ -464,25 +616,16 @@ static int stacked_train_critics(rlt_rocm_device* device, const rlt_sac_sequence
     forward[count] = {A->actor, base_next, D, next_reset, T, B, nullptr};
     int rc;
     if ((rc = rlt_seq_stack_forward(device, forward, count + 1))) return rc;
-    float* next_actions = A->next_state_action_value_input + OBS;
-    if ((rc = rlt_rocm_sas_forward(device, &A->sas, seq_output(A->actor, A->n_actor_layers), 2 * ACT, action_noise, ACT, next_actions, D, nullptr, 0,
-                                   A->next_log_probabilities, T * B, ACT))) return rc;
-    if ((rc = rlt_rocm_mask_copy(device, base_next + OBS, D, next_actions, D, next_final, 1, T * B, ACT))) return rc;
-    if ((rc = copy2d(device, base_next, D, A->next_state_action_value_input, D, T * B, OBS))) return rc;
+    if ((rc = sequence_next_actions(device, A, base_next, next_final, T * B, action_noise))) return rc;
     const rlt_stack_forward targets[2] = {{A->critics_target[0], A->next_state_action_value_input, D, next_reset, T, B, A->next_q[0]},
                                           {A->critics_target[1], A->next_state_action_value_input, D, next_reset, T, B, A->next_q[1]}};
     if ((rc = rlt_seq_stack_forward(device, targets, 2))) return rc;
-    if ((rc = rlt_rocm_sac_target_action_values(device, A->next_q[0] + first * B, A->next_q[1] + first * B, K.rewards, K.terminated, A->next_log_probabilities,
-                                               A->log_alpha.parameters, A->gamma, 0, A->target_action_value, S * B))) return rc;
+    // the last critic's loss gradient goes to the agent's buffer (where two calls leave it), the other's to the end of the workspace
+    float* const d_output[2] = {count == 1 ? A->d_output : (float*)((char*)A->workspace + 3 * ws_bytes), A->d_output};
+    if ((rc = sequence_targets(device, A, ci, count, first * B, d_output))) return rc;
     rlt_stack_backward backward[2];
-    for (int k = 0; k < count; k++) {
-        // the last critic's loss gradient goes to the agent's buffer (where two calls leave it), the other's to the end of the workspace
-        float* const d_output = k == count - 1 ? A->d_output : (float*)((char*)A->workspace + 3 * ws_bytes);
-        hipLaunchKernelGGL(sac_d_output_kernel, dim3(1), dim3(1024), 0, device->stream, seq_output(A->critics[ci + k], A->n_critic_layers), (const float*)A->target_action_value,
-                           (const uint8_t*)K.final_step_mask, d_output, S * B, 0);
-        if ((rc = rlt_launch_status(device))) return rc;
-        backward[k] = {A->critics[ci + k], K.observations_actions_base, D, d_output, nullptr, K.reset, S, B, 1, 1, (char*)A->workspace + k * ws_bytes};
-    }
+    for (int k = 0; k < count; k++)
+        backward[k] = {A->critics[ci + k], K.observations_actions_base, D, d_output[k], nullptr, K.reset, S, B, 1, 1, (char*)A->workspace + k * ws_bytes};
     if ((rc = rlt_seq_stack_backward(device, backward, count))) return rc;
     if (count == 2)
         return rlt_adam_step_pair(device, A->critic_adam_tensors[0], A->n_critic_adam_tensors, &A->critic_adam, A->critic_age[0], A->critic_adam_tensors[1], A->n_critic_adam_tensors,
@@ -517,11 +660,7 @@ int rlt_rocm_sac_sequence_train_critic(rlt_rocm_device* device, const rlt_sac_se
     const uint8_t* next_reset = K.next_reset_base + (size_t)next_offset * B;
     const uint8_t* next_final = K.next_final_step_mask_base + (size_t)next_offset * B;
     if ((rc = rlt_rocm_seq_forward(device, A->actor, A->n_actor_layers, base_next, D, next_reset, T, B, ws, ws_bytes))) return rc;           // :266-273
-    float* next_actions = A->next_state_action_value_input + OBS;
-    if ((rc = rlt_rocm_sas_forward(device, &A->sas, seq_output(A->actor, A->n_actor_layers), 2 * ACT, action_noise, ACT, next_actions, D, nullptr, 0,
-                                   A->next_log_probabilities, T * B, ACT))) return rc;
-    if ((rc = rlt_rocm_mask_copy(device, base_next + OBS, D, next_actions, D, next_final, 1, T * B, ACT))) return rc;                      // :274-277
-    if ((rc = copy2d(device, base_next, D, A->next_state_action_value_input, D, T * B, OBS))) return rc;                                   // :278
+    if ((rc = sequence_next_actions(device, A, base_next, next_final, T * B, action_noise))) return rc;
     for (int k = 1; k >= 0; k--) {                                                                                                         // :283-284 (target critic 1 on the side stream)
         const bool side = k == 1 && overlap && rlt_side_begin(device);
         rc = rlt_rocm_seq_forward(device, A->critics_target[k], A->n_critic_layers, A->next_state_action_value_input, D, next_reset, T, B, side ? ws_side : ws, ws_bytes);
@@ -530,12 +669,9 @@ int rlt_rocm_sac_sequence_train_critic(rlt_rocm_device* device, const rlt_sac_se
         if (rc) return rc;
     }
     if (overlap && (rc = rlt_side_join(device))) return rc;
-    // the value of the step after (offset B where the first step is included), the log-probability at the same index (:144-154)
-    if ((rc = rlt_rocm_sac_target_action_values(device, A->next_q[0] + first * B, A->next_q[1] + first * B, K.rewards, K.terminated, A->next_log_probabilities,
-                                               A->log_alpha.parameters, A->gamma, 0, A->target_action_value, S * B))) return rc;             // :289
-    hipLaunchKernelGGL(sac_d_output_kernel, dim3(1), dim3(1024), 0, device->stream, seq_output(critic, A->n_critic_layers), (const float*)A->target_action_value,
-                       (const uint8_t*)K.final_step_mask, A->d_output, S * B, 0);                                                          // :298-316
-    if ((rc = rlt_launch_status(device))) return rc;
+    // the value of the step after (offset B where the first step is included), the log-probability at the same index (:144-154); the loss gradient (:289-316)
+    float* const d_output[2] = {A->d_output, nullptr};
+    if ((rc = sequence_targets(device, A, ci, 1, first * B, d_output))) return rc;
     if ((rc = rlt_rocm_seq_backward(device, critic, A->n_critic_layers, K.observations_actions_base, D, A->d_output, nullptr, K.reset, S, B, 1, 0, ws, ws_bytes))) return rc;   // :329
     return rlt_rocm_adam_step(device, A->critic_adam_tensors[ci], A->n_critic_adam_tensors, &A->critic_adam, A->critic_age[ci], 0.0f, nullptr);   // :336
 }
@@ -573,11 +709,7 @@ int rlt_rocm_sac_sequence_train_critics(rlt_rocm_device* device, const rlt_sac_s
     const uint8_t* next_reset = K.next_reset_base + (size_t)next_offset * B;
     const uint8_t* next_final = K.next_final_step_mask_base + (size_t)next_offset * B;
     if ((rc = rlt_rocm_seq_forward(device, A->actor, A->n_actor_layers, base_next, D, next_reset, T, B, ws, ws_bytes))) return rc;
-    float* next_actions = A->next_state_action_value_input + OBS;
-    if ((rc = rlt_rocm_sas_forward(device, &A->sas, seq_output(A->actor, A->n_actor_layers), 2 * ACT, action_noise, ACT, next_actions, D, nullptr, 0,
-                                   A->next_log_probabilities, T * B, ACT))) return rc;
-    if ((rc = rlt_rocm_mask_copy(device, base_next + OBS, D, next_actions, D, next_final, 1, T * B, ACT))) return rc;
-    if ((rc = copy2d(device, base_next, D, A->next_state_action_value_input, D, T * B, OBS))) return rc;
+    if ((rc = sequence_next_actions(device, A, base_next, next_final, T * B, action_noise))) return rc;
     for (int k = 1; k >= 0; k--) {      // target critic 1 behind critic 0's forward pass on the side stream (it waits for the copies above), target critic 0 on the main stream
         if (k == 1 && overlap) rlt_side_begin(device);
         rc = rlt_rocm_seq_forward(device, A->critics_target[k], A->n_critic_layers, A->next_state_action_value_input, D, next_reset, T, B, device->side_return ? ws_side : ws, ws_bytes);
@@ -586,13 +718,8 @@ int rlt_rocm_sac_sequence_train_critics(rlt_rocm_device* device, const rlt_sac_s
         if (rc) return rc;
     }
     if (overlap && (rc = rlt_side_join(device))) return rc;
-    if ((rc = rlt_rocm_sac_target_action_values(device, A->next_q[0] + first * B, A->next_q[1] + first * B, K.rewards, K.terminated, A->next_log_probabilities,
-                                               A->log_alpha.parameters, A->gamma, 0, A->target_action_value, S * B))) return rc;
-    for (int k = 0; k < 2; k++) {
-        hipLaunchKernelGGL(sac_d_output_kernel, dim3(1), dim3(1024), 0, device->stream, seq_output(A->critics[k], A->n_critic_layers), (const float*)A->target_action_value,
-                           (const uint8_t*)K.final_step_mask, k ? A->d_output : d_output_first, S * B, 0);
-        if ((rc = rlt_launch_status(device))) return rc;
-    }
+    float* const d_output[2] = {d_output_first, A->d_output};
+    if ((rc = sequence_targets(device, A, 0, 2, first * B, d_output))) return rc;
     {
         if (overlap) rlt_side_begin(device);
         rc = rlt_rocm_seq_backward(device, A->critics[1], A->n_critic_layers, K.observations_actions_base, D, A->d_output, nullptr, K.reset, S, B, 1, 0, device->side_return ? ws_side : ws, ws_bytes);
@@ -645,20 +772,16 @@ int rlt_rocm_sac_sequence_train_actor(rlt_rocm_device* device, const rlt_sac_seq
     const bool overlap = S >= 48 && !stacked;      // short sequences: a pass is shorter than the two events that fork and join a stream cost on the host
     int rc;
     if (!stacked && (rc = rlt_rocm_seq_zero_gradient(device, A->actor, A->n_actor_layers))) return rc;                                      // :414
-    if ((rc = rlt_rocm_fill_f32(device, A->log_alpha.gradient, 1, 1, 1, 0.0f))) return rc;
     const float* obs = K.observations_actions_base;
     if ((rc = rlt_rocm_seq_forward(device, A->actor, A->n_actor_layers, obs, D, K.reset, S, B, ws, ws_bytes))) return rc;                   // :427
     const float* actor_out = seq_output(A->actor, A->n_actor_layers);
-    if ((rc = rlt_rocm_sas_forward(device, &A->sas, actor_out, 2 * ACT, action_noise, ACT, A->actor_actions, ACT, A->actor_pre_squashing, ACT,
-                                   A->actor_log_probabilities, R, ACT))) return rc;
-    float* sav_actions = A->state_action_value_input + OBS;
-    if ((rc = copy2d(device, A->actor_actions, ACT, sav_actions, D, R, ACT))) return rc;
-    if ((rc = rlt_rocm_mask_copy(device, obs + OBS, D, sav_actions, D, K.final_step_mask, 1, R, ACT))) return rc;                           // :428-430
-    if ((rc = copy2d(device, obs, D, A->state_action_value_input, D, R, OBS))) return rc;                                                   // :431
-    // the gradient at the critics' outputs is a constant per row (:437-453): formed first, so that each critic's forward pass and its gradient towards the input
-    // (:432-433, :458-459) can follow each other on a stream of their own -- critic 1 on the side stream, critic 0 on the main stream
-    hipLaunchKernelGGL(sac_d_output_kernel, dim3(1), dim3(1024), 0, device->stream, (const float*)nullptr, (const float*)nullptr, (const uint8_t*)K.final_step_mask,
-                       A->d_output, R, 1);
+    // sample, the critics' input rows (:428-431), and the gradient at the critics' outputs, a constant per row (:437-453): formed before the critics' passes, so that each
+    // critic's forward pass and its gradient towards the input (:432-433, :458-459) can follow each other on a stream of their own -- critic 1 on the side stream, critic 0 on the main stream
+    SequenceActions actions = {};
+    actions.sas = A->sas; actions.policy = actor_out; actions.noise = action_noise; actions.base = obs; actions.final_step = K.final_step_mask;
+    actions.critic_input = A->state_action_value_input; actions.log_probabilities = A->actor_log_probabilities; actions.actions = A->actor_actions;
+    actions.pre_squashing = A->actor_pre_squashing; actions.d_output = A->d_output; actions.rows = R; actions.obs = OBS; actions.act = ACT;
+    hipLaunchKernelGGL(sequence_actions_kernel, dim3(sequence_grid(R)), dim3(256), 0, device->stream, actions);
     if ((rc = rlt_launch_status(device))) return rc;
     // the inner layers of backward_input run without the reset mode (nn_models/sequential/operations_generic.h:399-407); the critics'
     // output layer has no activation function, so d_output survives the calls unchanged (both read it)
@@ -679,11 +802,17 @@ int rlt_rocm_sac_sequence_train_actor(rlt_rocm_device* device, const rlt_sac_seq
         if (rc) return rc;
     }
     if (overlap && (rc = rlt_side_join(device))) return rc;
-    if ((rc = rlt_rocm_sac_min_value_d_output(device, seq_output(A->critics[0], A->n_critic_layers), seq_output(A->critics[1], A->n_critic_layers), A->d_critic_input[0],
-                                             A->d_critic_input[1], D, D, ACT, A->d_actor_output_squashing, ACT, R))) return rc;             // :460
-    if ((rc = rlt_rocm_mask_zero(device, A->d_actor_output_squashing, ACT, K.final_step_mask, 1, R, ACT))) return rc;                       // :461-463
-    if ((rc = sas_backward_impl(device, &A->sas, actor_out, 2 * ACT, action_noise, ACT, A->actor_actions, ACT, A->actor_pre_squashing, ACT, A->d_actor_output_squashing, ACT,
-                                A->d_actor_output, 2 * ACT, A->log_alpha.parameters, A->log_alpha.gradient, K.reset, R, ACT))) return rc;   // :464
+    void* counters = nullptr;
+    if ((rc = rlt_counters(device, &counters))) return rc;
+    SequenceActorGradient gradient = {};
+    gradient.sas = A->sas; gradient.final_step = K.final_step_mask; gradient.reset = K.reset; gradient.policy = actor_out; gradient.noise = action_noise;
+    gradient.actions = A->actor_actions; gradient.pre_squashing = A->actor_pre_squashing; gradient.log_alpha = A->log_alpha.parameters;
+    for (int k = 0; k < 2; k++) { gradient.q[k] = seq_output(A->critics[k], A->n_critic_layers); gradient.d_critic_input[k] = A->d_critic_input[k]; }
+    gradient.d_action = A->d_actor_output_squashing; gradient.d_policy = A->d_actor_output; gradient.d_log_alpha = A->log_alpha.gradient;
+    gradient.partial = (float*)((char*)counters + 256); gradient.tickets = rlt_tickets_of(counters, 0);
+    gradient.rows = R; gradient.obs = OBS; gradient.act = ACT;
+    hipLaunchKernelGGL(sequence_actor_gradient_kernel, dim3(sequence_grid(R)), dim3(256), 0, device->stream, gradient);                    // :460-464
+    if ((rc = rlt_launch_status(device))) return rc;
     if (stacked) {
         const rlt_stack_backward backward = {A->actor, obs, D, A->d_actor_output, nullptr, K.reset, S, B, 1, 1, ws};
         if ((rc = rlt_seq_stack_backward(device, &backward, 1))) return rc;

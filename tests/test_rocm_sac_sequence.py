@@ -135,6 +135,30 @@ def test_sac_sequence_updates_at_larger_shapes(oracle, rocm, case):
         compare_agents(agents[1], agents[0], (case, i), tol=2e-5)
 
 
+@pytest.mark.parametrize("case", [(1, 1, 0), (7, 13, 3), (3, 85, 1), (2, 60001, 2)])
+def test_sac_sequence_updates_at_the_edges_of_the_steps_between_the_passes(oracle, rocm, case):
+    """One row, rows that fill neither a workgroup nor a word of the masks, masks off word boundaries, and more rows than the launches have threads; one loop step. The tolerance is
+    that of the larger shapes (fp32 sums over the rows in another order)."""
+    print("case", case, flush=True)
+    S, B, shift = case
+    OBS, ACT, H = 5, 2, 16
+    rng = np.random.default_rng(S + B)
+    actor_specs = [(0, OBS, H, "relu"), (1, H, H, "identity"), (0, H, 2 * ACT, "identity")]
+    critic_specs = [(0, OBS + ACT, H, "relu"), (1, H, H, "identity"), (0, H, 1, "identity")]
+    critics = [helpers.random_seq_params(rng, critic_specs) for _ in range(2)]
+    params = np.concatenate([helpers.random_seq_params(rng, actor_specs)] + critics + [c.copy() for c in critics] + [np.array([np.log(0.5)], np.float32)])
+    hyper = dict(sas=helpers.capi.SasParameters(-20.0, 2.0, 1e-6, -float(ACT)))
+    agents = [helpers.SacSequenceOnBackend(be, actor_specs, critic_specs, params, S, B, OBS, ACT, True, hyper) for be in (oracle, rocm)]
+    data = synthetic_sequence_batch(rng, S, B, OBS + ACT)
+    shifted = {k: rocm.array(np.concatenate([np.zeros(shift, np.uint8), data[k].ravel()])) for k in ("final_step_mask", "next_final_step_mask_base", "reset")}
+    for k, m in shifted.items():
+        setattr(agents[1].c.batch, k, m.offset(shift))
+    nc, na = rng.standard_normal((S + 1, B, ACT)).astype(np.float32), rng.standard_normal((S, B, ACT)).astype(np.float32)
+    for a in agents:
+        a.set_batch(data); a.train(nc, na)
+    compare_agents(agents[1], agents[0], case, tol=2e-5)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", [(100, 100, 3, 1, 32, True), (10, 100, 5, 2, 32, False), (48, 64, 11, 3, 64, True)])
 def test_both_critics_in_one_call_leave_the_bits_of_the_two_calls(rocm, case):
