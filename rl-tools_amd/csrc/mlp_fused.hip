@@ -6,7 +6,7 @@
 // ~0.4 GB of HBM traffic per call for 27.5 GFLOP, and eleven launches.
 //
 // Here one persistent workgroup per compute unit (4 wavefronts, one per SIMD, up to 512 registers each) walks over tiles of 64
-// batch rows. Per tile, in LDS: h1 and h2 (64 x 256 each, row stride 257), the input rows (64 x 33) and the output gradient
+// batch rows. Per tile, in LDS: h1 and h2 (64 x 256 each, row stride 260), the input rows (64 x 33) and the output gradient
 // (64 x 17). Per tile, on v_mfma_f32_32x32x2_f32 unless noted:
 //   P1  h1 = act(x W1^T + b1)                       K = in
 //   P2  h2 = act(h1 W2^T + b2)                      K = 256, W2 read from L2 in a pre-swizzled layout, one dwordx4 per 4 k-steps
@@ -29,6 +29,7 @@
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(3))) float* lptr;
+typedef __attribute__((address_space(3))) floatx4* lptr4;
 
 extern __shared__ __attribute__((aligned(16))) float rlt_mlp3_lds[];
 
@@ -36,7 +37,7 @@ namespace {
 
 constexpr int HID = 256;     // hidden width the kernel is built for
 constexpr int BM = 64;       // batch rows per tile
-constexpr int HS = HID + 1;  // LDS row stride of h1 / h2: odd, so that 32 rows read side by side fall into 32 banks
+constexpr int HS = HID + 4;  // LDS row stride of h1 / h2: 16 bytes of each of sixteen rows side by side fill the 64 banks
 constexpr int XSP = 33;      // LDS row stride of the input rows (in <= 32, zero padded)
 constexpr int DS = 17;       // LDS row stride of the output-gradient rows (out <= 16, zero padded)
 constexpr int THREADS = 256;
@@ -93,8 +94,8 @@ __device__ __forceinline__ void steps_dispatch(int steps, F&& body) {
 // Operand layouts of the matrix instructions (lane l):
 //   32x32x2: A[row l%32][k l/32], B[k l/32][col l%32], result v -> row 8(v/4) + 4(l/32) + v%4, col l%32
 //   16x16x4: A[row l%16][k l/16], B[k l/16][col l%16], result v -> row 4(l/16) + v, col l%16
-// w2f[nt][g][l][t] = W2[32nt + l%32][2(4g+t) + l/32]    B operand of h1 W2^T   for column tile nt, k-step 4g+t
-// w2b[it][g][l][t] = W2[2(4g+t) + l/32][32it + l%32]    B operand of d_pre2 W2 for column tile it
+// w2f[nt][g][l][t] = W2[32nt + l%32][8g + 4(l/32) + t]    B operand of h1 W2^T   for column tile nt, k-step 4g+t: the four steps of a group take eight consecutive k, so
+// w2b[it][g][l][t] = W2[8g + 4(l/32) + t][32it + l%32]    B operand of d_pre2 W2 for column tile it              that a lane's A operands of a group are 16 bytes
 // w1s[nt][j][l]    = W1[32nt + l%32][2j + l/32]         (0 beyond in)
 // W3 (out x 256) is small enough to sit in LDS for the whole launch (rows padded to 16 with zeros).
 __global__ void mlp3_prepare_kernel(const float* __restrict__ W1, const float* __restrict__ W2, int in, float* __restrict__ prep) {
@@ -102,7 +103,7 @@ __global__ void mlp3_prepare_kernel(const float* __restrict__ W1, const float* _
     float* w2f = prep; float* w2b = w2f + W2F_FLOATS; float* w1s = w2b + W2B_FLOATS;
     if (idx < 65536) {
         const int t = idx & 3, l = (idx >> 2) & 63, g = (idx >> 8) & 31, tile = idx >> 13;
-        const int k = 2 * (4 * g + t) + (l >> 5), c = 32 * tile + (l & 31);
+        const int k = 8 * g + 4 * (l >> 5) + t, c = 32 * tile + (l & 31);
         w2f[idx] = W2[c * HID + k];
         w2b[idx] = W2[k * HID + c];
     }
@@ -114,30 +115,30 @@ __global__ void mlp3_prepare_kernel(const float* __restrict__ W1, const float* _
 }
 
 // 64 x 64 block of  A[64 x 256] (LDS, row stride HS) times a pre-swizzled 256 x 256 weight: wavefront w owns column tiles 2w, 2w+1.
-// The LDS operands of k-step s+1 and the weight group two ahead are requested before the matrix instructions of step s are issued.
+// The LDS operands of the next group of four k-steps and the weight group two ahead are requested before the matrix instructions of a group are issued.
 __device__ __forceinline__ void contract_256(lptr a, const float* __restrict__ wsw, int w, int lane, floatx16 (&acc)[2][2]) {
     const int c32 = lane & 31, hi = lane >> 5;
     const floatx4* b0p = reinterpret_cast<const floatx4*>(wsw) + (size_t)(2 * w) * 32 * 64 + lane;
     const floatx4* b1p = b0p + 32 * 64;
-    const lptr a0 = a + c32 * HS + hi, a1 = a0 + 32 * HS;
+    const lptr a0 = a + c32 * HS + 4 * hi, a1 = a0 + 32 * HS;
     floatx4 b0 = b0p[0], b1 = b1p[0];
     floatx4 n0 = b0p[64], n1 = b1p[64];
-    float x0 = a0[0], x1 = a1[0];
+    floatx4 x0 = *(lptr4)a0, x1 = *(lptr4)a1;
 #pragma unroll       // fully unrolled: the rotation of the prefetch registers becomes renaming instead of copies that wait for the loads
     for (int g = 0; g < 32; g++) {
         const int gp = g + 2 < 32 ? g + 2 : 31;      // two groups ahead; the last iterations re-read the final group
+        const int next = g + 1 < 32 ? g + 1 : 31;
         const floatx4 p0 = b0p[gp * 64], p1 = b1p[gp * 64];
+        const floatx4 y0 = *(lptr4)(a0 + 8 * next), y1 = *(lptr4)(a1 + 8 * next);
         __builtin_amdgcn_sched_barrier(0);      // the requests above are not to be moved down to their first use
 #pragma unroll
         for (int t = 0; t < 4; t++) {
-            const int next = 4 * g + t + 1 < 128 ? 4 * g + t + 1 : 127;
-            const float y0 = a0[2 * next], y1 = a1[2 * next];
-            acc[0][0] = mfma32(x0, b0[t], acc[0][0]);
-            acc[0][1] = mfma32(x0, b1[t], acc[0][1]);
-            acc[1][0] = mfma32(x1, b0[t], acc[1][0]);
-            acc[1][1] = mfma32(x1, b1[t], acc[1][1]);
-            x0 = y0; x1 = y1;
+            acc[0][0] = mfma32(x0[t], b0[t], acc[0][0]);
+            acc[0][1] = mfma32(x0[t], b1[t], acc[0][1]);
+            acc[1][0] = mfma32(x1[t], b0[t], acc[1][0]);
+            acc[1][1] = mfma32(x1[t], b1[t], acc[1][1]);
         }
+        x0 = y0; x1 = y1;
         b0 = n0; b1 = n1; n0 = p0; n1 = p1;
     }
 }
@@ -157,7 +158,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
         for (int b = 0; b < 8; b++) aW2[a][b] = zero16; }
 #pragma unroll
     for (int t = 0; t < 4; t++) aW3[t] = zero4;
-    float db1 = 0.f, db2 = 0.f, db3 = 0.f;
+    // bias gradients: each lane's share of its columns, formed where the values are in registers anyway and added up across the lanes at the end of the launch
+    float db1[2] = {0.f, 0.f}, db2[2] = {0.f, 0.f}, db3[4] = {0.f, 0.f, 0.f, 0.f};
     const float bias1[2] = {A.b1[32 * (2 * w) + (lane_invariant & 31)], A.b1[32 * (2 * w + 1) + (lane_invariant & 31)]};
     const float bias2[2] = {A.b2[32 * (2 * w) + (lane_invariant & 31)], A.b2[32 * (2 * w + 1) + (lane_invariant & 31)]};
     const float bias3 = (lane_invariant & 15) < A.out ? A.b3[lane_invariant & 15] : 0.f;
@@ -199,7 +201,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
         for (int u = 0; u < NX; u++) xs[(tid >> 2) * XSP + (tid & 3) + 4 * u] = vx[u];
         if (MODE != MODE_FORWARD) {
 #pragma unroll
-            for (int u = 0; u < ND; u++) dp3[(tid >> 2) * DS + (tid & 3) + 4 * u] = vd[u];
+            for (int u = 0; u < ND; u++) { dp3[(tid >> 2) * DS + (tid & 3) + 4 * u] = vd[u]; if (MODE == MODE_BACKWARD) db3[u] += vd[u]; }
         }
         float wf[2][16];
         if (MODE != MODE_BACKWARD) {
@@ -226,7 +228,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
                         const int idx = tid + THREADS * (i0 + i), row = idx >> 6, c4 = (idx & 63) * 4;
                         const bool ok = r0 + row < A.batch;
 #pragma unroll
-                        for (int e = 0; e < 4; e++) dst[row * HS + c4 + e] = ok ? v[i][e] : 0.f;
+                        for (int e = 0; e < 4; e++) if (!ok) v[i][e] = 0.f;
+                        *(lptr4)(dst + row * HS + c4) = v[i];
                     }
                 }
             }
@@ -292,12 +295,16 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
             floatx4 acc = zero4, acc2 = zero4;
             const lptr wp = w3l + r16 * HS + 64 * q;
             const lptr ap = h2 + (16 * w + r16) * HS + 64 * q;
-#pragma unroll 16
-            for (int u = 0; u < 64; u += 2) {
-                acc = mfma16(ap[u], wp[u], acc);
-                acc2 = mfma16(ap[u + 1], wp[u + 1], acc2);
+#pragma unroll
+            for (int u = 0; u < 64; u += 4) {
+                const floatx4 av = *(lptr4)(ap + u), wv = *(lptr4)(wp + u);
+                acc = mfma16(av[0], wv[0], acc);
+                acc2 = mfma16(av[1], wv[1], acc2);
+                acc = mfma16(av[2], wv[2], acc);
+                acc2 = mfma16(av[3], wv[3], acc2);
             }
             acc += acc2;
+            float column = 0.f;
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 const int row = 16 * w + 4 * q + v, grow = r0 + row;
@@ -310,32 +317,36 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
                     const float raw = dp3[row * DS + r16];
                     float d = A.target ? (yv - raw) * A.mse_scale : raw;
                     d *= rlt_dact_from_output(yv, A.act3);
-                    dp3[row * DS + r16] = ok ? d : 0.f;
+                    d = ok ? d : 0.f;
+                    dp3[row * DS + r16] = d;
+                    column += d;
                 }
             }
+            if (MODE == MODE_FUSED) db3[0] += column;
             rlt_lds_barrier();
         }
         RLT_TICK(3)
         if (MODE == MODE_FORWARD) continue;
-        // ---- P4: dW3 += d_pre3^T h2 (rows = outputs, wavefront w owns columns [64w, 64w+64)); db3
-#pragma unroll 8
-        for (int j = 0; j < 16; j++) {
-            const float a = dp3[(4 * j + q) * DS + r16];
+        // ---- P4: dW3 += d_pre3^T h2 (rows = outputs, wavefront w owns columns [64w, 64w+64)); the operands of the next four rows requested before these rows' matrix instructions
+        {
+            const lptr dp = dp3 + q * DS + r16, hp = h2 + q * HS + 64 * w + r16;
+            float a = dp[0], b[4];
 #pragma unroll
-            for (int t = 0; t < 4; t++) aW3[t] = mfma16(a, h2[(4 * j + q) * HS + 64 * w + 16 * t + r16], aW3[t]);
-        }
-        if (tid < 16) {
-            float s = 0.f;
-#pragma unroll 1
-            for (int rb = 0; rb < BM; rb += 8) {
-                float v[8];
+            for (int t = 0; t < 4; t++) b[t] = hp[16 * t];
 #pragma unroll
-                for (int u = 0; u < 8; u++) v[u] = dp3[(rb + u) * DS + tid];
+            for (int j = 0; j < 16; j++) {
+                const int next = j + 1 < 16 ? j + 1 : j;
+                const float na = dp[4 * next * DS];
+                float nb[4];
+#pragma unroll
+                for (int t = 0; t < 4; t++) nb[t] = hp[4 * next * HS + 16 * t];
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int u = 0; u < 8; u++) s += v[u];
+                for (int t = 0; t < 4; t++) aW3[t] = mfma16(a, b[t], aW3[t]);
+                a = na;
+#pragma unroll
+                for (int t = 0; t < 4; t++) b[t] = nb[t];
             }
-            db3 += s;
         }
         rlt_lds_barrier();
         RLT_TICK(4)
@@ -343,7 +354,11 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
 #pragma unroll
         for (int a = 0; a < 2; a++) {
             const int nt = 2 * w + a;
-            floatx16 acc[2] = {zero16, zero16};
+            floatx16 acc[2] = {zero16, zero16}, hv[2];      // the outputs that the derivative is taken from travel while the products are formed
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) hv[mt][v] = h2[(32 * mt + row32(v, hi)) * HS + 32 * nt + c32];
             steps_dispatch(nk3, [&](auto steps) { constexpr int NK = decltype(steps)::value < 8 ? decltype(steps)::value : 8;
                 float da[2][NK], wb[NK];
 #pragma unroll
@@ -351,23 +366,22 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
 #pragma unroll
                 for (int j = 0; j < NK; j++) { acc[0] = mfma32(da[0][j], wb[j], acc[0]); acc[1] = mfma32(da[1][j], wb[j], acc[1]); }
             });
+            float column = 0.f;
             act_dispatch(A.act2, [&](auto kind) { constexpr int ACT = decltype(kind)::value;
 #pragma unroll
-            for (int mt = 0; mt < 2; mt++) {
+                for (int mt = 0; mt < 2; mt++)
 #pragma unroll
-                for (int vb = 0; vb < 16; vb += 8) {
-                    float hv[8];
-#pragma unroll
-                    for (int v = 0; v < 8; v++) hv[v] = h2[(32 * mt + row32(vb + v, hi)) * HS + 32 * nt + c32];
-#pragma unroll
-                    for (int v = 0; v < 8; v++) h2[(32 * mt + row32(vb + v, hi)) * HS + 32 * nt + c32] = acc[mt][vb + v] * dact_c<ACT>(hv[v]);
-                }
-            }
+                    for (int v = 0; v < 16; v++) {
+                        const float d = acc[mt][v] * dact_c<ACT>(hv[mt][v]);
+                        h2[(32 * mt + row32(v, hi)) * HS + 32 * nt + c32] = d;
+                        column += d;
+                    }
             });
+            db2[a] += column;
         }
         rlt_lds_barrier();
         RLT_TICK(5)
-        // ---- P6: dW2 += d_pre2^T h1 (wavefront w owns row tiles 2w, 2w+1 of it); db2; d_h1 = d_pre2 W2
+        // ---- P6: dW2 += d_pre2^T h1 (wavefront w owns row tiles 2w, 2w+1 of it); d_h1 = d_pre2 W2
         {
             const lptr dbase = h2 + hi * HS + c32 + 32 * (2 * w), hbase = h1 + hi * HS + c32;
             float a0 = dbase[0], a1 = dbase[32], bv[8];
@@ -391,19 +405,6 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
             }
         }
         {
-            float s = 0.f;
-#pragma unroll 1
-            for (int rb = 0; rb < BM; rb += 8) {
-                float v[8];
-#pragma unroll
-                for (int u = 0; u < 8; u++) v[u] = h2[(rb + u) * HS + tid];
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int u = 0; u < 8; u++) s += v[u];
-            }
-            db2 += s;
-        }
-        {
             floatx16 acc[2][2] = {{zero16, zero16}, {zero16, zero16}};
             contract_256(h2, A.w2b, w, lane, acc);
             rlt_lds_barrier();      // every wavefront is done reading h1
@@ -411,42 +412,42 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
             // ---- P7: d_pre1 = d_h1 * act'(h1), in place of h1
             act_dispatch(A.act1, [&](auto kind) { constexpr int ACT = decltype(kind)::value;
 #pragma unroll
-            for (int mt = 0; mt < 2; mt++)
+            for (int a = 0; a < 2; a++) {
+                float column = 0.f;
 #pragma unroll
-                for (int a = 0; a < 2; a++) {
+                for (int mt = 0; mt < 2; mt++) {
+                    float hv[16];
 #pragma unroll
-                    for (int vb = 0; vb < 16; vb += 8) {
-                        float hv[8];
+                    for (int v = 0; v < 16; v++) hv[v] = h1[(32 * mt + row32(v, hi)) * HS + 32 * (2 * w + a) + c32];
 #pragma unroll
-                        for (int v = 0; v < 8; v++) hv[v] = h1[(32 * mt + row32(vb + v, hi)) * HS + 32 * (2 * w + a) + c32];
-#pragma unroll
-                        for (int v = 0; v < 8; v++) h1[(32 * mt + row32(vb + v, hi)) * HS + 32 * (2 * w + a) + c32] = acc[mt][a][vb + v] * dact_c<ACT>(hv[v]);
+                    for (int v = 0; v < 16; v++) {
+                        const float d = acc[mt][a][v] * dact_c<ACT>(hv[v]);
+                        h1[(32 * mt + row32(v, hi)) * HS + 32 * (2 * w + a) + c32] = d;
+                        column += d;
                     }
                 }
+                db1[a] += column;
+            }
             });
         }
         rlt_lds_barrier();
         RLT_TICK(7)
-        // ---- P8: dW1 += d_pre1^T x ; db1
-#pragma unroll 8
-        for (int k = 0; k < BM / 2; k++) {
-            const float bv = xs[(2 * k + hi) * XSP + c32];
-            const lptr dr = h1 + (2 * k + hi) * HS + c32;
-            aW1[0] = mfma32(dr[32 * (2 * w)], bv, aW1[0]);
-            aW1[1] = mfma32(dr[32 * (2 * w + 1)], bv, aW1[1]);
-        }
+        // ---- P8: dW1 += d_pre1^T x, two row pairs at a time, the operands of the next two requested before these ones' matrix instructions
         {
-            float s = 0.f;
-#pragma unroll 1
-            for (int rb = 0; rb < BM; rb += 8) {
-                float v[8];
-#pragma unroll
-                for (int u = 0; u < 8; u++) v[u] = h1[(rb + u) * HS + tid];
+            const lptr xp = xs + hi * XSP + c32, dp = h1 + hi * HS + c32 + 32 * (2 * w);
+            float x0 = xp[0], x1 = xp[2 * XSP], d0[2] = {dp[0], dp[32]}, d1[2] = {dp[2 * HS], dp[2 * HS + 32]};
+#pragma unroll 4
+            for (int k = 0; k < BM / 2; k += 2) {
+                const int next = k + 2 < BM / 2 ? k + 2 : k;
+                const float nx0 = xp[2 * next * XSP], nx1 = xp[2 * (next + 1) * XSP];
+                const float nd0[2] = {dp[2 * next * HS], dp[2 * next * HS + 32]}, nd1[2] = {dp[2 * (next + 1) * HS], dp[2 * (next + 1) * HS + 32]};
                 __builtin_amdgcn_sched_barrier(0);
+                aW1[0] = mfma32(d0[0], x0, aW1[0]); aW1[1] = mfma32(d0[1], x0, aW1[1]);
+                aW1[0] = mfma32(d1[0], x1, aW1[0]); aW1[1] = mfma32(d1[1], x1, aW1[1]);
+                x0 = nx0; x1 = nx1;
 #pragma unroll
-                for (int u = 0; u < 8; u++) s += v[u];
+                for (int a = 0; a < 2; a++) { d0[a] = nd0[a]; d1[a] = nd1[a]; }
             }
-            db1 += s;
         }
         rlt_lds_barrier();
         RLT_TICK(8)
@@ -470,8 +471,26 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
     for (int t = 0; t < 4; t++)
 #pragma unroll
         for (int v = 0; v < 4; v++) { const int o = 4 * q + v; if (o < A.out) pW3[o * HID + 64 * w + 16 * t + r16] = aW3[t][v]; }
-    pb1[tid] = db1; pb2[tid] = db2;
-    if (tid < A.out) pb3[tid] = db3;
+    // the two halves of a wavefront hold the same columns' sums over different rows; the last layer's are spread over every thread
+#pragma unroll
+    for (int a = 0; a < 2; a++) {
+        const float s1 = db1[a] + __shfl_xor(db1[a], 32, 64), s2 = db2[a] + __shfl_xor(db2[a], 32, 64);
+        if (hi == 0) { pb1[32 * (2 * w + a) + c32] = s1; pb2[32 * (2 * w + a) + c32] = s2; }
+    }
+    constexpr int SHARES = MODE == MODE_BACKWARD ? BM : 16;      // per column: one per row of a tile, or one per sixteen lanes
+    if (MODE == MODE_BACKWARD) {
+#pragma unroll
+        for (int u = 0; u < ND; u++) dp3[(tid >> 2) * DS + (tid & 3) + 4 * u] = db3[u];
+    } else dp3[(4 * w + q) * DS + r16] = db3[0];
+    rlt_lds_barrier();
+    if (tid < A.out) {
+        float s[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int i = 0; i < SHARES; i += 4)
+#pragma unroll
+            for (int u = 0; u < 4; u++) s[u] += dp3[(i + u) * DS + tid];
+        pb3[tid] = (s[0] + s[1]) + (s[2] + s[3]);
+    }
 #ifdef RLT_MLP3_PROFILE
     RLT_TICK(9)
     if (blockIdx.x == 0 && threadIdx.x == 0) {
