@@ -1,18 +1,20 @@
 // Single-pass forward + backward of a 3-layer MLP in -> 64 -> 64 -> out for the narrow networks of PPO, TD3 and SAC
 // (nn_models/mlp/operations_generic.h:128-181 forward, :183-260 backward; nn/layers/dense/operations_generic.h:98-260).
 //
-// A workgroup of four wavefronts takes 64 batch rows per round. The work is split two ways:
-//   by rows      each wavefront runs its own 16 rows through the three layers, the loss and the input-gradient products
+// A workgroup of eight wavefronts takes 64 batch rows per round. The work is split two ways; wavefront w has row tile rt = w % 4 and half = w / 4 of the columns:
+//   by rows      four pairs of wavefronts run 16 rows each through the three layers, the loss and the input-gradient products, each wavefront half the columns of a layer
 //                  h1 = f(x W1^T + b1), h2 = f(h1 W2^T + b2), y = g(h2 W3^T + b3), d_pre3 from the caller's d_output / an MSE target / PPO's
 //                  clipped surrogate, d_pre2 = (d_pre3 W3) f'(h2), d_pre1 = (d_pre2 W2) f'(h1)
 //   by columns   for the weight gradients dW3 += d_pre3^T h2, dW2 += d_pre2^T h1, dW1 += d_pre1^T x the reduction runs over all 64 rows of the
-//                  round, and wavefront w owns the 16 output rows 16 w .. 16 w + 15 of dW1 and dW2 and 16 columns of dW3
+//                  round, and a wavefront owns the 16 output rows 16 rt .. 16 rt + 15 of half the columns of dW1 and dW2 (the second half 16 columns of dW3 too)
 // so every accumulator tile of a weight gradient lives in exactly one wavefront's registers for the whole kernel (8 + 4 + 1 tiles), no sums
 // are exchanged between wavefronts, and a workgroup writes one block of partial sums at the end, which a second kernel adds to the layers'
 // gradients in workgroup order: the result does not depend on scheduling. Activations and gradients of the round sit in LDS in the layouts
 // v_mfma_f32_16x16x4_f32 wants (lane l = r + 16 kk feeds A[r][kk] and B[kk][r] and receives D[4 kk + v][r], v = 0..3); the weights are staged
 // once per workgroup in LDS (padded rows, read as both W and W^T). Four workgroup barriers per round order the two kinds of phase.
-// Bound: the fp32 matrix pipe, 2 (in + 64 + out) 64 flop per row forward and twice that backward less the input gradient of layer 1.
+// Bound: latency. One round is 460 matrix instructions per SIMD (14.7 K cycles at 105 -> 64 -> 64 -> 8), between LDS round trips and the activations' chains, and 141 KB of LDS leave room
+// for one workgroup per compute unit: two wavefronts per SIMD instead of one (four that had all columns of their rows) took PPO's pair at 8,192 rows from 30.0 to 25.6 us and the
+// head 64 -> 64 -> 4 of a sequence model at 65,536 rows from 56.2 to 47.2 us, with the same sums in the same order.
 #include "mlp_small.h"
 #include "optim.h"
 #include "xcd_reduce.h"
@@ -20,7 +22,7 @@
 namespace {
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) float* lptr;
-constexpr int H = 64, HS = H + 1, WAVES = 4, ROWS = 16 * WAVES, THREADS = 64 * WAVES, MAX_IN = 128, MAX_OUT = 16, MAX_NT1 = MAX_IN / 16, D3S = MAX_OUT + 1,
+constexpr int H = 64, HS = H + 1, WAVES = 8, ROW_TILES = 4, ROWS = 16 * ROW_TILES, THREADS = 64 * WAVES, MAX_IN = 128, MAX_OUT = 16, MAX_NT1 = MAX_IN / 16, D3S = MAX_OUT + 1,
               N_EXTRA = 16, N_SUMS = 2 * H + MAX_OUT + N_EXTRA;
 enum { LOSS_GIVEN = 0, LOSS_MSE = 1, LOSS_PPO = 2 };
 
@@ -43,13 +45,6 @@ __device__ __forceinline__ floatx4 mfma16(float a, float b, floatx4 c) { return 
 template <int CTRL>
 __device__ __forceinline__ float dpp(float x) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, true)); }
 __device__ __forceinline__ float row16_sum(float x) { asm volatile("" : "+v"(x)); /* keeps a producing multiplication out of the first addition: all lanes then hold the same sum */ x += dpp<0xB1>(x); x += dpp<0x4E>(x); x += dpp<0x141>(x); x += dpp<0x140>(x); return x; }
-// lanes of one wavefront exchange data through LDS: the hardware executes a wavefront's LDS instructions in order, the fences keep
-// the compiler from moving them across
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 // sum over the four lane groups (lanes r, r + 16, r + 32, r + 48), in a fixed order
 __device__ __forceinline__ float groups_sum(float v) { asm volatile("" : "+v"(v)); v += __shfl_xor(v, 16, 64); v += __shfl_xor(v, 32, 64); return v; }
 
@@ -62,13 +57,13 @@ constexpr size_t lds_floats(int nt1c) {
 // global loads of one tile of 16 rows, issued together: the inputs (lane = column, up to two columns per lane) and what the loss needs of the
 // rows this lane will hold after the forward pass (rows 4 kk + v, column r); columns beyond the extent are clamped here and masked later.
 // `vrows`: the rows' indices, requested a round earlier so that nothing waits for them here.
-struct TileRegs { float xa[16], xb[16], in0[4], in1[4], in2[4]; };
-__device__ __forceinline__ void request_tile(const SmallArgs& A, uint32_t vrows, int lane, TileRegs& T) {
+struct TileRegs { float xa[8], xb[8], in0[4], in1[4], in2[4]; };
+__device__ __forceinline__ void request_tile(const SmallArgs& A, uint32_t vrows, int lane, int half, TileRegs& T) {
     const int r = lane & 15, kk = lane >> 4;
     const int c0 = min(lane, A.in - 1), c1 = min(64 + lane, A.in - 1), c = min(r, A.out - 1);
 #pragma unroll
-    for (int row = 0; row < 16; row++) {
-        const float* src = A.x + (size_t)(uint32_t)__builtin_amdgcn_readlane((int)vrows, row) * A.ldx;      // wavefront-uniform: scalar address arithmetic
+    for (int row = 0; row < 8; row++) {
+        const float* src = A.x + (size_t)(uint32_t)__builtin_amdgcn_readlane((int)vrows, 8 * half + row) * A.ldx;      // wavefront-uniform: scalar address arithmetic
         T.xa[row] = src[c0];
         T.xb[row] = A.in > 64 ? src[c1] : 0.f;
     }
@@ -76,6 +71,7 @@ __device__ __forceinline__ void request_tile(const SmallArgs& A, uint32_t vrows,
     for (int v = 0; v < 4; v++) {
         const size_t row = (size_t)(uint32_t)__shfl((int)vrows, 4 * kk + v, 64);
         T.in0[v] = T.in1[v] = T.in2[v] = 0.f;
+        if (half != 0) continue;      // the loss is the first half's
         if (A.loss == LOSS_GIVEN) T.in0[v] = A.d_output[row * A.ldd + c];
         else if (A.loss == LOSS_MSE) T.in0[v] = A.target[row * A.ldt + c];
         else { T.in0[v] = A.actions[row * A.ld_actions + c]; T.in1[v] = A.advantages[row * A.ld_adv]; T.in2[v] = A.log_probs[row * A.ld_lp]; }
@@ -113,15 +109,16 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K) {
     const int block = second ? blockIdx.x - groups0 : blockIdx.x, n_blocks = second ? gridDim.x - groups0 : groups0;
     const int lane = threadIdx.x & 63, r = lane & 15, kk = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);      // wavefront-uniform: addresses derived from it are computed on the scalar unit
+    const int rt = wave & 3, half = wave >> 2;      // row tile; half of every layer's columns
     const int IN = A.in, OUT = A.out, NT1 = (IN + 15) >> 4;
     constexpr int SX = 16 * NT1C + 1;        // row stride of the input tile and of W1 in LDS: a constant, so that LDS offsets fold into the instructions
     const lptr w1s = (lptr)lds_raw, w2s = w1s + H * SX, w3s = w2s + H * HS;
     const lptr xs_all = w3s + MAX_OUT * HS, h1s_all = xs_all + ROWS * SX, h2s_all = h1s_all + ROWS * HS, g2s_all = h2s_all + ROWS * HS, d3s_all = g2s_all + ROWS * HS;
-    const lptr xs = xs_all + 16 * wave * SX, h1s = h1s_all + 16 * wave * HS, h2s = h2s_all + 16 * wave * HS, g2s = g2s_all + 16 * wave * HS, d3s = d3s_all + 16 * wave * D3S;
-    const int n_tiles = (A.batch + 15) >> 4, n_rounds = (n_tiles + WAVES - 1) / WAVES;
+    const lptr xs = xs_all + 16 * rt * SX, h1s = h1s_all + 16 * rt * HS, h2s = h2s_all + 16 * rt * HS, g2s = g2s_all + 16 * rt * HS, d3s = d3s_all + 16 * rt * D3S;
+    const int n_tiles = (A.batch + 15) >> 4, n_rounds = (n_tiles + ROW_TILES - 1) / ROW_TILES;
     // lane l: the row of the input arrays that row (l & 15) of this wavefront's tile of round `round` reads; a tile beyond the batch is clamped here and masked later
     auto rows_of = [&](int round) -> uint32_t {
-        const int b = min(min(round * WAVES + wave, n_tiles - 1) * 16 + (lane & 15), A.batch - 1);
+        const int b = min(min(round * ROW_TILES + rt, n_tiles - 1) * 16 + (lane & 15), A.batch - 1);
         return A.rows ? A.rows[b] : (uint32_t)b;
     };
     // The launch's critical path starts with two dependent trips to memory (the row indices, then the rows): the index loads go out first, the
@@ -145,9 +142,9 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K) {
     for (int u = 0; u < H * H / THREADS; u++) v2[u] = LAYERS == 3 ? A.W2[u * THREADS + threadIdx.x] : 0.f;
 #pragma unroll
     for (int u = 0; u < MAX_OUT * H / THREADS; u++) v3[u] = A.W3[min(u * THREADS + (int)threadIdx.x, OUT * H - 1)];
-    float b1r[4], b2r[4];
+    float b1r[2], b2r[2];
 #pragma unroll
-    for (int nt = 0; nt < 4; nt++) { b1r[nt] = A.b1[16 * nt + r]; b2r[nt] = LAYERS == 3 ? A.b2[16 * nt + r] : 0.f; }
+    for (int nt = 0; nt < 2; nt++) { b1r[nt] = A.b1[16 * (2 * half + nt) + r]; b2r[nt] = LAYERS == 3 ? A.b2[16 * (2 * half + nt) + r] : 0.f; }
     const float b3r = A.b3[min(r, OUT - 1)];
     float ls = 0.f, adv_mean = 0.f, adv_std = 0.f;
     if (A.loss == LOSS_PPO) {
@@ -162,7 +159,7 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K) {
         sp0 = sp0 != 0.f ? sp0 : 1.f; sp1 = sp1 != 0.f ? sp1 : 1.f;
     }
     __builtin_amdgcn_sched_barrier(0);      // the loads above are issued before the first wait for the row indices
-    request_tile(A, rows_next, lane, T);
+    request_tile(A, rows_next, lane, half, T);
     RLT_TICK(1);
     // weights into LDS, rows padded to SX (zero beyond the input width, so the padded reduction steps add nothing)
     {
@@ -183,97 +180,103 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K) {
     rlt_lds_barrier();
 
     RLT_TICK(3);
-    // this wavefront's share of the weight gradients: rows 16 wave + 4 kk + v of dW1 (columns 16 nt + r) and of dW2, columns 16 wave + r of dW3 (rows 4 kk + v)
-    floatx4 aW1[NT1C], aW2[4], aW3a = zero4, aW3b = zero4;
+    // this wavefront's share of the weight gradients: rows 16 rt + 4 kk + v of half the columns of dW1 and of dW2 (tiles NT1H half + nt and 2 half + nt), and, in the second
+    // half (the first has the loss), columns 16 rt + r of dW3 (rows 4 kk + v)
+    constexpr int NT1H = NT1C / 2;
+    floatx4 aW1[NT1H], aW2[2], aW3a = zero4, aW3b = zero4;
 #pragma unroll
-    for (int nt = 0; nt < NT1C; nt++) aW1[nt] = zero4;
+    for (int nt = 0; nt < NT1H; nt++) aW1[nt] = zero4;
 #pragma unroll
-    for (int nt = 0; nt < 4; nt++) aW2[nt] = zero4;
-    float s1[4] = {0.f, 0.f, 0.f, 0.f}, s2[4] = {0.f, 0.f, 0.f, 0.f}, s3 = 0.f, gls = 0.f;      // bias gradients and the extra sums (PPO: log_std gradient; MSE: squared error) over this wavefront's rows
+    for (int nt = 0; nt < 2; nt++) aW2[nt] = zero4;
+    float s1[2] = {0.f, 0.f}, s2[2] = {0.f, 0.f}, s3 = 0.f, gls = 0.f;      // bias gradients and the extra sums (PPO: log_std gradient; MSE: squared error) over this wavefront's rows
 
     for (int round = block; round < n_rounds; round += n_blocks) {
-        const int tile = round * WAVES + wave, row0 = tile * 16;
+        const int tile = round * ROW_TILES + rt, row0 = tile * 16;
         // inputs of the tile into LDS, zero beyond the batch and beyond the input width
 #pragma unroll
-        for (int row = 0; row < 16; row++) {
+        for (int j = 0; j < 8; j++) {
+            const int row = 8 * half + j;
             const bool rok = row0 + row < A.batch;
-            if (lane < 16 * NT1C) xs[row * SX + lane] = (rok && lane < IN) ? (T.xa[row] - sm0) * sp0 : 0.f;
-            if (64 + lane < 16 * NT1C) xs[row * SX + 64 + lane] = (rok && 64 + lane < IN) ? (T.xb[row] - sm1) * sp1 : 0.f;
+            if (lane < 16 * NT1C) xs[row * SX + lane] = (rok && lane < IN) ? (T.xa[j] - sm0) * sp0 : 0.f;
+            if (64 + lane < 16 * NT1C) xs[row * SX + 64 + lane] = (rok && 64 + lane < IN) ? (T.xb[j] - sm1) * sp1 : 0.f;
         }
     RLT_TICK(4);
         float in0[4], in1[4], in2[4];
 #pragma unroll
         for (int v = 0; v < 4; v++) { in0[v] = T.in0[v]; in1[v] = T.in1[v]; in2[v] = T.in2[v]; }
-        wave_sync();
+        rlt_lds_barrier();      // both halves' rows of the tile are in place
         // the next round's loads travel while this one is computed, with row indices requested a round earlier
         if (round + n_blocks < n_rounds) {
             rows_next = rows_after;
             if (round + 2 * n_blocks < n_rounds) rows_after = rows_of(round + 2 * n_blocks);
-            request_tile(A, rows_next, lane, T);
+            request_tile(A, rows_next, lane, half, T);
         }
 
     RLT_TICK(5);
         // layer 1: groups of four reduction steps, the operands of the next group requested before this group's matrix instructions. Lane
         // group kk supplies input column 32 (g / 2) + 4 (g % 2) + q + koff with koff = 0, 16, 8, 24: the two lane groups that the LDS serves
         // together read columns 16 apart, that is different banks (rows are an odd number of floats apart)
-        floatx4 acc[4] = {zero4, zero4, zero4, zero4};
+        floatx4 acc[2] = {zero4, zero4};
+        const lptr w1h = w1s + 32 * half * SX, w2h = w2s + 32 * half * HS;      // this half's rows of W1 and W2
         {
             const int koff = 16 * (kk & 1) + 8 * (kk >> 1), n_groups = 2 * ((IN + 31) >> 5);
-            float a_c[4], b_c[4][4];
+            float a_c[4], b_c[4][2];
 #pragma unroll
             for (int q = 0; q < 4; q++) {
                 a_c[q] = xs[r * SX + koff + q];
 #pragma unroll
-                for (int nt = 0; nt < 4; nt++) b_c[q][nt] = w1s[(16 * nt + r) * SX + koff + q];
+                for (int nt = 0; nt < 2; nt++) b_c[q][nt] = w1h[(16 * nt + r) * SX + koff + q];
             }
             for (int g = 0; g < n_groups; g++) {
                 const int gn = min(g + 1, n_groups - 1), kn = 32 * (gn >> 1) + 4 * (gn & 1) + koff;
-                float a_n[4], b_n[4][4];
+                float a_n[4], b_n[4][2];
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
                     a_n[q] = xs[r * SX + kn + q];
 #pragma unroll
-                    for (int nt = 0; nt < 4; nt++) b_n[q][nt] = w1s[(16 * nt + r) * SX + kn + q];
+                    for (int nt = 0; nt < 2; nt++) b_n[q][nt] = w1h[(16 * nt + r) * SX + kn + q];
                 }
 #pragma unroll
                 for (int q = 0; q < 4; q++)
 #pragma unroll
-                    for (int nt = 0; nt < 4; nt++) acc[nt] = mfma16(a_c[q], b_c[q][nt], acc[nt]);
+                    for (int nt = 0; nt < 2; nt++) acc[nt] = mfma16(a_c[q], b_c[q][nt], acc[nt]);
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
                     a_c[q] = a_n[q];
 #pragma unroll
-                    for (int nt = 0; nt < 4; nt++) b_c[q][nt] = b_n[q][nt];
+                    for (int nt = 0; nt < 2; nt++) b_c[q][nt] = b_n[q][nt];
                 }
             }
         }
+        const int c0 = 32 * half + r;      // this lane's column of the half's first tile
 #pragma unroll
-        for (int nt = 0; nt < 4; nt++)
+        for (int nt = 0; nt < 2; nt++)
 #pragma unroll
-            for (int v = 0; v < 4; v++) h1s[(4 * kk + v) * HS + 16 * nt + r] = rlt_act(acc[nt][v] + b1r[nt], ACT_H);
-        wave_sync();
+            for (int v = 0; v < 4; v++) h1s[(4 * kk + v) * HS + 16 * nt + c0] = rlt_act(acc[nt][v] + b1r[nt], ACT_H);
+        rlt_lds_barrier();
 
     RLT_TICK(6);
         // layer 2
         if (LAYERS == 3) {
 #pragma unroll
-            for (int nt = 0; nt < 4; nt++) acc[nt] = zero4;
+            for (int nt = 0; nt < 2; nt++) acc[nt] = zero4;
 #pragma unroll
             for (int s = 0; s < 16; s++) {
                 const float a = h1s[r * HS + 16 * kk + s];
 #pragma unroll
-                for (int nt = 0; nt < 4; nt++) acc[nt] = mfma16(a, w2s[(16 * nt + r) * HS + 16 * kk + s], acc[nt]);
+                for (int nt = 0; nt < 2; nt++) acc[nt] = mfma16(a, w2h[(16 * nt + r) * HS + 16 * kk + s], acc[nt]);
             }
 #pragma unroll
-            for (int nt = 0; nt < 4; nt++)
+            for (int nt = 0; nt < 2; nt++)
 #pragma unroll
-                for (int v = 0; v < 4; v++) h2s[(4 * kk + v) * HS + 16 * nt + r] = rlt_act(acc[nt][v] + b2r[nt], ACT_H);
-            wave_sync();
+                for (int v = 0; v < 4; v++) h2s[(4 * kk + v) * HS + 16 * nt + c0] = rlt_act(acc[nt][v] + b2r[nt], ACT_H);
+            rlt_lds_barrier();
         }
         const lptr hls = LAYERS == 3 ? h2s : h1s, hls_all = LAYERS == 3 ? h2s_all : h1s_all;      // the last hidden layer's activations
 
     RLT_TICK(7);
         // layer 3 (two chains of matrix instructions) and the gradient at its pre-activations
+        if (half == 0) {
         floatx4 y0 = zero4, y1 = zero4;
 #pragma unroll
         for (int s = 0; s < 16; s += 2) {
@@ -309,36 +312,37 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K) {
             s3 += dp;
             d3s[(4 * kk + v) * D3S + r] = dp;
         }
+        }
     RLT_TICK(8);
         rlt_lds_barrier();      // every wavefront's last hidden activations and d_pre3 are in place
 
-        // dW3 (columns 16 wave + r) += d_pre3^T h over the 64 rows, two chains; in the weight gradients' reductions lane group kk supplies rows
-        // 16 kk + ks (wavefront kk's tile), so that the lane groups served together read different LDS banks
-        {
-            float a_c = d3s_all[16 * kk * D3S + r], b_c = hls_all[16 * kk * HS + 16 * wave + r];
+        // dW3 (columns 16 rt + r) += d_pre3^T h over the 64 rows, two chains; in the weight gradients' reductions lane group kk supplies rows
+        // 16 kk + ks (row tile kk), so that the lane groups served together read different LDS banks
+        if (half == 1) {
+            float a_c = d3s_all[16 * kk * D3S + r], b_c = hls_all[16 * kk * HS + 16 * rt + r];
 #pragma unroll
             for (int ks = 0; ks < ROWS / 4; ks++) {
                 const int kn = min(ks + 1, ROWS / 4 - 1);
-                const float a_n = d3s_all[(16 * kk + kn) * D3S + r], b_n = hls_all[(16 * kk + kn) * HS + 16 * wave + r];
+                const float a_n = d3s_all[(16 * kk + kn) * D3S + r], b_n = hls_all[(16 * kk + kn) * HS + 16 * rt + r];
                 if (ks & 1) aW3b = mfma16(a_c, b_c, aW3b); else aW3a = mfma16(a_c, b_c, aW3a);
                 a_c = a_n; b_c = b_n;
             }
         }
     RLT_TICK(9);
-        // d_pre2 = (d_pre3 W3) f'(h2) for the wavefront's own rows, into g2
+        // d_pre2 = (d_pre3 W3) f'(h2) for the wavefront's own rows and columns, into g2
 #pragma unroll
-        for (int nt = 0; nt < 4; nt++) acc[nt] = zero4;
+        for (int nt = 0; nt < 2; nt++) acc[nt] = zero4;
 #pragma unroll
         for (int ks = 0; ks < MAX_OUT / 4; ks++) {      // columns of d_pre3 and rows of W3 beyond `out` are zero
             const float a = d3s[r * D3S + 4 * ks + kk];
 #pragma unroll
-            for (int nt = 0; nt < 4; nt++) acc[nt] = mfma16(a, w3s[(4 * ks + kk) * HS + 16 * nt + r], acc[nt]);
+            for (int nt = 0; nt < 2; nt++) acc[nt] = mfma16(a, w3s[(4 * ks + kk) * HS + 16 * nt + c0], acc[nt]);
         }
 #pragma unroll
-        for (int nt = 0; nt < 4; nt++)
+        for (int nt = 0; nt < 2; nt++)
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                const int idx = (4 * kk + v) * HS + 16 * nt + r;
+                const int idx = (4 * kk + v) * HS + 16 * nt + c0;
                 const float dp = acc[nt][v] * rlt_dact_from_output(hls[idx], ACT_H);
                 if (LAYERS == 3) { g2s[idx] = dp; s2[nt] += dp; }
                 else { h2s[idx] = dp; s1[nt] += dp; }       // two layers: this is already the gradient at layer 1's pre-activations, kept where dW1 reads it
@@ -347,39 +351,39 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K) {
         rlt_lds_barrier();      // every wavefront's d_pre2 is in place, and nobody reads h2 any more
         if (LAYERS == 3) {
 
-        // dW2 (rows 16 wave + ..) += d_pre2^T h1 over the 64 rows
+        // dW2 (rows 16 rt + .., this half's columns) += d_pre2^T h1 over the 64 rows
         {
-            float a_c = g2s_all[16 * kk * HS + 16 * wave + r], b_c[4];
+            float a_c = g2s_all[16 * kk * HS + 16 * rt + r], b_c[2];
 #pragma unroll
-            for (int nt = 0; nt < 4; nt++) b_c[nt] = h1s_all[16 * kk * HS + 16 * nt + r];
+            for (int nt = 0; nt < 2; nt++) b_c[nt] = h1s_all[16 * kk * HS + 16 * nt + c0];
 #pragma unroll
             for (int ks = 0; ks < ROWS / 4; ks++) {
                 const int kn = min(ks + 1, ROWS / 4 - 1);
-                float a_n = g2s_all[(16 * kk + kn) * HS + 16 * wave + r], b_n[4];
+                float a_n = g2s_all[(16 * kk + kn) * HS + 16 * rt + r], b_n[2];
 #pragma unroll
-                for (int nt = 0; nt < 4; nt++) b_n[nt] = h1s_all[(16 * kk + kn) * HS + 16 * nt + r];
+                for (int nt = 0; nt < 2; nt++) b_n[nt] = h1s_all[(16 * kk + kn) * HS + 16 * nt + c0];
 #pragma unroll
-                for (int nt = 0; nt < 4; nt++) aW2[nt] = mfma16(a_c, b_c[nt], aW2[nt]);
+                for (int nt = 0; nt < 2; nt++) aW2[nt] = mfma16(a_c, b_c[nt], aW2[nt]);
                 a_c = a_n;
 #pragma unroll
-                for (int nt = 0; nt < 4; nt++) b_c[nt] = b_n[nt];
+                for (int nt = 0; nt < 2; nt++) b_c[nt] = b_n[nt];
             }
         }
     RLT_TICK(11);
-        // d_pre1 = (d_pre2 W2) f'(h1) for the wavefront's own rows, into the place of h2
+        // d_pre1 = (d_pre2 W2) f'(h1) for the wavefront's own rows and columns, into the place of h2
 #pragma unroll
-        for (int nt = 0; nt < 4; nt++) acc[nt] = zero4;
+        for (int nt = 0; nt < 2; nt++) acc[nt] = zero4;
 #pragma unroll
         for (int s = 0; s < 16; s++) {
             const float a = g2s[r * HS + 16 * kk + s];
 #pragma unroll
-            for (int nt = 0; nt < 4; nt++) acc[nt] = mfma16(a, w2s[(16 * kk + s) * HS + 16 * nt + r], acc[nt]);
+            for (int nt = 0; nt < 2; nt++) acc[nt] = mfma16(a, w2s[(16 * kk + s) * HS + 16 * nt + c0], acc[nt]);
         }
 #pragma unroll
-        for (int nt = 0; nt < 4; nt++)
+        for (int nt = 0; nt < 2; nt++)
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                const int idx = (4 * kk + v) * HS + 16 * nt + r;
+                const int idx = (4 * kk + v) * HS + 16 * nt + c0;
                 const float dp = acc[nt][v] * rlt_dact_from_output(h1s[idx], ACT_H);
                 h2s[idx] = dp; s1[nt] += dp;
             }
@@ -389,7 +393,7 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K) {
 
         // gradient with respect to the input, for the wavefront's own rows: d_x = d_pre1 W1, one tile of 16 input columns at a time
         if (A.d_input) {
-            for (int nt = 0; nt < NT1; nt++) {
+            for (int nt = half; nt < NT1; nt += 2) {
                 floatx4 dx = zero4;
 #pragma unroll
                 for (int s = 0; s < 16; s++) dx = mfma16(h2s[r * HS + 16 * kk + s], w1s[(16 * kk + s) * SX + 16 * nt + r], dx);
@@ -400,22 +404,23 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K) {
         }
 
     RLT_TICK(13);
-        // dW1 (rows 16 wave + ..) += d_pre1^T x over the 64 rows
+        // dW1 (rows 16 rt + .., this half's columns) += d_pre1^T x over the 64 rows
         {
-            float a_c = h2s_all[16 * kk * HS + 16 * wave + r], b_c[NT1C];
+            const lptr xh = xs_all + 16 * NT1H * half + r;
+            float a_c = h2s_all[16 * kk * HS + 16 * rt + r], b_c[NT1H];
 #pragma unroll
-            for (int nt = 0; nt < NT1C; nt++) b_c[nt] = xs_all[16 * kk * SX + 16 * nt + r];
+            for (int nt = 0; nt < NT1H; nt++) b_c[nt] = xh[16 * kk * SX + 16 * nt];
 #pragma unroll 4
             for (int ks = 0; ks < ROWS / 4; ks++) {
                 const int kn = min(ks + 1, ROWS / 4 - 1);
-                float a_n = h2s_all[(16 * kk + kn) * HS + 16 * wave + r], b_n[NT1C];
+                float a_n = h2s_all[(16 * kk + kn) * HS + 16 * rt + r], b_n[NT1H];
 #pragma unroll
-                for (int nt = 0; nt < NT1C; nt++) b_n[nt] = xs_all[(16 * kk + kn) * SX + 16 * nt + r];
+                for (int nt = 0; nt < NT1H; nt++) b_n[nt] = xh[(16 * kk + kn) * SX + 16 * nt];
 #pragma unroll
-                for (int nt = 0; nt < NT1C; nt++) aW1[nt] = mfma16(a_c, b_c[nt], aW1[nt]);
+                for (int nt = 0; nt < NT1H; nt++) aW1[nt] = mfma16(a_c, b_c[nt], aW1[nt]);
                 a_c = a_n;
 #pragma unroll
-                for (int nt = 0; nt < NT1C; nt++) b_c[nt] = b_n[nt];
+                for (int nt = 0; nt < NT1H; nt++) b_c[nt] = b_n[nt];
             }
         }
     RLT_TICK(14);
@@ -428,24 +433,26 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K) {
     const int o_b1 = H * IN, o_w2 = o_b1 + H, o_b2 = o_w2 + H * H, o_w3 = o_b2 + H, o_b3 = o_w3 + OUT * H, o_ex = o_b3 + OUT;
 #pragma unroll
     for (int v = 0; v < 4; v++) {
-        const int m = 16 * wave + 4 * kk + v;
+        const int m = 16 * rt + 4 * kk + v;
 #pragma unroll
-        for (int nt = 0; nt < NT1C; nt++)
-            if (nt < NT1 && 16 * nt + r < IN) dst[m * IN + 16 * nt + r] = aW1[nt][v];
+        for (int i = 0; i < NT1H; i++) {
+            const int nt = NT1H * half + i;
+            if (nt < NT1 && 16 * nt + r < IN) dst[m * IN + 16 * nt + r] = aW1[i][v];
+        }
 #pragma unroll
-        for (int nt = 0; nt < 4; nt++) dst[o_w2 + m * H + 16 * nt + r] = aW2[nt][v];
-        if (4 * kk + v < OUT) dst[o_w3 + (4 * kk + v) * H + 16 * wave + r] = aW3a[v] + aW3b[v];
+        for (int nt = 0; nt < 2; nt++) dst[o_w2 + m * H + 16 * (2 * half + nt) + r] = aW2[nt][v];
+        if (half == 1 && 4 * kk + v < OUT) dst[o_w3 + (4 * kk + v) * H + 16 * rt + r] = aW3a[v] + aW3b[v];
     }
     RLT_TICK(16);
-    // ... the bias and log_std gradients, which every wavefront holds for its own rows, summed in wavefront order through LDS
-    const lptr sums = (lptr)lds_raw;        // [WAVES][N_SUMS]; the weights are no longer needed
+    // ... the bias and log_std gradients, which every wavefront holds for its own rows and columns, summed in the order of the row tiles through LDS
+    const lptr sums = (lptr)lds_raw;        // [ROW_TILES][N_SUMS]; the weights are no longer needed
 #pragma unroll
-    for (int nt = 0; nt < 4; nt++) { s1[nt] = groups_sum(s1[nt]); s2[nt] = groups_sum(s2[nt]); }
+    for (int nt = 0; nt < 2; nt++) { s1[nt] = groups_sum(s1[nt]); s2[nt] = groups_sum(s2[nt]); }
     s3 = groups_sum(s3); gls = groups_sum(gls);
     if (kk == 0) {
 #pragma unroll
-        for (int nt = 0; nt < 4; nt++) { sums[wave * N_SUMS + 16 * nt + r] = s1[nt]; sums[wave * N_SUMS + H + 16 * nt + r] = s2[nt]; }
-        sums[wave * N_SUMS + 2 * H + r] = s3; sums[wave * N_SUMS + 2 * H + MAX_OUT + r] = gls;
+        for (int nt = 0; nt < 2; nt++) { sums[rt * N_SUMS + 32 * half + 16 * nt + r] = s1[nt]; sums[rt * N_SUMS + H + 32 * half + 16 * nt + r] = s2[nt]; }
+        if (half == 0) { sums[rt * N_SUMS + 2 * H + r] = s3; sums[rt * N_SUMS + 2 * H + MAX_OUT + r] = gls; }
     }
     rlt_lds_barrier();
     if (threadIdx.x < N_SUMS) {
