@@ -94,8 +94,9 @@ __device__ __forceinline__ void steps_dispatch(int steps, F&& body) {
 // Operand layouts of the matrix instructions (lane l):
 //   32x32x2: A[row l%32][k l/32], B[k l/32][col l%32], result v -> row 8(v/4) + 4(l/32) + v%4, col l%32
 //   16x16x4: A[row l%16][k l/16], B[k l/16][col l%16], result v -> row 4(l/16) + v, col l%16
-// w2f[nt][g][l][t] = W2[32nt + l%32][8g + 4(l/32) + t]    B operand of h1 W2^T   for column tile nt, k-step 4g+t: the four steps of a group take eight consecutive k, so
-// w2b[it][g][l][t] = W2[8g + 4(l/32) + t][32it + l%32]    B operand of d_pre2 W2 for column tile it              that a lane's A operands of a group are 16 bytes
+// w2f[nt][g][l][t] = W2[32nt + l%32][2(4g+t) + l/32]    B operand of h1 W2^T   for column tile nt, k-step 4g+t
+// w2b[it][g][l][t] = W2[2(4g+t) + l/32][32it + l%32]    B operand of d_pre2 W2 for column tile it
+// (the reduction runs through k in order, as the per-layer kernels' does: a pre-activation at zero falls on the same side in both)
 // w1s[nt][j][l]    = W1[32nt + l%32][2j + l/32]         (0 beyond in)
 // W3 (out x 256) is small enough to sit in LDS for the whole launch (rows padded to 16 with zeros).
 __global__ void mlp3_prepare_kernel(const float* __restrict__ W1, const float* __restrict__ W2, int in, float* __restrict__ prep) {
@@ -103,7 +104,7 @@ __global__ void mlp3_prepare_kernel(const float* __restrict__ W1, const float* _
     float* w2f = prep; float* w2b = w2f + W2F_FLOATS; float* w1s = w2b + W2B_FLOATS;
     if (idx < 65536) {
         const int t = idx & 3, l = (idx >> 2) & 63, g = (idx >> 8) & 31, tile = idx >> 13;
-        const int k = 8 * g + 4 * (l >> 5) + t, c = 32 * tile + (l & 31);
+        const int k = 2 * (4 * g + t) + (l >> 5), c = 32 * tile + (l & 31);
         w2f[idx] = W2[c * HID + k];
         w2b[idx] = W2[k * HID + c];
     }
@@ -115,30 +116,30 @@ __global__ void mlp3_prepare_kernel(const float* __restrict__ W1, const float* _
 }
 
 // 64 x 64 block of  A[64 x 256] (LDS, row stride HS) times a pre-swizzled 256 x 256 weight: wavefront w owns column tiles 2w, 2w+1.
-// The LDS operands of the next group of four k-steps and the weight group two ahead are requested before the matrix instructions of a group are issued.
+// The LDS operands of k-step s+1 and the weight group two ahead are requested before the matrix instructions of step s are issued.
 __device__ __forceinline__ void contract_256(lptr a, const float* __restrict__ wsw, int w, int lane, floatx16 (&acc)[2][2]) {
     const int c32 = lane & 31, hi = lane >> 5;
     const floatx4* b0p = reinterpret_cast<const floatx4*>(wsw) + (size_t)(2 * w) * 32 * 64 + lane;
     const floatx4* b1p = b0p + 32 * 64;
-    const lptr a0 = a + c32 * HS + 4 * hi, a1 = a0 + 32 * HS;
+    const lptr a0 = a + c32 * HS + hi, a1 = a0 + 32 * HS;
     floatx4 b0 = b0p[0], b1 = b1p[0];
     floatx4 n0 = b0p[64], n1 = b1p[64];
-    floatx4 x0 = *(lptr4)a0, x1 = *(lptr4)a1;
+    float x0 = a0[0], x1 = a1[0];
 #pragma unroll       // fully unrolled: the rotation of the prefetch registers becomes renaming instead of copies that wait for the loads
     for (int g = 0; g < 32; g++) {
         const int gp = g + 2 < 32 ? g + 2 : 31;      // two groups ahead; the last iterations re-read the final group
-        const int next = g + 1 < 32 ? g + 1 : 31;
         const floatx4 p0 = b0p[gp * 64], p1 = b1p[gp * 64];
-        const floatx4 y0 = *(lptr4)(a0 + 8 * next), y1 = *(lptr4)(a1 + 8 * next);
         __builtin_amdgcn_sched_barrier(0);      // the requests above are not to be moved down to their first use
 #pragma unroll
         for (int t = 0; t < 4; t++) {
-            acc[0][0] = mfma32(x0[t], b0[t], acc[0][0]);
-            acc[0][1] = mfma32(x0[t], b1[t], acc[0][1]);
-            acc[1][0] = mfma32(x1[t], b0[t], acc[1][0]);
-            acc[1][1] = mfma32(x1[t], b1[t], acc[1][1]);
+            const int next = 4 * g + t + 1 < 128 ? 4 * g + t + 1 : 127;
+            const float y0 = a0[2 * next], y1 = a1[2 * next];
+            acc[0][0] = mfma32(x0, b0[t], acc[0][0]);
+            acc[0][1] = mfma32(x0, b1[t], acc[0][1]);
+            acc[1][0] = mfma32(x1, b0[t], acc[1][0]);
+            acc[1][1] = mfma32(x1, b1[t], acc[1][1]);
+            x0 = y0; x1 = y1;
         }
-        x0 = y0; x1 = y1;
         b0 = n0; b1 = n1; n0 = p0; n1 = p1;
     }
 }
