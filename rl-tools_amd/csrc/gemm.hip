@@ -285,21 +285,24 @@ __global__ __launch_bounds__(256) void wgrad_reduce_kernel(float* __restrict__ d
 // ---- weight gradients of narrow layers over long batches ----------------------------------------------------------------------------
 // dW [M x N] with M <= 192, N <= 16 NT (a GRU's 3H x I and 3H x H at hidden width 64) over tens of thousands of rows: the tiled kernel above
 // cuts such a matrix into 64 x 64 tiles and every operand row is fetched by three workgroups, each with a short reduction of its own. Here a
-// workgroup keeps the WHOLE gradient in accumulators (wavefront w: rows 48 w ... 48 w + 47 of dW as 3 x NT tiles of v_mfma_f32_16x16x4_f32) and
+// workgroup keeps the WHOLE gradient in accumulators (eight wavefronts: rows 48 w ... 48 w + 47 of dW for w = wavefront % 4, half its columns each, as 3 x NT / 2
+// tiles of v_mfma_f32_16x16x4_f32) and
 // walks its share of the batch 16 rows at a time: both operands are read from memory exactly once, staged through LDS (double buffered, the
 // next 16 rows requested before the current ones are multiplied, one barrier per 16 rows). The bias gradient is summed on the side from the
 // registers the d_pre rows pass through. A workgroup writes one block of partial sums in the layout wgrad_reduce_kernel adds up.
+// At 65,536 rows: 192 x 146 49.4 us with eight wavefronts, two to a SIMD (54.5 with four that had all columns); 192 x 64 27.2 us (29.6 on the tiled kernel).
 typedef float wide_floatx4 __attribute__((ext_vector_type(4)));
-constexpr int WIDE_M = 192, WIDE_KT = 16, WIDE_GS = WIDE_M + 16;
+constexpr int WIDE_M = 192, WIDE_KT = 16, WIDE_GS = WIDE_M + 16, WIDE_THREADS = 512;
 struct WideArgs { const float* G; int ldg; const float* X; int ldx; int M, N, K, rows_per_group; float* ws; int want_bias; };
 template <int NT, int PF>
-__global__ __launch_bounds__(THREADS) void wgrad_wide_kernel(WideArgs a) {
+__global__ __launch_bounds__(WIDE_THREADS) void wgrad_wide_kernel(WideArgs a) {
     constexpr int XS = 16 * NT + 16;                        // both strides are 16 mod 32: the four k-rows a wavefront reads fall on two sets of banks
-    constexpr int GQ = WIDE_KT * WIDE_M / 4 / THREADS;      // float4 of d_pre per thread and 16 rows (3)
-    constexpr int XQ = (WIDE_KT * 8 * NT + THREADS - 1) / THREADS;      // float2 of x per thread and 16 rows
+    constexpr int NTH = NT / 2;                             // column tiles of a wavefront
+    constexpr int G4 = WIDE_KT * WIDE_M / 4, X2 = WIDE_KT * 8 * NT;      // float4 of d_pre and float2 of x per 16 rows
+    constexpr int GQ = (G4 + WIDE_THREADS - 1) / WIDE_THREADS, XQ = (X2 + WIDE_THREADS - 1) / WIDE_THREADS;      // ... and per thread
     __shared__ __align__(16) float gs[2][WIDE_KT * WIDE_GS];
     __shared__ __align__(16) float xs[2][WIDE_KT * XS];
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r = lane & 15, kk = lane >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, w = (tid >> 6) & 3, half = tid >> 8, r = lane & 15, kk = lane >> 4;
     const int k_begin = blockIdx.x * a.rows_per_group, k_end = min(a.K, k_begin + a.rows_per_group);
     // 16 rows of both operands as they travel from memory to LDS. A load under load takes longer than the matrix work on 16 rows, so PF such
     // tiles are on their way at any time (with one, the kernel ran at the rate of one tile per memory latency: 2 TB/s over the whole device).
@@ -311,34 +314,34 @@ __global__ __launch_bounds__(THREADS) void wgrad_wide_kernel(WideArgs a) {
         Tile t;
 #pragma unroll
         for (int q = 0; q < GQ; q++) {
-            const int idx = tid + THREADS * q, row = idx / (WIDE_M / 4), col = 4 * (idx % (WIDE_M / 4));
-            t.g[q] = (k0 + row < k_end && col < a.M) ? *reinterpret_cast<const float4*>(a.G + (size_t)(k0 + row) * a.ldg + col) : make_float4(0.f, 0.f, 0.f, 0.f);
+            const int idx = tid + WIDE_THREADS * q, row = idx / (WIDE_M / 4), col = 4 * (idx % (WIDE_M / 4));
+            t.g[q] = (idx < G4 && k0 + row < k_end && col < a.M) ? *reinterpret_cast<const float4*>(a.G + (size_t)(k0 + row) * a.ldg + col) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
 #pragma unroll
         for (int q = 0; q < XQ; q++) {
-            const int idx = tid + THREADS * q, row = idx / (8 * NT), col = 2 * (idx % (8 * NT));
-            t.x[q] = (idx < WIDE_KT * 8 * NT && k0 + row < k_end && col < a.N) ? *reinterpret_cast<const float2*>(a.X + (size_t)(k0 + row) * a.ldx + col) : make_float2(0.f, 0.f);
+            const int idx = tid + WIDE_THREADS * q, row = idx / (8 * NT), col = 2 * (idx % (8 * NT));
+            t.x[q] = (idx < X2 && k0 + row < k_end && col < a.N) ? *reinterpret_cast<const float2*>(a.X + (size_t)(k0 + row) * a.ldx + col) : make_float2(0.f, 0.f);
         }
         return t;
     };
     auto stage = [&](const Tile& t, int buf) {
 #pragma unroll
         for (int q = 0; q < GQ; q++) {
-            const int idx = tid + THREADS * q, row = idx / (WIDE_M / 4), col = 4 * (idx % (WIDE_M / 4));
-            *reinterpret_cast<float4*>(&gs[buf][row * WIDE_GS + col]) = t.g[q];
+            const int idx = tid + WIDE_THREADS * q, row = idx / (WIDE_M / 4), col = 4 * (idx % (WIDE_M / 4));
+            if (idx < G4) *reinterpret_cast<float4*>(&gs[buf][row * WIDE_GS + col]) = t.g[q];
             bsum[q].x += t.g[q].x; bsum[q].y += t.g[q].y; bsum[q].z += t.g[q].z; bsum[q].w += t.g[q].w;
         }
 #pragma unroll
         for (int q = 0; q < XQ; q++) {
-            const int idx = tid + THREADS * q, row = idx / (8 * NT), col = 2 * (idx % (8 * NT));
-            if (idx < WIDE_KT * 8 * NT) *reinterpret_cast<float2*>(&xs[buf][row * XS + col]) = t.x[q];
+            const int idx = tid + WIDE_THREADS * q, row = idx / (8 * NT), col = 2 * (idx % (8 * NT));
+            if (idx < X2) *reinterpret_cast<float2*>(&xs[buf][row * XS + col]) = t.x[q];
         }
     };
-    wide_floatx4 acc[3][NT];
+    wide_floatx4 acc[3][NTH];
 #pragma unroll
     for (int i = 0; i < 3; i++)
 #pragma unroll
-        for (int j = 0; j < NT; j++) acc[i][j] = wide_floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < NTH; j++) acc[i][j] = wide_floatx4{0.f, 0.f, 0.f, 0.f};
     Tile queue[PF];
     {
         const Tile first = request(k_begin);
@@ -352,18 +355,18 @@ __global__ __launch_bounds__(THREADS) void wgrad_wide_kernel(WideArgs a) {
         const Tile far = request(k0 + (PF + 1) * WIDE_KT);
         __builtin_amdgcn_sched_barrier(0);      // the requests go out first, and nothing that waits for them moves above the matrix work
         const float* g = gs[buf] + kk * WIDE_GS + 48 * w + r;
-        const float* x = xs[buf] + kk * XS + r;
+        const float* x = xs[buf] + kk * XS + 16 * NTH * half + r;
 #pragma unroll
         for (int s4 = 0; s4 < WIDE_KT / 4; s4++) {
-            float av[3], bv[NT];
+            float av[3], bv[NTH];
 #pragma unroll
             for (int i = 0; i < 3; i++) av[i] = g[4 * s4 * WIDE_GS + 16 * i];
 #pragma unroll
-            for (int j = 0; j < NT; j++) bv[j] = x[4 * s4 * XS + 16 * j];
+            for (int j = 0; j < NTH; j++) bv[j] = x[4 * s4 * XS + 16 * j];
 #pragma unroll
             for (int i = 0; i < 3; i++)
 #pragma unroll
-                for (int j = 0; j < NT; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], bv[j], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < NTH; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], bv[j], acc[i][j], 0, 0, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
         if (k0 + WIDE_KT < k_end) stage(queue[0], buf ^ 1);
@@ -373,7 +376,7 @@ __global__ __launch_bounds__(THREADS) void wgrad_wide_kernel(WideArgs a) {
         for (int d = 0; d + 1 < PF; d++) queue[d] = queue[d + 1];
         queue[PF - 1] = far;
     }
-    // element v of lane (r, kk) of tile (i, j): dW[48 w + 16 i + 4 kk + v][16 j + r]
+    // element v of lane (r, kk) of tile (i, j): dW[48 w + 16 i + 4 kk + v][16 (NTH half + j) + r]
     float* out = a.ws + (size_t)blockIdx.x * ((size_t)a.M * a.N + a.M);
 #pragma unroll
     for (int i = 0; i < 3; i++)
@@ -381,8 +384,8 @@ __global__ __launch_bounds__(THREADS) void wgrad_wide_kernel(WideArgs a) {
         for (int v = 0; v < 4; v++) {
             const int m = 48 * w + 16 * i + 4 * kk + v;
 #pragma unroll
-            for (int j = 0; j < NT; j++) {
-                const int n = 16 * j + r;
+            for (int j = 0; j < NTH; j++) {
+                const int n = 16 * (NTH * half + j) + r;
                 if (m < a.M && n < a.N) out[(size_t)m * a.N + n] = acc[i][j][v];
             }
         }
@@ -390,8 +393,8 @@ __global__ __launch_bounds__(THREADS) void wgrad_wide_kernel(WideArgs a) {
         float* bs = gs[0];
 #pragma unroll
         for (int q = 0; q < GQ; q++) {
-            const int idx = tid + THREADS * q, row = idx / (WIDE_M / 4), col = 4 * (idx % (WIDE_M / 4));
-            *reinterpret_cast<float4*>(&bs[row * WIDE_GS + col]) = bsum[q];
+            const int idx = tid + WIDE_THREADS * q, row = idx / (WIDE_M / 4), col = 4 * (idx % (WIDE_M / 4));
+            if (idx < G4) *reinterpret_cast<float4*>(&bs[row * WIDE_GS + col]) = bsum[q];
         }
         __syncthreads();
         if (tid < a.M) {
@@ -400,6 +403,111 @@ __global__ __launch_bounds__(THREADS) void wgrad_wide_kernel(WideArgs a) {
             for (int row = 0; row < WIDE_KT; row++) sum += bs[row * WIDE_GS + tid];
             out[(size_t)a.M * a.N + tid] = sum;
         }
+    }
+}
+
+// ---- forward contraction of a narrow layer over long batches ---------------------------------------------------------------------------
+// y [M x N] = x [M x K] W^T + b with N <= 192, K <= 16 NJ (a GRU's input gates) over thousands of rows. On the tiled kernel every workgroup fetches its share of W again, stages it through
+// LDS and waits for a barrier per 16 of K: 60 us and 61 TFLOP/s at 65,536 x 146 -> 192. Here a wavefront keeps the weights of its 48 columns in registers for the whole launch
+// (w = wavefront % 4, 3 tiles of v_mfma_f32_16x16x4_f32 by 4 NJ k-steps, 12 NJ registers), and only rows pass through LDS: 32 at a time (wavefront / 4 selects sixteen of them),
+// double buffered, the next 32 requested before the current ones are multiplied, one barrier each. Lane (r, kk) supplies the four k from 16 j + 4 kk of every sixteen, for both operands.
+// Measured, K = 146, N = 192 (tiled kernel -> this one): 1,024 rows 9.0 -> 10.3 us, 2,048 12.1 -> 10.5, 4,096 13.1 -> 11.2, 8,192 16.0 -> 12.5, 16,384 28.6 -> 17.8, 65,536 60 -> 46 us; K = 64:
+// 1,024 rows 5.1 -> 5.9 us, 2,048 7.9 -> 6.1, 65,536 35.4 -> 25.4 us: the line lies at 2,048 rows. Bound: the matrix pipe at long batches (27 us of 46, K padded to 160), the trip to memory
+// for the weights at short ones.
+struct RowsForward { const float* X; int ldx; const float* W; const float* bias; float* Y; int ldy; int M, N, K; };
+constexpr int RF_THREADS = 512, RF_ROWS = 32, ROWS_FORWARD_MIN_BATCH = 2048;
+template <int NJ>
+__global__ __launch_bounds__(RF_THREADS) void rows_forward_kernel(RowsForward a) {
+    constexpr int KP = 16 * NJ, XS = KP + 4, X2 = RF_ROWS * KP / 2, XQ = X2 / RF_THREADS;      // 16 bytes of each of sixteen rows fall on different banks
+    static_assert(X2 % RF_THREADS == 0, "every thread stages the same number of pairs");
+    __shared__ __align__(16) float xs[2][RF_ROWS * XS];
+    const int tid = threadIdx.x, lane = tid & 63, w = (tid >> 6) & 3, tile = tid >> 8, r = lane & 15, kk = lane >> 4;
+    auto request = [&](int row0, float2 (&v)[XQ]) {
+#pragma unroll
+        for (int q = 0; q < XQ; q++) {
+            const int idx = tid + RF_THREADS * q, row = row0 + idx / (KP / 2), col = 2 * (idx % (KP / 2));
+            v[q] = *reinterpret_cast<const float2*>(a.X + (size_t)min(row, a.M - 1) * a.ldx + min(col, a.K - 2));      // K is even; clamped instead of branched around
+        }
+    };
+    auto stage = [&](const float2 (&v)[XQ], int buf) {
+#pragma unroll
+        for (int q = 0; q < XQ; q++) {
+            const int idx = tid + RF_THREADS * q;
+            const int col = 2 * (idx % (KP / 2));
+            *reinterpret_cast<float2*>(&xs[buf][(idx / (KP / 2)) * XS + col]) = col < a.K ? v[q] : make_float2(0.f, 0.f);
+        }
+    };
+    const int blocks = (a.M + RF_ROWS - 1) / RF_ROWS;
+    float2 next[XQ];
+    request(blockIdx.x * RF_ROWS, next);
+    // W goes through the same LDS buffer, 64 rows at a time: read from memory row by row (a lane's own operands, rows apart, took as long as three blocks of rows)
+    float2 wv[3][NJ];
+#pragma unroll
+    for (int p = 0; p < 3; p++)
+#pragma unroll
+        for (int q = 0; q < NJ; q++) {
+            const int idx = tid + RF_THREADS * q, n = 64 * p + idx / (KP / 2), col = 2 * (idx % (KP / 2));
+            wv[p][q] = *reinterpret_cast<const float2*>(a.W + (size_t)min(n, a.N - 1) * a.K + min(col, a.K - 2));      // rows beyond the width repeat the last one and are not stored
+        }
+    float b[3][NJ][4], bias[3];
+#pragma unroll
+    for (int t = 0; t < 3; t++) bias[t] = a.bias[min(48 * w + 16 * t + r, a.N - 1)];
+#pragma unroll
+    for (int p = 0; p < 3; p++) {
+        if (p > 0) rlt_lds_barrier();      // the rows before have been read
+#pragma unroll
+        for (int q = 0; q < NJ; q++) {
+            const int idx = tid + RF_THREADS * q, col = 2 * (idx % (KP / 2));
+            *reinterpret_cast<float2*>(&xs[0][(idx / (KP / 2)) * XS + col]) = col < a.K ? wv[p][q] : make_float2(0.f, 0.f);
+        }
+        rlt_lds_barrier();
+#pragma unroll
+        for (int t = 0; t < 3; t++)
+            if ((48 * w + 16 * t) >> 6 == p) {      // sixteen columns lie in one of the three parts
+#pragma unroll
+                for (int j = 0; j < NJ; j++) {
+                    const wide_floatx4 v = *reinterpret_cast<const wide_floatx4*>(&xs[0][((48 * w + 16 * t + r) & 63) * XS + 16 * j + 4 * kk]);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) b[t][j][e] = v[e];
+                }
+            }
+    }
+    rlt_lds_barrier();
+    stage(next, 0);
+    rlt_lds_barrier();
+    int buf = 0;
+    for (int block = blockIdx.x; block < blocks; block += gridDim.x) {
+        request((block + (int)gridDim.x) * RF_ROWS, next);      // beyond the last row: the last one again
+        __builtin_amdgcn_sched_barrier(0);
+        const float* x = xs[buf] + (16 * tile + r) * XS + 4 * kk;
+        wide_floatx4 acc[3];
+#pragma unroll
+        for (int t = 0; t < 3; t++) acc[t] = wide_floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            const wide_floatx4 av = *reinterpret_cast<const wide_floatx4*>(x + 16 * j);
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int t = 0; t < 3; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[e], b[t][j][e], acc[t], 0, 0, 0);
+        }
+        // element v of lane (r, kk): row 4 kk + v, column r of the tile
+        const int row0 = block * RF_ROWS + 16 * tile + 4 * kk;
+        float* y = a.Y + (size_t)row0 * a.ldy + 48 * w + r;
+        if ((block + 1) * RF_ROWS <= a.M && 48 * (w + 1) <= a.N) {
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+#pragma unroll
+                for (int t = 0; t < 3; t++) y[(size_t)v * a.ldy + 16 * t] = acc[t][v] + bias[t];
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+#pragma unroll
+                for (int t = 0; t < 3; t++) if (row0 + v < a.M && 48 * w + 16 * t + r < a.N) y[(size_t)v * a.ldy + 16 * t] = acc[t][v] + bias[t];
+        }
+        stage(next, buf ^ 1);
+        rlt_lds_barrier();
+        buf ^= 1;
     }
 }
 
@@ -600,6 +708,16 @@ int rlt_gemm_forward(rlt_rocm_device* device, const float* x, int ldx, const flo
     return launch<0>(device, p, 1);
 }
 
+int rlt_gemm_rows_forward(rlt_rocm_device* device, const float* x, int ldx, const float* W, const float* bias, float* y, int ldy, int batch, int in_dim, int out_dim) {
+    if (out_dim <= 96 || out_dim > WIDE_M || in_dim <= 32 || in_dim > 160 || in_dim % 2 != 0 || ldx % 2 != 0 || batch < ROWS_FORWARD_MIN_BATCH ||
+        ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(W)) & 7u) != 0) return RLT_E_UNSUPPORTED;
+    const RowsForward a = {x, ldx, W, bias, y, ldy, batch, out_dim, in_dim};
+    const int blocks = rlt_div_up(batch, RF_ROWS), grid = blocks < device->compute_units ? blocks : device->compute_units;
+    if (in_dim <= 64) hipLaunchKernelGGL(rows_forward_kernel<4>, dim3(grid), dim3(RF_THREADS), 0, device->stream, a);
+    else hipLaunchKernelGGL(rows_forward_kernel<10>, dim3(grid), dim3(RF_THREADS), 0, device->stream, a);
+    return rlt_launch_status(device);
+}
+
 int rlt_gemm_backward_input(rlt_rocm_device* device, const float* d_pre, int ldd, const float* W, float* d_in, int ldi,
                             const float* dact_pre, int dact_kind, int dact_from_output, int batch, int in_dim, int out_dim) {
     if (rlt_div_up(batch, 32) > 65535) return RLT_E_UNSUPPORTED;
@@ -660,15 +778,16 @@ int rlt_gemm_wgrad(rlt_rocm_device* device, const float* d_pre, int ldd, const f
     p.vecA = vector_width(d_pre, ldd); p.vecB = vector_width(x, ldx);
     p.dW = dW; p.dbias = dbias;
     // narrow layer, long batch: one workgroup per share of the batch holds the whole gradient (wgrad_wide_kernel)
-    if (narrow_long && !static_scratch && out_dim <= WIDE_M && out_dim % 4 == 0 && in_dim > 64 && in_dim <= 160 && in_dim % 2 == 0 && batch >= 16384 && ldd % 4 == 0 && ldx % 2 == 0 &&
+    if (narrow_long && !static_scratch && out_dim <= WIDE_M && out_dim % 4 == 0 && in_dim > 32 && in_dim <= 160 && in_dim % 2 == 0 && batch >= 16384 && ldd % 4 == 0 && ldx % 2 == 0 &&
         (reinterpret_cast<uintptr_t>(d_pre) & 15u) == 0 && (reinterpret_cast<uintptr_t>(x) & 7u) == 0) {
         const int groups = device->compute_units < batch / 64 ? device->compute_units : batch / 64;
         const int rows_per_group = rlt_div_up(rlt_div_up(batch, groups), WIDE_KT) * WIDE_KT, used = rlt_div_up(batch, rows_per_group);
         void* ws = nullptr;
         int rc = rlt_scratch(device, (size_t)used * ((size_t)out_dim * in_dim + out_dim) * sizeof(float), &ws);
         if (rc) return rc;
-        WideArgs a = {d_pre, ldd, x, ldx, out_dim, in_dim, batch, rows_per_group, (float*)ws, 1};
-        hipLaunchKernelGGL((wgrad_wide_kernel<10, 2>), dim3(used), dim3(THREADS), 0, device->stream, a);
+        WideArgs a = {d_pre, ldd, x, ldx, out_dim, in_dim, batch, rows_per_group, (float*)ws, dbias ? 1 : 0};
+        if (in_dim <= 64) hipLaunchKernelGGL((wgrad_wide_kernel<4, 4>), dim3(used), dim3(WIDE_THREADS), 0, device->stream, a);
+        else hipLaunchKernelGGL((wgrad_wide_kernel<10, 2>), dim3(used), dim3(WIDE_THREADS), 0, device->stream, a);
         if ((rc = rlt_launch_status(device))) return rc;
         const int mn = out_dim * in_dim;
         hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(rlt_div_up(mn + out_dim, 64)), dim3(256), 0, device->stream, dW, dbias, (const float*)ws, mn, out_dim, used);

@@ -516,7 +516,9 @@ int rlt_rocm_gru_forward(rlt_rocm_device* device, const rlt_gru_layer* L, const 
     const int H = L->hidden_dim;
     if (lds_bytes(H, false) > (size_t)device->lds_bytes) return RLT_E_UNSUPPORTED;
     // W_i x + b_i for every step at once, into post_activation
-    int rc = rlt_gemm_forward(device, input, L->input_dim, L->weights_input, L->biases_input, RLT_ACT_IDENTITY, nullptr, nullptr, L->post_activation, 3 * H, S * B, L->input_dim, 3 * H);
+    int rc = rlt_gemm_rows_forward(device, input, L->input_dim, L->weights_input, L->biases_input, L->post_activation, 3 * H, S * B, L->input_dim, 3 * H);
+    if (rc == RLT_E_UNSUPPORTED)
+        rc = rlt_gemm_forward(device, input, L->input_dim, L->weights_input, L->biases_input, RLT_ACT_IDENTITY, nullptr, nullptr, L->post_activation, 3 * H, S * B, L->input_dim, 3 * H);
     if (rc) return rc;
     GruArgs a = {}; a.L = *L; a.input = input; a.reset = reset; a.S = S; a.B = B; a.rows_per_group = rows_per_group(H);
     if (H == 64 || H == 32 || H == 16) {
