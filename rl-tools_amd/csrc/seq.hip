@@ -102,7 +102,7 @@ extern "C" {
 size_t rlt_rocm_seq_workspace_bytes(const rlt_seq_layer* layers, int n, int steps, int batch) {
     if (!layers || n <= 0 || steps <= 0 || batch <= 0) return 0;
     const size_t by_layer = 2 * align256((size_t)steps * batch * max_width(layers, n) * sizeof(float)) + gru_bytes(layers, n, steps, batch) + 256;
-    return rlt_seq_stack_supported(layers, n, 1) ? std::max(by_layer, rlt_seq_stack_workspace_bytes(layers, steps, batch) + 256) : by_layer;
+    return rlt_seq_stack_shape(layers, n) ? std::max(by_layer, rlt_seq_stack_workspace_bytes(layers, steps, batch) + 256) : by_layer;
 }
 
 int rlt_rocm_seq_forward(rlt_rocm_device* device, const rlt_seq_layer* layers, int n, const float* x, int ldx, const uint8_t* reset, int steps, int batch,

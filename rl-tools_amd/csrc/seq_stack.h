@@ -2,6 +2,9 @@
 #pragma once
 #include "common.h"
 
+// true if the model's shape is the one that these passes take, whatever its buffers: a program may size a workspace before it has them
+bool rlt_seq_stack_shape(const rlt_seq_layer* layers, int n);
+
 // true if the model is dense (any activation but the output's, which is the identity) -> GRU -> GRU -> dense with one hidden width of 16 or 32 throughout, at most 16
 // inputs and outputs, and a sequence short enough that a batch row's inputs fit the LDS
 bool rlt_seq_stack_supported(const rlt_seq_layer* layers, int n, int steps);

@@ -482,14 +482,21 @@ size_t forward_lds(int H, int in, int S) { return (H == 32 ? sizeof(ForwardSlots
 size_t backward_lds(int H, int out, int S) { return (H == 32 ? sizeof(BackwardSlots<32>) : sizeof(BackwardSlots<16>)) + 16 + (size_t)S * ((out + 3) & ~3) * sizeof(float) + S; }
 }  // namespace
 
-bool rlt_seq_stack_supported(const rlt_seq_layer* L, int n, int steps) {
-    if (!L || n != 4 || steps < 1 || L[0].kind != 0 || L[1].kind != 1 || L[2].kind != 1 || L[3].kind != 0) return false;
+bool rlt_seq_stack_shape(const rlt_seq_layer* L, int n) {
+    if (!L || n != 4 || L[0].kind != 0 || L[1].kind != 1 || L[2].kind != 1 || L[3].kind != 0) return false;
     const int H = L[0].dense.out_dim, in = L[0].dense.in_dim, out = L[3].dense.out_dim;
-    if ((H != 16 && H != 32) || in < 1 || in > MAX_IN || out < 1 || out > MAX_OUT || L[3].dense.in_dim != H || L[3].dense.activation != RLT_ACT_IDENTITY) return false;
+    if ((H != 16 && H != 32) || in < 1 || in > MAX_IN || out < 1 || out > MAX_OUT || L[3].dense.in_dim != H) return false;
+    for (int l = 1; l < 3; l++) if (L[l].gru.input_dim != H || L[l].gru.hidden_dim != H) return false;
+    return true;
+}
+
+bool rlt_seq_stack_supported(const rlt_seq_layer* L, int n, int steps) {
+    if (!rlt_seq_stack_shape(L, n) || steps < 1 || L[3].dense.activation != RLT_ACT_IDENTITY) return false;
+    const int H = L[0].dense.out_dim, in = L[0].dense.in_dim, out = L[3].dense.out_dim;
     if (L[0].dense.activation < 0 || L[0].dense.activation > RLT_ACT_SIGMOID) return false;
     for (int l = 1; l < 3; l++) {
         const rlt_gru_layer& G = L[l].gru;
-        if (G.input_dim != H || G.hidden_dim != H || (G.fast_tanh != 0) != (L[1].gru.fast_tanh != 0)) return false;
+        if ((G.fast_tanh != 0) != (L[1].gru.fast_tanh != 0)) return false;
         if (!G.weights_input || !G.biases_input || !G.weights_hidden || !G.biases_hidden || !G.initial_hidden_state || !G.post_activation || !G.n_pre_pre_activation || !G.output) return false;
     }
     for (int l = 0; l < 4; l += 3) { const rlt_dense_layer& D = L[l].dense; if (!D.weights || !D.biases || !D.pre_activations || !D.output) return false; }
