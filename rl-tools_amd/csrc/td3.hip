@@ -152,13 +152,20 @@ bool agent_ok(const rlt_td3_agent* A) {
 
 // the soft update of a network's tensors, 32 to a launch (a launch per tensor: 27 us for the Ant actor's six, together 4.4)
 int polyak_mlp(rlt_rocm_device* device, const rlt_dense_layer* source, const rlt_dense_layer* target, int n, float polyak) {
-    RLT_REQUIRE(n <= 32);
-    const float* sources[64]; float* targets[64]; uint32_t counts[64];
-    for (int l = 0; l < n; l++) {
-        sources[2 * l] = source[l].weights; targets[2 * l] = target[l].weights; counts[2 * l] = (uint32_t)source[l].in_dim * source[l].out_dim;
-        sources[2 * l + 1] = source[l].biases; targets[2 * l + 1] = target[l].biases; counts[2 * l + 1] = (uint32_t)source[l].out_dim;
+    constexpr int LAYERS = 16;
+    for (int l = 0; l < n; l++) RLT_REQUIRE(source[l].weights && target[l].weights && source[l].biases && target[l].biases);
+    for (int base = 0; base < n; base += LAYERS) {
+        const int m = n - base < LAYERS ? n - base : LAYERS;
+        const float* sources[2 * LAYERS]; float* targets[2 * LAYERS]; uint32_t counts[2 * LAYERS];
+        for (int l = 0; l < m; l++) {
+            const rlt_dense_layer &S = source[base + l], &T = target[base + l];
+            sources[2 * l] = S.weights; targets[2 * l] = T.weights; counts[2 * l] = (uint32_t)S.in_dim * S.out_dim;
+            sources[2 * l + 1] = S.biases; targets[2 * l + 1] = T.biases; counts[2 * l + 1] = (uint32_t)S.out_dim;
+        }
+        const int rc = rlt_sac_polyak_list(device, sources, targets, counts, 2 * m, polyak);
+        if (rc) return rc;
     }
-    return rlt_sac_polyak_list(device, sources, targets, counts, 2 * n, polyak);
+    return 0;
 }
 
 }  // namespace

@@ -207,6 +207,21 @@ def fused_against_checker_and_per_operation(oracle, rocm, batch, obs, act, hidde
     assert np.abs(out["fused"]["params"] - params).max() > 1e-4
 
 
+def test_target_updates_refuse_a_missing_tensor(rocm):
+    obs, act, hidden = 3, 1, 64
+    nets = [helpers.random_params(np.random.default_rng(0), dims) for dims in [[obs, hidden, hidden, act]] * 2 + [[obs + act, hidden, hidden, 1]] * 4]
+    ag = helpers.Td3OnBackend(rocm, 16, hidden, np.concatenate(nets), masks=False, obs=obs, act=act)
+    lib, h = rocm.device.lib, rocm.device.handle
+    for update, target in ((lib.rlt_rocm_td3_update_actor_target, ag.c.actor_target), (lib.rlt_rocm_td3_update_critic_targets, ag.c.critics_target[1])):
+        for name in ("weights", "biases"):
+            keep = getattr(target[1], name)
+            setattr(target[1], name, None)
+            assert update(h, C.byref(ag.c)) == helpers.capi.RLT_E_INVALID_ARGUMENT
+            setattr(target[1], name, keep)
+        assert update(h, C.byref(ag.c)) == 0
+    rocm.sync()
+
+
 @pytest.mark.parametrize("batch,obs,act,hidden,hidden_act", [(256, 27, 8, 256, "relu"), (100, 6, 1, 256, "relu"), (48, 3, 1, 200, "tanh"), (256, 3, 1, 64, "relu")])
 def test_both_critics_in_one_call_leave_the_bits_of_the_two_calls(rocm, batch, obs, act, hidden, hidden_act):
     """rlt_rocm_td3_train_critics against rlt_rocm_td3_train_critic for critic 0 and then critic 1 on the same batch and target noise, each critic with its own sampling
