@@ -27,8 +27,8 @@ __device__ __forceinline__ void tile_product(const float* a, int lda, int m_coun
 #pragma unroll
             for (int q = 0; q < MT; q++) { va[q][s] = pa[q][(size_t)kc * lda]; if (k >= k1 || !m_ok[q]) va[q][s] = 0.f; }
             v0[s] = pb0[(size_t)kc * ldb]; v1[s] = pb1[(size_t)kc * ldb];
-            if (!a_ok) v0[s] = 0.f;
-            if (!b_ok) v1[s] = 0.f;
+            if (k >= k1 || !a_ok) v0[s] = 0.f;      // both operands: zero times another share's infinity is not zero
+            if (k >= k1 || !b_ok) v1[s] = 0.f;
         }
     };
     if (k0 < k1) request(k0);

@@ -128,3 +128,27 @@ def test_backward_alone_on_sixteen_row_tiles_matches_the_checker_and_the_other_p
             assert ew <= TOL and eb <= TOL, (name, off, ew, eb)
     assert not np.array_equal(got["grads"], other["grads"])      # two different kernels ran
 
+
+
+@pytest.mark.parametrize("B,row", [(300, 80), (300, 299), (1100, 150)])
+def test_an_infinite_input_stays_in_its_column_and_infinite(rocm, B, row):
+    """The wavefronts' shares of the batch do not end where their chunks of 32 rows do: a row behind a share's end is another share's, and its infinity meets no zero there.
+    d_pre1 of a tanh network is not zero, so that column of the first layer's gradient is infinite and everything else finite."""
+    dims = [17, 72, 72, 6]
+    rng = np.random.default_rng(B + row)
+    params = helpers.random_params(rng, dims)
+    x, dy = rng.standard_normal((B, 17)).astype(np.float32), rng.standard_normal((B, 6)).astype(np.float32)
+    net = Mlp(rocm, dims, params, B, "tanh", "identity")
+    xd, dyd = rocm.array(x), rocm.array(dy)
+    x[row, 3] = np.inf
+    xi = rocm.array(x)
+    ws, wsn = net.workspace()
+    rocm.call("mlp_zero_gradient", net.layers, net.n)
+    rocm.call("mlp_forward", net.layers, net.n, xd.ptr, 17, B)
+    rocm.call("mlp_backward", net.layers, net.n, xi.ptr, 17, dyd.ptr, 6, None, 0, B, 1, ws, wsn)
+    rocm.sync()
+    grads = net.grads.numpy()
+    off, nw, _ = net.offsets[0]
+    infinite = np.zeros(grads.shape, bool)
+    infinite[off:off + nw].reshape(72, 17)[:, 3] = True
+    assert np.isinf(grads[infinite]).all() and np.isfinite(grads[~infinite]).all()
