@@ -10,8 +10,9 @@
 // Bound: the instructions of a recurrence's step. A wavefront is alone on its SIMD and issues one instruction every four to five cycles whatever it is (vector, scalar,
 // wait), so a step takes its instruction count: about 115 at width 32, 48 of them the products. Hence the forms below: values exchanged between lanes instead of through
 // LDS, the r gate in one half of the lanes while z is in the other, stores and LDS writes by all lanes of a unit rather than under an exec mask, addresses moved on
-// instead of formed, loops unrolled to the slots' parity. TODO us per step at width 32 (TODO backward); a launch per layer with a row per 32 lanes took 0.58 us per step,
-// one layer after the other, plus launches for the dense layers, projections and gradients.
+// instead of formed, loops unrolled to the slots' parity. Per step of a whole pass, 100 sequences of 100 steps: 0.43 us at width 32 (0.41 backward, 0.48 with the values
+// that the weight gradients need stored), 0.30 and 0.38 at width 16; a launch per layer with a row per 32 lanes took 0.59 us per step at width 32 and 0.45 at 16, one
+// layer after the other, plus launches for the dense layers, projections and gradients.
 #include "seq_stack.h"
 #include "gemm.h"
 #include "batch_tile.h"
