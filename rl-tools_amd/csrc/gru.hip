@@ -111,13 +111,14 @@ __global__ __launch_bounds__(GRU_THREADS) void gru_backward_kernel(GruArgs A) {
     if (active && A.db_hn_partial) A.db_hn_partial[(size_t)b * H + j] = db_hn;
 }
 
-// ---- hidden widths 64, 32 and 16: W_h in registers, no LDS, no barrier -------------------------------------------------------
+// ---- hidden widths 32 and 16: W_h in registers, no workgroup barrier -----------------------------------------------------------
 // A wavefront carries 64 / H batch rows; lane (row, j) owns hidden unit j of its row and keeps rows j, H + j, 2H + j of W_h (3H values) in
-// registers for the whole sequence. The previous hidden state reaches the lanes of its row through H lane reads per step at H = 64, where the
-// wavefront is one row, and through a 64-float slot of LDS private to the wavefront below that (one write, H / 4 broadcast reads of four
-// values); a step needs no workgroup barrier, and the wavefronts of a workgroup are independent (they only share the launch). The step's inputs W_i x + b_i
-// are requested one step ahead.
-__device__ __forceinline__ float lane_read(float x, int k) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), k)); }
+// registers for the whole sequence. The previous hidden state reaches the lanes of its row through a 64-float slot of LDS private to the wavefront
+// (one write, H / 4 broadcast reads of four values); a step needs no workgroup barrier, and the wavefronts of a workgroup are independent (they only
+// share the launch). Rows beyond the batch repeat the last row, which the same wavefront holds: they read, compute and store the same values.
+// Bound: the chain of a step. What it reads is requested four steps ahead into registers that the unrolled loop names (as a queue whose entries move up it waited for
+// each step's own request), a wavefront reads 64 reset flags at a time. Whole model step of 64 x 16 sequences, width 16: 111 -> 99 us, 63 x 1,000: 200 -> 188 us; width 32,
+// where the 96 multiply-adds of a step hide the requests: 131.2 -> 129.7 us (64 x 64), 257 -> 254 us (64 x 1,024).
 // lanes of one wavefront exchange data through LDS: the hardware executes a wavefront's LDS instructions in order, the fences keep the
 // compiler from moving them across
 __device__ __forceinline__ void wave_sync() {
@@ -126,13 +127,43 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// The steps of a sequence in groups of D whose members know their number in the group (a queue's entries are indexed by it). Whole groups are straight-line code: with an
+// exit before every step the compiler waits for all requests where the paths meet. For the same reason everything requested before the loop is waited for in front of it: the
+// first step of a group then waits for its own values, requested D steps before, and not for the last ones.
+template <class F, int... K> __device__ __forceinline__ void gru_whole_group(int first, F& step, std::integer_sequence<int, K...>) { (step(std::integral_constant<int, K>{}, first + K), ...); }
+template <class F, int... K> __device__ __forceinline__ void gru_rest(int first, int S, F& step, std::integer_sequence<int, K...>) { ((first + K < S ? step(std::integral_constant<int, K>{}, first + K) : (void)0), ...); }
+template <int D, class F>
+__device__ __forceinline__ void gru_steps(int S, F&& step) {
+    int i = 0;
+    __builtin_amdgcn_s_waitcnt(0x0F70);      // vmcnt(0)
+    for (; i + D <= S; i += D) gru_whole_group(i, step, std::make_integer_sequence<int, D>{});
+    gru_rest(i, S, step, std::make_integer_sequence<int, D - 1>{});
+}
+
+// Reset flags of 64 consecutive steps from `first` on, as a mask in every lane of the row's group (bit i: step first + i starts an episode); steps from S on: no. A wavefront
+// reads a step per lane: a byte load per step would hold the recurrence up for its widening.
+template <int ROWS>
+__device__ __forceinline__ uint64_t gru_reset_flags(const uint8_t* reset, int first, int S, int B, int b0, int mine) {
+    if (!reset) return 0;
+    const int t = first + (int)(threadIdx.x & 63);
+    uint64_t mask = 0;
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) {
+        const uint64_t row = __ballot(t < S && reset[(size_t)min(t, S - 1) * B + min(b0 + r, B - 1)] != 0);
+        mask = mine == r ? row : mask;
+    }
+    return mask;
+}
+__device__ __forceinline__ float& gru_at(float* base, unsigned bytes) { return *reinterpret_cast<float*>(reinterpret_cast<char*>(base) + bytes); }
+
 template <int H, bool FAST>
 __global__ __launch_bounds__(GRU_THREADS) void gru_forward_reg_kernel(GruArgs A) {
-    constexpr int G = 64 / H;                               // batch rows per wavefront
-    __shared__ __align__(16) float exchange[GRU_THREADS / 64][1][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, u = lane & (H - 1), row_base = lane & ~(H - 1);
-    const int b = (blockIdx.x * (GRU_THREADS / 64) + wave) * G + lane / H;
-    if (b >= A.B) return;                                   // the lanes of whole rows leave; lane reads stay within a row; no barrier follows
+    constexpr int G = 64 / H, D = 4;                        // batch rows per wavefront; steps ahead that the inputs W_i x + b_i are requested
+    __shared__ __align__(16) float exchange[GRU_THREADS / 64][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), u = lane & (H - 1), row_base = lane & ~(H - 1);
+    const int b0 = (blockIdx.x * (GRU_THREADS / 64) + wave) * G;
+    if (b0 >= A.B) return;                                  // whole wavefronts; no barrier follows
+    const int row = min(lane / H, A.B - 1 - b0);
     float wr[H], wz[H], wn[H];
     {
         const float4* r4 = reinterpret_cast<const float4*>(A.L.weights_hidden + (size_t)u * H);
@@ -148,34 +179,26 @@ __global__ __launch_bounds__(GRU_THREADS) void gru_forward_reg_kernel(GruArgs A)
     }
     const float bhr = A.L.biases_hidden[u], bhz = A.L.biases_hidden[H + u], bhn = A.L.biases_hidden[2 * H + u];
     const float h0 = A.L.initial_hidden_state[u];
+    const size_t stride = (size_t)A.B * H;
+    const unsigned at = (row * H + u) * sizeof(float), at3 = (row * 3 * H + u) * sizeof(float);
+    float* post = A.L.post_activation + (size_t)b0 * 3 * H; float* npp = A.L.n_pre_pre_activation + (size_t)b0 * H; float* out = A.L.output + (size_t)b0 * H;
+    struct In { float r, z, n; };
+    float* in = post;
+    auto request = [&](int t, In& v) {      // in the order of the steps; the last steps request the last one again: no branch around the loads
+        v.r = gru_at(in, at3); v.z = gru_at(in + H, at3); v.n = gru_at(in + 2 * H, at3);
+        in += t + 1 < A.S ? 3 * stride : 0;
+    };
+    In q[D];
+#pragma unroll
+    for (int d = 0; d < D; d++) request(d, q[d]);
+    float* const xw = exchange[wave];
     float h = h0;
-    const size_t stride = (size_t)A.B * 3 * H;
-    float* post = A.L.post_activation + (size_t)b * 3 * H;
-    float xr = post[u], xz = post[H + u], xn = post[2 * H + u];
-    int rs = A.reset ? A.reset[b] : 0;
-    // The inputs of later steps are requested D steps ahead and wait in a queue of D - 1 entries. Consecutive steps lie 12 H B bytes apart, on
-    // other pages; two steps of distance pay at widths 16 and 32 (85 -> 59 us for 101 steps at 32), at 64 one step measures faster (60 against 67 us).
-    constexpr int D = H == 64 ? 1 : 2, Q = D > 1 ? D - 1 : 1;
-    float qr[Q], qz[Q], qn[Q]; int qs[Q];
-#pragma unroll
-    for (int d = 0; d < D - 1; d++) {
-        const int tq = d + 1 < A.S ? d + 1 : A.S - 1;
-        const float* pq = A.L.post_activation + (size_t)tq * stride + (size_t)b * 3 * H;
-        qr[d] = pq[u]; qz[d] = pq[H + u]; qn[d] = pq[2 * H + u]; qs[d] = A.reset ? A.reset[(size_t)tq * A.B + b] : 0;
-    }
-    for (int t = 0; t < A.S; t++) {
-        // (the last steps request the last one again: no branch around the loads)
-        const int tn = t + D < A.S ? t + D : A.S - 1;
-        const float* pn = A.L.post_activation + (size_t)tn * stride + (size_t)b * 3 * H;
-        const float fr = pn[u], fz = pn[H + u], fn = pn[2 * H + u];
-        const int fs = A.reset ? A.reset[(size_t)tn * A.B + b] : 0;
-        if (t == 0 || rs) h = h0;
-        float ar = bhr, az = bhz, an = bhn;
-        if (H == 64) {       // measured: 64 scalar lane reads beat the LDS slot here (60 against 67 us for 64 steps), in the reverse pass they lose (103 against 64 us)
-#pragma unroll
-            for (int k = 0; k < H; k++) { const float hk = lane_read(h, k); ar += hk * wr[k]; az += hk * wz[k]; an += hk * wn[k]; }
-        } else {
-            float* xw = &exchange[wave][0][0];
+    for (int first = 0; first < A.S; first += 64) {
+        uint64_t flags = gru_reset_flags<G>(A.reset, first + 1, A.S, A.B, b0, lane / H);      // of the steps after these
+        gru_steps<D>(min(64, A.S - first), [&](auto number, int i) {
+            constexpr int N = decltype(number)::value;
+            __builtin_amdgcn_sched_barrier(0);      // later steps' values are not touched (and waited for) before their step
+            float ar = bhr, az = bhz, an = bhn;
             xw[lane] = h;
             wave_sync();
 #pragma unroll
@@ -187,22 +210,15 @@ __global__ __launch_bounds__(GRU_THREADS) void gru_forward_reg_kernel(GruArgs A)
                 ar += hv.w * wr[k + 3]; az += hv.w * wz[k + 3]; an += hv.w * wn[k + 3];
             }
             wave_sync();
-        }
-        const float r = gate_sigmoid(xr + ar, FAST), z = gate_sigmoid(xz + az, FAST);
-        const float n = gate_tanh(xn + an * r, FAST);
-        float* po = A.L.post_activation + (size_t)t * stride + (size_t)b * 3 * H;
-        po[u] = r; po[H + u] = z; po[2 * H + u] = n;
-        const size_t at = ((size_t)t * A.B + b) * H + u;
-        A.L.n_pre_pre_activation[at] = an;
-        h = (1.0f - z) * n + z * h;
-        A.L.output[at] = h;
-        if (D == 1) { xr = fr; xz = fz; xn = fn; rs = fs; }
-        else {
-            xr = qr[0]; xz = qz[0]; xn = qn[0]; rs = qs[0];
-#pragma unroll
-            for (int d = 0; d + 1 < D - 1; d++) { qr[d] = qr[d + 1]; qz[d] = qz[d + 1]; qn[d] = qn[d + 1]; qs[d] = qs[d + 1]; }
-            qr[Q - 1] = fr; qz[Q - 1] = fz; qn[Q - 1] = fn; qs[Q - 1] = fs;
-        }
+            const float r = gate_sigmoid(q[N].r + ar, FAST), z = gate_sigmoid(q[N].z + az, FAST);
+            const float n = gate_tanh(q[N].n + an * r, FAST);
+            const float o = (1.0f - z) * n + z * h;
+            h = flags & 1 ? h0 : o;       // the next step starts an episode
+            flags >>= 1;
+            gru_at(post, at3) = r; gru_at(post + H, at3) = z; gru_at(post + 2 * H, at3) = n; gru_at(npp, at) = an; gru_at(out, at) = o;
+            post += 3 * stride; npp += stride; out += stride;
+            request(first + i + D, q[N]);      // behind the last use of the entry
+        });
     }
 }
 
@@ -210,54 +226,61 @@ __global__ __launch_bounds__(GRU_THREADS) void gru_forward_reg_kernel(GruArgs A)
 // d h_prev[k]); the gate gradients of the row's H units reach its lanes through three 64-float slots of LDS private to the wavefront.
 template <int H>
 __global__ __launch_bounds__(GRU_THREADS) void gru_backward_reg_kernel(GruArgs A) {
-    constexpr int G = 64 / H;
+    constexpr int G = 64 / H, D = 4;
     __shared__ __align__(16) float exchange[GRU_THREADS / 64][3][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, u = lane & (H - 1), row_base = lane & ~(H - 1);
-    const int b = (blockIdx.x * (GRU_THREADS / 64) + wave) * G + lane / H;
-    if (b >= A.B) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), u = lane & (H - 1), row_base = lane & ~(H - 1), S = A.S;
+    const int b0 = (blockIdx.x * (GRU_THREADS / 64) + wave) * G;
+    if (b0 >= A.B) return;
+    const int row = min(lane / H, A.B - 1 - b0);
     float cr[H], cz[H], cn[H];
 #pragma unroll
     for (int j = 0; j < H; j++) {
         cr[j] = A.L.weights_hidden[(size_t)j * H + u]; cz[j] = A.L.weights_hidden[(size_t)(H + j) * H + u]; cn[j] = A.L.weights_hidden[(size_t)(2 * H + j) * H + u];
     }
     const float h0 = A.L.initial_hidden_state[u];
-    float carry = 0.f, db_hn = 0.f;
-    // a step's saved values are requested two steps ahead (consecutive steps lie on different pages); steps before the first read the first again
-    struct Saved { float r, z, n, npp, dy, hp; int rs; };
-    auto request = [&](int t) {
-        const size_t a = (size_t)(t > 0 ? t : 0) * A.B + b;
-        Saved v;
-        v.r = A.L.post_activation[a * 3 * H + u]; v.z = A.L.post_activation[a * 3 * H + H + u]; v.n = A.L.post_activation[a * 3 * H + 2 * H + u];
-        v.npp = A.L.n_pre_pre_activation[a * H + u]; v.dy = A.d_output[a * H + u];
-        v.hp = A.L.output[((size_t)(t > 1 ? t - 1 : 0) * A.B + b) * H + u];
-        v.rs = A.reset ? A.reset[a] : 0;
-        return v;
+    const unsigned at = (row * H + u) * sizeof(float), at3 = (row * 3 * H + u) * sizeof(float);
+    const size_t stride = (size_t)A.B * H, last = (size_t)(S - 1) * stride + (size_t)b0 * H;
+    struct Saved { float r, z, n, npp, dy, hp; };
+    float *post = A.L.post_activation + 3 * last, *npp = A.L.n_pre_pre_activation + last, *dy = A.d_output + last, *state = A.L.output + last;
+    auto request = [&](int i, Saved& v) {      // i-th step from the end; steps before the first read the first again; the state is the one before the step (the first step's is not used)
+        const size_t on = i + 1 < S ? stride : 0;
+        state -= on;
+        v.r = gru_at(post, at3); v.z = gru_at(post + H, at3); v.n = gru_at(post + 2 * H, at3); v.npp = gru_at(npp, at); v.dy = gru_at(dy, at); v.hp = gru_at(state, at);
+        post -= 3 * on; npp -= on; dy -= on;
     };
-    Saved cur = request(A.S - 1), nxt = request(A.S - 2);
-    for (int t = A.S - 1; t >= 0; t--) {
-        const size_t at = (size_t)t * A.B + b;
-        const Saved far = request(t - 2);
-        const float r = cur.r, z = cur.z, n = cur.n, npp = cur.npp, dy = cur.dy, hp_raw = cur.hp;
-        const int rs = cur.rs;
-        const bool from_initial = t == 0 || rs;
-        const float hp = from_initial ? h0 : hp_raw;
-        const float dh = dy + carry;
-        A.d_output[at * H + u] = dh;
-        const float gz = dh * (hp - n) * z * (1.0f - z);
-        const float gn = dh * (1.0f - z) * (1.0f - n * n);
-        const float gr = gn * npp * r * (1.0f - r);
-        const float gnr = gn * r;
-        float* bi = A.buffer_input + at * 3 * H; float* bh = A.buffer_hidden + at * 3 * H;
-        bi[u] = gr; bi[H + u] = gz; bi[2 * H + u] = gn;
-        bh[u] = gr; bh[H + u] = gz; bh[2 * H + u] = gnr;
-        A.h_previous[at * H + u] = hp;
-        // the reference drops reset samples (t > 0) from the b_hn gradient (their buffer rows are zeroed before that sum, :716-749)
-        if (!(t > 0 && from_initial)) db_hn += gnr;
-        // the rows of one wavefront restart at different steps: every lane forms the sum, a restarting row drops it
-        float a0 = dh * z, a1 = 0.f, a2 = 0.f;
-        {
-            float* xw = &exchange[wave][0][0];
+    Saved q[D];
+#pragma unroll
+    for (int d = 0; d < D; d++) request(d, q[d]);
+    float *to_dy = A.d_output + last, *to_hp = A.h_previous + last, *bi = A.buffer_input + 3 * last, *bh = A.buffer_hidden + 3 * last;
+    float* const xw = &exchange[wave][0][0];
+    float carry = 0.f, db_hn = 0.f;
+    for (int back = 0; back < S; back += 64) {
+        const int steps = min(64, S - back);
+        const uint64_t flags = gru_reset_flags<G>(A.reset, S - back - steps, S, A.B, b0, lane / H);      // bit of step t = S - 1 - back - i: steps - 1 - i
+        uint64_t high = flags << (64 - steps);
+        gru_steps<D>(steps, [&](auto number, int i) {
+            constexpr int N = decltype(number)::value;
+            __builtin_amdgcn_sched_barrier(0);
+            const Saved cur = q[N];
+            const bool first = back + i + 1 == S, from_initial = first || (high >> 63);
+            high <<= 1;
+            const float hp = from_initial ? h0 : cur.hp;
+            const float dh = cur.dy + carry;
+            const float gz = dh * (hp - cur.n) * cur.z * (1.0f - cur.z);
+            const float gn = dh * (1.0f - cur.z) * (1.0f - cur.n * cur.n);
+            const float gr = gn * cur.npp * cur.r * (1.0f - cur.r);
+            const float gnr = gn * cur.r;
             xw[lane] = gr; xw[64 + lane] = gz; xw[128 + lane] = gnr;
+            // the rows of one wavefront restart at different steps: every lane forms the sum, a restarting row drops it
+            float a0 = dh * cur.z, a1 = 0.f, a2 = 0.f;
+            asm volatile("" : "+v"(a0));      // (not formed below by a multiply-add that would keep the entry's z)
+            request(back + i + D, q[N]);      // behind the last use of the entry
+            gru_at(to_dy, at) = dh; gru_at(to_hp, at) = hp;
+            gru_at(bi, at3) = gr; gru_at(bi + H, at3) = gz; gru_at(bi + 2 * H, at3) = gn;
+            gru_at(bh, at3) = gr; gru_at(bh + H, at3) = gz; gru_at(bh + 2 * H, at3) = gnr;
+            to_dy -= stride; to_hp -= stride; bi -= 3 * stride; bh -= 3 * stride;
+            // the reference drops reset samples (t > 0) from the b_hn gradient (their buffer rows are zeroed before that sum, :716-749)
+            db_hn += first || !from_initial ? gnr : 0.f;
             wave_sync();
 #pragma unroll
             for (int j = 0; j < H; j += 4) {
@@ -269,11 +292,10 @@ __global__ __launch_bounds__(GRU_THREADS) void gru_backward_reg_kernel(GruArgs A
                 a0 += vr.w * cr[j + 3]; a1 += vz.w * cz[j + 3]; a2 += vn.w * cn[j + 3];
             }
             wave_sync();
-        }
-        carry = from_initial ? 0.f : a0 + (a1 + a2);
-        cur = nxt; nxt = far;
+            carry = from_initial ? 0.f : a0 + (a1 + a2);
+        });
     }
-    if (A.db_hn_partial) A.db_hn_partial[(size_t)b * H + u] = db_hn;
+    if (A.db_hn_partial) gru_at(A.db_hn_partial + (size_t)b0 * H, at) = db_hn;
 }
 
 // ---- hidden width 64: the recurrence on the matrix cores -------------------------------------------------------------------------
@@ -309,34 +331,6 @@ __device__ __forceinline__ float sum_quarters(gru_floatx4 c) {
     auto swap16 = [](unsigned a, unsigned b) { return __builtin_amdgcn_permlane16_swap(a, b, false, false); };
     return across(across(c[0], c[2], swap32), across(c[1], c[3], swap32), swap16);
 }
-// The steps of a sequence in groups of D whose members know their number in the group (a queue's entries are indexed by it). Whole groups are straight-line code: with an
-// exit before every step the compiler waits for all requests where the paths meet. For the same reason everything requested before the loop is waited for in front of it: the
-// first step of a group then waits for its own values, requested D steps before, and not for the last ones.
-template <class F, int... K> __device__ __forceinline__ void gru_whole_group(int first, F& step, std::integer_sequence<int, K...>) { (step(std::integral_constant<int, K>{}, first + K), ...); }
-template <class F, int... K> __device__ __forceinline__ void gru_rest(int first, int S, F& step, std::integer_sequence<int, K...>) { ((first + K < S ? step(std::integral_constant<int, K>{}, first + K) : (void)0), ...); }
-template <int D, class F>
-__device__ __forceinline__ void gru_steps(int S, F&& step) {
-    int i = 0;
-    __builtin_amdgcn_s_waitcnt(0x0F70);      // vmcnt(0)
-    for (; i + D <= S; i += D) gru_whole_group(i, step, std::make_integer_sequence<int, D>{});
-    gru_rest(i, S, step, std::make_integer_sequence<int, D - 1>{});
-}
-
-// Reset flags of 64 consecutive steps from `first` on, as a mask in every lane of the row's group (bit i: step first + i starts an episode); steps from S on: no. A wavefront
-// reads a step per lane: a byte load per step would hold the recurrence up for its widening.
-__device__ __forceinline__ uint64_t gru_reset_flags(const uint8_t* reset, int first, int S, int B, int b0, int kg) {
-    if (!reset) return 0;
-    const int t = first + (int)(threadIdx.x & 63);
-    uint64_t mask = 0;
-#pragma unroll
-    for (int r = 0; r < GM_ROWS; r++) {
-        const uint64_t row = __ballot(t < S && reset[(size_t)min(t, S - 1) * B + min(b0 + r, B - 1)] != 0);
-        mask = kg == r ? row : mask;
-    }
-    return mask;
-}
-__device__ __forceinline__ float& gru_at(float* base, unsigned bytes) { return *reinterpret_cast<float*>(reinterpret_cast<char*>(base) + bytes); }
-
 // hs (two copies, by the parity of the step): the previous hidden state of the four rows in the order of the A operand: group kg's lane (cg, row) reads
 // units 16 kg + 4 s + cg, s = 0 ... 3, in one 16-byte read. One workgroup barrier per step. Lane = (row kg, unit) finishes its unit; rows beyond the batch repeat the last
 // row (the same wavefront's lanes hold it: they read, compute and store the same values). Memory is addressed by pointers of the workgroup that move from step to step and
@@ -373,7 +367,7 @@ __global__ __launch_bounds__(256, 2) void gru_forward_mfma_kernel(GruArgs A) {
     float h = h0;
     hs[0][place] = h;
     for (int first = 0; first < A.S; first += 64) {
-        uint64_t flags = gru_reset_flags(A.reset, first + 1, A.S, A.B, b0, kg);      // of the steps after these
+        uint64_t flags = gru_reset_flags<GM_ROWS>(A.reset, first + 1, A.S, A.B, b0, kg);      // of the steps after these
         gru_steps<D>(min(64, A.S - first), [&](auto number, int i) {
             constexpr int N = decltype(number)::value;
             __builtin_amdgcn_sched_barrier(0);      // later steps' values are not touched (and waited for) before their step
@@ -435,7 +429,7 @@ __global__ __launch_bounds__(256, 2) void gru_backward_mfma_kernel(GruArgs A) {
     float carry = 0.f, db_hn = 0.f;
     for (int back = 0; back < S; back += 64) {
         const int steps = min(64, S - back);
-        const uint64_t flags = gru_reset_flags(A.reset, S - back - steps, S, A.B, b0, kg);      // bit of step t = S - 1 - back - i: steps - 1 - i
+        const uint64_t flags = gru_reset_flags<GM_ROWS>(A.reset, S - back - steps, S, A.B, b0, kg);      // bit of step t = S - 1 - back - i: steps - 1 - i
         uint64_t high = flags << (64 - steps);
         gru_steps<D>(steps, [&](auto number, int i) {
             constexpr int N = decltype(number)::value;
