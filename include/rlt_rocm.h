@@ -680,11 +680,13 @@ int rlt_rocm_sac_train_actor_drawn(rlt_rocm_device* device, const rlt_sac_agent*
  * grids of at most 32 workgroups are placed on one XCD, whose L2 then serves the exchange; 0: spread over all XCDs. The environment
  * variables RLT_UPDATE_TAIL=0 and RLT_UPDATE_PLACEMENT=spread set the defaults of a process. No counterpart in the reference. */
 int rlt_rocm_set_update_options(rlt_rocm_device* device, int optimiser_in_kernel, int one_xcd);
-/* The kernels whose workgroups wait for each other (the persistent SAC loop; update kernels that end with the optimiser's step) poll a
- * bounded number of times, then give up: the kernel still ends normally, its results are void, and the next rlt_rocm_check_status returns
- * RLT_E_DEVICE_TIMEOUT. `polls` sets that bound (0: the default, about a second). With a bound of 1 every workgroup of an update kernel
- * but the last to arrive gives up without looking at the counter, which makes the give-up path testable from the host. No counterpart in
- * the reference. */
+/* The kernels whose workgroups wait for each other poll a bounded number of times, then give up: the kernel still ends normally, its results
+ * are void, and the next rlt_rocm_check_status returns RLT_E_DEVICE_TIMEOUT. These are the persistent SAC loop, the update kernels that end
+ * with the optimiser's step or with sums per XCD, and, whatever rlt_rocm_set_update_options says, the SAC and TD3 updates of agents that do
+ * not fit those (hidden widths up to 256, batches up to 2,048), whose network passes run in workgroups of their own and hand values over;
+ * an update of these that gives up leaves parameters, moments, target networks and ages as they were before it. `polls` sets that bound
+ * (0: the default, about a second). With a bound of 1 every workgroup that would wait gives up without looking (of an update kernel with the
+ * optimiser's step, all but the last to arrive), which makes the give-up path testable from the host. No counterpart in the reference. */
 int rlt_rocm_set_wait_limit(rlt_rocm_device* device, unsigned polls);
 
 /* The same n_steps iterations of sac::loop::core::step (rl/algorithms/sac/loop/core/operations_generic.h:110-155 past the warm-up,

@@ -16,7 +16,12 @@ struct rlt_gradient_net {
 // one more optimiser (log_alpha's): a scalar whose gradient is `scale` times the sum of `n` values (n <= 128)
 struct rlt_gradient_scalar { const float* values; int n; float scale; rlt_adam_tensor tensor; rlt_adam_parameters adam; const uint32_t* age; };
 
+// What the launch before may have left undone: its kernel gave up waiting (*fault set: the gradients are not those of the batch). Then the sums are stored, but no step is
+// taken and the ages, which that launch has advanced, get their values back. age[k]: of the networks' optimisers, then the scalar's; before: the values, in that order.
+struct rlt_gradient_guard { const unsigned* fault; uint32_t* age[3]; const uint32_t* before; };
+
 // floats that `partial` needs for these networks (0: none)
 size_t rlt_batch_gradients_partial_floats(const rlt_gradient_net* nets, int n_nets, int batch);
 // up to two networks on batches of the same size; one launch, or two where the batch is shared out (see batch_gradient.hip)
-int rlt_batch_gradients(rlt_rocm_device* device, const rlt_gradient_net* nets, int n_nets, int batch, float polyak, const rlt_gradient_scalar* scalar, float* partial);
+int rlt_batch_gradients(rlt_rocm_device* device, const rlt_gradient_net* nets, int n_nets, int batch, float polyak, const rlt_gradient_scalar* scalar, float* partial,
+                        const rlt_gradient_guard* guard = nullptr);

@@ -20,6 +20,7 @@ constexpr int WAVES = 4, THREADS = 64 * WAVES, SPLIT_ROWS = 512, MAX_SPLITS = 8;
 struct GradientLaunch {
     rlt_gradient_net net[2]; int blocks0, batch, splits, total0, total; float polyak;      // total0, total: gradient elements of the first network, of both
     rlt_gradient_scalar scalar; int has_scalar;
+    rlt_gradient_guard guard;      // fault NULL: nothing to look at
     float* partial;      // splits > 1: [splits][total] sums, the networks' elements one after the other, segments in order
 };
 
@@ -35,24 +36,32 @@ __device__ __forceinline__ Held hold(const rlt_gradient_net& N, int segment, siz
     }
     return h;
 }
-__device__ __forceinline__ void finish(const rlt_gradient_net& N, int segment, size_t at, float sum, Held h, float bc1, float bc2, float polyak) {
+__device__ __forceinline__ void finish(const rlt_gradient_net& N, int segment, size_t at, float sum, Held h, float bc1, float bc2, float polyak, bool is_void) {
     float* const gradient = N.gradient[segment] + at;
     if (!N.step) { *gradient += sum; return; }
     *gradient = sum;
+    if (is_void) return;
     rlt_adam_values(N.adam, N.flags[segment], sum, bc1, bc2, h.first, h.second, h.value);
     N.first_moment[segment][at] = h.first; N.second_moment[segment][at] = h.second; N.parameter[segment][at] = h.value;
     if (N.target[segment]) N.target[segment][at] = rlt_polyak_value(polyak, h.target, h.value);
 }
 // log_alpha's step, by one wavefront
-__device__ __forceinline__ void finish_scalar(const rlt_gradient_scalar& Z, int lane) {
+__device__ __forceinline__ void finish_scalar(const rlt_gradient_scalar& Z, int lane, bool is_void) {
     float s = (lane < Z.n ? Z.values[lane] : 0.f) + (64 + lane < Z.n ? Z.values[64 + lane] : 0.f);
     s = rlt_wave_sum(s);
     if (lane == 0) {
+        *Z.tensor.gradient = s * Z.scale;
+        if (is_void) return;
         float bc1, bc2;
         rlt_adam_bias_corrections(Z.adam, *Z.age, bc1, bc2);
-        *Z.tensor.gradient = s * Z.scale;
         rlt_adam_apply(Z.adam, Z.tensor, 0, s * Z.scale, bc1, bc2, 0.0f);
     }
+}
+
+__device__ __forceinline__ bool void_update(const rlt_gradient_guard& G) { return G.fault && *G.fault != 0; }
+__device__ __forceinline__ void give_ages_back(const rlt_gradient_guard& G) {      // by one thread of the launch (which reads the ages from `before`)
+#pragma unroll
+    for (int k = 0; k < 3; k++) if (G.age[k]) *G.age[k] = G.before[k];
 }
 
 // TM: rows of the tile. 16 where a workgroup sees the whole batch (few rows: as many workgroups as the gradients give); 32 where the batch is shared out, which gives
@@ -86,6 +95,7 @@ __global__ __launch_bounds__(THREADS) void batch_gradient_kernel(GradientLaunch 
         }
         if (N.step) rlt_adam_bias_corrections(N.adam, *N.age, bc1, bc2);
     }
+    const bool is_void = !SPLIT && void_update(K.guard);
     floatx4 c[TM / 16][2];
     float bias[TM / 16];
     tile_product<TM / 16>(a, lda, rows, TM * mt, b, ldb, cols, TN * nt, B, k0, k1, r, g, c, bias);
@@ -100,7 +110,7 @@ __global__ __launch_bounds__(THREADS) void batch_gradient_kernel(GradientLaunch 
             const float sum = (P.tile[0][em][en] + P.tile[1][em][en]) + (P.tile[2][em][en] + P.tile[3][em][en]);
             const size_t at = (size_t)(TM * mt + em) * cols + TN * nt + en;
             if (SPLIT) K.partial[first + at] = sum;
-            else finish(N, segment, at, sum, held[u], bc1, bc2, K.polyak);
+            else finish(N, segment, at, sum, held[u], bc1, bc2, K.polyak, is_void);
         }
     }
     // the layer's bias gradient: column sums of the left operand, by the workgroups of the first column tile
@@ -108,14 +118,16 @@ __global__ __launch_bounds__(THREADS) void batch_gradient_kernel(GradientLaunch 
         const int at = TM * mt + threadIdx.x;
         const float sum = (P.bias[0][threadIdx.x] + P.bias[1][threadIdx.x]) + (P.bias[2][threadIdx.x] + P.bias[3][threadIdx.x]);
         if (SPLIT) K.partial[first + (size_t)rows * cols + at] = sum;
-        else finish(N, segment + 1, at, sum, hold(N, segment + 1, at), bc1, bc2, K.polyak);
+        else finish(N, segment + 1, at, sum, hold(N, segment + 1, at), bc1, bc2, K.polyak, is_void);
     }
-    if (!SPLIT && K.has_scalar && blockIdx.x == gridDim.x - 1 && wave == 0) finish_scalar(K.scalar, lane);
+    if (!SPLIT && K.has_scalar && blockIdx.x == gridDim.x - 1 && wave == 0) finish_scalar(K.scalar, lane, is_void);
+    if (!SPLIT && is_void && blockIdx.x == 0 && threadIdx.x == 0) give_ages_back(K.guard);
 }
 
 // the splits' sums added up, in order, and the elements finished
 __global__ __launch_bounds__(256) void finish_kernel(GradientLaunch K) {
     const int e = blockIdx.x * 256 + threadIdx.x;
+    const bool is_void = void_update(K.guard);
     if (e < K.total) {
         const int y = e >= K.total0 ? 1 : 0;
         const rlt_gradient_net& N = y ? K.net[1] : K.net[0];
@@ -129,9 +141,10 @@ __global__ __launch_bounds__(256) void finish_kernel(GradientLaunch K) {
         float bc1 = 0.f, bc2 = 0.f;
         if (N.step) rlt_adam_bias_corrections(N.adam, *N.age, bc1, bc2);
         const float sum = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
-        finish(N, segment, at, sum, h, bc1, bc2, K.polyak);
+        finish(N, segment, at, sum, h, bc1, bc2, K.polyak, is_void);
     }
-    if (K.has_scalar && blockIdx.x == gridDim.x - 1 && threadIdx.x < 64) finish_scalar(K.scalar, threadIdx.x);
+    if (K.has_scalar && blockIdx.x == gridDim.x - 1 && threadIdx.x < 64) finish_scalar(K.scalar, threadIdx.x, is_void);
+    if (is_void && blockIdx.x == 0 && threadIdx.x == 0) give_ages_back(K.guard);
 }
 
 int blocks_of(const rlt_gradient_net& N, int TM) {
@@ -149,7 +162,8 @@ size_t rlt_batch_gradients_partial_floats(const rlt_gradient_net* nets, int n_ne
     return n * splits_for(batch);
 }
 
-int rlt_batch_gradients(rlt_rocm_device* device, const rlt_gradient_net* nets, int n_nets, int batch, float polyak, const rlt_gradient_scalar* scalar, float* partial) {
+int rlt_batch_gradients(rlt_rocm_device* device, const rlt_gradient_net* nets, int n_nets, int batch, float polyak, const rlt_gradient_scalar* scalar, float* partial,
+                        const rlt_gradient_guard* guard) {
     RLT_REQUIRE(nets && n_nets >= 1 && n_nets <= 2 && batch > 0 && (!scalar || scalar->n <= 128) && (n_nets == 1 || nets[0].step == nets[1].step));
     GradientLaunch K = {};
     int blocks = 0;
@@ -159,6 +173,7 @@ int rlt_batch_gradients(rlt_rocm_device* device, const rlt_gradient_net* nets, i
     }
     K.batch = batch; K.polyak = polyak; K.splits = splits_for(batch); K.partial = partial;
     if (scalar) { K.scalar = *scalar; K.has_scalar = 1; }
+    if (guard) K.guard = *guard;
     if (K.splits == 1) {
         hipLaunchKernelGGL(batch_gradient_kernel<false>, dim3(blocks), dim3(THREADS), 0, device->stream, K);
         return rlt_launch_status(device);

@@ -272,13 +272,20 @@ __device__ __forceinline__ void store_rows(lptr from, float* to, int hid, int ro
     for (int n = lane; n < hid; n += 64) row[n] = from[wave * S + n];
 }
 // A value handed from one workgroup to another of the same launch: one 8-byte store that carries its own tag, so that nothing has to be ordered around it. The wait is
-// bounded (rlt_rocm_set_wait_limit); a workgroup that gives up sets the fault word and goes on with zero, and the update's results are void.
+// bounded (rlt_rocm_set_wait_limit: at most max_poll - 1 looks, with a bound of one none); a workgroup that gives up sets the fault word and goes on with zero, and the next
+// launch, which has the gradients of nothing then, leaves parameters, moments, targets and ages as they were (rlt_gradient_guard).
 __device__ __forceinline__ void hand_over(uint64_t* word, float value) {
     __hip_atomic_store(word, (1ull << 32) | (uint64_t)__float_as_uint(value), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 template <int N>
 __device__ __forceinline__ void take_over(uint64_t* const (&word)[N], float (&value)[N], unsigned max_poll, unsigned* fault) {
     for (unsigned tries = 0;;) {
+        if (++tries >= max_poll) {
+#pragma unroll
+            for (int i = 0; i < N; i++) value[i] = 0.f;
+            __hip_atomic_store(fault, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return;
+        }
         bool all = true;
         uint64_t w[N];
 #pragma unroll
@@ -286,7 +293,6 @@ __device__ __forceinline__ void take_over(uint64_t* const (&word)[N], float (&va
 #pragma unroll
         for (int i = 0; i < N; i++) { all = all && (w[i] >> 32) != 0; value[i] = __uint_as_float((uint32_t)w[i]); }
         if (all) return;
-        if (++tries >= max_poll) { __hip_atomic_store(fault, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); return; }
         __builtin_amdgcn_s_sleep(1);
     }
 }
@@ -854,11 +860,12 @@ int launch_wide(rlt_rocm_device* device, WideArgs& a, int groups, const Optimise
 #undef RLT_LAUNCH_WIDE_ACT
 #undef RLT_LAUNCH_WIDE
     if ((rc = rlt_launch_status(device))) return rc;
+    const rlt_gradient_guard guard = {device->fault, {opts[0].age, n_opts > 1 ? opts[1].age : nullptr, opts[0].second ? opts[0].second_age : nullptr}, age_before};
     if (opts[0].second) {
         const rlt_gradient_scalar scalar = {a.extra, groups, opts[0].second_scale, *opts[0].second, *opts[0].second_parameters, age_before + 2};
-        return rlt_batch_gradients(device, net, n_opts, a.batch, polyak, &scalar, partial);
+        return rlt_batch_gradients(device, net, n_opts, a.batch, polyak, &scalar, partial, &guard);
     }
-    return rlt_batch_gradients(device, net, n_opts, a.batch, polyak, nullptr, partial);
+    return rlt_batch_gradients(device, net, n_opts, a.batch, polyak, nullptr, partial, &guard);
 }
 
 void set_noise(WideArgs& a, const rlt_update_noise& N) { a.noise = N.values; a.noise_seed = N.seed; a.noise_stream = N.stream; a.out_noise = N.values ? nullptr : N.drawn; }

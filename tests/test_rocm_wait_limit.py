@@ -1,5 +1,5 @@
 """The bounded waits of the kernels whose workgroups wait for each other (the persistent SAC loop, rl/algorithms/sac/loop/core/operations_generic.h:110-155
-in one launch; the update kernels that end with the optimiser's step): with the bound set to one poll from the host (rlt_rocm_set_wait_limit) the first
+in one launch; the update kernels that end with the optimiser's step; the updates of wider agents, whose passes hand values over): with the bound set to one poll from the host (rlt_rocm_set_wait_limit) the first
 workgroups to arrive give up at once, every kernel still ends normally, and the next rlt_rocm_check_status reports RLT_E_DEVICE_TIMEOUT. The error is
 sticky on that handle, so each case runs on a device handle of its own; the same calls on a fresh handle with the default bound succeed."""
 import ctypes as C
@@ -96,3 +96,54 @@ def test_update_kernel_that_sums_per_xcd_gives_up_and_reports():
         assert np.abs(agent.parameters() - params).max() > 1e-5 and int(agent.actor.age.numpy()[0]) == 2
     finally:
         patient.close()
+
+
+def wide_state(agent, nets):
+    """parameters, moments and ages of the trained networks, and every parameter of the agent"""
+    return [agent.parameters()] + [a.numpy() for n in nets for a in (n.m, n.v, n.age)]
+
+
+# (entry point, batch): one launch of gradients, and the batch shared out to groups of workgroups whose sums a third launch adds up
+@pytest.mark.parametrize("batch", [100, 513])
+@pytest.mark.parametrize("update", ["sac_train_critics", "sac_train_actor", "td3_train_critics"])
+def test_update_of_a_wider_agent_gives_up_and_leaves_the_agent_as_it_was(update, batch):
+    print("case", update, batch, flush=True)
+    obs, act, hidden, rng = 6, 2, 256, np.random.default_rng(batch)
+    nets = [[obs, hidden, hidden, 2 * act]] if update.startswith("sac") else [[obs, hidden, hidden, act]] * 2
+    params = np.concatenate([helpers.random_params(rng, dims) for dims in nets + [[obs + act, hidden, hidden, 1]] * 4] + ([np.array([np.log(0.5)], np.float32)] if update.startswith("sac") else []))
+    data, noise = batch_of(rng, batch, obs, act), rng.standard_normal((batch, act)).astype(np.float32)
+
+    def run(limit):
+        be = helpers.RocmBackend()
+        try:
+            if update.startswith("sac"):
+                agent = helpers.SacOnBackend(be, batch, hidden, params, masks=False, obs=obs, act=act)
+                agent.set_batch(*data)
+            else:
+                agent = helpers.Td3OnBackend(be, batch, hidden, params, obs=obs, act=act)
+                agent.set_batch(*data, 0.1 * noise)
+            trained = [agent.actor] if update.endswith("actor") else agent.critics
+            before = wide_state(agent, trained)
+            alpha = [agent.log_alpha.numpy(), agent.alpha_age.numpy()] if update == "sac_train_actor" else []
+            nd = be.array(noise)
+            be.call("set_wait_limit", limit)
+            lib, h = be.device.lib, be.device.handle
+            if update == "sac_train_critics":
+                rc = lib.rlt_rocm_sac_train_critics(h, C.byref(agent.c), nd.ptr, 1)
+            elif update == "sac_train_actor":
+                rc = lib.rlt_rocm_sac_train_actor(h, C.byref(agent.c), nd.ptr)
+            else:
+                rc = lib.rlt_rocm_td3_train_critics(h, C.byref(agent.c), nd.ptr, nd.ptr)
+            assert rc == 0
+            after = wide_state(agent, trained)      # read before the status, whose error sticks
+            if alpha:
+                assert np.array_equal(agent.log_alpha.numpy()[[0, 2, 3]], alpha[0][[0, 2, 3]]) == (limit == 1) and agent.alpha_age.numpy()[0] == alpha[1][0] + (limit != 1)
+            return before, after, lib.rlt_rocm_check_status(h)
+        finally:
+            be.close()
+
+    before, after, status = run(1)
+    assert status == capi.RLT_E_DEVICE_TIMEOUT
+    assert all(np.array_equal(a, b) for a, b in zip(before, after))
+    before, after, status = run(0)
+    assert status == 0 and not any(np.array_equal(a, b) for a, b in zip(before, after))
