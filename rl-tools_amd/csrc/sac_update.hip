@@ -270,7 +270,7 @@ __global__ __launch_bounds__(THREADS) void sac_update_kernel(UpdateArgs A) {
         for (int j = 0; j < XN; j++) {
             const int c = c0 + 32 * j;
             if (CRITIC) {
-                xa[j] = (rok && c < D) ? nxt[min(c, D - 1)] : 0.f;
+                xa[j] = (rok && c < OBS) ? nxt[min(c, D - 1)] : 0.f;      // the target's sample goes behind them; what the batch holds there could turn zero weights of the actor's last chunk into NaN
                 xb[j] = (rok && c < D) ? cur[min(c, D - 1)] : 0.f;
             } else {
                 xa[j] = (rok && c < OBS) ? cur[min(c, D - 1)] : 0.f;

@@ -371,10 +371,12 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
     const int set = target_role ? role >> 1 : 0;
 
     RLT_TICK(0);
-    // the input rows: next rows for the target roles, else the current ones (the actor reads their observation columns, zero beyond them until the sample is in place)
+    // the input rows: next rows for the target roles, else the current ones. The actor reads the observation columns, zero beyond them until the sample is in place: what the
+    // batch holds there meets zero weights in the actor's last chunk, and must not be a NaN or an infinity
     float in_row[3];
-    request_row(A.batch_base + (target_role ? (size_t)B * D : 0) + (size_t)min(row0 + wave, B - 1) * D, CRITIC ? D : OBS, lane, in_row);
-    if (CRITIC && !target_role) {
+    const bool trained_role = CRITIC && !target_role;
+    request_row(A.batch_base + (target_role ? (size_t)B * D : 0) + (size_t)min(row0 + wave, B - 1) * D, trained_role ? D : OBS, lane, in_row);
+    if (trained_role) {
         // ---- a trained critic
         const int y = role - n_target_roles;
         const WNet trained = y ? A.critic[1] : A.critic[0];      // by value: an index into the kernel's argument would keep all of it in private memory
@@ -382,7 +384,7 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
         const int HID = trained.hid, tiles = (HID + 15) >> 4;
         Operands<NT1C> W;
         load_operands<NT1C>(trained, wave, c, g, W);
-        place_row(xa + wave * SXS, row0 + wave < B, CRITIC ? D : OBS, SXS, lane, in_row);
+        place_row(xa + wave * SXS, row0 + wave < B, D, SXS, lane, in_row);
         float reward[4] = {0.f, 0.f, 0.f, 0.f}, alpha = 0.f, b3 = 0.f;
         bool terminated[4] = {false, false, false, false};
         if (scalar_wave) {
@@ -450,7 +452,7 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
     const WNet Q = CRITIC ? (critic_index ? A.target[1] : A.target[0]) : (critic_index ? A.critic[1] : A.critic[0]);
     Operands<NT1C> W;
     load_operands<NT1C>(A.actor, wave, c, g, W);      // on their way while the input rows are written
-    place_row(xa + wave * SXS, row0 + wave < B, CRITIC ? D : OBS, SXS, lane, in_row);
+    place_row(xa + wave * SXS, row0 + wave < B, OBS, SXS, lane, in_row);
     float noise[2] = {0.f, 0.f}, target_noise[2] = {0.f, 0.f}, alpha = 0.f, actor_b3 = 0.f, q_b3 = 0.f;
     if (scalar_wave) {
         actor_b3 = c < A.actor.out ? A.actor.b3[c] : 0.f; q_b3 = Q.b3[0];

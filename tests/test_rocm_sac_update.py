@@ -145,6 +145,34 @@ def test_wider_agents_at_large_batches(oracle, rocm, batch, hidden):
 
 
 
+@pytest.mark.parametrize("hidden", [64, 256])
+@pytest.mark.parametrize("algorithm", ["sac", "td3"])
+def test_next_actions_of_the_batch_are_not_looked_at(rocm, algorithm, hidden):
+    """The critic updates act on the next observations themselves; the rows' action columns behind them (which share a chunk of sixteen inputs with them) may hold anything."""
+    print("case", algorithm, hidden, flush=True)
+    batch, obs, act = 100, 6, 2
+    rng = np.random.default_rng(hidden)
+    actors = [[obs, hidden, hidden, 2 * act]] if algorithm == "sac" else [[obs, hidden, hidden, act]] * 2
+    params = np.concatenate([helpers.random_params(rng, dims) for dims in actors + [[obs + act, hidden, hidden, 1]] * 4] + ([np.array([np.log(0.5)], np.float32)] if algorithm == "sac" else []))
+    oab, rewards, terminated = batch_of(rng, batch, obs, act)
+    noise = rng.standard_normal((batch, act)).astype(np.float32)
+    results = []
+    for value in (0.0, np.nan, np.inf):
+        oab[1, :, obs:] = value
+        if algorithm == "sac":
+            agent = helpers.SacOnBackend(rocm, batch, hidden, params, masks=False, obs=obs, act=act)
+            agent.set_batch(oab, rewards, terminated)
+            rocm.call("sac_train_critics", C.byref(agent.c), rocm.array(noise).ptr, 1)
+        else:
+            agent = helpers.Td3OnBackend(rocm, batch, hidden, params, obs=obs, act=act)
+            agent.set_batch(oab, rewards, terminated, 0.1 * noise)
+            rocm.call("td3_train_critics", C.byref(agent.c), rocm.array(noise).ptr, rocm.array(noise).ptr)
+        rocm.sync()
+        results.append([agent.parameters()] + [c.grads.numpy() for c in agent.critics])
+        assert all(np.isfinite(a).all() for a in results[-1])
+    assert all(np.array_equal(a, b) for r in results[1:] for a, b in zip(results[0], r))
+
+
 def test_agents_outside_the_fused_shapes_take_the_per_operation_path(oracle, rocm):
     """an agent with sequence masks: same entry points, same results as the checker"""
     batch, obs, act = 64, 3, 1
