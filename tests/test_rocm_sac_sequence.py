@@ -54,7 +54,11 @@ def test_sequential_model_forward_and_backward_match_checker(oracle, rocm, case)
     S, B, I, H, O, n_gru, fast, with_reset = case
     rng = np.random.default_rng(S * 100 + B)
     specs = [(0, I, H, "relu")] + [(1, H, H, "identity")] * n_gru + [(0, H, H, "tanh"), (0, H, O, "identity")]
-    params = helpers.random_seq_params(rng, specs)
+    model_against_checker(oracle, rocm, rng, specs, helpers.random_seq_params(rng, specs), S, B, fast, with_reset)
+
+
+def model_against_checker(oracle, rocm, rng, specs, params, S, B, fast, with_reset):
+    I, O = specs[0][1], specs[-1][2]
     x, g = rng.standard_normal((S, B, I + 2)).astype(np.float32), rng.standard_normal((S, B, O)).astype(np.float32)      # the input has a leading dimension of I + 2
     reset = (rng.uniform(size=(S, B)) < 0.2).astype(np.uint8)
     res = {}
@@ -81,6 +85,88 @@ def test_sequential_model_forward_and_backward_match_checker(oracle, rocm, case)
     if with_reset and reset[1:].any() and S > 1:
         assert rel_err(res["oracle"]["dx_input_only_0"], res["oracle"]["dx_input_only_1"]) > 1e-3
         assert rel_err(res["oracle"]["dx_input_only_1"], res["oracle"]["dx"]) <= 1e-6
+
+
+def with_initial_states(rng, specs, params):
+    """The GRU layers' initial hidden states, which random_seq_params leaves at zero, drawn as well."""
+    at = 0
+    for kind, i, o, _ in specs:
+        at += o * i + o if kind == 0 else 3 * o * i + 3 * o + 3 * o * o + 4 * o
+        if kind:
+            params[at - o:at] = rng.uniform(-0.5, 0.5, o)
+    return params
+
+
+# dense, GRU, GRU, dense: all layers of a pass in one launch (seq_stack.hip). (steps, batch, in, hidden, out, fast_tanh, hidden activation): the narrowest and widest inputs and
+# outputs, one step, steps that fill neither the pairs nor the groups of six that the loops are unrolled to, exact and rational gates
+STACK_CASES = [(7, 3, 1, 16, 1, True, "relu"), (13, 5, 16, 16, 16, False, "tanh"), (1, 2, 4, 16, 2, False, "relu"), (6, 9, 1, 32, 16, False, "sigmoid"), (11, 4, 16, 32, 1, True, "relu"),
+               (1, 7, 3, 32, 3, True, "fast_tanh"), (2, 1, 5, 32, 2, False, "identity"), (100, 33, 9, 16, 5, True, "relu"), (65, 20, 13, 32, 7, False, "tanh")]
+
+
+@pytest.mark.parametrize("with_reset", [False, True])
+@pytest.mark.parametrize("case", STACK_CASES)
+def test_recurrent_approximators_in_one_launch_match_checker(oracle, rocm, case, with_reset):
+    print("case", case, with_reset, flush=True)
+    S, B, I, H, O, fast, act = case
+    rng = np.random.default_rng(S * 10 + I)
+    specs = [(0, I, H, act), (1, H, H, "identity"), (1, H, H, "identity"), (0, H, O, "identity")]
+    model_against_checker(oracle, rocm, rng, specs, with_initial_states(rng, specs, helpers.random_seq_params(rng, specs)), S, B, fast, with_reset)
+
+
+def stacked_agents(rng, backends, S, B, OBS, ACT, actor_hidden, critic_hidden, first, spread=1.0):
+    """SAC agents whose networks are all dense, GRU, GRU, dense"""
+    specs = lambda i, h, o: [(0, i, h, "relu"), (1, h, h, "identity"), (1, h, h, "identity"), (0, h, o, "identity")]
+    actor_specs, critic_specs = specs(OBS, actor_hidden, 2 * ACT), specs(OBS + ACT, critic_hidden, 1)
+    draw = lambda s: with_initial_states(rng, s, helpers.random_seq_params(rng, s))
+    critics = [draw(critic_specs) for _ in range(2)]
+    params = np.concatenate([draw(actor_specs)] + critics + [c.copy() * spread for c in critics] + [np.array([np.log(0.5)], np.float32)]).astype(np.float32)
+    hyper = dict(sas=helpers.capi.SasParameters(-20.0, 2.0, 1e-6, -float(ACT)))
+    return params, [helpers.SacSequenceOnBackend(be, actor_specs, critic_specs, params, S, B, OBS, ACT, first, hyper) for be in backends]
+
+
+# (steps, batch, observations, actions, actor's width, critics' width, first step in the targets)
+STACKED_AGENTS = [(1, 3, 3, 1, 16, 32, True), (7, 13, 5, 2, 16, 32, False), (13, 5, 12, 4, 32, 16, True), (31, 64, 3, 1, 16, 16, True), (100, 40, 8, 8, 32, 32, False)]
+
+
+@pytest.mark.parametrize("case", STACKED_AGENTS)
+def test_sac_sequence_updates_of_recurrent_approximators_in_shared_launches(oracle, rocm, case):
+    """Actor and critics dense, GRU, GRU, dense: the passes of an update share launches (stacked_train_critics), the gradients are stored instead of added onto what the last
+    update left, two optimisers share a launch. Three loop steps, the gradient tensors filled with other values before each."""
+    print("case", case, flush=True)
+    S, B, OBS, ACT = case[:4]
+    rng = np.random.default_rng(S + B)
+    _, agents = stacked_agents(rng, (oracle, rocm), S, B, OBS, ACT, *case[4:])
+    T = S + 1 if case[6] else S
+    for i in range(3):
+        data = synthetic_sequence_batch(rng, S, B, OBS + ACT)
+        nc, na = rng.standard_normal((T, B, ACT)).astype(np.float32), rng.standard_normal((S, B, ACT)).astype(np.float32)
+        copy_agent(agents[0], agents[1])
+        for a in agents:
+            for net in (a.actor, *a.critics):
+                stale = np.zeros(net.grads.shape, np.float32)      # the initial hidden states have no gradient: whatever stands there is the optimiser's
+                stale[:net.specs[0][1] * net.specs[0][2]] = 3.0
+                net.grads.upload(stale)
+            a.log_alpha.upload(np.where(np.arange(4) == 1, 5.0, a.log_alpha.numpy()))
+            a.set_batch(data); a.train(nc, na)
+        # (the tolerance of the larger shapes above: fp32 sums over the steps in another order)
+        compare_agents(agents[1], agents[0], (case, i), tol=2e-5)
+
+
+@pytest.mark.parametrize("case", STACKED_AGENTS)
+def test_both_critics_of_recurrent_approximators_in_one_call_leave_the_bits_of_the_two_calls(rocm, case):
+    S, B, OBS, ACT = case[:4]
+    rng = np.random.default_rng(S * 3 + B)
+    params, agents = stacked_agents(rng, (rocm, rocm), S, B, OBS, ACT, *case[4:], spread=0.9)
+    T = S + 1 if case[6] else S
+    for i in range(3):
+        data = synthetic_sequence_batch(rng, S, B, OBS + ACT)
+        nc, na = rng.standard_normal((T, B, ACT)).astype(np.float32), rng.standard_normal((S, B, ACT)).astype(np.float32)
+        for a, together in zip(agents, (False, True)):
+            a.set_batch(data); a.train(nc, na, both_critics_in_one_call=together)
+        assert np.array_equal(agents[0].parameters(), agents[1].parameters()) and agents[0].ages() == agents[1].ages(), (case, i)
+        for key in ("target", "d_output", "next_q0", "next_q1", "next_lp", "nsavi"):
+            assert np.array_equal(agents[0].buf[key].numpy(), agents[1].buf[key].numpy()), (case, i, key)
+    assert np.abs(agents[1].parameters() - params).max() > 1e-4
 
 
 @pytest.mark.parametrize("n_layers", [3, 5])

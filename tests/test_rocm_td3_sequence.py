@@ -13,7 +13,7 @@ from test_rocm_sac_sequence import synthetic_sequence_batch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("case", [(6, 16, 3, 1, 16, 1, True), (20, 64, 5, 2, 32, 2, True), (10, 100, 3, 1, 64, 1, False), (100, 100, 3, 1, 16, 2, True)])
+@pytest.mark.parametrize("case", [(6, 16, 3, 1, 16, 1, True), (20, 64, 5, 2, 32, 2, True), (10, 100, 3, 1, 64, 1, False), (100, 100, 3, 1, 16, 2, True), (50, 20, 5, 2, 16, 3, True), (7, 33, 3, 1, 32, 3, False)])
 def test_td3_sequence_updates_match_checker(oracle, rocm, case):
     """Three training steps (critics, critic targets, actor, actor target) from identical state; the device agent is re-synchronised to the checker's
     parameters before each step. Shapes: the reference's recurrent TD3 approximators (GRU, GRU[, dense], dense), also with an input dense layer."""
@@ -21,6 +21,8 @@ def test_td3_sequence_updates_match_checker(oracle, rocm, case):
     S, B, OBS, ACT, H, variant, include_first = case
     rng = np.random.default_rng(S * B + H)
     body = [(1, None, H, "identity"), (1, H, H, "identity")] + ([(0, H, H, "relu")] if variant == 2 else [])
+    if variant == 3:        # dense, GRU, GRU, dense: the form whose passes are one launch each
+        body = [(0, None, H, "relu"), (1, H, H, "identity"), (1, H, H, "identity")]
     nets = []
     for in_dim, out_dim in ((OBS, ACT), (OBS + ACT, 1)):
         specs = [(k, in_dim if i is None else i, o, a) for k, i, o, a in body] + [(0, H, out_dim, "identity")]
