@@ -1,5 +1,6 @@
 """Workgroup barriers that order LDS traffic (csrc/common.h, rlt_lds_barrier): no path may reach one with LDS operations of the wavefront outstanding. The compiler has been
 seen to drop the fence's wait where a barrier opens a loop, so this reads the device assembly of kernels with such loops, built here, along its control flow."""
+import concurrent.futures
 import os
 import re
 import subprocess
@@ -58,10 +59,30 @@ def test_the_check_sees_a_wait_that_the_way_round_a_loop_lacks():
     assert unwaited_barriers(loop % "") == (["_Zk"], 1) and unwaited_barriers(loop % "\ts_waitcnt lgkmcnt(0)\n") == ([], 1)
 
 
-@pytest.mark.parametrize("source", ["gru.hip", "seq_stack.hip", "batch_gradient.hip"])
-def test_barriers_wait_for_lds(tmp_path, source):
-    out = tmp_path / "device.s"
-    subprocess.run([os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"), "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fno-gpu-rdc", "-Xclang", "-target-feature", "-Xclang",
-                    "-packed-fp32-ops", "--cuda-device-only", "-S", os.path.join(ROOT, "rl-tools_amd", "csrc", source), "-o", str(out)], check=True, capture_output=True)
-    bad, barriers = unwaited_barriers(out.read_text())
+CSRC = os.path.join(ROOT, "rl-tools_amd", "csrc")
+SOURCES = sorted(f for f in os.listdir(CSRC) if f.endswith(".hip") and "rlt_lds_barrier" in open(os.path.join(CSRC, f)).read())
+
+
+@pytest.fixture(scope="module")
+def assemblies(tmp_path_factory):
+    """the device assembly of every source with such a barrier, compiled side by side"""
+    folder = tmp_path_factory.mktemp("assembly")
+
+    def assemble(source):
+        out = folder / (source + ".s")
+        subprocess.run([os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"), "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fno-gpu-rdc", "-Xclang", "-target-feature", "-Xclang",
+                        "-packed-fp32-ops", "--cuda-device-only", "-S", os.path.join(CSRC, source), "-o", str(out)], check=True, capture_output=True)
+        return out.read_text()
+
+    with concurrent.futures.ThreadPoolExecutor(max_workers=6) as pool:
+        return dict(zip(SOURCES, pool.map(assemble, SOURCES)))
+
+
+def test_every_kernel_with_such_a_barrier_is_looked_at():
+    assert {"gru.hip", "seq_stack.hip", "sac_wide.hip", "mlp_fused.hip", "mlp_small.hip", "mlp_row.hip", "gemm.hip"} <= set(SOURCES)
+
+
+@pytest.mark.parametrize("source", SOURCES)
+def test_barriers_wait_for_lds(assemblies, source):
+    bad, barriers = unwaited_barriers(assemblies[source])
     assert barriers and not bad
