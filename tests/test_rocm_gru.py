@@ -115,6 +115,16 @@ def test_gru_weight_gradients_over_a_long_batch(oracle, rocm):
         assert rel_err(whole[k][:, 256:512], parts[1][k]) <= 2e-6, k
 
 
+@pytest.mark.parametrize("hidden", [16, 32, 64])
+@pytest.mark.parametrize("steps,batch", [(1, 9), (3, 2), (62, 5), (63, 3), (64, 6), (65, 1), (127, 7), (130, 5)])
+def test_gru_at_the_edges_of_the_blocks_of_steps(oracle, rocm, steps, batch, hidden):
+    """Reset flags are read for 63 or 64 steps at once, saved values requested up to four steps ahead: sequences that end around both. The tolerance is that of the long sequences."""
+    print("case", steps, batch, hidden, flush=True)
+    want, got = run_pair(oracle, rocm, steps, batch, 5, hidden, steps + hidden, True)
+    for k in KEYS:
+        assert rel_err(got[k], want[k]) <= 2e-5, (k, rel_err(got[k], want[k]))
+
+
 @pytest.mark.parametrize("case", [(32, 64, 34, 64), (33, 63, 160, 64), (16, 129, 66, 33), (64, 256, 64, 50), (64, 257, 146, 64), (64, 256, 36, 16)])
 def test_gru_at_the_edges_of_the_kernels_that_keep_a_layer_in_registers(oracle, rocm, case):
     """Input gates with their weights in registers (2,048 rows and more, 97 to 192 gates, even inputs from 34 to 160) and weight gradients in one workgroup's accumulators (16,384 rows and
