@@ -5,7 +5,7 @@
 // y/out/pre (each optional) = act(x W^T + bias); pre/out are packed [batch x out_dim], y has leading dimension ldy
 int rlt_gemm_forward(rlt_rocm_device* device, const float* x, int ldx, const float* W, const float* bias, int act,
                      float* pre, float* out, float* y, int ldy, int batch, int in_dim, int out_dim);
-// y = x W^T + bias for a narrow layer (output 97 ... 192, even input 34 ... 160) over 2,048 rows or more, weights in registers: another summation order than rlt_gemm_forward's.
+// y = x W^T + bias for a narrow layer (output 129 ... 192, even input 34 ... 160) over 2,048 rows or more, weights in registers: another summation order than rlt_gemm_forward's.
 // RLT_E_UNSUPPORTED: the caller takes that one.
 int rlt_gemm_rows_forward(rlt_rocm_device* device, const float* x, int ldx, const float* W, const float* bias, float* y, int ldy, int batch, int in_dim, int out_dim);
 // d_in = d_pre W, optionally multiplied elementwise by act'(.) of the layer below: dact_pre (packed [batch x in_dim]) holds that

@@ -412,8 +412,10 @@ __global__ __launch_bounds__(WIDE_THREADS) void wgrad_wide_kernel(WideArgs a) {
 // (w = wavefront % 4, 3 tiles of v_mfma_f32_16x16x4_f32 by 4 NJ k-steps, 12 NJ registers), and only rows pass through LDS: 32 at a time (wavefront / 4 selects sixteen of them),
 // double buffered, the next 32 requested before the current ones are multiplied, one barrier each. Lane (r, kk) supplies the four k from 16 j + 4 kk of every sixteen, for both operands.
 // Measured, K = 146, N = 192 (tiled kernel -> this one): 1,024 rows 9.0 -> 10.3 us, 2,048 12.1 -> 10.5, 4,096 13.1 -> 11.2, 8,192 16.0 -> 12.5, 16,384 28.6 -> 17.8, 65,536 60 -> 46 us; K = 64:
-// 1,024 rows 5.1 -> 5.9 us, 2,048 7.9 -> 6.1, 65,536 35.4 -> 25.4 us: the line lies at 2,048 rows. Bound: the matrix pipe at long batches (27 us of 46, K padded to 160), the trip to memory
-// for the weights at short ones.
+// 1,024 rows 5.1 -> 5.9 us, 2,048 7.9 -> 6.1, 65,536 35.4 -> 25.4 us: the line lies at 2,048 rows. K is padded to 64, 96, 128 or 160 (with 160 for everything beyond 64, a layer of 66 inputs
+// was slower than on the tiled kernel: forward pass of 4,096 x 66 -> 192 and its recurrence 20.1 us there, 22.3 padded to 160, 18.9 padded to 96). N: all 192 columns are multiplied whatever
+// N is; at N = 99 the tiled kernel wins at 2,048 rows (17.3 against 19.4 us with 100 inputs) and at 65,536 (181 against 184 with 34), at 144 this one or neither does: the line lies at 128.
+// Bound: the matrix pipe at long batches (27 us of 46, K padded to 160), the trip to memory for the weights at short ones.
 struct RowsForward { const float* X; int ldx; const float* W; const float* bias; float* Y; int ldy; int M, N, K; };
 constexpr int RF_THREADS = 512, RF_ROWS = 32, ROWS_FORWARD_MIN_BATCH = 2048;
 template <int NJ>
@@ -709,11 +711,13 @@ int rlt_gemm_forward(rlt_rocm_device* device, const float* x, int ldx, const flo
 }
 
 int rlt_gemm_rows_forward(rlt_rocm_device* device, const float* x, int ldx, const float* W, const float* bias, float* y, int ldy, int batch, int in_dim, int out_dim) {
-    if (out_dim <= 96 || out_dim > WIDE_M || in_dim <= 32 || in_dim > 160 || in_dim % 2 != 0 || ldx % 2 != 0 || batch < ROWS_FORWARD_MIN_BATCH ||
+    if (out_dim <= 128 || out_dim > WIDE_M || in_dim <= 32 || in_dim > 160 || in_dim % 2 != 0 || ldx % 2 != 0 || batch < ROWS_FORWARD_MIN_BATCH ||
         ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(W)) & 7u) != 0) return RLT_E_UNSUPPORTED;
     const RowsForward a = {x, ldx, W, bias, y, ldy, batch, out_dim, in_dim};
     const int blocks = rlt_div_up(batch, RF_ROWS), grid = blocks < device->compute_units ? blocks : device->compute_units;
     if (in_dim <= 64) hipLaunchKernelGGL(rows_forward_kernel<4>, dim3(grid), dim3(RF_THREADS), 0, device->stream, a);
+    else if (in_dim <= 96) hipLaunchKernelGGL(rows_forward_kernel<6>, dim3(grid), dim3(RF_THREADS), 0, device->stream, a);
+    else if (in_dim <= 128) hipLaunchKernelGGL(rows_forward_kernel<8>, dim3(grid), dim3(RF_THREADS), 0, device->stream, a);
     else hipLaunchKernelGGL(rows_forward_kernel<10>, dim3(grid), dim3(RF_THREADS), 0, device->stream, a);
     return rlt_launch_status(device);
 }
@@ -777,8 +781,11 @@ int rlt_gemm_wgrad(rlt_rocm_device* device, const float* d_pre, int ldd, const f
     p.A = d_pre; p.lda = ldd; p.B = x; p.ldb = ldx; p.M = out_dim; p.N = in_dim; p.K = batch;
     p.vecA = vector_width(d_pre, ldd); p.vecB = vector_width(x, ldx);
     p.dW = dW; p.dbias = dbias;
-    // narrow layer, long batch: one workgroup per share of the batch holds the whole gradient (wgrad_wide_kernel)
-    if (narrow_long && !static_scratch && out_dim <= WIDE_M && out_dim % 4 == 0 && in_dim > 32 && in_dim <= 160 && in_dim % 2 == 0 && batch >= 16384 && ldd % 4 == 0 && ldx % 2 == 0 &&
+    // Narrow layer, long batch: one workgroup per share of the batch holds the whole gradient (wgrad_wide_kernel), all 192 rows of it whatever out_dim is. Inputs of 34 to 64 are
+    // better off on the tiled kernel below where that is less than 129 rows or the batch shorter than 65,536 (backward pass of a GRU of 64 inputs, tiled -> this kernel: 48 rows
+    // of dW at 16,384 41.6 -> 44.3 us, at 65,536 75.0 -> 82.3; 96 rows 50.1 -> 52.3, 97.1 -> 101.3; 120 rows 86.9 -> 89.5, 220.6 -> 231.8; 144 rows 95.1 -> 97.1, 253.3 -> 249.8;
+    // 192 rows 57.9 -> 62.2 at 16,384, 96.7 -> 97.7 at 49,152, 122.6 -> 115.8 at 65,536).
+    if (narrow_long && !static_scratch && out_dim <= WIDE_M && out_dim % 4 == 0 && (in_dim > 64 || (in_dim > 32 && out_dim > 128 && batch >= 65536)) && in_dim <= 160 && in_dim % 2 == 0 && batch >= 16384 && ldd % 4 == 0 && ldx % 2 == 0 &&
         (reinterpret_cast<uintptr_t>(d_pre) & 15u) == 0 && (reinterpret_cast<uintptr_t>(x) & 7u) == 0) {
         const int groups = device->compute_units < batch / 64 ? device->compute_units : batch / 64;
         const int rows_per_group = rlt_div_up(rlt_div_up(batch, groups), WIDE_KT) * WIDE_KT, used = rlt_div_up(batch, rows_per_group);

@@ -125,10 +125,12 @@ def test_gru_at_the_edges_of_the_blocks_of_steps(oracle, rocm, steps, batch, hid
         assert rel_err(got[k], want[k]) <= 2e-5, (k, rel_err(got[k], want[k]))
 
 
-@pytest.mark.parametrize("case", [(32, 64, 34, 64), (33, 63, 160, 64), (16, 129, 66, 33), (64, 256, 64, 50), (64, 257, 146, 64), (64, 256, 36, 16)])
+@pytest.mark.parametrize("case", [(32, 64, 34, 64), (33, 63, 160, 64), (16, 129, 66, 33), (64, 256, 64, 50), (64, 257, 146, 64), (64, 256, 36, 16),
+                                  (32, 64, 96, 64), (33, 63, 98, 43), (16, 129, 128, 43), (32, 65, 130, 64), (64, 1024, 34, 44)])
 def test_gru_at_the_edges_of_the_kernels_that_keep_a_layer_in_registers(oracle, rocm, case):
-    """Input gates with their weights in registers (2,048 rows and more, 97 to 192 gates, even inputs from 34 to 160) and weight gradients in one workgroup's accumulators (16,384 rows and
-    more, even widths from 34 to 160): the smallest and largest inputs, ragged last rows, gates and widths that fill no tile. Tolerance as for the long batch above."""
+    """Input gates with their weights in registers (2,048 rows and more, 129 to 192 gates, even inputs from 34 to 160, padded to 64, 96, 128 or 160) and weight gradients in one workgroup's
+    accumulators (16,384 rows and more, even widths from 66 to 160; from 34 on for 129 gates and 65,536 rows): the smallest and largest inputs, ragged last rows, gates and widths that fill
+    no tile. Tolerance as for the long batch above."""
     print("case", case, flush=True)
     S, B, I, H = case
     want, got = run_pair(oracle, rocm, S, B, I, H, 35, True)
