@@ -86,6 +86,17 @@ int rlt_zero_tensors(rlt_rocm_device* device, float* const* begins, const size_t
     return flush();
 }
 
+// Three-layer networks of hidden widths beyond 64 over a few thousand rows at most, evaluate() and forward() the same way (the same bits): a row or a few per workgroup where that
+// is the faster way, sixteen-row tiles with the weights read from a copy in consumption order else. Networks that the tiles do not take (hidden layers without an activation
+// function, or with two different ones) go back to the first way up to its last row.
+static int few_thousand_rows(rlt_rocm_device* device, const rlt_dense_layer* layers, int n, const float* x, int ldx, float* y, int ldy, int batch, bool keep) {
+    const bool first = rlt_mlp_row_first(device, layers, batch);
+    int rc = first ? rlt_mlp_row_forward(device, layers, n, x, ldx, y, ldy, batch, keep) : RLT_E_UNSUPPORTED;
+    if (rc == RLT_E_UNSUPPORTED) rc = rlt_mlp_wide_forward(device, layers, n, x, ldx, y, ldy, batch, keep);
+    if (rc == RLT_E_UNSUPPORTED && !first) rc = rlt_mlp_row_forward(device, layers, n, x, ldx, y, ldy, batch, keep);
+    return rc;
+}
+
 extern "C" {
 
 int rlt_rocm_dense_evaluate(rlt_rocm_device* device, const rlt_dense_layer* L, const float* x, int ldx, float* y, int ldy, int batch) {
@@ -137,8 +148,7 @@ int rlt_rocm_mlp_evaluate(rlt_rocm_device* device, const rlt_dense_layer* layers
     const size_t buf = align_up((size_t)batch * max_dim(layers, n) * sizeof(float));
     RLT_REQUIRE(n == 1 || (workspace && workspace_bytes >= 2 * buf));
     if (n == 3 && batch <= RLT_MLP_WIDE_MAX_BATCH && layers[0].out_dim > 64 && single_pass_enabled() && wide_enabled()) {      // as forward(): the same kernel, the same bits
-        int rc = batch <= RLT_MLP_ROW_MAX_BATCH ? rlt_mlp_row_forward(device, layers, n, x, ldx, y, ldy, batch, false) : RLT_E_UNSUPPORTED;
-        if (rc == RLT_E_UNSUPPORTED) rc = rlt_mlp_wide_forward(device, layers, n, x, ldx, y, ldy, batch, false);
+        const int rc = few_thousand_rows(device, layers, n, x, ldx, y, ldy, batch, false);
         if (rc != RLT_E_UNSUPPORTED) return rc;
     }
     if (n > 1 && batch <= RLT_MLP_ROWS_MAX_BATCH && rows_enabled()) {
@@ -162,10 +172,8 @@ int rlt_rocm_mlp_forward(rlt_rocm_device* device, const rlt_dense_layer* layers,
     RLT_REQUIRE(chain_ok(layers, n) && x && batch > 0 && ldx >= layers[0].in_dim);
     for (int l = 0; l < n; l++) RLT_REQUIRE(layers[l].pre_activations && layers[l].output);
     if (n == 3 && batch <= RLT_MLP_WIDE_MAX_BATCH && layers[0].out_dim > 64 && single_pass_enabled() && wide_enabled()) {
-        // hidden widths beyond 64 over a few thousand rows at most: sixteen-row tiles with the second layer's weights read from a copy in consumption order
         // (narrower networks' weights are few enough for the few-rows kernel below to read them as they lie)
-        int rc = batch <= RLT_MLP_ROW_MAX_BATCH ? rlt_mlp_row_forward(device, layers, n, x, ldx, nullptr, 0, batch, true) : RLT_E_UNSUPPORTED;
-        if (rc == RLT_E_UNSUPPORTED) rc = rlt_mlp_wide_forward(device, layers, n, x, ldx, nullptr, 0, batch, true);
+        const int rc = few_thousand_rows(device, layers, n, x, ldx, nullptr, 0, batch, true);
         if (rc != RLT_E_UNSUPPORTED) return rc;
     }
     if (n > 1 && batch <= RLT_MLP_ROWS_MAX_BATCH && batch < FUSED_MIN_BATCH && rows_enabled()) {

@@ -149,8 +149,8 @@ int rlt_mlp_row_forward(rlt_rocm_device* device, const rlt_dense_layer* L, int n
     }
     a.net.in = L[0].in_dim; a.net.hid = hid; a.net.n_out = L[2].out_dim;
     a.x = x; a.ldx = ldx; a.y = y; a.ldy = ldy; a.batch = batch;
-    // Workgroups are one to a compute unit. Rows per workgroup 1, 2, 4, 8: 5.7, 6.7, 8.8, 13.0 us per call of 17-256-256-6 (13.6 to 14.9 on sixteen-row tiles with the weight copies before them, which
-    // stay at 15.0 up to 4,096 rows: the line lies at 2,048).
+    // Workgroups are one to a compute unit. Rows per workgroup 1, 2, 4, 8, calls in a row in a graph: 6.7, 7.9, 10.3, 14.8 us per call of 17-256-256-6, 5.6, 6.4, 8.1, 11.4 us at width 128 (15.1 to 15.5 and
+    // 11.2 to 11.5 on sixteen-row tiles with the weight copies before them; where the line lies: rlt_mlp_row_first).
     const int units = device->compute_units > 0 ? device->compute_units : 256;
     if (batch <= units) launch<1>(device, a); else if (batch <= 2 * units) launch<2>(device, a); else if (batch <= 4 * units) launch<4>(device, a); else launch<8>(device, a);
     return rlt_launch_status(device);

@@ -22,6 +22,11 @@ CASES = [
     (513, 16, 252, 3, "relu", "tanh"),         # four rows per workgroup
     (1025, 17, 256, 6, "tanh", "identity"),    # eight
     (2048, 3, 96, 2, "identity", "identity"),  # the largest
+    (1024, 40, 200, 2, "relu", "identity"),    # the last batch of four rows for every network: from here on sixteen-row tiles ...
+    (1025, 33, 256, 6, "relu", "tanh"),
+    (2000, 17, 252, 6, "tanh", "identity"),
+    (2047, 32, 256, 4, "relu", "identity"),    # ... but for eight rows of the widest with few inputs
+    (1300, 40, 256, 2, "identity", "tanh"),    # ... and for networks that the tiles do not take
 ]
 
 
