@@ -578,6 +578,7 @@ size_t rlt_rocm_sac_sequence_workspace_bytes(const rlt_sac_sequence_agent* A) {
 // share one. The trained critics' loss gradients and backward passes follow, then their optimisers in one launch.
 static bool sequence_agent_stacked(const rlt_sac_sequence_agent* A) {
     const int T = A->batch.sequence_length + 1;
+    if (!rlt_seq_stack_faster(RLT_STACK_UPDATE, A->batch.sequence_length, A->batch.batch)) return false;
     if (!rlt_seq_stack_supported(A->actor, A->n_actor_layers, T)) return false;
     for (int k = 0; k < 2; k++)
         if (!rlt_seq_stack_supported(A->critics[k], A->n_critic_layers, T) || !rlt_seq_stack_supported(A->critics_target[k], A->n_critic_layers, T)) return false;

@@ -111,7 +111,7 @@ int rlt_rocm_seq_forward(rlt_rocm_device* device, const rlt_seq_layer* layers, i
     RLT_REQUIRE(layers_ok(layers, n) && x && steps > 0 && batch > 0 && ldx >= layer_in(layers[0]));
     Workspace W;
     RLT_REQUIRE(carve(layers, n, steps, batch, workspace, workspace_bytes, &W));
-    if (rlt_seq_stack_supported(layers, n, steps)) {
+    if (rlt_seq_stack_faster(RLT_STACK_PASS, steps, batch) && rlt_seq_stack_supported(layers, n, steps)) {
         const rlt_stack_forward pass = {layers, x, ldx, reset, steps, batch, nullptr};
         return rlt_seq_stack_forward(device, &pass, 1);
     }
@@ -138,7 +138,7 @@ int rlt_rocm_seq_backward(rlt_rocm_device* device, const rlt_seq_layer* layers, 
     const int rows = steps * batch;
     // backward and backward_full hand the mode to every layer; backward_input hands it on only when the model has a single layer
     const uint8_t* reset_here = (want_w || reset_in_backward_input || n == 1) ? reset : nullptr;
-    if (rlt_seq_stack_supported(layers, n, steps) && (want_w || d_input)) {
+    if (rlt_seq_stack_faster(want_w ? RLT_STACK_WEIGHT_GRADIENTS : RLT_STACK_PASS, steps, batch) && rlt_seq_stack_supported(layers, n, steps) && (want_w || d_input)) {
         const rlt_stack_backward pass = {layers, x, ldx, d_output, d_input, reset_here, steps, batch, want_w, 0, (void*)(((uintptr_t)workspace + 255) & ~(uintptr_t)255)};
         return rlt_seq_stack_backward(device, &pass, 1);
     }

@@ -100,7 +100,10 @@ def with_initial_states(rng, specs, params):
 # dense, GRU, GRU, dense: all layers of a pass in one launch (seq_stack.hip). (steps, batch, in, hidden, out, fast_tanh, hidden activation): the narrowest and widest inputs and
 # outputs, one step, steps that fill neither the pairs nor the groups of six that the loops are unrolled to, exact and rational gates
 STACK_CASES = [(7, 3, 1, 16, 1, True, "relu"), (13, 5, 16, 16, 16, False, "tanh"), (1, 2, 4, 16, 2, False, "relu"), (6, 9, 1, 32, 16, False, "sigmoid"), (11, 4, 16, 32, 1, True, "relu"),
-               (1, 7, 3, 32, 3, True, "fast_tanh"), (2, 1, 5, 32, 2, False, "identity"), (100, 33, 9, 16, 5, True, "relu"), (65, 20, 13, 32, 7, False, "tanh")]
+               (1, 7, 3, 32, 3, True, "fast_tanh"), (2, 1, 5, 32, 2, False, "identity"), (100, 33, 9, 16, 5, True, "relu"), (65, 20, 13, 32, 7, False, "tanh"),
+               # several hundred rows and the lines up to which a pass is one launch: the last with it, the first without (whose backward pass with weight gradients still is)
+               (5, 700, 4, 32, 1, True, "relu"), (2, 2048, 3, 16, 2, True, "relu"), (2, 2049, 3, 16, 2, True, "relu"), (17, 1024, 4, 32, 1, True, "relu"), (17, 1025, 4, 32, 1, True, "relu"),
+               (1, 16385, 2, 16, 1, True, "relu")]
 
 
 @pytest.mark.parametrize("with_reset", [False, True])
@@ -125,7 +128,8 @@ def stacked_agents(rng, backends, S, B, OBS, ACT, actor_hidden, critic_hidden, f
 
 
 # (steps, batch, observations, actions, actor's width, critics' width, first step in the targets)
-STACKED_AGENTS = [(1, 3, 3, 1, 16, 32, True), (7, 13, 5, 2, 16, 32, False), (13, 5, 12, 4, 32, 16, True), (31, 64, 3, 1, 16, 16, True), (100, 40, 8, 8, 32, 32, False)]
+STACKED_AGENTS = [(1, 3, 3, 1, 16, 32, True), (7, 13, 5, 2, 16, 32, False), (13, 5, 12, 4, 32, 16, True), (31, 64, 3, 1, 16, 16, True), (100, 40, 8, 8, 32, 32, False),
+                  (2, 4800, 3, 1, 16, 16, True), (2, 4801, 3, 1, 16, 16, True)]      # the last batch whose passes share launches, and the first that does not
 
 
 @pytest.mark.parametrize("case", STACKED_AGENTS)
