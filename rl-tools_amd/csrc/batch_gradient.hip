@@ -76,11 +76,11 @@ __global__ __launch_bounds__(THREADS) void batch_gradient_kernel(GradientLaunch 
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), B = K.batch;
     // which tile of which layer's gradient: layer 2 first (the most tiles), then 1, then 3
     const int MT = (N.hid + TM - 1) / TM, N2 = (N.hid + TN - 1) / TN, N1 = (N.in + TN - 1) / TN;
-    int t = block - (y ? K.blocks0 : 0), segment, tiles, rows, cols, lda, ldb;
+    int t = block - (y ? K.blocks0 : 0), segment, tiles, rows, cols, lda, ldb, before = 0;      // before: elements of the segments in front of this one
     const float *a, *b;
-    if (t < MT * N2) { segment = 2; tiles = N2; a = N.d2; lda = N.hid; rows = N.hid; b = N.h1; ldb = N.hid; cols = N.hid; }
+    if (t < MT * N2) { segment = 2; before = N.hid * N.in + N.hid; tiles = N2; a = N.d2; lda = N.hid; rows = N.hid; b = N.h1; ldb = N.hid; cols = N.hid; }
     else if ((t -= MT * N2) < MT * N1) { segment = 0; tiles = N1; a = N.d1; lda = N.hid; rows = N.hid; b = N.x; ldb = N.ldx; cols = N.in; }
-    else { t -= MT * N1; segment = 4; tiles = N2; a = N.d3; lda = N.ld3; rows = N.out; b = N.h2; ldb = N.hid; cols = N.hid; }
+    else { t -= MT * N1; segment = 4; before = N.hid * N.in + N.hid + N.hid * N.hid + N.hid; tiles = N2; a = N.d3; lda = N.ld3; rows = N.out; b = N.h2; ldb = N.hid; cols = N.hid; }
     const int mt = t / tiles, nt = t - mt * tiles;
     // this wavefront's rows of the batch
     const int shares = SPLIT ? WAVES * K.splits : WAVES, per = ((B + shares - 1) / shares + 3) & ~3, k0 = (WAVES * split + wave) * per, k1 = min(B, k0 + per);
@@ -101,8 +101,7 @@ __global__ __launch_bounds__(THREADS) void batch_gradient_kernel(GradientLaunch 
     tile_product<TM / 16>(a, lda, rows, TM * mt, b, ldb, cols, TN * nt, B, k0, k1, r, g, c, bias);
     place_parts(P, wave, r, g, c, bias);
     rlt_lds_barrier();
-    size_t first = SPLIT ? (size_t)split * K.total + (y ? K.total0 : 0) : 0;      // where this segment's sums of this split lie
-    if (SPLIT) for (int k = 0; k < segment; k++) first += segment_size(N, k);
+    const size_t first = SPLIT ? (size_t)split * K.total + (y ? K.total0 : 0) + before : 0;      // where this segment's sums of this split lie
 #pragma unroll
     for (int u = 0; u < PER_THREAD; u++) {
         const int e = threadIdx.x + u * THREADS, em = e / TN, en = e % TN;
@@ -152,34 +151,44 @@ int blocks_of(const rlt_gradient_net& N, int TM) {
     return MT * N2 + MT * rlt_div_up(N.in, TN) + rlt_div_up(N.out, TM) * N2;
 }
 int elements_of(const rlt_gradient_net& N) { int n = 0; for (int k = 0; k < 6; k++) n += segment_size(N, k); return n; }
-int splits_for(int batch) { int s = 1; while (s < MAX_SPLITS && batch > s * SPLIT_ROWS) s *= 2; return s; }
+// Groups of workgroups that the batch is shared out to: one per SPLIT_ROWS rows; and where there are several, and a launch behind this one adds their sums up anyway, as many
+// as give every compute unit a workgroup (a narrow network's gradients are few tiles: 15 at width 65)
+int splits_for(const rlt_gradient_net* nets, int n_nets, int batch) {
+    int s = 1, tiles = 0;
+    for (int k = 0; k < n_nets; k++) tiles += blocks_of(nets[k], 32);
+    while (s < MAX_SPLITS && batch > s * SPLIT_ROWS) s *= 2;
+    while (s > 1 && s < MAX_SPLITS && tiles * s < 256) s *= 2;
+    return s;
+}
 }  // namespace
 
 size_t rlt_batch_gradients_partial_floats(const rlt_gradient_net* nets, int n_nets, int batch) {
-    if (splits_for(batch) == 1) return 0;
+    const int splits = splits_for(nets, n_nets, batch);
+    if (splits == 1) return 0;
     size_t n = 0;
     for (int k = 0; k < n_nets; k++) n += elements_of(nets[k]);
-    return n * splits_for(batch);
+    return n * splits;
 }
 
 int rlt_batch_gradients(rlt_rocm_device* device, const rlt_gradient_net* nets, int n_nets, int batch, float polyak, const rlt_gradient_scalar* scalar, float* partial,
                         const rlt_gradient_guard* guard) {
     RLT_REQUIRE(nets && n_nets >= 1 && n_nets <= 2 && batch > 0 && (!scalar || scalar->n <= 128) && (n_nets == 1 || nets[0].step == nets[1].step));
     GradientLaunch K = {};
+    K.splits = splits_for(nets, n_nets, batch);
     int blocks = 0;
     for (int k = 0; k < n_nets; k++) {
-        K.net[k] = nets[k]; blocks += blocks_of(nets[k], splits_for(batch) > 1 ? 32 : 16); K.total += elements_of(nets[k]);
+        K.net[k] = nets[k]; blocks += blocks_of(nets[k], K.splits > 1 ? 32 : 16); K.total += elements_of(nets[k]);
         if (k == 0) { K.blocks0 = blocks; K.total0 = K.total; }
     }
-    K.batch = batch; K.polyak = polyak; K.splits = splits_for(batch); K.partial = partial;
+    K.batch = batch; K.polyak = polyak; K.partial = partial;
     if (scalar) { K.scalar = *scalar; K.has_scalar = 1; }
     if (guard) K.guard = *guard;
     if (K.splits == 1) {
-        hipLaunchKernelGGL(batch_gradient_kernel<false>, dim3(blocks), dim3(THREADS), 0, device->stream, K);
+        hipLaunchKernelGGL((batch_gradient_kernel<false>), dim3(blocks), dim3(THREADS), 0, device->stream, K);
         return rlt_launch_status(device);
     }
     RLT_REQUIRE(partial);
-    hipLaunchKernelGGL(batch_gradient_kernel<true>, dim3(blocks * K.splits), dim3(THREADS), 0, device->stream, K);
+    hipLaunchKernelGGL((batch_gradient_kernel<true>), dim3(blocks * K.splits), dim3(THREADS), 0, device->stream, K);
     const int rc = rlt_launch_status(device);
     if (rc) return rc;
     hipLaunchKernelGGL(finish_kernel, dim3(rlt_div_up(K.total, 256)), dim3(256), 0, device->stream, K);
