@@ -79,11 +79,21 @@ template <int ACT_H> __device__ __forceinline__ float dact_hidden(float o, int f
 // (forward copies of the first and second layers) or W[16 j + 4 g ... + 3][16 w + c] (backward copy of the second), zero beyond the layer's shape, and a wavefront's
 // load is 1 KB of consecutive addresses. Straight from W a lane's 16 bytes lie a row apart from its neighbour's: 64 lines per load, which the compute unit's address
 // pipeline takes 64 cycles for; first layers whose rows are no multiple of 16 bytes (17 or 35 inputs) take four such loads per chunk, 5 us at the start of a launch.
-template <int JN>
-__device__ __forceinline__ void load_swizzled(const float* __restrict__ copy, int tiles, int wave, int lane, int j0, floatx4 (&b)[JN]) {      // tiles: chunks of the copy
-    const float* const mine = copy + ((size_t)wave * tiles * 64 + lane) * 4;
+// What a wavefront will not use (chunks beyond the width, everything where it has no units) is asked for at one address by all lanes, which costs the address pipeline a cycle or two
+// instead of sixteen: at width 65 eleven of sixteen wavefronts and eleven of sixteen chunks are such.
+// EVERY: where every wavefront has units there is nothing to leave out, and the selects cost more than they save (forward + backward of 256 units 36.2 us with them, 35.4 without).
+template <int JN, bool EVERY = false>
+__device__ __forceinline__ void load_swizzled(const float* __restrict__ copy, int tiles, bool on, int wave, int lane, int j0, floatx4 (&b)[JN]) {      // tiles: chunks of the copy; on: this wavefront has units
+    if (EVERY) {
+        const float* const mine = copy + ((size_t)wave * tiles * 64 + lane) * 4;
 #pragma unroll
-    for (int j = 0; j < JN; j++) b[j] = *reinterpret_cast<const floatx4*>(mine + (size_t)min(j0 + j, tiles - 1) * 256);      // chunks beyond the width are not used
+        for (int j = 0; j < JN; j++) b[j] = *reinterpret_cast<const floatx4*>(mine + (size_t)min(j0 + j, tiles - 1) * 256);
+        return;
+    }
+    const uint32_t mine = ((uint32_t)wave * tiles * 64 + lane) * 16;
+#pragma unroll
+    for (int j = 0; j < JN; j++)
+        b[j] = *reinterpret_cast<const floatx4*>(reinterpret_cast<const char*>(copy) + (on && j0 + j < tiles ? mine + (uint32_t)(j0 + j) * 1024 : 0));
 }
 // acc += in[rows][16 (j0 + j) + ...] * b[j], the workgroup's 16 rows against this lane's column
 template <int JN>
@@ -126,13 +136,14 @@ __device__ __forceinline__ void mask_w3(const WNet& N, int wave, int c, int g, f
 }
 // everything of network N that forward3 reads from memory, requested at once (few first-layer operands leave room for the whole second layer; otherwise its second
 // half is requested after the first layer has run)
-template <int NT1C>
+template <int NT1C, bool EVERY = false>
 __device__ __forceinline__ void load_operands(const WNet& N, int wave, int c, int g, Operands<NT1C>& W) {
     const int n = 16 * wave + c, tiles = (N.hid + 15) >> 4, lane = c + 16 * g;
-    load_swizzled<NT1C>(N.W1f, (N.in + 15) >> 4, wave, lane, 0, W.w1);
+    const bool on = wave < tiles;
+    load_swizzled<NT1C, EVERY>(N.W1f, (N.in + 15) >> 4, on, wave, lane, 0, W.w1);
     W.b1 = N.b1[min(n, N.hid - 1)]; W.b2 = N.b2[min(n, N.hid - 1)];
-    load_swizzled<8>(N.W2f, tiles, wave, lane, 0, W.w2a);
-    if (NT1C <= FEW) load_swizzled<8>(N.W2f, tiles, wave, lane, 8, W.w2b);
+    load_swizzled<8, EVERY>(N.W2f, tiles, on, wave, lane, 0, W.w2a);
+    if (NT1C <= FEW) load_swizzled<8, EVERY>(N.W2f, tiles, on, wave, lane, 8, W.w2b);
     W.w3 = load_w3(N, wave, c, g);
 }
 
@@ -160,29 +171,29 @@ __device__ __forceinline__ void place_hidden(const WNet& N, const floatx4& acc, 
         }
     }
 }
-template <int ACT_H, int NT1C, bool PREFETCH, bool W1_READY, bool KEEP = false>
+template <int ACT_H, int NT1C, bool PREFETCH, bool W1_READY, bool KEEP = false, bool EVERY = false>
 __device__ __forceinline__ void forward3(const WNet& N, Operands<NT1C>& W, const WNet& next, lptr x, int xstride, lptr h1, lptr h2, lptr yp, int wave, int c, int g, const KeepArgs* keep = nullptr) {
     const int n = 16 * wave + c, tiles = (N.hid + 15) >> 4, lane = c + 16 * g, next_tiles = (next.hid + 15) >> 4;
-    const bool on = wave < tiles;
+    const bool on = wave < tiles, next_on = wave < next_tiles;
     const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
-    if (!W1_READY) load_swizzled<NT1C>(N.W1f, (N.in + 15) >> 4, wave, lane, 0, W.w1);
+    if (!W1_READY) load_swizzled<NT1C, EVERY>(N.W1f, (N.in + 15) >> 4, on, wave, lane, 0, W.w1);
     if (on) {
         floatx4 a0 = zero4, a1 = zero4;
         chunks<NT1C>(a0, a1, x, xstride, c, g, 0, (N.in + 15) >> 4, W.w1);
         place_hidden<ACT_H, KEEP>(N, a0 + a1, W.b1, h1, n, g, keep, 0);
     }
-    if (NT1C > FEW) load_swizzled<8>(N.W2f, tiles, wave, lane, 8, W.w2b);
+    if (NT1C > FEW) load_swizzled<8, EVERY>(N.W2f, tiles, on, wave, lane, 8, W.w2b);
     if (PREFETCH) {
-        if (NT1C <= FEW) load_swizzled<NT1C>(next.W1f, (next.in + 15) >> 4, wave, lane, 0, W.w1);
+        if (NT1C <= FEW) load_swizzled<NT1C, EVERY>(next.W1f, (next.in + 15) >> 4, next_on, wave, lane, 0, W.w1);
         W.b1 = next.b1[min(n, next.hid - 1)];
     }
     rlt_lds_barrier();
     {
         floatx4 a0 = zero4, a1 = zero4;
         if (on) chunks<8>(a0, a1, h1, S, c, g, 0, tiles, W.w2a);
-        if (PREFETCH) load_swizzled<8>(next.W2f, next_tiles, wave, lane, 0, W.w2a);
+        if (PREFETCH) load_swizzled<8, EVERY>(next.W2f, next_tiles, next_on, wave, lane, 0, W.w2a);
         if (on) chunks<8>(a0, a1, h1, S, c, g, 8, tiles, W.w2b);
-        if (PREFETCH && NT1C <= FEW) load_swizzled<8>(next.W2f, next_tiles, wave, lane, 8, W.w2b);
+        if (PREFETCH && NT1C <= FEW) load_swizzled<8, EVERY>(next.W2f, next_tiles, next_on, wave, lane, 8, W.w2b);
         if (on) place_hidden<ACT_H, KEEP>(N, a0 + a1, W.b2, h2, n, g, keep, 1);
         if (PREFETCH) W.b2 = next.b2[min(n, next.hid - 1)];
     }
@@ -219,39 +230,57 @@ __device__ __forceinline__ floatx4 output_tile(lptr yp, int tiles, int c, int g)
 
 // column n of W3 for this lane's share of the reduction over the outputs, and the second layer's backward copy: the operands of a backward pass, requested ahead of it
 struct BackOperands { float w3[MAX_OUT / 4]; floatx4 w2[MAX_H / 16]; };
+template <bool EVERY = false>
 __device__ __forceinline__ void load_back_operands(const WNet& N, int wave, int c, int g, BackOperands& W) {
     const int n = 16 * wave + c, tiles = (N.hid + 15) >> 4;
 #pragma unroll
     for (int ks = 0; ks < MAX_OUT / 4; ks++) W.w3[ks] = N.W3[(size_t)min(4 * ks + g, N.out - 1) * N.hid + min(n, N.hid - 1)];
-    load_swizzled<MAX_H / 16>(N.W2b, tiles, wave, c + 16 * g, 0, W.w2);
+    load_swizzled<MAX_H / 16, EVERY>(N.W2b, tiles, wave < tiles, wave, c + 16 * g, 0, W.w2);
 }
-// this wavefront's tile of d_pre2 = (d_pre3 W3) f'(h2) into g2 (may be h2 itself)
+// this wavefront's tile of d_pre2 = (d_pre3 W3) f'(h2) into g2 (may be h2 itself); returns the lane's share of its unit's column sum
 template <int ACT_H>
-__device__ __forceinline__ void backward_layer3(const WNet& N, const BackOperands& W, lptr d3, lptr h2, lptr g2, int wave, int c, int g) {
+__device__ __forceinline__ float backward_layer3(const WNet& N, const BackOperands& W, lptr d3, lptr h2, lptr g2, int wave, int c, int g) {
     const int n = 16 * wave + c;
     const bool n_ok = n < N.hid;
     floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+    float sum = 0.f;
 #pragma unroll
     for (int ks = 0; ks < MAX_OUT / 4; ks++) acc = mfma16(d3[c * D3S + 4 * ks + g], 4 * ks + g < N.out ? W.w3[ks] : 0.f, acc);      // columns of d_pre3 beyond the output width are zero
 #pragma unroll
     for (int v = 0; v < 4; v++) {
         const int idx = (4 * g + v) * S + n;
-        g2[idx] = n_ok ? acc[v] * dact_hidden<ACT_H>(h2[idx], N.act_h) : 0.f;
+        const float d = n_ok ? acc[v] * dact_hidden<ACT_H>(h2[idx], N.act_h) : 0.f;
+        g2[idx] = d; sum += d;
     }
+    return sum;
 }
-// this wavefront's tile of d_pre1 = (d_pre2 W2) f'(h1) into p1 (may be h1 itself)
+// this wavefront's tile of d_pre1 = (d_pre2 W2) f'(h1) into p1 (may be h1 itself); returns the lane's share of its unit's column sum
 template <int ACT_H>
-__device__ __forceinline__ void backward_layer2(const WNet& N, const BackOperands& W, lptr g2, lptr h1, lptr p1, int wave, int c, int g) {
+__device__ __forceinline__ float backward_layer2(const WNet& N, const BackOperands& W, lptr g2, lptr h1, lptr p1, int wave, int c, int g) {
     const int n = 16 * wave + c, tiles = (N.hid + 15) >> 4;
     const bool n_ok = n < N.hid;
     const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
     floatx4 a0 = zero4, a1 = zero4;
     chunks<MAX_H / 16>(a0, a1, g2, S, c, g, 0, tiles, W.w2);
     const floatx4 acc = a0 + a1;
+    float sum = 0.f;
 #pragma unroll
     for (int v = 0; v < 4; v++) {
         const int idx = (4 * g + v) * S + n;
-        p1[idx] = n_ok ? acc[v] * dact_hidden<ACT_H>(h1[idx], N.act_h) : 0.f;
+        const float d = n_ok ? acc[v] * dact_hidden<ACT_H>(h1[idx], N.act_h) : 0.f;
+        p1[idx] = d; sum += d;
+    }
+    return sum;
+}
+// A tile of a weight gradient over the workgroup's sixteen rows, d^T x: d [16][S], its columns 16 mt ...; x [16][stride], its columns 16 nt ...; into dst [rows][cols]
+__device__ __forceinline__ void gradient_tile(lptr d, int mt, lptr x, int stride, int nt, int rows, int cols, float* dst, int c, int g) {
+    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < ROWS / 4; ks++) acc = mfma16(d[(4 * ks + g) * S + 16 * mt + c], x[(4 * ks + g) * stride + 16 * nt + c], acc);
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const int m = 16 * mt + 4 * g + v, n = 16 * nt + c;
+        if (m < rows && n < cols) dst[(size_t)m * cols + n] = acc[v];
     }
 }
 // The workgroup's 16 rows of an array between memory and LDS: wavefront w takes row w, all of a lane's loads are on their way before the first is written (a loop that
@@ -297,7 +326,7 @@ __device__ __forceinline__ void take_over(uint64_t* const (&word)[N], float (&va
     }
 }
 // The copies of the weights that load_swizzled reads, made anew before every update (the optimisers change the weights between them): thread t of block (x, job) writes
-// the 16 bytes of lane t % 64 of one (wavefront, chunk) pair, for all sixteen wavefronts whatever the width (those beyond it find zeros). Forward copies read 16
+// the 16 bytes of lane t % 64 of one (wavefront, chunk) pair, for the wavefronts that have units. Forward copies read 16
 // consecutive bytes of a row, backward copies four values a row apart (the 16 lanes of a group read 64 consecutive bytes each time).
 constexpr int PREP_JOBS = 12;
 struct PrepArgs {
@@ -314,7 +343,7 @@ __global__ __launch_bounds__(256) void wide_prepare_kernel(PrepArgs P) {
         uint32_t* const age = threadIdx.x == 0 ? P.age[0] : threadIdx.x == 1 ? P.age[1] : P.age[2];
         if (age) { const uint32_t before = *age; P.age_before[threadIdx.x] = before; *age = before + 1; }
     }
-    if (t >= WAVES * chunks * 64) return;
+    if (t >= ((units + 15) >> 4) * chunks * 64) return;
     const int lane = t & 63, pair = t >> 6, w = pair / chunks, j = pair - w * chunks, c = lane & 15, g = lane >> 4;
     const int n = 16 * w + c, k = 16 * j + 4 * g;
     const float* W = P.W[job];
@@ -334,7 +363,7 @@ struct Copies {
         for (int q = 0; q < jobs; q++) if (args.W[q] == W && args.backward[q] == (int)backward) return args.dst[q];
         args.W[jobs] = W; args.dst[jobs] = next; args.units[jobs] = units; args.depth[jobs] = depth; args.backward[jobs] = backward;
         next += copy_floats(depth);
-        const int b = rlt_div_up(WAVES * ((depth + 15) >> 4) * 64, 256);
+        const int b = rlt_div_up(((units + 15) >> 4) * ((depth + 15) >> 4) * 64, 256);
         if (b > blocks) blocks = b;
         return args.dst[jobs++];
     }
@@ -633,21 +662,25 @@ constexpr size_t LDS_FLOATS = (size_t)ROWS * SXS + 4 * ROWS * S + 4 * ROWS * D3S
 
 // ---- Forward and backward pass of one three-layer network over a few thousand rows at most, on the same machinery (nn_models/mlp/operations_generic.h:103-204: forward, the
 // loss gradient given or formed from a target as the MSE's, backward with weight gradients): a workgroup takes 16 rows through the three layers and back and leaves
-// activations and pre-activation gradients in memory; the weight gradients over the whole batch are the next launch (batch_gradient.hip). Where a batch is too small to fill the chip with the 64-row tiles of the one-pass kernel for large batches (mlp_fused.hip: 4,096 rows are 64 tiles for 256
+// activations and pre-activation gradients in memory; the weight gradients over the whole batch are the next launch (batch_gradient.hip). Narrow networks, whose gradients are few
+// tiles there and few bytes here, go the other way (BLOCKS): a workgroup forms its sixteen rows' weight gradients out of LDS and leaves them as a block, and the next launch adds the
+// blocks up (which way is taken: sum_blocks()). Where a batch is too small to fill the chip with the 64-row tiles of the one-pass kernel for large batches (mlp_fused.hip: 4,096 rows are 64 tiles for 256
 // compute units, and a tile takes its 74 us whatever the batch), sixteen-row tiles are a launch of 256 workgroups.
 struct MlpWideArgs {
     WNet net;
     const float* x; int ldx; float* y; int ldy;
     const float* d_output; int ldd; const float* target; int ldt; float mse_scale;
     int batch;
+    float* partial; int count;                 // BLOCKS: [workgroups][count] blocks dW1 | db1 | dW2 | db2 | dW3 | db3
     Trained kept;                              // MLP_FORWARD_BACKWARD: hidden activations; both: the gradients at the hidden pre-activations (and, unless the caller's array serves, the last)
     const float* out1; const float* out2;      // MLP_BACKWARD: the outputs of layers 1 and 2 that a forward() left in memory, [batch x hid] each; d_output is then the gradient at the last pre-activations
     float* keep_pre[3]; float* keep_out[3]; int act3;      // MLP_FORWARD: every layer's pre-activations and outputs as forward() keeps them (each may be NULL); the last layer's activation
 };
 enum { MLP_FORWARD_BACKWARD = 0, MLP_BACKWARD = 1, MLP_FORWARD = 2 };
-template <int ACT_H, int NT1C, int PASS>
+enum { MLP_ANY = 0, MLP_BLOCKS = 1, MLP_EVERY = 2 };      // MLP_BLOCKS: weight gradients as blocks; MLP_EVERY: more than 240 units, every wavefront has some
+template <int ACT_H, int NT1C, int PASS, int FORM>
 __global__ __launch_bounds__(THREADS) void mlp_wide_kernel(MlpWideArgs A) {
-    constexpr bool BACKWARD_ONLY = PASS == MLP_BACKWARD;
+    constexpr bool BACKWARD_ONLY = PASS == MLP_BACKWARD, BLOCKS = FORM == MLP_BLOCKS, EVERY = FORM == MLP_EVERY;
     extern __shared__ __attribute__((aligned(16))) float lds_wide[];
     const int gi = blockIdx.x;
     const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
@@ -656,31 +689,47 @@ __global__ __launch_bounds__(THREADS) void mlp_wide_kernel(MlpWideArgs A) {
     const WNet N = A.net;
     const int B = A.batch, IN = N.in, HID = N.hid, OUT = N.out, tiles = (HID + 15) >> 4, row0 = gi * ROWS;
     const bool on = wave < tiles;
-    const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
     const bool my_row = row0 + wave < B;
     const size_t row_at = min(row0 + wave, B - 1);
     Operands<NT1C> W;
     BackOperands K;
-    float b3 = 0.f;
+    float b3 = 0.f, s3 = 0.f, given[4] = {0.f, 0.f, 0.f, 0.f};      // given: this lane's elements of the gradient at the output, or of the target it is formed from
+    auto request_given = [&] {
+        const float* const from = A.target ? A.target : A.d_output;
+        const int ld = A.target ? A.ldt : A.ldd;
+#pragma unroll
+        for (int v = 0; v < 4; v++) given[v] = from[(size_t)min(row0 + 4 * g + v, B - 1) * ld + min(c, OUT - 1)];
+    };
+    if (BACKWARD_ONLY || (PASS == MLP_FORWARD_BACKWARD && !EVERY)) request_given();
     if (BACKWARD_ONLY) {
         // the hidden activations come back from memory (zero beyond the batch and beyond the width, up to the multiple of 16 that the tiles run to)
-        float v1[4], v2[4];
+        float v1[4], v2[4], vx[3];
+        if (BLOCKS) request_row(A.x + row_at * A.ldx, IN, lane, vx);
         request_row(A.out1 + row_at * HID, HID, lane, v1);
         request_row(A.out2 + row_at * HID, HID, lane, v2);
-        load_back_operands(N, wave, c, g, K);
+        if (on) load_back_operands<EVERY>(N, wave, c, g, K);
         place_row(h1 + wave * S, my_row, HID, 16 * tiles, lane, v1);
         place_row(h2 + wave * S, my_row, HID, 16 * tiles, lane, v2);
+        if (BLOCKS) place_row(xa + wave * SXS, my_row, IN, SXS, lane, vx);
+        if (wave == 0) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const float d = c < OUT && row0 + 4 * g + v < B ? given[v] : 0.f;
+                d3[(4 * g + v) * D3S + c] = d;
+                s3 += d;
+            }
+        }
     } else {
         float v[3];
         request_row(A.x + row_at * A.ldx, IN, lane, v);
-        load_operands<NT1C>(N, wave, c, g, W);
+        load_operands<NT1C, EVERY>(N, wave, c, g, W);
         b3 = N.b3[min(c, OUT - 1)];
         place_row(xa + wave * SXS, my_row, IN, SXS, lane, v);
     }
     rlt_lds_barrier();
     if (PASS == MLP_FORWARD) {
         const KeepArgs keep = {{A.keep_pre[0], A.keep_pre[1]}, {A.keep_out[0], A.keep_out[1]}, row0, B};
-        forward3<ACT_H, NT1C, false, true, true>(N, W, N, xa, SXS, h1, h2, yp, wave, c, g, &keep);
+        forward3<ACT_H, NT1C, false, true, true, EVERY>(N, W, N, xa, SXS, h1, h2, yp, wave, c, g, &keep);
         if (wave == 0) {
             const floatx4 out = output_tile(yp, tiles, c, g);
 #pragma unroll
@@ -698,20 +747,15 @@ __global__ __launch_bounds__(THREADS) void mlp_wide_kernel(MlpWideArgs A) {
         return;
     }
     if (PASS == MLP_FORWARD_BACKWARD) {
-        forward3<ACT_H, NT1C, false, true>(N, W, N, xa, SXS, h1, h2, yp, wave, c, g);
-        load_back_operands(N, wave, c, g, K);
-        store_rows(h1, A.kept.h1, HID, row0, B, wave, lane);
-        store_rows(h2, A.kept.h2, HID, row0, B, wave, lane);
-    }
-    if (BACKWARD_ONLY) {
-        if (wave == 0) {
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int row = row0 + 4 * g + v;
-                d3[(4 * g + v) * D3S + c] = (c < OUT && row < B) ? A.d_output[(size_t)row * A.ldd + c] : 0.f;
-            }
+        forward3<ACT_H, NT1C, false, true, false, EVERY>(N, W, N, xa, SXS, h1, h2, yp, wave, c, g);
+        if (EVERY) request_given();      // (all of W fills the registers until here)
+        load_back_operands<EVERY>(N, wave, c, g, K);
+        if (!BLOCKS) {
+            store_rows(h1, A.kept.h1, HID, row0, B, wave, lane);
+            store_rows(h2, A.kept.h2, HID, row0, B, wave, lane);
         }
-    } else if (wave == 0) {
+    }
+    if (!BACKWARD_ONLY && wave == 0) {
         // lane (c, g): output column c of rows 4 g + v; the gradient at the output (the last layer has no activation): given, or the MSE's against the target
         const floatx4 out = output_tile(yp, tiles, c, g);
 #pragma unroll
@@ -721,18 +765,87 @@ __global__ __launch_bounds__(THREADS) void mlp_wide_kernel(MlpWideArgs A) {
             const float yv = out[v] + b3;
             if (ok && A.y) A.y[(size_t)row * A.ldy + c] = yv;
             float d = 0.f;
-            if (ok) d = A.target ? (yv - A.target[(size_t)row * A.ldt + c]) * A.mse_scale : A.d_output[(size_t)row * A.ldd + c];
+            if (ok) d = A.target ? (yv - given[v]) * A.mse_scale : given[v];
             d3[(4 * g + v) * D3S + c] = d;
-            if (row < B) A.kept.d3[(size_t)row * MAX_OUT + c] = d;
+            s3 += d;
+            if (!BLOCKS && row < B) A.kept.d3[(size_t)row * MAX_OUT + c] = d;
         }
     }
-    rlt_lds_barrier();      // d_pre3 is in place
-    if (on) backward_layer3<ACT_H>(N, K, d3, h2, ta, wave, c, g);
+    if (!BACKWARD_ONLY) rlt_lds_barrier();      // d_pre3 is in place (the backward pass alone: with the activations)
+    const float s2 = on ? backward_layer3<ACT_H>(N, K, d3, h2, ta, wave, c, g) : 0.f;
+    if (BLOCKS) {
+        float* const block = A.partial + (size_t)gi * A.count;
+        float* const to_b1 = block + HID * IN; float* const to_w2 = to_b1 + HID; float* const to_b2 = to_w2 + HID * HID; float* const to_w3 = to_b2 + HID; float* const to_b3 = to_w3 + OUT * HID;
+        const int n = 16 * wave + c, spare = WAVES - tiles;
+        // Wavefronts without units (half of them and more up to width 128) form dW3 and dW2 while the others go on with the backward pass and dW1; without enough of them each does its units' rows
+        const bool spread = spare >= tiles;
+        auto last_layer = [&](int u) {      // dW3: columns 16 u ...
+            floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < ROWS / 4; ks++) acc = mfma16(d3[(4 * ks + g) * D3S + c], h2[(4 * ks + g) * S + 16 * u + c], acc);
+#pragma unroll
+            for (int v = 0; v < 4; v++) if (4 * g + v < OUT && 16 * u + c < HID) to_w3[(4 * g + v) * HID + 16 * u + c] = acc[v];
+        };
+        if (spread ? !on && wave - tiles < tiles : on) last_layer(spread ? wave - tiles : wave);
+        rlt_lds_barrier();      // every wavefront's tile of d_pre2 is in place
+        if (on) {
+            const float s1 = backward_layer2<ACT_H>(N, K, ta, h1, tb, wave, c, g);
+            wave_sync();            // dW1's rows are this wavefront's own tile of d_pre1
+#pragma unroll 2
+            for (int nt = 0; nt < (IN + 15) >> 4; nt++) gradient_tile(tb, wave, xa, SXS, nt, HID, IN, block, c, g);
+            const float b1 = groups_sum(s1), b2 = groups_sum(s2);
+            if (g == 0 && n < HID) { to_b1[n] = b1; to_b2[n] = b2; }
+        }
+        if (!spread && on) {
+#pragma unroll 4
+            for (int nt = 0; nt < tiles; nt++) gradient_tile(ta, wave, h1, S, nt, HID, HID, to_w2, c, g);
+        } else if (spread && !on) {
+#pragma unroll 2
+            for (int p = wave - tiles; p < tiles * tiles; p += spare) gradient_tile(ta, p / tiles, h1, S, p % tiles, HID, HID, to_w2, c, g);
+        }
+        if (wave == 0) {
+            s3 = groups_sum(s3);
+            if (g == 0 && c < OUT) to_b3[c] = s3;
+        }
+        return;
+    }
     rlt_lds_barrier();      // every wavefront's tile of d_pre2 is in place
     store_rows(ta, A.kept.d2, HID, row0, B, wave, lane);
     if (on) backward_layer2<ACT_H>(N, K, ta, h1, tb, wave, c, g);
     rlt_lds_barrier();
     store_rows(tb, A.kept.d1, HID, row0, B, wave, lane);
+}
+// gradient[e] += the sum over the workgroups' blocks of element e: a workgroup takes 64 elements, its wavefronts a quarter of the blocks each, sixteen blocks' loads in flight
+struct BlockSum { const float* partial; int blocks, count, total; float* gradient[6]; int end[6]; };
+__global__ __launch_bounds__(256) void block_sum_kernel(BlockSum R) {
+    __shared__ float quarter[4][64];
+    const int lane = threadIdx.x & 63, q = threadIdx.x >> 6, e = blockIdx.x * 64 + lane, per = (R.blocks + 3) / 4, end = min(R.blocks, (q + 1) * per);
+    const float* from = R.partial + min(e, R.total - 1);
+    float sum = 0.f;
+    for (int b0 = q * per; b0 < end; b0 += 16) {
+        float v[16];
+#pragma unroll
+        for (int u = 0; u < 16; u++) v[u] = from[(size_t)min(b0 + u, end - 1) * R.count];
+#pragma unroll
+        for (int u = 0; u < 16; u++) sum += b0 + u < end ? v[u] : 0.f;
+    }
+    quarter[q][lane] = sum;
+    __syncthreads();
+    if (q != 0 || e >= R.total) return;
+    int k = 0, begin = 0;
+#pragma unroll
+    for (int i = 0; i < 5; i++) if (e >= R.end[i]) { k = i + 1; begin = R.end[i]; }
+    float* const to = k == 0 ? R.gradient[0] : k == 1 ? R.gradient[1] : k == 2 ? R.gradient[2] : k == 3 ? R.gradient[3] : k == 4 ? R.gradient[4] : R.gradient[5];
+    to[e - begin] += (quarter[0][lane] + quarter[1][lane]) + (quarter[2][lane] + quarter[3][lane]);
+}
+// Whether the workgroups' blocks are added up (else the weight gradients are a contraction over the whole batch of their own). Forward + backward with 17 inputs, blocks / contraction,
+// us: width 65 at 256 rows 16.7 / 19.4, 1,000 17.2 / 20.3, 4,096 21.1 / 25.9; width 100 at 256 19.0 / 20.5, 1,000 20.4 / 21.8, 4,096 27.0 / 28.1; width 128 at 64 20.4 / 19.2, at
+// 512 21.4 / 22.8, at 1,000 22.9 / 22.7; width 192 at 512 28.7 / 26.9. With 128 inputs, backward pass alone: width 64 at 256 14.9 / 15.2, 4,096 19.0 / 17.5. Width 112 with 40 inputs, backward
+// pass alone: 2,048 rows 19.6 / 23.2, 3,000 22.3 / 22.1, 4,096 25.0 / 23.9.
+bool sum_blocks(int hid, int in, int batch) {
+    const int products = hid * (hid + in);
+    if (hid <= 112 && products <= 18432) return batch <= 1024 || (in <= 64 && (int64_t)products * batch <= 62914560);
+    return products <= 24576 && batch > 256 && batch <= 768;
 }
 
 bool hidden_ok(int a) { return a == RLT_ACT_RELU || a == RLT_ACT_TANH || a == RLT_ACT_FAST_TANH || a == RLT_ACT_SIGMOID; }
@@ -1028,7 +1141,14 @@ static int mlp_wide_launch(rlt_rocm_device* device, const rlt_dense_layer* L, in
     rlt_gradient_net net = {};
     net.in = IN; net.hid = hid; net.out = OUT;
     float* partial = nullptr;
-    if (!forward_only) {
+    const bool blocks = !forward_only && sum_blocks(hid, IN, batch);
+    const int exact = hid * IN + hid + hid * hid + hid + OUT * hid + OUT;
+    if (blocks) {
+        void* scratch = nullptr;
+        a.count = (exact + 63) & ~63;
+        if ((rc = rlt_scratch(device, (size_t)groups * a.count * sizeof(float), &scratch))) return rc;
+        a.partial = (float*)scratch;
+    } else if (!forward_only) {
         void* scratch = nullptr;
         if ((rc = rlt_scratch(device, (trained_floats(hid, batch) + rlt_batch_gradients_partial_floats(&net, 1, batch)) * sizeof(float), &scratch))) return rc;
         a.kept = place_trained((float*)scratch, hid, batch);
@@ -1041,24 +1161,33 @@ static int mlp_wide_launch(rlt_rocm_device* device, const rlt_dense_layer* L, in
     if (!forward_only) copies.backward(a.net);
     if ((rc = copies.launch(device))) return rc;
     const size_t lds_bytes = LDS_FLOATS * sizeof(float);
-#define RLT_LAUNCH_MLP_WIDE(ACT, NT, BWD)                                                                                                                   \
-    do {                                                                                                                                                    \
-        RLT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(mlp_wide_kernel<ACT, NT, BWD>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes)); \
-        hipLaunchKernelGGL((mlp_wide_kernel<ACT, NT, BWD>), dim3(groups), dim3(THREADS), lds_bytes, device->stream, a);                                    \
+#define RLT_LAUNCH_MLP_WIDE(ACT, NT, P, FORM)                                                                                                                   \
+    do {                                                                                                                                                       \
+        RLT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(mlp_wide_kernel<ACT, NT, P, FORM>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes)); \
+        hipLaunchKernelGGL((mlp_wide_kernel<ACT, NT, P, FORM>), dim3(groups), dim3(THREADS), lds_bytes, device->stream, a);                                    \
     } while (0)
     const bool relu = a.net.act_h == RLT_ACT_RELU;
-#define RLT_LAUNCH_MLP_WIDE_PASS(P)                                                                                                       \
-    do {                                                                                                                                  \
-        if (IN <= 32) { if (relu) RLT_LAUNCH_MLP_WIDE(RLT_ACT_RELU, 2, P); else RLT_LAUNCH_MLP_WIDE(-1, 2, P); }                          \
-        else if (IN <= 64) { if (relu) RLT_LAUNCH_MLP_WIDE(RLT_ACT_RELU, 4, P); else RLT_LAUNCH_MLP_WIDE(-1, 4, P); }                     \
-        else { if (relu) RLT_LAUNCH_MLP_WIDE(RLT_ACT_RELU, MAX_D / 16, P); else RLT_LAUNCH_MLP_WIDE(-1, MAX_D / 16, P); }                  \
+#define RLT_LAUNCH_MLP_WIDE_PASS(P, FORM)                                                                                                                       \
+    do {                                                                                                                                                       \
+        if (IN <= 32) { if (relu) RLT_LAUNCH_MLP_WIDE(RLT_ACT_RELU, 2, P, FORM); else RLT_LAUNCH_MLP_WIDE(-1, 2, P, FORM); }                                     \
+        else if (IN <= 64) { if (relu) RLT_LAUNCH_MLP_WIDE(RLT_ACT_RELU, 4, P, FORM); else RLT_LAUNCH_MLP_WIDE(-1, 4, P, FORM); }                                \
+        else { if (relu) RLT_LAUNCH_MLP_WIDE(RLT_ACT_RELU, MAX_D / 16, P, FORM); else RLT_LAUNCH_MLP_WIDE(-1, MAX_D / 16, P, FORM); }                            \
     } while (0)
-    if (backward_only) RLT_LAUNCH_MLP_WIDE_PASS(MLP_BACKWARD); else if (forward_only) RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD); else RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD_BACKWARD);
+    const bool every = hid > MAX_H - 16;
+    if (forward_only) { if (every) RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD, MLP_EVERY); else RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD, MLP_ANY); }
+    else if (backward_only) { if (blocks) RLT_LAUNCH_MLP_WIDE_PASS(MLP_BACKWARD, MLP_BLOCKS); else if (every) RLT_LAUNCH_MLP_WIDE_PASS(MLP_BACKWARD, MLP_EVERY); else RLT_LAUNCH_MLP_WIDE_PASS(MLP_BACKWARD, MLP_ANY); }
+    else { if (blocks) RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD_BACKWARD, MLP_BLOCKS); else if (every) RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD_BACKWARD, MLP_EVERY); else RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD_BACKWARD, MLP_ANY); }
 #undef RLT_LAUNCH_MLP_WIDE_PASS
 #undef RLT_LAUNCH_MLP_WIDE
     if ((rc = rlt_launch_status(device))) return rc;
     if (forward_only) return 0;
     const Segments seg = segments_of(L);
+    if (blocks) {
+        BlockSum R = {a.partial, groups, a.count, exact, {}, {}};
+        for (int k = 0, end = 0; k < 6; k++) { R.gradient[k] = seg.gradient[k]; R.end[k] = end += (int)seg.size[k]; }
+        hipLaunchKernelGGL(block_sum_kernel, dim3(rlt_div_up(exact, 64)), dim3(256), 0, device->stream, R);
+        return rlt_launch_status(device);
+    }
     for (int k = 0; k < 6; k++) net.gradient[k] = seg.gradient[k];
     if (backward_only) { net.h1 = L[0].output; net.h2 = L[1].output; net.d3 = d_output; net.ld3 = ldd; }
     return rlt_batch_gradients(device, &net, 1, batch, 0.0f, nullptr, partial);

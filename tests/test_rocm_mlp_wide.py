@@ -40,6 +40,10 @@ CASES = [
     (512, 64, 33, 6, "tanh", False),         # the most rows that one workgroup of the gradients' launch takes; two columns of the second tile of 32
     (513, 65, 256, 2, "tanh", True),         # ... and one more: two groups of workgroups share the batch; the first layer in five chunks
     (2051, 17, 250, 3, "tanh", False),       # eight groups
+    (513, 128, 128, 3, "relu", False),       # few tiles: eight groups for two groups' rows
+    # the workgroups' blocks added up: the narrowest with spare wavefronts, the widest, the last and the first batch of each line, without spare wavefronts
+    (16, 3, 65, 1, "relu", True), (255, 1, 97, 16, "fast_tanh", False), (300, 60, 112, 2, "relu", False), (4096, 17, 100, 5, "tanh", True),
+    (1024, 65, 80, 3, "tanh", False), (1025, 65, 80, 3, "tanh", False), (768, 20, 144, 4, "relu", True), (769, 20, 144, 4, "relu", True), (257, 1, 150, 1, "sigmoid", False),
 ]
 
 
@@ -104,7 +108,8 @@ def forward_then_backward(backend, dims, params, x, dy, ha, oa):
 
 
 @pytest.mark.parametrize("case", [(256, 17, 256, 6, "relu", "identity"), (4096, 17, 256, 6, "relu", "tanh"), (37, 35, 200, 1, "tanh", "identity"), (100, 128, 72, 16, "fast_tanh", "sigmoid"),
-                                  (1000, 3, 64, 2, "sigmoid", "identity")])
+                                  (1000, 3, 64, 2, "sigmoid", "identity"), (300, 128, 64, 3, "relu", "identity"), (4096, 2, 33, 1, "tanh", "identity"), (768, 20, 144, 4, "relu", "tanh"),
+                                  (257, 128, 20, 16, "relu", "identity"), (1, 5, 16, 2, "tanh", "identity")])
 def test_backward_alone_on_sixteen_row_tiles_matches_the_checker_and_the_other_paths(oracle, rocm, case, monkeypatch):
     """backward() after forward(): the tiles read the hidden layers' outputs back from memory; the last layer may have any activation (its derivative is applied to the
     given gradient before the kernel runs, in place as in the reference)."""
@@ -130,11 +135,13 @@ def test_backward_alone_on_sixteen_row_tiles_matches_the_checker_and_the_other_p
 
 
 
+# (hidden width 72: the workgroups' blocks of sixteen rows; 200: the batch shared out to wavefronts and groups of workgroups)
+@pytest.mark.parametrize("H", [72, 200])
 @pytest.mark.parametrize("B,row", [(300, 80), (300, 299), (1100, 150)])
-def test_an_infinite_input_stays_in_its_column_and_infinite(rocm, B, row):
+def test_an_infinite_input_stays_in_its_column_and_infinite(rocm, B, row, H):
     """The wavefronts' shares of the batch do not end where their chunks of 32 rows do: a row behind a share's end is another share's, and its infinity meets no zero there.
     d_pre1 of a tanh network is not zero, so that column of the first layer's gradient is infinite and everything else finite."""
-    dims = [17, 72, 72, 6]
+    dims = [17, H, H, 6]
     rng = np.random.default_rng(B + row)
     params = helpers.random_params(rng, dims)
     x, dy = rng.standard_normal((B, 17)).astype(np.float32), rng.standard_normal((B, 6)).astype(np.float32)
@@ -150,5 +157,5 @@ def test_an_infinite_input_stays_in_its_column_and_infinite(rocm, B, row):
     grads = net.grads.numpy()
     off, nw, _ = net.offsets[0]
     infinite = np.zeros(grads.shape, bool)
-    infinite[off:off + nw].reshape(72, 17)[:, 3] = True
+    infinite[off:off + nw].reshape(H, 17)[:, 3] = True
     assert np.isinf(grads[infinite]).all() and np.isfinite(grads[~infinite]).all()
