@@ -942,10 +942,13 @@ typedef struct rlt_sac_sequence_agent {
     void* workspace; size_t workspace_bytes; /* >= rlt_rocm_sac_sequence_workspace_bytes */
 } rlt_sac_sequence_agent;
 
-/* The sequence updates below run network passes that do not depend on each other at the same time -- the trained critic's forward pass next to the (target) actor's,
+/* The sequence updates below run network passes that do not depend on each other at the same time. Where the actor and all critics are recurrent approximators (a dense
+ * layer, two GRUs of width 16 or 32, a dense layer; up to 4,800 sequences and 163,840 steps in all) a SAC update's passes of this kind share a launch on the stream the calls are enqueued on. For any
+ * other agent the trained critic's forward pass next to the (target) actor's,
  * the second target critic next to the first, in train_actor the second critic's forward pass and input gradient next to the first's -- the second of each pair on a
  * stream of the handle's own that waits for, and is waited for by, the stream the calls are enqueued on (each recurrence fills about a twentieth of the chip);
- * rlt_rocm_sac_sequence_train_critics uses two such streams. The workspace is three parts for that reason. Results are those of the passes in sequence, bit for bit. While the stream records a graph the passes stay in sequence. */
+ * rlt_rocm_sac_sequence_train_critics uses two such streams, and while the stream records a graph the passes stay in sequence. The workspace is three parts for that reason.
+ * Results are those of the passes in sequence, bit for bit. */
 size_t rlt_rocm_sac_sequence_workspace_bytes(const rlt_sac_sequence_agent* agent);
 /* train_critic on a sequence batch   rl/algorithms/sac/operations_generic.h:243-337
  *   action_noise [T x B x action_dim]: the N(0,1) noise of the actor's sample_and_squash layer on the `next` views.
@@ -954,7 +957,7 @@ size_t rlt_rocm_sac_sequence_workspace_bytes(const rlt_sac_sequence_agent* agent
 int rlt_rocm_sac_sequence_train_critic(rlt_rocm_device* device, const rlt_sac_sequence_agent* agent, int critic_index, const float* action_noise);
 /* train_critic for critic 0, then for critic 1, on the agent's batch with the same noise: the loop's SHARED_BATCH case (rl/algorithms/sac/loop/core/operations_generic.h:127-138,
  * where the second call repeats the actor's pass over the next rows, its sample, both target critics and the target values on unchanged inputs). Those are computed
- * once here, the two critics' own passes run next to each other on the handle's two streams, and the results are those of the two calls bit for bit (critic 1's loss
+ * once here, the two critics' own passes run next to each other as described above, and the results are those of the two calls bit for bit (critic 1's loss
  * gradient is left in agent->d_output, as they leave it; critic 0's goes to the end of the workspace). */
 int rlt_rocm_sac_sequence_train_critics(rlt_rocm_device* device, const rlt_sac_sequence_agent* agent, const float* action_noise);
 /* update_critic_targets   sac/operations_generic.h:486-527 (dense and GRU layers, incl. the initial hidden state) */

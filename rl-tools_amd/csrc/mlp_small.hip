@@ -11,7 +11,7 @@
 // are exchanged between wavefronts, and a workgroup writes one block of partial sums at the end, which a second kernel adds to the layers'
 // gradients in workgroup order: the result does not depend on scheduling. Activations and gradients of the round sit in LDS in the layouts
 // v_mfma_f32_16x16x4_f32 wants (lane l = r + 16 kk feeds A[r][kk] and B[kk][r] and receives D[4 kk + v][r], v = 0..3); the weights are staged
-// once per workgroup in LDS (padded rows, read as both W and W^T). Four workgroup barriers per round order the two kinds of phase.
+// once per workgroup in LDS (padded rows, read as both W and W^T). Seven workgroup barriers per round (five with two layers) order the phases.
 // Bound: latency. One round is 460 matrix instructions per SIMD (14.7 K cycles at 105 -> 64 -> 64 -> 8), between LDS round trips and the activations' chains, and 141 KB of LDS leave room
 // for one workgroup per compute unit: two wavefronts per SIMD instead of one (four that had all columns of their rows) took PPO's pair at 8,192 rows from 30.0 to 25.6 us and the
 // head 64 -> 64 -> 4 of a sequence model at 65,536 rows from 56.2 to 47.2 us, with the same sums in the same order.

@@ -21,7 +21,7 @@ int rlt_adam_step_pair(rlt_rocm_device* device, const rlt_adam_tensor* tensors_a
 
 // ---- device side -------------------------------------------------------------------------------------------------------------------
 // Words of the device handle's counters block (uint32 index) that the kernels with an optimiser tail use as tickets; every user
-// leaves its words zero. [0] and [16] belong to adam_kernel / adam_pair_kernel.
+// leaves its words zero. The tickets of adam_kernel and adam_pair_kernel lie behind them, from RLT_ADAM_TICKETS_OFFSET on (rlt_tickets_of).
 enum { RLT_TICKET_TAIL = 32 /* .. +7 */ };
 
 // The last workgroup through a launch advances the optimiser's age, which every workgroup reads. Nothing else passes between the workgroups (unless the squared norm is

@@ -427,7 +427,7 @@ int rlt_rocm_sac_train_critic(rlt_rocm_device* device, const rlt_sac_agent* A, i
 int rlt_rocm_sac_update_critic_targets(rlt_rocm_device* device, const rlt_sac_agent* A) {
     if (!device) return RLT_E_NOT_INITIALISED;
     RLT_REQUIRE(agent_ok(A));
-    if (!device->sac_per_operation && 4 * A->n_critic_layers <= 64) {      // all tensors in one launch (per 16)
+    if (!device->sac_per_operation && 4 * A->n_critic_layers <= 64) {      // all tensors in one launch (per 32)
         const float* sources[64]; float* targets[64]; uint32_t counts[64];
         int n = 0;
         for (int k = 0; k < 2; k++)
@@ -678,10 +678,11 @@ int rlt_rocm_sac_sequence_train_critic(rlt_rocm_device* device, const rlt_sac_se
 }
 
 // Both critics on one batch and one set of noise (the loop's SHARED_BATCH case, rl/algorithms/sac/loop/core/operations_generic.h:127-138): what the two calls of
-// train_critic would compute twice -- the actor on the next rows, its sample, both target critics, the target values -- is computed once, and the two critics'
-// passes run next to each other on the handle's three streams: first side stream critic 0 forward, then target critic 1; second side stream critic 1 forward; main
+// train_critic would compute twice -- the actor on the next rows, its sample, both target critics, the target values -- is computed once. Agents of recurrent
+// approximators (sequence_agent_stacked) take stacked_train_critics: both critics' passes and the actor's are one launch on the handle's stream, then the two target critics' one,
+// the two backward passes one, and one step of both optimisers. For any other agent the two critics' passes run next to each other on the handle's three streams: first side stream critic 0 forward, then target critic 1; second side stream critic 1 forward; main
 // stream actor, sample, target critic 0; after the join the target values and both loss gradients, then critic 0's backward pass on the main stream next to critic 1's
-// on a side stream, then both optimisers. Every pass is the launch sequence that the single calls make, on the same inputs: the results are theirs bit for bit.
+// on a side stream, then both optimisers. Every pass does what the single calls' does, on the same inputs: the results are theirs bit for bit.
 int rlt_rocm_sac_sequence_train_critics(rlt_rocm_device* device, const rlt_sac_sequence_agent* A, const float* action_noise) {
     if (!device) return RLT_E_NOT_INITIALISED;
     RLT_REQUIRE(sequence_agent_ok(A) && action_noise);

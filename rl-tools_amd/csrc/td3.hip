@@ -361,7 +361,7 @@ int copy_columns(rlt_rocm_device* device, const float* src, int lds, float* dst,
 }
 inline const float* seq_last_output(const rlt_seq_layer* layers, int n) { const rlt_seq_layer& L = layers[n - 1]; return L.kind ? L.gru.output : L.dense.output; }
 inline int seq_last_dim(const rlt_seq_layer* layers, int n) { const rlt_seq_layer& L = layers[n - 1]; return L.kind ? L.gru.hidden_dim : L.dense.out_dim; }
-// every tensor of a target network in one launch per sixteen tensors
+// every tensor of a target network in one launch per 32 tensors
 int polyak_seq(rlt_rocm_device* device, const rlt_seq_layer* source, const rlt_seq_layer* target, int n, float polyak) {
     RLT_REQUIRE(n <= RLT_SEQ_MAX_LAYERS);
     const float* sources[5 * RLT_SEQ_MAX_LAYERS]; float* targets[5 * RLT_SEQ_MAX_LAYERS]; uint32_t counts[5 * RLT_SEQ_MAX_LAYERS];
