@@ -7,7 +7,7 @@
 // gradients themselves at batch 256 and 250 times at batch 4,000.
 // Up to 512 rows a workgroup sees the whole batch and finishes its elements. Beyond that the batch is shared out to two, four or eight groups of workgroups that lie on
 // different XCDs: the rows of a large batch (16 MB at 4,001 rows) do not fit an XCD's 4 MB of L2, and with every XCD reading all of them the launch took 32.6 us at
-// 4,001 rows; with an eighth of the rows per XCD 15.3 us, and a second launch adds the eight sums up (4 us).
+// 4,001 rows; with an eighth of the rows per XCD 15.5 us, and a second launch adds the eight sums up (4 us).
 // Bound: latency up to a few hundred rows (the trip to memory for the first operands, 16 steps of the matrix pipe, the exchange between the wavefronts, the stores),
 // then the loads of the operands from L2: each row of a network is read by its 8 to 16 column tiles.
 #include "batch_gradient.h"
