@@ -5,8 +5,8 @@
 // Here the work is split by what depends on time:
 //   * W_i x + b_i for ALL steps is one contraction over sequence*batch rows (gemm.hip), written straight into post_activation;
 //   * the recurrence runs in ONE launch: batch rows are independent, so no grid-wide synchronisation is needed. At hidden width 64 a
-//     wavefront owns one row for the whole sequence with W_h in its registers; at other widths a workgroup owns a few rows and keeps W_h
-//     and its rows' hidden state in LDS;
+//     workgroup carries four rows through the sequence on the matrix cores, at 16 and 32 a wavefront 64 / width rows, both with W_h in registers; at other widths a workgroup owns a few
+//     rows and keeps W_h and its rows' hidden state in LDS;
 //   * backward does the same in reverse and stores, per step, the gradient at the gate pre-activations (one copy as the input path sees
 //     it, one as the hidden path sees it, which differs in the n gate by the factor r) and the previous hidden state; the weight
 //     gradients and d_input are then three contractions over sequence*batch rows.

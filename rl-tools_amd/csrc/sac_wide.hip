@@ -1063,7 +1063,7 @@ int rlt_td3_wide_update_critic(rlt_rocm_device* device, const rlt_td3_agent* A, 
     return launch_wide<MODE_TD3_CRITIC>(device, a, rlt_div_up(A->batch, ROWS), &O, 1, 0.0f, nullptr);
 }
 
-// both critics on the agent's batch in one launch (the workgroups' roles: target chains and trained critics, three per critic), each with its own sampling noise for the target actor's td3_sampling layer:
+// both critics on the agent's batch in one launch (three roles per critic: two target chains and the trained critic), each with its own sampling noise for the target actor's td3_sampling layer:
 // what rlt_td3_wide_update_critic for critic 0 and then for critic 1 leave, bit for bit
 int rlt_td3_wide_update_critics(rlt_rocm_device* device, const rlt_td3_agent* A, const float* sampling_noise_first, const float* sampling_noise_second, const rlt_td3_critic_draws* draws, bool update_targets) {
     if (!rlt_td3_wide_supported(device, A)) return RLT_E_UNSUPPORTED;
