@@ -155,15 +155,16 @@ __device__ __forceinline__ void load_operands(const WNet& N, int wave, int c, in
 // took as long as the layers' arithmetic when they were requested at the start of each pass.
 // First layers of more than two chunks fill too many registers for that: then only the second layer's first half (and the small operands) are requested ahead, the
 // first layer's own operands at the start of the pass (W1_READY = false) and the second half after the first layer, as before.
+// LIVE: the activations of rows from `live` on (beyond the batch) are zero -- zero inputs alone leave NaNs there where a weight or a bias is infinite
 // KEEP: the hidden layers' pre-activations and outputs are also stored to memory, rows [row0, row0 + 16) of [batch x hid] arrays (forward() of a network keeps them)
 struct KeepArgs { float* pre[2]; float* out[2]; int row0, batch; };
-template <int ACT_H, bool KEEP>
-__device__ __forceinline__ void place_hidden(const WNet& N, const floatx4& acc, float bias, lptr h, int n, int g, const KeepArgs* keep, int layer) {
+template <int ACT_H, bool KEEP, bool LIVE>
+__device__ __forceinline__ void place_hidden(const WNet& N, const floatx4& acc, float bias, lptr h, int n, int g, const KeepArgs* keep, int layer, int live) {
     const bool n_ok = n < N.hid;
 #pragma unroll
     for (int v = 0; v < 4; v++) {
         const float pre = acc[v] + bias, o = act_hidden<ACT_H>(pre, N.act_h);
-        h[(4 * g + v) * S + n] = n_ok ? o : 0.f;
+        h[(4 * g + v) * S + n] = n_ok && (!LIVE || 4 * g + v < live) ? o : 0.f;
         if (KEEP && n_ok && keep->row0 + 4 * g + v < keep->batch) {
             const size_t at = (size_t)(keep->row0 + 4 * g + v) * N.hid + n;
             if (keep->pre[layer]) keep->pre[layer][at] = pre;
@@ -171,8 +172,8 @@ __device__ __forceinline__ void place_hidden(const WNet& N, const floatx4& acc, 
         }
     }
 }
-template <int ACT_H, int NT1C, bool PREFETCH, bool W1_READY, bool KEEP = false, bool EVERY = false>
-__device__ __forceinline__ void forward3(const WNet& N, Operands<NT1C>& W, const WNet& next, lptr x, int xstride, lptr h1, lptr h2, lptr yp, int wave, int c, int g, const KeepArgs* keep = nullptr) {
+template <int ACT_H, int NT1C, bool PREFETCH, bool W1_READY, bool KEEP = false, bool EVERY = false, bool LIVE = false>
+__device__ __forceinline__ void forward3(const WNet& N, Operands<NT1C>& W, const WNet& next, lptr x, int xstride, lptr h1, lptr h2, lptr yp, int wave, int c, int g, const KeepArgs* keep = nullptr, int live = ROWS) {
     const int n = 16 * wave + c, tiles = (N.hid + 15) >> 4, lane = c + 16 * g, next_tiles = (next.hid + 15) >> 4;
     const bool on = wave < tiles, next_on = wave < next_tiles;
     const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
@@ -180,7 +181,7 @@ __device__ __forceinline__ void forward3(const WNet& N, Operands<NT1C>& W, const
     if (on) {
         floatx4 a0 = zero4, a1 = zero4;
         chunks<NT1C>(a0, a1, x, xstride, c, g, 0, (N.in + 15) >> 4, W.w1);
-        place_hidden<ACT_H, KEEP>(N, a0 + a1, W.b1, h1, n, g, keep, 0);
+        place_hidden<ACT_H, KEEP, LIVE>(N, a0 + a1, W.b1, h1, n, g, keep, 0, live);
     }
     if (NT1C > FEW) load_swizzled<8, EVERY>(N.W2f, tiles, on, wave, lane, 8, W.w2b);
     if (PREFETCH) {
@@ -194,7 +195,7 @@ __device__ __forceinline__ void forward3(const WNet& N, Operands<NT1C>& W, const
         if (PREFETCH) load_swizzled<8, EVERY>(next.W2f, next_tiles, next_on, wave, lane, 0, W.w2a);
         if (on) chunks<8>(a0, a1, h1, S, c, g, 8, tiles, W.w2b);
         if (PREFETCH && NT1C <= FEW) load_swizzled<8, EVERY>(next.W2f, next_tiles, next_on, wave, lane, 8, W.w2b);
-        if (on) place_hidden<ACT_H, KEEP>(N, a0 + a1, W.b2, h2, n, g, keep, 1);
+        if (on) place_hidden<ACT_H, KEEP, LIVE>(N, a0 + a1, W.b2, h2, n, g, keep, 1, live);
         if (PREFETCH) W.b2 = next.b2[min(n, next.hid - 1)];
     }
     rlt_lds_barrier();
@@ -238,8 +239,8 @@ __device__ __forceinline__ void load_back_operands(const WNet& N, int wave, int 
     load_swizzled<MAX_H / 16, EVERY>(N.W2b, tiles, wave < tiles, wave, c + 16 * g, 0, W.w2);
 }
 // this wavefront's tile of d_pre2 = (d_pre3 W3) f'(h2) into g2 (may be h2 itself); returns the lane's share of its unit's column sum
-template <int ACT_H>
-__device__ __forceinline__ float backward_layer3(const WNet& N, const BackOperands& W, lptr d3, lptr h2, lptr g2, int wave, int c, int g) {
+template <int ACT_H, bool LIVE = false>
+__device__ __forceinline__ float backward_layer3(const WNet& N, const BackOperands& W, lptr d3, lptr h2, lptr g2, int wave, int c, int g, int live = ROWS) {
     const int n = 16 * wave + c;
     const bool n_ok = n < N.hid;
     floatx4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -249,14 +250,14 @@ __device__ __forceinline__ float backward_layer3(const WNet& N, const BackOperan
 #pragma unroll
     for (int v = 0; v < 4; v++) {
         const int idx = (4 * g + v) * S + n;
-        const float d = n_ok ? acc[v] * dact_hidden<ACT_H>(h2[idx], N.act_h) : 0.f;
+        const float d = n_ok && (!LIVE || 4 * g + v < live) ? acc[v] * dact_hidden<ACT_H>(h2[idx], N.act_h) : 0.f;
         g2[idx] = d; sum += d;
     }
     return sum;
 }
 // this wavefront's tile of d_pre1 = (d_pre2 W2) f'(h1) into p1 (may be h1 itself); returns the lane's share of its unit's column sum
-template <int ACT_H>
-__device__ __forceinline__ float backward_layer2(const WNet& N, const BackOperands& W, lptr g2, lptr h1, lptr p1, int wave, int c, int g) {
+template <int ACT_H, bool LIVE = false>
+__device__ __forceinline__ float backward_layer2(const WNet& N, const BackOperands& W, lptr g2, lptr h1, lptr p1, int wave, int c, int g, int live = ROWS) {
     const int n = 16 * wave + c, tiles = (N.hid + 15) >> 4;
     const bool n_ok = n < N.hid;
     const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
@@ -267,7 +268,7 @@ __device__ __forceinline__ float backward_layer2(const WNet& N, const BackOperan
 #pragma unroll
     for (int v = 0; v < 4; v++) {
         const int idx = (4 * g + v) * S + n;
-        const float d = n_ok ? acc[v] * dact_hidden<ACT_H>(h1[idx], N.act_h) : 0.f;
+        const float d = n_ok && (!LIVE || 4 * g + v < live) ? acc[v] * dact_hidden<ACT_H>(h1[idx], N.act_h) : 0.f;
         p1[idx] = d; sum += d;
     }
     return sum;
@@ -747,7 +748,7 @@ __global__ __launch_bounds__(THREADS) void mlp_wide_kernel(MlpWideArgs A) {
         return;
     }
     if (PASS == MLP_FORWARD_BACKWARD) {
-        forward3<ACT_H, NT1C, false, true, false, EVERY>(N, W, N, xa, SXS, h1, h2, yp, wave, c, g);
+        forward3<ACT_H, NT1C, false, true, false, EVERY, BLOCKS>(N, W, N, xa, SXS, h1, h2, yp, wave, c, g, nullptr, B - row0);
         if (EVERY) request_given();      // (all of W fills the registers until here)
         load_back_operands<EVERY>(N, wave, c, g, K);
         if (!BLOCKS) {
@@ -772,7 +773,7 @@ __global__ __launch_bounds__(THREADS) void mlp_wide_kernel(MlpWideArgs A) {
         }
     }
     if (!BACKWARD_ONLY) rlt_lds_barrier();      // d_pre3 is in place (the backward pass alone: with the activations)
-    const float s2 = on ? backward_layer3<ACT_H>(N, K, d3, h2, ta, wave, c, g) : 0.f;
+    const float s2 = on ? backward_layer3<ACT_H, BLOCKS>(N, K, d3, h2, ta, wave, c, g, B - row0) : 0.f;
     if (BLOCKS) {
         float* const block = A.partial + (size_t)gi * A.count;
         float* const to_b1 = block + HID * IN; float* const to_w2 = to_b1 + HID; float* const to_b2 = to_w2 + HID * HID; float* const to_w3 = to_b2 + HID; float* const to_b3 = to_w3 + OUT * HID;
@@ -789,7 +790,7 @@ __global__ __launch_bounds__(THREADS) void mlp_wide_kernel(MlpWideArgs A) {
         if (spread ? !on && wave - tiles < tiles : on) last_layer(spread ? wave - tiles : wave);
         rlt_lds_barrier();      // every wavefront's tile of d_pre2 is in place
         if (on) {
-            const float s1 = backward_layer2<ACT_H>(N, K, ta, h1, tb, wave, c, g);
+            const float s1 = backward_layer2<ACT_H, BLOCKS>(N, K, ta, h1, tb, wave, c, g, B - row0);
             wave_sync();            // dW1's rows are this wavefront's own tile of d_pre1
 #pragma unroll 2
             for (int nt = 0; nt < (IN + 15) >> 4; nt++) gradient_tile(tb, wave, xa, SXS, nt, HID, IN, block, c, g);

@@ -159,3 +159,20 @@ def test_an_infinite_input_stays_in_its_column_and_infinite(rocm, B, row, H):
     infinite = np.zeros(grads.shape, bool)
     infinite[off:off + nw].reshape(H, 17)[:, 3] = True
     assert np.isinf(grads[infinite]).all() and np.isfinite(grads[~infinite]).all()
+
+
+@pytest.mark.parametrize("H", [72, 200])
+@pytest.mark.parametrize("B", [17, 300])
+def test_an_infinite_weight_that_the_activation_saturates_leaves_finite_gradients(oracle, rocm, B, H):
+    """The last tile's rows beyond the batch are zeros, which an infinite weight makes NaNs of; they are no part of the batch. One unit of the first hidden layer reads one
+    positive input through an infinite weight: its tanh is one and its derivative zero in every row, and no gradient is infinite."""
+    dims = [17, H, H, 6]
+    rng = np.random.default_rng(B + H)
+    params = helpers.random_params(rng, dims)
+    params[:H * 17].reshape(H, 17)[5, 2] = np.inf
+    x, dy = rng.standard_normal((B, 17)).astype(np.float32), rng.standard_normal((B, 6)).astype(np.float32)
+    x[:, 2] = np.abs(x[:, 2]) + 0.1
+    ref = run(oracle, dims, params, x, dy, "tanh", False, 0.0)
+    got = run(rocm, dims, params, x, dy, "tanh", False, 0.0)
+    assert np.isfinite(ref[1]).all() and np.isfinite(got[1]).all()
+    assert rel_err(got[0], ref[0]) <= TOL and rel_err(got[1], ref[1]) <= TOL
