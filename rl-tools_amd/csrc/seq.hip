@@ -44,6 +44,15 @@ bool carve(const rlt_seq_layer* layers, int n, int steps, int batch, void* works
     return true;
 }
 
+// Whether the input's gradient goes on top of what the weight gradients still read: the layers one after the other have read the loss gradient and the input before it is
+// written; the passes of all layers in one launch are followed by the weight gradients of all layers.
+bool overlap(const float* a, size_t na, const float* b, size_t nb) { return (uintptr_t)a < (uintptr_t)(b + nb) && (uintptr_t)b < (uintptr_t)(a + na); }
+bool in_place(const rlt_seq_layer* layers, int n, const float* x, int ldx, const float* d_output, const float* d_input, size_t rows, int want_w) {
+    if (!d_input) return false;
+    const size_t in = layer_in(layers[0]);
+    return overlap(d_input, rows * in, d_output, rows * layer_out(layers[n - 1])) || (want_w && overlap(d_input, rows * in, x, (rows - 1) * ldx + in));
+}
+
 // ---- rollout state of the GRU layers (nn/layers/gru/layer.h State) ---------------------------------------------------------------
 __global__ __launch_bounds__(256) void seq_reset_state_kernel(float* __restrict__ hidden, uint32_t* __restrict__ step, const float* __restrict__ h0,
                                                               const uint8_t* __restrict__ mask, int batch, int H) {
@@ -138,7 +147,8 @@ int rlt_rocm_seq_backward(rlt_rocm_device* device, const rlt_seq_layer* layers, 
     const int rows = steps * batch;
     // backward and backward_full hand the mode to every layer; backward_input hands it on only when the model has a single layer
     const uint8_t* reset_here = (want_w || reset_in_backward_input || n == 1) ? reset : nullptr;
-    if (rlt_seq_stack_faster(want_w ? RLT_STACK_WEIGHT_GRADIENTS : RLT_STACK_PASS, steps, batch) && rlt_seq_stack_supported(layers, n, steps) && (want_w || d_input)) {
+    if (rlt_seq_stack_faster(want_w ? RLT_STACK_WEIGHT_GRADIENTS : RLT_STACK_PASS, steps, batch) && rlt_seq_stack_supported(layers, n, steps) && (want_w || d_input) &&
+        !in_place(layers, n, x, ldx, d_output, d_input, rows, want_w)) {
         const rlt_stack_backward pass = {layers, x, ldx, d_output, d_input, reset_here, steps, batch, want_w, 0, (void*)(((uintptr_t)workspace + 255) & ~(uintptr_t)255)};
         return rlt_seq_stack_backward(device, &pass, 1);
     }

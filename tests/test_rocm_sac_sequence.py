@@ -116,6 +116,33 @@ def test_recurrent_approximators_in_one_launch_match_checker(oracle, rocm, case,
     model_against_checker(oracle, rocm, rng, specs, with_initial_states(rng, specs, helpers.random_seq_params(rng, specs)), S, B, fast, with_reset)
 
 
+@pytest.mark.parametrize("place", ["loss gradient", "input", "row behind the loss gradient"])
+@pytest.mark.parametrize("want_w", [1, 0])
+@pytest.mark.parametrize("H", [16, 32])
+def test_the_gradient_of_a_recurrent_approximators_input_may_replace_what_it_was_formed_from(rocm, H, want_w, place):
+    """d_input in the memory of d_output or of x, or over rows of d_output that other rows of the batch come to later: the results of the call with memory of its own. The
+    tolerance is that of the cases above (the call takes the layers one after the other then, other sums in fp32)."""
+    S, B, I, O = 9, 21, 5, 5
+    rng = np.random.default_rng(H + want_w)
+    specs = [(0, I, H, "relu"), (1, H, H, "identity"), (1, H, H, "identity"), (0, H, O, "identity")]
+    params = with_initial_states(rng, specs, helpers.random_seq_params(rng, specs))
+    x, g = rng.standard_normal((S, B, I)).astype(np.float32), rng.standard_normal((S, B, O)).astype(np.float32)
+    res = []
+    for apart in (True, False):
+        net = helpers.SeqNet(rocm, specs, params, S, B)
+        ws, wsn = net.workspace()
+        xd, gd = rocm.array(x), rocm.array(np.concatenate([g.ravel(), np.zeros(B * O, np.float32)]))
+        own = rocm.zeros((S, B, I))
+        rocm.call("seq_forward", net.layers, net.n, xd.ptr, I, None, S, B, ws, wsn)
+        to = own.ptr if apart else xd.ptr if place == "input" else gd.ptr if place == "loss gradient" else gd.offset(O)
+        rocm.call("seq_backward", net.layers, net.n, xd.ptr if want_w else None, I, gd.ptr, to, None, S, B, want_w, 0, ws, wsn)
+        rocm.sync()
+        dx = own.numpy().ravel() if apart else xd.numpy().ravel() if place == "input" else gd.numpy().ravel()[(0 if place == "loss gradient" else O):][:S * B * I]
+        res.append((dx.copy(), net.grads.numpy()))
+    assert rel_err(res[1][0], res[0][0]) <= TOL and rel_err(res[1][1], res[0][1]) <= TOL, (rel_err(res[1][0], res[0][0]), rel_err(res[1][1], res[0][1]))
+    assert np.abs(res[0][0]).max() > 0
+
+
 def stacked_agents(rng, backends, S, B, OBS, ACT, actor_hidden, critic_hidden, first, spread=1.0):
     """SAC agents whose networks are all dense, GRU, GRU, dense"""
     specs = lambda i, h, o: [(0, i, h, "relu"), (1, h, h, "identity"), (1, h, h, "identity"), (0, h, o, "identity")]
