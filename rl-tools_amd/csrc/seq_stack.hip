@@ -128,7 +128,7 @@ __device__ __forceinline__ float product_sum3(const Weights3<H>& R, float x, flo
         multiply<H>(R, x, y, z, acc, std::make_integer_sequence<int, 15>{});
         return sum_parts<2>(acc[0] + (acc[1] + acc[2]));
     }
-    float own = p == 0 ? x : p == 1 ? y : z;
+    float own = p == 0 ? x : p == 1 ? y : p == 2 ? z : 0.f;      // the fourth row of lanes has zero weights, and zero times an infinity is not zero
     wait_for_dpp(own);
     multiply<H>(R, own, own, own, acc, std::make_integer_sequence<int, 15>{});
     return sum_parts<4>(acc[0]);

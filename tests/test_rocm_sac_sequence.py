@@ -143,6 +143,30 @@ def test_the_gradient_of_a_recurrent_approximators_input_may_replace_what_it_was
     assert np.abs(res[0][0]).max() > 0
 
 
+@pytest.mark.parametrize("want_w", [1, 0])
+@pytest.mark.parametrize("H", [16, 32])
+def test_an_infinite_gradient_of_a_recurrent_approximator_stays_infinite(oracle, rocm, H, want_w):
+    """One output weight makes one unit's gradient overflow; every gate's gradient has the same sign and every weight on the way to the input is positive, so that the input's
+    gradient is plus infinity everywhere (lanes without a gate that multiplied it by a zero weight made NaNs of it)."""
+    S, B, I = 1, 3, 2
+    rng = np.random.default_rng(H)
+    specs = [(0, I, H, "identity"), (1, H, H, "identity"), (1, H, H, "identity"), (0, H, 1, "identity")]
+    parts = [rng.uniform(0.1, 0.2, I * H), np.zeros(H)]
+    for _ in range(2):      # n well below the initial state, the n gate's hidden part positive
+        parts += [rng.uniform(0.01, 0.02, 3 * H * H), np.concatenate([np.zeros(2 * H), np.full(H, -3.0)]), rng.uniform(0.01, 0.02, 3 * H * H), np.zeros(3 * H), np.full(H, 0.9)]
+    out = np.full(H, 1.0); out[3] = 1e30
+    params = np.concatenate(parts + [out, np.zeros(1)]).astype(np.float32)
+    x, g = rng.uniform(0.1, 1.0, (S, B, I)).astype(np.float32), np.full((S, B, 1), 1e20, np.float32)
+    for be in (oracle, rocm):
+        net = helpers.SeqNet(be, specs, params, S, B)
+        ws, wsn = net.workspace()
+        xd, gd, dx = be.array(x), be.array(g), be.zeros((S, B, I))
+        be.call("seq_forward", net.layers, net.n, xd.ptr, I, None, S, B, ws, wsn)
+        be.call("seq_backward", net.layers, net.n, xd.ptr if want_w else None, I, gd.ptr, dx.ptr, None, S, B, want_w, 0, ws, wsn)
+        be.sync()
+        assert (dx.numpy() == np.inf).all(), (be.name, dx.numpy())
+
+
 def stacked_agents(rng, backends, S, B, OBS, ACT, actor_hidden, critic_hidden, first, spread=1.0):
     """SAC agents whose networks are all dense, GRU, GRU, dense"""
     specs = lambda i, h, o: [(0, i, h, "relu"), (1, h, h, "identity"), (1, h, h, "identity"), (0, h, o, "identity")]
