@@ -319,7 +319,7 @@ int rlt_adam_step_pair(rlt_rocm_device* device, const rlt_adam_tensor* tensors_a
                        const rlt_adam_tensor* tensors_b, int n_b, const rlt_adam_parameters* parameters_b, uint32_t* age_b,
                        const rlt_adam_source* source_a, const rlt_adam_source* source_b, float polyak) {
     RLT_REQUIRE(tensors_a && tensors_b && n_a > 0 && n_b > 0 && parameters_a && parameters_b && age_a && age_b);
-    if (n_a > MAX_T || n_b > MAX_T) {
+    if (n_a > MAX_T || n_b > MAX_T || (age_a == age_b && !source_a && !source_b)) {      // (optimisers that share an age: the second steps with the age that the first leaves)
         RLT_REQUIRE(!source_a && !source_b);
         const int rc = adam_launch(device, tensors_a, n_a, parameters_a, age_a, 0.0f, nullptr, false);
         return rc ? rc : adam_launch(device, tensors_b, n_b, parameters_b, age_b, 0.0f, nullptr, false);

@@ -224,6 +224,28 @@ def test_both_critics_of_recurrent_approximators_in_one_call_leave_the_bits_of_t
     assert np.abs(agents[1].parameters() - params).max() > 1e-4
 
 
+@pytest.mark.parametrize("shared", ["critics", "actor and alpha"])
+def test_optimisers_of_recurrent_approximators_that_share_an_age_step_one_after_the_other(rocm, shared):
+    """One call for both critics against the two calls, and the actor's step against a copy whose ages are apart: where two optimisers count in one place the second goes on from
+    the first's count, as two steps in a row do."""
+    S, B, OBS, ACT = 7, 13, 5, 2
+    rng = np.random.default_rng(11)
+    _, agents = stacked_agents(rng, (rocm, rocm), S, B, OBS, ACT, 16, 32, False)
+    data = synthetic_sequence_batch(rng, S, B, OBS + ACT)
+    nc, na = rng.standard_normal((S, B, ACT)).astype(np.float32), rng.standard_normal((S, B, ACT)).astype(np.float32)
+    for a, together in zip(agents, (False, True)):
+        a.set_batch(data)
+        if shared == "critics":
+            a.c.critic_age[1] = a.c.critic_age[0]
+        elif together:
+            a.c.alpha_age = a.c.actor_age
+        else:
+            a.alpha_age.upload(np.array([2], np.uint32))
+        a.train(nc, na, both_critics_in_one_call=together)
+    assert np.array_equal(agents[0].parameters(), agents[1].parameters())
+    assert [a.ages()[1 if shared == "critics" else 0] for a in agents] == ([3, 3] if shared == "critics" else [2, 3])
+
+
 @pytest.mark.parametrize("n_layers", [3, 5])
 def test_sac_sequence_updates_against_reference_vectors(oracle, rocm, n_layers):
     """The reference's own run (fixture): every loop step on the device from the checker's state, compared after the step in gradients,
