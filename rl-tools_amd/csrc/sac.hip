@@ -577,12 +577,14 @@ size_t rlt_rocm_sac_sequence_workspace_bytes(const rlt_sac_sequence_agent* A) {
 // Agents whose networks are the reference's recurrent approximators (seq_stack.hip): a launch takes every layer of a pass, and the passes that do not depend on each other
 // share one. The trained critics' loss gradients and backward passes follow, then their optimisers in one launch.
 static bool sequence_agent_stacked(const rlt_sac_sequence_agent* A) {
-    const int T = A->batch.sequence_length + 1;
-    if (!rlt_seq_stack_faster(RLT_STACK_UPDATE, A->batch.sequence_length, A->batch.batch)) return false;
+    const int T = A->batch.sequence_length + 1, B = A->batch.batch;
+    if (!rlt_seq_stack_faster(RLT_STACK_UPDATE, A->batch.sequence_length, B)) return false;
     if (!rlt_seq_stack_supported(A->actor, A->n_actor_layers, T)) return false;
     for (int k = 0; k < 2; k++)
         if (!rlt_seq_stack_supported(A->critics[k], A->n_critic_layers, T) || !rlt_seq_stack_supported(A->critics_target[k], A->n_critic_layers, T)) return false;
-    return true;
+    // the workspace is sized by the first critic and its target: of a wider second one the passes below, which look at their share of it, refuse what does not fit
+    const size_t share = sequence_pass_workspace_bytes(A, T, B);
+    return rlt_rocm_seq_workspace_bytes(A->critics[1], A->n_critic_layers, T, B) <= share && rlt_rocm_seq_workspace_bytes(A->critics_target[1], A->n_critic_layers, T, B) <= share;
 }
 static int sequence_next_actions(rlt_rocm_device* device, const rlt_sac_sequence_agent* A, const float* base_next, const uint8_t* next_final, int rows, const float* action_noise) {
     SequenceActions a = {};

@@ -246,6 +246,20 @@ def test_optimisers_of_recurrent_approximators_that_share_an_age_step_one_after_
     assert [a.ages()[1 if shared == "critics" else 0] for a in agents] == ([3, 3] if shared == "critics" else [2, 3])
 
 
+def test_a_second_critic_wider_than_the_workspace_is_sized_for_is_refused(rocm):
+    S, B, OBS, ACT = 7, 13, 3, 1
+    rng = np.random.default_rng(12)
+    agent, wide = (stacked_agents(rng, (rocm,), S, B, OBS, ACT, 16, width, False)[1][0] for width in (16, 32))
+    noise = rocm.array(rng.standard_normal((S, B, ACT)).astype(np.float32))
+    lib, h = rocm.device.lib, rocm.device.handle
+    agent.set_batch(synthetic_sequence_batch(rng, S, B, OBS + ACT))
+    agent.c.critics[1], agent.c.critic_adam_tensors[1] = wide.critics[1].layers, wide.critics[1].adam
+    assert lib.rlt_rocm_sac_sequence_train_critics(h, C.byref(agent.c), noise.ptr) == helpers.capi.RLT_E_INVALID_ARGUMENT
+    assert lib.rlt_rocm_sac_sequence_train_critic(h, C.byref(agent.c), 1, noise.ptr) == helpers.capi.RLT_E_INVALID_ARGUMENT
+    assert lib.rlt_rocm_sac_sequence_train_actor(h, C.byref(agent.c), noise.ptr) == helpers.capi.RLT_E_INVALID_ARGUMENT
+    rocm.sync()
+
+
 @pytest.mark.parametrize("n_layers", [3, 5])
 def test_sac_sequence_updates_against_reference_vectors(oracle, rocm, n_layers):
     """The reference's own run (fixture): every loop step on the device from the checker's state, compared after the step in gradients,
