@@ -187,7 +187,7 @@ int rlt_rocm_mlp_zero_gradient(rlt_rocm_device* device, const rlt_dense_layer* l
 
 /* Fused forward + backward of a whole MLP for a caller that already holds the upstream gradient
  * (the standalone microbenchmark shape, and PPO's critic where d_output = mse gradient is fused via
- * `target`): one pass over the batch, activations never leave the chip.
+ * `target`): one pass over the batch; wide networks over up to 4,096 rows keep its activations in the handle's scratch for the weight gradients.
  *   y           [batch x out] network output (may be NULL)
  *   d_output    [batch x out] upstream gradient, used when target == NULL (not modified)
  *   target      if non-NULL, d_output is formed as (y - target) * mse_scale instead

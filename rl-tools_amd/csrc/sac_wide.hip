@@ -1142,7 +1142,9 @@ static int mlp_wide_launch(rlt_rocm_device* device, const rlt_dense_layer* L, in
     rlt_gradient_net net = {};
     net.in = IN; net.hid = hid; net.out = OUT;
     float* partial = nullptr;
-    const bool blocks = !forward_only && sum_blocks(hid, IN, batch);
+    // (an output in the memory of the input leaves the contraction over the whole batch without its operand; the blocks are formed out of LDS)
+    const bool in_place = y && (uintptr_t)y < (uintptr_t)(x + (size_t)(batch - 1) * ldx + IN) && (uintptr_t)x < (uintptr_t)(y + (size_t)(batch - 1) * ldy + OUT);
+    const bool blocks = !forward_only && (sum_blocks(hid, IN, batch) || in_place);
     const int exact = hid * IN + hid + hid * hid + hid + OUT * hid + OUT;
     if (blocks) {
         void* scratch = nullptr;

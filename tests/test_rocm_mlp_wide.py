@@ -82,6 +82,30 @@ def test_gradients_accumulate_and_the_output_may_be_null(oracle, rocm):
     assert rel_err(twice[1], ref[1]) <= TOL
 
 
+@pytest.mark.parametrize("B,H", [(256, 256), (300, 200), (1025, 128), (4096, 250)])
+def test_the_output_may_replace_the_input(rocm, B, H):
+    """y in the memory of x, in layers as wide as the output and in rows farther apart: outputs and gradients are those of the call with memory of its own."""
+    rng = np.random.default_rng(B)
+    for I, O, ld in ((6, 6, 6), (17, 3, 20)):
+        dims = [I, H, H, O]
+        params = helpers.random_params(rng, dims)
+        x, dy = rng.standard_normal((B, ld)).astype(np.float32), rng.standard_normal((B, O)).astype(np.float32)
+        res = []
+        for apart in (True, False):
+            net = Mlp(rocm, dims, params, B, "relu", "identity")
+            xd, yd, dyd = rocm.array(x), rocm.zeros((B, ld)), rocm.array(dy)
+            ws, wsn = net.workspace()
+            rocm.call("mlp_zero_gradient", net.layers, net.n)
+            y = yd if apart else xd
+            rocm.call("mlp_forward_backward", net.layers, net.n, xd.ptr, ld, y.ptr, ld, dyd.ptr, O, None, 0, 0.0, B, ws, wsn)
+            rocm.sync()
+            res.append((y.numpy()[:, :O], net.grads.numpy(), net.offsets))
+        assert np.array_equal(res[0][0], res[1][0])
+        for off, nw, nb in res[0][2]:
+            for at, n in ((off, nw), (off + nw, nb)):
+                assert rel_err(res[1][1][at:at + n], res[0][1][at:at + n]) <= TOL, (I, off, rel_err(res[1][1][at:at + n], res[0][1][at:at + n]))
+
+
 def test_the_call_takes_the_sixteen_row_tiles_where_this_file_says_so(rocm, monkeypatch):
     """Which path ran: the sixteen-row tiles and the path the call takes without them (RLT_MLP_WIDE=0) agree to tolerance but not bit for bit."""
     dims = [17, 256, 256, 6]
