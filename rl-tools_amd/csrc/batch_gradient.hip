@@ -95,7 +95,7 @@ __global__ __launch_bounds__(THREADS) void batch_gradient_kernel(GradientLaunch 
         }
         if (N.step) rlt_adam_bias_corrections(N.adam, *N.age, bc1, bc2);
     }
-    const bool is_void = !SPLIT && void_update(K.guard);
+    const bool is_void = !SPLIT && N.step && void_update(K.guard);
     floatx4 c[TM / 16][2];
     float bias[TM / 16];
     tile_product<TM / 16>(a, lda, rows, TM * mt, b, ldb, cols, TN * nt, B, k0, k1, r, g, c, bias);
