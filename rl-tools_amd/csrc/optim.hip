@@ -176,7 +176,13 @@ __device__ __forceinline__ void adam_body(const AdamLaunch& a, uint32_t block, u
     if ((threadIdx.x & 63) == 0) partial[threadIdx.x >> 6] = sq;
     __syncthreads();
     if (threadIdx.x == 0) {
-        a.block_partials[block] = partial[0] + partial[1] + partial[2] + partial[3];
+        const float own = partial[0] + partial[1] + partial[2] + partial[3];
+        if (n_blocks == 1) {      // nobody else's sum to wait for
+            *a.out_sq_norm = (a.accumulate_norm ? *a.out_sq_norm : 0.0f) + own;
+            if (a.increment_age) *a.age = age + 1;
+            return;
+        }
+        a.block_partials[block] = own;
         __threadfence();
         if (rlt_last_through(a.tickets, block, n_blocks)) {
             __threadfence();

@@ -9,7 +9,7 @@ import helpers
 from helpers import capi
 
 pytestmark = pytest.mark.gpu
-COUNTS = {"ragged": [5, 1, 1023, 1024, 1025, 3, 256], "network": [17 * 256, 256, 256 * 256, 256, 6 * 256, 6], "many": [130] * 37, "one": [1], "large": [1_500_001, 7]}
+COUNTS = {"ragged": [5, 1, 1023, 1024, 1025, 3, 256], "network": [17 * 256, 256, 256 * 256, 256, 6 * 256, 6], "many": [130] * 37, "one": [1], "sixteen workgroups": [16 * 1024], "seventeen": [16 * 1024 + 1], "large": [1_500_001, 7]}
 
 
 def step(rocm, counts, apart, parameters, arrays):
