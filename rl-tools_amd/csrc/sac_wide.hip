@@ -79,10 +79,13 @@ template <int ACT_H> __device__ __forceinline__ float dact_hidden(float o, int f
 // (forward copies of the first and second layers) or W[16 j + 4 g ... + 3][16 w + c] (backward copy of the second), zero beyond the layer's shape, and a wavefront's
 // load is 1 KB of consecutive addresses. Straight from W a lane's 16 bytes lie a row apart from its neighbour's: 64 lines per load, which the compute unit's address
 // pipeline takes 64 cycles for; first layers whose rows are no multiple of 16 bytes (17 or 35 inputs) take four such loads per chunk, 5 us at the start of a launch.
-// What a wavefront will not use (chunks beyond the width, everything where it has no units) is asked for at one address by all lanes, which costs the address pipeline a cycle or two
-// instead of sixteen: at width 65 eleven of sixteen wavefronts and eleven of sixteen chunks are such.
-// EVERY: where every wavefront has units there is nothing to leave out, and the selects cost more than they save (forward + backward of 256 units 36.2 us with them, 35.4 without).
-template <int JN, bool EVERY = false>
+// A wavefront without units asks for nothing, the others for chunks in groups of STEP up to the width; within a group, chunks beyond it are asked for at one address by all lanes. A load
+// that nobody uses still takes sixteen cycles of a compute unit's return path: at width 65, with all sixteen wavefronts asking for all chunks, 224 of 288 were such (SAC's
+// actor update at width 65 over 600 rows 32.5 -> 29.0 us, update set at width 32 over 100 rows 47.3 -> 41.2, forward + backward of 17-48-48-6 at 256 rows 12.5 -> 10.9). The first layer's few chunks one by one.
+// EVERY: where every wavefront has units and all sixteen chunks of the second layer are there, there is nothing to leave out, and the selects cost more than they save (forward +
+// backward of 256 units 36.2 us with them, 35.4 without; SAC's update set 86.2 and 86.0).
+template <int NT1C> constexpr int FIRST_STEP = NT1C <= FEW ? 1 : 4;      // (five chunks and more: the branches cost more)
+template <int JN, bool EVERY = false, int STEP = 4>
 __device__ __forceinline__ void load_swizzled(const float* __restrict__ copy, int tiles, bool on, int wave, int lane, int j0, floatx4 (&b)[JN]) {      // tiles: chunks of the copy; on: this wavefront has units
     if (EVERY) {
         const float* const mine = copy + ((size_t)wave * tiles * 64 + lane) * 4;
@@ -90,10 +93,15 @@ __device__ __forceinline__ void load_swizzled(const float* __restrict__ copy, in
         for (int j = 0; j < JN; j++) b[j] = *reinterpret_cast<const floatx4*>(mine + (size_t)min(j0 + j, tiles - 1) * 256);
         return;
     }
+    if (!on) return;
     const uint32_t mine = ((uint32_t)wave * tiles * 64 + lane) * 16;
 #pragma unroll
-    for (int j = 0; j < JN; j++)
-        b[j] = *reinterpret_cast<const floatx4*>(reinterpret_cast<const char*>(copy) + (on && j0 + j < tiles ? mine + (uint32_t)(j0 + j) * 1024 : 0));
+    for (int q = 0; q < JN; q += STEP) {
+        if (j0 + q >= tiles) return;
+#pragma unroll
+        for (int j = q; j < q + STEP && j < JN; j++)
+            b[j] = *reinterpret_cast<const floatx4*>(reinterpret_cast<const char*>(copy) + (j0 + j < tiles ? mine + (uint32_t)(j0 + j) * 1024 : 0));
+    }
 }
 // acc += in[rows][16 (j0 + j) + ...] * b[j], the workgroup's 16 rows against this lane's column
 template <int JN>
@@ -140,7 +148,8 @@ template <int NT1C, bool EVERY = false>
 __device__ __forceinline__ void load_operands(const WNet& N, int wave, int c, int g, Operands<NT1C>& W) {
     const int n = 16 * wave + c, tiles = (N.hid + 15) >> 4, lane = c + 16 * g;
     const bool on = wave < tiles;
-    load_swizzled<NT1C, EVERY>(N.W1f, (N.in + 15) >> 4, on, wave, lane, 0, W.w1);
+    if (!EVERY && !on) return;
+    load_swizzled<NT1C, false, FIRST_STEP<NT1C>>(N.W1f, (N.in + 15) >> 4, on, wave, lane, 0, W.w1);
     W.b1 = N.b1[min(n, N.hid - 1)]; W.b2 = N.b2[min(n, N.hid - 1)];
     load_swizzled<8, EVERY>(N.W2f, tiles, on, wave, lane, 0, W.w2a);
     if (NT1C <= FEW) load_swizzled<8, EVERY>(N.W2f, tiles, on, wave, lane, 8, W.w2b);
@@ -177,7 +186,7 @@ __device__ __forceinline__ void forward3(const WNet& N, Operands<NT1C>& W, const
     const int n = 16 * wave + c, tiles = (N.hid + 15) >> 4, lane = c + 16 * g, next_tiles = (next.hid + 15) >> 4;
     const bool on = wave < tiles, next_on = wave < next_tiles;
     const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
-    if (!W1_READY) load_swizzled<NT1C, EVERY>(N.W1f, (N.in + 15) >> 4, on, wave, lane, 0, W.w1);
+    if (!W1_READY) load_swizzled<NT1C, false, FIRST_STEP<NT1C>>(N.W1f, (N.in + 15) >> 4, on, wave, lane, 0, W.w1);
     if (on) {
         floatx4 a0 = zero4, a1 = zero4;
         chunks<NT1C>(a0, a1, x, xstride, c, g, 0, (N.in + 15) >> 4, W.w1);
@@ -185,7 +194,7 @@ __device__ __forceinline__ void forward3(const WNet& N, Operands<NT1C>& W, const
     }
     if (NT1C > FEW) load_swizzled<8, EVERY>(N.W2f, tiles, on, wave, lane, 8, W.w2b);
     if (PREFETCH) {
-        if (NT1C <= FEW) load_swizzled<NT1C, EVERY>(next.W1f, (next.in + 15) >> 4, next_on, wave, lane, 0, W.w1);
+        if (NT1C <= FEW) load_swizzled<NT1C, false, FIRST_STEP<NT1C>>(next.W1f, (next.in + 15) >> 4, next_on, wave, lane, 0, W.w1);
         W.b1 = next.b1[min(n, next.hid - 1)];
     }
     rlt_lds_barrier();
@@ -289,7 +298,7 @@ __device__ __forceinline__ void gradient_tile(lptr d, int mt, lptr x, int stride
 template <int N>
 __device__ __forceinline__ void request_row(const float* row, int cols, int lane, float (&v)[N]) {
 #pragma unroll
-    for (int u = 0; u < N; u++) v[u] = row[min(64 * u + lane, cols - 1)];
+    for (int u = 0; u < N; u++) { v[u] = 0.f; if (64 * u < cols) v[u] = row[min(64 * u + lane, cols - 1)]; }
 }
 template <int N>
 __device__ __forceinline__ void place_row(lptr to, bool ok, int cols, int end, int lane, const float (&v)[N]) {
@@ -377,7 +386,8 @@ struct Copies {
 };
 constexpr size_t MAX_COPY_FLOATS = (size_t)WAVES * (MAX_H / 16) * 256, MAX_W1_COPY_FLOATS = (size_t)WAVES * (MAX_D / 16) * 256;
 
-template <int MODE, int ACT_H, int NT1C>
+// EVERY: all networks have more than 240 units
+template <int MODE, int ACT_H, int NT1C, bool EVERY>
 __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
     constexpr bool CRITIC = MODE == MODE_CRITIC || MODE == MODE_TD3_CRITIC, TD3 = MODE == MODE_TD3_CRITIC || MODE == MODE_TD3_ACTOR;
     extern __shared__ __attribute__((aligned(16))) float lds_wide[];
@@ -413,7 +423,7 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
         const Trained T = y ? A.trained[1] : A.trained[0];
         const int HID = trained.hid, tiles = (HID + 15) >> 4;
         Operands<NT1C> W;
-        load_operands<NT1C>(trained, wave, c, g, W);
+        load_operands<NT1C, EVERY>(trained, wave, c, g, W);
         place_row(xa + wave * SXS, row0 + wave < B, D, SXS, lane, in_row);
         float reward[4] = {0.f, 0.f, 0.f, 0.f}, alpha = 0.f, b3 = 0.f;
         bool terminated[4] = {false, false, false, false};
@@ -425,10 +435,10 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
         }
         rlt_lds_barrier();      // the input rows are in place
         RLT_TICK(1);
-        forward3<ACT_H, NT1C, false, true>(trained, W, trained, xa, SXS, h1, h2, yp, wave, c, g);
+        forward3<ACT_H, NT1C, false, true, false, EVERY>(trained, W, trained, xa, SXS, h1, h2, yp, wave, c, g);
         RLT_TICK(2);
         BackOperands K;
-        load_back_operands(trained, wave, c, g, K);      // on their way while the targets' values are waited for
+        load_back_operands<EVERY>(trained, wave, c, g, K);      // on their way while the targets' values are waited for
         store_rows(h1, T.h1, HID, row0, B, wave, lane);
         store_rows(h2, T.h2, HID, row0, B, wave, lane);
         if (scalar_wave) {
@@ -481,7 +491,7 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
     const bool writes = target_role ? role == 0 : owner;      // of the roles that compute the same sample, the one that stores what is asked for
     const WNet Q = CRITIC ? (critic_index ? A.target[1] : A.target[0]) : (critic_index ? A.critic[1] : A.critic[0]);
     Operands<NT1C> W;
-    load_operands<NT1C>(A.actor, wave, c, g, W);      // on their way while the input rows are written
+    load_operands<NT1C, EVERY>(A.actor, wave, c, g, W);      // on their way while the input rows are written
     place_row(xa + wave * SXS, row0 + wave < B, OBS, SXS, lane, in_row);
     float noise[2] = {0.f, 0.f}, target_noise[2] = {0.f, 0.f}, alpha = 0.f, actor_b3 = 0.f, q_b3 = 0.f;
     if (scalar_wave) {
@@ -515,7 +525,7 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
     RLT_TICK(13);
     rlt_lds_barrier();      // the input rows are in place
     RLT_TICK(5);
-    forward3<ACT_H, NT1C, true, true>(A.actor, W, Q, xa, SXS, h1, h2, yp, wave, c, g);
+    forward3<ACT_H, NT1C, true, true, false, EVERY>(A.actor, W, Q, xa, SXS, h1, h2, yp, wave, c, g);
     RLT_TICK(6);
     if (scalar_wave) {
         const floatx4 out = output_tile(yp, (A.actor.hid + 15) >> 4, c, g);
@@ -546,7 +556,7 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
     }
     rlt_lds_barrier();      // the action columns of xa are in place
     RLT_TICK(7);
-    forward3<ACT_H, NT1C, false, NT1C <= FEW>(Q, W, Q, xa, SXS, ta, tb, yp, wave, c, g);
+    forward3<ACT_H, NT1C, false, NT1C <= FEW, false, EVERY>(Q, W, Q, xa, SXS, ta, tb, yp, wave, c, g);
     RLT_TICK(8);
     const int qtiles = (Q.hid + 15) >> 4;
     if (CRITIC) {
@@ -561,7 +571,7 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
     // ---- actor update: the gradient of -value / batch with respect to the action (TD3: critic 0 only, rl/algorithms/td3/operations_generic.h:260)
     const float loss_weight = (1.0f / (float)B) * -1.0f;       // rl/algorithms/sac/operations_generic.h:437-453 with n = batch rows
     BackOperands K;
-    load_back_operands(Q, wave, c, g, K);
+    load_back_operands<EVERY>(Q, wave, c, g, K);
     float w1[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) { const int unit = 16 * wave + 4 * g + i; w1[i] = (c < ACT && unit < Q.hid) ? Q.W1[(size_t)unit * D + OBS + c] : 0.f; }
@@ -602,7 +612,7 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
     const WNet trained = A.actor;
     const Trained T = A.trained[0];
     const int HID = trained.hid, tiles = (HID + 15) >> 4;
-    load_back_operands(trained, wave, c, g, K);
+    load_back_operands<EVERY>(trained, wave, c, g, K);
     store_rows(h1, T.h1, HID, row0, B, wave, lane);
     store_rows(h2, T.h2, HID, row0, B, wave, lane);
     if (scalar_wave) {
@@ -963,14 +973,22 @@ int launch_wide(rlt_rocm_device* device, WideArgs& a, int groups, const Optimise
     a.by_xcd = device->update_one_xcd && device->xcd_stride == 8 && a.roles * groups <= device->compute_units;
     const size_t lds_bytes = LDS_FLOATS * sizeof(float);
     const dim3 grid(a.by_xcd ? 8 * rlt_div_up(a.roles * groups, 8) : a.roles * groups);
-#define RLT_LAUNCH_WIDE(ACT, NT)                                                                                                                          \
+#define RLT_LAUNCH_WIDE(ACT, NT, EVERY)                                                                                                                   \
     do {                                                                                                                                                  \
-        RLT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(sac_wide_kernel<MODE, ACT, NT>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes)); \
-        hipLaunchKernelGGL((sac_wide_kernel<MODE, ACT, NT>), grid, dim3(THREADS), lds_bytes, device->stream, a);                                          \
+        RLT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(sac_wide_kernel<MODE, ACT, NT, EVERY>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes)); \
+        hipLaunchKernelGGL((sac_wide_kernel<MODE, ACT, NT, EVERY>), grid, dim3(THREADS), lds_bytes, device->stream, a);                                   \
     } while (0)
     int act = a.actor.act_h;
-    for (int k = 0; k < 2; k++) if (a.critic[k].act_h != act || a.target[k].act_h != act) act = -1;
-#define RLT_LAUNCH_WIDE_ACT(NT) do { if (act == RLT_ACT_RELU) RLT_LAUNCH_WIDE(RLT_ACT_RELU, NT); else if (act == RLT_ACT_FAST_TANH) RLT_LAUNCH_WIDE(RLT_ACT_FAST_TANH, NT); else RLT_LAUNCH_WIDE(-1, NT); } while (0)
+    bool every = a.actor.hid > MAX_H - 16;
+    for (int k = 0; k < 2; k++) {
+        if (a.critic[k].act_h != act || a.target[k].act_h != act) act = -1;
+        every = every && a.critic[k].hid > MAX_H - 16 && a.target[k].hid > MAX_H - 16;
+    }
+#define RLT_LAUNCH_WIDE_ACT(NT)                                                                                                                           \
+    do {                                                                                                                                                  \
+        if (act == RLT_ACT_RELU) { if (every) RLT_LAUNCH_WIDE(RLT_ACT_RELU, NT, true); else RLT_LAUNCH_WIDE(RLT_ACT_RELU, NT, false); }                    \
+        else if (act == RLT_ACT_FAST_TANH) RLT_LAUNCH_WIDE(RLT_ACT_FAST_TANH, NT, false); else RLT_LAUNCH_WIDE(-1, NT, false);                            \
+    } while (0)
     // the first layer's chunks that the code is unrolled for: up to 64 inputs they leave registers for all of a pass's weights at once
     if (a.obs + a.act <= 32) RLT_LAUNCH_WIDE_ACT(2); else if (a.obs + a.act <= 64) RLT_LAUNCH_WIDE_ACT(4); else RLT_LAUNCH_WIDE_ACT(MAX_D / 16);
 #undef RLT_LAUNCH_WIDE_ACT
