@@ -474,6 +474,79 @@ __global__ __launch_bounds__(256, 2) void gru_backward_mfma_kernel(GruArgs A) {
     if (A.db_hn_partial) gru_at(A.db_hn_partial + (size_t)b0 * H, at) = db_hn;
 }
 
+// The same for batches whose steps are bound by memory instead of the chain: thread (w, lane) finishes (row w, unit lane), so that a wavefront's loads and stores are whole rows
+// of 256 bytes (above: 64 bytes of each of four rows), and 106 instead of 145 registers leave room for four workgroups per compute unit instead of three. Wavefront w forms the
+// products of rows 48 w ... 48 w + 47 of W_h (lane = column) and the four partial sums of d h_prev meet in LDS: two workgroup barriers per step. Backward to the input, the kernel above / this
+// one: 16,384 sequences of 10 steps 181 / 157 us, 3,000 of 30 90.8 / 77.3, 1,500 of 100 173 / 157; but 2,048 of 30 52.0 / 53.2, 1,024 of 100 95 / 130.
+template <int ABID> __device__ __forceinline__ gru_floatx4 mfma4_all(float a, float b, gru_floatx4 c) { return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 4, ABID, 0); }      // every block's A from block ABID
+// 16 reduction steps: A register `a` holds, in block k, the four rows' values of reduction index base + k
+template <int... K> __device__ __forceinline__ void sixteen_steps(float a, const float* w, gru_floatx4 (&c)[4], std::integer_sequence<int, K...>) { ((c[K & 3] = mfma4_all<K>(a, w[K], c[K & 3])), ...); }
+__global__ __launch_bounds__(256) void gru_backward_rows_kernel(GruArgs A) {
+    constexpr int H = 64, D = 3, GS = 3 * H + 16;      // D: steps ahead that the saved values are requested; GS: row stride of the gate gradients in LDS, rows 16 banks apart
+    __shared__ float gs[GM_ROWS * GS];
+    __shared__ float part[4][GM_ROWS * 64];
+    const int u = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), S = A.S;
+    float wb[48];
+#pragma unroll
+    for (int k = 0; k < 48; k++) wb[k] = A.L.weights_hidden[(size_t)(48 * w + k) * H + u];
+    const bool live = blockIdx.x * GM_ROWS + w < A.B;
+    const int b = live ? blockIdx.x * GM_ROWS + w : A.B - 1;      // rows beyond the batch read the last row and store nothing
+    const float h0 = A.L.initial_hidden_state[u];
+    float carry = 0.f, db_hn = 0.f;
+    struct Saved { float r, z, n, npp, dy, hp; int restart; };
+    auto request = [&](int t) {      // steps before the first read the first again; the state is the one before the step (the first step's is not used)
+        const size_t at = (size_t)max(t, 0) * A.B + b;
+        const float* const post = A.L.post_activation + at * 3 * H + u;
+        Saved v = {post[0], post[H], post[2 * H], A.L.n_pre_pre_activation[at * H + u], A.d_output[at * H + u], A.L.output[((size_t)max(t - 1, 0) * A.B + b) * H + u], 0};
+        v.restart = t <= 0 || (A.reset && A.reset[at]);
+        return v;
+    };
+    Saved q[D];
+#pragma unroll
+    for (int d = 0; d < D; d++) q[d] = request(S - 1 - d);
+    for (int t = S - 1; t >= 0; t--) {
+        const size_t at = (size_t)t * A.B + b;
+        const Saved far = request(t - D), cur = q[0];
+        const float hp = cur.restart ? h0 : cur.hp;
+        const float dh = cur.dy + carry;
+        const float gz = dh * (hp - cur.n) * cur.z * (1.0f - cur.z);
+        const float gn = dh * (1.0f - cur.z) * (1.0f - cur.n * cur.n);
+        const float gr = gn * cur.npp * cur.r * (1.0f - cur.r);
+        const float gnr = gn * cur.r;
+        if (live) {
+            float* const bi = A.buffer_input + at * 3 * H + u; float* const bh = A.buffer_hidden + at * 3 * H + u;
+            A.d_output[at * H + u] = dh; A.h_previous[at * H + u] = hp;
+            bi[0] = gr; bi[H] = gz; bi[2 * H] = gn;
+            bh[0] = gr; bh[H] = gz; bh[2 * H] = gnr;
+        }
+        // the reference drops reset samples (t > 0) from the b_hn gradient (their buffer rows are zeroed before that sum, :716-749)
+        if (t == 0 || !cur.restart) db_hn += gnr;
+        gs[w * GS + u] = gr; gs[w * GS + H + u] = gz; gs[w * GS + 2 * H + u] = gnr;
+        rlt_lds_barrier();
+        const float* const ga = gs + (u & 3) * GS + 48 * w + (u >> 2);
+        const float a0 = ga[0], a1 = ga[16], a2 = ga[32];
+        const gru_floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+        gru_floatx4 c[4] = {zero, zero, zero, zero};
+        const auto steps = std::make_integer_sequence<int, 16>{};
+        sixteen_steps(a0, wb, c, steps); sixteen_steps(a1, wb + 16, c, steps); sixteen_steps(a2, wb + 32, c, steps);
+        const gru_floatx4 mine = (c[0] + c[1]) + (c[2] + c[3]);
+#pragma unroll
+        for (int row = 0; row < GM_ROWS; row++) part[w][64 * row + u] = mine[row];
+        rlt_lds_barrier();
+        const float sum = (part[0][64 * w + u] + part[1][64 * w + u]) + (part[2][64 * w + u] + part[3][64 * w + u]);
+        carry = cur.restart ? 0.f : dh * cur.z + sum;
+#pragma unroll
+        for (int d = 0; d + 1 < D; d++) q[d] = q[d + 1];
+        q[D - 1] = far;
+    }
+    if (live && A.db_hn_partial) A.db_hn_partial[(size_t)b * H + u] = db_hn;
+}
+// Which of the two: beyond three workgroups per compute unit, and beyond one where what the steps read and write (14 rows of 64 floats each) does not fit the 256 MB of last-level cache
+bool backward_by_rows(const rlt_rocm_device* device, int S, int B) {
+    const int units = device->compute_units > 0 ? device->compute_units : 256, blocks = rlt_div_up(B, GM_ROWS);
+    return blocks > 3 * units || (blocks > units && (size_t)S * B * 14 * 64 * sizeof(float) > (size_t)256 << 20);
+}
+
 // db_h[n part] += sum over batch rows of the per-row sums, db_h[r, z parts] = db_i[r, z parts] (the reference copies, :679-681).
 // One workgroup per hidden unit.
 __global__ __launch_bounds__(256) void gru_bias_hidden_kernel(const float* __restrict__ partial, int B, int H, const float* __restrict__ db_i, float* __restrict__ db_h) {
@@ -551,7 +624,8 @@ int rlt_rocm_gru_backward(rlt_rocm_device* device, const rlt_gru_layer* L, const
     a.h_previous = h_previous; a.db_hn_partial = want_weight_gradients ? db_hn_partial : nullptr; a.S = S; a.B = B; a.rows_per_group = rows_per_group(H);
     if (H == 64 || H == 32 || H == 16) {
         const dim3 grid(rlt_div_up(B, GRU_THREADS / H)), block(GRU_THREADS);
-        if (H == 64) hipLaunchKernelGGL(gru_backward_mfma_kernel, dim3(rlt_div_up(B, GM_ROWS)), block, 0, device->stream, a);
+        if (H == 64 && backward_by_rows(device, S, B)) hipLaunchKernelGGL(gru_backward_rows_kernel, dim3(rlt_div_up(B, GM_ROWS)), block, 0, device->stream, a);
+        else if (H == 64) hipLaunchKernelGGL(gru_backward_mfma_kernel, dim3(rlt_div_up(B, GM_ROWS)), block, 0, device->stream, a);
         else if (H == 32) hipLaunchKernelGGL(gru_backward_reg_kernel<32>, grid, block, 0, device->stream, a);
         else hipLaunchKernelGGL(gru_backward_reg_kernel<16>, grid, block, 0, device->stream, a);
     } else {

@@ -125,6 +125,18 @@ def test_gru_at_the_edges_of_the_blocks_of_steps(oracle, rocm, steps, batch, hid
         assert rel_err(got[k], want[k]) <= 2e-5, (k, rel_err(got[k], want[k]))
 
 
+@pytest.mark.parametrize("with_reset", [False, True])
+@pytest.mark.parametrize("case", [(1, 3072, 3, 64), (1, 3073, 3, 64), (5, 3074, 4, 64), (74, 1025, 2, 64), (73, 1025, 2, 64)])
+def test_gru_backward_on_both_sides_of_the_line_to_whole_rows(oracle, rocm, case, with_reset):
+    """Width 64: the last batch and sequences that go through the kernel of sixteen units per wavefront and the first through that of a row per wavefront (more than 3,072 rows; more than
+    1,024 and 256 MB of saved values and gradients), last workgroups of one, two and four rows, one step. Tolerance as for the long batch above."""
+    print("case", case, with_reset, flush=True)
+    S, B, I, H = case
+    want, got = run_pair(oracle, rocm, S, B, I, H, 36, with_reset)
+    for k in KEYS:
+        assert rel_err(got[k], want[k]) <= 2e-5, (k, rel_err(got[k], want[k]))
+
+
 @pytest.mark.parametrize("case", [(32, 64, 34, 64), (33, 63, 160, 64), (16, 129, 66, 33), (64, 256, 64, 50), (64, 257, 146, 64), (64, 256, 36, 16),
                                   (32, 64, 96, 64), (33, 63, 98, 43), (16, 129, 128, 43), (32, 65, 130, 64), (64, 1024, 34, 44)])
 def test_gru_at_the_edges_of_the_kernels_that_keep_a_layer_in_registers(oracle, rocm, case):
