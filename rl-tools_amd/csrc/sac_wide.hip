@@ -849,14 +849,17 @@ __global__ __launch_bounds__(256) void block_sum_kernel(BlockSum R) {
     float* const to = k == 0 ? R.gradient[0] : k == 1 ? R.gradient[1] : k == 2 ? R.gradient[2] : k == 3 ? R.gradient[3] : k == 4 ? R.gradient[4] : R.gradient[5];
     to[e - begin] += (quarter[0][lane] + quarter[1][lane]) + (quarter[2][lane] + quarter[3][lane]);
 }
-// Whether the workgroups' blocks are added up (else the weight gradients are a contraction over the whole batch of their own). Forward + backward with 17 inputs, blocks / contraction,
-// us: width 65 at 256 rows 16.7 / 19.4, 1,000 17.2 / 20.3, 4,096 21.1 / 25.9; width 100 at 256 19.0 / 20.5, 1,000 20.4 / 21.8, 4,096 27.0 / 28.1; width 128 at 64 20.4 / 19.2, at
-// 512 21.4 / 22.8, at 1,000 22.9 / 22.7; width 192 at 512 28.7 / 26.9. With 128 inputs, backward pass alone: width 64 at 256 14.9 / 15.2, 4,096 19.0 / 17.5. Width 112 with 40 inputs, backward
-// pass alone: 2,048 rows 19.6 / 23.2, 3,000 22.3 / 22.1, 4,096 25.0 / 23.9.
-bool sum_blocks(int hid, int in, int batch) {
+// Whether the workgroups' blocks are added up (else the weight gradients are a contraction over the whole batch of their own): where the network is narrow, and the batch not so long that
+// the blocks are many bytes; the backward pass alone, which has the activations in memory already, sooner goes the other way. Blocks / contraction, us, outputs 6. Forward + backward: 17-65 at
+// 256 rows 12.5 / 14.9, 4,096 16.5 / 21.2; 65-80 at 2,048 17.3 / 18.7; 17-100 at 64 14.2 / 14.5, 4,096 21.9 / 22.8; 17-112 at 4,096 23.2 / 23.3; 40-112 at 256 15.2 / 15.9, 2,048 19.7 / 19.3;
+// 17-128 at 128 15.9 / 15.0, 256 16.0 / 16.0, 512 16.6 / 18.1, 1,000 17.9 / 17.9; 60-128 at 512 17.9 / 18.4, 768 18.8 / 18.0; 20-144 at 512 20.5 / 21.0, 768 21.3 / 20.5; 17-160 at 512
+// 21.7 / 21.5. Backward alone: 17-65 at 4,096 14.0 / 17.1; 65-80 at 2,048 13.9 / 14.3; 17-100 at 64 11.6 / 11.2, 256 11.8 / 12.3, 2,048 15.1 / 14.8, 4,096 19.3 / 18.0; 17-112 at 1,000
+// 13.3 / 13.3, 2,048 15.7 / 15.0; 40-112 at 1,000 13.9 / 13.3; 17-128 at 300 13.2 / 13.1; 128-64 at 1,000 11.6 / 11.9, 4,096 17.6 / 15.9.
+bool sum_blocks(int hid, int in, int batch, bool backward_only) {
     const int products = hid * (hid + in);
-    if (hid <= 112 && products <= 18432) return batch <= 1024 || (in <= 64 && (int64_t)products * batch <= 62914560);
-    return products <= 24576 && batch > 256 && batch <= 768;
+    const int64_t work = (int64_t)products * batch;
+    if (backward_only) return products <= 15000 && work <= 24000000 && (batch > 128 || products <= 8192);
+    return products <= 15000 ? work <= 62914560 : products <= 24576 && batch > 256 && work <= 13000000;
 }
 
 bool hidden_ok(int a) { return a == RLT_ACT_RELU || a == RLT_ACT_TANH || a == RLT_ACT_FAST_TANH || a == RLT_ACT_SIGMOID; }
@@ -1162,7 +1165,7 @@ static int mlp_wide_launch(rlt_rocm_device* device, const rlt_dense_layer* L, in
     float* partial = nullptr;
     // (an output in the memory of the input leaves the contraction over the whole batch without its operand; the blocks are formed out of LDS)
     const bool in_place = y && (uintptr_t)y < (uintptr_t)(x + (size_t)(batch - 1) * ldx + IN) && (uintptr_t)x < (uintptr_t)(y + (size_t)(batch - 1) * ldy + OUT);
-    const bool blocks = !forward_only && (sum_blocks(hid, IN, batch) || in_place);
+    const bool blocks = !forward_only && (sum_blocks(hid, IN, batch, backward_only) || in_place);
     const int exact = hid * IN + hid + hid * hid + hid + OUT * hid + OUT;
     if (blocks) {
         void* scratch = nullptr;

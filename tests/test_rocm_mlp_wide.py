@@ -44,6 +44,7 @@ CASES = [
     # the workgroups' blocks added up: the narrowest with spare wavefronts, the widest, the last and the first batch of each line, without spare wavefronts
     (16, 3, 65, 1, "relu", True), (255, 1, 97, 16, "fast_tanh", False), (300, 60, 112, 2, "relu", False), (4096, 17, 100, 5, "tanh", True),
     (1024, 65, 80, 3, "tanh", False), (1025, 65, 80, 3, "tanh", False), (768, 20, 144, 4, "relu", True), (769, 20, 144, 4, "relu", True), (257, 1, 150, 1, "sigmoid", False),
+    (4096, 21, 112, 2, "relu", False), (4096, 22, 112, 2, "relu", True), (550, 20, 144, 4, "tanh", False), (551, 20, 144, 4, "tanh", True), (257, 60, 128, 3, "relu", True), (256, 60, 128, 3, "relu", True),
 ]
 
 
@@ -133,7 +134,8 @@ def forward_then_backward(backend, dims, params, x, dy, ha, oa):
 
 @pytest.mark.parametrize("case", [(256, 17, 256, 6, "relu", "identity"), (4096, 17, 256, 6, "relu", "tanh"), (37, 35, 200, 1, "tanh", "identity"), (100, 128, 72, 16, "fast_tanh", "sigmoid"),
                                   (1000, 3, 64, 2, "sigmoid", "identity"), (300, 128, 64, 3, "relu", "identity"), (4096, 2, 33, 1, "tanh", "identity"), (768, 20, 144, 4, "relu", "tanh"),
-                                  (257, 128, 20, 16, "relu", "identity"), (1, 5, 16, 2, "tanh", "identity")])
+                                  (257, 128, 20, 16, "relu", "identity"), (1, 5, 16, 2, "tanh", "identity"), (2051, 17, 100, 2, "tanh", "identity"), (2052, 17, 100, 2, "tanh", "identity"),
+                                  (128, 17, 100, 16, "relu", "tanh"), (129, 17, 100, 16, "relu", "tanh"), (600, 21, 112, 1, "relu", "identity"), (600, 22, 112, 1, "relu", "identity")])
 def test_backward_alone_on_sixteen_row_tiles_matches_the_checker_and_the_other_paths(oracle, rocm, case, monkeypatch):
     """backward() after forward(): the tiles read the hidden layers' outputs back from memory; the last layer may have any activation (its derivative is applied to the
     given gradient before the kernel runs, in place as in the reference)."""
