@@ -401,8 +401,11 @@ __global__ __launch_bounds__(256, 2) void gru_forward_mfma_kernel(GruArgs A) {
 // Reverse pass: the gate gradients of the four rows are the A side (192 reduction indices, quarter kg = the 48 of wavefront kg's units), a wavefront forms d h_prev of
 // its sixteen units. gs (two copies, by the parity of the step): lane (kg, cg, row) of the A operand reads its twelve values in three 16-byte reads (neighbours lie 12
 // floats apart: no two of a group share a bank). One workgroup barrier per step; lane = (row, unit) and addresses as in the forward pass.
-__global__ __launch_bounds__(256, 2) void gru_backward_mfma_kernel(GruArgs A) {
-    constexpr int H = 64, D = 4;
+// Four steps ahead take 145 registers, three workgroups per compute unit; where more want to run, two steps ahead and 117 registers for four (backward to the input, a row per
+// wavefront as below / this: 3,100 sequences of 3 steps 23.6 / 22.2 us, 5,000 of 3 26.2 / 25.2, 6,000 of 10 52.1 / 50.4, 8,192 of 3 32.0 / 31.1).
+template <int D, int WAVES>
+__global__ __launch_bounds__(256, WAVES) void gru_backward_mfma_kernel(GruArgs A) {
+    constexpr int H = 64;
     __shared__ __align__(16) float gs[2][3 * H * GM_ROWS];
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kg = lane >> 4, c16 = lane & 15, u = 16 * w + c16, S = A.S;
     // B operand: column u, reduction index (gate s >> 2, unit 16 kg + 4 (s & 3) + abid)
@@ -475,7 +478,7 @@ __global__ __launch_bounds__(256, 2) void gru_backward_mfma_kernel(GruArgs A) {
 }
 
 // The same for batches whose steps are bound by memory instead of the chain: thread (w, lane) finishes (row w, unit lane), so that a wavefront's loads and stores are whole rows
-// of 256 bytes (above: 64 bytes of each of four rows), and 106 instead of 145 registers leave room for four workgroups per compute unit instead of three. Wavefront w forms the
+// of 256 bytes (above: 64 bytes of each of four rows). Wavefront w forms the
 // products of rows 48 w ... 48 w + 47 of W_h (lane = column) and the four partial sums of d h_prev meet in LDS: two workgroup barriers per step. Backward to the input, the kernel above / this
 // one: 16,384 sequences of 10 steps 181 / 157 us, 3,000 of 30 90.8 / 77.3, 1,500 of 100 173 / 157; but 2,048 of 30 52.0 / 53.2, 1,024 of 100 95 / 130.
 template <int ABID> __device__ __forceinline__ gru_floatx4 mfma4_all(float a, float b, gru_floatx4 c) { return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 4, ABID, 0); }      // every block's A from block ABID
@@ -541,11 +544,8 @@ __global__ __launch_bounds__(256) void gru_backward_rows_kernel(GruArgs A) {
     }
     if (live && A.db_hn_partial) A.db_hn_partial[(size_t)b * H + u] = db_hn;
 }
-// Which of the two: beyond three workgroups per compute unit, and beyond one where what the steps read and write (14 rows of 64 floats each) does not fit the 256 MB of last-level cache
-bool backward_by_rows(const rlt_rocm_device* device, int S, int B) {
-    const int units = device->compute_units > 0 ? device->compute_units : 256, blocks = rlt_div_up(B, GM_ROWS);
-    return blocks > 3 * units || (blocks > units && (size_t)S * B * 14 * 64 * sizeof(float) > (size_t)256 << 20);
-}
+// Which of the two: beyond one workgroup per compute unit, where what the steps read and write (14 rows of 64 floats each) does not fit the 256 MB of last-level cache
+bool backward_by_rows(int units, int S, int B) { return rlt_div_up(B, GM_ROWS) > units && (size_t)S * B * 14 * 64 * sizeof(float) > (size_t)256 << 20; }
 
 // db_h[n part] += sum over batch rows of the per-row sums, db_h[r, z parts] = db_i[r, z parts] (the reference copies, :679-681).
 // One workgroup per hidden unit.
@@ -624,8 +624,13 @@ int rlt_rocm_gru_backward(rlt_rocm_device* device, const rlt_gru_layer* L, const
     a.h_previous = h_previous; a.db_hn_partial = want_weight_gradients ? db_hn_partial : nullptr; a.S = S; a.B = B; a.rows_per_group = rows_per_group(H);
     if (H == 64 || H == 32 || H == 16) {
         const dim3 grid(rlt_div_up(B, GRU_THREADS / H)), block(GRU_THREADS);
-        if (H == 64 && backward_by_rows(device, S, B)) hipLaunchKernelGGL(gru_backward_rows_kernel, dim3(rlt_div_up(B, GM_ROWS)), block, 0, device->stream, a);
-        else if (H == 64) hipLaunchKernelGGL(gru_backward_mfma_kernel, dim3(rlt_div_up(B, GM_ROWS)), block, 0, device->stream, a);
+        if (H == 64) {
+            const dim3 grid4(rlt_div_up(B, GM_ROWS));
+            const int units = device->compute_units > 0 ? device->compute_units : 256;
+            if (backward_by_rows(units, S, B)) hipLaunchKernelGGL(gru_backward_rows_kernel, grid4, block, 0, device->stream, a);
+            else if ((int)grid4.x > 3 * units) hipLaunchKernelGGL((gru_backward_mfma_kernel<2, 4>), grid4, block, 0, device->stream, a);
+            else hipLaunchKernelGGL((gru_backward_mfma_kernel<4, 2>), grid4, block, 0, device->stream, a);
+        }
         else if (H == 32) hipLaunchKernelGGL(gru_backward_reg_kernel<32>, grid, block, 0, device->stream, a);
         else hipLaunchKernelGGL(gru_backward_reg_kernel<16>, grid, block, 0, device->stream, a);
     } else {

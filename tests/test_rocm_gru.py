@@ -126,10 +126,11 @@ def test_gru_at_the_edges_of_the_blocks_of_steps(oracle, rocm, steps, batch, hid
 
 
 @pytest.mark.parametrize("with_reset", [False, True])
-@pytest.mark.parametrize("case", [(1, 3072, 3, 64), (1, 3073, 3, 64), (5, 3074, 4, 64), (74, 1025, 2, 64), (73, 1025, 2, 64)])
+@pytest.mark.parametrize("case", [(1, 3072, 3, 64), (1, 3073, 3, 64), (5, 3074, 4, 64), (24, 3121, 2, 64), (23, 3122, 2, 64), (74, 1025, 2, 64), (73, 1025, 2, 64)])
 def test_gru_backward_on_both_sides_of_the_line_to_whole_rows(oracle, rocm, case, with_reset):
-    """Width 64: the last batch and sequences that go through the kernel of sixteen units per wavefront and the first through that of a row per wavefront (more than 3,072 rows; more than
-    1,024 and 256 MB of saved values and gradients), last workgroups of one, two and four rows, one step. Tolerance as for the long batch above."""
+    """Width 64: the last batch with four steps' values requested ahead and the first with two (more than 3,072 rows), the last sequences that go through the kernel of sixteen units per
+    wavefront and the first through that of a row per wavefront (more than 1,024 rows and 256 MB of saved values and gradients), last workgroups of one and two rows, one step. Tolerance as
+    for the long batch above."""
     print("case", case, with_reset, flush=True)
     S, B, I, H = case
     want, got = run_pair(oracle, rocm, S, B, I, H, 36, with_reset)

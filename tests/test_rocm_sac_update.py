@@ -105,7 +105,9 @@ def test_fused_updates_match_the_checker_and_the_per_operation_path(oracle, rocm
 
 
 @pytest.mark.parametrize("batch,obs,act,hidden,hidden_act", [(256, 6, 1, 256, "fast_tanh"), (100, 17, 6, 128, "relu"), (48, 3, 1, 200, "relu"), (256, 27, 8, 256, "relu"),
-                                                             (30, 111, 8, 72, "tanh"), (512, 5, 2, 16, "sigmoid")])
+                                                             (30, 111, 8, 72, "tanh"), (512, 5, 2, 16, "sigmoid"),
+                                                             # every network beyond 240 units, and the first width that is not
+                                                             (70, 6, 1, 241, "relu"), (40, 111, 8, 256, "relu"), (70, 6, 1, 240, "relu")])
 def test_wider_agents_match_the_checker_on_both_paths(oracle, rocm, batch, obs, act, hidden, hidden_act):
     """Hidden widths other than 64 (the zoo's AcrobotSwingup agent: 6-256-256-2 and 7-256-256-1 at batch 256; Ant-sized: 27 / 8): one launch per update on the
     kernel for widths up to 256 (every network pass of the update by sixteen wavefronts per 16 rows, the optimiser as its last step), and one launch per
