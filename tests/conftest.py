@@ -9,7 +9,7 @@ sys.path.insert(0, ROOT)
 
 
 def pytest_configure(config):
-    config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu on the GPU box)")
+    config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu on a machine that has one)")
 
 
 @pytest.fixture(scope="session")

@@ -1,5 +1,5 @@
 """The CPU checker against the REAL reference compiled from /root/reference (oracle/_ref, built by oracle/Makefile): the whole
-seeded SAC-on-Pendulum loop, bit for bit. Skipped where the reference build is absent (the GPU box still carries the built
+seeded SAC-on-Pendulum loop, bit for bit. Skipped where the reference build is absent (a machine with the GPU still carries the built
 library; a machine without it relies on tests/test_oracle_golden.py)."""
 import ctypes as C
 import os
