@@ -4,7 +4,7 @@
 // reference: rl/algorithms/sac/operations_generic.h:243-337 (train_critic), :395-468 (train_actor),
 //            nn/layers/sample_and_squash/operations_generic.h:148-398, nn_models/mlp/operations_generic.h:128-260.
 //
-// A workgroup of sixteen wavefronts takes 16 rows of the batch through the passes that depend on each other; passes that do not depend on each other have workgroups
+// A workgroup of sixteen wavefronts takes 16, 8 or 4 rows of the batch (tile_rows()) through the passes that depend on each other; passes that do not depend on each other have workgroups
 // of their own (a role each), which hand over a few values per row through memory:
 //   critic update   target roles: actor on the next observations -> squashed sample and its log-probability -> one target critic on [next observation | sample];
 //                   critic roles: trained critic forward on the current rows -> (wait for the targets' values) -> TD target -> MSE gradient -> backward
@@ -14,7 +14,8 @@
 // td3_sampling layer): the critic update with the target actor, the smoothing noise on the next action and no entropy term (each critic's targets are formed with
 // sampling noise of its own, so each has its own pair of target roles), the actor update through critic 0 only.
 // Wavefront w owns hidden units 16 w .. 16 w + 15 of every layer: it computes that tile of the 16 x h activations from the whole previous
-// layer (LDS, behind a workgroup barrier), contributes the units' share of the output layer's reduction (the partial tiles are added in
+// layer (LDS, behind a workgroup barrier; the products of the first two layers and of the way back between them, `chunks`, run over the tile's rows only, the narrow ones
+// over sixteen whatever the tile, the rows beyond it being nobody's), contributes the units' share of the output layer's reduction (the partial tiles are added in
 // wavefront order), and in the backward pass owns the same units' pre-activation gradients.
 // Weights are read from memory (L2) straight into the B operands of v_mfma_f32_16x16x4_f32, the next pass's while this one runs; hidden widths that are no multiple
 // of 16 are completed with zero operands. The reduction index of a 16-deep chunk is dealt to the four lane groups as k = 16 j + 4 g + i for the i-th of four
@@ -23,8 +24,10 @@
 // launch (batch_gradient.hip). Before, a workgroup ended with its sixteen rows' weight gradients (6.5 us on the matrix pipe at width 256) and a block of partial sums
 // that the optimisers' launch added up, and took all passes one after the other. At width 256, batch 256 (kernel and optimisers' launch; before / now): SAC critics
 // 55.7 + 10.6 / 26.0 + 8.2 us, SAC actor 65.6 + 10.6 / 33.9 + 8.2 us; TD3 critics (27 + 8 inputs) 61.1 + 11.9 / 28.1 + 8.0 us, TD3 actor 50.5 + 8.4 / 35.9 + 8.0 us.
-// Bound: per workgroup, a 16 x 256 x 256 layer is 2.1 MFLOP = 4 us of one compute unit's matrix pipeline, and the longest chain has three of them (critic update)
-// or four (actor update); the trips to memory at the start (3 us) and for the values handed over (2 us) come on top.
+// With four rows per workgroup instead of sixteen: SAC critics / actor 26.5 / 33.8 -> 20.1 / 23.5 us, TD3 critics (eight) / actor 28.9 / 34.5 -> 24.9 / 25.2 us.
+// Bound: a workgroup's layer of R x 256 x 256 is R * 512 cycles of one compute unit's matrix pipeline (0.9 us with four rows, 3.4 with sixteen) and 256 KB of weights from L2 (1.7 us at
+// 64 B per cycle, while something else runs), and the longest chain has three of them (critic update) or four (actor update); the trips to memory at the start (3 us) and for the
+// values handed over (2 us) and the narrow layers between them come on top.
 #include "sac_update.h"
 #include "optim.h"
 #include "rng.h"
@@ -103,15 +106,70 @@ __device__ __forceinline__ void load_swizzled(const float* __restrict__ copy, in
             b[j] = *reinterpret_cast<const floatx4*>(reinterpret_cast<const char*>(copy) + (j0 + j < tiles ? mine + (uint32_t)(j0 + j) * 1024 : 0));
     }
 }
-// acc += in[rows][16 (j0 + j) + ...] * b[j], the workgroup's 16 rows against this lane's column
-template <int JN>
-__device__ __forceinline__ void chunks(floatx4& a0, floatx4& a1, lptr in, int stride, int c, int g, int j0, int steps, const floatx4 (&b)[JN]) {
+// A workgroup's rows R against this lane's column: sixteen on v_mfma_f32_16x16x4_f32, or eight or four on v_mfma_f32_4x4x1_16b_f32 (sixteen blocks of 4 x 1 by 1 x 4: block 4 g + q takes
+// columns 4 q .. 4 q + 3 of the wavefront's sixteen and lane group g's share of the reduction, so the weights lie in the lanes as the other instruction has them, and half the rows
+// are half the cycles). The activations of four chunks are one read per four rows: block q of a group of four holds those of chunk 4 J + q and hands them to the other three.
+template <int R> struct Sums { floatx4 s[R == 16 ? 1 : R / 4][2]; };
+template <int R> __device__ __forceinline__ void clear(Sums<R>& A) {
 #pragma unroll
-    for (int j = 0; j < JN; j++) {
-        if (j0 + j < steps) {
-            const floatx4 a = *(lptr4)(in + c * stride + 16 * (j0 + j) + 4 * g);
-            a0 = mfma16(a[0], b[j][0], a0); a1 = mfma16(a[1], b[j][1], a1);
-            a0 = mfma16(a[2], b[j][2], a0); a1 = mfma16(a[3], b[j][3], a1);
+    for (int h = 0; h < (R == 16 ? 1 : R / 4); h++) A.s[h][0] = A.s[h][1] = floatx4{0.f, 0.f, 0.f, 0.f};
+}
+template <int Q> __device__ __forceinline__ floatx4 mfma4(float a, float b, floatx4 c) { return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 2, Q, 0); }
+template <int R, int Q>
+__device__ __forceinline__ void chunk4(Sums<R>& A, const floatx4 (&a)[R / 4], floatx4 b) {
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int h = 0; h < R / 4; h++) A.s[h][i & 1] = mfma4<Q>(a[h][i], b[i], A.s[h][i & 1]);
+}
+// A += in[rows][16 (j0 + j) + ...] * b[j], j0 a multiple of four
+template <int R, int JN>
+__device__ __forceinline__ void chunks(Sums<R>& A, lptr in, int stride, int c, int g, int j0, int steps, const floatx4 (&b)[JN]) {
+    if constexpr (R == 16) {
+#pragma unroll
+        for (int j = 0; j < JN; j++) {
+            if (j0 + j < steps) {
+                const floatx4 a = *(lptr4)(in + c * stride + 16 * (j0 + j) + 4 * g);
+                A.s[0][0] = mfma16(a[0], b[j][0], A.s[0][0]); A.s[0][1] = mfma16(a[1], b[j][1], A.s[0][1]);
+                A.s[0][0] = mfma16(a[2], b[j][2], A.s[0][0]); A.s[0][1] = mfma16(a[3], b[j][3], A.s[0][1]);
+            }
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < JN; j += 4) {
+            if (j0 + j < steps) {
+                floatx4 a[R / 4];      // (columns of chunks beyond the width hold anything: nobody multiplies them)
+#pragma unroll
+                for (int h = 0; h < R / 4; h++) a[h] = *(lptr4)(in + ((c & 3) + 4 * h) * stride + 16 * (j0 + j + (c >> 2)) + 4 * g);
+                chunk4<R, 0>(A, a, b[j]);
+                if (j + 1 < JN && j0 + j + 1 < steps) chunk4<R, 1>(A, a, b[j + 1 < JN ? j + 1 : 0]);
+                if (j + 2 < JN && j0 + j + 2 < steps) chunk4<R, 2>(A, a, b[j + 2 < JN ? j + 2 : 0]);
+                if (j + 3 < JN && j0 + j + 3 < steps) chunk4<R, 3>(A, a, b[j + 3 < JN ? j + 3 : 0]);
+            }
+        }
+    }
+}
+// the finished sums: element v of lane (c, g) belongs to row R / 4 * g + v, column c (the shares of the lane groups are added up in exchanges that leave each half of the rows)
+template <int R>
+__device__ __forceinline__ void finished(const Sums<R>& A, float (&out)[R / 4]) {
+    floatx4 s[R == 16 ? 1 : R / 4];
+#pragma unroll
+    for (int h = 0; h < (R == 16 ? 1 : R / 4); h++) s[h] = A.s[h][0] + A.s[h][1];
+    if constexpr (R == 16) {
+#pragma unroll
+        for (int v = 0; v < 4; v++) out[v] = s[0][v];
+    } else {
+        constexpr int E = R / 4;
+        float t[2 * E];
+#pragma unroll
+        for (int v = 0; v < 2 * E; v++) {      // row v and row 2 E + v
+            const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(s[v / 4][v & 3]), __float_as_uint(s[(2 * E + v) / 4][(2 * E + v) & 3]), false, false);
+            t[v] = __uint_as_float(x[0]) + __uint_as_float(x[1]);
+        }
+#pragma unroll
+        for (int v = 0; v < E; v++) {
+            const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(t[v]), __float_as_uint(t[E + v]), false, false);
+            out[v] = __uint_as_float(x[0]) + __uint_as_float(x[1]);
         }
     }
 }
@@ -167,30 +225,34 @@ __device__ __forceinline__ void load_operands(const WNet& N, int wave, int c, in
 // LIVE: the activations of rows from `live` on (beyond the batch) are zero -- zero inputs alone leave NaNs there where a weight or a bias is infinite
 // KEEP: the hidden layers' pre-activations and outputs are also stored to memory, rows [row0, row0 + 16) of [batch x hid] arrays (forward() of a network keeps them)
 struct KeepArgs { float* pre[2]; float* out[2]; int row0, batch; };
-template <int ACT_H, bool KEEP, bool LIVE>
-__device__ __forceinline__ void place_hidden(const WNet& N, const floatx4& acc, float bias, lptr h, int n, int g, const KeepArgs* keep, int layer, int live) {
+template <int R, int ACT_H, bool KEEP, bool LIVE>
+__device__ __forceinline__ void place_hidden(const WNet& N, const Sums<R>& sums, float bias, lptr h, int n, int g, const KeepArgs* keep, int layer, int live) {
     const bool n_ok = n < N.hid;
+    float acc[R / 4];
+    finished<R>(sums, acc);
 #pragma unroll
-    for (int v = 0; v < 4; v++) {
+    for (int v = 0; v < R / 4; v++) {
+        const int row = R / 4 * g + v;
         const float pre = acc[v] + bias, o = act_hidden<ACT_H>(pre, N.act_h);
-        h[(4 * g + v) * S + n] = n_ok && (!LIVE || 4 * g + v < live) ? o : 0.f;
-        if (KEEP && n_ok && keep->row0 + 4 * g + v < keep->batch) {
-            const size_t at = (size_t)(keep->row0 + 4 * g + v) * N.hid + n;
+        h[row * S + n] = n_ok && (!LIVE || row < live) ? o : 0.f;
+        if (KEEP && n_ok && keep->row0 + row < keep->batch) {
+            const size_t at = (size_t)(keep->row0 + row) * N.hid + n;
             if (keep->pre[layer]) keep->pre[layer][at] = pre;
             if (keep->out[layer]) keep->out[layer][at] = o;
         }
     }
 }
-template <int ACT_H, int NT1C, bool PREFETCH, bool W1_READY, bool KEEP = false, bool EVERY = false, bool LIVE = false>
+template <int R, int ACT_H, int NT1C, bool PREFETCH, bool W1_READY, bool KEEP = false, bool EVERY = false, bool LIVE = false>
 __device__ __forceinline__ void forward3(const WNet& N, Operands<NT1C>& W, const WNet& next, lptr x, int xstride, lptr h1, lptr h2, lptr yp, int wave, int c, int g, const KeepArgs* keep = nullptr, int live = ROWS) {
     const int n = 16 * wave + c, tiles = (N.hid + 15) >> 4, lane = c + 16 * g, next_tiles = (next.hid + 15) >> 4;
     const bool on = wave < tiles, next_on = wave < next_tiles;
     const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
     if (!W1_READY) load_swizzled<NT1C, false, FIRST_STEP<NT1C>>(N.W1f, (N.in + 15) >> 4, on, wave, lane, 0, W.w1);
     if (on) {
-        floatx4 a0 = zero4, a1 = zero4;
-        chunks<NT1C>(a0, a1, x, xstride, c, g, 0, (N.in + 15) >> 4, W.w1);
-        place_hidden<ACT_H, KEEP, LIVE>(N, a0 + a1, W.b1, h1, n, g, keep, 0, live);
+        Sums<R> sums;
+        clear(sums);
+        chunks<R, NT1C>(sums, x, xstride, c, g, 0, (N.in + 15) >> 4, W.w1);
+        place_hidden<R, ACT_H, KEEP, LIVE>(N, sums, W.b1, h1, n, g, keep, 0, live);
     }
     if (NT1C > FEW) load_swizzled<8, EVERY>(N.W2f, tiles, on, wave, lane, 8, W.w2b);
     if (PREFETCH) {
@@ -199,12 +261,13 @@ __device__ __forceinline__ void forward3(const WNet& N, Operands<NT1C>& W, const
     }
     rlt_lds_barrier();
     {
-        floatx4 a0 = zero4, a1 = zero4;
-        if (on) chunks<8>(a0, a1, h1, S, c, g, 0, tiles, W.w2a);
+        Sums<R> sums;
+        clear(sums);
+        if (on) chunks<R, 8>(sums, h1, S, c, g, 0, tiles, W.w2a);
         if (PREFETCH) load_swizzled<8, EVERY>(next.W2f, next_tiles, next_on, wave, lane, 0, W.w2a);
-        if (on) chunks<8>(a0, a1, h1, S, c, g, 8, tiles, W.w2b);
+        if (on) chunks<R, 8>(sums, h1, S, c, g, 8, tiles, W.w2b);
         if (PREFETCH && NT1C <= FEW) load_swizzled<8, EVERY>(next.W2f, next_tiles, next_on, wave, lane, 8, W.w2b);
-        if (on) place_hidden<ACT_H, KEEP, LIVE>(N, a0 + a1, W.b2, h2, n, g, keep, 1, live);
+        if (on) place_hidden<R, ACT_H, KEEP, LIVE>(N, sums, W.b2, h2, n, g, keep, 1, live);
         if (PREFETCH) W.b2 = next.b2[min(n, next.hid - 1)];
     }
     rlt_lds_barrier();
@@ -265,19 +328,19 @@ __device__ __forceinline__ float backward_layer3(const WNet& N, const BackOperan
     return sum;
 }
 // this wavefront's tile of d_pre1 = (d_pre2 W2) f'(h1) into p1 (may be h1 itself); returns the lane's share of its unit's column sum
-template <int ACT_H, bool LIVE = false>
+template <int R, int ACT_H, bool LIVE = false>
 __device__ __forceinline__ float backward_layer2(const WNet& N, const BackOperands& W, lptr g2, lptr h1, lptr p1, int wave, int c, int g, int live = ROWS) {
     const int n = 16 * wave + c, tiles = (N.hid + 15) >> 4;
     const bool n_ok = n < N.hid;
-    const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
-    floatx4 a0 = zero4, a1 = zero4;
-    chunks<MAX_H / 16>(a0, a1, g2, S, c, g, 0, tiles, W.w2);
-    const floatx4 acc = a0 + a1;
-    float sum = 0.f;
+    Sums<R> sums;
+    clear(sums);
+    chunks<R, MAX_H / 16>(sums, g2, S, c, g, 0, tiles, W.w2);
+    float acc[R / 4], sum = 0.f;
+    finished<R>(sums, acc);
 #pragma unroll
-    for (int v = 0; v < 4; v++) {
-        const int idx = (4 * g + v) * S + n;
-        const float d = n_ok && (!LIVE || 4 * g + v < live) ? acc[v] * dact_hidden<ACT_H>(h1[idx], N.act_h) : 0.f;
+    for (int v = 0; v < R / 4; v++) {
+        const int row = R / 4 * g + v, idx = row * S + n;
+        const float d = n_ok && (!LIVE || row < live) ? acc[v] * dact_hidden<ACT_H>(h1[idx], N.act_h) : 0.f;
         p1[idx] = d; sum += d;
     }
     return sum;
@@ -305,10 +368,12 @@ __device__ __forceinline__ void place_row(lptr to, bool ok, int cols, int end, i
 #pragma unroll
     for (int u = 0; u < N; u++) if (64 * u + lane < end) to[64 * u + lane] = ok && 64 * u + lane < cols ? v[u] : 0.f;
 }
-__device__ __forceinline__ void store_rows(lptr from, float* to, int hid, int row0, int batch, int wave, int lane) {
-    if (row0 + wave >= batch) return;
-    float* const row = to + (size_t)(row0 + wave) * hid;
-    for (int n = lane; n < hid; n += 64) row[n] = from[wave * S + n];
+template <int R>
+__device__ __forceinline__ void store_rows(lptr from, float* to, int hid, int row0, int batch, int wave, int lane) {      // a row to each wavefront, or to two or four of them, 64 columns in turn
+    const int mine = R == WAVES ? wave : wave % R, part = R == WAVES ? 0 : wave / R;
+    if (row0 + mine >= batch) return;
+    float* const row = to + (size_t)(row0 + mine) * hid;
+    for (int n = lane + 64 * part; n < hid; n += 64 * WAVES / R) row[n] = from[mine * S + n];
 }
 // A value handed from one workgroup to another of the same launch: one 8-byte store that carries its own tag, so that nothing has to be ordered around it. The wait is
 // bounded (rlt_rocm_set_wait_limit: at most max_poll - 1 looks, with a bound of one none); a workgroup that gives up sets the fault word and goes on with zero, and the next
@@ -387,7 +452,7 @@ struct Copies {
 constexpr size_t MAX_COPY_FLOATS = (size_t)WAVES * (MAX_H / 16) * 256, MAX_W1_COPY_FLOATS = (size_t)WAVES * (MAX_D / 16) * 256;
 
 // EVERY: all networks have more than 240 units
-template <int MODE, int ACT_H, int NT1C, bool EVERY>
+template <int MODE, int ACT_H, int NT1C, bool EVERY, int R>
 __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
     constexpr bool CRITIC = MODE == MODE_CRITIC || MODE == MODE_TD3_CRITIC, TD3 = MODE == MODE_TD3_CRITIC || MODE == MODE_TD3_ACTOR;
     extern __shared__ __attribute__((aligned(16))) float lds_wide[];
@@ -401,10 +466,10 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
     const int OBS = A.obs, ACT = A.act, D = OBS + ACT, B = A.batch;
     const lptr xa = (lptr)lds_wide, h1 = xa + ROWS * SXS, h2 = h1 + ROWS * S, ta = h2 + ROWS * S, tb = ta + ROWS * S,
                d3 = tb + ROWS * S, d3c = d3 + ROWS * D3S, da = d3c + ROWS * D3S, yp = da + 2 * ROWS * D3S, misc = yp + WAVES * YP;
-    const int row0 = gi * ROWS;
+    const int row0 = gi * R, row_end = min(B, row0 + R);      // the tile's rows (with eight, the other eight of the sixteen that the narrow products run over belong to nobody)
     const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
     uint64_t* const exchange = A.exchange + (size_t)gi * EXCHANGE;
-    const bool row_ok = row0 + c < B;
+    const bool row_ok = row0 + c < row_end;
     // critic update: target roles [set][target critic] first, then a role per trained critic; actor update: critic 1's role (SAC), then the role that goes on with the actor
     const int n_target_roles = CRITIC ? 2 * (TD3 ? A.n_critics : 1) : 0;
     const bool target_role = CRITIC && role < n_target_roles;
@@ -415,7 +480,7 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
     // batch holds there meets zero weights in the actor's last chunk, and must not be a NaN or an infinity
     float in_row[3];
     const bool trained_role = CRITIC && !target_role;
-    request_row(A.batch_base + (target_role ? (size_t)B * D : 0) + (size_t)min(row0 + wave, B - 1) * D, trained_role ? D : OBS, lane, in_row);
+    request_row(A.batch_base + (target_role ? (size_t)B * D : 0) + (size_t)min(row0 + wave, row_end - 1) * D, trained_role ? D : OBS, lane, in_row);
     if (trained_role) {
         // ---- a trained critic
         const int y = role - n_target_roles;
@@ -424,7 +489,7 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
         const int HID = trained.hid, tiles = (HID + 15) >> 4;
         Operands<NT1C> W;
         load_operands<NT1C, EVERY>(trained, wave, c, g, W);
-        place_row(xa + wave * SXS, row0 + wave < B, D, SXS, lane, in_row);
+        place_row(xa + wave * SXS, row0 + wave < row_end, D, SXS, lane, in_row);
         float reward[4] = {0.f, 0.f, 0.f, 0.f}, alpha = 0.f, b3 = 0.f;
         bool terminated[4] = {false, false, false, false};
         if (scalar_wave) {
@@ -435,12 +500,12 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
         }
         rlt_lds_barrier();      // the input rows are in place
         RLT_TICK(1);
-        forward3<ACT_H, NT1C, false, true, false, EVERY>(trained, W, trained, xa, SXS, h1, h2, yp, wave, c, g);
+        forward3<R, ACT_H, NT1C, false, true, false, EVERY>(trained, W, trained, xa, SXS, h1, h2, yp, wave, c, g);
         RLT_TICK(2);
         BackOperands K;
         load_back_operands<EVERY>(trained, wave, c, g, K);      // on their way while the targets' values are waited for
-        store_rows(h1, T.h1, HID, row0, B, wave, lane);
-        store_rows(h2, T.h2, HID, row0, B, wave, lane);
+        store_rows<R>(h1, T.h1, HID, row0, row_end, wave, lane);
+        store_rows<R>(h2, T.h2, HID, row0, row_end, wave, lane);
         if (scalar_wave) {
             // TD target of rows 4 g + v (meaningful in the lanes c == 0, which hold output 0), MSE gradient at the critic's pre-activation:
             // loss weight batch * 0.5 / n with n = batch rows (no masks), times the MSE gradient's 2 / batch (rl/algorithms/sac/operations_generic.h:298-316)
@@ -464,23 +529,23 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
                 const float min_q = TD3 ? q_min : q_min - alpha * value[(TD3 ? 0 : 8) + v];
                 const float future = (terminated[v] && !(TD3 && A.ignore_termination)) ? 0.0f : A.gamma * min_q;
                 const float y_target = reward[v] + future;
-                const bool ok = c == 0 && row0 + row < B;
+                const bool ok = c == 0 && row0 + row < row_end;
                 // (SAC's critics share their targets; TD3's are formed with each critic's own sampling noise: the last critic's stay, as after two calls)
                 if (A.out_target_action_value && ok && y == (TD3 ? A.n_critics - 1 : 0)) A.out_target_action_value[row0 + row] = y_target;
                 const float diff = (yc[v] + b3) - y_target;
                 const float dp = ok ? diff * constant : 0.f;
                 d3[row * D3S + c] = dp;
-                if (row0 + row < B) T.d3[(size_t)(row0 + row) * MAX_OUT + c] = dp;
+                if (row0 + row < row_end) T.d3[(size_t)(row0 + row) * MAX_OUT + c] = dp;
             }
         }
         rlt_lds_barrier();      // d_pre3 is in place
         RLT_TICK(3);
         if (wave < tiles) backward_layer3<ACT_H>(trained, K, d3, h2, ta, wave, c, g);
         rlt_lds_barrier();      // every wavefront's tile of d_pre2 is in place
-        store_rows(ta, T.d2, HID, row0, B, wave, lane);
-        if (wave < tiles) backward_layer2<ACT_H>(trained, K, ta, h1, tb, wave, c, g);
+        store_rows<R>(ta, T.d2, HID, row0, row_end, wave, lane);
+        if (wave < tiles) backward_layer2<R, ACT_H>(trained, K, ta, h1, tb, wave, c, g);
         rlt_lds_barrier();
-        store_rows(tb, T.d1, HID, row0, B, wave, lane);
+        store_rows<R>(tb, T.d1, HID, row0, row_end, wave, lane);
         RLT_TICK(4);
         return;
     }
@@ -492,7 +557,7 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
     const WNet Q = CRITIC ? (critic_index ? A.target[1] : A.target[0]) : (critic_index ? A.critic[1] : A.critic[0]);
     Operands<NT1C> W;
     load_operands<NT1C, EVERY>(A.actor, wave, c, g, W);      // on their way while the input rows are written
-    place_row(xa + wave * SXS, row0 + wave < B, OBS, SXS, lane, in_row);
+    place_row(xa + wave * SXS, row0 + wave < row_end, OBS, SXS, lane, in_row);
     float noise[2] = {0.f, 0.f}, target_noise[2] = {0.f, 0.f}, alpha = 0.f, actor_b3 = 0.f, q_b3 = 0.f;
     if (scalar_wave) {
         actor_b3 = c < A.actor.out ? A.actor.b3[c] : 0.f; q_b3 = Q.b3[0];
@@ -525,7 +590,7 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
     RLT_TICK(13);
     rlt_lds_barrier();      // the input rows are in place
     RLT_TICK(5);
-    forward3<ACT_H, NT1C, true, true, false, EVERY>(A.actor, W, Q, xa, SXS, h1, h2, yp, wave, c, g);
+    forward3<R, ACT_H, NT1C, true, true, false, EVERY>(A.actor, W, Q, xa, SXS, h1, h2, yp, wave, c, g);
     RLT_TICK(6);
     if (scalar_wave) {
         const floatx4 out = output_tile(yp, (A.actor.hid + 15) >> 4, c, g);
@@ -556,7 +621,7 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
     }
     rlt_lds_barrier();      // the action columns of xa are in place
     RLT_TICK(7);
-    forward3<ACT_H, NT1C, false, NT1C <= FEW, false, EVERY>(Q, W, Q, xa, SXS, ta, tb, yp, wave, c, g);
+    forward3<R, ACT_H, NT1C, false, NT1C <= FEW, false, EVERY>(Q, W, Q, xa, SXS, ta, tb, yp, wave, c, g);
     RLT_TICK(8);
     const int qtiles = (Q.hid + 15) >> 4;
     if (CRITIC) {
@@ -580,7 +645,7 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
 #pragma unroll
         for (int v = 0; v < 4; v++) {
             if (c == 0) misc[4 * g + v] = out[v] + q_b3;
-            d3c[(4 * g + v) * D3S + c] = (c == 0 && row0 + 4 * g + v < B) ? loss_weight : 0.f;
+            d3c[(4 * g + v) * D3S + c] = (c == 0 && row0 + 4 * g + v < row_end) ? loss_weight : 0.f;
         }
     }
     rlt_lds_barrier();
@@ -588,7 +653,7 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
     rlt_lds_barrier();
     RLT_TICK(9);
     if (wave < qtiles) {
-        backward_layer2<ACT_H>(Q, K, tb, ta, ta, wave, c, g);
+        backward_layer2<R, ACT_H>(Q, K, tb, ta, ta, wave, c, g);
         wave_sync();
         // d value / d action = the action columns of d_pre1 W1: this wavefront's units' share of the reduction
         floatx4 acc = zero4;
@@ -613,8 +678,8 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
     const Trained T = A.trained[0];
     const int HID = trained.hid, tiles = (HID + 15) >> 4;
     load_back_operands<EVERY>(trained, wave, c, g, K);
-    store_rows(h1, T.h1, HID, row0, B, wave, lane);
-    store_rows(h2, T.h2, HID, row0, B, wave, lane);
+    store_rows<R>(h1, T.h1, HID, row0, row_end, wave, lane);
+    store_rows<R>(h2, T.h2, HID, row0, row_end, wave, lane);
     if (scalar_wave) {
         // sample_and_squash backward on the gradient of the smaller value; TD3: the td3_sampling layer's backward (zero where the sample was clamped,
         // nn/layers/td3_sampling/operations_generic.h:139-163) and the derivative of the actor's tanh output
@@ -655,17 +720,17 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
         const float tile_sum = row16_sum(per_row);
         wave_sync();
 #pragma unroll
-        for (int v = 0; v < 4; v++) if (row0 + 4 * g + v < B) T.d3[(size_t)(row0 + 4 * g + v) * MAX_OUT + c] = d3[(4 * g + v) * D3S + c];
+        for (int v = 0; v < 4; v++) if (row0 + 4 * g + v < row_end) T.d3[(size_t)(row0 + 4 * g + v) * MAX_OUT + c] = d3[(4 * g + v) * D3S + c];
         if (lane == 0 && A.extra) A.extra[gi] = tile_sum;
     }
     rlt_lds_barrier();      // d_pre3 is in place
     RLT_TICK(11);
     if (wave < tiles) backward_layer3<ACT_H>(trained, K, d3, h2, ta, wave, c, g);
     rlt_lds_barrier();      // every wavefront's tile of d_pre2 is in place
-    store_rows(ta, T.d2, HID, row0, B, wave, lane);
-    if (wave < tiles) backward_layer2<ACT_H>(trained, K, ta, h1, tb, wave, c, g);
+    store_rows<R>(ta, T.d2, HID, row0, row_end, wave, lane);
+    if (wave < tiles) backward_layer2<R, ACT_H>(trained, K, ta, h1, tb, wave, c, g);
     rlt_lds_barrier();
-    store_rows(tb, T.d1, HID, row0, B, wave, lane);
+    store_rows<R>(tb, T.d1, HID, row0, row_end, wave, lane);
     RLT_TICK(12);
 }
 
@@ -680,6 +745,7 @@ constexpr size_t LDS_FLOATS = (size_t)ROWS * SXS + 4 * ROWS * S + 4 * ROWS * D3S
 struct MlpWideArgs {
     WNet net;
     const float* x; int ldx; float* y; int ldy;
+    float* copy_x;                             // [batch x in], or NULL: the input rows once more, where y lies in their memory and the weight gradients are formed by the next launch
     const float* d_output; int ldd; const float* target; int ldt; float mse_scale;
     int batch;
     float* partial; int count;                 // BLOCKS: [workgroups][count] blocks dW1 | db1 | dW2 | db2 | dW3 | db3
@@ -689,19 +755,20 @@ struct MlpWideArgs {
 };
 enum { MLP_FORWARD_BACKWARD = 0, MLP_BACKWARD = 1, MLP_FORWARD = 2 };
 enum { MLP_ANY = 0, MLP_BLOCKS = 1, MLP_EVERY = 2 };      // MLP_BLOCKS: weight gradients as blocks; MLP_EVERY: more than 240 units, every wavefront has some
-template <int ACT_H, int NT1C, int PASS, int FORM>
+template <int ACT_H, int NT1C, int PASS, int FORM, int R>
 __global__ __launch_bounds__(THREADS) void mlp_wide_kernel(MlpWideArgs A) {
     constexpr bool BACKWARD_ONLY = PASS == MLP_BACKWARD, BLOCKS = FORM == MLP_BLOCKS, EVERY = FORM == MLP_EVERY;
     extern __shared__ __attribute__((aligned(16))) float lds_wide[];
+    static_assert(R == 16 || !BLOCKS, "blocks are formed over sixteen rows");
     const int gi = blockIdx.x;
     const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const lptr xa = (lptr)lds_wide, h1 = xa + ROWS * SXS, h2 = h1 + ROWS * S, ta = h2 + ROWS * S, tb = ta + ROWS * S, d3 = tb + ROWS * S, yp = d3 + 4 * ROWS * D3S;
     const WNet N = A.net;
-    const int B = A.batch, IN = N.in, HID = N.hid, OUT = N.out, tiles = (HID + 15) >> 4, row0 = gi * ROWS;
+    const int B = A.batch, IN = N.in, HID = N.hid, OUT = N.out, tiles = (HID + 15) >> 4, row0 = gi * R, row_end = min(B, row0 + R);
     const bool on = wave < tiles;
-    const bool my_row = row0 + wave < B;
-    const size_t row_at = min(row0 + wave, B - 1);
+    const bool my_row = row0 + wave < row_end;
+    const size_t row_at = min(row0 + wave, row_end - 1);
     Operands<NT1C> W;
     BackOperands K;
     float b3 = 0.f, s3 = 0.f, given[4] = {0.f, 0.f, 0.f, 0.f};      // given: this lane's elements of the gradient at the output, or of the target it is formed from
@@ -725,7 +792,7 @@ __global__ __launch_bounds__(THREADS) void mlp_wide_kernel(MlpWideArgs A) {
         if (wave == 0) {
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                const float d = c < OUT && row0 + 4 * g + v < B ? given[v] : 0.f;
+                const float d = c < OUT && row0 + 4 * g + v < row_end ? given[v] : 0.f;
                 d3[(4 * g + v) * D3S + c] = d;
                 s3 += d;
             }
@@ -736,17 +803,21 @@ __global__ __launch_bounds__(THREADS) void mlp_wide_kernel(MlpWideArgs A) {
         load_operands<NT1C, EVERY>(N, wave, c, g, W);
         b3 = N.b3[min(c, OUT - 1)];
         place_row(xa + wave * SXS, my_row, IN, SXS, lane, v);
+        if (PASS == MLP_FORWARD_BACKWARD && !BLOCKS && A.copy_x && my_row) {
+#pragma unroll
+            for (int u = 0; u < 3; u++) if (64 * u + lane < IN) A.copy_x[row_at * IN + 64 * u + lane] = v[u];
+        }
     }
     rlt_lds_barrier();
     if (PASS == MLP_FORWARD) {
-        const KeepArgs keep = {{A.keep_pre[0], A.keep_pre[1]}, {A.keep_out[0], A.keep_out[1]}, row0, B};
-        forward3<ACT_H, NT1C, false, true, true, EVERY>(N, W, N, xa, SXS, h1, h2, yp, wave, c, g, &keep);
+        const KeepArgs keep = {{A.keep_pre[0], A.keep_pre[1]}, {A.keep_out[0], A.keep_out[1]}, row0, row_end};
+        forward3<R, ACT_H, NT1C, false, true, true, EVERY>(N, W, N, xa, SXS, h1, h2, yp, wave, c, g, &keep);
         if (wave == 0) {
             const floatx4 out = output_tile(yp, tiles, c, g);
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 const int row = row0 + 4 * g + v;
-                if (c < OUT && row < B) {
+                if (c < OUT && row < row_end) {
                     const float pre = out[v] + b3;
                     if (A.keep_pre[2]) A.keep_pre[2][(size_t)row * OUT + c] = pre;
                     const float o = rlt_act(pre, A.act3);
@@ -758,12 +829,12 @@ __global__ __launch_bounds__(THREADS) void mlp_wide_kernel(MlpWideArgs A) {
         return;
     }
     if (PASS == MLP_FORWARD_BACKWARD) {
-        forward3<ACT_H, NT1C, false, true, false, EVERY, BLOCKS>(N, W, N, xa, SXS, h1, h2, yp, wave, c, g, nullptr, B - row0);
+        forward3<R, ACT_H, NT1C, false, true, false, EVERY, BLOCKS>(N, W, N, xa, SXS, h1, h2, yp, wave, c, g, nullptr, B - row0);
         if (EVERY) request_given();      // (all of W fills the registers until here)
         load_back_operands<EVERY>(N, wave, c, g, K);
         if (!BLOCKS) {
-            store_rows(h1, A.kept.h1, HID, row0, B, wave, lane);
-            store_rows(h2, A.kept.h2, HID, row0, B, wave, lane);
+            store_rows<R>(h1, A.kept.h1, HID, row0, row_end, wave, lane);
+            store_rows<R>(h2, A.kept.h2, HID, row0, row_end, wave, lane);
         }
     }
     if (!BACKWARD_ONLY && wave == 0) {
@@ -772,14 +843,14 @@ __global__ __launch_bounds__(THREADS) void mlp_wide_kernel(MlpWideArgs A) {
 #pragma unroll
         for (int v = 0; v < 4; v++) {
             const int row = row0 + 4 * g + v;
-            const bool ok = c < OUT && row < B;
+            const bool ok = c < OUT && row < row_end;
             const float yv = out[v] + b3;
             if (ok && A.y) A.y[(size_t)row * A.ldy + c] = yv;
             float d = 0.f;
             if (ok) d = A.target ? (yv - given[v]) * A.mse_scale : given[v];
             d3[(4 * g + v) * D3S + c] = d;
             s3 += d;
-            if (!BLOCKS && row < B) A.kept.d3[(size_t)row * MAX_OUT + c] = d;
+            if (!BLOCKS && row < row_end) A.kept.d3[(size_t)row * MAX_OUT + c] = d;
         }
     }
     if (!BACKWARD_ONLY) rlt_lds_barrier();      // d_pre3 is in place (the backward pass alone: with the activations)
@@ -800,7 +871,7 @@ __global__ __launch_bounds__(THREADS) void mlp_wide_kernel(MlpWideArgs A) {
         if (spread ? !on && wave - tiles < tiles : on) last_layer(spread ? wave - tiles : wave);
         rlt_lds_barrier();      // every wavefront's tile of d_pre2 is in place
         if (on) {
-            const float s1 = backward_layer2<ACT_H, BLOCKS>(N, K, ta, h1, tb, wave, c, g, B - row0);
+            const float s1 = backward_layer2<R, ACT_H, BLOCKS>(N, K, ta, h1, tb, wave, c, g, B - row0);
             wave_sync();            // dW1's rows are this wavefront's own tile of d_pre1
 #pragma unroll 2
             for (int nt = 0; nt < (IN + 15) >> 4; nt++) gradient_tile(tb, wave, xa, SXS, nt, HID, IN, block, c, g);
@@ -821,10 +892,10 @@ __global__ __launch_bounds__(THREADS) void mlp_wide_kernel(MlpWideArgs A) {
         return;
     }
     rlt_lds_barrier();      // every wavefront's tile of d_pre2 is in place
-    store_rows(ta, A.kept.d2, HID, row0, B, wave, lane);
-    if (on) backward_layer2<ACT_H>(N, K, ta, h1, tb, wave, c, g);
+    store_rows<R>(ta, A.kept.d2, HID, row0, row_end, wave, lane);
+    if (on) backward_layer2<R, ACT_H>(N, K, ta, h1, tb, wave, c, g);
     rlt_lds_barrier();
-    store_rows(tb, A.kept.d1, HID, row0, B, wave, lane);
+    store_rows<R>(tb, A.kept.d1, HID, row0, row_end, wave, lane);
 }
 // gradient[e] += the sum over the workgroups' blocks of element e: a workgroup takes 64 elements, its wavefronts a quarter of the blocks each, sixteen blocks' loads in flight
 struct BlockSum { const float* partial; int blocks, count, total; float* gradient[6]; int end[6]; };
@@ -927,8 +998,17 @@ Trained place_trained(float* base, int hid, int batch) {
 }
 void set_rows(rlt_gradient_net& N, const Trained& T, const float* x, int ldx) { N.x = x; N.ldx = ldx; N.h1 = T.h1; N.h2 = T.h2; N.d1 = T.d1; N.d2 = T.d2; N.d3 = T.d3; N.ld3 = MAX_OUT; }
 
+// Rows of a workgroup's tile: four (where there is such a kernel) or eight while every tile and role then has a compute unit of its own, sixteen beyond. Fewer rows are fewer
+// cycles of the matrix pipeline per layer (sixteen 8,192 at width 256, eight 4,096, four 2,048) on more compute units; the same weights travel to each. In us, sixteen / eight / four
+// rows, 256 rows of the batch, width 256: forward + backward, Adam and the gradients' clearing 35.1 / 32.2 / 29.0, SAC's update set 85.7 / 74.0 / 66.4, TD3's 90.7 / 80.9 / 77.9
+// (its critics' six roles take eight rows). Four and eight rows leave the same bits, sixteen others: a critic trained by a call of its own takes sixteen where both in one call do
+// (roles_of_both), as the two ways leave the same bits.
+int tile_rows(const rlt_rocm_device* device, int batch, int roles, int roles_of_both, bool four) {
+    const int most = device->compute_units < 256 ? device->compute_units : 256;
+    return rlt_div_up(batch, 8) * roles_of_both > most ? ROWS : four && rlt_div_up(batch, 4) * roles <= most ? 4 : 8;
+}
 template <int MODE>
-int launch_wide(rlt_rocm_device* device, WideArgs& a, int groups, const Optimiser* opts, int n_opts, float polyak, bool* targets_done) {
+int launch_wide(rlt_rocm_device* device, WideArgs& a, const Optimiser* opts, int n_opts, float polyak, bool* targets_done) {
     rlt_gradient_net net[2] = {};
     bool fused[2] = {false, false};
     for (int k = 0; k < n_opts; k++) {      // the agent's Adam tensors are not its networks' gradient buffers: the caller takes the per-operation path
@@ -939,15 +1019,25 @@ int launch_wide(rlt_rocm_device* device, WideArgs& a, int groups, const Optimise
     if (targets_done) *targets_done = fuse_targets;
     if (!fuse_targets) for (int k = 0; k < n_opts; k++) for (int q = 0; q < 6; q++) net[k].target[q] = nullptr;
     constexpr bool CRITIC_UPDATE = MODE == MODE_CRITIC || MODE == MODE_TD3_CRITIC;
+    a.n_critics = n_opts;
+    a.roles = MODE == MODE_CRITIC ? 2 + n_opts : MODE == MODE_TD3_CRITIC ? 3 * n_opts : MODE == MODE_ACTOR ? 2 : 1;
+    int act = a.actor.act_h;
+    bool every = a.actor.hid > MAX_H - 16;
+    for (int k = 0; k < 2; k++) {
+        if (a.critic[k].act_h != act || a.target[k].act_h != act) act = -1;
+        every = every && a.critic[k].hid > MAX_H - 16 && a.target[k].hid > MAX_H - 16;
+    }
+    const int rows = tile_rows(device, a.batch, a.roles, MODE == MODE_CRITIC ? 4 : MODE == MODE_TD3_CRITIC ? 6 : a.roles, every && act == RLT_ACT_RELU);
+    const int groups = rlt_div_up(a.batch, rows);
     const size_t copies_floats = 5 * (MAX_COPY_FLOATS + MAX_W1_COPY_FLOATS) + 3 * MAX_COPY_FLOATS;
     const size_t trained_each = trained_floats(net[0].hid, a.batch), exchange_words = (size_t)groups * EXCHANGE, extra_floats = (size_t)(groups + 63) & ~(size_t)63,
                  partial_floats = (rlt_batch_gradients_partial_floats(net, n_opts, a.batch) + 63) & ~(size_t)63;
     void* scratch = nullptr;
     int rc = rlt_scratch(device, (copies_floats + n_opts * trained_each + extra_floats + partial_floats) * sizeof(float) + exchange_words * sizeof(uint64_t) + 256, &scratch);
     if (rc) return rc;
-    float* const rows = (float*)scratch + copies_floats; float* const extra = rows + n_opts * trained_each;
+    float* const kept = (float*)scratch + copies_floats; float* const extra = kept + n_opts * trained_each;
     for (int k = 0; k < n_opts; k++) {
-        a.trained[k] = place_trained(rows + k * trained_each, net[k].hid, a.batch);
+        a.trained[k] = place_trained(kept + k * trained_each, net[k].hid, a.batch);
         set_rows(net[k], a.trained[k], a.batch_base, a.obs + a.act);
     }
     a.extra = opts[0].second ? extra : nullptr;
@@ -968,25 +1058,19 @@ int launch_wide(rlt_rocm_device* device, WideArgs& a, int groups, const Optimise
         if ((rc = copies.launch(device))) return rc;
     }
     a.stream_offset = device->stream_offset;
-    a.groups = groups; a.n_critics = n_opts;
-    a.roles = MODE == MODE_CRITIC ? 2 + n_opts : MODE == MODE_TD3_CRITIC ? 3 * n_opts : MODE == MODE_ACTOR ? 2 : 1;
+    a.groups = groups;
     // A workgroup waits for others of its tile only, and all are resident where there is a compute unit for each: then a role's workgroups are kept on neighbouring
     // positions of the XCDs' round (workgroup b runs on XCD b % 8), so that few XCDs read a network's weights. Larger grids are numbered role by role, so that whoever
     // is waited for was dispatched before whoever waits.
     a.by_xcd = device->update_one_xcd && device->xcd_stride == 8 && a.roles * groups <= device->compute_units;
     const size_t lds_bytes = LDS_FLOATS * sizeof(float);
     const dim3 grid(a.by_xcd ? 8 * rlt_div_up(a.roles * groups, 8) : a.roles * groups);
-#define RLT_LAUNCH_WIDE(ACT, NT, EVERY)                                                                                                                   \
+#define RLT_LAUNCH_WIDE_ROWS(ACT, NT, EVERY, R)                                                                                                           \
     do {                                                                                                                                                  \
-        RLT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(sac_wide_kernel<MODE, ACT, NT, EVERY>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes)); \
-        hipLaunchKernelGGL((sac_wide_kernel<MODE, ACT, NT, EVERY>), grid, dim3(THREADS), lds_bytes, device->stream, a);                                   \
+        RLT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(sac_wide_kernel<MODE, ACT, NT, EVERY, R>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes)); \
+        hipLaunchKernelGGL((sac_wide_kernel<MODE, ACT, NT, EVERY, R>), grid, dim3(THREADS), lds_bytes, device->stream, a);                                \
     } while (0)
-    int act = a.actor.act_h;
-    bool every = a.actor.hid > MAX_H - 16;
-    for (int k = 0; k < 2; k++) {
-        if (a.critic[k].act_h != act || a.target[k].act_h != act) act = -1;
-        every = every && a.critic[k].hid > MAX_H - 16 && a.target[k].hid > MAX_H - 16;
-    }
+#define RLT_LAUNCH_WIDE(ACT, NT, EVERY) do { if (rows == 4) RLT_LAUNCH_WIDE_ROWS(ACT, NT, EVERY, (EVERY ? 4 : 8)); else if (rows == 8) RLT_LAUNCH_WIDE_ROWS(ACT, NT, EVERY, 8); else RLT_LAUNCH_WIDE_ROWS(ACT, NT, EVERY, ROWS); } while (0)
 #define RLT_LAUNCH_WIDE_ACT(NT)                                                                                                                           \
     do {                                                                                                                                                  \
         if (act == RLT_ACT_RELU) { if (every) RLT_LAUNCH_WIDE(RLT_ACT_RELU, NT, true); else RLT_LAUNCH_WIDE(RLT_ACT_RELU, NT, false); }                    \
@@ -996,6 +1080,7 @@ int launch_wide(rlt_rocm_device* device, WideArgs& a, int groups, const Optimise
     if (a.obs + a.act <= 32) RLT_LAUNCH_WIDE_ACT(2); else if (a.obs + a.act <= 64) RLT_LAUNCH_WIDE_ACT(4); else RLT_LAUNCH_WIDE_ACT(MAX_D / 16);
 #undef RLT_LAUNCH_WIDE_ACT
 #undef RLT_LAUNCH_WIDE
+#undef RLT_LAUNCH_WIDE_ROWS
     if ((rc = rlt_launch_status(device))) return rc;
     const rlt_gradient_guard guard = {device->fault, {opts[0].age, n_opts > 1 ? opts[1].age : nullptr, opts[0].second ? opts[0].second_age : nullptr}, age_before};
     if (opts[0].second) {
@@ -1040,7 +1125,7 @@ int rlt_sac_wide_update_critics(rlt_rocm_device* device, const rlt_sac_agent* A,
         O[k] = {A->critics[first + k], A->critic_adam_tensors[first + k], A->n_critic_adam_tensors, &A->critic_adam, A->critic_age[first + k], nullptr, nullptr, nullptr, 0.0f,
                 update_targets ? A->critics_target[first + k] : nullptr};
     bool targets_done = false;
-    const int rc = launch_wide<MODE_CRITIC>(device, a, rlt_div_up(A->batch, ROWS), O, count, A->polyak, &targets_done);
+    const int rc = launch_wide<MODE_CRITIC>(device, a, O, count, A->polyak, &targets_done);
     if (rc || !update_targets || targets_done) return rc;
     return rlt_rocm_sac_update_critic_targets(device, A);
 }
@@ -1054,7 +1139,7 @@ int rlt_sac_wide_update_actor(rlt_rocm_device* device, const rlt_sac_agent* A, c
     set_noise(a, noise);
     a.out_log_probabilities = A->actor_log_probabilities; a.out_actions = A->actor_actions; a.out_pre_squashing = A->actor_pre_squashing;
     const Optimiser O = {A->actor, A->actor_adam_tensors, A->n_actor_adam_tensors, &A->actor_adam, A->actor_age, &A->log_alpha, &A->alpha_adam, A->alpha_age, 1.0f / (float)A->batch, nullptr};
-    return launch_wide<MODE_ACTOR>(device, a, rlt_div_up(A->batch, ROWS), &O, 1, 0.0f, nullptr);
+    return launch_wide<MODE_ACTOR>(device, a, &O, 1, 0.0f, nullptr);
 }
 
 // ---- TD3: the same kernel with the td3_sampling head (rl/algorithms/td3/operations_generic.h:170-281)
@@ -1082,7 +1167,7 @@ int rlt_td3_wide_update_critic(rlt_rocm_device* device, const rlt_td3_agent* A, 
     a.gamma = A->gamma; a.batch = A->batch; a.obs = A->observation_dim; a.act = A->action_dim;
     a.out_target_action_value = A->target_action_value;
     const Optimiser O = {A->critics[ci], A->critic_adam_tensors[ci], A->n_critic_adam_tensors, &A->critic_adam, A->critic_age[ci], nullptr, nullptr, nullptr, 0.0f, nullptr};
-    return launch_wide<MODE_TD3_CRITIC>(device, a, rlt_div_up(A->batch, ROWS), &O, 1, 0.0f, nullptr);
+    return launch_wide<MODE_TD3_CRITIC>(device, a, &O, 1, 0.0f, nullptr);
 }
 
 // both critics on the agent's batch in one launch (three roles per critic: two target chains and the trained critic), each with its own sampling noise for the target actor's td3_sampling layer:
@@ -1106,7 +1191,7 @@ int rlt_td3_wide_update_critics(rlt_rocm_device* device, const rlt_td3_agent* A,
     for (int k = 0; k < 2; k++)
         O[k] = {A->critics[k], A->critic_adam_tensors[k], A->n_critic_adam_tensors, &A->critic_adam, A->critic_age[k], nullptr, nullptr, nullptr, 0.0f, update_targets ? A->critics_target[k] : nullptr};
     bool targets_done = false;      // the targets' soft update rides along in the optimisers' launch where the tensors correspond
-    const int rc = launch_wide<MODE_TD3_CRITIC>(device, a, rlt_div_up(A->batch, ROWS), O, 2, A->critic_polyak, &targets_done);
+    const int rc = launch_wide<MODE_TD3_CRITIC>(device, a, O, 2, A->critic_polyak, &targets_done);
     if (rc || !update_targets || targets_done) return rc;
     return rlt_rocm_td3_update_critic_targets(device, A);
 }
@@ -1122,7 +1207,7 @@ int rlt_td3_wide_update_actor(rlt_rocm_device* device, const rlt_td3_agent* A, c
     a.gamma = A->gamma; a.batch = A->batch; a.obs = A->observation_dim; a.act = A->action_dim;
     a.out_pre_clip = A->actor_pre_clip;
     const Optimiser O = {A->actor, A->actor_adam_tensors, A->n_actor_adam_tensors, &A->actor_adam, A->actor_age, nullptr, nullptr, nullptr, 0.0f, nullptr};
-    return launch_wide<MODE_TD3_ACTOR>(device, a, rlt_div_up(A->batch, ROWS), &O, 1, 0.0f, nullptr);
+    return launch_wide<MODE_TD3_ACTOR>(device, a, &O, 1, 0.0f, nullptr);
 }
 
 
@@ -1158,14 +1243,16 @@ static int mlp_wide_launch(rlt_rocm_device* device, const rlt_dense_layer* L, in
     a.out1 = L[0].output; a.out2 = L[1].output;
     if (forward_only) for (int l = 0; l < 3; l++) { a.keep_pre[l] = L[l].pre_activations; a.keep_out[l] = L[l].output; }
     a.act3 = L[2].activation;
-    const int IN = L[0].in_dim, OUT = L[2].out_dim, groups = rlt_div_up(batch, ROWS);
+    const int IN = L[0].in_dim, OUT = L[2].out_dim;
     int rc = 0;
     rlt_gradient_net net = {};
     net.in = IN; net.hid = hid; net.out = OUT;
     float* partial = nullptr;
-    // (an output in the memory of the input leaves the contraction over the whole batch without its operand; the blocks are formed out of LDS)
+    // (an output in the memory of the input would leave the contraction over the whole batch without its operand: the rows are kept once more)
     const bool in_place = y && (uintptr_t)y < (uintptr_t)(x + (size_t)(batch - 1) * ldx + IN) && (uintptr_t)x < (uintptr_t)(y + (size_t)(batch - 1) * ldy + OUT);
-    const bool blocks = !forward_only && (sum_blocks(hid, IN, batch, backward_only) || in_place);
+    const bool blocks = !forward_only && sum_blocks(hid, IN, batch, backward_only);
+    const int rows = blocks ? ROWS : tile_rows(device, batch, 1, 1, hid > MAX_H - 16);
+    const int groups = rlt_div_up(batch, rows);
     const int exact = hid * IN + hid + hid * hid + hid + OUT * hid + OUT;
     if (blocks) {
         void* scratch = nullptr;
@@ -1174,10 +1261,12 @@ static int mlp_wide_launch(rlt_rocm_device* device, const rlt_dense_layer* L, in
         a.partial = (float*)scratch;
     } else if (!forward_only) {
         void* scratch = nullptr;
-        if ((rc = rlt_scratch(device, (trained_floats(hid, batch) + rlt_batch_gradients_partial_floats(&net, 1, batch)) * sizeof(float), &scratch))) return rc;
+        const size_t copy_floats = in_place ? ((size_t)batch * IN + 63) & ~(size_t)63 : 0;
+        if ((rc = rlt_scratch(device, (trained_floats(hid, batch) + copy_floats + rlt_batch_gradients_partial_floats(&net, 1, batch)) * sizeof(float), &scratch))) return rc;
         a.kept = place_trained((float*)scratch, hid, batch);
-        partial = (float*)scratch + trained_floats(hid, batch);
-        set_rows(net, a.kept, x, ldx);
+        a.copy_x = in_place ? (float*)scratch + trained_floats(hid, batch) : nullptr;
+        partial = (float*)scratch + trained_floats(hid, batch) + copy_floats;
+        set_rows(net, a.kept, in_place ? a.copy_x : x, in_place ? IN : ldx);
     }
     if ((rc = rlt_mlp_wide_reserve(device))) return rc;
     Copies copies((float*)device->copy_scratch);
@@ -1185,11 +1274,12 @@ static int mlp_wide_launch(rlt_rocm_device* device, const rlt_dense_layer* L, in
     if (!forward_only) copies.backward(a.net);
     if ((rc = copies.launch(device))) return rc;
     const size_t lds_bytes = LDS_FLOATS * sizeof(float);
-#define RLT_LAUNCH_MLP_WIDE(ACT, NT, P, FORM)                                                                                                                   \
+#define RLT_LAUNCH_MLP_WIDE_ROWS(ACT, NT, P, FORM, R)                                                                                                           \
     do {                                                                                                                                                       \
-        RLT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(mlp_wide_kernel<ACT, NT, P, FORM>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes)); \
-        hipLaunchKernelGGL((mlp_wide_kernel<ACT, NT, P, FORM>), dim3(groups), dim3(THREADS), lds_bytes, device->stream, a);                                    \
+        RLT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(mlp_wide_kernel<ACT, NT, P, FORM, R>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes)); \
+        hipLaunchKernelGGL((mlp_wide_kernel<ACT, NT, P, FORM, R>), dim3(groups), dim3(THREADS), lds_bytes, device->stream, a);                                 \
     } while (0)
+#define RLT_LAUNCH_MLP_WIDE(ACT, NT, P, FORM) do { if (rows == 4) RLT_LAUNCH_MLP_WIDE_ROWS(ACT, NT, P, FORM, (FORM == MLP_BLOCKS ? ROWS : FORM == MLP_EVERY ? 4 : 8)); else if (rows == 8) RLT_LAUNCH_MLP_WIDE_ROWS(ACT, NT, P, FORM, (FORM == MLP_BLOCKS ? ROWS : 8)); else RLT_LAUNCH_MLP_WIDE_ROWS(ACT, NT, P, FORM, ROWS); } while (0)
     const bool relu = a.net.act_h == RLT_ACT_RELU;
 #define RLT_LAUNCH_MLP_WIDE_PASS(P, FORM)                                                                                                                       \
     do {                                                                                                                                                       \
@@ -1203,6 +1293,7 @@ static int mlp_wide_launch(rlt_rocm_device* device, const rlt_dense_layer* L, in
     else { if (blocks) RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD_BACKWARD, MLP_BLOCKS); else if (every) RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD_BACKWARD, MLP_EVERY); else RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD_BACKWARD, MLP_ANY); }
 #undef RLT_LAUNCH_MLP_WIDE_PASS
 #undef RLT_LAUNCH_MLP_WIDE
+#undef RLT_LAUNCH_MLP_WIDE_ROWS
     if ((rc = rlt_launch_status(device))) return rc;
     if (forward_only) return 0;
     const Segments seg = segments_of(L);

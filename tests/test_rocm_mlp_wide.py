@@ -44,6 +44,9 @@ CASES = [
     # the workgroups' blocks added up: the narrowest with spare wavefronts, the widest, the last and the first batch of each line, without spare wavefronts
     (16, 3, 65, 1, "relu", True), (255, 1, 97, 16, "fast_tanh", False), (300, 60, 112, 2, "relu", False), (4096, 17, 100, 5, "tanh", True),
     (1024, 65, 80, 3, "tanh", False), (1025, 65, 80, 3, "tanh", False), (768, 20, 144, 4, "relu", True), (769, 20, 144, 4, "relu", True), (257, 1, 150, 1, "sigmoid", False),
+    # tiles of four, eight and sixteen rows: one row of a tile, the last batch of each and the first of the next (widths without tiles of four: from one to sixteen whole units of 16)
+    (5, 17, 256, 6, "relu", False), (1024, 17, 256, 6, "relu", True), (1025, 33, 256, 6, "relu", False), (2048, 17, 256, 1, "relu", False), (2049, 17, 256, 6, "relu", True),
+    (1021, 100, 241, 16, "tanh", False), (9, 17, 128, 2, "relu", False), (2047, 128, 240, 6, "tanh", True), (257, 5, 200, 6, "relu", False), (1030, 17, 200, 6, "fast_tanh", False),
     (4096, 21, 112, 2, "relu", False), (4096, 22, 112, 2, "relu", True), (550, 20, 144, 4, "tanh", False), (551, 20, 144, 4, "tanh", True), (257, 60, 128, 3, "relu", True), (256, 60, 128, 3, "relu", True),
 ]
 

@@ -107,7 +107,9 @@ def test_fused_updates_match_the_checker_and_the_per_operation_path(oracle, rocm
 @pytest.mark.parametrize("batch,obs,act,hidden,hidden_act", [(256, 6, 1, 256, "fast_tanh"), (100, 17, 6, 128, "relu"), (48, 3, 1, 200, "relu"), (256, 27, 8, 256, "relu"),
                                                              (30, 111, 8, 72, "tanh"), (512, 5, 2, 16, "sigmoid"),
                                                              # every network beyond 240 units, and the first width that is not
-                                                             (70, 6, 1, 241, "relu"), (40, 111, 8, 256, "relu"), (70, 6, 1, 240, "relu")])
+                                                             (70, 6, 1, 241, "relu"), (40, 111, 8, 256, "relu"), (70, 6, 1, 240, "relu"),
+                                                             # tiles of four rows: a last tile of one row, the last batch of the critics' tiles of four and the first of eight, and of sixteen
+                                                             (5, 6, 1, 256, "relu"), (257, 40, 3, 256, "relu"), (513, 6, 1, 256, "relu")])
 def test_wider_agents_match_the_checker_on_both_paths(oracle, rocm, batch, obs, act, hidden, hidden_act):
     """Hidden widths other than 64 (the zoo's AcrobotSwingup agent: 6-256-256-2 and 7-256-256-1 at batch 256; Ant-sized: 27 / 8): one launch per update on the
     kernel for widths up to 256 (every network pass of the update by sixteen wavefronts per 16 rows, the optimiser as its last step), and one launch per
@@ -259,7 +261,8 @@ def test_optimiser_in_the_kernel_and_placement_leave_the_same_bits(rocm, batch, 
     assert results[0]["ages"].tolist() == [4] * 4
 
 
-@pytest.mark.parametrize("batch,obs,act,hidden", [(256, 3, 1, 64), (64, 11, 3, 64), (300, 27, 8, 64), (256, 6, 1, 256), (96, 17, 6, 200)])
+@pytest.mark.parametrize("batch,obs,act,hidden", [(256, 3, 1, 64), (64, 11, 3, 64), (300, 27, 8, 64), (256, 6, 1, 256), (96, 17, 6, 200),
+                                                  (300, 6, 1, 256)])      # (the last: tiles of eight rows together, four apart)
 def test_both_critics_in_one_launch_equal_the_separate_calls(oracle, rocm, batch, obs, act, hidden):
     """rlt_rocm_sac_train_critics (both critics on the shared batch and the soft update of the targets in one launch; the noise an array or
     drawn by the kernel from its Philox stream) against train_critic(0), train_critic(1), update_critic_targets: bit for bit, and against the

@@ -162,7 +162,9 @@ def test_fused_updates_match_the_checker_and_the_per_operation_path(oracle, rocm
 @pytest.mark.parametrize("batch,obs,act,hidden,hidden_act", [(256, 6, 1, 256, "fast_tanh"), (100, 17, 6, 128, "relu"), (48, 3, 1, 200, "relu"), (256, 27, 8, 256, "relu"),
                                                              (30, 111, 8, 72, "tanh"), (512, 5, 2, 16, "sigmoid"),
                                                              # every network beyond 240 units, and the first width that is not
-                                                             (70, 6, 1, 241, "relu"), (40, 111, 8, 256, "relu"), (70, 6, 1, 240, "relu")])
+                                                             (70, 6, 1, 241, "relu"), (40, 111, 8, 256, "relu"), (70, 6, 1, 240, "relu"),
+                                                             # tiles of four rows: a last tile of one row, the last batch that every update takes so and the first with tiles of eight, and of sixteen
+                                                             (5, 6, 1, 256, "relu"), (168, 27, 8, 256, "relu"), (169, 40, 3, 256, "relu"), (337, 6, 1, 256, "relu")])
 def test_wider_agents_match_the_checker_on_both_paths(oracle, rocm, batch, obs, act, hidden, hidden_act):
     """The same at hidden widths other than 64 (up to 256; the kernel that takes 16 rows per workgroup of sixteen wavefronts through every pass, with the
     optimiser's launch adding up the workgroups' partial sums): the shapes that the SAC updates are tested at."""
@@ -224,7 +226,8 @@ def test_target_updates_refuse_a_missing_tensor(rocm):
     rocm.sync()
 
 
-@pytest.mark.parametrize("batch,obs,act,hidden,hidden_act", [(256, 27, 8, 256, "relu"), (100, 6, 1, 256, "relu"), (48, 3, 1, 200, "tanh"), (256, 3, 1, 64, "relu")])
+@pytest.mark.parametrize("batch,obs,act,hidden,hidden_act", [(256, 27, 8, 256, "relu"), (100, 6, 1, 256, "relu"), (48, 3, 1, 200, "tanh"), (256, 3, 1, 64, "relu"),
+                                                             (400, 6, 1, 256, "relu")])      # (sixteen rows both ways, where apart tiles of eight would have a compute unit each)
 def test_both_critics_in_one_call_leave_the_bits_of_the_two_calls(rocm, batch, obs, act, hidden, hidden_act):
     """rlt_rocm_td3_train_critics against rlt_rocm_td3_train_critic for critic 0 and then critic 1 on the same batch and target noise, each critic with its own sampling
     noise: three loop steps from the same parameters; every parameter, the gradients, the optimisers' ages and the target values (the second critic's), bit for bit.
