@@ -3,13 +3,15 @@
 // first). The reference walks the sequence on the host and issues a handful of small tensor operations per step.
 //
 // Here the work is split by what depends on time:
-//   * W_i x + b_i for ALL steps is one contraction over sequence*batch rows (gemm.hip), written straight into post_activation;
+//   * W_i x + b_i for ALL steps is one contraction over sequence*batch rows (gemm.hip), written straight into post_activation (at hidden width 64 and up to a thousand rows mostly
+//     formed beside the recurrence, inputs_beside);
 //   * the recurrence runs in ONE launch: batch rows are independent, so no grid-wide synchronisation is needed. At hidden width 64 a
 //     workgroup carries four rows through the sequence on the matrix cores, at 16 and 32 a wavefront 64 / width rows, both with W_h in registers; at other widths a workgroup owns a few
 //     rows and keeps W_h and its rows' hidden state in LDS;
 //   * backward does the same in reverse and stores, per step, the gradient at the gate pre-activations (one copy as the input path sees
 //     it, one as the hidden path sees it, which differs in the n gate by the factor r) and the previous hidden state; the weight
-//     gradients and d_input are then three contractions over sequence*batch rows.
+//     gradients and d_input are then three contractions over sequence*batch rows (the weight gradients, too, mostly beside the recurrence where that is one workgroup per compute unit,
+//     weights_beside).
 #include "common.h"
 #include "gemm.h"
 #include <utility>
@@ -21,7 +23,7 @@ constexpr int GRU_THREADS = 256;
 struct GruArgs {
     rlt_gru_layer L;
     const float* input; const uint8_t* reset;
-    float* d_output; float* buffer_input; float* buffer_hidden; float* h_previous; float* db_hn_partial;
+    float* d_output; float* buffer_input; float* buffer_hidden; float* h_previous; float* db_hn_partial; float* blocks;
     int S, B, rows_per_group;
 };
 
@@ -383,7 +385,6 @@ __global__ __launch_bounds__(256, 2) void gru_forward_mfma_kernel(GruArgs A) {
             cr = mfma4<2>(X, wb[0][4 * s + 2], cr); cn = mfma4<2>(X, wb[2][4 * s + 2], cn); cz = mfma4<2>(X, wb[1][4 * s + 2], cz); \
             cr = mfma4<3>(X, wb[0][4 * s + 3], cr); cn = mfma4<3>(X, wb[2][4 * s + 3], cn); cz = mfma4<3>(X, wb[1][4 * s + 3], cz);
             RLT_GRU_STEPS(a.x, 0) RLT_GRU_STEPS(a.y, 1) RLT_GRU_STEPS(a.z, 2) RLT_GRU_STEPS(a.w, 3)
-#undef RLT_GRU_STEPS
             const float ar = xr + sum_quarters(cr), an = bhn + sum_quarters(cn), az = xz + sum_quarters(cz);
             const float r = FAST ? gate_sigmoid(ar, 1) : hw_sigmoid(ar), z = FAST ? gate_sigmoid(az, 1) : hw_sigmoid(az);
             const float n = FAST ? gate_tanh(xn + an * r, 1) : hw_tanh(xn + an * r);
@@ -397,6 +398,146 @@ __global__ __launch_bounds__(256, 2) void gru_forward_mfma_kernel(GruArgs A) {
         });
     }
 }
+
+// The same with the input gates W_i x + b_i formed beside the recurrence instead of by a launch in front of it (inputs_beside): batches of at most one workgroup per compute unit. Four
+// more wavefronts, one per SIMD, form the gates of the next four steps (4 steps x 4 rows = the sixteen rows of v_mfma_f32_16x16x4) while the recurrence walks through these: wavefront p keeps
+// rows 48 p ... 48 p + 47 of W_i in registers as the B operand, the steps' inputs are staged through LDS a group of four steps ahead and requested another group ahead, the gates reach the
+// recurrence through LDS and never memory. Lane (n, kq) of both operands takes four consecutive inputs of every sixteen, in one 16-byte read
+// (the order of the sums in rows_forward_kernel, gemm.hip: the same bits).
+// Bound: the recurrence's chain and, beside it, 30 instructions of 32 cycles per step at 146 inputs, in which the SIMD's vector unit stands still: a step of 64 x 1,024 sequences takes 1.0 us
+// with 146 inputs, 0.69 with 3. The recurrence goes first (s_setprio); a second barrier per step that kept the others' products out of the recurrence's made it slower (64.5 -> 66.6 us).
+// Launch of the input gates + recurrence / this, 64 steps, 1,024 rows: 146 inputs 77.5 / 65.5 us, 64 inputs 61.1 / 49.0, 3 inputs 57.8 / 44.0.
+constexpr int GP_INPUTS = 160, GP_THREADS = 512, GP_LDX = 164, GP_LDG = 3 * 64 + 16, GP_STEP = GM_ROWS * GP_LDG + 16;      // inputs at most; row strides in LDS: eight lanes' 16-byte reads and sixteen lanes' words of four rows meet no bank twice
+typedef float gru_float4_a4 __attribute__((ext_vector_type(4), aligned(4)));      // four floats wherever they lie: rows of W_i start at any multiple of four bytes
+template <int GROUPS, bool FAST>      // GROUPS: sixteens of inputs, zeros behind the last
+__global__ __launch_bounds__(GP_THREADS) void gru_forward_inputs_kernel(GruArgs A) {
+    constexpr int H = 64, D = 4, E = (GM_ROWS * 16 * GROUPS + 255) / 256, TURNS = GROUPS;      // E: floats of a step that a thread stages; TURNS: reduction steps (of four inputs) between two steps of the recurrence
+    __shared__ __align__(16) float hs[2][H * GM_ROWS];
+    __shared__ __align__(16) float xs[2][4 * GM_ROWS * GP_LDX];      // inputs of four steps: row 4 step + batch row
+    __shared__ float gates[2][D * GP_STEP];                          // their input gates
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kg = lane >> 4, c16 = lane & 15;
+    const int b0 = blockIdx.x * GM_ROWS, I = A.L.input_dim, S = A.S;
+    for (int i = threadIdx.x; i < 2 * 4 * GM_ROWS * GP_LDX; i += GP_THREADS) (&xs[0][0])[i] = 0.f;      // columns beyond the inputs stay zero
+    rlt_lds_barrier();
+    if (wave >= 4) {
+        const int p = wave - 4, tid = threadIdx.x - 256, live = min(GM_ROWS, A.B - b0) * I;      // live: floats of a step that exist
+        float wb[3][GROUPS][4], bias[3];
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            const int gate = 48 * p + 16 * j + c16;
+            const float* const src = A.L.weights_input + (size_t)gate * I;
+            bias[j] = A.L.biases_input[gate];
+#pragma unroll
+            for (int g = 0; g < GROUPS; g++) {
+                const int at = 16 * g + 4 * kg;
+                if (at + 4 <= I) {
+                    const gru_float4_a4 v = *reinterpret_cast<const gru_float4_a4*>(src + at);
+                    wb[j][g][0] = v[0]; wb[j][g][1] = v[1]; wb[j][g][2] = v[2]; wb[j][g][3] = v[3];
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; r++) wb[j][g][r] = at + r < I ? src[at + r] : 0.f;
+                }
+            }
+        }
+        // This thread's floats of a step: where they lie in the step's inputs and in its rows in LDS. What does not exist is read as the last that does and is not used: a row beyond the batch
+        // goes through as some copy, floats beyond the rows go to a column that nothing reads. No branch around a load.
+        int from[E], place[E];
+#pragma unroll
+        for (int e = 0; e < E; e++) { const int i = tid + 256 * e, row = i / I; from[e] = min(i, live - 1); place[e] = row < GM_ROWS ? row * GP_LDX + i - row * I : GP_LDX - 1; }
+        float staged[D][E];
+        auto request = [&](int chunk) {
+#pragma unroll
+            for (int d = 0; d < D; d++) {
+                const float* const src = A.input + ((size_t)min(4 * chunk + d, S - 1) * A.B + b0) * I;
+#pragma unroll
+                for (int e = 0; e < E; e++) staged[d][e] = src[from[e]];
+            }
+        };
+        auto stage = [&](int chunk) {
+#pragma unroll
+            for (int d = 0; d < D; d++)
+#pragma unroll
+                for (int e = 0; e < E; e++) xs[chunk & 1][d * GM_ROWS * GP_LDX + place[e]] = staged[d][e];
+        };
+        gru_floatx4 c[3];
+        auto part = [&](auto number, int chunk) {      // a quarter of the products of a group of four steps
+            constexpr int N = decltype(number)::value, FIRST = TURNS * N, LOW = FIRST / 4, HIGH = (FIRST + TURNS + 3) / 4;
+            const float* const x = &xs[chunk & 1][c16 * GP_LDX + 4 * kg];
+            if (N == 0) for (int j = 0; j < 3; j++) c[j] = gru_floatx4{0.f, 0.f, 0.f, 0.f};
+            float4 a[HIGH - LOW];
+#pragma unroll
+            for (int g = LOW; g < HIGH; g++) a[g - LOW] = *reinterpret_cast<const float4*>(x + 16 * g);
+#pragma unroll
+            for (int s = FIRST; s < FIRST + TURNS; s++) {
+                const float4 v = a[s / 4 - LOW];
+#pragma unroll
+                for (int j = 0; j < 3; j++) c[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(s % 4 == 0 ? v.x : s % 4 == 1 ? v.y : s % 4 == 2 ? v.z : v.w, wb[j][s / 4][s % 4], c[j], 0, 0, 0);
+            }
+            if (N == 3) {
+#pragma unroll
+                for (int j = 0; j < 3; j++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) gates[chunk & 1][kg * GP_STEP + r * GP_LDG + 48 * p + 16 * j + c16] = c[j][r] + bias[j];      // D: row 4 kg + r = step kg, batch row r
+            }
+        };
+        request(0); stage(0); request(1); stage(1); request(2);
+        rlt_lds_barrier();
+        part(std::integral_constant<int, 0>{}, 0); part(std::integral_constant<int, 1>{}, 0); part(std::integral_constant<int, 2>{}, 0); part(std::integral_constant<int, 3>{}, 0);
+        int chunk = 0;
+        for (; 4 * (chunk + 1) < S; chunk++) {
+            rlt_lds_barrier();
+            stage(chunk + 2); request(chunk + 3);      // xs[chunk & 1] was read for the last time before this barrier
+            part(std::integral_constant<int, 0>{}, chunk + 1);
+            rlt_lds_barrier(); part(std::integral_constant<int, 1>{}, chunk + 1);
+            rlt_lds_barrier(); part(std::integral_constant<int, 2>{}, chunk + 1);
+            rlt_lds_barrier(); part(std::integral_constant<int, 3>{}, chunk + 1);
+        }
+        for (int t = 4 * chunk; t < S; t++) rlt_lds_barrier();
+        return;
+    }
+    __builtin_amdgcn_s_setprio(3);
+    const int w = wave, u = 16 * w + c16;
+    float wb[3][16];
+#pragma unroll
+    for (int g = 0; g < 3; g++) {
+        const float4* src = reinterpret_cast<const float4*>(A.L.weights_hidden + (size_t)(g * H + u) * H + 16 * kg);
+#pragma unroll
+        for (int q = 0; q < 4; q++) { const float4 v = src[q]; wb[g][4 * q] = v.x; wb[g][4 * q + 1] = v.y; wb[g][4 * q + 2] = v.z; wb[g][4 * q + 3] = v.w; }
+    }
+    const int row = min(kg, A.B - 1 - b0);
+    const unsigned at = (row * H + u) * sizeof(float), at3 = (row * 3 * H + u) * sizeof(float);
+    const float bhr = A.L.biases_hidden[u], bhz = A.L.biases_hidden[H + u], bhn = A.L.biases_hidden[2 * H + u];
+    const float h0 = A.L.initial_hidden_state[u];
+    const size_t stride = (size_t)A.B * H;
+    float* post = A.L.post_activation + (size_t)b0 * 3 * H; float* npp = A.L.n_pre_pre_activation + (size_t)b0 * H; float* out = A.L.output + (size_t)b0 * H;
+    const int place = ((4 * w + (c16 & 3)) * 4 + kg) * 4 + (c16 >> 2);      // this (row, unit) in hs
+    float h = h0;
+    hs[0][place] = h;
+    rlt_lds_barrier();
+    for (int first = 0; first < S; first += 64) {
+        uint64_t flags = gru_reset_flags<GM_ROWS>(A.reset, first + 1, S, A.B, b0, kg);      // of the steps after these
+        gru_steps<D>(min(64, S - first), [&](auto number, int i) {
+            constexpr int N = decltype(number)::value;
+            __builtin_amdgcn_sched_barrier(0);
+            rlt_lds_barrier();
+            const float4 a = *reinterpret_cast<const float4*>(&hs[N & 1][4 * lane]);
+            const float* const in = &gates[((first + i) >> 2) & 1][N * GP_STEP + row * GP_LDG + u];
+            const float xr = in[0] + bhr, xz = in[H] + bhz, xn = in[2 * H];
+            gru_floatx4 cr = {0.f, 0.f, 0.f, 0.f}, cz = cr, cn = cr;
+            RLT_GRU_STEPS(a.x, 0) RLT_GRU_STEPS(a.y, 1) RLT_GRU_STEPS(a.z, 2) RLT_GRU_STEPS(a.w, 3)
+            const float ar = xr + sum_quarters(cr), an = bhn + sum_quarters(cn), az = xz + sum_quarters(cz);
+            const float r = FAST ? gate_sigmoid(ar, 1) : hw_sigmoid(ar), z = FAST ? gate_sigmoid(az, 1) : hw_sigmoid(az);
+            const float n = FAST ? gate_tanh(xn + an * r, 1) : hw_tanh(xn + an * r);
+            const float o = (1.0f - z) * n + z * h;
+            h = flags & 1 ? h0 : o;       // the next step starts an episode
+            flags >>= 1;
+            hs[(N + 1) & 1][place] = h;
+            gru_at(post, at3) = r; gru_at(post + H, at3) = z; gru_at(post + 2 * H, at3) = n; gru_at(npp, at) = an; gru_at(out, at) = o;
+            post += 3 * stride; npp += stride; out += stride;
+        });
+    }
+}
+#undef RLT_GRU_STEPS
 
 // Reverse pass: the gate gradients of the four rows are the A side (192 reduction indices, quarter kg = the 48 of wavefront kg's units), a wavefront forms d h_prev of
 // its sixteen units. gs (two copies, by the parity of the step): lane (kg, cg, row) of the A operand reads its twelve values in three 16-byte reads (neighbours lie 12
@@ -469,12 +610,206 @@ __global__ __launch_bounds__(256, WAVES) void gru_backward_mfma_kernel(GruArgs A
             c0 = mfma4<2>(a0.X, wb[4 * k + 2], c0); c1 = mfma4<2>(a1.X, wb[16 + 4 * k + 2], c1); c2 = mfma4<2>(a2.X, wb[32 + 4 * k + 2], c2); \
             c0 = mfma4<3>(a0.X, wb[4 * k + 3], c0); c1 = mfma4<3>(a1.X, wb[16 + 4 * k + 3], c1); c2 = mfma4<3>(a2.X, wb[32 + 4 * k + 3], c2);
             RLT_GRU_STEPS(x, 0) RLT_GRU_STEPS(y, 1) RLT_GRU_STEPS(z, 2) RLT_GRU_STEPS(w, 3)
-#undef RLT_GRU_STEPS
             const float sum = sum_quarters(c0 + (c1 + c2));
             carry = from_initial ? 0.f : through + sum;
         });
     }
     if (A.db_hn_partial) gru_at(A.db_hn_partial + (size_t)b0 * H, at) = db_hn;
+}
+
+// The same with the weight gradients formed beside the recurrence instead of by five launches after it that read every step's gate gradients and states back: batches of at most one
+// workgroup per compute unit (weights_beside). Four more wavefronts, one per SIMD, take each step's gate gradients (gs, and the n gate's as the input path sees it), previous states and inputs from
+// LDS: v_mfma_f32_16x16x4 adds a step's four rows (the reduction) to a 16 x 16 tile of the gradient; wavefront p keeps rows 48 p ... 48 p + 47 of dW_i and dW_h in accumulators (three by ten
+// and three by four tiles), the recurrence's lanes add up their own gate gradients for db_i and the n gate's db_h. The inputs are staged through LDS, requested four steps ahead. A workgroup leaves one block of sums,
+// gru_gradient_finish_kernel adds the blocks up in order. Bound: the recurrence's chain and, beside it, 42 instructions of 32 cycles per step at 146 inputs, in which the SIMD's vector unit stands still.
+// Of a step only d_output (accumulated into, as before) and, for a gradient of the input, the input path's gate gradients go to memory.
+// Recurrence + weight gradients / this + the finish, 64 steps, 1,024 rows: 146 inputs 138.5 / 85.7 us, 64 inputs 104.4 / 63.0, 3 inputs 98.9 / 54.3.
+// Relative error against 64 bits (2-norm) at 3 to 146 inputs: dW_i 1.9e-7 ... 3.7e-7 (launches: 1.9e-7 ... 3.8e-7), db_i 1.1e-7 ... 2.3e-7 (1.2e-7 ... 2.2e-7).
+constexpr int GW_INPUTS = 160, GW_LDX = 176, GW_LDH = 80;      // inputs at most; row strides in LDS: sixteen lanes' words of four rows meet no bank twice
+__host__ __device__ constexpr size_t gru_gradient_block(int I) { return (size_t)3 * 64 * (I + 64) + 4 * 64; }      // floats: [192, I], [192, 64], 192 of db_i, 64 of the n gate's db_h
+template <int TILES>      // sixteens of inputs, zeros behind the last
+__global__ __launch_bounds__(GP_THREADS) void gru_backward_weights_kernel(GruArgs A) {
+    constexpr int H = 64, D = 4, E = (GM_ROWS * 16 * TILES + 255) / 256;      // E: floats of a step that a thread stages
+    __shared__ __align__(16) float gs[2][3 * H * GM_ROWS];
+    __shared__ float gn_input[2][H * GM_ROWS];
+    __shared__ float hp_rows[2][GM_ROWS * GW_LDH];
+    __shared__ float xs[2][GM_ROWS * GW_LDX];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kg = lane >> 4, c16 = lane & 15, S = A.S, I = A.L.input_dim;
+    const int b0 = blockIdx.x * GM_ROWS, live_rows = min(GM_ROWS, A.B - b0);
+    float* const block = A.blocks + (size_t)blockIdx.x * gru_gradient_block(I);
+    for (int i = threadIdx.x; i < 2 * GM_ROWS * GW_LDX; i += GP_THREADS) (&xs[0][0])[i] = 0.f;
+    rlt_lds_barrier();
+    if (wave >= 4) {
+        const int p = wave - 4, tid = threadIdx.x - 256, live = live_rows * I;
+        int from[E], place[E];      // as in the forward pass; rows beyond the batch are zeros
+#pragma unroll
+        for (int e = 0; e < E; e++) { const int i = tid + 256 * e, r = i / I; from[e] = min(i, live - 1); place[e] = r < GM_ROWS ? r * GW_LDX + i - r * I : GW_LDX - 1; }
+        const float* next = A.input + ((size_t)(S - 1) * A.B + b0) * I;      // from the last step to the first
+        float staged[D][E];
+        auto request = [&](int i, float (&v)[E]) {      // the steps before the first read the first again
+#pragma unroll
+            for (int e = 0; e < E; e++) v[e] = next[from[e]];
+            next -= i + 1 < S ? (size_t)A.B * I : 0;
+        };
+#pragma unroll
+        for (int d = 0; d < D; d++) request(d, staged[d]);
+        // A operand: lane (m, k) takes gate row 16 (3 p + a) + m of batch row k; in gs unit u of gate g lies at its place + 4 g
+        const int within = (4 * (c16 & 3) + kg);
+        int hidden_at[3], input_at[3];
+        bool n_gate[3];
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+            const int tile = 3 * p + a, g = tile >> 2, pl = 16 * (tile & 3) + within;
+            n_gate[a] = g == 2;
+            hidden_at[a] = 12 * pl + (c16 >> 2) + 4 * g;
+            input_at[a] = 4 * pl + (c16 >> 2);
+        }
+        gru_floatx4 ci[3][TILES], ch[3][4];
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+#pragma unroll
+            for (int j = 0; j < TILES; j++) ci[a][j] = gru_floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < 4; j++) ch[a][j] = gru_floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+        const bool exists = kg < live_rows;      // rows beyond the batch count nothing
+        gru_steps<D>(S, [&](auto number, int i) {
+            constexpr int N = decltype(number)::value;
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int e = 0; e < E; e++) xs[N & 1][place[e]] = tid + 256 * e < live ? staged[N][e] : 0.f;      // (read for the last time before the barrier of the step between)
+            request(i + D, staged[N]);
+            rlt_lds_barrier();
+            float ah[3], ai[3], bh[4], bx[TILES];
+#pragma unroll
+            for (int a = 0; a < 3; a++) {
+                const float v = gs[N & 1][hidden_at[a]], n = gn_input[N & 1][input_at[a]];
+                ah[a] = exists ? v : 0.f;
+                ai[a] = n_gate[a] ? (exists ? n : 0.f) : ah[a];
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) bh[j] = hp_rows[N & 1][kg * GW_LDH + 16 * j + c16];
+#pragma unroll
+            for (int j = 0; j < TILES; j++) bx[j] = xs[N & 1][kg * GW_LDX + 16 * j + c16];
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int a = 0; a < 3; a++) ch[a][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ah[a], bh[j], ch[a][j], 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < TILES; j++)
+#pragma unroll
+                for (int a = 0; a < 3; a++) ci[a][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ai[a], bx[j], ci[a][j], 0, 0, 0);
+        });
+        float* const hidden = block + (size_t)3 * H * I;
+#pragma unroll
+        for (int a = 0; a < 3; a++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int gate = 16 * (3 * p + a) + 4 * kg + r;
+#pragma unroll
+                for (int j = 0; j < TILES; j++) if (16 * j + c16 < I) block[gate * I + 16 * j + c16] = ci[a][j][r];
+#pragma unroll
+                for (int j = 0; j < 4; j++) hidden[gate * H + 16 * j + c16] = ch[a][j][r];
+            }
+        return;
+    }
+    __builtin_amdgcn_s_setprio(3);
+    const int w = wave, u = 16 * w + c16;
+    float wb[48];
+#pragma unroll
+    for (int s = 0; s < 12; s++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) wb[4 * s + k] = A.L.weights_hidden[(size_t)((s >> 2) * H + 16 * kg + 4 * (s & 3) + k) * H + u];
+    const int row = min(kg, live_rows - 1);
+    const bool exists = kg < live_rows;
+    const unsigned at = (row * H + u) * sizeof(float), at3 = (row * 3 * H + u) * sizeof(float);
+    const float h0 = A.L.initial_hidden_state[u];
+    const size_t stride = (size_t)A.B * H, last = (size_t)(S - 1) * stride + (size_t)b0 * H;
+    struct Saved { float r, z, n, npp, dy, hp; };
+    float *post = A.L.post_activation + 3 * last, *npp = A.L.n_pre_pre_activation + last, *dy = A.d_output + last, *state = A.L.output + last;
+    auto request = [&](int i, Saved& v) {      // as above
+        const size_t on = i + 1 < S ? stride : 0;
+        state -= on;
+        v.r = gru_at(post, at3); v.z = gru_at(post + H, at3); v.n = gru_at(post + 2 * H, at3); v.npp = gru_at(npp, at); v.dy = gru_at(dy, at); v.hp = gru_at(state, at);
+        post -= 3 * on; npp -= on; dy -= on;
+    };
+    Saved q[D];
+#pragma unroll
+    for (int d = 0; d < D; d++) if (d < S) request(d, q[d]);
+    float *to_dy = A.d_output + last, *bi = A.buffer_input ? A.buffer_input + 3 * last : nullptr;
+    const int place = ((4 * w + (c16 & 3)) * 4 + kg) * 12 + (c16 >> 2);
+    float carry = 0.f, db_hn = 0.f, db_r = 0.f, db_z = 0.f, db_n = 0.f;
+    for (int back = 0; back < S; back += 64) {
+        const int steps = min(64, S - back);
+        const uint64_t flags = gru_reset_flags<GM_ROWS>(A.reset, S - back - steps, S, A.B, b0, kg);
+        uint64_t high = flags << (64 - steps);
+        gru_steps<D>(steps, [&](auto number, int i) {
+            constexpr int N = decltype(number)::value;
+            __builtin_amdgcn_sched_barrier(0);
+            const Saved cur = q[N];
+            const bool first = back + i + 1 == S, from_initial = first || (high >> 63);
+            high <<= 1;
+            const float hp = from_initial ? h0 : cur.hp;
+            const float dh = cur.dy + carry;
+            const float gz = dh * (hp - cur.n) * cur.z * (1.0f - cur.z);
+            const float gn = dh * (1.0f - cur.z) * (1.0f - cur.n * cur.n);
+            const float gr = gn * cur.npp * cur.r * (1.0f - cur.r);
+            const float gnr = gn * cur.r;
+            float through = dh * cur.z;
+            asm volatile("" : "+v"(through));      // (not formed below by a multiply-add that would keep the entry's z)
+            request(back + i + D, q[N]);
+            float* g = &gs[N & 1][place];
+            g[0] = gr; g[4] = gz; g[8] = gnr;
+            gn_input[N & 1][((4 * w + (c16 & 3)) * 4 + kg) * 4 + (c16 >> 2)] = gn;
+            hp_rows[N & 1][kg * GW_LDH + u] = exists ? hp : 0.f;
+            rlt_lds_barrier();
+            const float4* ga = reinterpret_cast<const float4*>(&gs[N & 1][12 * lane]);
+            const float4 a0 = ga[0], a1 = ga[1], a2 = ga[2];
+            gru_at(to_dy, at) = dh;
+            to_dy -= stride;
+            if (bi) { gru_at(bi, at3) = gr; gru_at(bi + H, at3) = gz; gru_at(bi + 2 * H, at3) = gn; bi -= 3 * stride; }
+            // the reference drops reset samples (t > 0) from the b_hn gradient (their buffer rows are zeroed before that sum, :716-749)
+            db_hn += first || !from_initial ? gnr : 0.f;
+            db_r += gr; db_z += gz; db_n += gn;
+            gru_floatx4 c0 = {0.f, 0.f, 0.f, 0.f}, c1 = c0, c2 = c0;
+            RLT_GRU_STEPS(x, 0) RLT_GRU_STEPS(y, 1) RLT_GRU_STEPS(z, 2) RLT_GRU_STEPS(w, 3)
+            const float sum = sum_quarters(c0 + (c1 + c2));
+            carry = from_initial ? 0.f : through + sum;
+        });
+    }
+    auto rows_sum = [&](float v) { v = exists ? v : 0.f; v += __shfl_xor(v, 16, 64); return v + __shfl_xor(v, 32, 64); };
+    const float sums[4] = {rows_sum(db_r), rows_sum(db_z), rows_sum(db_n), rows_sum(db_hn)};
+    if (kg == 0)
+#pragma unroll
+        for (int g = 0; g < 4; g++) block[gru_gradient_block(I) - 4 * H + g * H + u] = sums[g];
+}
+#undef RLT_GRU_STEPS
+
+// The workgroups' blocks added up in their order into the gradients: 64 elements per workgroup, sixteen lanes with four elements each, every sixteenth block in another group of lanes.
+__global__ __launch_bounds__(256) void gru_gradient_finish_kernel(const float* __restrict__ blocks, int n, int I, float* dW_i, float* db_i, float* dW_h, float* db_h) {
+    constexpr int H = 64;
+    __shared__ float4 part[16][16];
+    const int c = threadIdx.x & 15, group = threadIdx.x >> 4;
+    const size_t size = gru_gradient_block(I);      // a multiple of 64
+    const float4* src = reinterpret_cast<const float4*>(blocks) + (size_t)blockIdx.x * 16 + c;
+    float4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int b = group; b < n; b += 16) { const float4 v = src[(size_t)b * (size / 4)]; s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w; }
+    part[group][c] = s;
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    float sum = 0.f;
+#pragma unroll
+    for (int g = 0; g < 16; g++) sum += reinterpret_cast<const float*>(&part[g][0])[threadIdx.x];
+    const int e = blockIdx.x * 64 + threadIdx.x, inputs = 3 * H * I, weights = inputs + 3 * H * H;
+    if (e < inputs) dW_i[e] += sum;
+    else if (e < weights) dW_h[e - inputs] += sum;
+    else if (e < weights + 3 * H) {
+        const int gate = e - weights;
+        const float d = db_i[gate] + sum;
+        db_i[gate] = d;
+        if (gate < 2 * H) db_h[gate] = d;      // (the reference copies, :679-681)
+    } else db_h[e - weights - H] += sum;
 }
 
 // The same for batches whose steps are bound by memory instead of the chain: thread (w, lane) finishes (row w, unit lane), so that a wavefront's loads and stores are whole rows
@@ -565,6 +900,31 @@ bool layer_ok(const rlt_gru_layer* L) {
     return L && L->weights_input && L->biases_input && L->weights_hidden && L->biases_hidden && L->initial_hidden_state && L->post_activation &&
            L->n_pre_pre_activation && L->output && L->input_dim >= 1 && L->hidden_dim >= 1 && L->hidden_dim <= GRU_THREADS;
 }
+int compute_units(const rlt_rocm_device* device) { return device->compute_units > 0 ? device->compute_units : 256; }
+bool one_group_per_unit(const rlt_rocm_device* device, const rlt_gru_layer* L, int B) { return L->hidden_dim == 64 && rlt_div_up(B, GM_ROWS) <= compute_units(device); }
+int even_sixteens(int columns) { return 2 * rlt_div_up(columns, 32); }
+// Where the input gates / the weight gradients are formed beside the recurrence. The fp32 matrix instructions and the vector unit of a SIMD take turns, so that what goes beside the
+// recurrence lengthens its steps by the time it takes (44 ns per step and sixteen inputs; 54 ns and 46 per sixteen inputs), on as many compute units as there are workgroups, and saves what
+// the launches cost that share the work out over all of them (in ns, fitted to both sides at 3 to 146 inputs, 16 to 64 steps, 16 to 1,024 rows). us, launches / beside, 64 steps:
+//   forward  146 inputs  16 rows 43.0 / 60.9, 512 rows 62.9 / 63.8, 640 rows 66.6 / 64.0, 1,024 rows 77.5 / 65.5; 40 inputs 64 rows 41.4 / 44.3, 256 rows 49.2 / 46.0; 20 inputs 16 rows 40.3 / 38.7
+//   backward 146 inputs 128 rows 73.9 / 75.1, 256 rows 79.8 / 77.3, 1,024 rows 138.5 / 85.7; 64 inputs 64 rows 57.9 / 56.6, 256 rows 70.2 / 58.5; 32 inputs 128 rows 64.3 / 51.7; 3 inputs 64 rows 56.7 / 50.9
+bool inputs_beside(const rlt_rocm_device* device, const rlt_gru_layer* L, int S, int B) {
+    if (!one_group_per_unit(device, L, B) || L->input_dim > GP_INPUTS) return false;
+    return 44.0 * S * even_sixteens(L->input_dim) <= 7000.0 + (0.15 + 0.0033 * L->input_dim) * S * B;
+}
+bool weights_beside(const rlt_rocm_device* device, const rlt_gru_layer* L, int S, int B, size_t room) {      // room: bytes of the caller's workspace that nothing else is kept in
+    if (!one_group_per_unit(device, L, B) || L->input_dim > GW_INPUTS || rlt_div_up(B, GM_ROWS) * gru_gradient_block(L->input_dim) * sizeof(float) > room) return false;
+    return S * (54.0 + 46.0 * even_sixteens(L->input_dim)) <= 12000.0 + (1.0 + 0.009 * L->input_dim) * S * B;
+}
+// the kernels' sixteens of `columns` (at most 160) columns: an even number, so that a few instances do
+template <class F>
+void by_sixteens(int columns, F&& launch) {
+    if (columns <= 32) launch(std::integral_constant<int, 2>{});
+    else if (columns <= 64) launch(std::integral_constant<int, 4>{});
+    else if (columns <= 96) launch(std::integral_constant<int, 6>{});
+    else if (columns <= 128) launch(std::integral_constant<int, 8>{});
+    else launch(std::integral_constant<int, 10>{});
+}
 int rows_per_group(int H) { return GRU_THREADS / H; }
 size_t lds_bytes(int H, bool backward) { return ((size_t)3 * H * H + (size_t)rows_per_group(H) * (backward ? 3 * H : H)) * sizeof(float); }
 
@@ -584,12 +944,20 @@ int rlt_rocm_gru_forward(rlt_rocm_device* device, const rlt_gru_layer* L, const 
     RLT_REQUIRE(layer_ok(L) && input && S > 0 && B > 0);
     const int H = L->hidden_dim;
     if (lds_bytes(H, false) > (size_t)device->lds_bytes) return RLT_E_UNSUPPORTED;
+    GruArgs a = {}; a.L = *L; a.input = input; a.reset = reset; a.S = S; a.B = B; a.rows_per_group = rows_per_group(H);
+    if (inputs_beside(device, L, S, B)) {
+        const dim3 grid4(rlt_div_up(B, GM_ROWS)), block(GP_THREADS);
+        by_sixteens(L->input_dim, [&](auto groups) {
+            constexpr int G = decltype(groups)::value;
+            if (L->fast_tanh) hipLaunchKernelGGL((gru_forward_inputs_kernel<G, true>), grid4, block, 0, device->stream, a); else hipLaunchKernelGGL((gru_forward_inputs_kernel<G, false>), grid4, block, 0, device->stream, a);
+        });
+        return rlt_launch_status(device);
+    }
     // W_i x + b_i for every step at once, into post_activation
     int rc = rlt_gemm_rows_forward(device, input, L->input_dim, L->weights_input, L->biases_input, L->post_activation, 3 * H, S * B, L->input_dim, 3 * H);
     if (rc == RLT_E_UNSUPPORTED)
         rc = rlt_gemm_forward(device, input, L->input_dim, L->weights_input, L->biases_input, RLT_ACT_IDENTITY, nullptr, nullptr, L->post_activation, 3 * H, S * B, L->input_dim, 3 * H);
     if (rc) return rc;
-    GruArgs a = {}; a.L = *L; a.input = input; a.reset = reset; a.S = S; a.B = B; a.rows_per_group = rows_per_group(H);
     if (H == 64 || H == 32 || H == 16) {
         const dim3 grid(rlt_div_up(B, GRU_THREADS / H)), block(GRU_THREADS);      // GRU_THREADS / 64 wavefronts of 64 / H rows
         const bool fast = L->fast_tanh != 0;      // a template parameter: as a run-time switch inside the step it cost 10% at width 64
@@ -620,13 +988,25 @@ int rlt_rocm_gru_backward(rlt_rocm_device* device, const rlt_gru_layer* L, const
     float* buffer_hidden = (float*)w; w += align256((size_t)rows * 3 * H * sizeof(float));
     float* h_previous = (float*)w; w += align256((size_t)rows * H * sizeof(float));
     float* db_hn_partial = (float*)w;
-    GruArgs a = {}; a.L = *L; a.input = input; a.reset = reset; a.d_output = d_output; a.buffer_input = buffer_input; a.buffer_hidden = buffer_hidden;
-    a.h_previous = h_previous; a.db_hn_partial = want_weight_gradients ? db_hn_partial : nullptr; a.S = S; a.B = B; a.rows_per_group = rows_per_group(H);
+    GruArgs a = {}; a.L = *L; a.input = input; a.reset = reset; a.d_output = d_output; a.S = S; a.B = B;
+    float* const blocks = d_input ? buffer_hidden : buffer_input;
+    if (want_weight_gradients && weights_beside(device, L, S, B, (size_t)((char*)workspace + workspace_bytes - (char*)blocks))) {
+        const int groups = rlt_div_up(B, GM_ROWS);
+        a.buffer_input = d_input ? buffer_input : nullptr; a.blocks = blocks;
+        by_sixteens(I, [&](auto tiles) { hipLaunchKernelGGL(gru_backward_weights_kernel<decltype(tiles)::value>, dim3(groups), dim3(GP_THREADS), 0, device->stream, a); });
+        hipLaunchKernelGGL(gru_gradient_finish_kernel, dim3((unsigned)(gru_gradient_block(I) / 64)), dim3(256), 0, device->stream, (const float*)blocks, groups, I, L->d_weights_input, L->d_biases_input,
+                           L->d_weights_hidden, L->d_biases_hidden);
+        const int rc = rlt_launch_status(device);
+        if (rc || !d_input) return rc;
+        return rlt_gemm_backward_input(device, buffer_input, 3 * H, L->weights_input, d_input, I, nullptr, 0, 0, rows, I, 3 * H);      // :688
+    }
+    a.buffer_input = buffer_input; a.buffer_hidden = buffer_hidden;
+    a.h_previous = h_previous; a.db_hn_partial = want_weight_gradients ? db_hn_partial : nullptr; a.rows_per_group = rows_per_group(H);
     if (H == 64 || H == 32 || H == 16) {
         const dim3 grid(rlt_div_up(B, GRU_THREADS / H)), block(GRU_THREADS);
         if (H == 64) {
             const dim3 grid4(rlt_div_up(B, GM_ROWS));
-            const int units = device->compute_units > 0 ? device->compute_units : 256;
+            const int units = compute_units(device);
             if (backward_by_rows(units, S, B)) hipLaunchKernelGGL(gru_backward_rows_kernel, grid4, block, 0, device->stream, a);
             else if ((int)grid4.x > 3 * units) hipLaunchKernelGGL((gru_backward_mfma_kernel<2, 4>), grid4, block, 0, device->stream, a);
             else hipLaunchKernelGGL((gru_backward_mfma_kernel<4, 2>), grid4, block, 0, device->stream, a);

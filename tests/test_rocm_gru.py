@@ -149,3 +149,16 @@ def test_gru_at_the_edges_of_the_kernels_that_keep_a_layer_in_registers(oracle, 
     want, got = run_pair(oracle, rocm, S, B, I, H, 35, True)
     for k in KEYS:
         assert rel_err(got[k], want[k]) <= 2e-5, (k, rel_err(got[k], want[k]))
+
+
+@pytest.mark.parametrize("want_d_input", [False, True])
+@pytest.mark.parametrize("case", [(1, 1, 1), (2, 3, 15), (3, 5, 16), (4, 4, 17), (5, 2, 31), (22, 4, 146), (23, 4, 146), (40, 6, 146), (65, 7, 145), (130, 9, 158), (66, 6, 159), (71, 5, 160),
+                                  (70, 3, 161), (24, 1021, 40), (24, 1024, 33), (24, 1025, 33), (24, 1022, 146), (25, 1023, 159), (25, 1023, 160), (26, 1024, 161), (25, 998, 130), (27, 1001, 100), (64, 40, 64), (64, 129, 64)])
+def test_gru_with_input_gates_and_weight_gradients_beside_the_recurrence(oracle, rocm, case, want_d_input):
+    """Width 64 over at most 1,024 rows: inputs around whole sixteens, the most that the accumulators and the registers of W_i hold (160) and one more, steps around the groups of
+    four, last workgroups of one to four rows, workspaces that just hold the blocks of sums and that do not, both sides of the lines to the launches. Tolerance as for the long batch above."""
+    print("case", case, want_d_input, flush=True)
+    S, B, I = case
+    want, got = run_pair(oracle, rocm, S, B, I, 64, 37, True, want_d_input=want_d_input)
+    for k in KEYS:
+        assert rel_err(got[k], want[k]) <= 2e-5, (k, rel_err(got[k], want[k]))
