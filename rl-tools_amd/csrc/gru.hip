@@ -626,7 +626,7 @@ __global__ __launch_bounds__(256, WAVES) void gru_backward_mfma_kernel(GruArgs A
 // Recurrence + weight gradients / this + the finish, 64 steps, 1,024 rows: 146 inputs 138.5 / 85.7 us, 64 inputs 104.4 / 63.0, 3 inputs 98.9 / 54.3.
 // Relative error against 64 bits (2-norm) at 3 to 146 inputs: dW_i 1.9e-7 ... 3.7e-7 (launches: 1.9e-7 ... 3.8e-7), db_i 1.1e-7 ... 2.3e-7 (1.2e-7 ... 2.2e-7).
 constexpr int GW_INPUTS = 160, GW_LDX = 176, GW_LDH = 80;      // inputs at most; row strides in LDS: sixteen lanes' words of four rows meet no bank twice
-__host__ __device__ constexpr size_t gru_gradient_block(int I) { return (size_t)3 * 64 * (I + 64) + 4 * 64; }      // floats: [192, I], [192, 64], 192 of db_i, 64 of the n gate's db_h
+__host__ __device__ constexpr size_t gru_gradient_block(int I) { return (size_t)3 * 64 * (I + 64 + 1) + 64; }      // floats: [192, I], [192, 64], 192 of db_i, 64 of the n gate's db_h
 template <int TILES>      // sixteens of inputs, zeros behind the last
 __global__ __launch_bounds__(GP_THREADS) void gru_backward_weights_kernel(GruArgs A) {
     constexpr int H = 64, D = 4, E = (GM_ROWS * 16 * TILES + 255) / 256;      // E: floats of a step that a thread stages
@@ -785,16 +785,109 @@ __global__ __launch_bounds__(GP_THREADS) void gru_backward_weights_kernel(GruArg
 }
 #undef RLT_GRU_STEPS
 
-// The workgroups' blocks added up in their order into the gradients: 64 elements per workgroup, sixteen lanes with four elements each, every sixteenth block in another group of lanes.
-__global__ __launch_bounds__(256) void gru_gradient_finish_kernel(const float* __restrict__ blocks, int n, int I, float* dW_i, float* db_i, float* dW_h, float* db_h) {
-    constexpr int H = 64;
+// The weight gradients after a backward pass that has left the gate gradients and the previous states of every step in memory: dW_i, dW_h and db_i of all rows in one launch (SUBSETS = H / 16
+// times 48 gate rows). A workgroup takes two 16-column tiles of the inputs or of the states and a share of the rows, a wavefront 48 gate rows (three tiles; at the smaller widths also a
+// share of the workgroup's rows): six tiles of v_mfma_f32_16x16x4 in accumulators, operands straight from memory (lane (m, k): row k of four, sixteen consecutive columns), requested eight
+// steps of four rows ahead. Every share leaves a block of sums. Bound: latency, 2.3 us of matrix instructions per wavefront at 4,096 rows of 146 inputs among loads that memory answers in one.
+// As a contraction and a sum per gradient and a launch for db_h these were five launches. Backward pass, five / this and the finish, us: 64 steps, 146 inputs, width 64: 16 rows 53.7 / 42.9,
+// 64 rows 64.4 / 49.6, 256 rows 79.6 / 61.3; width 32: 64 rows 64.6 / 51.4, 1,024 rows 115.1 / 81.2; width 16: 64 rows 42.0 / 32.5. Relative error against 64 bits (2-norm) over these: dW_i
+// 1.4e-7 ... 3.5e-7 (five launches 1.9e-7 ... 5.2e-7), dW_h 2.0e-7 ... 4.2e-7 (2.4e-7 ... 4.5e-7).
+struct GradientArgs { const float *d_input_path, *d_hidden_path, *input, *h_previous; float* blocks; int rows, I, input_pairs; };
+__host__ __device__ constexpr size_t gradient_block(int H, int I) { return (size_t)3 * H * (I + H + 1); }      // floats: [3 H, I], [3 H, H], 3 H of db_i
+template <int SUBSETS>
+__global__ __launch_bounds__(256) void gru_gradients_kernel(GradientArgs A) {
+    constexpr int H = 16 * SUBSETS, PARTS = 4 / SUBSETS, D = 8, CHAINS = 4;      // CHAINS: accumulators per tile, a quarter of the steps each (shorter sums: a smaller error)
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), m = lane & 15, k = lane >> 4, subset = wave % SUBSETS;
+    const int share = blockIdx.y * PARTS + wave / SUBSETS, shares = gridDim.y * PARTS, steps = (A.rows + 3) >> 2;
+    const int first = (int)((long long)steps * share / shares), end = (int)((long long)steps * (share + 1) / shares);
+    const bool hidden = (int)blockIdx.x >= A.input_pairs;
+    const int pair = hidden ? blockIdx.x - A.input_pairs : blockIdx.x, width = hidden ? H : A.I;
+    const float* const d = (hidden ? A.d_hidden_path : A.d_input_path) + 48 * subset + m;
+    const float* const x = hidden ? A.h_previous : A.input;
+    const int c0 = min(32 * pair + m, width - 1), c1 = min(32 * pair + 16 + m, width - 1);      // columns beyond the width repeat the last one and are not stored
+    struct Step { float a[3], b[2]; };
+    auto request = [&](int s, Step& v) {      // steps and rows that do not exist read the last row
+        const size_t row = (size_t)min(4 * s + k, A.rows - 1);
+#pragma unroll
+        for (int t = 0; t < 3; t++) v.a[t] = d[row * 3 * H + 16 * t];
+        v.b[0] = x[row * width + c0]; v.b[1] = x[row * width + c1];
+    };
+    gru_floatx4 c[CHAINS][3][2];
+    float bias[CHAINS][3] = {};
+#pragma unroll
+    for (int i = 0; i < CHAINS; i++)
+#pragma unroll
+        for (int t = 0; t < 3; t++) c[i][t][0] = c[i][t][1] = gru_floatx4{0.f, 0.f, 0.f, 0.f};
+    Step v[D], ahead[D];
+#pragma unroll
+    for (int i = 0; i < D; i++) request(first + i, v[i]);
+    for (int s = first; s < end; s += D) {
+#pragma unroll
+        for (int i = 0; i < D; i++) request(s + D + i, ahead[i]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < D; i++) {
+            if (s + D > end || 4 * (s + i) + 3 >= A.rows) {      // the last group of a share, the last rows: what does not exist counts nothing
+                const bool exists = s + i < end && 4 * (s + i) + k < A.rows;
+#pragma unroll
+                for (int t = 0; t < 3; t++) v[i].a[t] = exists ? v[i].a[t] : 0.f;
+                v[i].b[0] = exists ? v[i].b[0] : 0.f; v[i].b[1] = exists ? v[i].b[1] : 0.f;
+            }
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int t = 0; t < 3; t++) c[i % CHAINS][t][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i].a[t], v[i].b[j], c[i % CHAINS][t][j], 0, 0, 0);
+            if (blockIdx.x == 0)
+#pragma unroll
+                for (int t = 0; t < 3; t++) bias[i % CHAINS][t] += v[i].a[t];
+        }
+#pragma unroll
+        for (int i = 0; i < D; i++) v[i] = ahead[i];
+    }
+    float* const block = A.blocks + (size_t)share * gradient_block(H, A.I);
+    float* const to = block + (hidden ? (size_t)3 * H * A.I : 0);
+#pragma unroll
+    for (int t = 0; t < 3; t++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int gate = 48 * subset + 16 * t + 4 * k + r, col = 32 * pair + 16 * j + m;
+                if (col < width) to[(size_t)gate * width + col] = (c[0][t][j][r] + c[1][t][j][r]) + (c[2][t][j][r] + c[3][t][j][r]);
+            }
+    if (blockIdx.x == 0)
+#pragma unroll
+        for (int t = 0; t < 3; t++) {
+            float sum = (bias[0][t] + bias[1][t]) + (bias[2][t] + bias[3][t]);
+            sum += __shfl_xor(sum, 16, 64); sum += __shfl_xor(sum, 32, 64);
+            if (k == 0) block[(size_t)3 * H * (A.I + H) + 48 * subset + 16 * t + m] = sum;
+        }
+}
+
+// Blocks of sums added up in their order into the gradients: 64 elements per workgroup, sixteen lanes with four elements each, every sixteenth block in another group of lanes. The last
+// H / 4 workgroups take four elements each of the n gate's db_h from blocks of its own (n_hidden of them, `hidden_stride` floats apart), every 256th in another thread.
+__global__ __launch_bounds__(256) void gru_gradient_finish_kernel(const float* __restrict__ blocks, int n, size_t stride, const float* __restrict__ hidden, int n_hidden, size_t hidden_stride, int H, int I,
+                                                                  float* dW_i, float* db_i, float* dW_h, float* db_h) {
     __shared__ float4 part[16][16];
-    const int c = threadIdx.x & 15, group = threadIdx.x >> 4;
-    const size_t size = gru_gradient_block(I);      // a multiple of 64
-    const float4* src = reinterpret_cast<const float4*>(blocks) + (size_t)blockIdx.x * 16 + c;
+    const int c = threadIdx.x & 15, group = threadIdx.x >> 4, count = (int)gradient_block(H, I);      // a multiple of four
+    const int quad = (int)blockIdx.x - ((int)gridDim.x - H / 4);
+    const bool last = quad >= 0;
+    const float* const src = last ? hidden + 4 * quad : blocks + min((int)blockIdx.x * 64 + 4 * c, count - 4);
+    const int many = last ? n_hidden : n, by = last ? 256 : 16;
+    const size_t apart = last ? hidden_stride : stride;
     float4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
-    for (int b = group; b < n; b += 16) { const float4 v = src[(size_t)b * (size / 4)]; s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w; }
+    for (int b = last ? threadIdx.x : group; b < many; b += by) { const float4 v = *reinterpret_cast<const float4*>(src + (size_t)b * apart); s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w; }
+    if (last) {
+        s.x = rlt_wave_sum(s.x); s.y = rlt_wave_sum(s.y); s.z = rlt_wave_sum(s.z); s.w = rlt_wave_sum(s.w);
+        if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6][0] = s;
+        __syncthreads();
+        if (threadIdx.x < 4) {
+            const float* const v = reinterpret_cast<const float*>(&part[0][0]) + threadIdx.x;
+            db_h[2 * H + 4 * quad + threadIdx.x] += (v[0] + v[64]) + (v[128] + v[192]);
+        }
+        return;
+    }
     part[group][c] = s;
     __syncthreads();
     if (threadIdx.x >= 64) return;
@@ -804,12 +897,12 @@ __global__ __launch_bounds__(256) void gru_gradient_finish_kernel(const float* _
     const int e = blockIdx.x * 64 + threadIdx.x, inputs = 3 * H * I, weights = inputs + 3 * H * H;
     if (e < inputs) dW_i[e] += sum;
     else if (e < weights) dW_h[e - inputs] += sum;
-    else if (e < weights + 3 * H) {
+    else if (e < count) {
         const int gate = e - weights;
         const float d = db_i[gate] + sum;
         db_i[gate] = d;
         if (gate < 2 * H) db_h[gate] = d;      // (the reference copies, :679-681)
-    } else db_h[e - weights - H] += sum;
+    }
 }
 
 // The same for batches whose steps are bound by memory instead of the chain: thread (w, lane) finishes (row w, unit lane), so that a wavefront's loads and stores are whole rows
@@ -907,14 +1000,37 @@ int even_sixteens(int columns) { return 2 * rlt_div_up(columns, 32); }
 // recurrence lengthens its steps by the time it takes (44 ns per step and sixteen inputs; 54 ns and 46 per sixteen inputs), on as many compute units as there are workgroups, and saves what
 // the launches cost that share the work out over all of them (in ns, fitted to both sides at 3 to 146 inputs, 16 to 64 steps, 16 to 1,024 rows). us, launches / beside, 64 steps:
 //   forward  146 inputs  16 rows 43.0 / 60.9, 512 rows 62.9 / 63.8, 640 rows 66.6 / 64.0, 1,024 rows 77.5 / 65.5; 40 inputs 64 rows 41.4 / 44.3, 256 rows 49.2 / 46.0; 20 inputs 16 rows 40.3 / 38.7
-//   backward 146 inputs 128 rows 73.9 / 75.1, 256 rows 79.8 / 77.3, 1,024 rows 138.5 / 85.7; 64 inputs 64 rows 57.9 / 56.6, 256 rows 70.2 / 58.5; 32 inputs 128 rows 64.3 / 51.7; 3 inputs 64 rows 56.7 / 50.9
+//   backward 146 inputs 256 rows 61.6 / 78.0, 512 rows 81.1 / 80.0, 1,024 rows 132.7 / 85.7; 64 inputs 256 rows 52.5 / 58.6, 512 rows 64.3 / 60.2; 3 inputs 64 rows 47.5 / 50.6, 1,024 rows 79.1 / 55.3;
+//            146 inputs 1,024 rows 24 steps 57.7 / 44.0
 bool inputs_beside(const rlt_rocm_device* device, const rlt_gru_layer* L, int S, int B) {
     if (!one_group_per_unit(device, L, B) || L->input_dim > GP_INPUTS) return false;
     return 44.0 * S * even_sixteens(L->input_dim) <= 7000.0 + (0.15 + 0.0033 * L->input_dim) * S * B;
 }
 bool weights_beside(const rlt_rocm_device* device, const rlt_gru_layer* L, int S, int B, size_t room) {      // room: bytes of the caller's workspace that nothing else is kept in
     if (!one_group_per_unit(device, L, B) || L->input_dim > GW_INPUTS || rlt_div_up(B, GM_ROWS) * gru_gradient_block(L->input_dim) * sizeof(float) > room) return false;
-    return S * (54.0 + 46.0 * even_sixteens(L->input_dim)) <= 12000.0 + (1.0 + 0.009 * L->input_dim) * S * B;
+    return S * (54.0 + 46.0 * even_sixteens(L->input_dim)) <= 3400.0 + (0.35 + 0.0037 * L->input_dim) * S * B;
+}
+// The weight gradients of gru_gradients_kernel: pairs of column tiles, shares of the rows (workgroups for the whole chip, but at least eight steps of four rows to a wavefront; once, twice ... so many that no sum is longer than
+// 256 steps, for its error's sake), blocks of sums
+struct GradientShape { int columns, shares, blocks; };
+GradientShape gradient_shape(const rlt_rocm_device* device, const rlt_gru_layer* L, int rows) {
+    const int H = L->hidden_dim, parts = H == 64 ? 1 : H == 32 ? 2 : 4, columns = rlt_div_up(L->input_dim, 32) + rlt_div_up(H, 32);
+    const int chip = compute_units(device) / columns > 1 ? compute_units(device) / columns : 1, most = rows / (32 * parts) > 1 ? rows / (32 * parts) : 1;
+    const int shares = most < chip ? most : chip * rlt_div_up(rows, 4 * 256 * parts * chip);
+    return {columns, shares, shares * parts};
+}
+// Where they are (widths 16, 32, 64): not where width 64 meets 65,536 rows and more of 66 to 160 inputs, an even number, which wgrad_wide_kernel (gemm.hip) reads once. us of the backward pass
+// with contractions and sums per gradient / this, width 64: 146 inputs 16 steps 4,000 rows 141 / 127, 64 steps 2,048 rows 230 / 249, 16 steps 8,192 rows 247 / 303; 33 inputs 64 steps 2,048 rows 200 / 179,
+// 170 inputs 64 steps 1,024 rows 167 / 143; width 32, 146 inputs 64 steps 4,096 rows 296 / 243; width 16, 146 inputs 32 steps 8,192 rows 262 / 147.
+bool gradients_in_one(const rlt_gru_layer* L, int S, int B) {
+    const int H = L->hidden_dim, I = L->input_dim;
+    return (H == 16 || H == 32 || H == 64) && I <= 1024 && !(H == 64 && (size_t)S * B >= 65536 && I > 64 && I <= 160 && I % 2 == 0);
+}
+int finish_gradients(rlt_rocm_device* device, const rlt_gru_layer* L, const float* blocks, int n, size_t stride, const float* hidden, int n_hidden, size_t hidden_stride) {
+    const int H = L->hidden_dim, I = L->input_dim;
+    hipLaunchKernelGGL(gru_gradient_finish_kernel, dim3((unsigned)((gradient_block(H, I) + 63) / 64 + H / 4)), dim3(256), 0, device->stream, blocks, n, stride, hidden, n_hidden, hidden_stride, H, I,
+                       L->d_weights_input, L->d_biases_input, L->d_weights_hidden, L->d_biases_hidden);
+    return rlt_launch_status(device);
 }
 // the kernels' sixteens of `columns` (at most 160) columns: an even number, so that a few instances do
 template <class F>
@@ -994,9 +1110,7 @@ int rlt_rocm_gru_backward(rlt_rocm_device* device, const rlt_gru_layer* L, const
         const int groups = rlt_div_up(B, GM_ROWS);
         a.buffer_input = d_input ? buffer_input : nullptr; a.blocks = blocks;
         by_sixteens(I, [&](auto tiles) { hipLaunchKernelGGL(gru_backward_weights_kernel<decltype(tiles)::value>, dim3(groups), dim3(GP_THREADS), 0, device->stream, a); });
-        hipLaunchKernelGGL(gru_gradient_finish_kernel, dim3((unsigned)(gru_gradient_block(I) / 64)), dim3(256), 0, device->stream, (const float*)blocks, groups, I, L->d_weights_input, L->d_biases_input,
-                           L->d_weights_hidden, L->d_biases_hidden);
-        const int rc = rlt_launch_status(device);
+        const int rc = finish_gradients(device, L, blocks, groups, gru_gradient_block(I), blocks + gradient_block(H, I), groups, gru_gradient_block(I));
         if (rc || !d_input) return rc;
         return rlt_gemm_backward_input(device, buffer_input, 3 * H, L->weights_input, d_input, I, nullptr, 0, 0, rows, I, 3 * H);      // :688
     }
@@ -1020,7 +1134,16 @@ int rlt_rocm_gru_backward(rlt_rocm_device* device, const rlt_gru_layer* L, const
     }
     int rc = rlt_launch_status(device);
     if (rc) return rc;
-    if (want_weight_gradients) {
+    float* shares = nullptr;
+    const GradientShape shape = gradient_shape(device, L, rows);
+    if (want_weight_gradients && gradients_in_one(L, S, B) && rlt_scratch(device, shape.blocks * gradient_block(H, I) * sizeof(float), (void**)&shares) == 0) {
+        const GradientArgs g = {buffer_input, buffer_hidden, input, h_previous, shares, rows, I, rlt_div_up(I, 32)};
+        const dim3 grid(shape.columns, shape.shares), block(256);
+        if (H == 64) hipLaunchKernelGGL(gru_gradients_kernel<4>, grid, block, 0, device->stream, g);
+        else if (H == 32) hipLaunchKernelGGL(gru_gradients_kernel<2>, grid, block, 0, device->stream, g);
+        else hipLaunchKernelGGL(gru_gradients_kernel<1>, grid, block, 0, device->stream, g);
+        if ((rc = finish_gradients(device, L, shares, shape.blocks, gradient_block(H, I), db_hn_partial, B, H))) return rc;
+    } else if (want_weight_gradients) {
         if ((rc = rlt_gemm_wgrad(device, buffer_input, 3 * H, input, I, L->d_weights_input, L->d_biases_input, rows, I, 3 * H, false, true))) return rc;       // :677-678
         if ((rc = rlt_gemm_wgrad(device, buffer_hidden, 3 * H, h_previous, H, L->d_weights_hidden, nullptr, rows, H, 3 * H, false, true))) return rc;         // :693-742
         hipLaunchKernelGGL(gru_bias_hidden_kernel, dim3(H), dim3(256), 0, device->stream, (const float*)db_hn_partial, B, H, (const float*)L->d_biases_input, L->d_biases_hidden);

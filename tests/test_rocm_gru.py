@@ -162,3 +162,16 @@ def test_gru_with_input_gates_and_weight_gradients_beside_the_recurrence(oracle,
     want, got = run_pair(oracle, rocm, S, B, I, 64, 37, True, want_d_input=want_d_input)
     for k in KEYS:
         assert rel_err(got[k], want[k]) <= 2e-5, (k, rel_err(got[k], want[k]))
+
+
+@pytest.mark.parametrize("case", [(1, 1, 1, 16), (1, 2, 33, 32), (3, 1, 32, 64), (1, 31, 5, 16), (3, 43, 65, 32), (5, 26, 31, 64), (9, 57, 64, 64), (4, 257, 1, 16), (2, 1100, 3, 32), (33, 128, 97, 16), (64, 71, 146, 64),
+                                  (40, 1100, 66, 64), (31, 2114, 66, 64), (32, 2048, 66, 64), (32, 2048, 67, 64), (3, 5, 1024, 16), (3, 5, 1025, 16)])
+def test_gru_weight_gradients_of_all_steps_in_one_launch(oracle, rocm, case):
+    """Shares of the rows of less than eight steps of four rows, last steps of one to three rows, inputs around pairs of column tiles, more sequences than a workgroup has threads, both sides
+    of the line to the kernel that keeps a whole gradient in one workgroup and of the most inputs. Tolerance as for the long batch above."""
+    print("case", case, flush=True)
+    S, B, I, H = case
+    for want_d_input in (False, True):
+        want, got = run_pair(oracle, rocm, S, B, I, H, 38, True, want_d_input=want_d_input)
+        for k in KEYS:
+            assert rel_err(got[k], want[k]) <= 2e-5, (k, rel_err(got[k], want[k]))
