@@ -74,12 +74,26 @@ __device__ __forceinline__ float rlt_fast_tanh(float x) {
     float x2 = x * x;
     return x * (27.0f + x2) / (27.0f + 9.0f * x2);
 }
+// tanh without a branch: x + x^3 P(x^2) below 1 (P fitted to the least relative error, 5e-9), 1 - 2 / (e^{2 |x|} + 1) above, on v_exp_f32 and v_rcp_f32 with the argument's rounding error
+// carried along and one Newton step. Against 64 bits over every float from 2^-11 to 12: relative error at most 8.3e-8, root mean square 2.4e-8 below 0.625, 3.0e-8 to 0.75, 2.7e-8 to 1, 2.1e-8 to 2
+// (tanhf: at most 1.5e-7; 2.4e-8, 4.5e-8, 3.4e-8, 2.1e-8). The library's branch at 0.625 keeps the compiler from interleaving the activations of a lane: each waits for its own chain.
+__device__ __forceinline__ float rlt_tanh(float x) {
+    const float a = fabsf(x), z = a * a;
+    float p = fmaf(-0x1.77dd2ep-12f, z, 0x1.2da4f6p-9f);
+    p = fmaf(p, z, -0x1.0460c4p-7f); p = fmaf(p, z, 0x1.600992p-6f); p = fmaf(p, z, -0x1.b96222p-5f); p = fmaf(p, z, 0x1.110be2p-3f); p = fmaf(p, z, -0x1.55553cp-2f);
+    const float small = fmaf(a * z, p, a);      // a NaN ends up here
+    constexpr float C = 2.8853900817779268f, C_REST = (float)(2.8853900817779268 - (double)C);      // 2 / ln 2
+    const float c = fminf(a, 10.0f), hi = c * C, lo = fmaf(c, C_REST, fmaf(c, C, -hi));
+    const float e = __builtin_amdgcn_exp2f(hi), d = fmaf(e, lo * 0.69314718f, e) + 1.0f, q = __builtin_amdgcn_rcpf(d);
+    const float large = fmaf(-2.0f, fmaf(fmaf(-d, q, 1.0f), q, q), 1.0f);
+    return copysignf(a >= 1.0f ? large : small, x);
+}
 __device__ __forceinline__ float rlt_act(float x, int f) {
     switch (f) {
         case RLT_ACT_RELU: return x > 0.0f ? x : 0.0f;
         // the reference's GELU constant is FRAC_2_SQRTPI * SQRT1_2 * 0.5, half of the textbook sqrt(2/pi) (nn/activation_functions.h:33-36)
         case RLT_ACT_GELU: { const float a = 0.3989422804014327f; return 0.5f * (x + x * tanhf(a * (0.044715f * x * x * x + x))); }
-        case RLT_ACT_TANH: return tanhf(x);
+        case RLT_ACT_TANH: return rlt_tanh(x);
         case RLT_ACT_FAST_TANH: return rlt_fast_tanh(x);
         case RLT_ACT_SIGMOID: return 1.0f / (1.0f + expf(-x));
         default: return x;
@@ -93,7 +107,7 @@ __device__ __forceinline__ float rlt_dact(float x, int f) {
             float t = tanhf(a * (b * x * x * x + x));
             return 0.5f * (1.0f + t) + 0.5f * x * (1.0f - t * t) * a * (3.0f * b * x * x + 1.0f);
         }
-        case RLT_ACT_TANH: { float t = tanhf(x); return 1.0f - t * t; }
+        case RLT_ACT_TANH: { float t = rlt_tanh(x); return 1.0f - t * t; }
         case RLT_ACT_FAST_TANH: { float t = rlt_fast_tanh(x); return 1.0f - t * t; }
         case RLT_ACT_SIGMOID: { float s = 1.0f / (1.0f + expf(-x)); return s * (1.0f - s); }
         default: return 1.0f;

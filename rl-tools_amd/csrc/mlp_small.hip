@@ -15,6 +15,7 @@
 // Bound: latency. One round is 460 matrix instructions per SIMD (14.7 K cycles at 105 -> 64 -> 64 -> 8), between LDS round trips and the activations' chains, and 141 KB of LDS leave room
 // for one workgroup per compute unit: two wavefronts per SIMD instead of one (four that had all columns of their rows) took PPO's pair at 8,192 rows from 30.0 to 25.6 us and the
 // head 64 -> 64 -> 4 of a sequence model at 65,536 rows from 56.2 to 47.2 us, with the same sums in the same order.
+// Both halves form the loss, for two of a lane's four rows each (stage 2.3 -> 1.6 us; PPO's pair, with the tanh of common.h that has no branch, 25.3 -> 25.0).
 #include "mlp_small.h"
 #include "optim.h"
 #include "xcd_reduce.h"
@@ -55,9 +56,9 @@ constexpr size_t lds_floats(int nt1c) {
 }
 
 // global loads of one tile of 16 rows, issued together: the inputs (lane = column, up to two columns per lane) and what the loss needs of the
-// rows this lane will hold after the forward pass (rows 4 kk + v, column r); columns beyond the extent are clamped here and masked later.
+// rows whose loss this lane forms after the forward pass (rows 4 kk + 2 half + u, column r); columns beyond the extent are clamped here and masked later.
 // `vrows`: the rows' indices, requested a round earlier so that nothing waits for them here.
-struct TileRegs { float xa[8], xb[8], in0[4], in1[4], in2[4]; };
+struct TileRegs { float xa[8], xb[8], in0[2], in1[2], in2[2]; };
 __device__ __forceinline__ void request_tile(const SmallArgs& A, uint32_t vrows, int lane, int half, TileRegs& T) {
     const int r = lane & 15, kk = lane >> 4;
     const int c0 = min(lane, A.in - 1), c1 = min(64 + lane, A.in - 1), c = min(r, A.out - 1);
@@ -68,10 +69,9 @@ __device__ __forceinline__ void request_tile(const SmallArgs& A, uint32_t vrows,
         T.xb[row] = A.in > 64 ? src[c1] : 0.f;
     }
 #pragma unroll
-    for (int v = 0; v < 4; v++) {
-        const size_t row = (size_t)(uint32_t)__shfl((int)vrows, 4 * kk + v, 64);
+    for (int v = 0; v < 2; v++) {
+        const size_t row = (size_t)(uint32_t)__shfl((int)vrows, 4 * kk + 2 * half + v, 64);
         T.in0[v] = T.in1[v] = T.in2[v] = 0.f;
-        if (half != 0) continue;      // the loss is the first half's
         if (A.loss == LOSS_GIVEN) T.in0[v] = A.d_output[row * A.ldd + c];
         else if (A.loss == LOSS_MSE) T.in0[v] = A.target[row * A.ldt + c];
         else { T.in0[v] = A.actions[row * A.ld_actions + c]; T.in1[v] = A.advantages[row * A.ld_adv]; T.in2[v] = A.log_probs[row * A.ld_lp]; }
@@ -181,7 +181,7 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K) {
 
     RLT_TICK(3);
     // this wavefront's share of the weight gradients: rows 16 rt + 4 kk + v of half the columns of dW1 and of dW2 (tiles NT1H half + nt and 2 half + nt), and, in the second
-    // half (the first has the loss), columns 16 rt + r of dW3 (rows 4 kk + v)
+    // half, columns 16 rt + r of dW3 (rows 4 kk + v)
     constexpr int NT1H = NT1C / 2;
     floatx4 aW1[NT1H], aW2[2], aW3a = zero4, aW3b = zero4;
 #pragma unroll
@@ -201,9 +201,9 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K) {
             if (64 + lane < 16 * NT1C) xs[row * SX + 64 + lane] = (rok && 64 + lane < IN) ? (T.xb[j] - sm1) * sp1 : 0.f;
         }
     RLT_TICK(4);
-        float in0[4], in1[4], in2[4];
+        float in0[2], in1[2], in2[2];
 #pragma unroll
-        for (int v = 0; v < 4; v++) { in0[v] = T.in0[v]; in1[v] = T.in1[v]; in2[v] = T.in2[v]; }
+        for (int v = 0; v < 2; v++) { in0[v] = T.in0[v]; in1[v] = T.in1[v]; in2[v] = T.in2[v]; }
         rlt_lds_barrier();      // both halves' rows of the tile are in place
         // the next round's loads travel while this one is computed, with row indices requested a round earlier
         if (round + n_blocks < n_rounds) {
@@ -275,8 +275,8 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K) {
         const lptr hls = LAYERS == 3 ? h2s : h1s, hls_all = LAYERS == 3 ? h2s_all : h1s_all;      // the last hidden layer's activations
 
     RLT_TICK(7);
-        // layer 3 (two chains of matrix instructions) and the gradient at its pre-activations
-        if (half == 0) {
+        // layer 3 (two chains of matrix instructions, in both halves: the loss takes longer than they do, and each half forms it for two of a lane's four rows) and the gradient at its
+        // pre-activations
         floatx4 y0 = zero4, y1 = zero4;
 #pragma unroll
         for (int s = 0; s < 16; s += 2) {
@@ -284,10 +284,10 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K) {
             y1 = mfma16(hls[r * HS + 16 * kk + s + 1], w3s[r * HS + 16 * kk + s + 1], y1);
         }
 #pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const int row = row0 + 4 * kk + v;
+        for (int v = 0; v < 2; v++) {
+            const int row = row0 + 4 * kk + 2 * half + v;
             const bool ok = row < A.batch && r < OUT;
-            const float yv = rlt_act((y0[v] + y1[v]) + b3r, A.act3);
+            const float yv = rlt_act((half ? y0[2 + v] + y1[2 + v] : y0[v] + y1[v]) + b3r, A.act3);
             if (A.y && ok) A.y[(size_t)row * A.ldy + r] = yv;
             float d = 0.f;
             if (A.loss == LOSS_GIVEN) d = in0[v];
@@ -310,8 +310,7 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K) {
             }
             const float dp = ok ? d * rlt_dact_from_output(yv, A.act3) : 0.f;
             s3 += dp;
-            d3s[(4 * kk + v) * D3S + r] = dp;
-        }
+            d3s[(4 * kk + 2 * half + v) * D3S + r] = dp;
         }
     RLT_TICK(8);
         rlt_lds_barrier();      // every wavefront's last hidden activations and d_pre3 are in place
@@ -445,19 +444,21 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K) {
     }
     RLT_TICK(16);
     // ... the bias and log_std gradients, which every wavefront holds for its own rows and columns, summed in the order of the row tiles through LDS
-    const lptr sums = (lptr)lds_raw;        // [ROW_TILES][N_SUMS]; the weights are no longer needed
+    const lptr sums = (lptr)lds_raw, sums2 = sums + ROW_TILES * N_SUMS;        // [ROW_TILES][N_SUMS], the loss's of the second half [ROW_TILES][2 MAX_OUT]; the weights are no longer needed
 #pragma unroll
     for (int nt = 0; nt < 2; nt++) { s1[nt] = groups_sum(s1[nt]); s2[nt] = groups_sum(s2[nt]); }
     s3 = groups_sum(s3); gls = groups_sum(gls);
     if (kk == 0) {
 #pragma unroll
         for (int nt = 0; nt < 2; nt++) { sums[rt * N_SUMS + 32 * half + 16 * nt + r] = s1[nt]; sums[rt * N_SUMS + H + 32 * half + 16 * nt + r] = s2[nt]; }
-        if (half == 0) { sums[rt * N_SUMS + 2 * H + r] = s3; sums[rt * N_SUMS + 2 * H + MAX_OUT + r] = gls; }
+        const lptr loss_sums = half == 0 ? sums + rt * N_SUMS + 2 * H : sums2 + rt * 2 * MAX_OUT;
+        loss_sums[r] = s3; loss_sums[MAX_OUT + r] = gls;
     }
     rlt_lds_barrier();
     if (threadIdx.x < N_SUMS) {
         const int i = threadIdx.x;
-        const float total = (sums[i] + sums[N_SUMS + i]) + (sums[2 * N_SUMS + i] + sums[3 * N_SUMS + i]);
+        float total = (sums[i] + sums[N_SUMS + i]) + (sums[2 * N_SUMS + i] + sums[3 * N_SUMS + i]);
+        if (i >= 2 * H) { const lptr s = sums2 + i - 2 * H; total += (s[0] + s[2 * MAX_OUT]) + (s[4 * MAX_OUT] + s[6 * MAX_OUT]); }
         if (i < H) dst[o_b1 + i] = total;
         else if (i < 2 * H) dst[o_b2 + i - H] = total;
         else if (i < 2 * H + MAX_OUT) { if (i - 2 * H < OUT) dst[o_b3 + i - 2 * H] = total; }
@@ -466,7 +467,7 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K) {
     RLT_TICK(17);
     if (K.xr.enabled)       // the block joins those of the workgroups on this XCD: eight blocks of sums per network leave the launch
         rlt_xcd_group_reduce<THREADS>(K.xr, xgroup, block >> 3, n_blocks >> 3, xepoch, A.partial + (size_t)(block & 7) * A.count, A.count,
-                                      (second ? K.xsum[1] : K.xsum[0]) + (size_t)(block & 7) * A.count, (__attribute__((address_space(3))) int*)((lptr)lds_raw + 4 * N_SUMS));
+                                      (second ? K.xsum[1] : K.xsum[0]) + (size_t)(block & 7) * A.count, (__attribute__((address_space(3))) int*)(sums2 + ROW_TILES * 2 * MAX_OUT));
     RLT_TICK(18);
 #ifdef RLT_SMALL_PROFILE
     __builtin_amdgcn_s_waitcnt(0);
