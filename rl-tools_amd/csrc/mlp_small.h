@@ -26,6 +26,10 @@ bool rlt_mlp3s_pair_supported(const rlt_dense_layer* a, int n_a, const rlt_dense
 // d_log_std); *stepped then is true. Otherwise the gradients are formed as without `steps` and the caller steps the optimisers.
 struct rlt_mlp3s_step { const rlt_adam_tensor* tensors; int n; const rlt_adam_parameters* parameters; uint32_t* age; };
 
+// optional: this launch's minibatch is number `index` of `n` that follow each other with the same networks and optimisers, nothing of the library's in between but launches that leave the handle's scratch
+// buffer and the networks alone. The step of a minibatch may then wait for the next one's launch; after the last all are done. loss_before: where the loss of the one before goes (NULL: nowhere).
+struct rlt_mlp3s_epoch { int index, n; float* loss_before; };
+
 // The same actor pass and the critic's forward + MSE gradient + backward (:289-300) in ONE launch, each network on half of the compute units,
 // straight from the dataset: every input column has the dataset's row stride `ld`, and minibatch row b is dataset row rows[b] (rows == NULL: b).
 // Means [batch x action_dim] and values [batch] are written packed; out_critic_loss (optional, critic output width 1) receives
@@ -39,7 +43,7 @@ int rlt_mlp3s_ppo_actor_critic(rlt_rocm_device* device, const rlt_dense_layer* a
                                const float* target_values, float mse_scale, float* out_critic_loss, int ld, const uint32_t* rows, int batch,
                                const float* actor_std_mean = nullptr, const float* actor_std_precision = nullptr,
                                const float* critic_std_mean = nullptr, const float* critic_std_precision = nullptr,
-                               const rlt_mlp3s_step* steps = nullptr, bool* stepped = nullptr);
+                               const rlt_mlp3s_step* steps = nullptr, bool* stepped = nullptr, const rlt_mlp3s_epoch* epoch = nullptr);
 
 // For kernels that write blocks of partial sums in this file's layout (dW1 [64 x in], db1 [64], dW2 [64 x 64], db2 [64], dW3 [out x 64], db3 [out],
 // extra [16]): the floats per block, and the launch that adds `groups` blocks up in block order into the layers' gradients (overwrite != 0:

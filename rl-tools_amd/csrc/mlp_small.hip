@@ -39,6 +39,7 @@ struct SmallArgs {
     float epsilon_clip, advantage_epsilon; int normalize_advantage;
     float* partial; int count;      // per workgroup: dW1 [64 x in], db1 [64], dW2 [64 x 64], db2 [64], dW3 [out x 64], db3 [out], extra [16]
     float* d_input; int ld_di;      // optional: gradient with respect to x, written at row b
+    int step_log_std;               // with a step in front: log_std is one of the stepped tensors
     const float* std_mean; const float* std_precision;      // optional standardize layer in front: the network reads (x - mean) * precision (the factor where it is not 0)
 };
 
@@ -96,8 +97,74 @@ __device__ unsigned long long rlt_small_spans[512][2];
 // gradient at layer 1's pre-activations is formed directly from the output layer's.
 // xr (optional): the blocks of partial sums are added up per XCD inside the launch (xcd_reduce.h); network j's eight blocks of sums then lie at xsum[j]
 struct SmallLaunch { SmallArgs a0, a1; int groups0; rlt_xcd_reduce_args xr; float* xsum[2]; };
-template <int ACT_H, int NT1C, int LAYERS>
-__global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K) {
+
+// The optimisers' step of one minibatch at the head of the launch of the next (rlt_mlp3s_epoch). Each XCD steps a copy of the network of its own: the workgroups of a network on one XCD take a
+// slice of its elements each (the eight XCDs' sums of the launch before, Adam), wait for each other through that XCD's L2 and load the weights from the copy. No workgroup waits for another XCD, and the
+// copies stay equal, since the same sums in the same order make them. The slice's loads travel with the row indices, Adam's arithmetic runs while the rows travel.
+// PPO at 8,192 rows, both networks 105 -> 64 -> 64: a launch of its own for the step takes 6.7 us per minibatch, at the head of the pass it adds @@.
+struct SmallStepTensor { uint32_t begin, count, flags; float scale, add; float *parameters, *first, *second, *gradient; };      // elements [begin, begin + count) of a block of partial sums
+struct SmallStep {
+    SmallStepTensor t[RLT_TAIL_TENSORS]; int n, count, stride;      // floats per block; floats per array of a copy
+    int from_tensors;               // the first step reads the tensors, the others the copies
+    const float* sums;              // the eight XCDs' blocks of sums
+    float* copies;                  // per XCD: parameters, first and second moments, in the order of a block
+    rlt_adam_parameters p; const uint32_t* age; uint32_t steps_before;      // the age word is advanced at the end of the epoch
+    float* extra_out; uint32_t extra_offset; float extra_scale;      // optional: one more sum
+};
+struct SmallSteps { static constexpr bool present = true; SmallStep s[2]; };
+struct NoSteps { static constexpr bool present = false; };
+struct StepElement { bool stepped; uint32_t flags; float scale, add, m, v, param, blocks[RLT_XCD_GROUPS]; };
+// everything that the step of element e reads (stepped: a tensor has it)
+__device__ __forceinline__ void request_element(const SmallStep& S, const float* copy, uint32_t e, uint32_t end, StepElement& E) {
+    const uint32_t ec = min(e, end - 1u);
+    const float *p = copy + ec, *m = p + S.stride, *v = m + S.stride;
+    E.stepped = false; E.flags = 0; E.scale = 1.f; E.add = 0.f;
+    for (int i = 0; i < S.n; i++)
+        if (ec - S.t[i].begin < S.t[i].count) {
+            E.stepped = true; E.flags = S.t[i].flags; E.scale = S.t[i].scale; E.add = S.t[i].add;
+            if (S.from_tensors) { const uint32_t j = ec - S.t[i].begin; p = S.t[i].parameters + j; m = S.t[i].first + j; v = S.t[i].second + j; }
+        }
+    E.param = __builtin_nontemporal_load(p); E.m = __builtin_nontemporal_load(m); E.v = __builtin_nontemporal_load(v);      // (no line of a copy stays in this compute unit's cache)
+#pragma unroll
+    for (int g = 0; g < RLT_XCD_GROUPS; g++) E.blocks[g] = S.sums[(size_t)g * S.count + ec];
+}
+// sum of the blocks in the order of rlt_sum_of_blocks
+__device__ __forceinline__ float element_sum(const StepElement& E) {
+    float q[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) { float s = 0.f; s += E.blocks[2 * i]; s += E.blocks[2 * i + 1]; q[i] = s; }
+    return (q[0] + q[1]) + (q[2] + q[3]);
+}
+static_assert(RLT_XCD_GROUPS == 8, "element_sum adds quarters of two blocks");
+// the last step of an epoch: from the copy of XCD 0 into the tensors, whose gradients receive the last minibatch's; blocks [0, blocks0) take the first network
+__global__ __launch_bounds__(256) void mlp3s_step_kernel(SmallSteps K, int blocks0, uint32_t* age0, uint32_t* age1, uint32_t* tickets) {
+    const bool second = (int)blockIdx.x >= blocks0;
+    const SmallStep& S = K.s[second ? 1 : 0];
+    const uint32_t e = (second ? blockIdx.x - blocks0 : blockIdx.x) * 256u + threadIdx.x;
+    const uint32_t age = *S.age + S.steps_before;
+    StepElement E;
+    request_element(S, S.copies, e, S.count, E);
+    float bc1, bc2;
+    rlt_adam_bias_corrections(S.p, age, bc1, bc2);
+    const float sum = element_sum(E);
+    const float g = rlt_scaled_sum(sum, E.scale, E.add);
+    rlt_adam_values(S.p, E.flags, g, bc1, bc2, E.m, E.v, E.param);
+    for (int i = 0; i < S.n; i++) {
+        const uint32_t j = e - S.t[i].begin;
+        if (j < S.t[i].count) { S.t[i].gradient[j] = g; S.t[i].first[j] = E.m; S.t[i].second[j] = E.v; S.t[i].parameters[j] = E.param; }
+    }
+    if (S.extra_out && e == S.extra_offset) *S.extra_out = sum * S.extra_scale;
+    asm volatile("" :: "v"(bc1), "v"(bc2));      // every thread has read the age before the workgroup's ticket is drawn
+    rlt_lds_barrier();
+    if (threadIdx.x == 0 && rlt_last_through(tickets, blockIdx.x, gridDim.x)) { *age0 += K.s[0].steps_before + 1u; *age1 += K.s[1].steps_before + 1u; }
+}
+
+// a parameter of the pass; with a step in front another compute unit wrote it in this launch
+template <bool STEP> __device__ __forceinline__ float load_parameter(const float* p) { if (STEP) return rlt_load_shared<1>(p); return *p; }
+
+template <int ACT_H, int NT1C, int LAYERS, class STEPS>
+__global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K, STEPS steps) {
+    constexpr bool STEP = STEPS::present;
     RLT_TICK(0);
 #ifdef RLT_SMALL_PROFILE
     if (threadIdx.x == 0) rlt_small_spans[blockIdx.x][0] = wall_clock64();
@@ -106,6 +173,8 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K) {
     const int groups0 = K.groups0;
     const bool second = (int)blockIdx.x >= groups0;
     const SmallArgs& A = second ? K.a1 : K.a0;
+    const float *W1 = A.W1, *b1 = A.b1, *W2 = A.W2, *b2 = A.b2, *W3 = A.W3, *b3 = A.b3, *log_std = A.log_std;
+    auto load = [](const float* p) { return load_parameter<STEP>(p); };
     const int block = second ? blockIdx.x - groups0 : blockIdx.x, n_blocks = second ? gridDim.x - groups0 : groups0;
     const int lane = threadIdx.x & 63, r = lane & 15, kk = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);      // wavefront-uniform: addresses derived from it are computed on the scalar unit
@@ -131,24 +200,62 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K) {
     const int xgroup = (second ? RLT_XCD_GROUPS : 0) + (block & 7);      // with the XCD-level sums: this workgroup's group (network, XCD)
     uint32_t xepoch = 0;
     if (K.xr.enabled) xepoch = rlt_xcd_epoch(K.xr, xgroup);
+    const int member = block >> 3, n_members = (n_blocks - (block & 7) + 7) >> 3;
+    if constexpr (STEP) {
+        const SmallStep& S = steps.s[second ? 1 : 0];
+        float* const copy = S.copies + (size_t)(block & 7) * 3 * S.stride;
+        // whole lines of 128 bytes: no cache holds a line that two compute units write
+        const uint32_t count = S.count, chunk = ((count + n_members - 1) / n_members + 31u) & ~31u, begin = min(count, member * chunk), end = min(count, begin + chunk);
+        constexpr int E = 2;
+        StepElement el[E];
+        const uint32_t age = *S.age + S.steps_before;
+#pragma unroll
+        for (int u = 0; u < E; u++) request_element(S, copy, begin + u * THREADS + threadIdx.x, max(end, 1u), el[u]);
+        __builtin_amdgcn_sched_barrier(0);
+        request_tile(A, rows_next, lane, half, T);
+        float bc1, bc2;
+        rlt_adam_bias_corrections(S.p, age, bc1, bc2);
+        for (uint32_t base = begin; base < end; base += E * THREADS) {
+            if (base != begin) {
+#pragma unroll
+                for (int u = 0; u < E; u++) request_element(S, copy, base + u * THREADS + threadIdx.x, end, el[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < E; u++) {
+                const uint32_t e = base + u * THREADS + threadIdx.x;
+                if (e >= end) continue;
+                const float sum = element_sum(el[u]);
+                if (el[u].stepped) {
+                    rlt_adam_values(S.p, el[u].flags, rlt_scaled_sum(sum, el[u].scale, el[u].add), bc1, bc2, el[u].m, el[u].v, el[u].param);
+                    copy[e] = el[u].param; copy[S.stride + e] = el[u].m; copy[2 * S.stride + e] = el[u].v;
+                }
+                if (S.extra_out && (block & 7) == 0 && e == S.extra_offset) *S.extra_out = sum * S.extra_scale;
+            }
+        }
+        // a member that gives up has set the fault word: the epoch's results are void, and the tensors are as they were until its last launch
+        rlt_xcd_wait(K.xr, xgroup, member, n_members, xepoch + 1u, false, (__attribute__((address_space(3))) int*)(lptr)lds_raw);
+        xepoch++;
+        W1 = copy; b1 = W1 + H * IN; W2 = b1 + H; b2 = W2 + H * H; W3 = b2 + H; b3 = W3 + OUT * H;
+        if (A.step_log_std) log_std = b3 + OUT;
+    }
     float v1[H / WAVES][2], v2[H * H / THREADS], v3[MAX_OUT * H / THREADS];
 #pragma unroll
     for (int j = 0; j < H / WAVES; j++) {
-        const float* src = A.W1 + (size_t)(wave * (H / WAVES) + j) * IN;
-        v1[j][0] = src[min(lane, IN - 1)];
-        v1[j][1] = IN > 64 ? src[min(64 + lane, IN - 1)] : 0.f;
+        const float* src = W1 + (size_t)(wave * (H / WAVES) + j) * IN;
+        v1[j][0] = load(src + min(lane, IN - 1));
+        v1[j][1] = IN > 64 ? load(src + min(64 + lane, IN - 1)) : 0.f;
     }
 #pragma unroll
-    for (int u = 0; u < H * H / THREADS; u++) v2[u] = LAYERS == 3 ? A.W2[u * THREADS + threadIdx.x] : 0.f;
+    for (int u = 0; u < H * H / THREADS; u++) v2[u] = LAYERS == 3 ? load(W2 + u * THREADS + threadIdx.x) : 0.f;
 #pragma unroll
-    for (int u = 0; u < MAX_OUT * H / THREADS; u++) v3[u] = A.W3[min(u * THREADS + (int)threadIdx.x, OUT * H - 1)];
+    for (int u = 0; u < MAX_OUT * H / THREADS; u++) v3[u] = load(W3 + min(u * THREADS + (int)threadIdx.x, OUT * H - 1));
     float b1r[2], b2r[2];
 #pragma unroll
-    for (int nt = 0; nt < 2; nt++) { b1r[nt] = A.b1[16 * (2 * half + nt) + r]; b2r[nt] = LAYERS == 3 ? A.b2[16 * (2 * half + nt) + r] : 0.f; }
-    const float b3r = A.b3[min(r, OUT - 1)];
+    for (int nt = 0; nt < 2; nt++) { b1r[nt] = load(b1 + 16 * (2 * half + nt) + r); b2r[nt] = LAYERS == 3 ? load(b2 + 16 * (2 * half + nt) + r) : 0.f; }
+    const float b3r = load(b3 + min(r, OUT - 1));
     float ls = 0.f, adv_mean = 0.f, adv_std = 0.f;
     if (A.loss == LOSS_PPO) {
-        ls = A.log_std[min(r, OUT - 1)];
+        ls = load(log_std + min(r, OUT - 1));
         if (A.normalize_advantage) { adv_mean = A.stats[0]; adv_std = A.stats[1]; }
     }
     // the standardize layer's constants for this lane's columns (nn/layers/standardize/operations_generic.h:68-86); without one: x - 0 times 1
@@ -159,8 +266,9 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K) {
         sp0 = sp0 != 0.f ? sp0 : 1.f; sp1 = sp1 != 0.f ? sp1 : 1.f;
     }
     __builtin_amdgcn_sched_barrier(0);      // the loads above are issued before the first wait for the row indices
-    request_tile(A, rows_next, lane, half, T);
+    if constexpr (!STEP) request_tile(A, rows_next, lane, half, T);
     RLT_TICK(1);
+    if constexpr (STEP) rlt_lds_barrier();      // every wavefront has read the word of the wait
     // weights into LDS, rows padded to SX (zero beyond the input width, so the padded reduction steps add nothing)
     {
 #pragma unroll
@@ -466,7 +574,7 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K) {
     }
     RLT_TICK(17);
     if (K.xr.enabled)       // the block joins those of the workgroups on this XCD: eight blocks of sums per network leave the launch
-        rlt_xcd_group_reduce<THREADS>(K.xr, xgroup, block >> 3, n_blocks >> 3, xepoch, A.partial + (size_t)(block & 7) * A.count, A.count,
+        rlt_xcd_group_reduce<THREADS>(K.xr, xgroup, member, n_members, xepoch, A.partial + (size_t)(block & 7) * A.count, A.count,
                                       (second ? K.xsum[1] : K.xsum[0]) + (size_t)(block & 7) * A.count, (__attribute__((address_space(3))) int*)(sums2 + ROW_TILES * 2 * MAX_OUT));
     RLT_TICK(18);
 #ifdef RLT_SMALL_PROFILE
@@ -561,10 +669,40 @@ bool map_step(const SmallJob& job, const rlt_mlp3s_step& S, bool extra_is_gradie
     return covered == 63u && extra_covered == (extra_is_gradient && job.extra != nullptr);
 }
 
+// The steps of two mapped optimisers for launches that read the blocks' elements: false unless the stepped parameters are the ones that the networks read, every tensor is complete and the ages
+// are two words. Tensors that follow each other everywhere are one, as a network laid out as an arena is: an element looks for its tensor.
+constexpr int EPOCH_MIN_GROUPS = 64;
+bool fill_steps(const SmallJob* jobs, const rlt_mlp3s_step* steps, const uint32_t (*offsets)[12], const float (*scales)[12], const float (*adds)[12], SmallSteps& S) {
+    if (!steps[0].parameters || !steps[1].parameters || !steps[0].age || !steps[1].age || steps[0].age == steps[1].age) return false;
+    for (int j = 0; j < 2; j++) {
+        const rlt_dense_layer* L = jobs[j].L;
+        SmallStep& D = S.s[j];
+        D.count = jobs[j].a.count; D.p = *steps[j].parameters; D.age = steps[j].age;
+        const float* at[7] = {L[0].weights, L[0].biases, L[1].weights, L[1].biases, L[2].weights, L[2].biases, jobs[j].a.log_std};
+        const uint32_t size[7] = {(uint32_t)(H * L[0].in_dim), H, H * H, H, (uint32_t)(L[2].out_dim * H), (uint32_t)L[2].out_dim, N_EXTRA};
+        const uint32_t flags = (D.p.enable_weight_decay ? 1u : 0u) | (D.p.enable_bias_lr_factor ? 2u : 0u);      // those that make a difference
+        for (uint32_t k = 0, begin = 0; k < 7; begin += size[k], k++)
+            for (int i = 0; i < steps[j].n; i++) {
+                const rlt_adam_tensor& T = steps[j].tensors[i];
+                if (!T.parameters || !T.gradient || !T.first_moment || !T.second_moment) return false;
+                const uint32_t o = offsets[j][i];
+                if (begin >= o && begin < o + T.count && T.parameters + (begin - o) != at[k]) return false;      // a tensor covers whole layers' buffers
+                if (o != begin) continue;
+                if (D.n > 0) {
+                    SmallStepTensor& B = D.t[D.n - 1];
+                    if (B.begin + B.count == o && B.parameters + B.count == T.parameters && B.first + B.count == T.first_moment && B.second + B.count == T.second_moment &&
+                        B.gradient + B.count == T.gradient && ((B.flags ^ T.flags) & flags) == 0 && B.scale == scales[j][i] && B.add == adds[j][i]) { B.count += T.count; continue; }
+                }
+                D.t[D.n++] = {o, T.count, T.flags, scales[j][i], adds[j][i], T.parameters, T.first_moment, T.second_moment, T.gradient};
+            }
+    }
+    return true;
+}
+
 // one or two networks in one launch; two only if they share the hidden activation and the input-width bucket. `steps` (optional, one per
 // job): the optimisers' steps follow in one launch that reads the blocks of partial sums itself (a gradient's extra values only for job 0;
 // job 1's single extra value is an output); *stepped tells whether they did, else the gradients were formed and the caller steps.
-int launch(rlt_rocm_device* device, SmallJob* jobs, int n_jobs, const rlt_mlp3s_step* steps = nullptr, bool* stepped = nullptr) {
+int launch(rlt_rocm_device* device, SmallJob* jobs, int n_jobs, const rlt_mlp3s_step* steps = nullptr, bool* stepped = nullptr, const rlt_mlp3s_epoch* epoch = nullptr) {
     if (stepped) *stepped = false;
     int groups[2] = {0, 0};
     size_t offset[2] = {0, 0}, total = 0;
@@ -589,14 +727,24 @@ int launch(rlt_rocm_device* device, SmallJob* jobs, int n_jobs, const rlt_mlp3s_
     const bool steps_mapped = steps && n_jobs == 2 && jobs[0].overwrite && jobs[1].overwrite && (!jobs[1].extra || jobs[1].n_extra == 1) &&
                               map_step(jobs[0], steps[0], true, offsets[0], scales[0], adds[0]) && map_step(jobs[1], steps[1], false, offsets[1], scales[1], adds[1]);
     SmallLaunch K = {};
-    // sums per XCD inside the launch: where workgroup i runs on XCD i % 8, every network's workgroups are a multiple of 8 (at most 32 per XCD)
-    // and the grid is resident as a whole
+    // sums per XCD inside the launch: where workgroup i runs on XCD i % 8 (a network's workgroups that are equal modulo 8 then share one, wherever its first lies; at most 32) and the grid is
+    // resident as a whole
     bool xcd_sums = device->update_tail && device->xcd_stride == 8 && groups[0] + groups[n_jobs - 1] * (n_jobs - 1) <= device->compute_units;
     size_t xsum_offset[2] = {0, 0};
     for (int j = 0; j < n_jobs; j++) {
-        xcd_sums = xcd_sums && groups[j] % RLT_XCD_GROUPS == 0 && groups[j] >= 2 * RLT_XCD_GROUPS && groups[j] <= RLT_XCD_GROUPS * RLT_XCD_MAX_MEMBERS;
+        xcd_sums = xcd_sums && groups[j] >= 2 * RLT_XCD_GROUPS && groups[j] <= RLT_XCD_GROUPS * RLT_XCD_MAX_MEMBERS;
         xsum_offset[j] = total; total += ((size_t)RLT_XCD_GROUPS * jobs[j].a.count + 63) & ~(size_t)63;
     }
+    // An epoch's steps at the head of the next minibatch's launch: a step takes each workgroup @@RULE
+    SmallSteps S = {};
+    const bool in_epoch = epoch && xcd_sums && steps_mapped && epoch->n > 1 && fill_steps(jobs, steps, offsets, scales, adds, S) && groups[0] >= EPOCH_MIN_GROUPS && groups[1] >= EPOCH_MIN_GROUPS;
+    size_t copies_offset[2] = {0, 0}, second_sums[2] = {0, 0};
+    if (in_epoch)
+        for (int j = 0; j < 2; j++) {
+            S.s[j].stride = (jobs[j].a.count + 63) & ~63;
+            second_sums[j] = total; total += ((size_t)RLT_XCD_GROUPS * jobs[j].a.count + 63) & ~(size_t)63;
+            copies_offset[j] = total; total += (size_t)RLT_XCD_GROUPS * 3 * S.s[j].stride;
+        }
     void* scratch = nullptr;
     int rc = rlt_scratch(device, total * sizeof(float), &scratch);
     if (rc) return rc;
@@ -608,17 +756,30 @@ int launch(rlt_rocm_device* device, SmallJob* jobs, int n_jobs, const rlt_mlp3s_
         for (int j = 0; j < n_jobs; j++) K.xsum[j] = (float*)scratch + xsum_offset[j];
         device->fault_armed = 1;
     }
+    float* sums_before[2] = {nullptr, nullptr};
+    if (in_epoch)
+        for (int j = 0; j < 2; j++) {
+            // launches leave their sums in two places by turns: a workgroup may be through with its pass before another has read the sums of the launch before
+            float* const places[2] = {(float*)scratch + xsum_offset[j], (float*)scratch + second_sums[j]};
+            K.xsum[j] = places[epoch->index & 1]; sums_before[j] = places[(epoch->index + 1) & 1];
+            S.s[j].copies = (float*)scratch + copies_offset[j];
+            S.s[j].sums = sums_before[j]; S.s[j].from_tensors = epoch->index == 1; S.s[j].steps_before = epoch->index - 1;
+            if (j == 1 && epoch->loss_before) { S.s[1].extra_out = epoch->loss_before; S.s[1].extra_offset = (uint32_t)(jobs[1].a.count - N_EXTRA); S.s[1].extra_scale = 1.0f / (float)jobs[1].a.batch; }
+            jobs[j].a.step_log_std = j == 0 && jobs[0].extra != nullptr;
+        }
+    const bool step_first = in_epoch && epoch->index > 0;
     K.a0 = jobs[0].a; K.a1 = jobs[n_jobs - 1].a; K.groups0 = groups[0];
     const int grid = groups[0] + (n_jobs == 2 ? groups[1] : 0);
     const bool two_layers = jobs[0].n_layers == 2;
-#define RLT_LAUNCH_SMALL_AS(ACT, NT, LAYERS)                                                                                                                    \
-    do {                                                                                                                                                        \
-        RLT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(mlp3s_kernel<ACT, NT, LAYERS>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes)); \
-        hipLaunchKernelGGL((mlp3s_kernel<ACT, NT, LAYERS>), dim3(grid), dim3(THREADS), lds_bytes, device->stream, K);                                         \
+    NoSteps no_steps;
+#define RLT_LAUNCH_SMALL_AS(ACT, NT, LAYERS, STEPS)                                                                                                                    \
+    do {                                                                                                                                                               \
+        RLT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(mlp3s_kernel<ACT, NT, LAYERS, decltype(STEPS)>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes)); \
+        hipLaunchKernelGGL((mlp3s_kernel<ACT, NT, LAYERS, decltype(STEPS)>), dim3(grid), dim3(THREADS), lds_bytes, device->stream, K, STEPS);                         \
     } while (0)
 #define RLT_LAUNCH_SMALL(ACT, NT)                                                                                                                               \
     do {                                                                                                                                                        \
-        if (two_layers) RLT_LAUNCH_SMALL_AS(ACT, NT, 2); else RLT_LAUNCH_SMALL_AS(ACT, NT, 3);                                                                  \
+        if (two_layers) RLT_LAUNCH_SMALL_AS(ACT, NT, 2, no_steps); else if (step_first) RLT_LAUNCH_SMALL_AS(ACT, NT, 3, S); else RLT_LAUNCH_SMALL_AS(ACT, NT, 3, no_steps); \
     } while (0)
     switch (act) {
         case RLT_ACT_RELU: if (bucket == 2) RLT_LAUNCH_SMALL(RLT_ACT_RELU, 2); else if (bucket == 4) RLT_LAUNCH_SMALL(RLT_ACT_RELU, 4); else RLT_LAUNCH_SMALL(RLT_ACT_RELU, MAX_NT1); break;
@@ -628,6 +789,17 @@ int launch(rlt_rocm_device* device, SmallJob* jobs, int n_jobs, const rlt_mlp3s_
 #undef RLT_LAUNCH_SMALL
 #undef RLT_LAUNCH_SMALL_AS
     if ((rc = rlt_launch_status(device))) return rc;
+    if (in_epoch) {
+        *stepped = true;
+        if (epoch->index + 1 < epoch->n) return 0;      // the step is the next launch's
+        void* counters = nullptr;
+        if ((rc = rlt_counters(device, &counters))) return rc;
+        int blocks[2];
+        for (int j = 0; j < 2; j++) { S.s[j].sums = K.xsum[j]; S.s[j].from_tensors = 0; S.s[j].steps_before = epoch->index; blocks[j] = (jobs[j].a.count + 255) / 256; }
+        S.s[1].extra_out = jobs[1].extra; S.s[1].extra_offset = (uint32_t)(jobs[1].a.count - N_EXTRA); S.s[1].extra_scale = jobs[1].extra_scale;
+        hipLaunchKernelGGL(mlp3s_step_kernel, dim3(blocks[0] + blocks[1]), dim3(256), 0, device->stream, S, blocks[0], steps[0].age, steps[1].age, rlt_tickets_of(counters, 0));
+        return rlt_launch_status(device);
+    }
     const float* sums[2]; int n_sums[2];      // what is left to add up: the workgroups' blocks, or one block per XCD
     for (int j = 0; j < n_jobs; j++) { sums[j] = xcd_sums ? K.xsum[j] : jobs[j].a.partial; n_sums[j] = xcd_sums ? RLT_XCD_GROUPS : groups[j]; }
     if (steps_mapped) {
@@ -715,7 +887,7 @@ int rlt_mlp3s_ppo_actor_critic(rlt_rocm_device* device, const rlt_dense_layer* a
                                const rlt_dense_layer* critic, int n_critic, const float* x_critic, float* values, int ld_values,
                                const float* target_values, float mse_scale, float* out_critic_loss, int ld, const uint32_t* rows, int batch,
                                const float* actor_std_mean, const float* actor_std_precision, const float* critic_std_mean, const float* critic_std_precision,
-                               const rlt_mlp3s_step* steps, bool* stepped) {
+                               const rlt_mlp3s_step* steps, bool* stepped, const rlt_mlp3s_epoch* epoch) {
     if (!rlt_mlp3s_pair_supported(actor, n_actor, critic, n_critic) || (out_critic_loss && critic[2].out_dim != 1)) return RLT_E_UNSUPPORTED;
     SmallJob jobs[2] = {ppo_actor_job(actor, x, ld, means, ld_means, log_std, actions, ld, log_probs, ld, advantages, ld, stats, P, d_log_std,
                                       log_std_gradient_offset, batch, 1, rows),
@@ -723,7 +895,7 @@ int rlt_mlp3s_ppo_actor_critic(rlt_rocm_device* device, const rlt_dense_layer* a
     if (out_critic_loss) { jobs[1].extra = out_critic_loss; jobs[1].n_extra = 1; jobs[1].extra_scale = 1.0f / (float)batch; jobs[1].extra_offset = 0.0f; }
     jobs[0].a.std_mean = actor_std_mean; jobs[0].a.std_precision = actor_std_mean ? actor_std_precision : nullptr;
     jobs[1].a.std_mean = critic_std_mean; jobs[1].a.std_precision = critic_std_mean ? critic_std_precision : nullptr;
-    return launch(device, jobs, 2, steps, stepped);
+    return launch(device, jobs, 2, steps, stepped, epoch);
 }
 
 #ifdef RLT_SMALL_PROFILE

@@ -339,7 +339,7 @@ static int pair_mode(const rlt_ppo_agent* A) {
 // actor and critic of the supported narrow shape in one launch (stats = {advantage mean, std} of the minibatch on the device), then both Adam steps in one
 static int ppo_pair_update(rlt_rocm_device* device, const rlt_ppo_agent* A, const rlt_ppo_parameters* P, const float* observations, const float* observations_privileged,
                            const float* actions, const float* action_log_probs, const float* advantages, const float* target_values, int ld, const uint32_t* row_indices,
-                           const float* stats, float* values, float* out_critic_loss) {
+                           const float* stats, float* values, float* out_critic_loss, const rlt_mlp3s_epoch* epoch = nullptr) {
     const int B = A->batch, AD = A->action_dim;
     int rc;
     const rlt_dense_layer* actor = A->actor; const rlt_dense_layer* critic = A->critic;
@@ -360,7 +360,7 @@ static int ppo_pair_update(rlt_rocm_device* device, const rlt_ppo_agent* A, cons
                                     action_log_probs, advantages, stats, P, P->learn_action_std ? A->d_log_std : nullptr, -P->action_entropy_coefficient,
                                     critic, A->n_critic_layers, observations_privileged, values, 1, target_values, 1.0f / (float)B, out_critic_loss,   // :303
                                     ld, row_indices, B, A->actor_standardize_mean, A->actor_standardize_precision, A->critic_standardize_mean,
-                                    A->critic_standardize_precision, fuse_steps ? steps : nullptr, &stepped);
+                                    A->critic_standardize_precision, fuse_steps ? steps : nullptr, &stepped, epoch);
     if (rc || stepped) return rc;
     if (pad_a) if ((rc = rlt_unpad_gradients(device, A->actor, &padded_actor))) return rc;
     if (pad_c) if ((rc = rlt_unpad_gradients(device, A->critic, &padded_critic))) return rc;
@@ -453,9 +453,11 @@ extern "C" int rlt_rocm_ppo_train_epoch(rlt_rocm_device* device, const rlt_ppo_a
         }
         hipLaunchKernelGGL(ppo_epoch_stats_final_kernel, dim3(1), dim3(EPOCH_CHUNK), 0, device->stream, partial_all, groups, B, P->normalize_advantage, n, stats_all);
         if ((rc = rlt_launch_status(device))) return rc;
-        for (int mb = first; mb < first + n; mb++)
+        for (int mb = first; mb < first + n; mb++) {
+            const rlt_mlp3s_epoch epoch = {mb, n_minibatches, out_critic_losses && mb > 0 ? out_critic_losses + mb - 1 : nullptr};
             if ((rc = ppo_pair_update(device, A, P, observations, observations_privileged, actions, action_log_probs, advantages, target_values, ld,
-                                      row_indices + (size_t)mb * B, stats_all + 2 * (mb - first), values, out_critic_losses ? out_critic_losses + mb : nullptr))) return rc;
+                                      row_indices + (size_t)mb * B, stats_all + 2 * (mb - first), values, out_critic_losses ? out_critic_losses + mb : nullptr, &epoch))) return rc;
+        }
     }
     return 0;
 }

@@ -11,7 +11,8 @@
 // The wait is bounded (the device handle's wait limit): the members of a group must be resident together, which the host only asks for
 // where the grid has at most one workgroup per compute unit. A member that gives up sets *fault and skips its slice.
 // Announcements: member m stores epoch + 1 in flags[m]; `epoch` is the group's own word, which member 0 advances after its wait, when every
-// member has read it (each reads it before it announces). The words only ever grow, so nothing has to be cleared between launches.
+// member has read it (each reads it before it announces). A launch may wait twice: the members then announce epoch + 1 and epoch + 2, and the word is advanced at the last wait. The words
+// only ever grow, so nothing has to be cleared between launches.
 #pragma once
 #include "common.h"
 #include "optim.h"
@@ -33,11 +34,10 @@ struct rlt_xcd_reduce_args {
 __device__ __forceinline__ uint32_t rlt_xcd_epoch(const rlt_xcd_reduce_args& X, int group) {
     return __hip_atomic_load(X.words + group * RLT_XCD_GROUP_WORDS + RLT_XCD_MAX_MEMBERS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-template <int THREADS>
-__device__ __forceinline__ void rlt_xcd_group_reduce(const rlt_xcd_reduce_args& X, int group, int member, int n_members, uint32_t epoch0, const float* blocks, int count, float* out,
-                                                     __attribute__((address_space(3))) int* lds_word) {
+// The wait: announces the workgroup's stores (every thread's) as `target` and returns, after a workgroup barrier, whether all members have announced theirs. Its loads of what
+// they wrote are rlt_load_shared<1>.
+__device__ __forceinline__ bool rlt_xcd_wait(const rlt_xcd_reduce_args& X, int group, int member, int n_members, uint32_t target, bool last, __attribute__((address_space(3))) int* lds_word) {
     uint32_t* const flags = X.words + group * RLT_XCD_GROUP_WORDS;
-    const uint32_t target = epoch0 + 1u;
     __builtin_amdgcn_s_waitcnt(0);        // this wavefront's stores are in the L2
     __syncthreads();
     if (threadIdx.x < 64) {
@@ -56,11 +56,16 @@ __device__ __forceinline__ void rlt_xcd_group_reduce(const rlt_xcd_reduce_args& 
         }
         if (threadIdx.x == 0) {
             *lds_word = ok;
-            if (ok && member == 0) __hip_atomic_store(flags + RLT_XCD_MAX_MEMBERS, target, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (ok && last && member == 0) __hip_atomic_store(flags + RLT_XCD_MAX_MEMBERS, target, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
     __syncthreads();
-    if (!*lds_word) return;
+    return *lds_word != 0;
+}
+template <int THREADS>
+__device__ __forceinline__ void rlt_xcd_group_reduce(const rlt_xcd_reduce_args& X, int group, int member, int n_members, uint32_t epoch0, const float* blocks, int count, float* out,
+                                                     __attribute__((address_space(3))) int* lds_word) {
+    if (!rlt_xcd_wait(X, group, member, n_members, epoch0 + 1u, true, lds_word)) return;
     // this member's slice of the elements, summed over the members' blocks in member order
     const int chunk = (count + n_members - 1) / n_members, begin = member * chunk, end = min(count, begin + chunk);
     const size_t stride = (size_t)RLT_XCD_GROUPS * count;

@@ -211,6 +211,39 @@ def test_train_epoch_matches_checker_and_minibatch_calls(oracle, rocm, normalize
     assert rel_err(got[0], want[0]) <= 2e-4 and rel_err(got[1], want[1]) <= 1e-4 and rel_err(got[2], want[2]) <= 1e-3
 
 
+# minibatches from the smallest on whose optimiser step joins the next one's launch, with rows that are no whole rounds of 64 or share the XCDs unevenly, one and both halves of the input buckets
+@pytest.mark.parametrize("O, A, B, NMB", [(105, 8, 8192, 5), (105, 8, 4096, 2), (3, 1, 5000, 3), (33, 16, 7001, 4), (128, 1, 4033, 33), (17, 6, 4032, 3)])
+def test_train_epoch_of_large_minibatches_is_the_minibatch_calls(rocm, O, A, B, NMB):
+    capi = helpers.capi
+    H, rng = 64, np.random.default_rng(O + B)
+    params = np.concatenate([helpers.random_params(rng, [O, H, H, A]), np.log(np.full(A, 0.5, np.float32)), helpers.random_params(rng, [O, H, H, 1])])
+    rows, ld = 3 * B, O + A + 3
+    data = rng.standard_normal((rows, ld)).astype(np.float32)
+    data[:, O + A] = -0.9 * A + 0.1 * data[:, O + A]
+    index = rng.integers(0, rows, NMB * B).astype(np.uint32)
+    adam = capi.adam_parameters(3e-4, epsilon=1e-8)
+    adam.weight_decay, adam.enable_weight_decay, adam.bias_lr_factor, adam.enable_bias_lr_factor = 0.01, 1, 1.5, 1
+    pp = capi.ppo_parameters()
+    results = []
+    for epoch_call in (True, False):
+        agent = helpers.PpoOnBackend(rocm, O, A, H, H, B, params, "tanh", "tanh", adam)
+        dd, idx, losses = rocm.array(data), rocm.array(index), rocm.zeros((NMB,))
+        args = (dd.offset(0), dd.offset(0), dd.offset(O), dd.offset(O + A), dd.offset(O + A + 1), dd.offset(O + A + 2), ld)
+        for _ in range(2):      # the second epoch starts from the first one's moments and ages
+            if epoch_call:
+                rocm.call("ppo_train_epoch", C.byref(agent.c), C.byref(pp), *args, idx.ptr, NMB, losses.ptr)
+            else:
+                for k in range(NMB):
+                    rocm.call("ppo_train_minibatch", C.byref(agent.c), C.byref(pp), *args, idx.offset(k * B), losses.offset(k))
+        rocm.sync()
+        nets = [agent.actor, agent.critic]
+        results.append([agent.parameters(), losses.numpy(), agent.d_log_std.numpy(), agent.m_log_std.numpy(), agent.v_log_std.numpy()] +
+                       [t.numpy() for net in nets for t in (net.grads, net.m, net.v, net.age)])
+    assert int(results[0][-1][0]) == 1 + 2 * NMB and np.abs(results[0][0] - params).max() > 1e-5 and all(np.all(np.isfinite(r)) for r in results[0])
+    for got, want in zip(*results):
+        assert np.array_equal(got, want)        # the same sums in the same order
+
+
 def test_ppo_against_reference_vectors(rocm):
     """GAE bit-exact structure aside (fp32, same operation order per environment), the 30 minibatch updates of two loop steps reproduce the
     reference's parameters; the dataset, permutations and parameters come from the reference's own run (tests/golden/ppo_pendulum_seed0.npz)."""

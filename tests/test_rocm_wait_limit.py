@@ -64,7 +64,8 @@ def test_persistent_loop_gives_up_and_reports(oracle):
         oracle.lib.rlt_oracle_sac_loop_destroy(loop)
 
 
-def test_update_kernel_that_sums_per_xcd_gives_up_and_reports():
+@pytest.mark.parametrize("minibatches", [0, 3])      # 0: a minibatch call; an epoch of three waits at the head of its launches too
+def test_update_kernel_that_sums_per_xcd_gives_up_and_reports(minibatches):
     """PPO's minibatch kernel at 8,192 rows (rl/algorithms/ppo/operations_generic.h:163-309): its 256 workgroups add their blocks of partial gradient sums up
     per XCD inside the launch, which makes the 16 workgroups of a network on one XCD wait for each other."""
     O, A, H, B = 105, 8, 64, 8192
@@ -77,8 +78,11 @@ def test_update_kernel_that_sums_per_xcd_gives_up_and_reports():
     def one_update(backend):
         agent = helpers.PpoOnBackend(backend, O, A, H, H, B, params, "tanh", "tanh", capi.adam_parameters(3e-4, epsilon=1e-8))
         dd = backend.array(data)
-        rc = backend.device.lib.rlt_rocm_ppo_train_minibatch(backend.device.handle, C.byref(agent.c), C.byref(pp), dd.offset(0), dd.offset(0), dd.offset(O), dd.offset(O + A),
-                                                             dd.offset(O + A + 1), dd.offset(O + A + 2), ld, None, None)
+        index = backend.array(np.tile(np.arange(B, dtype=np.uint32), max(minibatches, 1)))
+        columns = (dd.offset(0), dd.offset(0), dd.offset(O), dd.offset(O + A), dd.offset(O + A + 1), dd.offset(O + A + 2), ld)
+        lib, h = backend.device.lib, backend.device.handle
+        if minibatches: rc = lib.rlt_rocm_ppo_train_epoch(h, C.byref(agent.c), C.byref(pp), *columns, index.ptr, minibatches, None)
+        else: rc = lib.rlt_rocm_ppo_train_minibatch(h, C.byref(agent.c), C.byref(pp), *columns, None, None)
         return rc, agent
 
     impatient = helpers.RocmBackend()
@@ -93,7 +97,7 @@ def test_update_kernel_that_sums_per_xcd_gives_up_and_reports():
     try:
         rc, agent = one_update(patient)
         assert rc == 0 and patient.device.lib.rlt_rocm_check_status(patient.device.handle) == 0
-        assert np.abs(agent.parameters() - params).max() > 1e-5 and int(agent.actor.age.numpy()[0]) == 2
+        assert np.abs(agent.parameters() - params).max() > 1e-5 and int(agent.actor.age.numpy()[0]) == 1 + max(minibatches, 1)
     finally:
         patient.close()
 
