@@ -60,6 +60,7 @@ constexpr size_t lds_floats(int nt1c) {
 // rows whose loss this lane forms after the forward pass (rows 4 kk + 2 half + u, column r); columns beyond the extent are clamped here and masked later.
 // `vrows`: the rows' indices, requested a round earlier so that nothing waits for them here.
 struct TileRegs { float xa[8], xb[8], in0[2], in1[2], in2[2]; };
+template <bool WIDE>      // more than 64 inputs
 __device__ __forceinline__ void request_tile(const SmallArgs& A, uint32_t vrows, int lane, int half, TileRegs& T) {
     const int r = lane & 15, kk = lane >> 4;
     const int c0 = min(lane, A.in - 1), c1 = min(64 + lane, A.in - 1), c = min(r, A.out - 1);
@@ -67,15 +68,15 @@ __device__ __forceinline__ void request_tile(const SmallArgs& A, uint32_t vrows,
     for (int row = 0; row < 8; row++) {
         const float* src = A.x + (size_t)(uint32_t)__builtin_amdgcn_readlane((int)vrows, 8 * half + row) * A.ldx;      // wavefront-uniform: scalar address arithmetic
         T.xa[row] = src[c0];
-        T.xb[row] = A.in > 64 ? src[c1] : 0.f;
+        if (WIDE) T.xb[row] = src[c1];
     }
+    const float* const p0 = A.loss == LOSS_GIVEN ? A.d_output : A.loss == LOSS_MSE ? A.target : A.actions;
+    const int l0 = A.loss == LOSS_GIVEN ? A.ldd : A.loss == LOSS_MSE ? A.ldt : A.ld_actions;
 #pragma unroll
     for (int v = 0; v < 2; v++) {
         const size_t row = (size_t)(uint32_t)__shfl((int)vrows, 4 * kk + 2 * half + v, 64);
-        T.in0[v] = T.in1[v] = T.in2[v] = 0.f;
-        if (A.loss == LOSS_GIVEN) T.in0[v] = A.d_output[row * A.ldd + c];
-        else if (A.loss == LOSS_MSE) T.in0[v] = A.target[row * A.ldt + c];
-        else { T.in0[v] = A.actions[row * A.ld_actions + c]; T.in1[v] = A.advantages[row * A.ld_adv]; T.in2[v] = A.log_probs[row * A.ld_lp]; }
+        T.in0[v] = p0[row * l0 + c];
+        if (A.loss == LOSS_PPO) { T.in1[v] = A.advantages[row * A.ld_adv]; T.in2[v] = A.log_probs[row * A.ld_lp]; }
     }
 }
 
@@ -101,7 +102,7 @@ struct SmallLaunch { SmallArgs a0, a1; int groups0; rlt_xcd_reduce_args xr; floa
 // The optimisers' step of one minibatch at the head of the launch of the next (rlt_mlp3s_epoch). Each XCD steps a copy of the network of its own: the workgroups of a network on one XCD take a
 // slice of its elements each (the eight XCDs' sums of the launch before, Adam), wait for each other through that XCD's L2 and load the weights from the copy. No workgroup waits for another XCD, and the
 // copies stay equal, since the same sums in the same order make them. The slice's loads travel with the row indices, Adam's arithmetic runs while the rows travel.
-// PPO at 8,192 rows, both networks 105 -> 64 -> 64: a launch of its own for the step takes 6.7 us per minibatch, at the head of the pass it adds @@.
+// PPO at 8,192 rows, both networks 105 -> 64 -> 64: a launch of its own for the step takes 6.7 us per minibatch, at the head of the pass it adds 4.2.
 struct SmallStepTensor { uint32_t begin, count, flags; float scale, add; float *parameters, *first, *second, *gradient; };      // elements [begin, begin + count) of a block of partial sums
 struct SmallStep {
     SmallStepTensor t[RLT_TAIL_TENSORS]; int n, count, stride;      // floats per block; floats per array of a copy
@@ -119,11 +120,14 @@ __device__ __forceinline__ void request_element(const SmallStep& S, const float*
     const uint32_t ec = min(e, end - 1u);
     const float *p = copy + ec, *m = p + S.stride, *v = m + S.stride;
     E.stepped = false; E.flags = 0; E.scale = 1.f; E.add = 0.f;
-    for (int i = 0; i < S.n; i++)
-        if (ec - S.t[i].begin < S.t[i].count) {
-            E.stepped = true; E.flags = S.t[i].flags; E.scale = S.t[i].scale; E.add = S.t[i].add;
-            if (S.from_tensors) { const uint32_t j = ec - S.t[i].begin; p = S.t[i].parameters + j; m = S.t[i].first + j; v = S.t[i].second + j; }
-        }
+    auto look = [&](const SmallStepTensor& T) {
+        const uint32_t j = ec - T.begin;
+        const bool in = j < T.count;
+        E.stepped = E.stepped || in; E.flags = in ? T.flags : E.flags; E.scale = in ? T.scale : E.scale; E.add = in ? T.add : E.add;
+        const bool from = in && S.from_tensors;
+        p = from ? T.parameters + j : p; m = from ? T.first + j : m; v = from ? T.second + j : v;
+    };
+    for (int i = 0; i < S.n; i++) look(S.t[i]);
     E.param = __builtin_nontemporal_load(p); E.m = __builtin_nontemporal_load(m); E.v = __builtin_nontemporal_load(v);      // (no line of a copy stays in this compute unit's cache)
 #pragma unroll
     for (int g = 0; g < RLT_XCD_GROUPS; g++) E.blocks[g] = S.sums[(size_t)g * S.count + ec];
@@ -180,26 +184,26 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K, STEPS ste
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);      // wavefront-uniform: addresses derived from it are computed on the scalar unit
     const int rt = wave & 3, half = wave >> 2;      // row tile; half of every layer's columns
     const int IN = A.in, OUT = A.out, NT1 = (IN + 15) >> 4;
+    constexpr bool WIDE = NT1C > 4;          // the bucket of more than 64 inputs (tile_bucket)
     constexpr int SX = 16 * NT1C + 1;        // row stride of the input tile and of W1 in LDS: a constant, so that LDS offsets fold into the instructions
     const lptr w1s = (lptr)lds_raw, w2s = w1s + H * SX, w3s = w2s + H * HS;
     const lptr xs_all = w3s + MAX_OUT * HS, h1s_all = xs_all + ROWS * SX, h2s_all = h1s_all + ROWS * HS, g2s_all = h2s_all + ROWS * HS, d3s_all = g2s_all + ROWS * HS;
     const lptr xs = xs_all + 16 * rt * SX, h1s = h1s_all + 16 * rt * HS, h2s = h2s_all + 16 * rt * HS, g2s = g2s_all + 16 * rt * HS, d3s = d3s_all + 16 * rt * D3S;
     const int n_tiles = (A.batch + 15) >> 4, n_rounds = (n_tiles + ROW_TILES - 1) / ROW_TILES;
     // lane l: the row of the input arrays that row (l & 15) of this wavefront's tile of round `round` reads; a tile beyond the batch is clamped here and masked later
-    auto rows_of = [&](int round) -> uint32_t {
-        const int b = min(min(round * ROW_TILES + rt, n_tiles - 1) * 16 + (lane & 15), A.batch - 1);
-        return A.rows ? A.rows[b] : (uint32_t)b;
-    };
+    const uint32_t* const row_words = A.rows ? A.rows : (const uint32_t*)A.W1;      // without indices any address that holds a word
+    auto batch_row = [&](int round) { return (uint32_t)min(min(round * ROW_TILES + rt, n_tiles - 1) * 16 + (lane & 15), A.batch - 1); };
+    auto rows_of = [&](int round) -> uint32_t { return row_words[A.rows ? batch_row(round) : 0u]; };
+    auto row_or = [&](uint32_t index, int round) { return A.rows ? index : batch_row(round); };
     // The launch's critical path starts with two dependent trips to memory (the row indices, then the rows): the index loads go out first, the
     // weights' and constants' loads follow while the indices travel, then the first tile's loads, and the weights are stored to LDS while those
-    // travel.
-    uint32_t rows_next = rows_of(block), rows_after = rows_next;
-    if (block + n_blocks < n_rounds) rows_after = rows_of(block + n_blocks);
+    // travel. None of these loads is under a condition and none of their values is chosen or copied before the tile's loads are out: where paths with and without a load meet, the compiler
+    // waits for it (the indices, the epoch word and the loss's constants were three trips to memory one after the other in front of the rows; PPO's epoch at 8,192 rows 30.3 -> 29.9 us per minibatch).
+    uint32_t rows_next = rows_of(block), rows_after = rows_of(block + n_blocks);
     TileRegs T;
     const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
     const int xgroup = (second ? RLT_XCD_GROUPS : 0) + (block & 7);      // with the XCD-level sums: this workgroup's group (network, XCD)
-    uint32_t xepoch = 0;
-    if (K.xr.enabled) xepoch = rlt_xcd_epoch(K.xr, xgroup);
+    uint32_t xepoch = rlt_xcd_epoch(K.xr, xgroup);
     const int member = block >> 3, n_members = (n_blocks - (block & 7) + 7) >> 3;
     if constexpr (STEP) {
         const SmallStep& S = steps.s[second ? 1 : 0];
@@ -212,7 +216,7 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K, STEPS ste
 #pragma unroll
         for (int u = 0; u < E; u++) request_element(S, copy, begin + u * THREADS + threadIdx.x, max(end, 1u), el[u]);
         __builtin_amdgcn_sched_barrier(0);
-        request_tile(A, rows_next, lane, half, T);
+        request_tile<WIDE>(A, row_or(rows_next, block), lane, half, T);
         float bc1, bc2;
         rlt_adam_bias_corrections(S.p, age, bc1, bc2);
         for (uint32_t base = begin; base < end; base += E * THREADS) {
@@ -243,7 +247,7 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K, STEPS ste
     for (int j = 0; j < H / WAVES; j++) {
         const float* src = W1 + (size_t)(wave * (H / WAVES) + j) * IN;
         v1[j][0] = load(src + min(lane, IN - 1));
-        v1[j][1] = IN > 64 ? load(src + min(64 + lane, IN - 1)) : 0.f;
+        v1[j][1] = WIDE ? load(src + min(64 + lane, IN - 1)) : 0.f;
     }
 #pragma unroll
     for (int u = 0; u < H * H / THREADS; u++) v2[u] = LAYERS == 3 ? load(W2 + u * THREADS + threadIdx.x) : 0.f;
@@ -253,20 +257,22 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K, STEPS ste
 #pragma unroll
     for (int nt = 0; nt < 2; nt++) { b1r[nt] = load(b1 + 16 * (2 * half + nt) + r); b2r[nt] = LAYERS == 3 ? load(b2 + 16 * (2 * half + nt) + r) : 0.f; }
     const float b3r = load(b3 + min(r, OUT - 1));
-    float ls = 0.f, adv_mean = 0.f, adv_std = 0.f;
-    if (A.loss == LOSS_PPO) {
-        ls = load(log_std + min(r, OUT - 1));
-        if (A.normalize_advantage) { adv_mean = A.stats[0]; adv_std = A.stats[1]; }
-    }
+    const bool ppo = A.loss == LOSS_PPO, normalized = ppo && A.normalize_advantage;
+    const float ls_read = load(ppo ? log_std + min(r, OUT - 1) : b1);
+    const float* const stats = normalized ? A.stats : A.b1;
+    const float adv_mean = stats[0], adv_std = stats[1];      // used where advantages are normalized
     // the standardize layer's constants for this lane's columns (nn/layers/standardize/operations_generic.h:68-86); without one: x - 0 times 1
-    float sm0 = 0.f, sp0 = 1.f, sm1 = 0.f, sp1 = 1.f;
-    if (A.std_mean) {
-        sm0 = A.std_mean[min(lane, IN - 1)]; sp0 = A.std_precision[min(lane, IN - 1)];
-        if (IN > 64) { sm1 = A.std_mean[min(64 + lane, IN - 1)]; sp1 = A.std_precision[min(64 + lane, IN - 1)]; }
-        sp0 = sp0 != 0.f ? sp0 : 1.f; sp1 = sp1 != 0.f ? sp1 : 1.f;
-    }
+    const bool standardized = A.std_mean != nullptr;
+    const float *const std_mean = standardized ? A.std_mean : A.b1, *const std_precision = standardized ? A.std_precision : A.b1;
+    const int s0 = standardized ? min(lane, IN - 1) : 0, s1_ = standardized ? min(64 + lane, IN - 1) : 0;
+    float sm0 = std_mean[s0], sp0 = std_precision[s0], sm1 = 0.f, sp1 = 1.f;
+    if (WIDE) { sm1 = std_mean[s1_]; sp1 = std_precision[s1_]; }
     __builtin_amdgcn_sched_barrier(0);      // the loads above are issued before the first wait for the row indices
-    if constexpr (!STEP) request_tile(A, rows_next, lane, half, T);
+    if constexpr (!STEP) request_tile<WIDE>(A, row_or(rows_next, block), lane, half, T);
+    __builtin_amdgcn_sched_barrier(0);
+    const float ls = ppo ? ls_read : 0.f;
+    sm0 = standardized ? sm0 : 0.f; sp0 = standardized && sp0 != 0.f ? sp0 : 1.f;
+    if (WIDE) { sm1 = standardized ? sm1 : 0.f; sp1 = standardized && sp1 != 0.f ? sp1 : 1.f; }
     RLT_TICK(1);
     if constexpr (STEP) rlt_lds_barrier();      // every wavefront has read the word of the wait
     // weights into LDS, rows padded to SX (zero beyond the input width, so the padded reduction steps add nothing)
@@ -275,7 +281,7 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K, STEPS ste
         for (int j = 0; j < H / WAVES; j++) {
             const lptr dst = w1s + (wave * (H / WAVES) + j) * SX;
             if (lane < SX) dst[lane] = lane < IN ? v1[j][0] : 0.f;
-            if (64 + lane < SX) dst[64 + lane] = 64 + lane < IN ? v1[j][1] : 0.f;
+            if (WIDE && 64 + lane < SX) dst[64 + lane] = 64 + lane < IN ? v1[j][1] : 0.f;
             if (lane == 0 && SX > 128) dst[128] = 0.f;
         }
 #pragma unroll
@@ -306,7 +312,7 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K, STEPS ste
             const int row = 8 * half + j;
             const bool rok = row0 + row < A.batch;
             if (lane < 16 * NT1C) xs[row * SX + lane] = (rok && lane < IN) ? (T.xa[j] - sm0) * sp0 : 0.f;
-            if (64 + lane < 16 * NT1C) xs[row * SX + 64 + lane] = (rok && 64 + lane < IN) ? (T.xb[j] - sm1) * sp1 : 0.f;
+            if (WIDE && 64 + lane < 16 * NT1C) xs[row * SX + 64 + lane] = (rok && 64 + lane < IN) ? (T.xb[j] - sm1) * sp1 : 0.f;
         }
     RLT_TICK(4);
         float in0[2], in1[2], in2[2];
@@ -317,7 +323,7 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K, STEPS ste
         if (round + n_blocks < n_rounds) {
             rows_next = rows_after;
             if (round + 2 * n_blocks < n_rounds) rows_after = rows_of(round + 2 * n_blocks);
-            request_tile(A, rows_next, lane, half, T);
+            request_tile<WIDE>(A, row_or(rows_next, round + n_blocks), lane, half, T);
         }
 
     RLT_TICK(5);
@@ -735,7 +741,7 @@ int launch(rlt_rocm_device* device, SmallJob* jobs, int n_jobs, const rlt_mlp3s_
         xcd_sums = xcd_sums && groups[j] >= 2 * RLT_XCD_GROUPS && groups[j] <= RLT_XCD_GROUPS * RLT_XCD_MAX_MEMBERS;
         xsum_offset[j] = total; total += ((size_t)RLT_XCD_GROUPS * jobs[j].a.count + 63) & ~(size_t)63;
     }
-    // An epoch's steps at the head of the next minibatch's launch: a step takes each workgroup @@RULE
+    // An epoch's steps at the head of the next minibatch's launch: every workgroup steps a slice of its XCD's copy
     SmallSteps S = {};
     const bool in_epoch = epoch && xcd_sums && steps_mapped && epoch->n > 1 && fill_steps(jobs, steps, offsets, scales, adds, S) && groups[0] >= EPOCH_MIN_GROUPS && groups[1] >= EPOCH_MIN_GROUPS;
     size_t copies_offset[2] = {0, 0}, second_sums[2] = {0, 0};
@@ -749,10 +755,11 @@ int launch(rlt_rocm_device* device, SmallJob* jobs, int n_jobs, const rlt_mlp3s_
     int rc = rlt_scratch(device, total * sizeof(float), &scratch);
     if (rc) return rc;
     for (int j = 0; j < n_jobs; j++) jobs[j].a.partial = (float*)scratch + offset[j];
+    void* counters = nullptr;
+    if ((rc = rlt_counters(device, &counters))) return rc;
+    K.xr.words = (uint32_t*)counters + RLT_XCD_WORDS_OFFSET;      // a launch that waits for nobody reads its epoch word all the same
     if (xcd_sums) {
-        void* counters = nullptr;
-        if ((rc = rlt_counters(device, &counters))) return rc;
-        K.xr.enabled = 1; K.xr.max_poll = device->wait_limit; K.xr.words = (uint32_t*)counters + RLT_XCD_WORDS_OFFSET; K.xr.fault = device->fault;
+        K.xr.enabled = 1; K.xr.max_poll = device->wait_limit; K.xr.fault = device->fault;
         for (int j = 0; j < n_jobs; j++) K.xsum[j] = (float*)scratch + xsum_offset[j];
         device->fault_armed = 1;
     }
@@ -792,8 +799,6 @@ int launch(rlt_rocm_device* device, SmallJob* jobs, int n_jobs, const rlt_mlp3s_
     if (in_epoch) {
         *stepped = true;
         if (epoch->index + 1 < epoch->n) return 0;      // the step is the next launch's
-        void* counters = nullptr;
-        if ((rc = rlt_counters(device, &counters))) return rc;
         int blocks[2];
         for (int j = 0; j < 2; j++) { S.s[j].sums = K.xsum[j]; S.s[j].from_tensors = 0; S.s[j].steps_before = epoch->index; blocks[j] = (jobs[j].a.count + 255) / 256; }
         S.s[1].extra_out = jobs[1].extra; S.s[1].extra_offset = (uint32_t)(jobs[1].a.count - N_EXTRA); S.s[1].extra_scale = jobs[1].extra_scale;
