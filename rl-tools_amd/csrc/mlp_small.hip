@@ -675,9 +675,9 @@ bool map_step(const SmallJob& job, const rlt_mlp3s_step& S, bool extra_is_gradie
     return covered == 63u && extra_covered == (extra_is_gradient && job.extra != nullptr);
 }
 
+constexpr int XCD_MIN_GROUPS = 64;      // workgroups of each network from which on their sums are formed per XCD (launch)
 // The steps of two mapped optimisers for launches that read the blocks' elements: false unless the stepped parameters are the ones that the networks read, every tensor is complete and the ages
 // are two words. Tensors that follow each other everywhere are one, as a network laid out as an arena is: an element looks for its tensor.
-constexpr int EPOCH_MIN_GROUPS = 64;
 bool fill_steps(const SmallJob* jobs, const rlt_mlp3s_step* steps, const uint32_t (*offsets)[12], const float (*scales)[12], const float (*adds)[12], SmallSteps& S) {
     if (!steps[0].parameters || !steps[1].parameters || !steps[0].age || !steps[1].age || steps[0].age == steps[1].age) return false;
     for (int j = 0; j < 2; j++) {
@@ -734,16 +734,19 @@ int launch(rlt_rocm_device* device, SmallJob* jobs, int n_jobs, const rlt_mlp3s_
                               map_step(jobs[0], steps[0], true, offsets[0], scales[0], adds[0]) && map_step(jobs[1], steps[1], false, offsets[1], scales[1], adds[1]);
     SmallLaunch K = {};
     // sums per XCD inside the launch: where workgroup i runs on XCD i % 8 (a network's workgroups that are equal modulo 8 then share one, wherever its first lies; at most 32) and the grid is
-    // resident as a whole
-    bool xcd_sums = device->update_tail && device->xcd_stride == 8 && groups[0] + groups[n_jobs - 1] * (n_jobs - 1) <= device->compute_units;
+    // resident as a whole. Only for pairs, whose optimisers' launch adds the blocks up, and from 64 blocks on: the wait costs what fewer blocks cost that launch (per minibatch of 105 and of 17 inputs without /
+    // with it: 16 blocks 26.9 / 37.5 and 22.0 / 28.6 us, 32 blocks 28.4 / 33.6 and 22.7 / 26.3, 64 blocks 31.4 / 32.4 and 24.9 / 25.9, 128 blocks 37.4 / 32.7 and 29.2 / 27.0). One network's blocks are
+    // added up by a launch of many more threads, which needs it at no number of them (GRU step with a head of 64 inputs, 16 blocks: 74.4 / 82.5, 64: 114.3 / 117.9, 256: 151.5 / 152.7).
+    bool xcd_sums = n_jobs == 2 && device->update_tail && device->xcd_stride == 8 && groups[0] + groups[n_jobs - 1] * (n_jobs - 1) <= device->compute_units;
     size_t xsum_offset[2] = {0, 0};
     for (int j = 0; j < n_jobs; j++) {
-        xcd_sums = xcd_sums && groups[j] >= 2 * RLT_XCD_GROUPS && groups[j] <= RLT_XCD_GROUPS * RLT_XCD_MAX_MEMBERS;
+        xcd_sums = xcd_sums && groups[j] >= XCD_MIN_GROUPS && groups[j] <= RLT_XCD_GROUPS * RLT_XCD_MAX_MEMBERS;
         xsum_offset[j] = total; total += ((size_t)RLT_XCD_GROUPS * jobs[j].a.count + 63) & ~(size_t)63;
     }
-    // An epoch's steps at the head of the next minibatch's launch: every workgroup steps a slice of its XCD's copy
+    // An epoch's steps at the head of the next minibatch's launch, wherever the sums are formed per XCD: each workgroup steps a slice of its XCD's copy, which has to be short (a launch for the step / at the
+    // head, 105 and 17 inputs: 128 blocks 32.7 / 30.2 and 27.0 / 24.2 us, 64 blocks 32.4 / 31.4 and 25.9 / 23.1; 32 blocks, with the sums per XCD, 33.6 / 35.2 and 26.3 / 25.7)
     SmallSteps S = {};
-    const bool in_epoch = epoch && xcd_sums && steps_mapped && epoch->n > 1 && fill_steps(jobs, steps, offsets, scales, adds, S) && groups[0] >= EPOCH_MIN_GROUPS && groups[1] >= EPOCH_MIN_GROUPS;
+    const bool in_epoch = epoch && xcd_sums && steps_mapped && epoch->n > 1 && fill_steps(jobs, steps, offsets, scales, adds, S);
     size_t copies_offset[2] = {0, 0}, second_sums[2] = {0, 0};
     if (in_epoch)
         for (int j = 0; j < 2; j++) {
