@@ -102,7 +102,7 @@ struct SmallLaunch { SmallArgs a0, a1; int groups0; rlt_xcd_reduce_args xr; floa
 // The optimisers' step of one minibatch at the head of the launch of the next (rlt_mlp3s_epoch). Each XCD steps a copy of the network of its own: the workgroups of a network on one XCD take a
 // slice of its elements each (the eight XCDs' sums of the launch before, Adam), wait for each other through that XCD's L2 and load the weights from the copy. No workgroup waits for another XCD, and the
 // copies stay equal, since the same sums in the same order make them. The slice's loads travel with the row indices, Adam's arithmetic runs while the rows travel.
-// PPO at 8,192 rows, both networks 105 -> 64 -> 64: a launch of its own for the step takes 6.7 us per minibatch, at the head of the pass it adds 4.2.
+// PPO at 8,192 rows, both networks 105 -> 64 -> 64: a launch of its own for the step takes 6.7 us per minibatch, at the head of the pass it adds 3.5.
 struct SmallStepTensor { uint32_t begin, count, flags; float scale, add; float *parameters, *first, *second, *gradient; };      // elements [begin, begin + count) of a block of partial sums
 struct SmallStep {
     SmallStepTensor t[RLT_TAIL_TENSORS]; int n, count, stride;      // floats per block; floats per array of a copy
