@@ -1224,7 +1224,14 @@ int rlt_mlp_wide_reserve(rlt_rocm_device* device) {
     return 0;
 }
 
-// ---- forward + backward of a three-layer network on sixteen-row tiles (see mlp_wide_kernel), or the backward pass alone from the outputs that a forward() left in
+// Whether rows of y lie in the memory of other rows of `in`: a tile's outputs may then be written before the tile of those rows has read them.
+static bool rows_cross(const float* y, int ldy, int cols, const float* in, int ld, int in_cols, int batch) {
+    if (!y || !in) return false;
+    const intptr_t W = sizeof(float), apart = (intptr_t)y - (intptr_t)in, row = ld * W;
+    if (apart >= (batch - 1) * row + in_cols * W || -apart >= ((intptr_t)(batch - 1) * ldy + cols) * W) return false;
+    return ldy != ld || apart + cols * W > row || apart + row < in_cols * W;
+}
+// ---- forward + backward of a three-layer network on tiles of a few rows (see mlp_wide_kernel), or the backward pass alone from the outputs that a forward() left in
 // the layers; RLT_E_UNSUPPORTED: the caller takes another path
 static int mlp_wide_launch(rlt_rocm_device* device, const rlt_dense_layer* L, int n_layers, const float* x, int ldx, float* y, int ldy,
                            const float* d_output, int ldd, const float* target, int ldt, float mse_scale, int batch, int pass) {
@@ -1251,7 +1258,16 @@ static int mlp_wide_launch(rlt_rocm_device* device, const rlt_dense_layer* L, in
     // (an output in the memory of the input would leave the contraction over the whole batch without its operand: the rows are kept once more)
     const bool in_place = y && (uintptr_t)y < (uintptr_t)(x + (size_t)(batch - 1) * ldx + IN) && (uintptr_t)x < (uintptr_t)(y + (size_t)(batch - 1) * ldy + OUT);
     const bool blocks = !forward_only && sum_blocks(hid, IN, batch, backward_only);
-    const int rows = blocks ? ROWS : tile_rows(device, batch, 1, 1, hid > MAX_H - 16);
+    int rows = blocks ? ROWS : tile_rows(device, batch, 1, 1, hid > MAX_H - 16);
+    // one tile reads all of its rows before it writes any: a batch of at most sixteen stays one where its outputs lie in the memory of other rows' inputs
+    auto crosses = [&](const float* out, int ld, int cols) {
+        return rows_cross(out, ld, cols, x, ldx, IN, batch) || rows_cross(out, ld, cols, target, ldt, OUT, batch) || rows_cross(out, ld, cols, d_output, ldd, OUT, batch);
+    };
+    if (rows < batch && batch <= ROWS && !backward_only) {
+        bool apart = !crosses(y, ldy, OUT);
+        for (int l = 0; l < 3; l++) apart = apart && !crosses(a.keep_pre[l], L[l].out_dim, L[l].out_dim) && !crosses(a.keep_out[l], L[l].out_dim, L[l].out_dim);
+        if (!apart) rows = ROWS;
+    }
     const int groups = rlt_div_up(batch, rows);
     const int exact = hid * IN + hid + hid * hid + hid + OUT * hid + OUT;
     if (blocks) {

@@ -110,6 +110,46 @@ def test_the_output_may_replace_the_input(rocm, B, H):
                 assert rel_err(res[1][1][at:at + n], res[0][1][at:at + n]) <= TOL, (I, off, rel_err(res[1][1][at:at + n], res[0][1][at:at + n]))
 
 
+@pytest.mark.parametrize("place", [(17, 0, 6), (6, 0, 20), (17, 17, 17), (17, 5, 17), (20, 3, 6)])
+@pytest.mark.parametrize("B, H", [(5, 256), (9, 200), (16, 256), (16, 250)])
+def test_the_output_may_replace_other_rows_of_the_input_where_one_workgroup_has_the_batch(oracle, rocm, B, H, place):
+    """Up to sixteen rows: y packed over the rows of x, farther apart than they are, a row behind them, across the end of a row; y over the rows of the target; hidden outputs and y of a pass that is
+    only forward. Outputs and gradients are those of the checker's call with memory of its own. (tanh: a relu unit whose pre-activation rounding
+    moves across 0, 5.8e-8 from it at (9, 200, second place), has another gradient.)"""
+    ldx, shift, ldy = place
+    dims, O, rng = [6 if ldx == 6 else 17, H, H, 6], 6, np.random.default_rng(B + H + ldy)
+    params = helpers.random_params(rng, dims)
+    memory = rng.standard_normal(B * 20 + 64).astype(np.float32)
+    rows = lambda m, at, ld, n: np.stack([m[at + b * ld:at + b * ld + n] for b in range(B)])      # noqa: E731
+    x, target = rows(memory, 0, ldx, dims[0]), rng.standard_normal((B, O)).astype(np.float32)
+    want = run(oracle, dims, params, x, target, "tanh", True, 1.0 / B)
+    over_target = memory.copy()
+    for b in range(B):
+        over_target[b * ldx:b * ldx + O] = target[b]
+    for over in ("x", "target"):
+        net = Mlp(rocm, dims, params, B, "tanh", "identity")
+        ws, wsn = net.workspace()
+        xd, td = (rocm.array(memory), rocm.array(target)) if over == "x" else (rocm.array(x), rocm.array(over_target))
+        y = xd if over == "x" else td
+        rocm.call("mlp_zero_gradient", net.layers, net.n)
+        rocm.call("mlp_forward_backward", net.layers, net.n, xd.ptr, ldx if over == "x" else dims[0], y.offset(shift), ldy, None, 0, td.ptr, O if over == "x" else ldx, 1.0 / B, B, ws, wsn)
+        rocm.sync()
+        assert rel_err(rows(y.numpy(), shift, ldy, O), want[0]) <= TOL
+        for off, nw, nb in want[2]:
+            for at, n in ((off, nw), (off + nw, nb)):
+                assert rel_err(net.grads.numpy()[at:at + n], want[1][at:at + n]) <= TOL, (over, at)
+    if H % 4:      # (the other widths' passes of few rows are the one-row kernel's)
+        net = Mlp(rocm, dims, params, B, "tanh", "identity")
+        ws, wsn = net.workspace()
+        xd = rocm.array(memory)
+        rocm.call("mlp_evaluate", net.layers, net.n, xd.ptr, ldx, xd.offset(shift), ldy, B, ws, wsn)
+        xh = rocm.array(np.concatenate([memory, np.zeros(B * H, np.float32)]))
+        net.layers[0].output = xh.ptr
+        rocm.call("mlp_forward", net.layers, net.n, xh.ptr, ldx, B)
+        rocm.sync()
+        assert rel_err(rows(xd.numpy(), shift, ldy, O), want[0]) <= TOL and rel_err(net.out[2].numpy(), want[0]) <= TOL
+
+
 def test_the_call_takes_the_sixteen_row_tiles_where_this_file_says_so(rocm, monkeypatch):
     """Which path ran: the sixteen-row tiles and the path the call takes without them (RLT_MLP_WIDE=0) agree to tolerance but not bit for bit."""
     dims = [17, 256, 256, 6]
