@@ -403,7 +403,7 @@ __global__ __launch_bounds__(256, 2) void gru_forward_mfma_kernel(GruArgs A) {
 // more wavefronts, one per SIMD, form the gates of the next four steps (4 steps x 4 rows = the sixteen rows of v_mfma_f32_16x16x4) while the recurrence walks through these: wavefront p keeps
 // rows 48 p ... 48 p + 47 of W_i in registers as the B operand, the steps' inputs are staged through LDS a group of four steps ahead and requested another group ahead, the gates reach the
 // recurrence through LDS and never memory. Lane (n, kq) of both operands takes four consecutive inputs of every sixteen, in one 16-byte read
-// (the order of the sums in rows_forward_kernel, gemm.hip: the same bits).
+// (the order of the sums in rows_forward_kernel, gemm.hip: the same bits as where that is the launch in front; the tiled contraction of other shapes sums in another order).
 // Bound: the recurrence's chain and, beside it, 30 instructions of 32 cycles per step at 146 inputs, in which the SIMD's vector unit stands still: a step of 64 x 1,024 sequences takes 1.0 us
 // with 146 inputs, 0.69 with 3. The recurrence goes first (s_setprio); a second barrier per step that kept the others' products out of the recurrence's made it slower (64.5 -> 66.6 us).
 // Launch of the input gates + recurrence / this, 64 steps, 1,024 rows: 146 inputs 77.5 / 65.5 us, 64 inputs 61.1 / 49.0, 3 inputs 57.8 / 44.0.
@@ -995,6 +995,7 @@ bool layer_ok(const rlt_gru_layer* L) {
 }
 int compute_units(const rlt_rocm_device* device) { return device->compute_units > 0 ? device->compute_units : 256; }
 bool one_group_per_unit(const rlt_rocm_device* device, const rlt_gru_layer* L, int B) { return L->hidden_dim == 64 && rlt_div_up(B, GM_ROWS) <= compute_units(device); }
+bool overlap(const float* a, size_t n, const float* b, size_t m) { return (uintptr_t)a < (uintptr_t)(b + m) && (uintptr_t)b < (uintptr_t)(a + n); }
 int even_sixteens(int columns) { return 2 * rlt_div_up(columns, 32); }
 // Where the input gates / the weight gradients are formed beside the recurrence. The fp32 matrix instructions and the vector unit of a SIMD take turns, so that what goes beside the
 // recurrence lengthens its steps by the time it takes (44 ns per step and sixteen inputs; 54 ns and 46 per sixteen inputs), on as many compute units as there are workgroups, and saves what
@@ -1002,8 +1003,11 @@ int even_sixteens(int columns) { return 2 * rlt_div_up(columns, 32); }
 //   forward  146 inputs  16 rows 43.0 / 60.9, 512 rows 62.9 / 63.8, 640 rows 66.6 / 64.0, 1,024 rows 77.5 / 65.5; 40 inputs 64 rows 41.4 / 44.3, 256 rows 49.2 / 46.0; 20 inputs 16 rows 40.3 / 38.7
 //   backward 146 inputs 256 rows 61.6 / 78.0, 512 rows 81.1 / 80.0, 1,024 rows 132.7 / 85.7; 64 inputs 256 rows 52.5 / 58.6, 512 rows 64.3 / 60.2; 3 inputs 64 rows 47.5 / 50.6, 1,024 rows 79.1 / 55.3;
 //            146 inputs 1,024 rows 24 steps 57.7 / 44.0
-bool inputs_beside(const rlt_rocm_device* device, const rlt_gru_layer* L, int S, int B) {
+bool inputs_beside(const rlt_rocm_device* device, const rlt_gru_layer* L, const float* input, int S, int B) {
     if (!one_group_per_unit(device, L, B) || L->input_dim > GP_INPUTS) return false;
+    // steps are read after earlier ones are written: not where the outputs replace the inputs (the launch in front has read all of them)
+    const size_t rows = (size_t)S * B, inputs = rows * L->input_dim;
+    if (overlap(input, inputs, L->output, rows * 64) || overlap(input, inputs, L->n_pre_pre_activation, rows * 64) || overlap(input, inputs, L->post_activation, rows * 3 * 64)) return false;
     return 44.0 * S * even_sixteens(L->input_dim) <= 7000.0 + (0.15 + 0.0033 * L->input_dim) * S * B;
 }
 bool weights_beside(const rlt_rocm_device* device, const rlt_gru_layer* L, int S, int B, size_t room) {      // room: bytes of the caller's workspace that nothing else is kept in
@@ -1061,7 +1065,7 @@ int rlt_rocm_gru_forward(rlt_rocm_device* device, const rlt_gru_layer* L, const 
     const int H = L->hidden_dim;
     if (lds_bytes(H, false) > (size_t)device->lds_bytes) return RLT_E_UNSUPPORTED;
     GruArgs a = {}; a.L = *L; a.input = input; a.reset = reset; a.S = S; a.B = B; a.rows_per_group = rows_per_group(H);
-    if (inputs_beside(device, L, S, B)) {
+    if (inputs_beside(device, L, input, S, B)) {
         const dim3 grid4(rlt_div_up(B, GM_ROWS)), block(GP_THREADS);
         by_sixteens(L->input_dim, [&](auto groups) {
             constexpr int G = decltype(groups)::value;

@@ -1,6 +1,8 @@
 """GRU forward and backward through time on the GPU, through the C ABI, against the CPU checker and against vectors written by the reference.
 
 fp32 tolerance: 1e-5 relative to the largest magnitude of the tensor compared (contraction orders differ from the checker's)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -175,3 +177,24 @@ def test_gru_weight_gradients_of_all_steps_in_one_launch(oracle, rocm, case):
         want, got = run_pair(oracle, rocm, S, B, I, H, 38, True, want_d_input=want_d_input)
         for k in KEYS:
             assert rel_err(got[k], want[k]) <= 2e-5, (k, rel_err(got[k], want[k]))
+
+
+@pytest.mark.parametrize("case", [(64, 4, 3), (33, 70, 17), (40, 1000, 146), (30, 9, 64)])
+def test_gru_states_may_replace_the_inputs(rocm, case):
+    """A forward pass whose output buffer begins where its inputs do (rows narrower, wider and as wide as the states): the results of the call with memory of its own, whose input
+    gates may be summed in another order."""
+    S, B, I = case
+    H, rng = 64, np.random.default_rng(S + I)
+    params, x, _, reset = helpers.gru_random_case(rng, S, B, I, H, True)
+    results = []
+    for apart in (True, False):
+        g = helpers.GruOnBackend(rocm, S, B, I, H, params)
+        memory = rocm.array(np.concatenate([x.ravel(), np.zeros(S * B * max(H - I, 0), np.float32)]))
+        flags = rocm.array(reset)
+        if not apart:
+            g.c.output = memory.ptr
+        rocm.call("gru_forward", C.byref(g.c), memory.ptr, flags.ptr, S, B, g.ws, g.wsn)
+        rocm.sync()
+        results.append([g.out.numpy().ravel() if apart else memory.numpy()[:S * B * H], g.post.numpy(), g.npp.numpy()])
+    for want, got in zip(*results):
+        assert want.any() and rel_err(got, want) <= TOL
