@@ -140,12 +140,14 @@ __device__ __forceinline__ float element_sum(const StepElement& E) {
     return (q[0] + q[1]) + (q[2] + q[3]);
 }
 static_assert(RLT_XCD_GROUPS == 8, "element_sum adds quarters of two blocks");
-// the last step of an epoch: from the copy of XCD 0 into the tensors, whose gradients receive the last minibatch's; blocks [0, blocks0) take the first network
-__global__ __launch_bounds__(256) void mlp3s_step_kernel(SmallSteps K, int blocks0, uint32_t* age0, uint32_t* age1, uint32_t* tickets) {
+// the last step of an epoch: from the copy of XCD 0 into the tensors, whose gradients receive the last minibatch's; blocks [0, blocks0) take the first network. Where a workgroup of the epoch gave up
+// waiting (*faults) the copies are stepped with sums of nothing, and tensors and ages stay as they were before the epoch.
+__global__ __launch_bounds__(256) void mlp3s_step_kernel(SmallSteps K, int blocks0, uint32_t* age0, uint32_t* age1, uint32_t* tickets, const unsigned* faults) {
     const bool second = (int)blockIdx.x >= blocks0;
     const SmallStep& S = K.s[second ? 1 : 0];
     const uint32_t e = (second ? blockIdx.x - blocks0 : blockIdx.x) * 256u + threadIdx.x;
     const uint32_t age = *S.age + S.steps_before;
+    const bool is_void = *faults != 0;
     StepElement E;
     request_element(S, S.copies, e, S.count, E);
     float bc1, bc2;
@@ -155,12 +157,12 @@ __global__ __launch_bounds__(256) void mlp3s_step_kernel(SmallSteps K, int block
     rlt_adam_values(S.p, E.flags, g, bc1, bc2, E.m, E.v, E.param);
     for (int i = 0; i < S.n; i++) {
         const uint32_t j = e - S.t[i].begin;
-        if (j < S.t[i].count) { S.t[i].gradient[j] = g; S.t[i].first[j] = E.m; S.t[i].second[j] = E.v; S.t[i].parameters[j] = E.param; }
+        if (j < S.t[i].count && !is_void) { S.t[i].gradient[j] = g; S.t[i].first[j] = E.m; S.t[i].second[j] = E.v; S.t[i].parameters[j] = E.param; }
     }
     if (S.extra_out && e == S.extra_offset) *S.extra_out = sum * S.extra_scale;
     asm volatile("" :: "v"(bc1), "v"(bc2));      // every thread has read the age before the workgroup's ticket is drawn
     rlt_lds_barrier();
-    if (threadIdx.x == 0 && rlt_last_through(tickets, blockIdx.x, gridDim.x)) { *age0 += K.s[0].steps_before + 1u; *age1 += K.s[1].steps_before + 1u; }
+    if (threadIdx.x == 0 && rlt_last_through(tickets, blockIdx.x, gridDim.x) && !is_void) { *age0 += K.s[0].steps_before + 1u; *age1 += K.s[1].steps_before + 1u; }
 }
 
 // a parameter of the pass; with a step in front another compute unit wrote it in this launch
@@ -236,7 +238,7 @@ __global__ __launch_bounds__(THREADS) void mlp3s_kernel(SmallLaunch K, STEPS ste
                 if (S.extra_out && (block & 7) == 0 && e == S.extra_offset) *S.extra_out = sum * S.extra_scale;
             }
         }
-        // a member that gives up has set the fault word: the epoch's results are void, and the tensors are as they were until its last launch
+        // a member that gives up has set the fault word: the epoch's results are void, and its last launch leaves the tensors as they were
         rlt_xcd_wait(K.xr, xgroup, member, n_members, xepoch + 1u, false, (__attribute__((address_space(3))) int*)(lptr)lds_raw);
         xepoch++;
         W1 = copy; b1 = W1 + H * IN; W2 = b1 + H; b2 = W2 + H * H; W3 = b2 + H; b3 = W3 + OUT * H;
@@ -805,7 +807,7 @@ int launch(rlt_rocm_device* device, SmallJob* jobs, int n_jobs, const rlt_mlp3s_
         int blocks[2];
         for (int j = 0; j < 2; j++) { S.s[j].sums = K.xsum[j]; S.s[j].from_tensors = 0; S.s[j].steps_before = epoch->index; blocks[j] = (jobs[j].a.count + 255) / 256; }
         S.s[1].extra_out = jobs[1].extra; S.s[1].extra_offset = (uint32_t)(jobs[1].a.count - N_EXTRA); S.s[1].extra_scale = jobs[1].extra_scale;
-        hipLaunchKernelGGL(mlp3s_step_kernel, dim3(blocks[0] + blocks[1]), dim3(256), 0, device->stream, S, blocks[0], steps[0].age, steps[1].age, rlt_tickets_of(counters, 0));
+        hipLaunchKernelGGL(mlp3s_step_kernel, dim3(blocks[0] + blocks[1]), dim3(256), 0, device->stream, S, blocks[0], steps[0].age, steps[1].age, rlt_tickets_of(counters, 0), (const unsigned*)device->fault);
         return rlt_launch_status(device);
     }
     const float* sums[2]; int n_sums[2];      // what is left to add up: the workgroups' blocks, or one block per XCD

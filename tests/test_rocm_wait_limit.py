@@ -102,6 +102,32 @@ def test_update_kernel_that_sums_per_xcd_gives_up_and_reports(minibatches):
         patient.close()
 
 
+def test_ppo_epoch_that_gives_up_leaves_the_agent_as_it_was():
+    """An epoch of three minibatches of 8,192 rows steps copies of the networks and brings them into the tensors with its last launch, which leaves parameters, log_std, moments and ages alone
+    where a workgroup of the epoch gave up."""
+    O, A, H, B, NMB = 17, 6, 64, 8192, 3
+    rng = np.random.default_rng(6)
+    params = np.concatenate([helpers.random_params(rng, [O, H, H, A]), np.log(np.full(A, 0.5, np.float32)), helpers.random_params(rng, [O, H, H, 1])])
+    ld = O + A + 3
+    data, pp = rng.standard_normal((B, ld)).astype(np.float32), capi.ppo_parameters()
+    for limit, status in ((1, capi.RLT_E_DEVICE_TIMEOUT), (0, 0)):
+        be = helpers.RocmBackend()
+        try:
+            agent = helpers.PpoOnBackend(be, O, A, H, H, B, params, "tanh", "tanh", capi.adam_parameters(3e-4, epsilon=1e-8))
+            dd, index = be.array(data), be.array(np.tile(np.arange(B, dtype=np.uint32), NMB))
+            state = lambda: [agent.parameters(), agent.m_log_std.numpy(), agent.v_log_std.numpy()] + [t.numpy() for net in (agent.actor, agent.critic) for t in (net.m, net.v, net.age)]      # noqa: E731
+            before = state()
+            be.call("set_wait_limit", limit)
+            lib, h = be.device.lib, be.device.handle
+            assert lib.rlt_rocm_ppo_train_epoch(h, C.byref(agent.c), C.byref(pp), dd.offset(0), dd.offset(0), dd.offset(O), dd.offset(O + A), dd.offset(O + A + 1), dd.offset(O + A + 2), ld,
+                                                index.ptr, NMB, None) == 0
+            after = state()      # read before the status, whose error sticks
+            assert lib.rlt_rocm_check_status(h) == status
+            assert [np.array_equal(a, b) for a, b in zip(before, after)] == [limit == 1] * len(before)
+        finally:
+            be.close()
+
+
 def wide_state(agent, nets):
     """parameters, moments and ages of the trained networks, and every parameter of the agent"""
     return [agent.parameters()] + [a.numpy() for n in nets for a in (n.m, n.v, n.age)]
