@@ -61,6 +61,9 @@ int rlt_side_join(rlt_rocm_device* device);
 
 // Grow-only scratch owned by the device handle.
 int rlt_scratch(rlt_rocm_device* device, size_t bytes, void** out);
+// Whether rlt_scratch may hand out so many bytes now: while the stream records a graph the buffer does not grow. For a path that wants more than another one for the same call, which is then taken;
+// never by trying rlt_scratch itself, whose errors are the call's.
+bool rlt_scratch_reaches(const rlt_rocm_device* device, size_t bytes);
 // RLT_COUNTERS_BYTES of zero-initialised device memory for last-workgroup-done tickets and per-workgroup partials.
 int rlt_counters(rlt_rocm_device* device, void** out);
 // Returns hipGetLastError() folded into the return convention; called after every launch.

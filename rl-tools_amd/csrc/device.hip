@@ -48,6 +48,9 @@ int rlt_scratch(rlt_rocm_device* device, size_t bytes, void** out) {
     *out = buffer;
     return 0;
 }
+bool rlt_scratch_reaches(const rlt_rocm_device* device, size_t bytes) {
+    return !device->capturing || bytes <= (device->side_return ? device->side_scratch_bytes[device->side_active] : device->scratch_bytes);
+}
 
 int rlt_counters(rlt_rocm_device* device, void** out) {
     *out = device->counters;

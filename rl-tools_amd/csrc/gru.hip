@@ -1025,7 +1025,8 @@ GradientShape gradient_shape(const rlt_rocm_device* device, const rlt_gru_layer*
 }
 // Where they are (widths 16, 32, 64): not where width 64 meets 65,536 rows and more of 66 to 160 inputs, an even number, which wgrad_wide_kernel (gemm.hip) reads once. us of the backward pass
 // with contractions and sums per gradient / this, width 64: 146 inputs 16 steps 4,000 rows 141 / 127, 64 steps 2,048 rows 230 / 249, 16 steps 8,192 rows 247 / 303; 33 inputs 64 steps 2,048 rows 200 / 179,
-// 170 inputs 64 steps 1,024 rows 167 / 143; width 32, 146 inputs 64 steps 4,096 rows 296 / 243; width 16, 146 inputs 32 steps 8,192 rows 262 / 147.
+// 170 inputs 64 steps 1,024 rows 167 / 143; width 32, 146 inputs 64 steps 4,096 rows 296 / 243; width 16, 146 inputs 32 steps 8,192 rows 262 / 147. A stream that records a graph while the handle's
+// scratch memory has room for a contraction's shares but not for these (rlt_scratch_reaches) takes the contractions too.
 bool gradients_in_one(const rlt_gru_layer* L, int S, int B) {
     const int H = L->hidden_dim, I = L->input_dim;
     return (H == 16 || H == 32 || H == 64) && I <= 1024 && !(H == 64 && (size_t)S * B >= 65536 && I > 64 && I <= 160 && I % 2 == 0);
@@ -1138,9 +1139,11 @@ int rlt_rocm_gru_backward(rlt_rocm_device* device, const rlt_gru_layer* L, const
     }
     int rc = rlt_launch_status(device);
     if (rc) return rc;
-    float* shares = nullptr;
     const GradientShape shape = gradient_shape(device, L, rows);
-    if (want_weight_gradients && gradients_in_one(L, S, B) && rlt_scratch(device, shape.blocks * gradient_block(H, I) * sizeof(float), (void**)&shares) == 0) {
+    const size_t shares_bytes = shape.blocks * gradient_block(H, I) * sizeof(float);
+    if (want_weight_gradients && gradients_in_one(L, S, B) && rlt_scratch_reaches(device, shares_bytes)) {
+        float* shares = nullptr;
+        if ((rc = rlt_scratch(device, shares_bytes, (void**)&shares))) return rc;
         const GradientArgs g = {buffer_input, buffer_hidden, input, h_previous, shares, rows, I, rlt_div_up(I, 32)};
         const dim3 grid(shape.columns, shape.shares), block(256);
         if (H == 64) hipLaunchKernelGGL(gru_gradients_kernel<4>, grid, block, 0, device->stream, g);

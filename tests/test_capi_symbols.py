@@ -49,3 +49,22 @@ def test_structure_sizes_match_the_header():
     for line in out.strip().splitlines():
         n, size = line.split()
         assert C.sizeof(names[n]) == int(size), (n, C.sizeof(names[n]), size)
+
+
+def scratch_requests(text):
+    """(requests for the handle's scratch memory in a source, those whose error the function returns)"""
+    requests = re.findall(r"[^\n]*\brlt_scratch\(device,[^\n]*\n[^\n]*", text)
+    returned = [r for r in requests if re.search(r"if \(\(rc = rlt_scratch\(.*\)\)\) return rc;", r) or re.search(r"int rc = rlt_scratch\(.*\);\s*if \(rc\) return rc;", r)]
+    return requests, returned
+
+
+def test_a_failed_request_for_scratch_memory_is_the_calls_error():
+    """An allocation that failed has marked the handle, and a stream that records has no memory to add: the code goes to the caller, no call goes on another way and reports success."""
+    folder, n = os.path.join(helpers.ROOT, "rl-tools_amd", "csrc"), 0
+    for name in sorted(os.listdir(folder)):
+        if name.endswith(".hip"):
+            requests, returned = scratch_requests(open(os.path.join(folder, name)).read())
+            n += len(requests)
+            assert requests == returned, (name, [r for r in requests if r not in returned])
+    assert n >= 12
+    assert scratch_requests("    if (wanted && rlt_scratch(device, bytes, &p) == 0) {\n        use(p);\n") == (["    if (wanted && rlt_scratch(device, bytes, &p) == 0) {\n        use(p);"], [])

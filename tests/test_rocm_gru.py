@@ -198,3 +198,40 @@ def test_gru_states_may_replace_the_inputs(rocm, case):
         results.append([g.out.numpy().ravel() if apart else memory.numpy()[:S * B * H], g.post.numpy(), g.npp.numpy()])
     for want, got in zip(*results):
         assert want.any() and rel_err(got, want) <= TOL
+
+
+def test_a_backward_pass_is_recorded_with_the_scratch_memory_of_a_shorter_one(rocm):
+    """A handle whose scratch memory a call of a few steps has sized: a longer backward pass is recorded all the same (its shares of the rows want 1.3 MB, contractions less), and every replay
+    leaves the gradients of the call on a handle that may allocate, to the file's tolerance."""
+    S, B, I, H, rng = 16, 16, 146, 64, np.random.default_rng(3)
+    params, x, dy, reset = helpers.gru_random_case(rng, S, B, I, H, True)
+    want = helpers.GruOnBackend(rocm, S, B, I, H, params)
+    want.forward(x, reset)
+    want.backward(dy)
+    rocm.sync()
+    want, be, graph = want.results(), helpers.RocmBackend(), C.c_void_p()
+    try:
+        few = helpers.GruOnBackend(be, 2, 2, I, H, params)
+        few.forward(x[:2, :2], reset[:2, :2])
+        few.backward(dy[:2, :2])
+        g = helpers.GruOnBackend(be, S, B, I, H, params)
+        g.forward(x, reset)
+        g.dy, g.dx = be.array(dy), be.zeros((S, B, I))
+        be.sync()
+        be.call("graph_begin_capture")
+        try:
+            rc = be.device.lib.rlt_rocm_gru_backward(be.device.handle, C.byref(g.c), g.x.ptr, g.dy.ptr, g.dx.ptr, g.reset.ptr, S, B, 1, g.ws, g.wsn)
+        finally:
+            be.call("graph_end_capture", C.byref(graph))
+        assert rc == 0
+        for _ in range(3):
+            g.dy.upload(dy)
+            be.call("fill_f32", g.grads.ptr, 1, g.grads.shape[0], g.grads.shape[0], 0.0)
+            be.call("graph_launch", graph)
+            be.sync()
+            got = g.results()
+            for k in KEYS:
+                assert rel_err(got[k], want[k]) <= TOL, k
+        be.call("graph_destroy", graph)
+    finally:
+        be.close()
