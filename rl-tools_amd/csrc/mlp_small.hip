@@ -748,14 +748,19 @@ int launch(rlt_rocm_device* device, SmallJob* jobs, int n_jobs, const rlt_mlp3s_
     // An epoch's steps at the head of the next minibatch's launch, wherever the sums are formed per XCD: each workgroup steps a slice of its XCD's copy, which has to be short (a launch for the step / at the
     // head, 105 and 17 inputs: 128 blocks 32.7 / 30.2 and 27.0 / 24.2 us, 64 blocks 32.4 / 31.4 and 25.9 / 23.1; 32 blocks, with the sums per XCD, 33.6 / 35.2 and 26.3 / 25.7)
     SmallSteps S = {};
-    const bool in_epoch = epoch && xcd_sums && steps_mapped && epoch->n > 1 && fill_steps(jobs, steps, offsets, scales, adds, S);
+    bool in_epoch = epoch && xcd_sums && steps_mapped && epoch->n > 1 && fill_steps(jobs, steps, offsets, scales, adds, S);
     size_t copies_offset[2] = {0, 0}, second_sums[2] = {0, 0};
-    if (in_epoch)
+    if (in_epoch) {
+        size_t with_copies = total;
         for (int j = 0; j < 2; j++) {
             S.s[j].stride = (jobs[j].a.count + 63) & ~63;
-            second_sums[j] = total; total += ((size_t)RLT_XCD_GROUPS * jobs[j].a.count + 63) & ~(size_t)63;
-            copies_offset[j] = total; total += (size_t)RLT_XCD_GROUPS * 3 * S.s[j].stride;
+            second_sums[j] = with_copies; with_copies += ((size_t)RLT_XCD_GROUPS * jobs[j].a.count + 63) & ~(size_t)63;
+            copies_offset[j] = with_copies; with_copies += (size_t)RLT_XCD_GROUPS * 3 * S.s[j].stride;
         }
+        // a stream that records with room for a minibatch call only: a launch for the step, the same bits (nothing grows while it records, so all of an epoch goes one way)
+        in_epoch = rlt_scratch_reaches(device, with_copies * sizeof(float));
+        if (in_epoch) total = with_copies;
+    }
     void* scratch = nullptr;
     int rc = rlt_scratch(device, total * sizeof(float), &scratch);
     if (rc) return rc;

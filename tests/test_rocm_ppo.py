@@ -244,6 +244,50 @@ def test_train_epoch_of_large_minibatches_is_the_minibatch_calls(rocm, O, A, B, 
         assert np.array_equal(got, want)        # the same sums in the same order
 
 
+def test_an_epoch_is_recorded_with_the_scratch_memory_of_a_minibatch_call():
+    """A program that sizes the handle's scratch memory with a minibatch call may record an epoch, whose optimisers' step then has launches of its own: the same bits on every replay as the
+    minibatch calls outside."""
+    capi = helpers.capi
+    O, A, H, B, NMB = 105, 8, 64, 4096, 3
+    rng = np.random.default_rng(11)
+    params = np.concatenate([helpers.random_params(rng, [O, H, H, A]), np.log(np.full(A, 0.5, np.float32)), helpers.random_params(rng, [O, H, H, 1])])
+    ld = O + A + 3
+    data = rng.standard_normal((B, ld)).astype(np.float32)
+    data[:, O + A] = -0.9 * A + 0.1 * data[:, O + A]
+    index = rng.integers(0, B, NMB * B).astype(np.uint32)
+    pp, graph = capi.ppo_parameters(), C.c_void_p()
+    be = helpers.RocmBackend()      # a handle whose scratch memory nobody has sized before
+    try:
+        recorded, eager = (helpers.PpoOnBackend(be, O, A, H, H, B, params, "tanh", "tanh", capi.adam_parameters(3e-4, epsilon=1e-8)) for _ in range(2))
+        dd, idx, losses = be.array(data), be.array(index), [be.zeros((NMB,)), be.zeros((NMB,))]
+        args = (dd.offset(0), dd.offset(0), dd.offset(O), dd.offset(O + A), dd.offset(O + A + 1), dd.offset(O + A + 2), ld)
+
+        def minibatches():
+            for k in range(NMB):
+                be.call("ppo_train_minibatch", C.byref(eager.c), C.byref(pp), *args, idx.offset(k * B), losses[1].offset(k))
+            be.sync()
+
+        def state(agent, losses):
+            return [agent.parameters(), losses.numpy(), agent.actor.v.numpy(), agent.critic.m.numpy(), agent.actor.grads.numpy(), agent.actor.age.numpy()]
+        minibatches()
+        be.call("graph_begin_capture")
+        try:
+            rc = be.device.lib.rlt_rocm_ppo_train_epoch(be.device.handle, C.byref(recorded.c), C.byref(pp), *args, idx.ptr, NMB, losses[0].ptr)
+        finally:
+            be.call("graph_end_capture", C.byref(graph))
+        assert rc == 0
+        for replay in range(3):
+            if replay:
+                minibatches()
+            be.call("graph_launch", graph)
+            be.sync()
+            for got, want in zip(state(recorded, losses[0]), state(eager, losses[1])):
+                assert np.array_equal(got, want), replay
+        be.call("graph_destroy", graph)
+    finally:
+        be.close()
+
+
 def test_ppo_against_reference_vectors(rocm):
     """GAE bit-exact structure aside (fp32, same operation order per environment), the 30 minibatch updates of two loop steps reproduce the
     reference's parameters; the dataset, permutations and parameters come from the reference's own run (tests/golden/ppo_pendulum_seed0.npz)."""
