@@ -737,7 +737,7 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
 constexpr size_t LDS_FLOATS = (size_t)ROWS * SXS + 4 * ROWS * S + 4 * ROWS * D3S + WAVES * YP + MISC;
 
 // ---- Forward and backward pass of one three-layer network over a few thousand rows at most, on the same machinery (nn_models/mlp/operations_generic.h:103-204: forward, the
-// loss gradient given or formed from a target as the MSE's, backward with weight gradients): a workgroup takes 16 rows through the three layers and back and leaves
+// loss gradient given or formed from a target as the MSE's, backward with weight gradients): a workgroup takes 16, 8 or 4 rows through the three layers and back and leaves
 // activations and pre-activation gradients in memory; the weight gradients over the whole batch are the next launch (batch_gradient.hip). Narrow networks, whose gradients are few
 // tiles there and few bytes here, go the other way (BLOCKS): a workgroup forms its sixteen rows' weight gradients out of LDS and leaves them as a block, and the next launch adds the
 // blocks up (which way is taken: sum_blocks()). Where a batch is too small to fill the chip with the 64-row tiles of the one-pass kernel for large batches (mlp_fused.hip: 4,096 rows are 64 tiles for 256
@@ -998,7 +998,8 @@ Trained place_trained(float* base, int hid, int batch) {
 }
 void set_rows(rlt_gradient_net& N, const Trained& T, const float* x, int ldx) { N.x = x; N.ldx = ldx; N.h1 = T.h1; N.h2 = T.h2; N.d1 = T.d1; N.d2 = T.d2; N.d3 = T.d3; N.ld3 = MAX_OUT; }
 
-// Rows of a workgroup's tile: four (where there is such a kernel) or eight while every tile and role then has a compute unit of its own, sixteen beyond. Fewer rows are fewer
+// Rows of a workgroup's tile: four or eight while every tile and role then has a compute unit of its own, sixteen beyond; four only where every network has more than 240 units (MLP passes with any
+// activation function, SAC and TD3 updates with relu; the other instances were not built). Fewer rows are fewer
 // cycles of the matrix pipeline per layer (sixteen 8,192 at width 256, eight 4,096, four 2,048) on more compute units; the same weights travel to each. In us, sixteen / eight / four
 // rows, 256 rows of the batch, width 256: forward + backward, Adam and the gradients' clearing 35.1 / 32.2 / 29.0, SAC's update set 85.7 / 74.0 / 66.4, TD3's 90.7 / 80.9 / 77.9
 // (its critics' six roles take eight rows). Four and eight rows leave the same bits, sixteen others: a critic trained by a call of its own takes sixteen where both in one call do
@@ -1027,7 +1028,8 @@ int launch_wide(rlt_rocm_device* device, WideArgs& a, const Optimiser* opts, int
         if (a.critic[k].act_h != act || a.target[k].act_h != act) act = -1;
         every = every && a.critic[k].hid > MAX_H - 16 && a.target[k].hid > MAX_H - 16;
     }
-    const int rows = tile_rows(device, a.batch, a.roles, MODE == MODE_CRITIC ? 4 : MODE == MODE_TD3_CRITIC ? 6 : a.roles, every && act == RLT_ACT_RELU);
+    const bool every_relu = every && act == RLT_ACT_RELU;      // the instances of EVERY, and with them those of four rows
+    const int rows = tile_rows(device, a.batch, a.roles, MODE == MODE_CRITIC ? 4 : MODE == MODE_TD3_CRITIC ? 6 : a.roles, every_relu);
     const int groups = rlt_div_up(a.batch, rows);
     const size_t copies_floats = 5 * (MAX_COPY_FLOATS + MAX_W1_COPY_FLOATS) + 3 * MAX_COPY_FLOATS;
     const size_t trained_each = trained_floats(net[0].hid, a.batch), exchange_words = (size_t)groups * EXCHANGE, extra_floats = (size_t)(groups + 63) & ~(size_t)63,
@@ -1070,16 +1072,19 @@ int launch_wide(rlt_rocm_device* device, WideArgs& a, const Optimiser* opts, int
         RLT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(sac_wide_kernel<MODE, ACT, NT, EVERY, R>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes)); \
         hipLaunchKernelGGL((sac_wide_kernel<MODE, ACT, NT, EVERY, R>), grid, dim3(THREADS), lds_bytes, device->stream, a);                                \
     } while (0)
-#define RLT_LAUNCH_WIDE(ACT, NT, EVERY) do { if (rows == 4) RLT_LAUNCH_WIDE_ROWS(ACT, NT, EVERY, (EVERY ? 4 : 8)); else if (rows == 8) RLT_LAUNCH_WIDE_ROWS(ACT, NT, EVERY, 8); else RLT_LAUNCH_WIDE_ROWS(ACT, NT, EVERY, ROWS); } while (0)
+#define RLT_LAUNCH_WIDE(ACT, NT) do { if (rows == 8) RLT_LAUNCH_WIDE_ROWS(ACT, NT, false, 8); else RLT_LAUNCH_WIDE_ROWS(ACT, NT, false, ROWS); } while (0)
+#define RLT_LAUNCH_WIDE_EVERY(ACT, NT) do { if (rows == 4) RLT_LAUNCH_WIDE_ROWS(ACT, NT, true, 4); else if (rows == 8) RLT_LAUNCH_WIDE_ROWS(ACT, NT, true, 8); else RLT_LAUNCH_WIDE_ROWS(ACT, NT, true, ROWS); } while (0)
 #define RLT_LAUNCH_WIDE_ACT(NT)                                                                                                                           \
     do {                                                                                                                                                  \
-        if (act == RLT_ACT_RELU) { if (every) RLT_LAUNCH_WIDE(RLT_ACT_RELU, NT, true); else RLT_LAUNCH_WIDE(RLT_ACT_RELU, NT, false); }                    \
-        else if (act == RLT_ACT_FAST_TANH) RLT_LAUNCH_WIDE(RLT_ACT_FAST_TANH, NT, false); else RLT_LAUNCH_WIDE(-1, NT, false);                            \
+        if (every_relu) RLT_LAUNCH_WIDE_EVERY(RLT_ACT_RELU, NT);                                                                                          \
+        else if (act == RLT_ACT_RELU) RLT_LAUNCH_WIDE(RLT_ACT_RELU, NT);                                                                                  \
+        else if (act == RLT_ACT_FAST_TANH) RLT_LAUNCH_WIDE(RLT_ACT_FAST_TANH, NT); else RLT_LAUNCH_WIDE(-1, NT);                                          \
     } while (0)
     // the first layer's chunks that the code is unrolled for: up to 64 inputs they leave registers for all of a pass's weights at once
     if (a.obs + a.act <= 32) RLT_LAUNCH_WIDE_ACT(2); else if (a.obs + a.act <= 64) RLT_LAUNCH_WIDE_ACT(4); else RLT_LAUNCH_WIDE_ACT(MAX_D / 16);
 #undef RLT_LAUNCH_WIDE_ACT
 #undef RLT_LAUNCH_WIDE
+#undef RLT_LAUNCH_WIDE_EVERY
 #undef RLT_LAUNCH_WIDE_ROWS
     if ((rc = rlt_launch_status(device))) return rc;
     const rlt_gradient_guard guard = {device->fault, {opts[0].age, n_opts > 1 ? opts[1].age : nullptr, opts[0].second ? opts[0].second_age : nullptr}, age_before};
@@ -1258,7 +1263,8 @@ static int mlp_wide_launch(rlt_rocm_device* device, const rlt_dense_layer* L, in
     // (an output in the memory of the input would leave the contraction over the whole batch without its operand: the rows are kept once more)
     const bool in_place = y && (uintptr_t)y < (uintptr_t)(x + (size_t)(batch - 1) * ldx + IN) && (uintptr_t)x < (uintptr_t)(y + (size_t)(batch - 1) * ldy + OUT);
     const bool blocks = !forward_only && sum_blocks(hid, IN, batch, backward_only);
-    int rows = blocks ? ROWS : tile_rows(device, batch, 1, 1, hid > MAX_H - 16);
+    const bool every = hid > MAX_H - 16;
+    int rows = blocks ? ROWS : tile_rows(device, batch, 1, 1, every);      // (the instances of MLP_EVERY are those of four rows, MLP_BLOCKS has sixteen only)
     // one tile reads all of its rows before it writes any: a batch of at most sixteen stays one where its outputs lie in the memory of other rows' inputs
     auto crosses = [&](const float* out, int ld, int cols) {
         return rows_cross(out, ld, cols, x, ldx, IN, batch) || rows_cross(out, ld, cols, target, ldt, OUT, batch) || rows_cross(out, ld, cols, d_output, ldd, OUT, batch);
@@ -1295,7 +1301,14 @@ static int mlp_wide_launch(rlt_rocm_device* device, const rlt_dense_layer* L, in
         RLT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(mlp_wide_kernel<ACT, NT, P, FORM, R>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes)); \
         hipLaunchKernelGGL((mlp_wide_kernel<ACT, NT, P, FORM, R>), dim3(groups), dim3(THREADS), lds_bytes, device->stream, a);                                 \
     } while (0)
-#define RLT_LAUNCH_MLP_WIDE(ACT, NT, P, FORM) do { if (rows == 4) RLT_LAUNCH_MLP_WIDE_ROWS(ACT, NT, P, FORM, (FORM == MLP_BLOCKS ? ROWS : FORM == MLP_EVERY ? 4 : 8)); else if (rows == 8) RLT_LAUNCH_MLP_WIDE_ROWS(ACT, NT, P, FORM, (FORM == MLP_BLOCKS ? ROWS : 8)); else RLT_LAUNCH_MLP_WIDE_ROWS(ACT, NT, P, FORM, ROWS); } while (0)
+#define RLT_LAUNCH_MLP_WIDE(ACT, NT, P, FORM)                                                                                                                   \
+    do {                                                                                                                                                       \
+        constexpr int FEWEST = FORM == MLP_BLOCKS ? ROWS : FORM == MLP_EVERY ? 4 : 8;                                                                          \
+        if (rows < FEWEST) return RLT_E_UNSUPPORTED;                                                                                                           \
+        if (rows == 4) RLT_LAUNCH_MLP_WIDE_ROWS(ACT, NT, P, FORM, FEWEST);                                                                                     \
+        else if (rows == 8) RLT_LAUNCH_MLP_WIDE_ROWS(ACT, NT, P, FORM, (FEWEST > 8 ? FEWEST : 8));                                                             \
+        else RLT_LAUNCH_MLP_WIDE_ROWS(ACT, NT, P, FORM, ROWS);                                                                                                 \
+    } while (0)
     const bool relu = a.net.act_h == RLT_ACT_RELU;
 #define RLT_LAUNCH_MLP_WIDE_PASS(P, FORM)                                                                                                                       \
     do {                                                                                                                                                       \
@@ -1303,7 +1316,6 @@ static int mlp_wide_launch(rlt_rocm_device* device, const rlt_dense_layer* L, in
         else if (IN <= 64) { if (relu) RLT_LAUNCH_MLP_WIDE(RLT_ACT_RELU, 4, P, FORM); else RLT_LAUNCH_MLP_WIDE(-1, 4, P, FORM); }                                \
         else { if (relu) RLT_LAUNCH_MLP_WIDE(RLT_ACT_RELU, MAX_D / 16, P, FORM); else RLT_LAUNCH_MLP_WIDE(-1, MAX_D / 16, P, FORM); }                            \
     } while (0)
-    const bool every = hid > MAX_H - 16;
     if (forward_only) { if (every) RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD, MLP_EVERY); else RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD, MLP_ANY); }
     else if (backward_only) { if (blocks) RLT_LAUNCH_MLP_WIDE_PASS(MLP_BACKWARD, MLP_BLOCKS); else if (every) RLT_LAUNCH_MLP_WIDE_PASS(MLP_BACKWARD, MLP_EVERY); else RLT_LAUNCH_MLP_WIDE_PASS(MLP_BACKWARD, MLP_ANY); }
     else { if (blocks) RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD_BACKWARD, MLP_BLOCKS); else if (every) RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD_BACKWARD, MLP_EVERY); else RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD_BACKWARD, MLP_ANY); }
