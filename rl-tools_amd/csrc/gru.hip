@@ -998,17 +998,24 @@ bool one_group_per_unit(const rlt_rocm_device* device, const rlt_gru_layer* L, i
 bool overlap(const float* a, size_t n, const float* b, size_t m) { return (uintptr_t)a < (uintptr_t)(b + m) && (uintptr_t)b < (uintptr_t)(a + n); }
 int even_sixteens(int columns) { return 2 * rlt_div_up(columns, 32); }
 // Where the input gates / the weight gradients are formed beside the recurrence. The fp32 matrix instructions and the vector unit of a SIMD take turns, so that what goes beside the
-// recurrence lengthens its steps by the time it takes (44 ns per step and sixteen inputs; 54 ns and 46 per sixteen inputs), on as many compute units as there are workgroups, and saves what
-// the launches cost that share the work out over all of them (in ns, fitted to both sides at 3 to 146 inputs, 16 to 64 steps, 16 to 1,024 rows). us, launches / beside, 64 steps:
-//   forward  146 inputs  16 rows 43.0 / 60.9, 512 rows 62.9 / 63.8, 640 rows 66.6 / 64.0, 1,024 rows 77.5 / 65.5; 40 inputs 64 rows 41.4 / 44.3, 256 rows 49.2 / 46.0; 20 inputs 16 rows 40.3 / 38.7
-//   backward 146 inputs 256 rows 61.6 / 78.0, 512 rows 81.1 / 80.0, 1,024 rows 132.7 / 85.7; 64 inputs 256 rows 52.5 / 58.6, 512 rows 64.3 / 60.2; 3 inputs 64 rows 47.5 / 50.6, 1,024 rows 79.1 / 55.3;
-//            146 inputs 1,024 rows 24 steps 57.7 / 44.0
+// recurrence lengthens its steps by the time it takes, on as many compute units as there are workgroups, and saves what the launches cost that share the work out over all of them.
+// Forward (ns, fitted to both sides at 1 to 200 steps, 1 to 1,024 rows, 3 to 160 inputs; groups of four steps are whole): the launch in front costs a constant, by the kernel that it is and the words
+// of its loads, and a share of every row; beside the recurrence a step takes 27 or 24 per sixteen inputs longer than the launch's own. us, launches / beside:
+//   146 inputs 16 steps   16 rows 19.0 / 20.2, 256 rows 22.3 / 21.1; 64 steps 512 rows 62.6 / 64.8, 1,024 rows 77.5 / 65.3; 1 step 64 rows 11.5 / 8.3
+//   128 inputs 13 steps   64 rows 15.8 / 17.8; 20 steps 16 rows 19.2 / 22.3; 24 steps 400 rows 31.1 / 27.0
+//    64 inputs 16 steps   16 rows 15.8 / 14.9; 32 steps 16 rows 23.5 / 24.8, 256 rows 27.9 / 26.2; 64 steps 256 rows 49.0 / 46.3; 20 inputs 64 steps 16 rows 40.4 / 39.1, 1,024 rows 60.8 / 42.0
+// Backward (54 ns a step and 46 per sixteen inputs), us, launches / beside, 64 steps:
+//   146 inputs 256 rows 61.6 / 78.0, 512 rows 81.1 / 80.0, 1,024 rows 132.7 / 85.7; 64 inputs 256 rows 52.5 / 58.6, 512 rows 64.3 / 60.2; 3 inputs 64 rows 47.5 / 50.6, 1,024 rows 79.1 / 55.3;
+//   146 inputs 1,024 rows 24 steps 57.7 / 44.0
 bool inputs_beside(const rlt_rocm_device* device, const rlt_gru_layer* L, const float* input, int S, int B) {
     if (!one_group_per_unit(device, L, B) || L->input_dim > GP_INPUTS) return false;
     // steps are read after earlier ones are written: not where the outputs replace the inputs (the launch in front has read all of them)
     const size_t rows = (size_t)S * B, inputs = rows * L->input_dim;
     if (overlap(input, inputs, L->output, rows * 64) || overlap(input, inputs, L->n_pre_pre_activation, rows * 64) || overlap(input, inputs, L->post_activation, rows * 3 * 64)) return false;
-    return 44.0 * S * even_sixteens(L->input_dim) <= 7000.0 + (0.15 + 0.0033 * L->input_dim) * S * B;
+    const int I = L->input_dim;
+    const bool by_rows = I > 32 && I % 2 == 0 && rows >= 2048;      // the launch in front is rows_forward_kernel (rlt_gemm_rows_forward)
+    const double launch = by_rows ? 3750.0 : I <= 32 ? 5800.0 : I % 4 == 0 ? 2400.0 : I % 2 == 0 ? 2600.0 : 3200.0;
+    return (by_rows ? 27.2 : 23.8) * 4 * rlt_div_up(S, 4) * even_sixteens(I) <= launch + ((by_rows ? 0.143 : 0.185) + 0.0017 * I) * rows;
 }
 bool weights_beside(const rlt_rocm_device* device, const rlt_gru_layer* L, int S, int B, size_t room) {      // room: bytes of the caller's workspace that nothing else is kept in
     if (!one_group_per_unit(device, L, B) || L->input_dim > GW_INPUTS || rlt_div_up(B, GM_ROWS) * gru_gradient_block(L->input_dim) * sizeof(float) > room) return false;
