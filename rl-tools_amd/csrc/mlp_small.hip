@@ -677,7 +677,7 @@ bool map_step(const SmallJob& job, const rlt_mlp3s_step& S, bool extra_is_gradie
     return covered == 63u && extra_covered == (extra_is_gradient && job.extra != nullptr);
 }
 
-constexpr int XCD_MIN_GROUPS = 64;      // workgroups of each network from which on their sums are formed per XCD (launch)
+constexpr int XCD_MIN_GROUPS_PAIR = 64, XCD_MIN_GROUPS = 144;      // workgroups of each network of a pair, of a network alone from which on their sums are formed per XCD (launch)
 // The steps of two mapped optimisers for launches that read the blocks' elements: false unless the stepped parameters are the ones that the networks read, every tensor is complete and the ages
 // are two words. Tensors that follow each other everywhere are one, as a network laid out as an arena is: an element looks for its tensor.
 bool fill_steps(const SmallJob* jobs, const rlt_mlp3s_step* steps, const uint32_t (*offsets)[12], const float (*scales)[12], const float (*adds)[12], SmallSteps& S) {
@@ -736,13 +736,16 @@ int launch(rlt_rocm_device* device, SmallJob* jobs, int n_jobs, const rlt_mlp3s_
                               map_step(jobs[0], steps[0], true, offsets[0], scales[0], adds[0]) && map_step(jobs[1], steps[1], false, offsets[1], scales[1], adds[1]);
     SmallLaunch K = {};
     // sums per XCD inside the launch: where workgroup i runs on XCD i % 8 (a network's workgroups that are equal modulo 8 then share one, wherever its first lies; at most 32) and the grid is
-    // resident as a whole. Only for pairs, whose optimisers' launch adds the blocks up, and from 64 blocks on: the wait costs what fewer blocks cost that launch (per minibatch of 105 and of 17 inputs without /
-    // with it: 16 blocks 26.9 / 37.5 and 22.0 / 28.6 us, 32 blocks 28.4 / 33.6 and 22.7 / 26.3, 64 blocks 31.4 / 32.4 and 24.9 / 25.9, 128 blocks 37.4 / 32.7 and 29.2 / 27.0). One network's blocks are
-    // added up by a launch of many more threads, which needs it at no number of them (GRU step with a head of 64 inputs, 16 blocks: 74.4 / 82.5, 64: 114.3 / 117.9, 256: 151.5 / 152.7).
-    bool xcd_sums = n_jobs == 2 && device->update_tail && device->xcd_stride == 8 && groups[0] + groups[n_jobs - 1] * (n_jobs - 1) <= device->compute_units;
+    // resident as a whole. A pair's blocks are added up by the optimisers' launch, which takes up to 64 of them in the time of the wait (per minibatch of 105 and of 17 inputs without / with it: 16 blocks
+    // 26.9 / 37.5 and 22.0 / 28.6 us, 32 blocks 28.4 / 33.6 and 22.7 / 26.3, 64 blocks 31.4 / 32.4 and 24.9 / 25.9, 128 blocks 37.4 / 32.7 and 29.2 / 27.0). One network's are added up by a launch of many
+    // more threads, which takes up to 144 in that time (forward + backward of 17-64-64-6, 105-64-64-8 and 64-64-4: 64 blocks 17.9 / 20.2, 23.1 / 26.0 and 14.6 / 17.5 us, 128 blocks 19.6 / 20.2,
+    // 25.7 / 25.5 and 16.7 / 17.0, 172 blocks 21.0 / 20.3, 27.3 / 26.0 and 18.1 / 17.3, 256 blocks 22.6 / 20.7, 30.1 / 26.7 and 20.6 / 17.8). A network that hands a gradient on to its inputs stands behind
+    // others: as the head of a sequence model's step it is faster without at every number (190 blocks 120.2 / 121.0 us of the step, 256 blocks 145.1 / 145.7 and 206.9 / 207.7), called by itself with it
+    // from 144 blocks on (64-64-4, 256 blocks 22.7 / 19.8).
+    bool xcd_sums = (n_jobs == 2 || !jobs[0].a.d_input) && device->update_tail && device->xcd_stride == 8 && groups[0] + groups[n_jobs - 1] * (n_jobs - 1) <= device->compute_units;
     size_t xsum_offset[2] = {0, 0};
     for (int j = 0; j < n_jobs; j++) {
-        xcd_sums = xcd_sums && groups[j] >= XCD_MIN_GROUPS && groups[j] <= RLT_XCD_GROUPS * RLT_XCD_MAX_MEMBERS;
+        xcd_sums = xcd_sums && groups[j] >= (n_jobs == 2 ? XCD_MIN_GROUPS_PAIR : XCD_MIN_GROUPS) && groups[j] <= RLT_XCD_GROUPS * RLT_XCD_MAX_MEMBERS;
         xsum_offset[j] = total; total += ((size_t)RLT_XCD_GROUPS * jobs[j].a.count + 63) & ~(size_t)63;
     }
     // An epoch's steps at the head of the next minibatch's launch, wherever the sums are formed per XCD: each workgroup steps a slice of its XCD's copy, which has to be short (a launch for the step / at the

@@ -63,6 +63,21 @@ def test_narrow_forward_backward_matches_checker(oracle, rocm, case):
         assert ew <= TOL and eb <= TOL, (off, ew, eb)
 
 
+# one network's workgroups around the line from which the blocks of partial sums are added up per XCD (144 workgroups of 64 rows), shared unevenly by the XCDs, the most, and with a second round
+@pytest.mark.parametrize("case", [(143 * 64, 17, 6), (144 * 64, 105, 8), (145 * 64 - 3, 3, 1), (250 * 64, 50, 4), (256 * 64, 128, 16), (257 * 64 + 1, 17, 6)])
+def test_one_network_of_many_workgroups_matches_checker(oracle, rocm, case):
+    print("case", case, flush=True)
+    B, I, O = case
+    dims, rng = [I, 64, 64, O], np.random.default_rng(B)
+    params = helpers.random_params(rng, dims)
+    x, dy = rng.standard_normal((B, I)).astype(np.float32), rng.standard_normal((B, O)).astype(np.float32)
+    want, got = (run(b, dims, params, x, dy, "tanh", "identity", False, 0.0, repeat=2) for b in (oracle, rocm))
+    assert rel_err(got[0], want[0]) <= TOL
+    for off, nw, nb in want[2]:
+        for at, n in ((off, nw), (off + nw, nb)):
+            assert rel_err(got[1][at:at + n], want[1][at:at + n]) <= TOL, (off, rel_err(got[1][at:at + n], want[1][at:at + n]))
+
+
 def test_narrow_accumulates_and_skips_null_output(rocm):
     dims = [105, 64, 64, 8]
     rng = np.random.default_rng(5)
