@@ -3,9 +3,9 @@
 #include "common.h"
 
 constexpr int RLT_MLP_ROW_MAX_BATCH = 2048;
-// Whether it is the faster way for a network that the sixteen-row tiles take too. Up to four rows per workgroup (1,024 rows) at every width and input; eight only for the
-// 256-wide networks of up to 32 inputs, whose weights leave registers for it: evaluate() / forward() of 2,048 rows here against the tiles, 17-256-256-6 14.8 / 16.1 us against
-// 15.5 / 16.4, but 17-128-128-6 11.4 / 12.4 against 11.5 / 12.0, 33-256-256-6 16.8 / 18.1 against 16.1 / 17.1, 64-192-192-6 15.8 / 17.4 against 14.1 / 14.9.
+// Whether it is the faster way for a network that the tiles of mlp_wide_kernel take too. Up to four rows per workgroup (1,024 rows) at every width and input (here / there, evaluate(): 17-256-256-6 7.7 / 11.3 us,
+// 60-128-128-8 8.2 / 9.2, 64-192-192-6 10.1 / 10.9); eight for the 256-wide networks of up to 32 inputs (2,048 rows 11.2 / 12.6), not for more inputs, whose weights leave no registers for it (33-256-256-6
+// 16.1 / 12.8, 60-128-128-8 11.1 / 9.2, 64-192-192-6 13.8 / 11.1). Narrower networks of up to 32 inputs stay on the tiles there, though they would be served here in 7.9 / 8.9 us (17-128-128-6) and 9.9 / 10.7 (17-192-192-6).
 inline bool rlt_mlp_row_first(const rlt_rocm_device* device, const rlt_dense_layer* layers, int batch) {
     const int units = device->compute_units > 0 ? device->compute_units : 256;
     return batch <= 4 * units || (layers[0].out_dim == 256 && layers[0].in_dim <= 32);

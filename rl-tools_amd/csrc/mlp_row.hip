@@ -8,7 +8,7 @@
 // positions 4 c + 64 j ... + 3 of the rows of units 16 w + 4 q + g, so a load instruction reads four runs of 256 bytes; all of a wavefront's weights of all
 // layers are requested before the first layer starts, the sixteen lanes' sums meet in row operations, and only the activations go through LDS.
 // One row of 17-256-256-6: 13.0 -> 5.2 us per call (10.6 us of sixteen-row tile and 3.1 of copies before; 4 us is what a call that launches anything costs);
-// 256 rows: 14.9 -> 5.7 us; 1,024: 14.8 -> 8.8 us. What is left is the launch and the one trip to memory.
+// 256 rows: 14.9 -> 5.7 us; 1,024: 14.8 -> 7.7 us. What is left is the launch and the one trip to memory.
 #include "mlp_row.h"
 #include "sac_heads.h"
 #include "sac_update.h"
@@ -60,14 +60,19 @@ __global__ __launch_bounds__(THREADS) void mlp_row_kernel(RowLaunch A) {
         const row_floatx4 v = *reinterpret_cast<const row_floatx4*>(N.W[2] + (size_t)min(wave, OUT - 1) * HID + min(4 * lane, HID - 4));
         w3 = FULL || 4 * lane < HID ? v : none;
     }
-    auto finish = [&](int l, float (&s)[4], float bias, float (&next)[MAX_H], int r) {
-        float kept = 0.f;
+    // A row's sums meet in all of their sixteen lanes: PACK rows of a unit lie in lanes c = 4 (row of the PACK) + q, which apply the activation function to all of them at once (a row at a time it
+    // is a chain for each, 16 of 64 lanes at work: 1,024 rows of 17-256-256-6 9.0 -> 7.7 us, 2,048 13.6 -> 11.2; with tanh 10.3 -> 7.9 and 15.9 -> 11.9)
+    constexpr int PACK = R < 4 ? R : 4;
+    auto keep = [&](float& kept, float (&s)[4], int u) {
 #pragma unroll
-        for (int q = 0; q < 4; q++) { const float sum = rlt_sac::row16_sum(s[q]); kept = (c & 3) == q ? sum : kept; }
-        if (c < 4) {
+        for (int q = 0; q < 4; q++) { const float sum = rlt_sac::row16_sum(s[q]); kept = (PACK == 1 ? c & 3 : c) == 4 * u + q ? sum : kept; }
+    };
+    auto finish = [&](int l, float kept, float bias, float (*next)[MAX_H], int first) {
+        const int r = PACK == 1 ? first : first + (c >> 2);
+        if (c < 4 * PACK) {
             const float pre = kept + bias, o = rlt_act(pre, N.act[l]);
             const bool ok = FULL || mine < HID;
-            next[mine] = ok ? o : 0.f;
+            next[r][mine] = ok ? o : 0.f;
             if (ok && row0 + r < A.batch) {
                 if (N.pre[l]) N.pre[l][(size_t)(row0 + r) * HID + mine] = pre;
                 if (N.out[l]) N.out[l][(size_t)(row0 + r) * HID + mine] = o;
@@ -77,15 +82,20 @@ __global__ __launch_bounds__(THREADS) void mlp_row_kernel(RowLaunch A) {
     rlt_lds_barrier();
     if (on) {
 #pragma unroll
-        for (int r = 0; r < R; r++) {
-            float s[4] = {0.f, 0.f, 0.f, 0.f};
+        for (int first = 0; first < R; first += PACK) {
+            float kept = 0.f;
 #pragma unroll
-            for (int j = 0; j < N1; j++) {
-                const float a = xs[r][c + 16 * j];
+            for (int u = 0; u < PACK; u++) {
+                float s[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int q = 0; q < 4; q++) s[q] += w1[q][j] * a;
+                for (int j = 0; j < N1; j++) {
+                    const float a = xs[first + u][c + 16 * j];
+#pragma unroll
+                    for (int q = 0; q < 4; q++) s[q] += w1[q][j] * a;
+                }
+                keep(kept, s, u);
             }
-            finish(0, s, b1, h1[r], r);
+            finish(0, kept, b1, h1, first);
         }
     } else if (c < 4) {
 #pragma unroll
@@ -94,32 +104,39 @@ __global__ __launch_bounds__(THREADS) void mlp_row_kernel(RowLaunch A) {
     rlt_lds_barrier();
     if (on) {
 #pragma unroll
-        for (int r = 0; r < R; r++) {
-            float s[4] = {0.f, 0.f, 0.f, 0.f};
+        for (int first = 0; first < R; first += PACK) {
+            float kept = 0.f;
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const row_floatx4 a = *reinterpret_cast<const row_floatx4*>(&h1[r][4 * c + 64 * j]);
+            for (int u = 0; u < PACK; u++) {
+                float s[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int q = 0; q < 4; q++)
+                for (int j = 0; j < 4; j++) {
+                    const row_floatx4 a = *reinterpret_cast<const row_floatx4*>(&h1[first + u][4 * c + 64 * j]);
 #pragma unroll
-                    for (int e = 0; e < 4; e++) s[q] += w2[q][j][e] * a[e];
+                    for (int q = 0; q < 4; q++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++) s[q] += w2[q][j][e] * a[e];
+                }
+                keep(kept, s, u);
             }
-            finish(1, s, b2, h2[r], r);
+            finish(1, kept, b2, h2, first);
         }
     }
     rlt_lds_barrier();
     if (wave < OUT) {
+        float kept = 0.f;      // row r's output in lane r
 #pragma unroll
         for (int r = 0; r < R; r++) {
             const row_floatx4 a = *reinterpret_cast<const row_floatx4*>(&h2[r][4 * lane]);
             const float s = rlt_sac::groups_sum(rlt_sac::row16_sum((w3[0] * a[0] + w3[1] * a[1]) + (w3[2] * a[2] + w3[3] * a[3])));
-            if (lane == 0 && row0 + r < A.batch) {
-                const size_t row = row0 + r;
-                const float pre = s + b3, o = rlt_act(pre, N.act[2]);
-                if (N.pre[2]) N.pre[2][row * OUT + wave] = pre;
-                if (N.out[2]) N.out[2][row * OUT + wave] = o;
-                if (A.y) A.y[row * A.ldy + wave] = o;
-            }
+            kept = lane == r ? s : kept;
+        }
+        if (lane < R && row0 + lane < A.batch) {
+            const size_t row = row0 + lane;
+            const float pre = kept + b3, o = rlt_act(pre, N.act[2]);
+            if (N.pre[2]) N.pre[2][row * OUT + wave] = pre;
+            if (N.out[2]) N.out[2][row * OUT + wave] = o;
+            if (A.y) A.y[row * A.ldy + wave] = o;
         }
     }
 }
@@ -149,8 +166,8 @@ int rlt_mlp_row_forward(rlt_rocm_device* device, const rlt_dense_layer* L, int n
     }
     a.net.in = L[0].in_dim; a.net.hid = hid; a.net.n_out = L[2].out_dim;
     a.x = x; a.ldx = ldx; a.y = y; a.ldy = ldy; a.batch = batch;
-    // Workgroups are one to a compute unit. Rows per workgroup 1, 2, 4, 8, calls in a row in a graph: 6.7, 7.9, 10.3, 14.8 us per call of 17-256-256-6, 5.6, 6.4, 8.1, 11.4 us at width 128 (15.1 to 15.5 and
-    // 11.2 to 11.5 on sixteen-row tiles with the weight copies before them; where the line lies: rlt_mlp_row_first).
+    // Workgroups are one to a compute unit. Rows per workgroup 1, 2, 4, 8 (256 ... 2,048 rows), calls in a row: 5.8, 6.2, 7.7, 11.2 us per call of 17-256-256-6, 5.2, 5.1, 6.0, 7.9 us at width 128 (11.3 to
+    // 12.6 and 8.7 to 8.9 on the tiles of mlp_wide_kernel with the weight copies before them; where the line lies: rlt_mlp_row_first).
     const int units = device->compute_units > 0 ? device->compute_units : 256;
     if (batch <= units) launch<1>(device, a); else if (batch <= 2 * units) launch<2>(device, a); else if (batch <= 4 * units) launch<4>(device, a); else launch<8>(device, a);
     return rlt_launch_status(device);

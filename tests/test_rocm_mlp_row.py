@@ -21,6 +21,8 @@ CASES = [
     (512, 128, 200, 5, "sigmoid", "sigmoid"),  # the most inputs; a width that ends inside a wavefront's units
     (513, 16, 252, 3, "relu", "tanh"),         # four rows per workgroup
     (1025, 17, 256, 6, "tanh", "identity"),    # eight
+    (1023, 17, 128, 6, "tanh", "tanh"),        # three rows in the last workgroup of four; wavefronts without units
+    (1607, 5, 256, 16, "tanh", "sigmoid"),     # seven in the last of eight
     (2048, 3, 96, 2, "identity", "identity"),  # the largest
     (1024, 40, 200, 2, "relu", "identity"),    # the last batch of four rows for every network: from here on sixteen-row tiles ...
     (1025, 33, 256, 6, "relu", "tanh"),
