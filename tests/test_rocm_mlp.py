@@ -283,3 +283,28 @@ def test_adam_step_at_the_edges_of_its_launch(oracle, rocm, counts, shift, norm)
     # an element's step is a dozen roundings of 6e-8; the norm's summands are positive, so that their sum is off by no more than their roundings
     for r, ref in zip(res[1], res[0]):
         assert rel_err(r, ref) <= 1e-6 if ref.size > 1 else rel_err(r, ref) <= 1e-5
+
+
+def test_tanh_against_64_bits(rocm):
+    """tanh of the layers (csrc/common.h, rlt_tanh) through a layer of one input with weight 1, on floats all over its ranges: tiny ones, both sides of 1 where the form changes, of 10 where the argument is
+    held, beyond. Bound: 1 - q with q = 2 / (e^2x + 1) at x >= 1, q at most 0.2384 and a share of 0.881 of e^2x's error; exp2 and the reciprocal within one unit in the last place (1.2e-7 each, of which the
+    Newton step leaves its own rounding), four roundings of 6.0e-8: (0.881 * (1.2 + 0.6) + 0.6 + 0.6) * 0.2384 / 0.7616 + 0.39 = 1.27 in units of 1e-7. Below 1 x + x^3 P: the result's rounding 0.6, and a share of
+    at most 0.31 for x^3 P's (four roundings and P's fit): 0.6 + 0.31 * 2.4 = 1.35."""
+    rng = np.random.default_rng(0)
+    edges = [np.float32(v) for v in (1.0, 0.625, 2.0, 10.0, 20.0, 1e-3)]
+    near = np.concatenate([np.arange(-2000, 2001, dtype=np.int32) + v.view(np.int32) for v in edges]).view(np.float32)
+    spread = np.exp(rng.uniform(np.log(1e-30), np.log(12.0), 400000)).astype(np.float32)
+    dense = rng.uniform(1e-3, 10.0, 400000).astype(np.float32)
+    x = np.concatenate([near, spread, dense, np.array([88.0, 3e38, np.inf], np.float32)])
+    x = np.concatenate([x, -x, np.array([0.0, np.nan], np.float32)])
+    net = Mlp(rocm, [1, 1], np.array([1.0, 0.0], np.float32), 1, out_act="tanh", trainable=False)
+    xd, yd = rocm.array(x.reshape(-1, 1)), rocm.zeros((x.size, 1))
+    rocm.call("mlp_evaluate", net.layers, 1, xd.ptr, 1, yd.ptr, 1, x.size, None, 0)
+    rocm.sync()
+    y = yd.numpy()[:, 0]
+    assert y[-2] == 0.0 and np.isnan(y[-1])
+    want = np.tanh(x[:-2].astype(np.float64))
+    error = np.abs(y[:-2] - want) / np.abs(want)
+    print("largest relative error", error.max(), "at", x[:-2][error.argmax()])
+    assert error.max() <= 1.35e-7
+    assert np.array_equal(y[:-2][np.abs(x[:-2]) > 10], np.sign(x[:-2][np.abs(x[:-2]) > 10]))

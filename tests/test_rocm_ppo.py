@@ -244,6 +244,47 @@ def test_train_epoch_of_large_minibatches_is_the_minibatch_calls(rocm, O, A, B, 
         assert np.array_equal(got, want)        # the same sums in the same order
 
 
+# what the optimisers' step in the next minibatch's launch tells apart besides: neighbouring tensors of one setting, which are one for it (no weight decay and no factor for biases, the default), a log_std
+# that no optimiser steps and that is read where it lies, standardize layers in front, no place for the losses
+@pytest.mark.parametrize("form", ["default Adam", "fixed log_std", "standardize layers", "no losses"])
+def test_train_epoch_of_large_minibatches_in_its_other_forms(rocm, form):
+    capi = helpers.capi
+    O, A, H, B, NMB = 70, 5, 64, 4100, 4
+    rng = np.random.default_rng(len(form))
+    params = np.concatenate([helpers.random_params(rng, [O, H, H, A]), np.log(rng.uniform(0.3, 0.8, A).astype(np.float32)), helpers.random_params(rng, [O, H, H, 1])])
+    rows, ld = 2 * B, O + A + 3
+    data = rng.standard_normal((rows, ld)).astype(np.float32)
+    data[:, O + A] = -0.9 * A + 0.1 * data[:, O + A]
+    index = rng.integers(0, rows, NMB * B).astype(np.uint32)
+    standardize = [rng.standard_normal(O), rng.uniform(0.3, 0.6, O), rng.standard_normal(O), rng.uniform(0.3, 0.6, O)] if form == "standardize layers" else None
+    if standardize:
+        standardize[1][3] = 0.0
+    pp = capi.ppo_parameters()
+    results = []
+    for epoch_call in (True, False):
+        agent = helpers.PpoOnBackend(rocm, O, A, H, H, B, params, "tanh", "tanh", capi.adam_parameters(3e-4, epsilon=1e-8), standardize=standardize)
+        if form == "fixed log_std":
+            pp.learn_action_std, agent.c.d_log_std = 0, None
+            agent.c.n_actor_adam_tensors -= 1
+        dd, idx, losses = rocm.array(data), rocm.array(index), rocm.zeros((NMB,))
+        args = (dd.offset(0), dd.offset(0), dd.offset(O), dd.offset(O + A), dd.offset(O + A + 1), dd.offset(O + A + 2), ld)
+        for _ in range(2):
+            if epoch_call:
+                rocm.call("ppo_train_epoch", C.byref(agent.c), C.byref(pp), *args, idx.ptr, NMB, None if form == "no losses" else losses.ptr)
+            else:
+                for k in range(NMB):
+                    rocm.call("ppo_train_minibatch", C.byref(agent.c), C.byref(pp), *args, idx.offset(k * B), None if form == "no losses" else losses.offset(k))
+        rocm.sync()
+        results.append([agent.parameters(), losses.numpy(), agent.d_log_std.numpy(), agent.m_log_std.numpy(), agent.v_log_std.numpy()] +
+                       [t.numpy() for net in (agent.actor, agent.critic) for t in (net.grads, net.m, net.v, net.age)])
+    n_actor = helpers.mlp_param_count([O, H, H, A])
+    moved = results[0][0] != params
+    assert moved[:n_actor].mean() > 0.9 and moved[n_actor + A:].mean() > 0.9 and moved[n_actor:n_actor + A].all() == (form != "fixed log_std") and results[0][1].any() == (form != "no losses")
+    assert int(results[0][-1][0]) == 1 + 2 * NMB and all(np.all(np.isfinite(r)) for r in results[0])
+    for got, want in zip(*results):
+        assert np.array_equal(got, want)        # the same sums in the same order
+
+
 def test_an_epoch_is_recorded_with_the_scratch_memory_of_a_minibatch_call():
     """A program that sizes the handle's scratch memory with a minibatch call may record an epoch, whose optimisers' step then has launches of its own: the same bits on every replay as the
     minibatch calls outside."""
