@@ -78,8 +78,9 @@ __device__ __forceinline__ float rlt_fast_tanh(float x) {
     return x * (27.0f + x2) / (27.0f + 9.0f * x2);
 }
 // tanh without a branch: x + x^3 P(x^2) below 1 (P fitted to the least relative error, 5e-9), 1 - 2 / (e^{2 |x|} + 1) above, on v_exp_f32 and v_rcp_f32 with the argument's rounding error
-// carried along and one Newton step. Against 64 bits over every float from 2^-11 to 12: relative error at most 8.3e-8, root mean square 2.4e-8 below 0.625, 3.0e-8 to 0.75, 2.7e-8 to 1, 2.1e-8 to 2
-// (tanhf: at most 1.5e-7; 2.4e-8, 4.5e-8, 3.4e-8, 2.1e-8). The library's branch at 0.625 keeps the compiler from interleaving the activations of a lane: each waits for its own chain.
+// carried along and one Newton step. Against 64 bits, on the card, every float from 2^-11 to 12: relative error at most 8.4e-8 (tanhf: 1.5e-7), root mean square (tanhf) 2.4e-8 below 0.625 (2.4e-8),
+// 3.0e-8 to 0.75 (4.5e-8), 2.7e-8 to 1 (3.4e-8), 2.1e-8 to 2 (2.1e-8; at most 8.4e-8 against 7.8e-8 there), 1.7e-8 beyond (1.7e-8). With both instructions off by one unit in the last place 1.3e-7
+// could be reached. The library's branch at 0.625 keeps the compiler from interleaving the activations of a lane: each waits for its own chain.
 __device__ __forceinline__ float rlt_tanh(float x) {
     const float a = fabsf(x), z = a * a;
     float p = fmaf(-0x1.77dd2ep-12f, z, 0x1.2da4f6p-9f);

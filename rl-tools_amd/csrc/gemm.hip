@@ -782,9 +782,8 @@ int rlt_gemm_wgrad(rlt_rocm_device* device, const float* d_pre, int ldd, const f
     p.vecA = vector_width(d_pre, ldd); p.vecB = vector_width(x, ldx);
     p.dW = dW; p.dbias = dbias;
     // Narrow layer, long batch: one workgroup per share of the batch holds the whole gradient (wgrad_wide_kernel), all 192 rows of it whatever out_dim is. Inputs of 34 to 64 are
-    // better off on the tiled kernel below where that is less than 129 rows or the batch shorter than 65,536 (backward pass of a GRU of 64 inputs, tiled -> this kernel: 48 rows
-    // of dW at 16,384 41.6 -> 44.3 us, at 65,536 75.0 -> 82.3; 96 rows 50.1 -> 52.3, 97.1 -> 101.3; 120 rows 86.9 -> 89.5, 220.6 -> 231.8; 144 rows 95.1 -> 97.1, 253.3 -> 249.8;
-    // 192 rows 57.9 -> 62.2 at 16,384, 96.7 -> 97.7 at 49,152, 122.6 -> 115.8 at 65,536).
+    // better off on the tiled kernel below where that is less than 129 rows or the batch shorter than 65,536 (backward pass of a GRU of 64 inputs, tiled -> this kernel: 120 rows of dW at 16,384
+    // 86.9 -> 89.5 us, at 65,536 220.6 -> 231.8; 144 rows 95.1 -> 97.1, 253.3 -> 249.8; 192 rows, which come here as dW_h at 65,536 and more, 122.6 -> 115.8 at 65,536).
     if (narrow_long && !static_scratch && out_dim <= WIDE_M && out_dim % 4 == 0 && (in_dim > 64 || (in_dim > 32 && out_dim > 128 && batch >= 65536)) && in_dim <= 160 && in_dim % 2 == 0 && batch >= 16384 && ldd % 4 == 0 && ldx % 2 == 0 &&
         (reinterpret_cast<uintptr_t>(d_pre) & 15u) == 0 && (reinterpret_cast<uintptr_t>(x) & 7u) == 0) {
         const int groups = device->compute_units < batch / 64 ? device->compute_units : batch / 64;

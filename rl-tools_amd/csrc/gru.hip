@@ -1032,7 +1032,8 @@ GradientShape gradient_shape(const rlt_rocm_device* device, const rlt_gru_layer*
 }
 // Where they are (widths 16, 32, 64): not where width 64 meets 65,536 rows and more of 66 to 160 inputs, an even number, which wgrad_wide_kernel (gemm.hip) reads once. us of the backward pass
 // with contractions and sums per gradient / this, width 64: 146 inputs 16 steps 4,000 rows 141 / 127, 64 steps 2,048 rows 230 / 249, 16 steps 8,192 rows 247 / 303; 33 inputs 64 steps 2,048 rows 200 / 179,
-// 170 inputs 64 steps 1,024 rows 167 / 143; width 32, 146 inputs 64 steps 4,096 rows 296 / 243; width 16, 146 inputs 32 steps 8,192 rows 262 / 147. A stream that records a graph while the handle's
+// 170 inputs 64 steps 1,024 rows 167 / 143, 300 inputs 64 rows 65.9 / 52.5, 1,024 rows 212 / 189, 1,000 inputs 64 rows 78.7 / 66.5, 1,024 rows 503 / 436; width 32, 500 inputs 64 rows 84.4 / 54.0, 1,000 inputs 1,024 rows
+// 256 / 250, 146 inputs 64 steps 4,096 rows 296 / 243; width 16, 146 inputs 32 steps 8,192 rows 262 / 147, 1,000 inputs 64 steps 1,024 rows 179 / 142. A stream that records a graph while the handle's
 // scratch memory has room for a contraction's shares but not for these (rlt_scratch_reaches) takes the contractions too.
 bool gradients_in_one(const rlt_gru_layer* L, int S, int B) {
     const int H = L->hidden_dim, I = L->input_dim;

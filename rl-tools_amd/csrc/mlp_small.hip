@@ -14,8 +14,9 @@
 // once per workgroup in LDS (padded rows, read as both W and W^T). Seven workgroup barriers per round (five with two layers) order the phases.
 // Bound: latency. One round is 460 matrix instructions per SIMD (14.7 K cycles at 105 -> 64 -> 64 -> 8), between LDS round trips and the activations' chains, and 141 KB of LDS leave room
 // for one workgroup per compute unit: two wavefronts per SIMD instead of one (four that had all columns of their rows) took PPO's pair at 8,192 rows from 30.0 to 25.6 us and the
-// head 64 -> 64 -> 4 of a sequence model at 65,536 rows from 56.2 to 47.2 us, with the same sums in the same order.
-// Both halves form the loss, for two of a lane's four rows each (stage 2.3 -> 1.6 us; PPO's pair, with the tanh of common.h that has no branch, 25.3 -> 25.0).
+// head 64 -> 64 -> 4 of a sequence model at 65,536 rows from 56.2 to 47.2 us, with the weight gradients' sums in the same order.
+// Both halves form the loss, for two of a lane's four rows each (stage 2.3 -> 1.6 us; PPO's pair, with the tanh of common.h that has no branch, 25.3 -> 25.0); its sums (db3, the log_std gradient, the loss) are
+// added up per half first.
 #include "mlp_small.h"
 #include "optim.h"
 #include "xcd_reduce.h"

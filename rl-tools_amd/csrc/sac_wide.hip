@@ -1002,7 +1002,9 @@ void set_rows(rlt_gradient_net& N, const Trained& T, const float* x, int ldx) { 
 // activation function, SAC and TD3 updates with relu; the other instances were not built). Fewer rows are fewer
 // cycles of the matrix pipeline per layer (sixteen 8,192 at width 256, eight 4,096, four 2,048) on more compute units; the same weights travel to each. In us, sixteen / eight / four
 // rows, 256 rows of the batch, width 256: forward + backward, Adam and the gradients' clearing 35.1 / 32.2 / 29.0, SAC's update set 85.7 / 74.0 / 66.4, TD3's 90.7 / 80.9 / 77.9
-// (its critics' six roles take eight rows). Four and eight rows leave the same bits, sixteen others: a critic trained by a call of its own takes sixteen where both in one call do
+// (its critics' six roles take eight rows). Sixteen rows everywhere / this rule: forward + backward of 17 inputs, width 256, 512 rows 29.0 / 23.2, 1,024 32.5 / 27.2, 2,048 (eight) 38.3 / 34.9; width 240
+// (eight) at 64, 256, 2,048 rows 25.0 / 21.9, 26.3 / 22.7, 39.1 / 36.0; 192 21.1 / 19.3 at 256, 27.9 / 26.2 at 2,048; 128 16.9 / 16.4 and 21.4 / 21.3. SAC's set, width 256, 512 rows 92.0 / 76.2, 1,024 (critics
+// sixteen, actor eight) 104.2 / 97.8; fast_tanh (eight) at 256 88.6 / 79.3; width 192 67.8 / 62.5, 128 54.9 / 52.3, 80 50.9 / 49.8 at 256. TD3's, 256 wide, 512 rows 94.3 / 85.3; 80 wide, 256 rows 51.8 / 51.0. Four and eight rows leave the same bits, sixteen others: a critic trained by a call of its own takes sixteen where both in one call do
 // (roles_of_both), as the two ways leave the same bits.
 int tile_rows(const rlt_rocm_device* device, int batch, int roles, int roles_of_both, bool four) {
     const int most = device->compute_units < 256 ? device->compute_units : 256;
