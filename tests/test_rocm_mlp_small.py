@@ -65,7 +65,7 @@ def test_narrow_forward_backward_matches_checker(oracle, rocm, case):
 
 # one network's workgroups around the line from which the blocks of partial sums are added up per XCD (144 workgroups of 64 rows), shared unevenly by the XCDs, the most, and with a second round
 @pytest.mark.parametrize("case", [(143 * 64, 17, 6), (144 * 64, 105, 8), (145 * 64 - 3, 3, 1), (250 * 64, 50, 4), (256 * 64, 128, 16), (257 * 64 + 1, 17, 6)])
-def test_one_network_of_many_workgroups_matches_checker(oracle, rocm, case):
+def test_one_network_of_many_workgroups_matches_the_oracle(oracle, rocm, case):
     print("case", case, flush=True)
     B, I, O = case
     dims, rng = [I, 64, 64, O], np.random.default_rng(B)

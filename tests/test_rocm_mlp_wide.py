@@ -114,7 +114,7 @@ def test_the_output_may_replace_the_input(rocm, B, H):
 @pytest.mark.parametrize("B, H", [(5, 256), (9, 200), (16, 256), (16, 250)])
 def test_the_output_may_replace_other_rows_of_the_input_where_one_workgroup_has_the_batch(oracle, rocm, B, H, place):
     """Up to sixteen rows: y packed over the rows of x, farther apart than they are, a row behind them, across the end of a row; y over the rows of the target; hidden outputs and y of a pass that is
-    only forward. Outputs and gradients are those of the checker's call with memory of its own. (tanh: a relu unit whose pre-activation rounding
+    only forward. Outputs and gradients are those of the oracle's call with memory of its own. (tanh: a relu unit whose pre-activation rounding
     moves across 0, 5.8e-8 from it at (9, 200, second place), has another gradient.)"""
     ldx, shift, ldy = place
     dims, O, rng = [6 if ldx == 6 else 17, H, H, 6], 6, np.random.default_rng(B + H + ldy)
