@@ -24,7 +24,7 @@
 // launch (batch_gradient.hip). Before, a workgroup ended with its sixteen rows' weight gradients (6.5 us on the matrix pipe at width 256) and a block of partial sums
 // that the optimisers' launch added up, and took all passes one after the other. At width 256, batch 256 (kernel and optimisers' launch; before / now): SAC critics
 // 55.7 + 10.6 / 26.0 + 8.2 us, SAC actor 65.6 + 10.6 / 33.9 + 8.2 us; TD3 critics (27 + 8 inputs) 61.1 + 11.9 / 28.1 + 8.0 us, TD3 actor 50.5 + 8.4 / 35.9 + 8.0 us.
-// With four rows per workgroup instead of sixteen: SAC critics / actor 26.5 / 33.8 -> 20.1 / 23.5 us, TD3 critics (eight) / actor 28.9 / 34.5 -> 24.9 / 25.2 us.
+// With four rows per workgroup instead of sixteen: SAC critics / actor 26.5 / 33.8 -> 20.1 / 23.5 us, TD3 critics (eight) / actor 28.9 / 34.5 -> 24.9 / 25.2 us (23.9 / 23.0 with the noise drawn by several wavefronts).
 // Bound: a workgroup's layer of R x 256 x 256 is R * 512 cycles of one compute unit's matrix pipeline (0.9 us with four rows, 3.4 with sixteen) and 256 KB of weights from L2 (1.7 us at
 // 64 B per cycle, while something else runs), and the longest chain has three of them (critic update) or four (actor update); the trips to memory at the start (3 us) and for the
 // values handed over (2 us) and the narrow layers between them come on top.
@@ -558,33 +558,33 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
     Operands<NT1C> W;
     load_operands<NT1C, EVERY>(A.actor, wave, c, g, W);      // on their way while the input rows are written
     place_row(xa + wave * SXS, row0 + wave < row_end, OBS, SXS, lane, in_row);
-    float noise[2] = {0.f, 0.f}, target_noise[2] = {0.f, 0.f}, alpha = 0.f, actor_b3 = 0.f, q_b3 = 0.f;
+    float alpha = 0.f, actor_b3 = 0.f, q_b3 = 0.f;
     if (scalar_wave) {
         actor_b3 = c < A.actor.out ? A.actor.b3[c] : 0.f; q_b3 = Q.b3[0];
         if (!TD3) alpha = expf(*A.log_alpha);
-        if (MODE == MODE_TD3_CRITIC) {
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                if (g + 4 * j < ACT && row_ok) {
-                    const size_t i = (size_t)(row0 + c) * ACT + g + 4 * j;
-                    if (A.target_noise) target_noise[j] = A.target_noise[i];
-                    else {
-                        const float scaled = rlt_randn_element(A.noise_seed, A.target_noise_stream + *A.stream_offset, i) * A.target_noise_std + 0.0f;
-                        target_noise[j] = clampf(scaled, -A.target_noise_clip, A.target_noise_clip);
-                        if (writes) A.out_target_noise[i] = target_noise[j];
-                    }
+    }
+    // The noise of the sample's values a = g and g + 4 by wavefronts 1 and 2, the smoothing noise by 3 and 4, into LDS for the first wavefront: a draw is a few hundred instructions, and one wavefront that
+    // made up to four of them kept all others waiting at the first barrier, 5.2 us after the start of TD3's critics with 8 actions, 3.9 of its actor (critics 26.2 -> 23.9 us, actor 25.8 -> 23.0, the set at
+    // 256 rows 78.2 -> 72.8; SAC with one action makes a single draw: 66.3 -> 66.0)
+    if (wave >= 1 && wave <= (MODE == MODE_TD3_CRITIC ? 4 : 2)) {
+        const int a = g + 4 * ((wave - 1) & 1);
+        float value = 0.f;
+        if (a < ACT && row_ok) {
+            const size_t i = (size_t)(row0 + c) * ACT + a;
+            if (MODE == MODE_TD3_CRITIC && wave > 2) {
+                if (A.target_noise) value = A.target_noise[i];
+                else {
+                    const float scaled = rlt_randn_element(A.noise_seed, A.target_noise_stream + *A.stream_offset, i) * A.target_noise_std + 0.0f;
+                    value = clampf(scaled, -A.target_noise_clip, A.target_noise_clip);
+                    if (writes) A.out_target_noise[i] = value;
                 }
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            if (g + 4 * j < ACT && row_ok) {
-                const size_t i = (size_t)(row0 + c) * ACT + g + 4 * j;
+            } else {
                 const float* const given = (MODE == MODE_TD3_CRITIC && set) ? A.noise_second : A.noise;
-                noise[j] = given ? given[i] : rlt_randn_element(A.noise_seed, ((MODE == MODE_TD3_CRITIC && set) ? A.noise_stream_second : A.noise_stream) + *A.stream_offset, i);
-                if (A.out_noise && writes) A.out_noise[i] = noise[j];
+                value = given ? given[i] : rlt_randn_element(A.noise_seed, ((MODE == MODE_TD3_CRITIC && set) ? A.noise_stream_second : A.noise_stream) + *A.stream_offset, i);
+                if (A.out_noise && writes) A.out_noise[i] = value;
             }
         }
+        d3c[64 * (wave - 1) + lane] = value;      // (d3c is next written by the first wavefront, after it has read these)
     }
     HeadItem item[2];
     RLT_TICK(13);
@@ -596,6 +596,7 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
         const floatx4 out = output_tile(yp, (A.actor.hid + 15) >> 4, c, g);
 #pragma unroll
         for (int v = 0; v < 4; v++) d3[(4 * g + v) * D3S + c] = c < A.actor.out ? out[v] + actor_b3 : 0.f;
+        const float noise[2] = {d3c[lane], d3c[64 + lane]}, target_noise[2] = {MODE == MODE_TD3_CRITIC ? d3c[128 + lane] : 0.f, MODE == MODE_TD3_CRITIC ? d3c[192 + lane] : 0.f};
         wave_sync();
         float log_prob = 0.f;
         if (TD3) td3_head_forward(OBS, ACT, A.sampling_std, d3, D3S, xa, SXS, noise, target_noise, CRITIC, c, g, item);
