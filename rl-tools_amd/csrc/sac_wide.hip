@@ -88,6 +88,89 @@ template <int ACT_H> __device__ __forceinline__ float dact_hidden(float o, int f
 // EVERY: where every wavefront has units and all sixteen chunks of the second layer are there, there is nothing to leave out, and the selects cost more than they save (forward +
 // backward of 256 units 36.2 us with them, 35.4 without; SAC's update set 86.2 and 86.0).
 template <int NT1C> constexpr int FIRST_STEP = NT1C <= FEW ? 1 : 4;      // (five chunks and more: the branches cost more)
+// How the weights come: FORM_ANY and FORM_EVERY (see EVERY above) from the copies; FORM_DIRECT, MLP passes of exactly 256 units whose second layer lies on 16 bytes, from the layers themselves, without
+// the launch that makes the copies (3.2 to 3.7 us). What a lane needs of the second layer on the way forward is four values that lie a row apart from its neighbours'; it is asked for as it lies, four
+// neighbouring lanes 64 bytes of one row (a 256 x 256 layer in 1.85 us, as from the copies; 6.96 where every lane has a row of its own), and dealt out in registers by selects that fetch from the
+// neighbouring lane, 128 per wavefront and layer beside 64 matrix instructions. On the way back only tiles of sixteen rows need such a dealing. Rows of the first layer are any number of floats; its few
+// chunks go through the wavefront's own part of the LDS. 17-256-256-6 with the gradients' clearing and Adam, copies / direct: forward + backward in one call 29.6 / 28.9 us at 256 rows, 36.1 / 35.2 at
+// 1,000, 43.9 / 43.5 at 2,048, 49.3 / 48.5 at 3,000, 54.0 / 53.9 at 4,096; as calls of their own 32.5 / 31.0, 41.1 / 38.5, 51.2 / 49.3, 57.7 / 54.9 and 62.1 / 58.9. The updates of SAC and TD3, whose
+// chains have two or three layers to deal out one after the other, keep the copies (sets at 256 rows 66.3 / 67.6 and 78.0 / 78.7).
+enum { FORM_ANY = 0, FORM_EVERY = 1, FORM_DIRECT = 2 };
+constexpr int W1S = 36, W1_STAGE = 16 * W1S;      // a wavefront's sixteen rows of two chunks, the rows four banks apart
+// a's values of the upper lanes of pairs against b's of the lower ones, as selects whose first operand comes through the lane control (left to the compiler, the exchange is an instruction of its own).
+// The data of such an operand must have been written two wait states before it is read, which the compiler does not see to inside an asm statement.
+#define RLT_EXCHANGE(FROM_LOWER, FROM_UPPER)                                                                                                                          \
+    floatx4 x, y;                                                                                                                                                     \
+    _Pragma("unroll") for (int i = 0; i < 4; i += 2) {                                                                                                                \
+        float x0, x1, y0, y1;                                                                                                                                         \
+        asm("s_nop 1\n\ts_mov_b64 vcc, %8\n\t"                                                                                                                       \
+            "v_cndmask_b32_dpp %0, %6, %4, vcc " FROM_LOWER " row_mask:0xf bank_mask:0xf bound_ctrl:0\n\tv_cndmask_b32_dpp %1, %7, %5, vcc " FROM_LOWER " row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t" \
+            "s_mov_b64 vcc, %9\n\t"                                                                                                                                  \
+            "v_cndmask_b32_dpp %2, %4, %6, vcc " FROM_UPPER " row_mask:0xf bank_mask:0xf bound_ctrl:0\n\tv_cndmask_b32_dpp %3, %5, %7, vcc " FROM_UPPER " row_mask:0xf bank_mask:0xf bound_ctrl:0"   \
+            : "=&v"(x0), "=&v"(x1), "=&v"(y0), "=&v"(y1) : "v"(a[i]), "v"(a[i + 1]), "v"(b[i]), "v"(b[i + 1]), "s"(~upper), "s"(upper) : "vcc");                       \
+        x[i] = x0; x[i + 1] = x1; y[i] = y0; y[i + 1] = y1;                                                                                                           \
+    }                                                                                                                                                                 \
+    a = x; b = y
+constexpr uint64_t LANES_1 = 0xAAAAAAAAAAAAAAAAull, LANES_2 = 0xCCCCCCCCCCCCCCCCull, LANES_4 = 0xF0F0F0F0F0F0F0F0ull, LANES_8 = 0xFF00FF00FF00FF00ull;      // lanes with that bit
+template <uint64_t upper> __device__ __forceinline__ void exchange(floatx4& a, floatx4& b) {
+    if constexpr (upper == LANES_1) { RLT_EXCHANGE("quad_perm:[1,0,3,2]", "quad_perm:[1,0,3,2]"); }
+    else if constexpr (upper == LANES_2) { RLT_EXCHANGE("quad_perm:[2,3,0,1]", "quad_perm:[2,3,0,1]"); }
+    else if constexpr (upper == LANES_4) { RLT_EXCHANGE("row_shr:4", "row_shl:4"); }      // (lanes without a partner on that side keep their own: bound_ctrl has them written all the same)
+    else { RLT_EXCHANGE("row_ror:8", "row_ror:8"); }
+}
+#undef RLT_EXCHANGE
+// 16 bytes of load t in lane u of a group of four lanes <-> load u in lane t
+__device__ __forceinline__ void deal_loads(floatx4& b0, floatx4& b1, floatx4& b2, floatx4& b3) {
+    exchange<LANES_1>(b0, b1); exchange<LANES_1>(b2, b3);
+    exchange<LANES_2>(b0, b2); exchange<LANES_2>(b1, b3);
+}
+// value i of four loads in group of four lanes q of sixteen <-> value q in group i
+__device__ __forceinline__ void deal_values(floatx4& b0, floatx4& b1, floatx4& b2, floatx4& b3) {
+    floatx4 x0 = {b0[0], b1[0], b2[0], b3[0]}, x1 = {b0[1], b1[1], b2[1], b3[1]}, x2 = {b0[2], b1[2], b2[2], b3[2]}, x3 = {b0[3], b1[3], b2[3], b3[3]};
+    exchange<LANES_4>(x0, x1); exchange<LANES_4>(x2, x3);
+    exchange<LANES_8>(x0, x2); exchange<LANES_8>(x1, x3);
+    b0 = floatx4{x0[0], x1[0], x2[0], x3[0]}; b1 = floatx4{x0[1], x1[1], x2[1], x3[1]}; b2 = floatx4{x0[2], x1[2], x2[2], x3[2]}; b3 = floatx4{x0[3], x1[3], x2[3], x3[3]};
+}
+// forward: rows 16 w + c of W2, half h of the reduction; after deal_second() element 4 p + t of lane (c, g) holds k = 64 p + 16 g + 4 t ...
+__device__ __forceinline__ void request_second(const float* W2, int wave, int c, int g, int half, floatx4 (&b)[8]) {
+    const float* const mine = W2 + (size_t)(16 * wave + (c & 12)) * MAX_H + 128 * half + 16 * g + 4 * (c & 3);
+#pragma unroll
+    for (int p = 0; p < 2; p++)
+#pragma unroll
+        for (int t = 0; t < 4; t++) b[4 * p + t] = *reinterpret_cast<const floatx4*>(mine + t * MAX_H + 64 * p);
+}
+__device__ __forceinline__ void deal_second(floatx4 (&b)[8]) { deal_loads(b[0], b[1], b[2], b[3]); deal_loads(b[4], b[5], b[6], b[7]); }
+// backward: columns 16 w ... of W2. Tiles of sixteen rows: after deal_values() element j of lane (c, g) holds rows 16 j + 4 g ... + 3 of column own_column(w, c). Tiles of four and eight need no
+// dealing: element j of lane l holds row 16 (l / 4) + j, columns 16 w + 4 (l % 4) ... + 3 (column_products), and the sums end in the same column.
+template <int R>
+__device__ __forceinline__ void request_second_columns(const float* W2, int wave, int c, int g, floatx4 (&b)[MAX_H / 16]) {
+    const float* const mine = W2 + (size_t)(R == ROWS ? 4 * g + (c >> 2) : 16 * (4 * g + (c >> 2))) * MAX_H + 16 * wave + 4 * (c & 3);
+#pragma unroll
+    for (int j = 0; j < MAX_H / 16; j++) b[j] = *reinterpret_cast<const floatx4*>(mine + (size_t)(R == ROWS ? 16 : 1) * j * MAX_H);
+}
+template <int FORM> __device__ __forceinline__ int own_column(int wave, int c) { return 16 * wave + (FORM == FORM_DIRECT ? 4 * (c & 3) + (c >> 2) : c); }
+// first layer: rows 16 w + 4 q + g, column 16 j + c into element q of chunk j; place_first() turns them into the operands that the copies hold
+template <int NT1C>
+__device__ __forceinline__ void request_first(const float* W1, int in, int wave, int c, int g, floatx4 (&b)[NT1C]) {
+#pragma unroll
+    for (int j = 0; j < NT1C; j++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) b[j][q] = W1[(size_t)(16 * wave + 4 * q + g) * in + min(16 * j + c, in - 1)];
+}
+template <int NT1C>
+__device__ __forceinline__ void place_first(int in, lptr stage, int c, int g, floatx4 (&b)[NT1C]) {
+#pragma unroll
+    for (int j0 = 0; j0 < NT1C; j0 += 2) {
+#pragma unroll
+        for (int j = j0; j < j0 + 2; j++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) stage[(4 * q + g) * W1S + 16 * (j & 1) + c] = 16 * j + c < in ? b[j][q] : 0.f;
+        wave_sync();
+#pragma unroll
+        for (int j = j0; j < j0 + 2; j++) b[j] = *(lptr4)(stage + c * W1S + 16 * (j & 1) + 4 * g);
+        wave_sync();
+    }
+}
 template <int JN, bool EVERY = false, int STEP = 4>
 __device__ __forceinline__ void load_swizzled(const float* __restrict__ copy, int tiles, bool on, int wave, int lane, int j0, floatx4 (&b)[JN]) {      // tiles: chunks of the copy; on: this wavefront has units
     if (EVERY) {
@@ -122,14 +205,14 @@ __device__ __forceinline__ void chunk4(Sums<R>& A, const floatx4 (&a)[R / 4], fl
 #pragma unroll
         for (int h = 0; h < R / 4; h++) A.s[h][i & 1] = mfma4<Q>(a[h][i], b[i], A.s[h][i & 1]);
 }
-// A += in[rows][16 (j0 + j) + ...] * b[j], j0 a multiple of four
-template <int R, int JN>
+// A += in[rows][16 (j0 + j) + ...] * b[j], j0 a multiple of four; ROWS_AS_THEY_LIE: b[4 p + t] holds k = 64 p + 16 g + 4 t ... (deal_second) instead of 16 (4 p + t) + 4 g ...
+template <int R, bool ROWS_AS_THEY_LIE = false, int JN>
 __device__ __forceinline__ void chunks(Sums<R>& A, lptr in, int stride, int c, int g, int j0, int steps, const floatx4 (&b)[JN]) {
     if constexpr (R == 16) {
 #pragma unroll
         for (int j = 0; j < JN; j++) {
             if (j0 + j < steps) {
-                const floatx4 a = *(lptr4)(in + c * stride + 16 * (j0 + j) + 4 * g);
+                const floatx4 a = *(lptr4)(in + c * stride + (ROWS_AS_THEY_LIE ? 64 * ((j0 + j) >> 2) + 16 * g + 4 * (j & 3) : 16 * (j0 + j) + 4 * g));
                 A.s[0][0] = mfma16(a[0], b[j][0], A.s[0][0]); A.s[0][1] = mfma16(a[1], b[j][1], A.s[0][1]);
                 A.s[0][0] = mfma16(a[2], b[j][2], A.s[0][0]); A.s[0][1] = mfma16(a[3], b[j][3], A.s[0][1]);
             }
@@ -140,7 +223,7 @@ __device__ __forceinline__ void chunks(Sums<R>& A, lptr in, int stride, int c, i
             if (j0 + j < steps) {
                 floatx4 a[R / 4];      // (columns of chunks beyond the width hold anything: nobody multiplies them)
 #pragma unroll
-                for (int h = 0; h < R / 4; h++) a[h] = *(lptr4)(in + ((c & 3) + 4 * h) * stride + 16 * (j0 + j + (c >> 2)) + 4 * g);
+                for (int h = 0; h < R / 4; h++) a[h] = *(lptr4)(in + ((c & 3) + 4 * h) * stride + 16 * (j0 + j) + (ROWS_AS_THEY_LIE ? 16 * g + (c & 12) : 4 * (c & 12) + 4 * g));
                 chunk4<R, 0>(A, a, b[j]);
                 if (j + 1 < JN && j0 + j + 1 < steps) chunk4<R, 1>(A, a, b[j + 1 < JN ? j + 1 : 0]);
                 if (j + 2 < JN && j0 + j + 2 < steps) chunk4<R, 2>(A, a, b[j + 2 < JN ? j + 2 : 0]);
@@ -174,6 +257,54 @@ __device__ __forceinline__ void finished(const Sums<R>& A, float (&out)[R / 4]) 
     }
 }
 
+// Tiles of four and eight rows times 256 rows of W as request_second_columns() has asked for them: block l / 4 of the matrix instruction takes its sixteen rows of the reduction, instruction i column
+// i of each lane's four. out: as finished() leaves it, for column own_column(): the blocks' shares are added up in exchanges that leave each half of the rows, then each half of the columns.
+template <int CTRL> __device__ __forceinline__ float lane_move(float x) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, true)); }
+template <int R>
+__device__ __forceinline__ void column_products(lptr in, int stride, int lane, const floatx4 (&b)[MAX_H / 16], float (&out)[R / 4]) {
+    constexpr int N = R / 4, E = R / 4;
+    floatx4 sum[N][4];
+#pragma unroll
+    for (int h = 0; h < N; h++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) sum[h][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j0 = 0; j0 < MAX_H / 16; j0 += 4) {
+        floatx4 a[N];
+#pragma unroll
+        for (int h = 0; h < N; h++) a[h] = *(lptr4)(in + ((lane & 3) + 4 * h) * stride + 16 * (lane >> 2) + j0);
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int h = 0; h < N; h++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) sum[h][i] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[h][j], b[j0 + j][i], sum[h][i], 0, 0, 0);
+    }
+    float t[E][4];      // rows E g + v, column i of the lane's four, summed over the lane groups
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        float s[2 * E];
+#pragma unroll
+        for (int v = 0; v < 2 * E; v++) {
+            const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(sum[v / 4][i][v & 3]), __float_as_uint(sum[(2 * E + v) / 4][i][(2 * E + v) & 3]), false, false);
+            s[v] = __uint_as_float(x[0]) + __uint_as_float(x[1]);
+        }
+#pragma unroll
+        for (int v = 0; v < E; v++) {
+            const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(s[v]), __float_as_uint(s[E + v]), false, false);
+            t[v][i] = __uint_as_float(x[0]) + __uint_as_float(x[1]);
+        }
+    }
+    const bool third = lane & 8, second = lane & 4;      // which column of the four this lane ends with: (lane / 4) % 4
+#pragma unroll
+    for (int v = 0; v < E; v++) {
+        const float p = (third ? t[v][2] : t[v][0]) + lane_move<0x128>(third ? t[v][0] : t[v][2]);
+        const float q = (third ? t[v][3] : t[v][1]) + lane_move<0x128>(third ? t[v][1] : t[v][3]);
+        const float lower = lane_move<0x104>(p), upper = lane_move<0x114>(q);      // the first column's share of the group above, the second's of the group below
+        out[v] = second ? q + upper : p + lower;
+    }
+}
+
 // profiling builds (-DRLT_WIDE_PROFILE): thread 0 of workgroup 0 notes the constant-rate clock at the stage boundaries, rlt_sac_wide_ticks copies the notes out
 #ifdef RLT_WIDE_PROFILE
 __device__ unsigned long long rlt_wide_ticks[2][32];
@@ -202,15 +333,25 @@ __device__ __forceinline__ void mask_w3(const WNet& N, int wave, int c, int g, f
 }
 // everything of network N that forward3 reads from memory, requested at once (few first-layer operands leave room for the whole second layer; otherwise its second
 // half is requested after the first layer has run)
-template <int NT1C, bool EVERY = false>
+template <int NT1C, int FORM>
+__device__ __forceinline__ void load_first(const WNet& N, bool on, int wave, int c, int g, floatx4 (&b)[NT1C]) {
+    if (FORM == FORM_DIRECT) request_first(N.W1, N.in, wave, c, g, b);
+    else load_swizzled<NT1C, false, FIRST_STEP<NT1C>>(N.W1f, (N.in + 15) >> 4, on, wave, c + 16 * g, 0, b);
+}
+template <int FORM>
+__device__ __forceinline__ void load_second(const WNet& N, int tiles, bool on, int wave, int c, int g, int half, floatx4 (&b)[8]) {
+    if (FORM == FORM_DIRECT) request_second(N.W2, wave, c, g, half, b);
+    else load_swizzled<8, FORM == FORM_EVERY>(N.W2f, tiles, on, wave, c + 16 * g, 8 * half, b);
+}
+template <int NT1C, int FORM = FORM_ANY>
 __device__ __forceinline__ void load_operands(const WNet& N, int wave, int c, int g, Operands<NT1C>& W) {
-    const int n = 16 * wave + c, tiles = (N.hid + 15) >> 4, lane = c + 16 * g;
+    const int n = 16 * wave + c, tiles = (N.hid + 15) >> 4;
     const bool on = wave < tiles;
-    if (!EVERY && !on) return;
-    load_swizzled<NT1C, false, FIRST_STEP<NT1C>>(N.W1f, (N.in + 15) >> 4, on, wave, lane, 0, W.w1);
+    if (FORM == FORM_ANY && !on) return;
+    load_first<NT1C, FORM>(N, on, wave, c, g, W.w1);
     W.b1 = N.b1[min(n, N.hid - 1)]; W.b2 = N.b2[min(n, N.hid - 1)];
-    load_swizzled<8, EVERY>(N.W2f, tiles, on, wave, lane, 0, W.w2a);
-    if (NT1C <= FEW) load_swizzled<8, EVERY>(N.W2f, tiles, on, wave, lane, 8, W.w2b);
+    load_second<FORM>(N, tiles, on, wave, c, g, 0, W.w2a);
+    if (NT1C <= FEW) load_second<FORM>(N, tiles, on, wave, c, g, 1, W.w2b);
     W.w3 = load_w3(N, wave, c, g);
 }
 
@@ -242,31 +383,36 @@ __device__ __forceinline__ void place_hidden(const WNet& N, const Sums<R>& sums,
         }
     }
 }
-template <int R, int ACT_H, int NT1C, bool PREFETCH, bool W1_READY, bool KEEP = false, bool EVERY = false, bool LIVE = false>
-__device__ __forceinline__ void forward3(const WNet& N, Operands<NT1C>& W, const WNet& next, lptr x, int xstride, lptr h1, lptr h2, lptr yp, int wave, int c, int g, const KeepArgs* keep = nullptr, int live = ROWS) {
-    const int n = 16 * wave + c, tiles = (N.hid + 15) >> 4, lane = c + 16 * g, next_tiles = (next.hid + 15) >> 4;
-    const bool on = wave < tiles, next_on = wave < next_tiles;
+template <int R, int ACT_H, int NT1C, bool PREFETCH, bool W1_READY, bool KEEP = false, int FORM = FORM_ANY, bool LIVE = false>
+__device__ __forceinline__ void forward3(const WNet& N, Operands<NT1C>& W, const WNet& next, lptr x, int xstride, lptr h1, lptr h2, lptr yp, lptr stage, int wave, int c, int g, const KeepArgs* keep = nullptr,
+                                         int live = ROWS) {
+    constexpr bool DIRECT = FORM == FORM_DIRECT;
+    const int n = 16 * wave + c, tiles = DIRECT ? MAX_H / 16 : (N.hid + 15) >> 4, lane = c + 16 * g, next_tiles = DIRECT ? MAX_H / 16 : (next.hid + 15) >> 4;
+    const bool on = DIRECT || wave < tiles, next_on = DIRECT || wave < next_tiles;
     const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
-    if (!W1_READY) load_swizzled<NT1C, false, FIRST_STEP<NT1C>>(N.W1f, (N.in + 15) >> 4, on, wave, lane, 0, W.w1);
+    if (!W1_READY) load_first<NT1C, FORM>(N, on, wave, c, g, W.w1);
+    if (DIRECT) place_first(N.in, stage, c, g, W.w1);
     if (on) {
         Sums<R> sums;
         clear(sums);
-        chunks<R, NT1C>(sums, x, xstride, c, g, 0, (N.in + 15) >> 4, W.w1);
+        chunks<R>(sums, x, xstride, c, g, 0, (N.in + 15) >> 4, W.w1);
         place_hidden<R, ACT_H, KEEP, LIVE>(N, sums, W.b1, h1, n, g, keep, 0, live);
     }
-    if (NT1C > FEW) load_swizzled<8, EVERY>(N.W2f, tiles, on, wave, lane, 8, W.w2b);
+    if (NT1C > FEW) load_second<FORM>(N, tiles, on, wave, c, g, 1, W.w2b);
     if (PREFETCH) {
-        if (NT1C <= FEW) load_swizzled<NT1C, false, FIRST_STEP<NT1C>>(next.W1f, (next.in + 15) >> 4, next_on, wave, lane, 0, W.w1);
+        if (NT1C <= FEW) load_first<NT1C, FORM>(next, next_on, wave, c, g, W.w1);
         W.b1 = next.b1[min(n, next.hid - 1)];
     }
+    if (DIRECT) deal_second(W.w2a);      // (while the others finish their tiles of the first layer)
     rlt_lds_barrier();
     {
         Sums<R> sums;
         clear(sums);
-        if (on) chunks<R, 8>(sums, h1, S, c, g, 0, tiles, W.w2a);
-        if (PREFETCH) load_swizzled<8, EVERY>(next.W2f, next_tiles, next_on, wave, lane, 0, W.w2a);
-        if (on) chunks<R, 8>(sums, h1, S, c, g, 8, tiles, W.w2b);
-        if (PREFETCH && NT1C <= FEW) load_swizzled<8, EVERY>(next.W2f, next_tiles, next_on, wave, lane, 8, W.w2b);
+        if (on) chunks<R, DIRECT>(sums, h1, S, c, g, 0, tiles, W.w2a);
+        if (PREFETCH) load_second<FORM>(next, next_tiles, next_on, wave, c, g, 0, W.w2a);
+        if (DIRECT) deal_second(W.w2b);
+        if (on) chunks<R, DIRECT>(sums, h1, S, c, g, 8, tiles, W.w2b);
+        if (PREFETCH && NT1C <= FEW) load_second<FORM>(next, next_tiles, next_on, wave, c, g, 1, W.w2b);
         if (on) place_hidden<R, ACT_H, KEEP, LIVE>(N, sums, W.b2, h2, n, g, keep, 1, live);
         if (PREFETCH) W.b2 = next.b2[min(n, next.hid - 1)];
     }
@@ -303,12 +449,13 @@ __device__ __forceinline__ floatx4 output_tile(lptr yp, int tiles, int c, int g)
 
 // column n of W3 for this lane's share of the reduction over the outputs, and the second layer's backward copy: the operands of a backward pass, requested ahead of it
 struct BackOperands { float w3[MAX_OUT / 4]; floatx4 w2[MAX_H / 16]; };
-template <bool EVERY = false>
+template <int R, int FORM = FORM_ANY>
 __device__ __forceinline__ void load_back_operands(const WNet& N, int wave, int c, int g, BackOperands& W) {
     const int n = 16 * wave + c, tiles = (N.hid + 15) >> 4;
 #pragma unroll
     for (int ks = 0; ks < MAX_OUT / 4; ks++) W.w3[ks] = N.W3[(size_t)min(4 * ks + g, N.out - 1) * N.hid + min(n, N.hid - 1)];
-    load_swizzled<MAX_H / 16, EVERY>(N.W2b, tiles, wave < tiles, wave, c + 16 * g, 0, W.w2);
+    if (FORM == FORM_DIRECT) request_second_columns<R>(N.W2, wave, c, g, W.w2);
+    else load_swizzled<MAX_H / 16, FORM == FORM_EVERY>(N.W2b, tiles, wave < tiles, wave, c + 16 * g, 0, W.w2);
 }
 // this wavefront's tile of d_pre2 = (d_pre3 W3) f'(h2) into g2 (may be h2 itself); returns the lane's share of its unit's column sum
 template <int ACT_H, bool LIVE = false>
@@ -328,15 +475,22 @@ __device__ __forceinline__ float backward_layer3(const WNet& N, const BackOperan
     return sum;
 }
 // this wavefront's tile of d_pre1 = (d_pre2 W2) f'(h1) into p1 (may be h1 itself); returns the lane's share of its unit's column sum
-template <int R, int ACT_H, bool LIVE = false>
-__device__ __forceinline__ float backward_layer2(const WNet& N, const BackOperands& W, lptr g2, lptr h1, lptr p1, int wave, int c, int g, int live = ROWS) {
-    const int n = 16 * wave + c, tiles = (N.hid + 15) >> 4;
+template <int R, int ACT_H, int FORM = FORM_ANY, bool LIVE = false>
+__device__ __forceinline__ float backward_layer2(const WNet& N, BackOperands& W, lptr g2, lptr h1, lptr p1, int wave, int c, int g, int live = ROWS) {
+    const int n = own_column<FORM>(wave, c), tiles = FORM == FORM_DIRECT ? MAX_H / 16 : (N.hid + 15) >> 4;
     const bool n_ok = n < N.hid;
-    Sums<R> sums;
-    clear(sums);
-    chunks<R, MAX_H / 16>(sums, g2, S, c, g, 0, tiles, W.w2);
     float acc[R / 4], sum = 0.f;
-    finished<R>(sums, acc);
+    if constexpr (FORM == FORM_DIRECT && R != ROWS) column_products<R>(g2, S, c + 16 * g, W.w2, acc);
+    else {
+        Sums<R> sums;
+        clear(sums);
+        if (FORM == FORM_DIRECT) {
+#pragma unroll
+            for (int j = 0; j < MAX_H / 16; j += 4) deal_values(W.w2[j], W.w2[j + 1], W.w2[j + 2], W.w2[j + 3]);
+        }
+        chunks<R>(sums, g2, S, c, g, 0, tiles, W.w2);
+        finished<R>(sums, acc);
+    }
 #pragma unroll
     for (int v = 0; v < R / 4; v++) {
         const int row = R / 4 * g + v, idx = row * S + n;
@@ -454,6 +608,7 @@ constexpr size_t MAX_COPY_FLOATS = (size_t)WAVES * (MAX_H / 16) * 256, MAX_W1_CO
 // EVERY: all networks have more than 240 units
 template <int MODE, int ACT_H, int NT1C, bool EVERY, int R>
 __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
+    constexpr int FORM = EVERY ? FORM_EVERY : FORM_ANY;
     constexpr bool CRITIC = MODE == MODE_CRITIC || MODE == MODE_TD3_CRITIC, TD3 = MODE == MODE_TD3_CRITIC || MODE == MODE_TD3_ACTOR;
     extern __shared__ __attribute__((aligned(16))) float lds_wide[];
     const int G = A.groups;
@@ -488,7 +643,7 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
         const Trained T = y ? A.trained[1] : A.trained[0];
         const int HID = trained.hid, tiles = (HID + 15) >> 4;
         Operands<NT1C> W;
-        load_operands<NT1C, EVERY>(trained, wave, c, g, W);
+        load_operands<NT1C, FORM>(trained, wave, c, g, W);
         place_row(xa + wave * SXS, row0 + wave < row_end, D, SXS, lane, in_row);
         float reward[4] = {0.f, 0.f, 0.f, 0.f}, alpha = 0.f, b3 = 0.f;
         bool terminated[4] = {false, false, false, false};
@@ -500,10 +655,10 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
         }
         rlt_lds_barrier();      // the input rows are in place
         RLT_TICK(1);
-        forward3<R, ACT_H, NT1C, false, true, false, EVERY>(trained, W, trained, xa, SXS, h1, h2, yp, wave, c, g);
+        forward3<R, ACT_H, NT1C, false, true, false, FORM>(trained, W, trained, xa, SXS, h1, h2, yp, nullptr, wave, c, g);
         RLT_TICK(2);
         BackOperands K;
-        load_back_operands<EVERY>(trained, wave, c, g, K);      // on their way while the targets' values are waited for
+        load_back_operands<R, FORM>(trained, wave, c, g, K);      // on their way while the targets' values are waited for
         store_rows<R>(h1, T.h1, HID, row0, row_end, wave, lane);
         store_rows<R>(h2, T.h2, HID, row0, row_end, wave, lane);
         if (scalar_wave) {
@@ -556,7 +711,7 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
     const bool writes = target_role ? role == 0 : owner;      // of the roles that compute the same sample, the one that stores what is asked for
     const WNet Q = CRITIC ? (critic_index ? A.target[1] : A.target[0]) : (critic_index ? A.critic[1] : A.critic[0]);
     Operands<NT1C> W;
-    load_operands<NT1C, EVERY>(A.actor, wave, c, g, W);      // on their way while the input rows are written
+    load_operands<NT1C, FORM>(A.actor, wave, c, g, W);      // on their way while the input rows are written
     place_row(xa + wave * SXS, row0 + wave < row_end, OBS, SXS, lane, in_row);
     float alpha = 0.f, actor_b3 = 0.f, q_b3 = 0.f;
     if (scalar_wave) {
@@ -590,7 +745,7 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
     RLT_TICK(13);
     rlt_lds_barrier();      // the input rows are in place
     RLT_TICK(5);
-    forward3<R, ACT_H, NT1C, true, true, false, EVERY>(A.actor, W, Q, xa, SXS, h1, h2, yp, wave, c, g);
+    forward3<R, ACT_H, NT1C, true, true, false, FORM>(A.actor, W, Q, xa, SXS, h1, h2, yp, nullptr, wave, c, g);
     RLT_TICK(6);
     if (scalar_wave) {
         const floatx4 out = output_tile(yp, (A.actor.hid + 15) >> 4, c, g);
@@ -622,7 +777,7 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
     }
     rlt_lds_barrier();      // the action columns of xa are in place
     RLT_TICK(7);
-    forward3<R, ACT_H, NT1C, false, NT1C <= FEW, false, EVERY>(Q, W, Q, xa, SXS, ta, tb, yp, wave, c, g);
+    forward3<R, ACT_H, NT1C, false, NT1C <= FEW, false, FORM>(Q, W, Q, xa, SXS, ta, tb, yp, nullptr, wave, c, g);
     RLT_TICK(8);
     const int qtiles = (Q.hid + 15) >> 4;
     if (CRITIC) {
@@ -637,7 +792,7 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
     // ---- actor update: the gradient of -value / batch with respect to the action (TD3: critic 0 only, rl/algorithms/td3/operations_generic.h:260)
     const float loss_weight = (1.0f / (float)B) * -1.0f;       // rl/algorithms/sac/operations_generic.h:437-453 with n = batch rows
     BackOperands K;
-    load_back_operands<EVERY>(Q, wave, c, g, K);
+    load_back_operands<R, FORM>(Q, wave, c, g, K);
     float w1[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) { const int unit = 16 * wave + 4 * g + i; w1[i] = (c < ACT && unit < Q.hid) ? Q.W1[(size_t)unit * D + OBS + c] : 0.f; }
@@ -678,7 +833,7 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
     const WNet trained = A.actor;
     const Trained T = A.trained[0];
     const int HID = trained.hid, tiles = (HID + 15) >> 4;
-    load_back_operands<EVERY>(trained, wave, c, g, K);
+    load_back_operands<R, FORM>(trained, wave, c, g, K);
     store_rows<R>(h1, T.h1, HID, row0, row_end, wave, lane);
     store_rows<R>(h2, T.h2, HID, row0, row_end, wave, lane);
     if (scalar_wave) {
@@ -735,7 +890,7 @@ __global__ __launch_bounds__(THREADS) void sac_wide_kernel(WideArgs A) {
     RLT_TICK(12);
 }
 
-constexpr size_t LDS_FLOATS = (size_t)ROWS * SXS + 4 * ROWS * S + 4 * ROWS * D3S + WAVES * YP + MISC;
+constexpr size_t LDS_FLOATS = (size_t)ROWS * SXS + 4 * ROWS * S + 4 * ROWS * D3S + WAVES * YP + MISC, DIRECT_LDS_FLOATS = LDS_FLOATS + WAVES * W1_STAGE;
 
 // ---- Forward and backward pass of one three-layer network over a few thousand rows at most, on the same machinery (nn_models/mlp/operations_generic.h:103-204: forward, the
 // loss gradient given or formed from a target as the MSE's, backward with weight gradients): a workgroup takes 16, 8 or 4 rows through the three layers and back and leaves
@@ -755,16 +910,18 @@ struct MlpWideArgs {
     float* keep_pre[3]; float* keep_out[3]; int act3;      // MLP_FORWARD: every layer's pre-activations and outputs as forward() keeps them (each may be NULL); the last layer's activation
 };
 enum { MLP_FORWARD_BACKWARD = 0, MLP_BACKWARD = 1, MLP_FORWARD = 2 };
-enum { MLP_ANY = 0, MLP_BLOCKS = 1, MLP_EVERY = 2 };      // MLP_BLOCKS: weight gradients as blocks; MLP_EVERY: more than 240 units, every wavefront has some
-template <int ACT_H, int NT1C, int PASS, int FORM, int R>
+enum { MLP_ANY = 0, MLP_BLOCKS = 1, MLP_EVERY = 2, MLP_DIRECT = 3 };      // MLP_BLOCKS: weight gradients as blocks; MLP_EVERY: more than 240 units, every wavefront has some; MLP_DIRECT: FORM_DIRECT
+template <int ACT_H, int NT1C, int PASS, int KIND, int R>
 __global__ __launch_bounds__(THREADS) void mlp_wide_kernel(MlpWideArgs A) {
-    constexpr bool BACKWARD_ONLY = PASS == MLP_BACKWARD, BLOCKS = FORM == MLP_BLOCKS, EVERY = FORM == MLP_EVERY;
+    constexpr bool BACKWARD_ONLY = PASS == MLP_BACKWARD, BLOCKS = KIND == MLP_BLOCKS;
+    constexpr int FORM = KIND == MLP_DIRECT ? FORM_DIRECT : KIND == MLP_EVERY ? FORM_EVERY : FORM_ANY;
+    constexpr bool EVERY = FORM != FORM_ANY;
     extern __shared__ __attribute__((aligned(16))) float lds_wide[];
     static_assert(R == 16 || !BLOCKS, "blocks are formed over sixteen rows");
     const int gi = blockIdx.x;
     const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const lptr xa = (lptr)lds_wide, h1 = xa + ROWS * SXS, h2 = h1 + ROWS * S, ta = h2 + ROWS * S, tb = ta + ROWS * S, d3 = tb + ROWS * S, yp = d3 + 4 * ROWS * D3S;
+    const lptr xa = (lptr)lds_wide, h1 = xa + ROWS * SXS, h2 = h1 + ROWS * S, ta = h2 + ROWS * S, tb = ta + ROWS * S, d3 = tb + ROWS * S, yp = d3 + 4 * ROWS * D3S, stage = yp + WAVES * YP + MISC + wave * W1_STAGE;
     const WNet N = A.net;
     const int B = A.batch, IN = N.in, HID = N.hid, OUT = N.out, tiles = (HID + 15) >> 4, row0 = gi * R, row_end = min(B, row0 + R);
     const bool on = wave < tiles;
@@ -786,7 +943,7 @@ __global__ __launch_bounds__(THREADS) void mlp_wide_kernel(MlpWideArgs A) {
         if (BLOCKS) request_row(A.x + row_at * A.ldx, IN, lane, vx);
         request_row(A.out1 + row_at * HID, HID, lane, v1);
         request_row(A.out2 + row_at * HID, HID, lane, v2);
-        if (on) load_back_operands<EVERY>(N, wave, c, g, K);
+        if (on) load_back_operands<R, FORM>(N, wave, c, g, K);
         place_row(h1 + wave * S, my_row, HID, 16 * tiles, lane, v1);
         place_row(h2 + wave * S, my_row, HID, 16 * tiles, lane, v2);
         if (BLOCKS) place_row(xa + wave * SXS, my_row, IN, SXS, lane, vx);
@@ -801,7 +958,7 @@ __global__ __launch_bounds__(THREADS) void mlp_wide_kernel(MlpWideArgs A) {
     } else {
         float v[3];
         request_row(A.x + row_at * A.ldx, IN, lane, v);
-        load_operands<NT1C, EVERY>(N, wave, c, g, W);
+        load_operands<NT1C, FORM>(N, wave, c, g, W);
         b3 = N.b3[min(c, OUT - 1)];
         place_row(xa + wave * SXS, my_row, IN, SXS, lane, v);
         if (PASS == MLP_FORWARD_BACKWARD && !BLOCKS && A.copy_x && my_row) {
@@ -812,7 +969,7 @@ __global__ __launch_bounds__(THREADS) void mlp_wide_kernel(MlpWideArgs A) {
     rlt_lds_barrier();
     if (PASS == MLP_FORWARD) {
         const KeepArgs keep = {{A.keep_pre[0], A.keep_pre[1]}, {A.keep_out[0], A.keep_out[1]}, row0, row_end};
-        forward3<R, ACT_H, NT1C, false, true, true, EVERY>(N, W, N, xa, SXS, h1, h2, yp, wave, c, g, &keep);
+        forward3<R, ACT_H, NT1C, false, true, true, FORM>(N, W, N, xa, SXS, h1, h2, yp, stage, wave, c, g, &keep);
         if (wave == 0) {
             const floatx4 out = output_tile(yp, tiles, c, g);
 #pragma unroll
@@ -830,9 +987,9 @@ __global__ __launch_bounds__(THREADS) void mlp_wide_kernel(MlpWideArgs A) {
         return;
     }
     if (PASS == MLP_FORWARD_BACKWARD) {
-        forward3<R, ACT_H, NT1C, false, true, false, EVERY, BLOCKS>(N, W, N, xa, SXS, h1, h2, yp, wave, c, g, nullptr, B - row0);
+        forward3<R, ACT_H, NT1C, false, true, false, FORM, BLOCKS>(N, W, N, xa, SXS, h1, h2, yp, stage, wave, c, g, nullptr, B - row0);
         if (EVERY) request_given();      // (all of W fills the registers until here)
-        load_back_operands<EVERY>(N, wave, c, g, K);
+        load_back_operands<R, FORM>(N, wave, c, g, K);
         if (!BLOCKS) {
             store_rows<R>(h1, A.kept.h1, HID, row0, row_end, wave, lane);
             store_rows<R>(h2, A.kept.h2, HID, row0, row_end, wave, lane);
@@ -872,7 +1029,7 @@ __global__ __launch_bounds__(THREADS) void mlp_wide_kernel(MlpWideArgs A) {
         if (spread ? !on && wave - tiles < tiles : on) last_layer(spread ? wave - tiles : wave);
         rlt_lds_barrier();      // every wavefront's tile of d_pre2 is in place
         if (on) {
-            const float s1 = backward_layer2<R, ACT_H, BLOCKS>(N, K, ta, h1, tb, wave, c, g, B - row0);
+            const float s1 = backward_layer2<R, ACT_H, FORM, BLOCKS>(N, K, ta, h1, tb, wave, c, g, B - row0);
             wave_sync();            // dW1's rows are this wavefront's own tile of d_pre1
 #pragma unroll 2
             for (int nt = 0; nt < (IN + 15) >> 4; nt++) gradient_tile(tb, wave, xa, SXS, nt, HID, IN, block, c, g);
@@ -894,7 +1051,7 @@ __global__ __launch_bounds__(THREADS) void mlp_wide_kernel(MlpWideArgs A) {
     }
     rlt_lds_barrier();      // every wavefront's tile of d_pre2 is in place
     store_rows<R>(ta, A.kept.d2, HID, row0, row_end, wave, lane);
-    if (on) backward_layer2<R, ACT_H>(N, K, ta, h1, tb, wave, c, g);
+    if (on) backward_layer2<R, ACT_H, FORM>(N, K, ta, h1, tb, wave, c, g);
     rlt_lds_barrier();
     store_rows<R>(tb, A.kept.d1, HID, row0, row_end, wave, lane);
 }
@@ -1293,12 +1450,15 @@ static int mlp_wide_launch(rlt_rocm_device* device, const rlt_dense_layer* L, in
         partial = (float*)scratch + trained_floats(hid, batch) + copy_floats;
         set_rows(net, a.kept, in_place ? a.copy_x : x, in_place ? IN : ldx);
     }
-    if ((rc = rlt_mlp_wide_reserve(device))) return rc;
-    Copies copies((float*)device->copy_scratch);
-    if (!backward_only) copies.forward(a.net);
-    if (!forward_only) copies.backward(a.net);
-    if ((rc = copies.launch(device))) return rc;
-    const size_t lds_bytes = LDS_FLOATS * sizeof(float);
+    const bool direct = !blocks && hid == MAX_H && aligned16(a.net.W2) && DIRECT_LDS_FLOATS * sizeof(float) <= (size_t)device->lds_bytes;
+    if (!direct) {
+        if ((rc = rlt_mlp_wide_reserve(device))) return rc;
+        Copies copies((float*)device->copy_scratch);
+        if (!backward_only) copies.forward(a.net);
+        if (!forward_only) copies.backward(a.net);
+        if ((rc = copies.launch(device))) return rc;
+    }
+    const size_t lds_bytes = (direct ? DIRECT_LDS_FLOATS : LDS_FLOATS) * sizeof(float);
 #define RLT_LAUNCH_MLP_WIDE_ROWS(ACT, NT, P, FORM, R)                                                                                                           \
     do {                                                                                                                                                       \
         RLT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(mlp_wide_kernel<ACT, NT, P, FORM, R>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes)); \
@@ -1306,7 +1466,7 @@ static int mlp_wide_launch(rlt_rocm_device* device, const rlt_dense_layer* L, in
     } while (0)
 #define RLT_LAUNCH_MLP_WIDE(ACT, NT, P, FORM)                                                                                                                   \
     do {                                                                                                                                                       \
-        constexpr int FEWEST = FORM == MLP_BLOCKS ? ROWS : FORM == MLP_EVERY ? 4 : 8;                                                                          \
+        constexpr int FEWEST = FORM == MLP_BLOCKS ? ROWS : FORM >= MLP_EVERY ? 4 : 8;                                                                          \
         if (rows < FEWEST) return RLT_E_UNSUPPORTED;                                                                                                           \
         if (rows == 4) RLT_LAUNCH_MLP_WIDE_ROWS(ACT, NT, P, FORM, FEWEST);                                                                                     \
         else if (rows == 8) RLT_LAUNCH_MLP_WIDE_ROWS(ACT, NT, P, FORM, (FEWEST > 8 ? FEWEST : 8));                                                             \
@@ -1319,9 +1479,9 @@ static int mlp_wide_launch(rlt_rocm_device* device, const rlt_dense_layer* L, in
         else if (IN <= 64) { if (relu) RLT_LAUNCH_MLP_WIDE(RLT_ACT_RELU, 4, P, FORM); else RLT_LAUNCH_MLP_WIDE(-1, 4, P, FORM); }                                \
         else { if (relu) RLT_LAUNCH_MLP_WIDE(RLT_ACT_RELU, MAX_D / 16, P, FORM); else RLT_LAUNCH_MLP_WIDE(-1, MAX_D / 16, P, FORM); }                            \
     } while (0)
-    if (forward_only) { if (every) RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD, MLP_EVERY); else RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD, MLP_ANY); }
-    else if (backward_only) { if (blocks) RLT_LAUNCH_MLP_WIDE_PASS(MLP_BACKWARD, MLP_BLOCKS); else if (every) RLT_LAUNCH_MLP_WIDE_PASS(MLP_BACKWARD, MLP_EVERY); else RLT_LAUNCH_MLP_WIDE_PASS(MLP_BACKWARD, MLP_ANY); }
-    else { if (blocks) RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD_BACKWARD, MLP_BLOCKS); else if (every) RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD_BACKWARD, MLP_EVERY); else RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD_BACKWARD, MLP_ANY); }
+    if (forward_only) { if (direct) RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD, MLP_DIRECT); else if (every) RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD, MLP_EVERY); else RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD, MLP_ANY); }
+    else if (backward_only) { if (blocks) RLT_LAUNCH_MLP_WIDE_PASS(MLP_BACKWARD, MLP_BLOCKS); else if (direct) RLT_LAUNCH_MLP_WIDE_PASS(MLP_BACKWARD, MLP_DIRECT); else if (every) RLT_LAUNCH_MLP_WIDE_PASS(MLP_BACKWARD, MLP_EVERY); else RLT_LAUNCH_MLP_WIDE_PASS(MLP_BACKWARD, MLP_ANY); }
+    else { if (blocks) RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD_BACKWARD, MLP_BLOCKS); else if (direct) RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD_BACKWARD, MLP_DIRECT); else if (every) RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD_BACKWARD, MLP_EVERY); else RLT_LAUNCH_MLP_WIDE_PASS(MLP_FORWARD_BACKWARD, MLP_ANY); }
 #undef RLT_LAUNCH_MLP_WIDE_PASS
 #undef RLT_LAUNCH_MLP_WIDE
 #undef RLT_LAUNCH_MLP_WIDE_ROWS

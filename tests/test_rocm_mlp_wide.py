@@ -245,3 +245,33 @@ def test_an_infinite_weight_that_the_activation_saturates_leaves_finite_gradient
     got = run(rocm, dims, params, x, dy, "tanh", False, 0.0)
     assert np.isfinite(ref[1]).all() and np.isfinite(got[1]).all()
     assert rel_err(got[0], ref[0]) <= TOL and rel_err(got[1], ref[1]) <= TOL
+
+
+@pytest.mark.parametrize("B, I", [(1, 1), (3, 16), (5, 33), (1024, 128), (1025, 64), (2047, 17), (2049, 36), (4095, 3)])
+def test_second_layers_of_256_units_wherever_they_lie(oracle, rocm, B, I):
+    """256 units: a second layer on 16 bytes is read as it lies, one that is not from copies. Forward + backward in one call and as calls of their own, tiles of four, eight and sixteen rows, the first
+    layer in one to eight chunks of sixteen columns."""
+    dims = [I, 256, 256, 6]
+    rng = np.random.default_rng(B + I)
+    params = helpers.random_params(rng, dims)
+    x, dy = rng.standard_normal((B, I)).astype(np.float32), rng.standard_normal((B, 6)).astype(np.float32)
+    ref = run(oracle, dims, params, x, dy, "tanh", False, 0.0)
+    for shift in (0, 1):
+        net = Mlp(rocm, dims, params, B, "tanh", "identity")
+        off, nw, _ = net.offsets[1]
+        second = rocm.array(np.concatenate([np.zeros(shift, np.float32), params[off:off + nw]]))
+        net.layers[1].weights = second.offset(shift)
+        xd, yd, dyd = rocm.array(x), rocm.zeros((B, 6)), rocm.array(dy)
+        ws, wsn = net.workspace()
+        for separate in (False, True):
+            rocm.call("mlp_zero_gradient", net.layers, net.n)
+            if separate:
+                rocm.call("mlp_forward", net.layers, net.n, xd.ptr, I, B)
+                rocm.call("mlp_backward", net.layers, net.n, xd.ptr, I, dyd.ptr, 6, None, 0, B, 1, ws, wsn)
+            else:
+                rocm.call("mlp_forward_backward", net.layers, net.n, xd.ptr, I, yd.ptr, 6, dyd.ptr, 6, None, 0, 0.0, B, ws, wsn)
+            rocm.sync()
+            y, grads = (net.out[2] if separate else yd).numpy(), net.grads.numpy()
+            assert rel_err(y, ref[0]) <= TOL, (shift, separate)
+            for off, nw, nb in ref[2]:
+                assert rel_err(grads[off:off + nw], ref[1][off:off + nw]) <= TOL and rel_err(grads[off + nw:off + nw + nb], ref[1][off + nw:off + nw + nb]) <= TOL, (shift, separate, off)
