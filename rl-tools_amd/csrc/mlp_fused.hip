@@ -5,18 +5,21 @@
 // per-layer path of this library) materialises every layer's activations in memory: at batch 65,536 and width 256 that is
 // ~0.4 GB of HBM traffic per call for 27.5 GFLOP, and eleven launches.
 //
-// Here one persistent workgroup per compute unit (4 wavefronts, one per SIMD, up to 512 registers each) walks over tiles of 64
-// batch rows. Per tile, in LDS: h1 and h2 (64 x 256 each, row stride 260), the input rows (64 x 33) and the output gradient
+// Here one persistent workgroup per compute unit (8 wavefronts, two per SIMD, 256 registers each) walks over tiles of 64
+// batch rows. The matrix pipeline bounds it (441 of 549 K cycles for four tiles); what is left are the narrow layers and the
+// element-wise ends of the phases, dependent LDS and memory accesses that the second wavefront of a SIMD hides in part. Four
+// wavefronts of 512 registers took 590 K cycles: a step of 17-256-256-6 (clear, forward + backward, Adam) 282 -> 260 us at 65,536
+// rows, 158.7 -> 143.3 at 20,000; with forward, loss gradient and backward as calls 196.8 -> 171.8 at 20,000, 116 -> 97 at 4,100. Per tile, in LDS: h1 and h2 (64 x 256 each, row stride 260), the input rows (64 x 33) and the output gradient
 // (64 x 17). Per tile, on v_mfma_f32_32x32x2_f32 unless noted:
 //   P1  h1 = act(x W1^T + b1)                       K = in
 //   P2  h2 = act(h1 W2^T + b2)                      K = 256, W2 read from L2 in a pre-swizzled layout, one dwordx4 per 4 k-steps
-//   P3  y = act(h2 W3^T + b3), d_pre3               16x16x4, wavefront w owns rows [16w, 16w+16)
+//   P3  y = act(h2 W3^T + b3), d_pre3               16x16x4, wavefronts w and w + 4 share rows [16w, 16w+16), half the reduction each
 //   P4  dW3 += d_pre3^T h2                          16x16x4
 //   P5  d_pre2 = (d_pre3 W3) * act'(h2)  in place of h2
 //   P6  dW2 += d_pre2^T h1 ; d_h1 = d_pre2 W2       K = 64 rows / K = 256
 //   P7  d_pre1 = d_h1 * act'(h1)  in place of h1
 //   P8  dW1 += d_pre1^T x
-// The weight-gradient accumulators (256 + 32 + 16 registers per lane) live in registers for the whole launch; at the end every
+// The weight-gradient accumulators (128 + 16 + 8 registers per lane) live in registers for the whole launch; at the end every
 // workgroup writes its partial gradients and a second kernel sums them in a fixed order into the layers' gradients (beta = 1).
 // act' is taken from the layer output, which relu / tanh / fast_tanh / sigmoid / identity allow.
 //
@@ -40,7 +43,7 @@ constexpr int BM = 64;       // batch rows per tile
 constexpr int HS = HID + 4;  // LDS row stride of h1 / h2: 16 bytes of each of sixteen rows side by side fill the 64 banks
 constexpr int XSP = 33;      // LDS row stride of the input rows (in <= 32, zero padded)
 constexpr int DS = 17;       // LDS row stride of the output-gradient rows (out <= 16, zero padded)
-constexpr int THREADS = 256;
+constexpr int THREADS = 512;   // two wavefronts per SIMD, 32 columns of every hidden layer each
 constexpr int MAX_WORKGROUPS = 256;
 constexpr int LDS_FLOATS = 2 * BM * HS + BM * XSP + BM * DS + 16 * HS;   // h1, h2, input rows, output-gradient rows, W3 (zero padded to 16 rows)
 
@@ -115,54 +118,54 @@ __global__ void mlp3_prepare_kernel(const float* __restrict__ W1, const float* _
     }
 }
 
-// 64 x 64 block of  A[64 x 256] (LDS, row stride HS) times a pre-swizzled 256 x 256 weight: wavefront w owns column tiles 2w, 2w+1.
-// The LDS operands of k-step s+1 and the weight group two ahead are requested before the matrix instructions of step s are issued.
-__device__ __forceinline__ void contract_256(lptr a, const float* __restrict__ wsw, int w, int lane, floatx16 (&acc)[2][2]) {
+// 64 x 32 block of  A[64 x 256] (LDS, row stride HS) times a pre-swizzled 256 x 256 weight: wavefront w owns column tile w.
+// The LDS operands of k-step s+1 and the weight group two ahead are requested before the matrix instructions of step s are issued, the first
+// two groups (request_weights) before the phase in front.
+struct WeightGroups { const floatx4* p; floatx4 b, n; };
+__device__ __forceinline__ void request_weights(const float* __restrict__ wsw, int w, int lane, WeightGroups& W) {
+    W.p = reinterpret_cast<const floatx4*>(wsw) + (size_t)w * 32 * 64 + lane;
+    W.b = W.p[0]; W.n = W.p[64];
+    __builtin_amdgcn_sched_barrier(0);
+}
+__device__ __forceinline__ void contract_256(lptr a, const WeightGroups& W, int lane, floatx16 (&acc)[2]) {
     const int c32 = lane & 31, hi = lane >> 5;
-    const floatx4* b0p = reinterpret_cast<const floatx4*>(wsw) + (size_t)(2 * w) * 32 * 64 + lane;
-    const floatx4* b1p = b0p + 32 * 64;
+    const floatx4* const bp = W.p;
     const lptr a0 = a + c32 * HS + hi, a1 = a0 + 32 * HS;
-    floatx4 b0 = b0p[0], b1 = b1p[0];
-    floatx4 n0 = b0p[64], n1 = b1p[64];
+    floatx4 b = W.b, n = W.n;
     float x0 = a0[0], x1 = a1[0];
 #pragma unroll       // fully unrolled: the rotation of the prefetch registers becomes renaming instead of copies that wait for the loads
     for (int g = 0; g < 32; g++) {
         const int gp = g + 2 < 32 ? g + 2 : 31;      // two groups ahead; the last iterations re-read the final group
-        const floatx4 p0 = b0p[gp * 64], p1 = b1p[gp * 64];
-        __builtin_amdgcn_sched_barrier(0);      // the requests above are not to be moved down to their first use
+        const floatx4 p = bp[gp * 64];
+        __builtin_amdgcn_sched_barrier(0);      // the request above is not to be moved down to its first use
 #pragma unroll
         for (int t = 0; t < 4; t++) {
             const int next = 4 * g + t + 1 < 128 ? 4 * g + t + 1 : 127;
             const float y0 = a0[2 * next], y1 = a1[2 * next];
-            acc[0][0] = mfma32(x0, b0[t], acc[0][0]);
-            acc[0][1] = mfma32(x0, b1[t], acc[0][1]);
-            acc[1][0] = mfma32(x1, b0[t], acc[1][0]);
-            acc[1][1] = mfma32(x1, b1[t], acc[1][1]);
+            acc[0] = mfma32(x0, b[t], acc[0]);
+            acc[1] = mfma32(x1, b[t], acc[1]);
             x0 = y0; x1 = y1;
         }
-        b0 = n0; b1 = n1; n0 = p0; n1 = p1;
+        b = n; n = p;
     }
 }
 
 template <int MODE>
-__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) void mlp3_fused_kernel(Mlp3Args A) {
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void mlp3_fused_kernel(Mlp3Args A) {
     const lptr h1 = (lptr)rlt_mlp3_lds, h2 = h1 + BM * HS, xs = h2 + BM * HS, dp3 = xs + BM * XSP, w3l = dp3 + BM * DS;
     const int lane_invariant = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nk1 = (A.in + 1) >> 1, nk3 = (A.out + 1) >> 1;
     const floatx16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
-    floatx16 aW2[2][8], aW1[2];
-    floatx4 aW3[4];
+    floatx16 aW2[2][4], aW1 = zero16;      // dW2: row tiles 2(w & 3) and the next, column tiles 4(w >> 2) and the three next; dW1: row tile w; dW3: columns [32w, 32w + 32)
+    floatx4 aW3[2] = {zero4, zero4};
 #pragma unroll
-    for (int a = 0; a < 2; a++) { aW1[a] = zero16;
+    for (int a = 0; a < 2; a++)
 #pragma unroll
-        for (int b = 0; b < 8; b++) aW2[a][b] = zero16; }
-#pragma unroll
-    for (int t = 0; t < 4; t++) aW3[t] = zero4;
+        for (int b = 0; b < 4; b++) aW2[a][b] = zero16;
     // bias gradients: each lane's share of its columns, formed where the values are in registers anyway and added up across the lanes at the end of the launch
-    float db1[2] = {0.f, 0.f}, db2[2] = {0.f, 0.f}, db3[4] = {0.f, 0.f, 0.f, 0.f};
-    const float bias1[2] = {A.b1[32 * (2 * w) + (lane_invariant & 31)], A.b1[32 * (2 * w + 1) + (lane_invariant & 31)]};
-    const float bias2[2] = {A.b2[32 * (2 * w) + (lane_invariant & 31)], A.b2[32 * (2 * w + 1) + (lane_invariant & 31)]};
+    float db1 = 0.f, db2 = 0.f, db3[2] = {0.f, 0.f};
+    const float bias1 = A.b1[32 * w + (lane_invariant & 31)], bias2 = A.b2[32 * w + (lane_invariant & 31)];
     const float bias3 = (lane_invariant & 15) < A.out ? A.b3[lane_invariant & 15] : 0.f;
 
 #ifdef RLT_MLP3_PROFILE      // build-time profiling aid: shader clock cycles workgroup 0 spends in each phase, printed at the end
@@ -171,62 +174,66 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
 #else
 #define RLT_TICK(i)
 #endif
-    // W3 into LDS once (rows beyond out stay zero)
-    for (int idx = threadIdx.x; idx < 16 * HS; idx += THREADS) { const int n = idx / HS, k = idx - n * HS; w3l[idx] = (n < A.out && k < HID) ? A.W3[n * HID + k] : 0.f; }
+    float w3v[16 * HID / THREADS];
+#pragma unroll
+    for (int u = 0; u < 16 * HID / THREADS; u++) w3v[u] = A.W3[min(u * THREADS + (int)threadIdx.x, A.out * HID - 1)];
     // input rows and upstream gradient (or target) rows of a tile travel through registers: requested a whole tile ahead
-    // four threads per row: thread t covers columns (t & 3) + 4u of row t >> 2
-    constexpr int NX = 8, ND = 4;
+    // eight threads per row: thread t covers columns (t & 7) + 8u of row t >> 3
+    constexpr int NX = 4, ND = 2;
     float vx[NX], vd[ND];
     const float* dsrc = MODE == MODE_FORWARD ? A.x : (A.target ? A.target : A.d_output); const int ldsrc = A.target ? A.ldt : A.ldd;
     auto request_tile = [&](int tile, int tid) {
-        const int row = tid >> 2, c0 = tid & 3, grow = tile * BM + row;
+        const int row = tid >> 3, c0 = tid & 7, grow = tile * BM + row;
         const bool row_ok = grow < A.batch;
         const float* xr = A.x + (size_t)(row_ok ? grow : 0) * A.ldx;
         const float* dr = dsrc + (size_t)(row_ok ? grow : 0) * ldsrc;
 #pragma unroll
-        for (int u = 0; u < NX; u++) { const int c = c0 + 4 * u; const bool ok = row_ok && c < A.in; const float v = xr[ok ? c : 0]; vx[u] = ok ? v : 0.f; }
+        for (int u = 0; u < NX; u++) { const int c = c0 + 8 * u; const bool ok = row_ok && c < A.in; const float v = xr[ok ? c : 0]; vx[u] = ok ? v : 0.f; }
         if (MODE != MODE_FORWARD) {
 #pragma unroll
-            for (int u = 0; u < ND; u++) { const int c = c0 + 4 * u; const bool ok = row_ok && c < A.out; const float v = dr[ok ? c : 0]; vd[u] = ok ? v : 0.f; }
+            for (int u = 0; u < ND; u++) { const int c = c0 + 8 * u; const bool ok = row_ok && c < A.out; const float v = dr[ok ? c : 0]; vd[u] = ok ? v : 0.f; }
         }
     };
     request_tile(blockIdx.x, threadIdx.x);
+    // layer-1 weight fragments: requested in the last phase of the tile before
+    float wf[16];
+    auto request_fragments = [&](int lane) {
+#pragma unroll
+        for (int j = 0; j < 16; j++) wf[j] = A.w1s[(w * 16 + j) * 64 + lane];
+    };
+    if (MODE != MODE_BACKWARD) request_fragments(lane_invariant);
+    __builtin_amdgcn_sched_barrier(0);
+    // W3 into LDS once (rows beyond out stay zero)
+#pragma unroll
+    for (int u = 0; u < 16 * HID / THREADS; u++) { const int n = (u * THREADS + (int)threadIdx.x) >> 8, k = threadIdx.x & (HID - 1); w3l[n * HS + k] = n < A.out ? w3v[u] : 0.f; }
     int lane = lane_invariant;
     for (int tile = blockIdx.x; tile < A.n_tiles; tile += gridDim.x) {
         // per-lane addresses derive from a lane index the optimiser cannot see through, or it hoists them all out of this loop and spills them
         asm volatile("" : "+v"(lane));
         const int tid = (w << 6) | lane, c32 = lane & 31, hi = lane >> 5, r16 = lane & 15, q = lane >> 4;
         const int r0 = tile * BM;
-        // ---- P0: this tile's rows into LDS (zero padded), the next tile's requested; layer-1 weight fragments requested
+        // ---- P0: this tile's rows into LDS (zero padded), the next tile's requested
 #pragma unroll
-        for (int u = 0; u < NX; u++) xs[(tid >> 2) * XSP + (tid & 3) + 4 * u] = vx[u];
+        for (int u = 0; u < NX; u++) xs[(tid >> 3) * XSP + (tid & 7) + 8 * u] = vx[u];
         if (MODE != MODE_FORWARD) {
 #pragma unroll
-            for (int u = 0; u < ND; u++) { dp3[(tid >> 2) * DS + (tid & 3) + 4 * u] = vd[u]; if (MODE == MODE_BACKWARD) db3[u] += vd[u]; }
-        }
-        float wf[2][16];
-        if (MODE != MODE_BACKWARD) {
-#pragma unroll
-            for (int a = 0; a < 2; a++)
-#pragma unroll
-                for (int j = 0; j < 16; j++) wf[a][j] = A.w1s[((2 * w + a) * 16 + j) * 64 + lane];
+            for (int u = 0; u < ND; u++) { dp3[(tid >> 3) * DS + (tid & 7) + 8 * u] = vd[u]; if (MODE == MODE_BACKWARD) db3[u] += vd[u]; }
         }
         if (MODE == MODE_BACKWARD) {
             // the outputs of layers 1 and 2 of this tile, as forward() left them in memory, into LDS (rows beyond the batch as zeros)
 #pragma unroll 1
             for (int half = 0; half < 2; half++) {
                 const float* src = A.act_out[half]; const lptr dst = half ? h2 : h1;
-#pragma unroll
-                for (int i0 = 0; i0 < 16; i0 += 8) {
+                {
                     floatx4 v[8];
 #pragma unroll
                     for (int i = 0; i < 8; i++) {
-                        const int idx = tid + THREADS * (i0 + i), row = idx >> 6, grow = r0 + row;
+                        const int idx = tid + THREADS * i, row = idx >> 6, grow = r0 + row;
                         v[i] = reinterpret_cast<const floatx4*>(src + (size_t)(grow < A.batch ? grow : 0) * HID)[idx & 63];
                     }
 #pragma unroll
                     for (int i = 0; i < 8; i++) {
-                        const int idx = tid + THREADS * (i0 + i), row = idx >> 6, c4 = (idx & 63) * 4;
+                        const int idx = tid + THREADS * i, row = idx >> 6, c4 = (idx & 63) * 4;
                         const bool ok = r0 + row < A.batch;
 #pragma unroll
                         for (int e = 0; e < 4; e++) if (!ok) v[i][e] = 0.f;
@@ -238,66 +245,69 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
         if (tile + (int)gridDim.x < A.n_tiles) request_tile(tile + gridDim.x, tid);
         rlt_lds_barrier();
         RLT_TICK(0)
-        // ---- P1: h1 = act(x W1^T + b1); wavefront w owns columns [64w, 64w+64)
+        // ---- P1: h1 = act(x W1^T + b1); wavefront w owns columns [32w, 32w+32)
+        WeightGroups weights;
         if (MODE != MODE_BACKWARD) {
-#pragma unroll
-        for (int a = 0; a < 2; a++) {
-            const int nt = 2 * w + a;
             floatx16 acc[2] = {zero16, zero16};
+            request_weights(A.w2f, w, lane, weights);
             steps_dispatch(nk1, [&](auto steps) { constexpr int NK = decltype(steps)::value;
                 float xa[2][NK];
 #pragma unroll
                 for (int j = 0; j < NK; j++) { xa[0][j] = xs[c32 * XSP + 2 * j + hi]; xa[1][j] = xs[(32 + c32) * XSP + 2 * j + hi]; }
 #pragma unroll
-                for (int j = 0; j < NK; j++) { acc[0] = mfma32(xa[0][j], wf[a][j], acc[0]); acc[1] = mfma32(xa[1][j], wf[a][j], acc[1]); }
+                for (int j = 0; j < NK; j++) { acc[0] = mfma32(xa[0][j], wf[j], acc[0]); acc[1] = mfma32(xa[1][j], wf[j], acc[1]); }
             });
             act_dispatch(A.act1, [&](auto kind) { constexpr int ACT = decltype(kind)::value;
 #pragma unroll
             for (int mt = 0; mt < 2; mt++)
 #pragma unroll
                 for (int v = 0; v < 16; v++) {
-                    const float pre = acc[mt][v] + bias1[a], o = act_c<ACT>(pre);
-                    h1[(32 * mt + row32(v, hi)) * HS + 32 * nt + c32] = o;
+                    const float pre = acc[mt][v] + bias1, o = act_c<ACT>(pre);
+                    h1[(32 * mt + row32(v, hi)) * HS + 32 * w + c32] = o;
                     if (MODE == MODE_FORWARD) {
                         const int grow = r0 + 32 * mt + row32(v, hi);
-                        if (grow < A.batch) { if (A.act_pre[0]) A.act_pre[0][(size_t)grow * HID + 32 * nt + c32] = pre; if (A.act_out[0]) A.act_out[0][(size_t)grow * HID + 32 * nt + c32] = o; }
+                        if (grow < A.batch) { if (A.act_pre[0]) A.act_pre[0][(size_t)grow * HID + 32 * w + c32] = pre; if (A.act_out[0]) A.act_out[0][(size_t)grow * HID + 32 * w + c32] = o; }
                     }
                 }
             });
-        }
-        rlt_lds_barrier();
+            rlt_lds_barrier();
         }
         RLT_TICK(1)
         // ---- P2: h2 = act(h1 W2^T + b2)
+        float raw[4];      // upstream gradient or target of the rows and column whose output this lane finishes: the halves of the sums pass through their place
         if (MODE != MODE_BACKWARD) {
-            floatx16 acc[2][2] = {{zero16, zero16}, {zero16, zero16}};
-            contract_256(h1, A.w2f, w, lane, acc);
+            floatx16 acc[2] = {zero16, zero16};
+            contract_256(h1, weights, lane, acc);
             act_dispatch(A.act2, [&](auto kind) { constexpr int ACT = decltype(kind)::value;
 #pragma unroll
             for (int mt = 0; mt < 2; mt++)
 #pragma unroll
-                for (int a = 0; a < 2; a++)
-#pragma unroll
-                    for (int v = 0; v < 16; v++) {
-                        const float pre = acc[mt][a][v] + bias2[a], o = act_c<ACT>(pre);
-                        h2[(32 * mt + row32(v, hi)) * HS + 32 * (2 * w + a) + c32] = o;
-                        if (MODE == MODE_FORWARD) {
-                            const int grow = r0 + 32 * mt + row32(v, hi);
-                            if (grow < A.batch) { if (A.act_pre[1]) A.act_pre[1][(size_t)grow * HID + 32 * (2 * w + a) + c32] = pre; if (A.act_out[1]) A.act_out[1][(size_t)grow * HID + 32 * (2 * w + a) + c32] = o; }
-                        }
+                for (int v = 0; v < 16; v++) {
+                    const float pre = acc[mt][v] + bias2, o = act_c<ACT>(pre);
+                    h2[(32 * mt + row32(v, hi)) * HS + 32 * w + c32] = o;
+                    if (MODE == MODE_FORWARD) {
+                        const int grow = r0 + 32 * mt + row32(v, hi);
+                        if (grow < A.batch) { if (A.act_pre[1]) A.act_pre[1][(size_t)grow * HID + 32 * w + c32] = pre; if (A.act_out[1]) A.act_out[1][(size_t)grow * HID + 32 * w + c32] = o; }
                     }
+                }
             });
+            if (MODE == MODE_FUSED) {
+#pragma unroll
+                for (int v = 0; v < 4; v++) raw[v] = dp3[(16 * (w & 3) + 4 * q + v) * DS + r16];
+            }
             rlt_lds_barrier();
         }
         RLT_TICK(2)
-        // ---- P3: y = act(h2 W3^T + b3) for rows [16w, 16w+16) (lane group q takes the reduction range [64q, 64q+64)), then d_pre3
+        // ---- P3: y = act(h2 W3^T + b3) for rows [16(w & 3), 16(w & 3) + 16), wavefronts 0 to 3 the first half of the reduction, 4 to 7 the second (lane group q 32 of its
+        // 128), then d_pre3 by wavefronts 0 to 3
         // (BACKWARD is handed d_pre3 itself: the caller has applied the output activation's derivative, as dense backward does in place)
         if (MODE != MODE_BACKWARD) {
             floatx4 acc = zero4, acc2 = zero4;
-            const lptr wp = w3l + r16 * HS + 64 * q;
-            const lptr ap = h2 + (16 * w + r16) * HS + 64 * q;
+            const int k0 = 128 * (w >> 2) + 32 * q, rows = 16 * (w & 3);
+            const lptr wp = w3l + r16 * HS + k0;
+            const lptr ap = h2 + (rows + r16) * HS + k0;
 #pragma unroll
-            for (int u = 0; u < 64; u += 4) {
+            for (int u = 0; u < 32; u += 4) {
                 const floatx4 av = *(lptr4)(ap + u), wv = *(lptr4)(wp + u);
                 acc = mfma16(av[0], wv[0], acc);
                 acc2 = mfma16(av[1], wv[1], acc2);
@@ -305,68 +315,72 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
                 acc2 = mfma16(av[3], wv[3], acc2);
             }
             acc += acc2;
-            float column = 0.f;
+            if (w >= 4) {
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int row = 16 * w + 4 * q + v, grow = r0 + row;
-                const bool ok = r16 < A.out && grow < A.batch;
-                const float pre = acc[v] + bias3, yv = rlt_act(pre, A.act3);
-                if (ok && A.y) A.y[(size_t)grow * A.ldy + r16] = yv;
-                if (MODE == MODE_FORWARD) {
-                    if (ok && A.act_pre[2]) A.act_pre[2][(size_t)grow * A.out + r16] = pre;
-                } else {
-                    const float raw = dp3[row * DS + r16];
-                    float d = A.target ? (yv - raw) * A.mse_scale : raw;
-                    d *= rlt_dact_from_output(yv, A.act3);
-                    d = ok ? d : 0.f;
-                    dp3[row * DS + r16] = d;
-                    column += d;
-                }
+                for (int v = 0; v < 4; v++) dp3[(rows + 4 * q + v) * DS + r16] = acc[v];
             }
-            if (MODE == MODE_FUSED) db3[0] += column;
+            rlt_lds_barrier();
+            if (w < 4) {
+                float column = 0.f;
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int row = rows + 4 * q + v, grow = r0 + row;
+                    const bool ok = r16 < A.out && grow < A.batch;
+                    const float pre = (acc[v] + dp3[row * DS + r16]) + bias3, yv = rlt_act(pre, A.act3);
+                    if (ok && A.y) A.y[(size_t)grow * A.ldy + r16] = yv;
+                    if (MODE == MODE_FORWARD) {
+                        if (ok && A.act_pre[2]) A.act_pre[2][(size_t)grow * A.out + r16] = pre;
+                    } else {
+                        float d = A.target ? (yv - raw[v]) * A.mse_scale : raw[v];
+                        d *= rlt_dact_from_output(yv, A.act3);
+                        d = ok ? d : 0.f;
+                        dp3[row * DS + r16] = d;
+                        column += d;
+                    }
+                }
+                if (MODE == MODE_FUSED) db3[0] += column;
+            }
             rlt_lds_barrier();
         }
         RLT_TICK(3)
-        if (MODE == MODE_FORWARD) continue;
-        // ---- P4: dW3 += d_pre3^T h2 (rows = outputs, wavefront w owns columns [64w, 64w+64)); the operands of the next four rows requested before these rows' matrix instructions
+        if (MODE == MODE_FORWARD) { request_fragments(lane); continue; }
+        // ---- P4: dW3 += d_pre3^T h2 (rows = outputs, wavefront w owns columns [32w, 32w+32)); the operands of the next four rows requested before these rows' matrix instructions
         {
-            const lptr dp = dp3 + q * DS + r16, hp = h2 + q * HS + 64 * w + r16;
-            float a = dp[0], b[4];
+            const lptr dp = dp3 + q * DS + r16, hp = h2 + q * HS + 32 * w + r16;
+            float a = dp[0], b[2];
 #pragma unroll
-            for (int t = 0; t < 4; t++) b[t] = hp[16 * t];
+            for (int t = 0; t < 2; t++) b[t] = hp[16 * t];
 #pragma unroll
             for (int j = 0; j < 16; j++) {
                 const int next = j + 1 < 16 ? j + 1 : j;
                 const float na = dp[4 * next * DS];
-                float nb[4];
+                float nb[2];
 #pragma unroll
-                for (int t = 0; t < 4; t++) nb[t] = hp[4 * next * HS + 16 * t];
+                for (int t = 0; t < 2; t++) nb[t] = hp[4 * next * HS + 16 * t];
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int t = 0; t < 4; t++) aW3[t] = mfma16(a, b[t], aW3[t]);
+                for (int t = 0; t < 2; t++) aW3[t] = mfma16(a, b[t], aW3[t]);
                 a = na;
 #pragma unroll
-                for (int t = 0; t < 4; t++) b[t] = nb[t];
+                for (int t = 0; t < 2; t++) b[t] = nb[t];
             }
         }
-        rlt_lds_barrier();
         RLT_TICK(4)
         // ---- P5: d_pre2 = (d_pre3 W3) * act'(h2), in place of h2
-#pragma unroll
-        for (int a = 0; a < 2; a++) {
-            const int nt = 2 * w + a;
+        {
             floatx16 acc[2] = {zero16, zero16}, hv[2];      // the outputs that the derivative is taken from travel while the products are formed
 #pragma unroll
             for (int mt = 0; mt < 2; mt++)
 #pragma unroll
-                for (int v = 0; v < 16; v++) hv[mt][v] = h2[(32 * mt + row32(v, hi)) * HS + 32 * nt + c32];
+                for (int v = 0; v < 16; v++) hv[mt][v] = h2[(32 * mt + row32(v, hi)) * HS + 32 * w + c32];
             steps_dispatch(nk3, [&](auto steps) { constexpr int NK = decltype(steps)::value < 8 ? decltype(steps)::value : 8;
                 float da[2][NK], wb[NK];
 #pragma unroll
-                for (int j = 0; j < NK; j++) { wb[j] = w3l[(2 * j + hi) * HS + 32 * nt + c32]; da[0][j] = dp3[c32 * DS + 2 * j + hi]; da[1][j] = dp3[(32 + c32) * DS + 2 * j + hi]; }
+                for (int j = 0; j < NK; j++) { wb[j] = w3l[(2 * j + hi) * HS + 32 * w + c32]; da[0][j] = dp3[c32 * DS + 2 * j + hi]; da[1][j] = dp3[(32 + c32) * DS + 2 * j + hi]; }
 #pragma unroll
                 for (int j = 0; j < NK; j++) { acc[0] = mfma32(da[0][j], wb[j], acc[0]); acc[1] = mfma32(da[1][j], wb[j], acc[1]); }
             });
+            rlt_lds_barrier();      // every wavefront is done reading h2 for P4
             float column = 0.f;
             act_dispatch(A.act2, [&](auto kind) { constexpr int ACT = decltype(kind)::value;
 #pragma unroll
@@ -374,80 +388,77 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
 #pragma unroll
                     for (int v = 0; v < 16; v++) {
                         const float d = acc[mt][v] * dact_c<ACT>(hv[mt][v]);
-                        h2[(32 * mt + row32(v, hi)) * HS + 32 * nt + c32] = d;
+                        h2[(32 * mt + row32(v, hi)) * HS + 32 * w + c32] = d;
                         column += d;
                     }
             });
-            db2[a] += column;
+            db2 += column;
         }
         rlt_lds_barrier();
         RLT_TICK(5)
-        // ---- P6: dW2 += d_pre2^T h1 (wavefront w owns row tiles 2w, 2w+1 of it); d_h1 = d_pre2 W2
+        // ---- P6: dW2 += d_pre2^T h1 (wavefront w owns row tiles 2(w & 3), 2(w & 3) + 1 and four column tiles of it); d_h1 = d_pre2 W2
         {
-            const lptr dbase = h2 + hi * HS + c32 + 32 * (2 * w), hbase = h1 + hi * HS + c32;
-            float a0 = dbase[0], a1 = dbase[32], bv[8];
+            request_weights(A.w2b, w, lane, weights);
+            const lptr dbase = h2 + hi * HS + c32 + 64 * (w & 3), hbase = h1 + hi * HS + c32 + 128 * (w >> 2);
+            float a0 = dbase[0], a1 = dbase[32], bv[4];
 #pragma unroll
-            for (int b = 0; b < 8; b++) bv[b] = hbase[32 * b];
-#pragma unroll 2
+            for (int b = 0; b < 4; b++) bv[b] = hbase[32 * b];
+#pragma unroll 4
             for (int k = 0; k < BM / 2; k++) {
                 const int kn = k + 1 < BM / 2 ? k + 1 : k;       // operands of the next row pair, requested before this pair's matrix instructions
                 const float na0 = dbase[2 * kn * HS], na1 = dbase[2 * kn * HS + 32];
-                float nb[8];
+                float nb[4];
 #pragma unroll
-                for (int b = 0; b < 8; b++) nb[b] = hbase[2 * kn * HS + 32 * b];
+                for (int b = 0; b < 4; b++) nb[b] = hbase[2 * kn * HS + 32 * b];
 #pragma unroll
-                for (int b = 0; b < 8; b++) {
+                for (int b = 0; b < 4; b++) {
                     aW2[0][b] = mfma32(a0, bv[b], aW2[0][b]);
                     aW2[1][b] = mfma32(a1, bv[b], aW2[1][b]);
                 }
                 a0 = na0; a1 = na1;
 #pragma unroll
-                for (int b = 0; b < 8; b++) bv[b] = nb[b];
+                for (int b = 0; b < 4; b++) bv[b] = nb[b];
             }
         }
         {
-            floatx16 acc[2][2] = {{zero16, zero16}, {zero16, zero16}};
-            contract_256(h2, A.w2b, w, lane, acc);
-            rlt_lds_barrier();      // every wavefront is done reading h1
+            floatx16 acc[2] = {zero16, zero16};
+            contract_256(h2, weights, lane, acc);
             RLT_TICK(6)
             // ---- P7: d_pre1 = d_h1 * act'(h1), in place of h1
+            rlt_lds_barrier();      // every wavefront is done reading h1
             act_dispatch(A.act1, [&](auto kind) { constexpr int ACT = decltype(kind)::value;
-#pragma unroll
-            for (int a = 0; a < 2; a++) {
                 float column = 0.f;
 #pragma unroll
                 for (int mt = 0; mt < 2; mt++) {
                     float hv[16];
 #pragma unroll
-                    for (int v = 0; v < 16; v++) hv[v] = h1[(32 * mt + row32(v, hi)) * HS + 32 * (2 * w + a) + c32];
+                    for (int v = 0; v < 16; v++) hv[v] = h1[(32 * mt + row32(v, hi)) * HS + 32 * w + c32];
 #pragma unroll
                     for (int v = 0; v < 16; v++) {
-                        const float d = acc[mt][a][v] * dact_c<ACT>(hv[v]);
-                        h1[(32 * mt + row32(v, hi)) * HS + 32 * (2 * w + a) + c32] = d;
+                        const float d = acc[mt][v] * dact_c<ACT>(hv[v]);
+                        h1[(32 * mt + row32(v, hi)) * HS + 32 * w + c32] = d;
                         column += d;
                     }
                 }
-                db1[a] += column;
-            }
+                db1 += column;
             });
         }
         rlt_lds_barrier();
         RLT_TICK(7)
         // ---- P8: dW1 += d_pre1^T x, two row pairs at a time, the operands of the next two requested before these ones' matrix instructions
         {
-            const lptr xp = xs + hi * XSP + c32, dp = h1 + hi * HS + c32 + 32 * (2 * w);
-            float x0 = xp[0], x1 = xp[2 * XSP], d0[2] = {dp[0], dp[32]}, d1[2] = {dp[2 * HS], dp[2 * HS + 32]};
+            if (MODE == MODE_FUSED) request_fragments(lane);
+            const lptr xp = xs + hi * XSP + c32, dp = h1 + hi * HS + c32 + 32 * w;
+            float x0 = xp[0], x1 = xp[2 * XSP], d0 = dp[0], d1 = dp[2 * HS];
 #pragma unroll 4
             for (int k = 0; k < BM / 2; k += 2) {
                 const int next = k + 2 < BM / 2 ? k + 2 : k;
                 const float nx0 = xp[2 * next * XSP], nx1 = xp[2 * (next + 1) * XSP];
-                const float nd0[2] = {dp[2 * next * HS], dp[2 * next * HS + 32]}, nd1[2] = {dp[2 * (next + 1) * HS], dp[2 * (next + 1) * HS + 32]};
+                const float nd0 = dp[2 * next * HS], nd1 = dp[2 * (next + 1) * HS];
                 __builtin_amdgcn_sched_barrier(0);
-                aW1[0] = mfma32(d0[0], x0, aW1[0]); aW1[1] = mfma32(d0[1], x0, aW1[1]);
-                aW1[0] = mfma32(d1[0], x1, aW1[0]); aW1[1] = mfma32(d1[1], x1, aW1[1]);
-                x0 = nx0; x1 = nx1;
-#pragma unroll
-                for (int a = 0; a < 2; a++) { d0[a] = nd0[a]; d1[a] = nd1[a]; }
+                aW1 = mfma32(d0, x0, aW1);
+                aW1 = mfma32(d1, x1, aW1);
+                x0 = nx0; x1 = nx1; d0 = nd0; d1 = nd1;
             }
         }
         rlt_lds_barrier();
@@ -460,29 +471,25 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
     float* P = A.partial + (size_t)blockIdx.x * ((count + 63) & ~63);      // blocks start on 256-byte boundaries: a wavefront's 256-byte load or store touches two 128-byte lines, not three
     float* pW1 = P; float* pb1 = pW1 + HID * A.in; float* pW2 = pb1 + HID; float* pb2 = pW2 + HID * HID; float* pW3 = pb2 + HID; float* pb3 = pW3 + A.out * HID;
 #pragma unroll
+    for (int v = 0; v < 16; v++) if (c32 < A.in) pW1[(32 * w + row32(v, hi)) * A.in + c32] = aW1[v];
+#pragma unroll
     for (int a = 0; a < 2; a++)
 #pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int o = 32 * (2 * w + a) + row32(v, hi);
-            if (c32 < A.in) pW1[o * A.in + c32] = aW1[a][v];
+        for (int v = 0; v < 16; v++)
 #pragma unroll
-            for (int b = 0; b < 8; b++) pW2[o * HID + 32 * b + c32] = aW2[a][b][v];
-        }
+            for (int b = 0; b < 4; b++) pW2[(32 * (2 * (w & 3) + a) + row32(v, hi)) * HID + 32 * (4 * (w >> 2) + b) + c32] = aW2[a][b][v];
 #pragma unroll
-    for (int t = 0; t < 4; t++)
+    for (int t = 0; t < 2; t++)
 #pragma unroll
-        for (int v = 0; v < 4; v++) { const int o = 4 * q + v; if (o < A.out) pW3[o * HID + 64 * w + 16 * t + r16] = aW3[t][v]; }
-    // the two halves of a wavefront hold the same columns' sums over different rows; the last layer's are spread over every thread
-#pragma unroll
-    for (int a = 0; a < 2; a++) {
-        const float s1 = db1[a] + __shfl_xor(db1[a], 32, 64), s2 = db2[a] + __shfl_xor(db2[a], 32, 64);
-        if (hi == 0) { pb1[32 * (2 * w + a) + c32] = s1; pb2[32 * (2 * w + a) + c32] = s2; }
-    }
+        for (int v = 0; v < 4; v++) { const int o = 4 * q + v; if (o < A.out) pW3[o * HID + 32 * w + 16 * t + r16] = aW3[t][v]; }
+    // the two halves of a wavefront hold the same columns' sums over different rows; the last layer's are spread over wavefronts 0 to 3, or every thread
+    const float s1 = db1 + __shfl_xor(db1, 32, 64), s2 = db2 + __shfl_xor(db2, 32, 64);
+    if (hi == 0) { pb1[32 * w + c32] = s1; pb2[32 * w + c32] = s2; }
     constexpr int SHARES = MODE == MODE_BACKWARD ? BM : 16;      // per column: one per row of a tile, or one per sixteen lanes
     if (MODE == MODE_BACKWARD) {
 #pragma unroll
-        for (int u = 0; u < ND; u++) dp3[(tid >> 2) * DS + (tid & 3) + 4 * u] = db3[u];
-    } else dp3[(4 * w + q) * DS + r16] = db3[0];
+        for (int u = 0; u < ND; u++) dp3[(tid >> 3) * DS + (tid & 7) + 8 * u] = db3[u];
+    } else if (w < 4) dp3[(4 * w + q) * DS + r16] = db3[0];
     rlt_lds_barrier();
     if (tid < A.out) {
         float s[4] = {0.f, 0.f, 0.f, 0.f};
