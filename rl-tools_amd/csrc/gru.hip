@@ -6,7 +6,7 @@
 //   * W_i x + b_i for ALL steps is one contraction over sequence*batch rows (gemm.hip), written straight into post_activation (at hidden width 64 and up to a thousand rows mostly
 //     formed beside the recurrence, inputs_beside);
 //   * the recurrence runs in ONE launch: batch rows are independent, so no grid-wide synchronisation is needed. At hidden width 64 a
-//     workgroup carries four rows through the sequence on the matrix cores, at 16 and 32 a wavefront 64 / width rows, both with W_h in registers; at other widths a workgroup owns a few
+//     workgroup carries four rows through the sequence on the matrix cores or, up to two rows per compute unit, one row on the vector units, at 16 and 32 a wavefront 64 / width rows, both with W_h in registers; at other widths a workgroup owns a few
 //     rows and keeps W_h and its rows' hidden state in LDS;
 //   * backward does the same in reverse and stores, per step, the gradient at the gate pre-activations (one copy as the input path sees
 //     it, one as the hidden path sees it, which differs in the n gate by the factor r) and the previous hidden state; the weight
@@ -326,6 +326,7 @@ __device__ __forceinline__ float corrected_rcp(float d) {      // 1 / d for d >=
 __device__ __forceinline__ float hw_sigmoid(float x) { return corrected_rcp(1.0f + __expf(-x)); }
 __device__ __forceinline__ float hw_tanh(float x) { return fmaf(-2.0f, corrected_rcp(__expf(2.0f * x) + 1.0f), 1.0f); }
 typedef float gru_floatx4 __attribute__((ext_vector_type(4)));
+typedef float gru_float4_a4 __attribute__((ext_vector_type(4), aligned(4)));      // four floats wherever they lie: rows of W_i start at any multiple of four bytes
 constexpr int GM_ROWS = 4;
 template <int ABID> __device__ __forceinline__ gru_floatx4 mfma4(float a, float b, gru_floatx4 c) { return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 2, ABID, 0); }
 // The four quarters of the reduction added up: c[row] of a lane in group kg (lanes 16 kg ...) is row `row`'s sum over quarter kg; the result is row kg's sum over all of them
@@ -408,7 +409,6 @@ __global__ __launch_bounds__(256, 2) void gru_forward_mfma_kernel(GruArgs A) {
 // with 146 inputs, 0.69 with 3. The recurrence goes first (s_setprio); a second barrier per step that kept the others' products out of the recurrence's made it slower (64.5 -> 66.6 us).
 // Launch of the input gates + recurrence / this, 64 steps, 1,024 rows: 146 inputs 77.5 / 65.5 us, 64 inputs 61.1 / 49.0, 3 inputs 57.8 / 44.0.
 constexpr int GP_INPUTS = 160, GP_THREADS = 512, GP_LDX = 164, GP_LDG = 3 * 64 + 16, GP_STEP = GM_ROWS * GP_LDG + 16;      // inputs at most; row strides in LDS: eight lanes' 16-byte reads and sixteen lanes' words of four rows meet no bank twice
-typedef float gru_float4_a4 __attribute__((ext_vector_type(4), aligned(4)));      // four floats wherever they lie: rows of W_i start at any multiple of four bytes
 template <int GROUPS, bool FAST>      // GROUPS: sixteens of inputs, zeros behind the last
 __global__ __launch_bounds__(GP_THREADS) void gru_forward_inputs_kernel(GruArgs A) {
     constexpr int H = 64, D = 4, E = (GM_ROWS * 16 * GROUPS + 255) / 256, TURNS = GROUPS;      // E: floats of a step that a thread stages; TURNS: reduction steps (of four inputs) between two steps of the recurrence
@@ -615,6 +615,227 @@ __global__ __launch_bounds__(256, WAVES) void gru_backward_mfma_kernel(GruArgs A
         });
     }
     if (A.db_hn_partial) gru_at(A.db_hn_partial + (size_t)b0 * H, at) = db_hn;
+}
+
+// ---- hidden width 64, a workgroup per row (row_groups_forward, row_groups_backward) ----------------------------------------------
+// With few rows most compute units are idle on the kernels above, and a step of one row on the vector units is the shorter chain: the matrix instruction forms four rows in
+// 384 cycles whether they are there or not, the vector unit one row in 192. Wavefronts 0 to 3 carry the recurrence: four lanes share a hidden unit, the parts of the reduction meet in exchanges
+// within four (eight) lanes. What bounds them is the number of instructions that one wavefront issues per step (about five cycles each), so wavefronts 4 to 7 do the rest beside them: they request
+// what the steps read (D steps ahead), hand it over through LDS a step ahead and store what the steps leave there a step later. One workgroup barrier per step.
+// 64 steps at batch 64, four rows to a workgroup on the matrix cores / a row: forward recurrence 35.9 / 23 us, backward 33.2 / 25.5 (without wavefronts 4 to 7 25 and 29.9).
+constexpr int GR_THREADS = 512;
+__device__ __forceinline__ float quad_xor1(float v) { return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true)); }
+__device__ __forceinline__ float quad_xor2(float v) { return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xF, 0xF, true)); }
+__device__ __forceinline__ float quad_low(float v) { return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x44, 0xF, 0xF, true)); }        // lanes 0, 1, 0, 1 of the four
+__device__ __forceinline__ float quad_high(float v) { return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xEE, 0xF, 0xF, true)); }       // lanes 2, 3, 2, 3
+__device__ __forceinline__ float half_mirror(float v) { return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x141, 0xF, 0xF, true)); }    // lane 7 - i of the eight
+__device__ __forceinline__ float row_half(float v) { return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x128, 0xF, 0xF, true)); }       // lane i ^ 8 of the sixteen
+__device__ __forceinline__ float masked(float v, float mask) { return __int_as_float(__float_as_int(v) & __float_as_int(mask)); }
+// steps 0 ... S - 1, their parity a constant
+template <class F> __device__ __forceinline__ void gru_by_parity(int S, F&& step) {
+    int t = 0;
+    for (; t + 2 <= S; t += 2) { step(std::integral_constant<int, 0>{}); step(std::integral_constant<int, 1>{}); }
+    if (t < S) step(std::integral_constant<int, 0>{});
+}
+// Lane (unit, kq): quarter kq of the reduction, summed in the order of the kernel on the matrix cores; lanes 0 and 1 of the four finish r, 2 and 3 z.
+template <bool FAST>
+__global__ __launch_bounds__(GR_THREADS, 4) void gru_forward_row_kernel(GruArgs A) {
+    constexpr int H = 64, D = 4;
+    __shared__ __align__(16) float hs[2][H];                  // the previous state, by the parity of the step
+    __shared__ __align__(16) float given[2][2][4 * H];        // r (z) gate's input part, n gate's, and the state that follows: (output & third) | fourth
+    __shared__ float left[2][5 * H];                          // r, n, z, the n gate's hidden part, the output
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), b = blockIdx.x;
+    const size_t stride = (size_t)A.B * H;
+    if (w >= 4) {
+        const int role = w - 4, u = lane, gate = role < 3 ? role : 0;      // r, z, n gate; the resets and the other two outputs
+        float* in = A.L.post_activation + (size_t)b * 3 * H + gate * H;
+        float* to = role < 3 ? in : A.L.n_pre_pre_activation + (size_t)b * H;
+        float* out = A.L.output + (size_t)b * H;
+        const size_t step = role < 3 ? 3 * stride : stride;
+        const int from = (role == 0 ? 0 : role == 1 ? 2 : role == 2 ? 1 : 3) * H + u;
+        const unsigned at = u * sizeof(float);
+        const float bias = role < 2 ? A.L.biases_hidden[role * H + u] : 0.f, h0 = A.L.initial_hidden_state[u];
+        auto request = [&](int t, float& v) { v = gru_at(in, at); in += t + 1 < A.S ? 3 * stride : 0; };      // the last steps request the last one again: no branch around the loads
+        auto give = [&](int parity, float v, bool reset) {
+            if (role < 2) given[parity][role][4 * u] = v + bias;
+            else if (role == 2) { given[parity][0][4 * u + 1] = v; given[parity][1][4 * u + 1] = v; }
+            else {
+                const float keep = __int_as_float(reset ? 0 : -1), instead = reset ? h0 : 0.f;
+#pragma unroll
+                for (int g = 0; g < 2; g++) { given[parity][g][4 * u + 2] = keep; given[parity][g][4 * u + 3] = instead; }
+            }
+        };
+        auto store = [&](int parity) {
+            gru_at(to, at) = left[parity][from]; to += step;
+            if (role == 3) { gru_at(out, at) = left[parity][4 * H + u]; out += stride; }
+        };
+        float q[D];
+#pragma unroll
+        for (int d = 0; d < D; d++) if (d < A.S) request(d, q[d]);
+        uint64_t flags = gru_reset_flags<1>(A.reset, 1, A.S, A.B, b, 0);      // lowest bit: the step after the one that is handed over starts an episode
+        give(0, q[0], flags & 1);
+        rlt_lds_barrier();
+        for (int first = 0; first < A.S; first += 64) {
+            const uint64_t later = gru_reset_flags<1>(A.reset, first + 65, A.S, A.B, b, 0);      // of the steps after these
+            gru_steps<D>(min(64, A.S - first), [&](auto number, int i) {
+                constexpr int N = decltype(number)::value;
+                __builtin_amdgcn_sched_barrier(0);
+                flags = i + 1 < 64 ? flags >> 1 : later;
+                give((N + 1) & 1, q[(N + 1) % D], flags & 1);
+                request(first + i + D, q[N]);
+                if (first + i > 0) store((N + 1) & 1);
+                rlt_lds_barrier();
+            });
+        }
+        store((A.S - 1) & 1);
+        return;
+    }
+    const int kq = lane & 3, u = 16 * w + (lane >> 2);
+    const bool is_z = kq & 2, odd = kq & 1;
+    float wb[3][16];
+#pragma unroll
+    for (int g = 0; g < 3; g++) {
+        const float4* src = reinterpret_cast<const float4*>(A.L.weights_hidden + (size_t)(g * H + u) * H + 16 * kq);
+#pragma unroll
+        for (int q = 0; q < 4; q++) { const float4 v = src[q]; wb[g][4 * q] = v.x; wb[g][4 * q + 1] = v.y; wb[g][4 * q + 2] = v.z; wb[g][4 * q + 3] = v.w; }
+    }
+    const float bhn = A.L.biases_hidden[2 * H + u];
+    float h = A.L.initial_hidden_state[u];
+    hs[0][u] = h;
+    __builtin_amdgcn_s_setprio(1);
+    rlt_lds_barrier();
+    gru_by_parity(A.S, [&](auto parity) {
+        constexpr int P = decltype(parity)::value;
+        gru_floatx4 a[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) a[k] = reinterpret_cast<const gru_floatx4*>(&hs[P][16 * kq])[k];
+        const gru_floatx4 x = *reinterpret_cast<const gru_floatx4*>(&given[P][kq >> 1][4 * u]);
+        __builtin_amdgcn_sched_barrier(0);      // all reads are under way before the first product
+        float cr = 0.f, cz = 0.f, cn = 0.f;
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) { cr = fmaf(a[k][j], wb[0][4 * k + j], cr); cz = fmaf(a[k][j], wb[1][4 * k + j], cz); cn = fmaf(a[k][j], wb[2][4 * k + j], cn); }
+        float c = (is_z ? cz : cr) + quad_xor2(is_z ? cr : cz);
+        cn += quad_xor2(cn);
+        c += quad_xor1(c); cn += quad_xor1(cn);
+        const float ac = x[0] + c, an = bhn + cn;
+        const float gate = FAST ? gate_sigmoid(ac, 1) : hw_sigmoid(ac), r = quad_low(gate), z = quad_high(gate);
+        const float n = FAST ? gate_tanh(x[1] + an * r, 1) : hw_tanh(x[1] + an * r);
+        const float o = (1.0f - z) * n + z * h;
+        h = __int_as_float((__float_as_int(o) & __float_as_int(x[2])) | __float_as_int(x[3]));
+        hs[P ^ 1][u] = h;
+        left[P][kq * H + u] = odd ? is_z ? an : n : gate;
+        left[P][4 * H + u] = o;
+        rlt_lds_barrier();
+    });
+}
+// Reverse pass: lane (four units, sixteenth kq of the 64 units of each gate) forms the four units' sums over its 12 gate gradients (three 16-byte reads: with two units to a lane and six reads LDS,
+// which serves a wavefront's in eight cycles each, was the longer chain), the sixteenths meet in four exchanges, the first two of which leave a unit to each four lanes. Every gate gradient is the gradient at the state times a factor of saved values, which the wavefronts beside the recurrence form.
+__global__ __launch_bounds__(GR_THREADS, 2) void gru_backward_row_kernel(GruArgs A) {
+    constexpr int H = 64, D = 4;
+    __shared__ __align__(16) float gs[2][4 * H];               // gradients at the r, z and n gate as the hidden path sees them, and at the state
+    __shared__ float factor[2][4 * H];                         // of these, by the gradient at the state
+    __shared__ __align__(16) float given[2][4 * H];            // gradient at the output, mask of what the step before hands on, z gate
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), b = blockIdx.x, S = A.S;
+    const size_t stride = (size_t)A.B * H, last = (size_t)(S - 1) * stride + (size_t)b * H;
+    if (w >= 4) {
+        const int role = w - 4, u = lane;      // r, z, n gate, state
+        const unsigned at = u * sizeof(float);
+        const float h0 = A.L.initial_hidden_state[u];
+        struct Saved { float z, n, first, second; };      // r gate: r, npp; z: -, state before; n: r, -; state: gradient at the output, state before (what is not named is read and not used)
+        const bool from_gates = role != 3, from_state = role != 0;
+        float *post = A.L.post_activation + 3 * last, *first_from = from_gates ? post : A.d_output + last;
+        float* second_from = role == 0 ? A.L.n_pre_pre_activation + last : A.L.output + last - (S > 1 ? stride : 0);      // (the state before the first step is not used)
+        const size_t first_step = from_gates ? 3 * stride : stride;
+        auto request = [&](int i, Saved& v) {      // i-th step from the end; steps before the first read the first again
+            v.z = gru_at(post + H, at); v.n = gru_at(post + 2 * H, at); v.first = gru_at(first_from, at); v.second = gru_at(second_from, at);
+            const bool on = i + 1 < S;
+            post -= on ? 3 * stride : 0; first_from -= on ? first_step : 0; second_from -= on && (!from_state || i + 2 < S) ? stride : 0;
+        };
+        Saved q[D];
+#pragma unroll
+        for (int d = 0; d < D; d++) if (d < S) request(d, q[d]);
+        struct Kept { float n, hp; bool counts; } now, next;      // what the stores of a step need
+        bool carried = false;      // the step before hands a gradient on
+        auto give = [&](int parity, const Saved& v, int i, uint64_t flags) {
+            const bool first = i + 1 >= S, from_initial = first || (flags >> 63);
+            const float over = 1.0f - v.z, n = over * (1.0f - v.n * v.n), hp = from_initial ? h0 : v.second;
+            if (role == 0) factor[parity][u] = n * v.second * v.first * (1.0f - v.first);
+            else if (role == 1) factor[parity][H + u] = (hp - v.n) * v.z * over;
+            else if (role == 2) factor[parity][2 * H + u] = n * v.first;
+            else { const gru_floatx4 g = {v.first, __int_as_float(carried ? -1 : 0), v.z, 0.f}; *reinterpret_cast<gru_floatx4*>(&given[parity][4 * u]) = g; }
+            carried = !from_initial;
+            next.n = n; next.hp = hp; next.counts = first || !from_initial;      // the reference drops reset samples (t > 0) from the b_hn gradient (their buffer rows are zeroed before that sum, :716-749)
+        };
+        float *to_input = A.buffer_input + 3 * last + (role < 2 ? role : 2) * H, *to_hidden = role < 3 ? A.buffer_hidden + 3 * last + role * H : A.h_previous + last, *to_dy = A.d_output + last;
+        const size_t hidden_step = role < 3 ? 3 * stride : stride;
+        float db_hn = 0.f;
+        auto store = [&](int parity) {
+            const float g = gs[parity][role * H + u];
+            if (role < 2) gru_at(to_input, at) = g;
+            else if (role == 3) { gru_at(to_input, at) = g * now.n; gru_at(to_dy, at) = g; }
+            else db_hn += now.counts ? g : 0.f;
+            gru_at(to_hidden, at) = role < 3 ? g : now.hp;
+            to_input -= 3 * stride; to_hidden -= hidden_step; to_dy -= stride;
+        };
+        if (role == 3) { factor[0][3 * H + u] = 1.f; factor[1][3 * H + u] = 1.f; }
+        uint64_t flags = gru_reset_flags<1>(A.reset, max(S - 64, 0), S, A.B, b, 0) << (64 - min(64, S));      // the highest bit: the step that is handed over, t = S - 1 - i
+        __builtin_amdgcn_s_waitcnt(0x0F70);      // vmcnt(0)
+        give(0, q[0], 0, flags);
+        rlt_lds_barrier();
+        for (int back = 0; back < S; back += 64) {
+            const int steps = min(64, S - back), rest = S - back - 64;
+            const uint64_t later = rest > 0 ? gru_reset_flags<1>(A.reset, max(rest - 64, 0), rest, A.B, b, 0) << (64 - min(64, rest)) : 0;      // of the steps after these
+            gru_steps<D>(steps, [&](auto number, int i) {
+                constexpr int N = decltype(number)::value;
+                __builtin_amdgcn_sched_barrier(0);
+                if (back + i > 0) store((N + 1) & 1);      // of the step before
+                now = next;
+                flags = i + 1 < 64 ? flags << 1 : later;
+                give((N + 1) & 1, q[(N + 1) % D], back + i + 1, flags);
+                request(back + i + D, q[N]);
+                rlt_lds_barrier();
+            });
+        }
+        store((S - 1) & 1);
+        if (role == 2 && A.db_hn_partial) gru_at(A.db_hn_partial + (size_t)b * H, at) = db_hn;
+        return;
+    }
+    const int kq = lane & 15, u0 = 16 * w + 4 * (lane >> 4), u = 16 * w + (lane >> 2), place = (lane & 3) * H + u;
+    const bool upper8 = lane & 8, upper4 = lane & 4;
+    gru_floatx4 wb[12];
+#pragma unroll
+    for (int g = 0; g < 3; g++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) wb[4 * g + k] = *reinterpret_cast<const gru_float4_a4*>(A.L.weights_hidden + (size_t)(g * H + 4 * kq + k) * H + u0);
+    __builtin_amdgcn_s_setprio(1);
+    rlt_lds_barrier();
+    float f = factor[0][place], carry = 0.f;
+    gru_floatx4 x = *reinterpret_cast<const gru_floatx4*>(&given[0][4 * u]);
+    gru_by_parity(S, [&](auto parity) {
+        constexpr int P = decltype(parity)::value;
+        const float dh = x[0] + masked(carry, x[1]), z = x[2];
+        gs[P][place] = dh * f;
+        rlt_lds_barrier();
+        gru_floatx4 v[3];
+#pragma unroll
+        for (int g = 0; g < 3; g++) v[g] = *reinterpret_cast<const gru_floatx4*>(&gs[P][g * H + 4 * kq]);
+        f = factor[P ^ 1][place];
+        x = *reinterpret_cast<const gru_floatx4*>(&given[P ^ 1][4 * u]);
+        __builtin_amdgcn_sched_barrier(0);      // all reads are under way before the first product
+        float c[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int g = 0; g < 3; g++)
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+#pragma unroll
+                for (int a = 0; a < 4; a++) c[a] = fmaf(v[g][k], wb[4 * g + k][a], c[a]);
+        const float c0 = (upper8 ? c[2] : c[0]) + row_half(upper8 ? c[0] : c[2]), c1 = (upper8 ? c[3] : c[1]) + row_half(upper8 ? c[1] : c[3]);
+        float sum = (upper4 ? c1 : c0) + half_mirror(upper4 ? c0 : c1);
+        sum += quad_xor2(sum); sum += quad_xor1(sum);
+        carry = dh * z + sum;
+    });
 }
 
 // The same with the weight gradients formed beside the recurrence instead of by five launches after it that read every step's gate gradients and states back: batches of at most one
@@ -995,6 +1216,11 @@ bool layer_ok(const rlt_gru_layer* L) {
 }
 int compute_units(const rlt_rocm_device* device) { return device->compute_units > 0 ? device->compute_units : 256; }
 bool one_group_per_unit(const rlt_rocm_device* device, const rlt_gru_layer* L, int B) { return L->hidden_dim == 64 && rlt_div_up(B, GM_ROWS) <= compute_units(device); }
+// Where the recurrence at width 64 takes a workgroup per row (with input gates and weight gradients as launches of their own). us of the calls, four rows to a workgroup / a row, 64 steps:
+// forward, 3 inputs 64 rows 41.0 / 28.3, 256 rows 50.0 / 37.4, 512 rows 53.4 / 44.5, 600 rows (three rounds of rows) 53.9 / 55.1; 8 steps 512 rows 13.4 / 13.3; 1 step 64 rows 8.0 / 7.2;
+// backward to the input 64 rows 33.2 / 25.5, 256 rows 34.1 / 26.7, 512 rows 34.4 / 33.0; 16 steps 64 rows 10.2 / 8.8, 512 rows 11.6 / 13.0; 1 step 3.85 / 4.0.
+bool rows_forward(const rlt_rocm_device* device, int B) { return B <= 2 * compute_units(device); }
+bool rows_backward(const rlt_rocm_device* device, int S, int B) { return B <= compute_units(device) && S >= 4; }
 bool overlap(const float* a, size_t n, const float* b, size_t m) { return (uintptr_t)a < (uintptr_t)(b + m) && (uintptr_t)b < (uintptr_t)(a + n); }
 int even_sixteens(int columns) { return 2 * rlt_div_up(columns, 32); }
 // Where the input gates / the weight gradients are formed beside the recurrence. The fp32 matrix instructions and the vector unit of a SIMD take turns, so that what goes beside the
@@ -1004,6 +1230,9 @@ int even_sixteens(int columns) { return 2 * rlt_div_up(columns, 32); }
 //   146 inputs 16 steps   16 rows 19.0 / 20.2, 256 rows 22.3 / 21.1; 64 steps 512 rows 62.6 / 64.8, 1,024 rows 77.5 / 65.3; 1 step 64 rows 11.5 / 8.3
 //   128 inputs 13 steps   64 rows 15.8 / 17.8; 20 steps 16 rows 19.2 / 22.3; 24 steps 400 rows 31.1 / 27.0
 //    64 inputs 16 steps   16 rows 15.8 / 14.9; 32 steps 16 rows 23.5 / 24.8, 256 rows 27.9 / 26.2; 64 steps 256 rows 49.0 / 46.3; 20 inputs 64 steps 16 rows 40.4 / 39.1, 1,024 rows 60.8 / 42.0
+// Up to two rows per compute unit the recurrence of its own is the faster one (rows_forward; the figures above are with four rows to a workgroup): 3 inputs 16 steps 64 rows 12.8 / 13.3, 64 steps 256 rows
+// 37.4 / 41.4, 512 rows 44.4 / 42.5; 146 inputs 8 steps 64 rows 13.4 / 13.0, 16 steps 256 rows 18.9 / 20.9. Over 528 shapes (1 to 128 steps, 16 to 512 rows, 3 to 160 inputs) the side that the
+// rule takes is 0.4 % above the faster one on average, and nowhere more than 3 % slower than the one taken before a workgroup per row.
 // Backward (54 ns a step and 46 per sixteen inputs), us, launches / beside, 64 steps:
 //   146 inputs 256 rows 61.6 / 78.0, 512 rows 81.1 / 80.0, 1,024 rows 132.7 / 85.7; 64 inputs 256 rows 52.5 / 58.6, 512 rows 64.3 / 60.2; 3 inputs 64 rows 47.5 / 50.6, 1,024 rows 79.1 / 55.3;
 //   146 inputs 1,024 rows 24 steps 57.7 / 44.0
@@ -1013,13 +1242,15 @@ bool inputs_beside(const rlt_rocm_device* device, const rlt_gru_layer* L, const 
     const size_t rows = (size_t)S * B, inputs = rows * L->input_dim;
     if (overlap(input, inputs, L->output, rows * 64) || overlap(input, inputs, L->n_pre_pre_activation, rows * 64) || overlap(input, inputs, L->post_activation, rows * 3 * 64)) return false;
     const int I = L->input_dim;
+    const int units = compute_units(device);
+    const double by_row = B <= units ? 280.0 * S - 2000.0 : rows_forward(device, B) ? 70.0 * S - 500.0 : 0.0;      // what the recurrence of its own has from a workgroup per row
     const bool by_rows = I > 32 && I % 2 == 0 && rows >= 2048;      // the launch in front is rows_forward_kernel (rlt_gemm_rows_forward)
     const double launch = by_rows ? 3750.0 : I <= 32 ? 5800.0 : I % 4 == 0 ? 2400.0 : I % 2 == 0 ? 2600.0 : 3200.0;
-    return (by_rows ? 27.2 : 23.8) * 4 * rlt_div_up(S, 4) * even_sixteens(I) <= launch + ((by_rows ? 0.143 : 0.185) + 0.0017 * I) * rows;
+    return (by_rows ? 27.2 : 23.8) * 4 * rlt_div_up(S, 4) * even_sixteens(I) + by_row <= launch + ((by_rows ? 0.143 : 0.185) + 0.0017 * I) * rows;
 }
 bool weights_beside(const rlt_rocm_device* device, const rlt_gru_layer* L, int S, int B, size_t room) {      // room: bytes of the caller's workspace that nothing else is kept in
     if (!one_group_per_unit(device, L, B) || L->input_dim > GW_INPUTS || rlt_div_up(B, GM_ROWS) * gru_gradient_block(L->input_dim) * sizeof(float) > room) return false;
-    return S * (54.0 + 46.0 * even_sixteens(L->input_dim)) <= 3400.0 + (0.35 + 0.0037 * L->input_dim) * S * B;
+    return S * (54.0 + 46.0 * even_sixteens(L->input_dim)) + (rows_backward(device, S, B) ? 80.0 * S - 1500.0 : 0.0) <= 3400.0 + (0.35 + 0.0037 * L->input_dim) * S * B;
 }
 // The weight gradients of gru_gradients_kernel: pairs of column tiles, shares of the rows (workgroups for the whole chip, but at least eight steps of four rows to a wavefront; once, twice ... so many that no sum is longer than
 // 256 steps, for its error's sake), blocks of sums
@@ -1092,7 +1323,8 @@ int rlt_rocm_gru_forward(rlt_rocm_device* device, const rlt_gru_layer* L, const 
         const bool fast = L->fast_tanh != 0;      // a template parameter: as a run-time switch inside the step it cost 10% at width 64
         if (H == 64) {
             const dim3 grid4(rlt_div_up(B, GM_ROWS));
-            if (fast) hipLaunchKernelGGL(gru_forward_mfma_kernel<true>, grid4, block, 0, device->stream, a); else hipLaunchKernelGGL(gru_forward_mfma_kernel<false>, grid4, block, 0, device->stream, a);
+            if (rows_forward(device, B)) { if (fast) hipLaunchKernelGGL(gru_forward_row_kernel<true>, dim3(B), dim3(GR_THREADS), 0, device->stream, a); else hipLaunchKernelGGL(gru_forward_row_kernel<false>, dim3(B), dim3(GR_THREADS), 0, device->stream, a); }
+            else if (fast) hipLaunchKernelGGL(gru_forward_mfma_kernel<true>, grid4, block, 0, device->stream, a); else hipLaunchKernelGGL(gru_forward_mfma_kernel<false>, grid4, block, 0, device->stream, a);
         }
         else if (H == 32) { if (fast) hipLaunchKernelGGL((gru_forward_reg_kernel<32, true>), grid, block, 0, device->stream, a); else hipLaunchKernelGGL((gru_forward_reg_kernel<32, false>), grid, block, 0, device->stream, a); }
         else { if (fast) hipLaunchKernelGGL((gru_forward_reg_kernel<16, true>), grid, block, 0, device->stream, a); else hipLaunchKernelGGL((gru_forward_reg_kernel<16, false>), grid, block, 0, device->stream, a); }
@@ -1134,7 +1366,8 @@ int rlt_rocm_gru_backward(rlt_rocm_device* device, const rlt_gru_layer* L, const
         if (H == 64) {
             const dim3 grid4(rlt_div_up(B, GM_ROWS));
             const int units = compute_units(device);
-            if (backward_by_rows(units, S, B)) hipLaunchKernelGGL(gru_backward_rows_kernel, grid4, block, 0, device->stream, a);
+            if (rows_backward(device, S, B)) hipLaunchKernelGGL(gru_backward_row_kernel, dim3(B), dim3(GR_THREADS), 0, device->stream, a);
+            else if (backward_by_rows(units, S, B)) hipLaunchKernelGGL(gru_backward_rows_kernel, grid4, block, 0, device->stream, a);
             else if ((int)grid4.x > 3 * units) hipLaunchKernelGGL((gru_backward_mfma_kernel<2, 4>), grid4, block, 0, device->stream, a);
             else hipLaunchKernelGGL((gru_backward_mfma_kernel<4, 2>), grid4, block, 0, device->stream, a);
         }

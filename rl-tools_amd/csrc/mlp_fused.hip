@@ -9,8 +9,9 @@
 // batch rows. The matrix pipeline bounds it (441 of 549 K cycles for four tiles); what is left are the narrow layers and the
 // element-wise ends of the phases, dependent LDS and memory accesses that the second wavefront of a SIMD hides in part. Four
 // wavefronts of 512 registers took 590 K cycles: a step of 17-256-256-6 (clear, forward + backward, Adam) 282 -> 260 us at 65,536
-// rows, 158.7 -> 143.3 at 20,000; with forward, loss gradient and backward as calls 196.8 -> 171.8 at 20,000, 116 -> 97 at 4,100. Per tile, in LDS: h1 and h2 (64 x 256 each, row stride 260), the input rows (64 x 33) and the output gradient
-// (64 x 17). Per tile, on v_mfma_f32_32x32x2_f32 unless noted:
+// rows, 158.7 -> 143.3 at 20,000; with forward, loss gradient and backward as calls 196.8 -> 171.8 at 20,000, 116 -> 97 at 4,100.
+// Per tile, in LDS: h1 and h2 (64 x 256 each, row stride 260), the input rows (64 x 33) and the output gradient (64 x 17).
+// Per tile, on v_mfma_f32_32x32x2_f32 unless noted:
 //   P1  h1 = act(x W1^T + b1)                       K = in
 //   P2  h2 = act(h1 W2^T + b2)                      K = 256, W2 read from L2 in a pre-swizzled layout, one dwordx4 per 4 k-steps
 //   P3  y = act(h2 W3^T + b3), d_pre3               16x16x4, wavefronts w and w + 4 share rows [16w, 16w+16), half the reduction each

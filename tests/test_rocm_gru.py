@@ -153,6 +153,26 @@ def test_gru_at_the_edges_of_the_kernels_that_keep_a_layer_in_registers(oracle, 
         assert rel_err(got[k], want[k]) <= 2e-5, (k, rel_err(got[k], want[k]))
 
 
+@pytest.mark.parametrize("fast_tanh", [False, True])
+@pytest.mark.parametrize("case", [(1, 1), (2, 3), (3, 2), (4, 5), (5, 256), (5, 257), (4, 512), (4, 513), (63, 2), (64, 3), (65, 1), (66, 2), (128, 1), (129, 2)])
+def test_gru_with_a_workgroup_per_row(oracle, rocm, case, fast_tanh):
+    """Width 64 over at most 512 rows (backward 256, from four steps on) with more inputs than the kernels beside the recurrence take: steps around the groups of four and the 64 whose reset
+    flags are read at once, with resets and without, the last batches of a row per workgroup and the first of four. Tolerance as for the long batch above."""
+    print("case", case, fast_tanh, flush=True)
+    S, B = case
+    for with_reset in (False, True):
+        params, x, dy, reset = helpers.gru_random_case(np.random.default_rng(39 + S + B), S, B, 161, 64, with_reset)
+        results = []
+        for b in (oracle, rocm):
+            g = helpers.GruOnBackend(b, S, B, 161, 64, params, fast_tanh=fast_tanh)
+            g.forward(x, reset)
+            g.backward(dy)
+            b.sync()
+            results.append(g.results())
+        for k in KEYS:
+            assert rel_err(results[1][k], results[0][k]) <= 2e-5, (k, rel_err(results[1][k], results[0][k]))
+
+
 @pytest.mark.parametrize("want_d_input", [False, True])
 @pytest.mark.parametrize("case", [(1, 1, 1), (2, 3, 15), (3, 5, 16), (4, 4, 17), (5, 2, 31), (22, 4, 146), (23, 4, 146), (40, 6, 146), (65, 7, 145), (130, 9, 158), (66, 6, 159), (71, 5, 160),
                                   (70, 3, 161), (24, 1021, 40), (24, 1024, 33), (24, 1025, 33), (24, 1022, 146), (25, 1023, 159), (25, 1023, 160), (26, 1024, 161), (25, 998, 130), (27, 1001, 100), (64, 40, 64), (64, 129, 64)])
