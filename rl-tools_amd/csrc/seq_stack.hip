@@ -10,8 +10,8 @@
 // Bound: the instructions of a recurrence's step. A wavefront is alone on its SIMD and issues one instruction every four to five cycles whatever it is (vector, scalar,
 // wait), so a step takes its instruction count: about 115 at width 32, 48 of them the products. Hence the forms below: values exchanged between lanes instead of through
 // LDS, the r gate in one half of the lanes while z is in the other, stores and LDS writes by all lanes of a unit rather than under an exec mask, addresses moved on
-// instead of formed, loops unrolled to the slots' parity. Per step of a whole pass, 100 sequences of 100 steps: 0.43 us at width 32 (0.41 backward, 0.48 with the values
-// that the weight gradients need stored), 0.30 and 0.38 at width 16; a launch per layer with a row per 32 lanes took 0.59 us per step at width 32 and 0.45 at 16, one
+// instead of formed, loops unrolled to the slots' parity. The training set of 100 sequences of 100 steps (actor of width 16, critics of width 32) has four forward launches of 38.4 us on average and
+// three backward launches of 37.4; a launch per layer with a row per 32 lanes took 0.59 us per step at width 32 and 0.45 at 16, one
 // layer after the other, plus launches for the dense layers, projections and gradients.
 #include "seq_stack.h"
 #include "gemm.h"
@@ -59,11 +59,32 @@ template <bool FAST> __device__ __forceinline__ float gate_tanh(float x) { retur
 // tests/test_dpp_wait_states.py looks the built instructions over.)
 __device__ __forceinline__ void wait_for_dpp(float& x) { asm volatile("s_nop 1" : "+v"(x)); }
 __device__ __forceinline__ void wait_for_dpp(float& x, float& y, float& z) { asm volatile("s_nop 1" : "+v"(x), "+v"(y), "+v"(z)); }
-template <int K> __device__ __forceinline__ void broadcast_fma(float& acc, float x, float w) {
-    if (K < 0) return;
-    asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(x), "v"(w), "n"(K < 0 ? 0 : K));
+// Several to a statement: the compiler separates statements that hand a register on by an idle instruction, whatever they hold (sixteen of them for 48 products: the training set of 100
+// sequences of 100 steps 364 -> 354 us).
+#define RLT_BCAST(op, acc, x, w, k) "v_" op "_f32_dpp %" #acc ", %" #x ", %" #w " row_newbcast:" #k " row_mask:0xf bank_mask:0xf\n\t"
+#define RLT_BCAST3(op, w0, w1, w2, k) RLT_BCAST(op, 0, 3, w0, k) RLT_BCAST(op, 1, 4, w1, k) RLT_BCAST(op, 2, 5, w2, k)
+#define RLT_WEIGHTS8(w, k) "v"(w[k]), "v"(w[k + 1]), "v"(w[k + 2]), "v"(w[k + 3]), "v"(w[k + 4]), "v"(w[k + 5]), "v"(w[k + 6]), "v"(w[k + 7])
+// acc[i] = the products of x, y, z with sixteen weights each
+__device__ __forceinline__ void broadcast_products(float (&acc)[3], float x, float y, float z, const float (&a)[16], const float (&b)[16], const float (&c)[16]) {
+    asm(RLT_BCAST3("mul", 6, 14, 22, 0) RLT_BCAST3("fmac", 7, 15, 23, 1) RLT_BCAST3("fmac", 8, 16, 24, 2) RLT_BCAST3("fmac", 9, 17, 25, 3)
+        RLT_BCAST3("fmac", 10, 18, 26, 4) RLT_BCAST3("fmac", 11, 19, 27, 5) RLT_BCAST3("fmac", 12, 20, 28, 6) RLT_BCAST3("fmac", 13, 21, 29, 7)
+        : "=&v"(acc[0]), "=&v"(acc[1]), "=&v"(acc[2]) : "v"(x), "v"(y), "v"(z), RLT_WEIGHTS8(a, 0), RLT_WEIGHTS8(b, 0), RLT_WEIGHTS8(c, 0));
+    asm(RLT_BCAST3("fmac", 6, 14, 22, 8) RLT_BCAST3("fmac", 7, 15, 23, 9) RLT_BCAST3("fmac", 8, 16, 24, 10) RLT_BCAST3("fmac", 9, 17, 25, 11)
+        RLT_BCAST3("fmac", 10, 18, 26, 12) RLT_BCAST3("fmac", 11, 19, 27, 13) RLT_BCAST3("fmac", 12, 20, 28, 14) RLT_BCAST3("fmac", 13, 21, 29, 15)
+        : "+&v"(acc[0]), "+&v"(acc[1]), "+&v"(acc[2]) : "v"(x), "v"(y), "v"(z), RLT_WEIGHTS8(a, 8), RLT_WEIGHTS8(b, 8), RLT_WEIGHTS8(c, 8));
 }
-__device__ __forceinline__ float broadcast_first(float x, float w) { float acc; asm("v_mul_f32_dpp %0, %1, %2 row_newbcast:0 row_mask:0xf bank_mask:0xf" : "=v"(acc) : "v"(x), "v"(w)); return acc; }
+// the products of x with sixteen weights, in three sums
+__device__ __forceinline__ void broadcast_products(float (&acc)[3], float x, const float (&a)[16]) {
+#define RLT_BCAST1(op, i, w, k) RLT_BCAST(op, i, 3, w, k)
+    asm(RLT_BCAST1("mul", 0, 4, 0) RLT_BCAST1("mul", 1, 5, 1) RLT_BCAST1("mul", 2, 6, 2) RLT_BCAST1("fmac", 0, 7, 3) RLT_BCAST1("fmac", 1, 8, 4) RLT_BCAST1("fmac", 2, 9, 5)
+        RLT_BCAST1("fmac", 0, 10, 6) RLT_BCAST1("fmac", 1, 11, 7) RLT_BCAST1("fmac", 2, 12, 8) RLT_BCAST1("fmac", 0, 13, 9) RLT_BCAST1("fmac", 1, 14, 10) RLT_BCAST1("fmac", 2, 15, 11)
+        RLT_BCAST1("fmac", 0, 16, 12) RLT_BCAST1("fmac", 1, 17, 13) RLT_BCAST1("fmac", 2, 18, 14) RLT_BCAST1("fmac", 0, 19, 15)
+        : "=&v"(acc[0]), "=&v"(acc[1]), "=&v"(acc[2]) : "v"(x), RLT_WEIGHTS8(a, 0), RLT_WEIGHTS8(a, 8));
+#undef RLT_BCAST1
+}
+#undef RLT_BCAST3
+#undef RLT_BCAST
+#undef RLT_WEIGHTS8
 // a lane's weights of a [3H x H] matrix: width 32: rows (or columns) u of the three blocks, half p of the reduction index; width 16: row (column) u of block p
 template <int H> struct Weights3 { float w[H == 32 ? 3 : 1][16]; };
 template <int H>
@@ -88,16 +109,10 @@ __device__ __forceinline__ void load_columns3(const float* W, int u, int p, Weig
 }
 __device__ __forceinline__ float half_in_rows(float v, int p) { float w = v; swap16(v, w); return p ? w : v; }
 // (x, y, z have passed wait_for_dpp)
-template <int H, int... Q>
-__device__ __forceinline__ void multiply(const Weights3<H>& R, const float& x, const float& y, const float& z, float (&acc)[3], std::integer_sequence<int, Q...>) {
-    if (H == 32) {
-        acc[0] = broadcast_first(x, R.w[0][0]); acc[1] = broadcast_first(y, R.w[H == 32 ? 1 : 0][0]); acc[2] = broadcast_first(z, R.w[H == 32 ? 2 : 0][0]);
-        ((broadcast_fma<Q + 1>(acc[0], x, R.w[0][Q + 1]), broadcast_fma<Q + 1>(acc[1], y, R.w[H == 32 ? 1 : 0][Q + 1]), broadcast_fma<Q + 1>(acc[2], z, R.w[H == 32 ? 2 : 0][Q + 1])), ...);
-    } else {
-        acc[0] = broadcast_first(x, R.w[0][0]); acc[1] = 0.f; acc[2] = 0.f;
-        (broadcast_fma<Q + 1>(acc[(Q + 1) % 3], x, R.w[0][Q + 1]), ...);
-        acc[0] += acc[1] + acc[2];
-    }
+template <int H>
+__device__ __forceinline__ void multiply(const Weights3<H>& R, const float& x, const float& y, const float& z, float (&acc)[3]) {
+    if constexpr (H == 32) broadcast_products(acc, x, y, z, R.w[0], R.w[1], R.w[2]);
+    else { broadcast_products(acc, x, R.w[0]); acc[0] += acc[1] + acc[2]; }
 }
 // The products of a vector (element u in the lanes of unit u) with rows u of the three blocks. rz: the first block's in the lanes with p = 0, the second's where p = 1
 // (width 16: also the third's where p = 2); n: the third's in every lane.
@@ -106,7 +121,7 @@ __device__ __forceinline__ void products3(const Weights3<H>& R, float v, int p, 
     float acc[3];
     float x = H == 32 ? half_in_rows(v, p) : v;
     wait_for_dpp(x);
-    multiply<H>(R, x, x, x, acc, std::make_integer_sequence<int, 15>{});
+    multiply<H>(R, x, x, x, acc);
     if (H == 32) {
         swap32(acc[0], acc[1]);
         rz = acc[0] + acc[1];
@@ -125,27 +140,38 @@ __device__ __forceinline__ float product_sum3(const Weights3<H>& R, float x, flo
     if (H == 32) {
         x = half_in_rows(x, p); y = half_in_rows(y, p); z = half_in_rows(z, p);
         wait_for_dpp(x, y, z);
-        multiply<H>(R, x, y, z, acc, std::make_integer_sequence<int, 15>{});
+        multiply<H>(R, x, y, z, acc);
         return sum_parts<2>(acc[0] + (acc[1] + acc[2]));
     }
     float own = p == 0 ? x : p == 1 ? y : p == 2 ? z : 0.f;      // the fourth row of lanes has zero weights, and zero times an infinity is not zero
     wait_for_dpp(own);
-    multiply<H>(R, own, own, own, acc, std::make_integer_sequence<int, 15>{});
+    multiply<H>(R, own, own, own, acc);
     return sum_parts<4>(acc[0]);
 }
 
 // A stage: `before` ticks until its first step is there, one per step, `after` ticks for the stages behind it. The steps are unrolled U at a time with their number in the
-// group as a constant (slots and queues are indexed by it).
+// group as a constant (slots and queues are indexed by it). Whole groups are straight-line code: with an exit before every step, or a request under a condition, the compiler waits where the paths
+// meet, once in a group, for everything that is under way (100 sequences of 100 steps, with four steps ahead instead of six, whose queue fits 128 registers,
+// 354 -> 341 us a set, 1,000 sequences 1,584 -> 1,480). What was requested before the first step is waited for in front of it,
+// so that a step waits for its own values and not for the last ones.
 template <class F, int... D>
-__device__ __forceinline__ void stage_group(int i, int S, F& step, std::integer_sequence<int, D...>) {
+__device__ __forceinline__ void stage_group(int i, F& step, std::integer_sequence<int, D...>) {
+    ((__builtin_amdgcn_sched_barrier(0), step(std::integral_constant<int, D>{}, i + D), rlt_lds_barrier()), ...);
+}
+template <class F, int... D>
+__device__ __forceinline__ void stage_rest(int i, int S, F& step, std::integer_sequence<int, D...>) {
     ((i + D < S ? (step(std::integral_constant<int, D>{}, i + D), rlt_lds_barrier()) : (void)0), ...);
 }
 template <int U, class F>
 __device__ __forceinline__ void stage(int S, int before, int after, F&& step) {
     for (int k = 0; k < before; k++) rlt_lds_barrier();
-    for (int i = 0; i < S; i += U) stage_group(i, S, step, std::make_integer_sequence<int, U>{});
+    int i = 0;
+    __builtin_amdgcn_s_waitcnt(0x0F70);      // vmcnt(0)
+    for (; i + U <= S; i += U) stage_group(i, step, std::make_integer_sequence<int, U>{});
+    stage_rest(i, S, step, std::make_integer_sequence<int, U - 1>{});
     for (int k = 0; k < after; k++) rlt_lds_barrier();
 }
+template <class F> __device__ __forceinline__ void by_condition(bool condition, F&& body) { if (condition) body(std::true_type{}); else body(std::false_type{}); }
 
 // What a workgroup stages in LDS before its first step: the row's `width` values of S steps (at steps * x_step apart, rows of width4 floats) and its reset flags. request() asks for the first values of
 // every thread without a condition and waits for nothing; store() writes them down, after the stages have asked for their weights: one trip to memory instead of one per value, flag and the weights.
@@ -218,9 +244,12 @@ __device__ __forceinline__ void recurrence(const Forward& P, int layer, int lag,
     stage<2>(P.S, lag, FORWARD_STAGES - 1 - lag, [&](auto d, int t) {
         constexpr int PAR = decltype(d)::value & 1;
         const float x = in[PAR][PARTS == 2 ? p * H + u : min(p, 1) * H + u], xn = in[PAR][2 * H + u];
-        const bool restart = flags[t + 1];      // the next step starts from the initial state (the flags end with one more entry)
+        const uint8_t flag = flags[t + 1];      // the next step starts from the initial state (the flags end with one more entry)
         float rz, n_hidden;
+        __builtin_amdgcn_sched_barrier(0);
         products3<H>(R, h, p, rz, n_hidden);
+        __builtin_amdgcn_sched_barrier(0);      // the three words travel while the products are formed
+        const bool restart = flag;
         const float an = n_hidden + bn, s = gate_sigmoid<FAST>(x + rz);
         float r = s, z = s;
         if (PARTS == 2) swap32(r, z);
@@ -321,7 +350,7 @@ struct Backward {
 };
 struct BackwardLaunch { Backward pass[MAX_PASSES]; int n; };
 template <int H> struct BackwardSlots { float dy2[2][H], g2[2][3 * H], dy1[2][H], g1[2][3 * H], dp0[2][H]; };
-constexpr int AHEAD = 6;      // steps ahead of its use that a saved value is requested (a load takes several steps)
+constexpr int AHEAD = 4;      // steps ahead of its use that a saved value is requested (a load takes several steps)
 
 // A recurrence's way back, step i of S (from the last on). dy: the gradient at its output from the stage above, held in a register from the tick before.
 template <int H, class READY>
@@ -335,11 +364,11 @@ __device__ __forceinline__ void recurrence_back(const Backward& P, int layer, in
     const float* post = G.post + 3 * last + u; const float* npp = G.npp + last + u; const float* state = G.out + last + u;
     struct Saved { float r, z, n, npp, hp; };
     Saved queue[AHEAD];
-    auto request = [&](int i, Saved& v) {      // step i's values; the state is the one before the step (the first step takes the initial one)
-        if (i >= S) return;
-        if (i + 1 < S) state -= stride;
+    auto request = [&](int i, Saved& v) {      // step i's values, beyond the last step the last one's again; the state is the one before the step (the first step takes the initial one)
+        const size_t on = i + 1 < S ? stride : 0;
+        state -= on;
         v.r = post[0]; v.z = post[H]; v.n = post[2 * H]; v.npp = *npp; v.hp = *state;
-        post -= 3 * stride; npp -= stride;
+        post -= 3 * on; npp -= on;
     };
 #pragma unroll
     for (int d = 0; d < AHEAD; d++) request(d, queue[d]);
@@ -349,29 +378,33 @@ __device__ __forceinline__ void recurrence_back(const Backward& P, int layer, in
     ready();
     for (int k = 0; k < lag - 1; k++) rlt_lds_barrier();
     above = dy[0][u];
+    uint8_t flag = flags[0];
     rlt_lds_barrier();
-    stage<AHEAD>(S, 0, BACKWARD_STAGES + 1 - lag, [&](auto d, int i) {
+    by_condition(want_w, [&](auto want) { stage<AHEAD>(S, 0, BACKWARD_STAGES + 1 - lag, [&](auto d, int i) {
         constexpr int N = decltype(d)::value;
         const Saved v = queue[N];
-        request(i + AHEAD, queue[N]);
         const float dh = above + carry;
         above = dy[(N + 1) & 1][u];      // the next step's
-        const bool from_initial = flags[i];
+        const bool from_initial = flag;
+        flag = flags[min(i + 1, S - 1)];
         const float hp = from_initial ? h0 : v.hp, t = dh * (1.0f - v.z);
         const float gz = t * (hp - v.n) * v.z;
         const float gn = t * (1.0f - v.n * v.n);
         const float gr = gn * v.npp * v.r * (1.0f - v.r);
         const float gnr = gn * v.r;
+        float through = dh * v.z;
+        asm volatile("" : "+v"(through));      // (not formed below by a multiply-add that would keep the entry's z)
+        request(i + AHEAD, queue[N]);      // behind the last use of the entry: before it, the group would start with copies of all entries, and with waits for them
         g[N & 1][u] = gr; g[N & 1][H + u] = gz; g[N & 1][2 * H + u] = gn;
         const float sum = product_sum3<H>(R, gr, gz, gnr, p);
-        carry = from_initial ? 0.f : dh * v.z + sum;
-        if (want_w) {
+        carry = from_initial ? 0.f : through + sum;
+        if constexpr (decltype(want)::value) {
             to_g[0] = gr; to_g[H] = gz; to_g[2 * H] = gn; *to_gnr = gnr; *to_hp = hp;
             to_g -= 3 * stride; to_gnr -= stride; to_hp -= stride;
             // the reference drops reset samples from the b_hn gradient, but for the sequence's first step (their buffer rows are zeroed before that sum, gru/operations_generic.h:716-749)
             db_hn += from_initial && i + 1 < S ? 0.f : gnr;
         }
-    });
+    }); });
     if (want_w && p == 0) G.db_hn[(size_t)b * H + u] = db_hn;
 }
 template <int H>
@@ -421,18 +454,19 @@ __device__ __forceinline__ void backward_row(const Backward& P, int b, char* lds
         const float* from = P.pre0 + last;
         float* to = P.want_w ? P.d_pre0 + last : nullptr;
         const int act0 = P.act0;
-        auto request = [&](int i, float& v) { if (i < S) { v = *from; from -= stride; } };
+        auto request = [&](int i, float& v) { v = *from; from -= i + 1 < S ? stride : 0; };
 #pragma unroll
         for (int d = 0; d < AHEAD; d++) request(d, queue[d]);
         ready();
-        stage<AHEAD>(S, 6, 1, [&](auto d, int i) {
+        by_condition(to != nullptr, [&](auto want) { stage<AHEAD>(S, 6, 1, [&](auto d, int i) {
             constexpr int N = decltype(d)::value, PAR = N & 1;
-            const float pre = queue[N];
+            float slope = rlt_dact(queue[N], act0);
+            asm volatile("" : "+v"(slope));
             request(i + AHEAD, queue[N]);
-            const float v = product_sum3<H>(R, L.g1[PAR][u], L.g1[PAR][H + u], L.g1[PAR][2 * H + u], p) * rlt_dact(pre, act0);
+            const float v = product_sum3<H>(R, L.g1[PAR][u], L.g1[PAR][H + u], L.g1[PAR][2 * H + u], p) * slope;
             L.dp0[PAR][u] = v;
-            if (to) { *to = v; to -= stride; }
-        });
+            if constexpr (decltype(want)::value) { *to = v; to -= stride; }
+        }); });
     } else {
         float w0[H];
         const int k = min(lane, P.in - 1);
@@ -454,7 +488,7 @@ __device__ __forceinline__ void backward_row(const Backward& P, int b, char* lds
         });
     }
 }
-__global__ __launch_bounds__(64 * BACKWARD_STAGES) void seq_stack_backward_kernel(BackwardLaunch K) {
+__global__ __launch_bounds__(64 * BACKWARD_STAGES, 4) void seq_stack_backward_kernel(BackwardLaunch K) {
     extern __shared__ __attribute__((aligned(16))) char lds_stack[];
     int k = 0;
     if (K.n > 1 && (int)blockIdx.x >= K.pass[1].first_block) k = 1;
