@@ -6,7 +6,7 @@
 //   * W_i x + b_i for ALL steps is one contraction over sequence*batch rows (gemm.hip), written straight into post_activation (at hidden width 64 and up to a thousand rows mostly
 //     formed beside the recurrence, inputs_beside);
 //   * the recurrence runs in ONE launch: batch rows are independent, so no grid-wide synchronisation is needed. At hidden width 64 a
-//     workgroup carries four rows through the sequence on the matrix cores or, up to two rows per compute unit, one row on the vector units, at 16 and 32 a wavefront 64 / width rows, both with W_h in registers; at other widths a workgroup owns a few
+//     workgroup carries four rows through the sequence on the matrix cores at 16 and 32 a wavefront 64 / width rows, both with W_h in registers, and up to a few rows per compute unit a workgroup one row on the vector units; at other widths a workgroup owns a few
 //     rows and keeps W_h and its rows' hidden state in LDS;
 //   * backward does the same in reverse and stores, per step, the gradient at the gate pre-activations (one copy as the input path sees
 //     it, one as the hidden path sees it, which differs in the n gate by the factor r) and the previous hidden state; the weight
@@ -617,13 +617,16 @@ __global__ __launch_bounds__(256, WAVES) void gru_backward_mfma_kernel(GruArgs A
     if (A.db_hn_partial) gru_at(A.db_hn_partial + (size_t)b0 * H, at) = db_hn;
 }
 
-// ---- hidden width 64, a workgroup per row (row_groups_forward, row_groups_backward) ----------------------------------------------
-// With few rows most compute units are idle on the kernels above, and a step of one row on the vector units is the shorter chain: the matrix instruction forms four rows in
-// 384 cycles whether they are there or not, the vector unit one row in 192. Wavefronts 0 to 3 carry the recurrence: four lanes share a hidden unit, the parts of the reduction meet in exchanges
-// within four (eight) lanes. What bounds them is the number of instructions that one wavefront issues per step (about five cycles each), so wavefronts 4 to 7 do the rest beside them: they request
+// ---- hidden widths 16, 32 and 64, a workgroup per row (rows_forward, rows_backward) -----------------------------------------------
+// With few rows most compute units are idle on the kernels above, and a step of one row on the vector units is the shorter chain: at width 64 the matrix instruction forms four rows in
+// 384 cycles whether they are there or not, the vector unit one row in 192; at 16 and 32 a wavefront that carries whole rows forms all their products, gates and stores one after the other. The
+// first H / 16 wavefronts carry the recurrence, sixteen units each: four lanes share a hidden unit, the parts of the reduction meet in exchanges
+// within four (eight) lanes. What bounds them is the number of instructions that one wavefront issues per step (about five cycles each), so four more wavefronts do the rest beside them: they request
 // what the steps read (D steps ahead), hand it over through LDS a step ahead and store what the steps leave there a step later. One workgroup barrier per step.
-// 64 steps at batch 64, four rows to a workgroup on the matrix cores / a row: forward recurrence 35.9 / 23 us, backward 33.2 / 25.5 (without wavefronts 4 to 7 25 and 29.9).
-constexpr int GR_THREADS = 512;
+// 64 steps at batch 64, four rows to a workgroup on the matrix cores / a row: forward recurrence 35.9 / 23 us, backward 33.2 / 25.5 (without the four wavefronts beside it 25 and 29.9);
+// width 32: the steps' share of a call 0.58 -> 0.37 us forward (library gates), 0.56 -> 0.33 backward.
+constexpr int gru_row_threads(int H) { return 64 * (H / 16 + 4); }
+enum { GATES_HARDWARE, GATES_FAST, GATES_EXACT };
 __device__ __forceinline__ float quad_xor1(float v) { return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true)); }
 __device__ __forceinline__ float quad_xor2(float v) { return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xF, 0xF, true)); }
 __device__ __forceinline__ float quad_low(float v) { return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x44, 0xF, 0xF, true)); }        // lanes 0, 1, 0, 1 of the four
@@ -637,17 +640,19 @@ template <class F> __device__ __forceinline__ void gru_by_parity(int S, F&& step
     for (; t + 2 <= S; t += 2) { step(std::integral_constant<int, 0>{}); step(std::integral_constant<int, 1>{}); }
     if (t < S) step(std::integral_constant<int, 0>{});
 }
-// Lane (unit, kq): quarter kq of the reduction, summed in the order of the kernel on the matrix cores; lanes 0 and 1 of the four finish r, 2 and 3 z.
-template <bool FAST>
-__global__ __launch_bounds__(GR_THREADS, 4) void gru_forward_row_kernel(GruArgs A) {
-    constexpr int H = 64, D = 4;
+// Lane (unit, kq): quarter kq of the reduction; lanes 0 and 1 of the four finish r, 2 and 3 z.
+template <int H, int GATES>
+__global__ __launch_bounds__(gru_row_threads(H), 4) void gru_forward_row_kernel(GruArgs A) {
+    constexpr int CHAIN = H / 16, QUARTER = H / 4, D = 4;
+    auto sigmoid = [](float x) { return GATES == GATES_HARDWARE ? hw_sigmoid(x) : gate_sigmoid(x, GATES == GATES_FAST); };
+    auto tanh_ = [](float x) { return GATES == GATES_HARDWARE ? hw_tanh(x) : gate_tanh(x, GATES == GATES_FAST); };
     __shared__ __align__(16) float hs[2][H];                  // the previous state, by the parity of the step
     __shared__ __align__(16) float given[2][2][4 * H];        // r (z) gate's input part, n gate's, and the state that follows: (output & third) | fourth
     __shared__ float left[2][5 * H];                          // r, n, z, the n gate's hidden part, the output
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), b = blockIdx.x;
     const size_t stride = (size_t)A.B * H;
-    if (w >= 4) {
-        const int role = w - 4, u = lane, gate = role < 3 ? role : 0;      // r, z, n gate; the resets and the other two outputs
+    if (w >= CHAIN) {
+        const int role = w - CHAIN, u = lane & (H - 1), gate = role < 3 ? role : 0;      // r, z, n gate; the resets and the other two outputs
         float* in = A.L.post_activation + (size_t)b * 3 * H + gate * H;
         float* to = role < 3 ? in : A.L.n_pre_pre_activation + (size_t)b * H;
         float* out = A.L.output + (size_t)b * H;
@@ -692,12 +697,12 @@ __global__ __launch_bounds__(GR_THREADS, 4) void gru_forward_row_kernel(GruArgs 
     }
     const int kq = lane & 3, u = 16 * w + (lane >> 2);
     const bool is_z = kq & 2, odd = kq & 1;
-    float wb[3][16];
+    float wb[3][QUARTER];
 #pragma unroll
     for (int g = 0; g < 3; g++) {
-        const float4* src = reinterpret_cast<const float4*>(A.L.weights_hidden + (size_t)(g * H + u) * H + 16 * kq);
+        const gru_float4_a4* src = reinterpret_cast<const gru_float4_a4*>(A.L.weights_hidden + (size_t)(g * H + u) * H + QUARTER * kq);
 #pragma unroll
-        for (int q = 0; q < 4; q++) { const float4 v = src[q]; wb[g][4 * q] = v.x; wb[g][4 * q + 1] = v.y; wb[g][4 * q + 2] = v.z; wb[g][4 * q + 3] = v.w; }
+        for (int q = 0; q < QUARTER / 4; q++) { const gru_float4_a4 v = src[q]; wb[g][4 * q] = v[0]; wb[g][4 * q + 1] = v[1]; wb[g][4 * q + 2] = v[2]; wb[g][4 * q + 3] = v[3]; }
     }
     const float bhn = A.L.biases_hidden[2 * H + u];
     float h = A.L.initial_hidden_state[u];
@@ -706,22 +711,22 @@ __global__ __launch_bounds__(GR_THREADS, 4) void gru_forward_row_kernel(GruArgs 
     rlt_lds_barrier();
     gru_by_parity(A.S, [&](auto parity) {
         constexpr int P = decltype(parity)::value;
-        gru_floatx4 a[4];
+        gru_floatx4 a[QUARTER / 4];
 #pragma unroll
-        for (int k = 0; k < 4; k++) a[k] = reinterpret_cast<const gru_floatx4*>(&hs[P][16 * kq])[k];
+        for (int k = 0; k < QUARTER / 4; k++) a[k] = reinterpret_cast<const gru_floatx4*>(&hs[P][QUARTER * kq])[k];
         const gru_floatx4 x = *reinterpret_cast<const gru_floatx4*>(&given[P][kq >> 1][4 * u]);
         __builtin_amdgcn_sched_barrier(0);      // all reads are under way before the first product
         float cr = 0.f, cz = 0.f, cn = 0.f;
 #pragma unroll
-        for (int k = 0; k < 4; k++)
+        for (int k = 0; k < QUARTER / 4; k++)
 #pragma unroll
             for (int j = 0; j < 4; j++) { cr = fmaf(a[k][j], wb[0][4 * k + j], cr); cz = fmaf(a[k][j], wb[1][4 * k + j], cz); cn = fmaf(a[k][j], wb[2][4 * k + j], cn); }
         float c = (is_z ? cz : cr) + quad_xor2(is_z ? cr : cz);
         cn += quad_xor2(cn);
         c += quad_xor1(c); cn += quad_xor1(cn);
         const float ac = x[0] + c, an = bhn + cn;
-        const float gate = FAST ? gate_sigmoid(ac, 1) : hw_sigmoid(ac), r = quad_low(gate), z = quad_high(gate);
-        const float n = FAST ? gate_tanh(x[1] + an * r, 1) : hw_tanh(x[1] + an * r);
+        const float gate = sigmoid(ac), r = quad_low(gate), z = quad_high(gate);
+        const float n = tanh_(x[1] + an * r);
         const float o = (1.0f - z) * n + z * h;
         h = __int_as_float((__float_as_int(o) & __float_as_int(x[2])) | __float_as_int(x[3]));
         hs[P ^ 1][u] = h;
@@ -730,17 +735,18 @@ __global__ __launch_bounds__(GR_THREADS, 4) void gru_forward_row_kernel(GruArgs 
         rlt_lds_barrier();
     });
 }
-// Reverse pass: lane (four units, sixteenth kq of the 64 units of each gate) forms the four units' sums over its 12 gate gradients (three 16-byte reads: with two units to a lane and six reads LDS,
+// Reverse pass: lane (four units, sixteenth kq of the units of each gate) forms the four units' sums over its gate gradients (width 64: 12 in three 16-byte reads; with two units to a lane and six reads LDS,
 // which serves a wavefront's in eight cycles each, was the longer chain), the sixteenths meet in four exchanges, the first two of which leave a unit to each four lanes. Every gate gradient is the gradient at the state times a factor of saved values, which the wavefronts beside the recurrence form.
-__global__ __launch_bounds__(GR_THREADS, 2) void gru_backward_row_kernel(GruArgs A) {
-    constexpr int H = 64, D = 4;
+template <int H>
+__global__ __launch_bounds__(gru_row_threads(H), 4) void gru_backward_row_kernel(GruArgs A) {
+    constexpr int CHAIN = H / 16, K = H / 16, D = 4;      // K: gate gradients of a gate that a lane multiplies
     __shared__ __align__(16) float gs[2][4 * H];               // gradients at the r, z and n gate as the hidden path sees them, and at the state
     __shared__ float factor[2][4 * H];                         // of these, by the gradient at the state
     __shared__ __align__(16) float given[2][4 * H];            // gradient at the output, mask of what the step before hands on, z gate
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), b = blockIdx.x, S = A.S;
     const size_t stride = (size_t)A.B * H, last = (size_t)(S - 1) * stride + (size_t)b * H;
-    if (w >= 4) {
-        const int role = w - 4, u = lane;      // r, z, n gate, state
+    if (w >= CHAIN) {
+        const int role = w - CHAIN, u = lane & (H - 1);      // r, z, n gate, state
         const unsigned at = u * sizeof(float);
         const float h0 = A.L.initial_hidden_state[u];
         struct Saved { float z, n, first, second; };      // r gate: r, npp; z: -, state before; n: r, -; state: gradient at the output, state before (what is not named is read and not used)
@@ -804,11 +810,11 @@ __global__ __launch_bounds__(GR_THREADS, 2) void gru_backward_row_kernel(GruArgs
     }
     const int kq = lane & 15, u0 = 16 * w + 4 * (lane >> 4), u = 16 * w + (lane >> 2), place = (lane & 3) * H + u;
     const bool upper8 = lane & 8, upper4 = lane & 4;
-    gru_floatx4 wb[12];
+    gru_floatx4 wb[3 * K];
 #pragma unroll
     for (int g = 0; g < 3; g++)
 #pragma unroll
-        for (int k = 0; k < 4; k++) wb[4 * g + k] = *reinterpret_cast<const gru_float4_a4*>(A.L.weights_hidden + (size_t)(g * H + 4 * kq + k) * H + u0);
+        for (int k = 0; k < K; k++) wb[K * g + k] = *reinterpret_cast<const gru_float4_a4*>(A.L.weights_hidden + (size_t)(g * H + K * kq + k) * H + u0);
     __builtin_amdgcn_s_setprio(1);
     rlt_lds_barrier();
     float f = factor[0][place], carry = 0.f;
@@ -818,9 +824,10 @@ __global__ __launch_bounds__(GR_THREADS, 2) void gru_backward_row_kernel(GruArgs
         const float dh = x[0] + masked(carry, x[1]), z = x[2];
         gs[P][place] = dh * f;
         rlt_lds_barrier();
-        gru_floatx4 v[3];
+        typedef float Own __attribute__((ext_vector_type(K)));
+        Own v[3];
 #pragma unroll
-        for (int g = 0; g < 3; g++) v[g] = *reinterpret_cast<const gru_floatx4*>(&gs[P][g * H + 4 * kq]);
+        for (int g = 0; g < 3; g++) v[g] = *reinterpret_cast<const Own*>(&gs[P][g * H + K * kq]);
         f = factor[P ^ 1][place];
         x = *reinterpret_cast<const gru_floatx4*>(&given[P ^ 1][4 * u]);
         __builtin_amdgcn_sched_barrier(0);      // all reads are under way before the first product
@@ -828,9 +835,9 @@ __global__ __launch_bounds__(GR_THREADS, 2) void gru_backward_row_kernel(GruArgs
 #pragma unroll
         for (int g = 0; g < 3; g++)
 #pragma unroll
-            for (int k = 0; k < 4; k++)
+            for (int k = 0; k < K; k++)
 #pragma unroll
-                for (int a = 0; a < 4; a++) c[a] = fmaf(v[g][k], wb[4 * g + k][a], c[a]);
+                for (int a = 0; a < 4; a++) c[a] = fmaf(v[g][k], wb[K * g + k][a], c[a]);
         const float c0 = (upper8 ? c[2] : c[0]) + row_half(upper8 ? c[0] : c[2]), c1 = (upper8 ? c[3] : c[1]) + row_half(upper8 ? c[1] : c[3]);
         float sum = (upper4 ? c1 : c0) + half_mirror(upper4 ? c0 : c1);
         sum += quad_xor2(sum); sum += quad_xor1(sum);
@@ -1216,11 +1223,14 @@ bool layer_ok(const rlt_gru_layer* L) {
 }
 int compute_units(const rlt_rocm_device* device) { return device->compute_units > 0 ? device->compute_units : 256; }
 bool one_group_per_unit(const rlt_rocm_device* device, const rlt_gru_layer* L, int B) { return L->hidden_dim == 64 && rlt_div_up(B, GM_ROWS) <= compute_units(device); }
-// Where the recurrence at width 64 takes a workgroup per row (with input gates and weight gradients as launches of their own). us of the calls, four rows to a workgroup / a row, 64 steps:
-// forward, 3 inputs 64 rows 41.0 / 28.3, 256 rows 50.0 / 37.4, 512 rows 53.4 / 44.5, 600 rows (three rounds of rows) 53.9 / 55.1; 8 steps 512 rows 13.4 / 13.3; 1 step 64 rows 8.0 / 7.2;
+// Where the recurrence takes a workgroup per row (with input gates and weight gradients as launches of their own). us of the calls, several rows to a workgroup / a row, 64 steps:
+// width 64: forward, 3 inputs 64 rows 41.0 / 28.3, 256 rows 50.0 / 37.4, 512 rows 53.4 / 44.5, 600 rows (three rounds of rows) 53.9 / 55.1; 8 steps 512 rows 13.4 / 13.3; 1 step 64 rows 8.0 / 7.2;
 // backward to the input 64 rows 33.2 / 25.5, 256 rows 34.1 / 26.7, 512 rows 34.4 / 33.0; 16 steps 64 rows 10.2 / 8.8, 512 rows 11.6 / 13.0; 1 step 3.85 / 4.0.
-bool rows_forward(const rlt_rocm_device* device, int B) { return B <= 2 * compute_units(device); }
-bool rows_backward(const rlt_rocm_device* device, int S, int B) { return B <= compute_units(device) && S >= 4; }
+// Width 32, 64 inputs: forward 64 rows 44.3 / 30.8, 512 rows 58.0 / 46.4, 1,024 rows 64.8 / 54.1, 1,536 rows 70.6 / 81.0; backward with weight gradients 64 rows 49.3 / 34.2, 512 rows 58.6 / 46.9, 700 rows
+// 61.0 / 53.7, 1,024 rows 66.2 / 64.3, but of 8 steps 24.1 / 24.9. Width 16: forward 64 rows 33.0 / 23.1, 1,024 rows 47.7 / 38.3, 1,536 rows 50.4 / 57.4; backward 64 rows 31.4 / 30.8, 256 rows
+// 38.6 / 37.3, 300 rows 38.4 / 40.2.
+bool rows_forward(const rlt_rocm_device* device, int H, int B) { return B <= (H == 64 ? 2 : 4) * compute_units(device); }
+bool rows_backward(const rlt_rocm_device* device, int H, int S, int B) { return S >= 4 && B <= (H == 32 ? 3 : 1) * compute_units(device); }
 bool overlap(const float* a, size_t n, const float* b, size_t m) { return (uintptr_t)a < (uintptr_t)(b + m) && (uintptr_t)b < (uintptr_t)(a + n); }
 int even_sixteens(int columns) { return 2 * rlt_div_up(columns, 32); }
 // Where the input gates / the weight gradients are formed beside the recurrence. The fp32 matrix instructions and the vector unit of a SIMD take turns, so that what goes beside the
@@ -1243,14 +1253,14 @@ bool inputs_beside(const rlt_rocm_device* device, const rlt_gru_layer* L, const 
     if (overlap(input, inputs, L->output, rows * 64) || overlap(input, inputs, L->n_pre_pre_activation, rows * 64) || overlap(input, inputs, L->post_activation, rows * 3 * 64)) return false;
     const int I = L->input_dim;
     const int units = compute_units(device);
-    const double by_row = B <= units ? 280.0 * S - 2000.0 : rows_forward(device, B) ? 70.0 * S - 500.0 : 0.0;      // what the recurrence of its own has from a workgroup per row
+    const double by_row = B <= units ? 280.0 * S - 2000.0 : rows_forward(device, 64, B) ? 70.0 * S - 500.0 : 0.0;      // what the recurrence of its own has from a workgroup per row
     const bool by_rows = I > 32 && I % 2 == 0 && rows >= 2048;      // the launch in front is rows_forward_kernel (rlt_gemm_rows_forward)
     const double launch = by_rows ? 3750.0 : I <= 32 ? 5800.0 : I % 4 == 0 ? 2400.0 : I % 2 == 0 ? 2600.0 : 3200.0;
     return (by_rows ? 27.2 : 23.8) * 4 * rlt_div_up(S, 4) * even_sixteens(I) + by_row <= launch + ((by_rows ? 0.143 : 0.185) + 0.0017 * I) * rows;
 }
 bool weights_beside(const rlt_rocm_device* device, const rlt_gru_layer* L, int S, int B, size_t room) {      // room: bytes of the caller's workspace that nothing else is kept in
     if (!one_group_per_unit(device, L, B) || L->input_dim > GW_INPUTS || rlt_div_up(B, GM_ROWS) * gru_gradient_block(L->input_dim) * sizeof(float) > room) return false;
-    return S * (54.0 + 46.0 * even_sixteens(L->input_dim)) + (rows_backward(device, S, B) ? 80.0 * S - 1500.0 : 0.0) <= 3400.0 + (0.35 + 0.0037 * L->input_dim) * S * B;
+    return S * (54.0 + 46.0 * even_sixteens(L->input_dim)) + (rows_backward(device, 64, S, B) ? 80.0 * S - 1500.0 : 0.0) <= 3400.0 + (0.35 + 0.0037 * L->input_dim) * S * B;
 }
 // The weight gradients of gru_gradients_kernel: pairs of column tiles, shares of the rows (workgroups for the whole chip, but at least eight steps of four rows to a wavefront; once, twice ... so many that no sum is longer than
 // 256 steps, for its error's sake), blocks of sums
@@ -1319,12 +1329,18 @@ int rlt_rocm_gru_forward(rlt_rocm_device* device, const rlt_gru_layer* L, const 
         rc = rlt_gemm_forward(device, input, L->input_dim, L->weights_input, L->biases_input, RLT_ACT_IDENTITY, nullptr, nullptr, L->post_activation, 3 * H, S * B, L->input_dim, 3 * H);
     if (rc) return rc;
     if (H == 64 || H == 32 || H == 16) {
-        const dim3 grid(rlt_div_up(B, GRU_THREADS / H)), block(GRU_THREADS);      // GRU_THREADS / 64 wavefronts of 64 / H rows
         const bool fast = L->fast_tanh != 0;      // a template parameter: as a run-time switch inside the step it cost 10% at width 64
+        if (rows_forward(device, H, B)) {
+            auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(B), dim3(gru_row_threads(H)), 0, device->stream, a); };
+            if (H == 64) { if (fast) launch(gru_forward_row_kernel<64, GATES_FAST>); else launch(gru_forward_row_kernel<64, GATES_HARDWARE>); }
+            else if (H == 32) { if (fast) launch(gru_forward_row_kernel<32, GATES_FAST>); else launch(gru_forward_row_kernel<32, GATES_EXACT>); }
+            else { if (fast) launch(gru_forward_row_kernel<16, GATES_FAST>); else launch(gru_forward_row_kernel<16, GATES_EXACT>); }
+            return rlt_launch_status(device);
+        }
+        const dim3 grid(rlt_div_up(B, GRU_THREADS / H)), block(GRU_THREADS);      // GRU_THREADS / 64 wavefronts of 64 / H rows
         if (H == 64) {
             const dim3 grid4(rlt_div_up(B, GM_ROWS));
-            if (rows_forward(device, B)) { if (fast) hipLaunchKernelGGL(gru_forward_row_kernel<true>, dim3(B), dim3(GR_THREADS), 0, device->stream, a); else hipLaunchKernelGGL(gru_forward_row_kernel<false>, dim3(B), dim3(GR_THREADS), 0, device->stream, a); }
-            else if (fast) hipLaunchKernelGGL(gru_forward_mfma_kernel<true>, grid4, block, 0, device->stream, a); else hipLaunchKernelGGL(gru_forward_mfma_kernel<false>, grid4, block, 0, device->stream, a);
+            if (fast) hipLaunchKernelGGL(gru_forward_mfma_kernel<true>, grid4, block, 0, device->stream, a); else hipLaunchKernelGGL(gru_forward_mfma_kernel<false>, grid4, block, 0, device->stream, a);
         }
         else if (H == 32) { if (fast) hipLaunchKernelGGL((gru_forward_reg_kernel<32, true>), grid, block, 0, device->stream, a); else hipLaunchKernelGGL((gru_forward_reg_kernel<32, false>), grid, block, 0, device->stream, a); }
         else { if (fast) hipLaunchKernelGGL((gru_forward_reg_kernel<16, true>), grid, block, 0, device->stream, a); else hipLaunchKernelGGL((gru_forward_reg_kernel<16, false>), grid, block, 0, device->stream, a); }
@@ -1363,11 +1379,13 @@ int rlt_rocm_gru_backward(rlt_rocm_device* device, const rlt_gru_layer* L, const
     a.h_previous = h_previous; a.db_hn_partial = want_weight_gradients ? db_hn_partial : nullptr; a.rows_per_group = rows_per_group(H);
     if (H == 64 || H == 32 || H == 16) {
         const dim3 grid(rlt_div_up(B, GRU_THREADS / H)), block(GRU_THREADS);
-        if (H == 64) {
+        if (rows_backward(device, H, S, B)) {
+            auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(B), dim3(gru_row_threads(H)), 0, device->stream, a); };
+            if (H == 64) launch(gru_backward_row_kernel<64>); else if (H == 32) launch(gru_backward_row_kernel<32>); else launch(gru_backward_row_kernel<16>);
+        } else if (H == 64) {
             const dim3 grid4(rlt_div_up(B, GM_ROWS));
             const int units = compute_units(device);
-            if (rows_backward(device, S, B)) hipLaunchKernelGGL(gru_backward_row_kernel, dim3(B), dim3(GR_THREADS), 0, device->stream, a);
-            else if (backward_by_rows(units, S, B)) hipLaunchKernelGGL(gru_backward_rows_kernel, grid4, block, 0, device->stream, a);
+            if (backward_by_rows(units, S, B)) hipLaunchKernelGGL(gru_backward_rows_kernel, grid4, block, 0, device->stream, a);
             else if ((int)grid4.x > 3 * units) hipLaunchKernelGGL((gru_backward_mfma_kernel<2, 4>), grid4, block, 0, device->stream, a);
             else hipLaunchKernelGGL((gru_backward_mfma_kernel<4, 2>), grid4, block, 0, device->stream, a);
         }

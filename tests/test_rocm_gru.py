@@ -154,17 +154,19 @@ def test_gru_at_the_edges_of_the_kernels_that_keep_a_layer_in_registers(oracle, 
 
 
 @pytest.mark.parametrize("fast_tanh", [False, True])
-@pytest.mark.parametrize("case", [(1, 1), (2, 3), (3, 2), (4, 5), (5, 256), (5, 257), (4, 512), (4, 513), (63, 2), (64, 3), (65, 1), (66, 2), (128, 1), (129, 2)])
+@pytest.mark.parametrize("case", [(1, 1, 64), (2, 3, 64), (3, 2, 64), (4, 5, 64), (5, 256, 64), (5, 257, 64), (4, 512, 64), (4, 513, 64), (63, 2, 64), (64, 3, 64), (65, 1, 64), (66, 2, 64),
+                                  (128, 1, 64), (129, 2, 64), (3, 1, 16), (4, 256, 16), (4, 257, 16), (2, 1024, 16), (2, 1025, 16), (65, 2, 16), (129, 1, 16), (3, 5, 32), (4, 768, 32),
+                                  (4, 769, 32), (2, 1024, 32), (2, 1025, 32), (64, 2, 32), (130, 1, 32)])
 def test_gru_with_a_workgroup_per_row(oracle, rocm, case, fast_tanh):
-    """Width 64 over at most 512 rows (backward 256, from four steps on) with more inputs than the kernels beside the recurrence take: steps around the groups of four and the 64 whose reset
-    flags are read at once, with resets and without, the last batches of a row per workgroup and the first of four. Tolerance as for the long batch above."""
+    """Widths 64, 32 and 16 over at most 512, 1,024 and 1,024 rows (backward 256, 768 and 256, from four steps on), with more inputs than the kernels beside the recurrence take: steps around the
+    groups of four and the 64 whose reset flags are read at once, with resets and without, the last batches of a row per workgroup and the first of several. Tolerance as for the long batch above."""
     print("case", case, fast_tanh, flush=True)
-    S, B = case
+    S, B, H = case
     for with_reset in (False, True):
-        params, x, dy, reset = helpers.gru_random_case(np.random.default_rng(39 + S + B), S, B, 161, 64, with_reset)
+        params, x, dy, reset = helpers.gru_random_case(np.random.default_rng(39 + S + B), S, B, 161, H, with_reset)
         results = []
         for b in (oracle, rocm):
-            g = helpers.GruOnBackend(b, S, B, 161, 64, params, fast_tanh=fast_tanh)
+            g = helpers.GruOnBackend(b, S, B, 161, H, params, fast_tanh=fast_tanh)
             g.forward(x, reset)
             g.backward(dy)
             b.sync()
