@@ -415,10 +415,12 @@ __global__ __launch_bounds__(WIDE_THREADS) void wgrad_wide_kernel(WideArgs a) {
 // 1,024 rows 5.1 -> 5.9 us, 2,048 7.9 -> 6.1, 65,536 35.4 -> 25.4 us: the line lies at 2,048 rows. K is padded to 64, 96, 128 or 160 (with 160 for everything beyond 64, a layer of 66 inputs
 // was slower than on the tiled kernel: forward pass of 4,096 x 66 -> 192 and its recurrence 20.1 us there, 22.3 padded to 160, 18.9 padded to 96). N: all 192 columns are multiplied whatever
 // N is; at N = 99 the tiled kernel wins at 2,048 rows (17.3 against 19.4 us with 100 inputs) and at 65,536 (181 against 184 with 34), at 144 this one or neither does: the line lies at 128.
-// Bound: the matrix pipe at long batches (27 us of 46, K padded to 160), the trip to memory for the weights at short ones.
+// Bound: the matrix pipe at long batches (27 us of 46, K padded to 160), the trip to memory for the weights and their way through LDS at short ones. Up to one block of rows for every second
+// compute unit (4,096 rows) a workgroup therefore takes 64 of the columns: a third of the weights to load and of the matrix instructions (forward pass of a layer of width 64, all columns / 64 of them,
+// 146 inputs, 2,048 rows 17.5 / 13.6 us, 4,096 rows 32.9 / 30.6, 8,192 rows 35.4 / 35.9, 16,384 rows 43.1 / 45.6; 64 inputs, 4,096 rows 29.0 / 27.8, 8,192 rows 31.1 / 30.7).
 struct RowsForward { const float* X; int ldx; const float* W; const float* bias; float* Y; int ldy; int M, N, K; };
 constexpr int RF_THREADS = 512, RF_ROWS = 32, ROWS_FORWARD_MIN_BATCH = 2048;
-template <int NJ>
+template <int NJ, int T>      // T: sixteens of columns per wavefront; 3: all columns, 1: the 64 of blockIdx.y
 __global__ __launch_bounds__(RF_THREADS) void rows_forward_kernel(RowsForward a) {
     constexpr int KP = 16 * NJ, XS = KP + 4, X2 = RF_ROWS * KP / 2, XQ = X2 / RF_THREADS;      // 16 bytes of each of sixteen rows fall on different banks
     static_assert(X2 % RF_THREADS == 0, "every thread stages the same number of pairs");
@@ -439,23 +441,24 @@ __global__ __launch_bounds__(RF_THREADS) void rows_forward_kernel(RowsForward a)
             *reinterpret_cast<float2*>(&xs[buf][(idx / (KP / 2)) * XS + col]) = col < a.K ? v[q] : make_float2(0.f, 0.f);
         }
     };
+    const int part0 = T == 3 ? 0 : blockIdx.y, col0 = T == 3 ? 48 * w : 64 * part0 + 16 * w;      // first of W's parts of 64 rows, this wavefront's first column
     const int blocks = (a.M + RF_ROWS - 1) / RF_ROWS;
     float2 next[XQ];
     request(blockIdx.x * RF_ROWS, next);
     // W goes through the same LDS buffer, 64 rows at a time: read from memory row by row (a lane's own operands, rows apart, took as long as three blocks of rows)
-    float2 wv[3][NJ];
+    float2 wv[T][NJ];
 #pragma unroll
-    for (int p = 0; p < 3; p++)
+    for (int p = 0; p < T; p++)
 #pragma unroll
         for (int q = 0; q < NJ; q++) {
-            const int idx = tid + RF_THREADS * q, n = 64 * p + idx / (KP / 2), col = 2 * (idx % (KP / 2));
+            const int idx = tid + RF_THREADS * q, n = 64 * (part0 + p) + idx / (KP / 2), col = 2 * (idx % (KP / 2));
             wv[p][q] = *reinterpret_cast<const float2*>(a.W + (size_t)min(n, a.N - 1) * a.K + min(col, a.K - 2));      // rows beyond the width repeat the last one and are not stored
         }
-    float b[3][NJ][4], bias[3];
+    float b[T][NJ][4], bias[T];
 #pragma unroll
-    for (int t = 0; t < 3; t++) bias[t] = a.bias[min(48 * w + 16 * t + r, a.N - 1)];
+    for (int t = 0; t < T; t++) bias[t] = a.bias[min(col0 + 16 * t + r, a.N - 1)];
 #pragma unroll
-    for (int p = 0; p < 3; p++) {
+    for (int p = 0; p < T; p++) {
         if (p > 0) rlt_lds_barrier();      // the rows before have been read
 #pragma unroll
         for (int q = 0; q < NJ; q++) {
@@ -464,11 +467,11 @@ __global__ __launch_bounds__(RF_THREADS) void rows_forward_kernel(RowsForward a)
         }
         rlt_lds_barrier();
 #pragma unroll
-        for (int t = 0; t < 3; t++)
-            if ((48 * w + 16 * t) >> 6 == p) {      // sixteen columns lie in one of the three parts
+        for (int t = 0; t < T; t++)
+            if ((col0 + 16 * t) >> 6 == part0 + p) {      // sixteen columns lie in one of the three parts
 #pragma unroll
                 for (int j = 0; j < NJ; j++) {
-                    const wide_floatx4 v = *reinterpret_cast<const wide_floatx4*>(&xs[0][((48 * w + 16 * t + r) & 63) * XS + 16 * j + 4 * kk]);
+                    const wide_floatx4 v = *reinterpret_cast<const wide_floatx4*>(&xs[0][((col0 + 16 * t + r) & 63) * XS + 16 * j + 4 * kk]);
 #pragma unroll
                     for (int e = 0; e < 4; e++) b[t][j][e] = v[e];
                 }
@@ -482,30 +485,30 @@ __global__ __launch_bounds__(RF_THREADS) void rows_forward_kernel(RowsForward a)
         request((block + (int)gridDim.x) * RF_ROWS, next);      // beyond the last row: the last one again
         __builtin_amdgcn_sched_barrier(0);
         const float* x = xs[buf] + (16 * tile + r) * XS + 4 * kk;
-        wide_floatx4 acc[3];
+        wide_floatx4 acc[T];
 #pragma unroll
-        for (int t = 0; t < 3; t++) acc[t] = wide_floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int t = 0; t < T; t++) acc[t] = wide_floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
             const wide_floatx4 av = *reinterpret_cast<const wide_floatx4*>(x + 16 * j);
 #pragma unroll
             for (int e = 0; e < 4; e++)
 #pragma unroll
-                for (int t = 0; t < 3; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[e], b[t][j][e], acc[t], 0, 0, 0);
+                for (int t = 0; t < T; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[e], b[t][j][e], acc[t], 0, 0, 0);
         }
         // element v of lane (r, kk): row 4 kk + v, column r of the tile
         const int row0 = block * RF_ROWS + 16 * tile + 4 * kk;
-        float* y = a.Y + (size_t)row0 * a.ldy + 48 * w + r;
-        if ((block + 1) * RF_ROWS <= a.M && 48 * (w + 1) <= a.N) {
+        float* y = a.Y + (size_t)row0 * a.ldy + col0 + r;
+        if ((block + 1) * RF_ROWS <= a.M && col0 + 16 * T <= a.N) {
 #pragma unroll
             for (int v = 0; v < 4; v++)
 #pragma unroll
-                for (int t = 0; t < 3; t++) y[(size_t)v * a.ldy + 16 * t] = acc[t][v] + bias[t];
+                for (int t = 0; t < T; t++) y[(size_t)v * a.ldy + 16 * t] = acc[t][v] + bias[t];
         } else {
 #pragma unroll
             for (int v = 0; v < 4; v++)
 #pragma unroll
-                for (int t = 0; t < 3; t++) if (row0 + v < a.M && 48 * w + 16 * t + r < a.N) y[(size_t)v * a.ldy + 16 * t] = acc[t][v] + bias[t];
+                for (int t = 0; t < T; t++) if (row0 + v < a.M && col0 + 16 * t + r < a.N) y[(size_t)v * a.ldy + 16 * t] = acc[t][v] + bias[t];
         }
         stage(next, buf ^ 1);
         rlt_lds_barrier();
@@ -715,10 +718,14 @@ int rlt_gemm_rows_forward(rlt_rocm_device* device, const float* x, int ldx, cons
         ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(W)) & 7u) != 0) return RLT_E_UNSUPPORTED;
     const RowsForward a = {x, ldx, W, bias, y, ldy, batch, out_dim, in_dim};
     const int blocks = rlt_div_up(batch, RF_ROWS), grid = blocks < device->compute_units ? blocks : device->compute_units;
-    if (in_dim <= 64) hipLaunchKernelGGL(rows_forward_kernel<4>, dim3(grid), dim3(RF_THREADS), 0, device->stream, a);
-    else if (in_dim <= 96) hipLaunchKernelGGL(rows_forward_kernel<6>, dim3(grid), dim3(RF_THREADS), 0, device->stream, a);
-    else if (in_dim <= 128) hipLaunchKernelGGL(rows_forward_kernel<8>, dim3(grid), dim3(RF_THREADS), 0, device->stream, a);
-    else hipLaunchKernelGGL(rows_forward_kernel<10>, dim3(grid), dim3(RF_THREADS), 0, device->stream, a);
+    auto launch = [&](auto all, auto part) {
+        if (2 * blocks <= device->compute_units) hipLaunchKernelGGL(part, dim3(blocks, rlt_div_up(out_dim, 64)), dim3(RF_THREADS), 0, device->stream, a);
+        else hipLaunchKernelGGL(all, dim3(grid), dim3(RF_THREADS), 0, device->stream, a);
+    };
+    if (in_dim <= 64) launch(rows_forward_kernel<4, 3>, rows_forward_kernel<4, 1>);
+    else if (in_dim <= 96) launch(rows_forward_kernel<6, 3>, rows_forward_kernel<6, 1>);
+    else if (in_dim <= 128) launch(rows_forward_kernel<8, 3>, rows_forward_kernel<8, 1>);
+    else launch(rows_forward_kernel<10, 3>, rows_forward_kernel<10, 1>);
     return rlt_launch_status(device);
 }
 

@@ -141,10 +141,10 @@ def test_gru_backward_on_both_sides_of_the_line_to_whole_rows(oracle, rocm, case
 
 
 @pytest.mark.parametrize("case", [(32, 64, 34, 64), (33, 63, 160, 64), (16, 129, 66, 33), (64, 256, 64, 50), (64, 257, 146, 64), (64, 256, 36, 16),
-                                  (32, 64, 96, 64), (33, 63, 98, 43), (16, 129, 128, 43), (32, 65, 130, 64), (64, 1024, 34, 44)])
+                                  (32, 64, 96, 64), (33, 63, 98, 43), (16, 129, 128, 43), (32, 65, 130, 64), (64, 1024, 34, 44), (64, 64, 98, 44), (17, 241, 98, 43)])
 def test_gru_at_the_edges_of_the_kernels_that_keep_a_layer_in_registers(oracle, rocm, case):
     """Input gates with their weights in registers (2,048 rows and more, 129 to 192 gates, even inputs from 34 to 160, padded to 64, 96, 128 or 160) and weight gradients in one workgroup's
-    accumulators (16,384 rows and more, even widths from 66 to 160; from 34 on for 129 gates and 65,536 rows): the smallest and largest inputs, ragged last rows, gates and widths that fill
+    accumulators (16,384 rows and more, even widths from 66 to 160; from 34 on for 129 gates and 65,536 rows), the last batch whose columns are shared out (4,096 rows) and the first behind it: the smallest and largest inputs, ragged last rows, gates and widths that fill
     no tile. Tolerance as for the long batch above."""
     print("case", case, flush=True)
     S, B, I, H = case
