@@ -623,8 +623,8 @@ __global__ __launch_bounds__(256, WAVES) void gru_backward_mfma_kernel(GruArgs A
 // first H / 16 wavefronts carry the recurrence, sixteen units each: four lanes share a hidden unit, the parts of the reduction meet in exchanges
 // within four (eight) lanes. What bounds them is the number of instructions that one wavefront issues per step (about five cycles each), so four more wavefronts do the rest beside them: they request
 // what the steps read (D steps ahead), hand it over through LDS a step ahead and store what the steps leave there a step later. One workgroup barrier per step.
-// 64 steps at batch 64, four rows to a workgroup on the matrix cores / a row: forward recurrence 35.9 / 23 us, backward 33.2 / 25.5 (without the four wavefronts beside it 25 and 29.9);
-// width 32: the steps' share of a call 0.58 -> 0.37 us forward (library gates), 0.56 -> 0.33 backward.
+// 64 steps at batch 64, four rows to a workgroup on the matrix cores / a row: forward recurrence 35.9 / 23 us, backward 33.2 / 23.2 (without the four wavefronts beside it 25 and 29.9);
+// width 32, a step: forward 0.52 / 0.38 us (library gates), backward 0.56 / 0.25; width 16: 0.40 / 0.24 and 0.30 / 0.19.
 constexpr int gru_row_threads(int H) { return 64 * (H / 16 + 4); }
 enum { GATES_HARDWARE, GATES_FAST, GATES_EXACT };
 __device__ __forceinline__ float quad_xor1(float v) { return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true)); }
@@ -634,6 +634,12 @@ __device__ __forceinline__ float quad_high(float v) { return __int_as_float(__bu
 __device__ __forceinline__ float half_mirror(float v) { return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x141, 0xF, 0xF, true)); }    // lane 7 - i of the eight
 __device__ __forceinline__ float row_half(float v) { return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x128, 0xF, 0xF, true)); }       // lane i ^ 8 of the sixteen
 __device__ __forceinline__ float masked(float v, float mask) { return __int_as_float(__float_as_int(v) & __float_as_int(mask)); }
+// The roles of the wavefronts beside the recurrence, each with a loop of its own: as branches within a step they held every step's barrier up (backward, 64 steps of
+// 64 rows: width 16 21.7 -> 14.7 us, width 32 23.0 -> 17.8, width 64 26.3 -> 23.2).
+template <class F> __device__ __forceinline__ void by_role(int role, F&& body) {
+    if (role == 0) body(std::integral_constant<int, 0>{}); else if (role == 1) body(std::integral_constant<int, 1>{});
+    else if (role == 2) body(std::integral_constant<int, 2>{}); else body(std::integral_constant<int, 3>{});
+}
 // steps 0 ... S - 1, their parity a constant
 template <class F> __device__ __forceinline__ void gru_by_parity(int S, F&& step) {
     int t = 0;
@@ -652,7 +658,9 @@ __global__ __launch_bounds__(gru_row_threads(H), 4) void gru_forward_row_kernel(
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), b = blockIdx.x;
     const size_t stride = (size_t)A.B * H;
     if (w >= CHAIN) {
-        const int role = w - CHAIN, u = lane & (H - 1), gate = role < 3 ? role : 0;      // r, z, n gate; the resets and the other two outputs
+        by_role(w - CHAIN, [&](auto number_of_role) {
+        constexpr int role = decltype(number_of_role)::value;
+        const int u = lane & (H - 1), gate = role < 3 ? role : 0;      // r, z, n gate; the resets and the other two outputs
         float* in = A.L.post_activation + (size_t)b * 3 * H + gate * H;
         float* to = role < 3 ? in : A.L.n_pre_pre_activation + (size_t)b * H;
         float* out = A.L.output + (size_t)b * H;
@@ -693,6 +701,7 @@ __global__ __launch_bounds__(gru_row_threads(H), 4) void gru_forward_row_kernel(
             });
         }
         store((A.S - 1) & 1);
+        });
         return;
     }
     const int kq = lane & 3, u = 16 * w + (lane >> 2);
@@ -746,7 +755,9 @@ __global__ __launch_bounds__(gru_row_threads(H), 4) void gru_backward_row_kernel
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), b = blockIdx.x, S = A.S;
     const size_t stride = (size_t)A.B * H, last = (size_t)(S - 1) * stride + (size_t)b * H;
     if (w >= CHAIN) {
-        const int role = w - CHAIN, u = lane & (H - 1);      // r, z, n gate, state
+        by_role(w - CHAIN, [&](auto number_of_role) {
+        constexpr int role = decltype(number_of_role)::value;
+        const int u = lane & (H - 1);      // r, z, n gate, state
         const unsigned at = u * sizeof(float);
         const float h0 = A.L.initial_hidden_state[u];
         struct Saved { float z, n, first, second; };      // r gate: r, npp; z: -, state before; n: r, -; state: gradient at the output, state before (what is not named is read and not used)
@@ -806,6 +817,7 @@ __global__ __launch_bounds__(gru_row_threads(H), 4) void gru_backward_row_kernel
         }
         store((S - 1) & 1);
         if (role == 2 && A.db_hn_partial) gru_at(A.db_hn_partial + (size_t)b * H, at) = db_hn;
+        });
         return;
     }
     const int kq = lane & 15, u0 = 16 * w + 4 * (lane >> 4), u = 16 * w + (lane >> 2), place = (lane & 3) * H + u;
@@ -1223,14 +1235,18 @@ bool layer_ok(const rlt_gru_layer* L) {
 }
 int compute_units(const rlt_rocm_device* device) { return device->compute_units > 0 ? device->compute_units : 256; }
 bool one_group_per_unit(const rlt_rocm_device* device, const rlt_gru_layer* L, int B) { return L->hidden_dim == 64 && rlt_div_up(B, GM_ROWS) <= compute_units(device); }
-// Where the recurrence takes a workgroup per row (with input gates and weight gradients as launches of their own). us of the calls, several rows to a workgroup / a row, 64 steps:
-// width 64: forward, 3 inputs 64 rows 41.0 / 28.3, 256 rows 50.0 / 37.4, 512 rows 53.4 / 44.5, 600 rows (three rounds of rows) 53.9 / 55.1; 8 steps 512 rows 13.4 / 13.3; 1 step 64 rows 8.0 / 7.2;
-// backward to the input 64 rows 33.2 / 25.5, 256 rows 34.1 / 26.7, 512 rows 34.4 / 33.0; 16 steps 64 rows 10.2 / 8.8, 512 rows 11.6 / 13.0; 1 step 3.85 / 4.0.
-// Width 32, 64 inputs: forward 64 rows 44.3 / 30.8, 512 rows 58.0 / 46.4, 1,024 rows 64.8 / 54.1, 1,536 rows 70.6 / 81.0; backward with weight gradients 64 rows 49.3 / 34.2, 512 rows 58.6 / 46.9, 700 rows
-// 61.0 / 53.7, 1,024 rows 66.2 / 64.3, but of 8 steps 24.1 / 24.9. Width 16: forward 64 rows 33.0 / 23.1, 1,024 rows 47.7 / 38.3, 1,536 rows 50.4 / 57.4; backward 64 rows 31.4 / 30.8, 256 rows
-// 38.6 / 37.3, 300 rows 38.4 / 40.2.
-bool rows_forward(const rlt_rocm_device* device, int H, int B) { return B <= (H == 64 ? 2 : 4) * compute_units(device); }
-bool rows_backward(const rlt_rocm_device* device, int H, int S, int B) { return S >= 4 && B <= (H == 32 ? 3 : 1) * compute_units(device); }
+// Where the recurrence takes a workgroup per row (with input gates and weight gradients as launches of their own). us, several rows to a workgroup / a row:
+// forward calls of 64 steps, width 64, 3 inputs 64 rows 41.0 / 28.3, 256 rows 50.0 / 37.4, 512 rows 53.4 / 44.5, 600 rows (three rounds of rows) 53.9 / 55.1; width 32, 64 inputs 64 rows 44.3 / 30.6, 512 rows
+// 58.0 / 46.2, 1,024 rows 64.8 / 54.1; 200 inputs 1,280 rows 100 / 92, 1,536 rows 108 / 114; width 16 64 rows 33.0 / 22.7, 1,024 rows 47.7 / 38.3; 200 inputs 1,280 rows 63 / 56, 1,536 rows 68 / 75;
+// 1 step at 1,280 rows 14.6 / 12.5 and 12.4 / 12.4;
+// backward to the input, 64 steps, width 64 256 rows 34.1 / 24.3, 512 rows 34.3 / 28.4, 768 rows 34.9 / 37; width 32 256 rows 39.5 / 18.6, 1,024 rows 39.6 / 27.3, 1,280 rows 39.8 / 32.0, 1,536 rows 40.2 / 41.6;
+// width 16 256 rows 22.6 / 15.4, 768 rows 23.1 / 21.4, 1,024 rows 23.2 / 24.4; 16 steps, width 64 256 rows 11.0 / 9.0, 512 rows 11.5 / 11.6, width 32 1,280 rows 13.3 / 12.1, width 16 768 rows 8.4 / 8.0;
+// 4 steps, width 64 512 rows 5.4 / 6.8, width 32 1,280 rows 6.1 / 6.2; 1 step 3.85 / 4.0.
+bool rows_forward(const rlt_rocm_device* device, int H, int B) { return B <= (H == 64 ? 2 : 5) * compute_units(device); }
+bool rows_backward(const rlt_rocm_device* device, int H, int S, int B) {
+    const int units = compute_units(device);
+    return B <= units ? S >= 4 : B <= (H == 64 ? 2 : H == 32 ? 5 : 3) * units && S >= (H == 64 ? 20 : 8);
+}
 bool overlap(const float* a, size_t n, const float* b, size_t m) { return (uintptr_t)a < (uintptr_t)(b + m) && (uintptr_t)b < (uintptr_t)(a + n); }
 int even_sixteens(int columns) { return 2 * rlt_div_up(columns, 32); }
 // Where the input gates / the weight gradients are formed beside the recurrence. The fp32 matrix instructions and the vector unit of a SIMD take turns, so that what goes beside the
@@ -1260,7 +1276,7 @@ bool inputs_beside(const rlt_rocm_device* device, const rlt_gru_layer* L, const 
 }
 bool weights_beside(const rlt_rocm_device* device, const rlt_gru_layer* L, int S, int B, size_t room) {      // room: bytes of the caller's workspace that nothing else is kept in
     if (!one_group_per_unit(device, L, B) || L->input_dim > GW_INPUTS || rlt_div_up(B, GM_ROWS) * gru_gradient_block(L->input_dim) * sizeof(float) > room) return false;
-    return S * (54.0 + 46.0 * even_sixteens(L->input_dim)) + (rows_backward(device, 64, S, B) ? 80.0 * S - 1500.0 : 0.0) <= 3400.0 + (0.35 + 0.0037 * L->input_dim) * S * B;
+    return S * (54.0 + 46.0 * even_sixteens(L->input_dim)) + (rows_backward(device, 64, S, B) ? 110.0 * S - (B <= compute_units(device) ? 1500.0 : 2000.0) : 0.0) <= 3400.0 + (0.35 + 0.0037 * L->input_dim) * S * B;
 }
 // The weight gradients of gru_gradients_kernel: pairs of column tiles, shares of the rows (workgroups for the whole chip, but at least eight steps of four rows to a wavefront; once, twice ... so many that no sum is longer than
 // 256 steps, for its error's sake), blocks of sums

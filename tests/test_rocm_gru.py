@@ -154,12 +154,12 @@ def test_gru_at_the_edges_of_the_kernels_that_keep_a_layer_in_registers(oracle, 
 
 
 @pytest.mark.parametrize("fast_tanh", [False, True])
-@pytest.mark.parametrize("case", [(1, 1, 64), (2, 3, 64), (3, 2, 64), (4, 5, 64), (5, 256, 64), (5, 257, 64), (4, 512, 64), (4, 513, 64), (63, 2, 64), (64, 3, 64), (65, 1, 64), (66, 2, 64),
-                                  (128, 1, 64), (129, 2, 64), (3, 1, 16), (4, 256, 16), (4, 257, 16), (2, 1024, 16), (2, 1025, 16), (65, 2, 16), (129, 1, 16), (3, 5, 32), (4, 768, 32),
-                                  (4, 769, 32), (2, 1024, 32), (2, 1025, 32), (64, 2, 32), (130, 1, 32)])
+@pytest.mark.parametrize("case", [(1, 1, 64), (2, 3, 64), (3, 2, 64), (4, 5, 64), (5, 256, 64), (5, 257, 64), (4, 512, 64), (4, 513, 64), (20, 512, 64), (20, 513, 64), (19, 400, 64), (63, 2, 64),
+                                  (64, 3, 64), (65, 1, 64), (66, 2, 64), (128, 1, 64), (129, 2, 64), (3, 1, 16), (4, 256, 16), (4, 257, 16), (8, 768, 16), (8, 769, 16), (2, 1280, 16),
+                                  (2, 1281, 16), (65, 2, 16), (129, 1, 16), (3, 5, 32), (7, 300, 32), (8, 1280, 32), (8, 1281, 32), (64, 2, 32), (130, 1, 32)])
 def test_gru_with_a_workgroup_per_row(oracle, rocm, case, fast_tanh):
-    """Widths 64, 32 and 16 over at most 512, 1,024 and 1,024 rows (backward 256, 768 and 256, from four steps on), with more inputs than the kernels beside the recurrence take: steps around the
-    groups of four and the 64 whose reset flags are read at once, with resets and without, the last batches of a row per workgroup and the first of several. Tolerance as for the long batch above."""
+    """Widths 64, 32 and 16 over at most 512, 1,280 and 1,280 rows (backward 512, 1,280 and 768, from four, eight or twenty steps on), with more inputs than the kernels beside the recurrence
+    take: steps around the groups of four and the 64 whose reset flags are read at once, with resets and without, the last batches of a row per workgroup and the first of several. Tolerance as for the long batch above."""
     print("case", case, fast_tanh, flush=True)
     S, B, H = case
     for with_reset in (False, True):
