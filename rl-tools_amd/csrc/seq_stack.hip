@@ -10,8 +10,9 @@
 // Bound: the instructions of a recurrence's step. A wavefront is alone on its SIMD and issues one instruction every four to five cycles whatever it is (vector, scalar,
 // wait), so a step takes its instruction count: about 115 at width 32, 48 of them the products. Hence the forms below: values exchanged between lanes instead of through
 // LDS, the r gate in one half of the lanes while z is in the other, stores and LDS writes by all lanes of a unit rather than under an exec mask, addresses moved on
-// instead of formed, loops unrolled to the slots' parity. The training set of 100 sequences of 100 steps (actor of width 16, critics of width 32) has four forward launches of 38.4 us on average and
-// three backward launches of 37.4; a launch per layer with a row per 32 lanes took 0.59 us per step at width 32 and 0.45 at 16, one
+// instead of formed, loops unrolled to the slots' parity, the stages around the recurrences without a choice of activation per step where it is relu (a tick takes as long as its longest stage: 341 -> 332 us
+// for the training set of 100 sequences of 100 steps, 1,000 sequences 1,481 -> 1,456). That set (actor of width 16, critics of width 32) has four forward launches of 37.9 us on average and three backward
+// launches of 35.3; a launch per layer with a row per 32 lanes took 0.59 us per step at width 32 and 0.45 at 16, one
 // layer after the other, plus launches for the dense layers, projections and gradients.
 #include "seq_stack.h"
 #include "gemm.h"
@@ -289,18 +290,18 @@ __device__ __forceinline__ void forward_row(const Forward& P, int b, char* lds) 
         const int in = P.in, act0 = P.act0;
         const float* row = xs;
         ready();
-        stage<2>(S, 0, FORWARD_STAGES - 1, [&](auto d, int) {
+        by_condition(act0 == RLT_ACT_RELU, [&](auto relu) { stage<2>(S, 0, FORWARD_STAGES - 1, [&](auto d, int) {      // the approximators' activation without the others' branches in every step
             float acc = b0;
             const floatx4* x = reinterpret_cast<const floatx4*>(row);
 #pragma unroll
             for (int q = 0; q < MAX_IN / 4; q++)
                 if (q == 0 || 4 * q < in) { const floatx4 v = x[q]; acc += v[0] * w0[4 * q]; acc += v[1] * w0[4 * q + 1]; acc += v[2] * w0[4 * q + 2]; acc += v[3] * w0[4 * q + 3]; }
             row += in4;
-            const float o = rlt_act(acc, act0);
+            const float o = rlt_act(acc, decltype(relu)::value ? (int)RLT_ACT_RELU : act0);
             *keep = (p & 1) ? o : acc;
             keep += stride;
             project<H>(J, o, u, p, L.p1[decltype(d)::value & 1]);
-        });
+        }); });
     }
     else if (wave == 1) recurrence<H, FAST>(P, 0, 1, L.p1, L.h1, flags, b, lane, ready);
     else if (wave == 2) {
@@ -332,7 +333,7 @@ __device__ __forceinline__ void forward_row(const Forward& P, int b, char* lds) 
         });
     }
 }
-__global__ __launch_bounds__(64 * FORWARD_STAGES) void seq_stack_forward_kernel(ForwardLaunch K) {
+__global__ __launch_bounds__(64 * FORWARD_STAGES, 5) void seq_stack_forward_kernel(ForwardLaunch K) {
     extern __shared__ __attribute__((aligned(16))) char lds_stack[];
     int k = 0;
     if (K.n > 1 && (int)blockIdx.x >= K.pass[1].first_block) k = 1;
@@ -458,15 +459,15 @@ __device__ __forceinline__ void backward_row(const Backward& P, int b, char* lds
 #pragma unroll
         for (int d = 0; d < AHEAD; d++) request(d, queue[d]);
         ready();
-        by_condition(to != nullptr, [&](auto want) { stage<AHEAD>(S, 6, 1, [&](auto d, int i) {
+        by_condition(to != nullptr, [&](auto want) { by_condition(act0 == RLT_ACT_RELU, [&](auto relu) { stage<AHEAD>(S, 6, 1, [&](auto d, int i) {
             constexpr int N = decltype(d)::value, PAR = N & 1;
-            float slope = rlt_dact(queue[N], act0);
+            float slope = rlt_dact(queue[N], decltype(relu)::value ? (int)RLT_ACT_RELU : act0);
             asm volatile("" : "+v"(slope));
             request(i + AHEAD, queue[N]);
             const float v = product_sum3<H>(R, L.g1[PAR][u], L.g1[PAR][H + u], L.g1[PAR][2 * H + u], p) * slope;
             L.dp0[PAR][u] = v;
             if constexpr (decltype(want)::value) { *to = v; to -= stride; }
-        }); });
+        }); }); });
     } else {
         float w0[H];
         const int k = min(lane, P.in - 1);
