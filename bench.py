@@ -842,7 +842,7 @@ def main():
         rooflines["ppo_minibatch_update_8192"] = mfma("mlp3s_kernel (the optimisers' step at its head)", ppo["tflops"], PPO_UPDATE_HBM_BYTES, "106,368 flop per row and epoch (actor 105-64-64-8 and critic 105-64-64-1, forward + backward)")
     if gru:
         for g in gru:
-            rooflines["gru_training_step_b%d" % g["batch"]] = mfma("gru_forward_mfma_kernel + gru_backward_mfma_kernel + rows_forward_kernel + gru_gradients_kernel" if g["batch"] <= 64 else "gru_forward_inputs_kernel + gru_backward_weights_kernel", g["tflops"], None, "forward + backward through time, 64 steps, input 146, hidden 64")
+            rooflines["gru_training_step_b%d" % g["batch"]] = mfma("gru_forward_row_kernel + gru_backward_row_kernel + rows_forward_kernel + gru_gradients_kernel" if g["batch"] <= 64 else "gru_forward_inputs_kernel + gru_backward_weights_kernel", g["tflops"], None, "forward + backward through time, 64 steps, input 146, hidden 64")
     if rooflines:
         line["rooflines"] = rooflines
     if env:
