@@ -91,44 +91,61 @@ template <int NT1C> constexpr int FIRST_STEP = NT1C <= FEW ? 1 : 4;      // (fiv
 // How the weights come: FORM_ANY and FORM_EVERY (see EVERY above) from the copies; FORM_DIRECT, MLP passes of exactly 256 units whose second layer lies on 16 bytes, from the layers themselves, without
 // the launch that makes the copies (3.2 to 3.7 us). What a lane needs of the second layer on the way forward is four values that lie a row apart from its neighbours'; it is asked for as it lies, four
 // neighbouring lanes 64 bytes of one row (a 256 x 256 layer in 1.85 us, as from the copies; 6.96 where every lane has a row of its own), and dealt out in registers by selects that fetch from the
-// neighbouring lane, 128 per wavefront and layer beside 64 matrix instructions. On the way back only tiles of sixteen rows need such a dealing. Rows of the first layer are any number of floats; its few
-// chunks go through the wavefront's own part of the LDS. 17-256-256-6 with the gradients' clearing and Adam, copies / direct: forward + backward in one call 29.6 / 28.9 us at 256 rows, 36.1 / 35.2 at
-// 1,000, 43.9 / 43.5 at 2,048, 49.3 / 48.5 at 3,000, 54.0 / 53.9 at 4,096; as calls of their own 32.5 / 31.0, 41.1 / 38.5, 51.2 / 49.3, 57.7 / 54.9 and 62.1 / 58.9. The updates of SAC and TD3, whose
+// neighbouring lane, 128 per wavefront and layer beside 64 matrix instructions. On the way back only tiles of sixteen rows need such a dealing, by moves that the compiler sees (deal_values). Rows of the first layer are any number of floats; its few
+// chunks go through the wavefront's own part of the LDS. 17-256-256-6, copies / direct: step with the gradients' clearing, forward + backward in one call and Adam 28.5 / 28.1 us at 256 rows, 34.8 / 34.5 at
+// 1,000, 42.9 / 42.6 at 2,048, 48.4 / 48.1 at 3,000, 52.7 / 52.5 at 4,096; forward pass alone 15.0 / 13.8 at 2,049 rows, 16.5 / 15.1 at 4,096; backward pass alone 16.0 / 12.7 at 256, 21.3 / 19.2 at 1,000,
+// 27.3 / 25.7 at 2,048, 30.7 / 29.3 at 3,000, 34.0 / 33.0 at 4,096. The updates of SAC and TD3, whose
 // chains have two or three layers to deal out one after the other, keep the copies (sets at 256 rows 66.3 / 67.6 and 78.0 / 78.7).
 enum { FORM_ANY = 0, FORM_EVERY = 1, FORM_DIRECT = 2 };
 constexpr int W1S = 36, W1_STAGE = 16 * W1S;      // a wavefront's sixteen rows of two chunks, the rows four banks apart
 // a's values of the upper lanes of pairs against b's of the lower ones, as selects whose first operand comes through the lane control (left to the compiler, the exchange is an instruction of its own).
-// The data of such an operand must have been written two wait states before it is read, which the compiler does not see to inside an asm statement.
-#define RLT_EXCHANGE(FROM_LOWER, FROM_UPPER)                                                                                                                          \
-    floatx4 x, y;                                                                                                                                                     \
-    _Pragma("unroll") for (int i = 0; i < 4; i += 2) {                                                                                                                \
-        float x0, x1, y0, y1;                                                                                                                                         \
-        asm("s_nop 1\n\ts_mov_b64 vcc, %8\n\t"                                                                                                                       \
-            "v_cndmask_b32_dpp %0, %6, %4, vcc " FROM_LOWER " row_mask:0xf bank_mask:0xf bound_ctrl:0\n\tv_cndmask_b32_dpp %1, %7, %5, vcc " FROM_LOWER " row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t" \
-            "s_mov_b64 vcc, %9\n\t"                                                                                                                                  \
-            "v_cndmask_b32_dpp %2, %4, %6, vcc " FROM_UPPER " row_mask:0xf bank_mask:0xf bound_ctrl:0\n\tv_cndmask_b32_dpp %3, %5, %7, vcc " FROM_UPPER " row_mask:0xf bank_mask:0xf bound_ctrl:0"   \
-            : "=&v"(x0), "=&v"(x1), "=&v"(y0), "=&v"(y1) : "v"(a[i]), "v"(a[i + 1]), "v"(b[i]), "v"(b[i + 1]), "s"(~upper), "s"(upper) : "vcc");                       \
-        x[i] = x0; x[i + 1] = x1; y[i] = y0; y[i + 1] = y1;                                                                                                           \
-    }                                                                                                                                                                 \
-    a = x; b = y
-constexpr uint64_t LANES_1 = 0xAAAAAAAAAAAAAAAAull, LANES_2 = 0xCCCCCCCCCCCCCCCCull, LANES_4 = 0xF0F0F0F0F0F0F0F0ull, LANES_8 = 0xFF00FF00FF00FF00ull;      // lanes with that bit
-template <uint64_t upper> __device__ __forceinline__ void exchange(floatx4& a, floatx4& b) {
-    if constexpr (upper == LANES_1) { RLT_EXCHANGE("quad_perm:[1,0,3,2]", "quad_perm:[1,0,3,2]"); }
-    else if constexpr (upper == LANES_2) { RLT_EXCHANGE("quad_perm:[2,3,0,1]", "quad_perm:[2,3,0,1]"); }
-    else if constexpr (upper == LANES_4) { RLT_EXCHANGE("row_shr:4", "row_shl:4"); }      // (lanes without a partner on that side keep their own: bound_ctrl has them written all the same)
-    else { RLT_EXCHANGE("row_ror:8", "row_ror:8"); }
+// The compiler does not look into an asm statement, so the statement brings its wait states itself (tests/test_dpp_wait_states.py looks the built instructions over): two between what writes an operand and
+// the lane control that reads it; two behind a deal's last ones before a matrix instruction reads what they leave; and it must not write a register that a matrix instruction is still writing. On tiles of
+// four and eight rows those are the 4 x 4 x 1 ones, which take four: the three states in front of the first select and one more. On tiles of sixteen rows they take ten, too many to wait for; there no
+// output is of the compiler's choice: b is exchanged in place, a goes to spare's registers and leaves its own as the next exchange's, so that each holds a value that the compiler itself wrote there.
+#define RLT_SELECT(to, from, own, CONTROL) "v_cndmask_b32_dpp %" #to ", %" #from ", %" #own ", vcc " CONTROL " row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+#define RLT_EXCHANGE(CONTROL, END)                                                                                                                                 \
+    if constexpr (R == ROWS)                                                                                                                                       \
+        asm("s_nop 1\n\ts_mov_b64 vcc, %6\n\t" RLT_SELECT(0, 2, 4, CONTROL) RLT_SELECT(1, 3, 5, CONTROL) "s_mov_b64 vcc, %7\n\t" RLT_SELECT(2, 4, 2, CONTROL)      \
+            RLT_SELECT(3, 5, 3, CONTROL) END : "+&v"(x0), "+&v"(x1), "+&v"(b0), "+&v"(b1), "+&v"(a0), "+&v"(a1) : "s"(~upper), "s"(upper) : "vcc");                 \
+    else                                                                                                                                                           \
+        asm("s_nop 2\n\ts_mov_b64 vcc, %8\n\t" RLT_SELECT(0, 6, 4, CONTROL) RLT_SELECT(1, 7, 5, CONTROL) "s_mov_b64 vcc, %9\n\t" RLT_SELECT(2, 4, 6, CONTROL)      \
+            RLT_SELECT(3, 5, 7, CONTROL) END : "=&v"(x0), "=&v"(x1), "=&v"(y0), "=&v"(y1) : "v"(a0), "v"(a1), "v"(b0), "v"(b1), "s"(~upper), "s"(upper) : "vcc")
+constexpr uint64_t LANES_1 = 0xAAAAAAAAAAAAAAAAull, LANES_2 = 0xCCCCCCCCCCCCCCCCull;      // lanes with that bit
+template <int R, uint64_t upper> __device__ __forceinline__ void exchange(floatx4& a, floatx4& b, floatx4& spare) {
+#pragma unroll
+    for (int i = 0; i < 4; i += 2) {
+        float a0 = a[i], a1 = a[i + 1], b0 = b[i], b1 = b[i + 1], x0 = spare[i], x1 = spare[i + 1], y0 = 0.f, y1 = 0.f;
+        if constexpr (upper == LANES_1) { RLT_EXCHANGE("quad_perm:[1,0,3,2]", ""); }
+        else { RLT_EXCHANGE("quad_perm:[2,3,0,1]", "s_nop 1"); }
+        a[i] = x0; a[i + 1] = x1;
+        if constexpr (R == ROWS) { b[i] = b0; b[i + 1] = b1; spare[i] = a0; spare[i + 1] = a1; } else { b[i] = y0; b[i + 1] = y1; }
+    }
 }
 #undef RLT_EXCHANGE
+#undef RLT_SELECT
 // 16 bytes of load t in lane u of a group of four lanes <-> load u in lane t
-__device__ __forceinline__ void deal_loads(floatx4& b0, floatx4& b1, floatx4& b2, floatx4& b3) {
-    exchange<LANES_1>(b0, b1); exchange<LANES_1>(b2, b3);
-    exchange<LANES_2>(b0, b2); exchange<LANES_2>(b1, b3);
+template <int R>
+__device__ __forceinline__ void deal_loads(floatx4& b0, floatx4& b1, floatx4& b2, floatx4& b3, floatx4& spare) {
+    exchange<R, LANES_1>(b0, b1, spare); exchange<R, LANES_1>(b2, b3, spare);
+    exchange<R, LANES_2>(b0, b2, spare); exchange<R, LANES_2>(b1, b3, spare);
+}
+// The same between groups of four lanes: moves that leave a group its own
+template <int CONTROL, int GROUPS> __device__ __forceinline__ float into_groups(float own, float from) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(own), __float_as_int(from), CONTROL, 0xF, GROUPS, false));
+}
+template <int FROM_LOWER, int FROM_UPPER, int UPPER> __device__ __forceinline__ void exchange_groups(floatx4& a, floatx4& b) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const float x = into_groups<FROM_LOWER, UPPER>(a[i], b[i]), y = into_groups<FROM_UPPER, 0xF & ~UPPER>(b[i], a[i]);
+        a[i] = x; b[i] = y;
+    }
 }
 // value i of four loads in group of four lanes q of sixteen <-> value q in group i
 __device__ __forceinline__ void deal_values(floatx4& b0, floatx4& b1, floatx4& b2, floatx4& b3) {
     floatx4 x0 = {b0[0], b1[0], b2[0], b3[0]}, x1 = {b0[1], b1[1], b2[1], b3[1]}, x2 = {b0[2], b1[2], b2[2], b3[2]}, x3 = {b0[3], b1[3], b2[3], b3[3]};
-    exchange<LANES_4>(x0, x1); exchange<LANES_4>(x2, x3);
-    exchange<LANES_8>(x0, x2); exchange<LANES_8>(x1, x3);
+    exchange_groups<0x114, 0x104, 0xA>(x0, x1); exchange_groups<0x114, 0x104, 0xA>(x2, x3);      // row_shr:4, row_shl:4
+    exchange_groups<0x128, 0x128, 0xC>(x0, x2); exchange_groups<0x128, 0x128, 0xC>(x1, x3);      // row_ror:8
     b0 = floatx4{x0[0], x1[0], x2[0], x3[0]}; b1 = floatx4{x0[1], x1[1], x2[1], x3[1]}; b2 = floatx4{x0[2], x1[2], x2[2], x3[2]}; b3 = floatx4{x0[3], x1[3], x2[3], x3[3]};
 }
 // forward: rows 16 w + c of W2, half h of the reduction; after deal_second() element 4 p + t of lane (c, g) holds k = 64 p + 16 g + 4 t ...
@@ -139,7 +156,11 @@ __device__ __forceinline__ void request_second(const float* W2, int wave, int c,
 #pragma unroll
         for (int t = 0; t < 4; t++) b[4 * p + t] = *reinterpret_cast<const floatx4*>(mine + t * MAX_H + 64 * p);
 }
-__device__ __forceinline__ void deal_second(floatx4 (&b)[8]) { deal_loads(b[0], b[1], b[2], b[3]); deal_loads(b[4], b[5], b[6], b[7]); }
+template <int R>
+__device__ __forceinline__ void deal_second(floatx4 (&b)[8]) {
+    floatx4 spare = {0.f, 0.f, 0.f, 0.f};
+    deal_loads<R>(b[0], b[1], b[2], b[3], spare); deal_loads<R>(b[4], b[5], b[6], b[7], spare);
+}
 // backward: columns 16 w ... of W2. Tiles of sixteen rows: after deal_values() element j of lane (c, g) holds rows 16 j + 4 g ... + 3 of column own_column(w, c). Tiles of four and eight need no
 // dealing: element j of lane l holds row 16 (l / 4) + j, columns 16 w + 4 (l % 4) ... + 3 (column_products), and the sums end in the same column.
 template <int R>
@@ -403,14 +424,14 @@ __device__ __forceinline__ void forward3(const WNet& N, Operands<NT1C>& W, const
         if (NT1C <= FEW) load_first<NT1C, FORM>(next, next_on, wave, c, g, W.w1);
         W.b1 = next.b1[min(n, next.hid - 1)];
     }
-    if (DIRECT) deal_second(W.w2a);      // (while the others finish their tiles of the first layer)
+    if (DIRECT) deal_second<R>(W.w2a);      // (while the others finish their tiles of the first layer)
     rlt_lds_barrier();
     {
         Sums<R> sums;
         clear(sums);
         if (on) chunks<R, DIRECT>(sums, h1, S, c, g, 0, tiles, W.w2a);
         if (PREFETCH) load_second<FORM>(next, next_tiles, next_on, wave, c, g, 0, W.w2a);
-        if (DIRECT) deal_second(W.w2b);
+        if (DIRECT) deal_second<R>(W.w2b);
         if (on) chunks<R, DIRECT>(sums, h1, S, c, g, 8, tiles, W.w2b);
         if (PREFETCH && NT1C <= FEW) load_second<FORM>(next, next_tiles, next_on, wave, c, g, 1, W.w2b);
         if (on) place_hidden<R, ACT_H, KEEP, LIVE>(N, sums, W.b2, h2, n, g, keep, 1, live);
