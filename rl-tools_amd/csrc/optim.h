@@ -28,8 +28,9 @@ enum { RLT_TICKET_TAIL = 32 /* .. +7 */ };
 // asked for), so the ticket needs no fence: a workgroup's reads of the age have returned before its ticket is drawn. The tickets are two levels deep because atomics
 // on one word are served one after the other, about 80 ns each across the XCDs. At 72 k parameters the launch took 23 us with 281 workgroups on one word, 10.4 us
 // with them behind a device-wide fence each (which writes the XCD's L2 back), and 6.1 us (5.6 since a workgroup steps one tensor) with sixteen leaves in lines of their own, no fence and four elements
-// per thread. Drawing the ticket before the elements are stepped, so that its answer travels meanwhile, was no faster (6.0 us; 8.0 instead of 6.9 us with sixteen
-// blocks per element): the workgroup then waits for the age before anything else.
+// per thread. Drawing the ticket before the elements are stepped, so that its answer travels meanwhile, was no faster where one of the stepping wavefronts does it (6.0 us; 8.0 instead of 6.9 us with
+// sixteen blocks per element): the workgroup then waits for the age before anything else. Drawn by a wavefront of its own it takes the launch to 4.5 us, although that wait is still in front of the
+// elements' first loads (adam_body, optim.hip).
 constexpr uint32_t RLT_TICKET_LEAVES = 16, RLT_TICKET_STRIDE = 32;      // words
 constexpr size_t RLT_TICKET_BYTES = (RLT_TICKET_LEAVES + 1) * RLT_TICKET_STRIDE * sizeof(uint32_t);
 // Up to sixteen workgroups draw from the root alone, a single one draws none: with a leaf each they made one trip to memory more

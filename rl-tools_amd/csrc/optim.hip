@@ -54,8 +54,9 @@ __device__ __forceinline__ float sum_of_blocks(const float* __restrict__ p, int 
 }
 
 // the step for one optimiser by workgroups [0, n_blocks) numbered `block`. With a fifth wavefront in the workgroups (TICKETS_APART) that one draws the tickets and stores the incremented age while the others
-// step the elements: behind the stores the two levels of tickets were two more trips to memory at the launch's end (a step of 17-256-256-6, us: 256 rows 29.0 -> 28.1, 1,000 rows 35.5 -> 34.3; the GRU's
-// training step with 64 sequences 96.0 -> 94.9).
+// step the elements: behind the stores the two levels of tickets were two more trips to memory at the launch's end. Such a step never adds blocks of sums up, so the kernel is built without the registers for
+// them (from_blocks): with them three workgroups of five wavefronts fit a compute unit and 944 came in two rounds. Launches in a row, us, four wavefronts / five with those registers / five: 10 elements
+// 4.9 / 5.0 / 4.2, 72,000 in one tensor 5.9 / 5.0 / 4.5, 700,000 7.7 / 8.8 / 6.2, 2,000,000 11.2 / 13.1 / 9.5, 500,000 in six tensors on no 16 bytes 8.3 / 9.9 / 7.0, 50,000,000 292 / 297 / 289.
 constexpr uint32_t STEP_THREADS = 256;
 template <bool TICKETS_APART>
 __device__ __forceinline__ void adam_body(const AdamLaunch& a, uint32_t block, uint32_t n_blocks) {
@@ -76,8 +77,9 @@ __device__ __forceinline__ void adam_body(const AdamLaunch& a, uint32_t block, u
     const uint32_t begin = (block - a.first_block[ti]) * a.span[ti], end = begin + min(a.span[ti], T.count - begin);
     const float* __restrict__ const source = a.source + a.source_offset[ti];
     const float scale = a.source_scale[ti], add = a.source_add[ti];
+    const bool from_blocks = !TICKETS_APART && a.source;
     float sq = 0.0f;
-    if (a.source && a.groups > 16) {
+    if (from_blocks && a.groups > 16) {
         // many blocks: 64 elements per pass of a workgroup, four threads per element each add up a quarter of the blocks (the order of
         // rlt_sum_of_blocks) with all of a quarter's loads of up to 32 blocks in flight at once
         __shared__ float quarter[4][64];
@@ -126,7 +128,7 @@ __device__ __forceinline__ void adam_body(const AdamLaunch& a, uint32_t block, u
         f4 target = {0.f, 0.f, 0.f, 0.f};
         if (T.polyak_target) target = *reinterpret_cast<const f4*>(T.polyak_target + j);
         f4 g;
-        if (a.source) {
+        if (from_blocks) {
             const float* __restrict__ p = source + j;
             const int per = (a.groups + 3) / 4;
             f4 blk[16];
@@ -156,7 +158,7 @@ __device__ __forceinline__ void adam_body(const AdamLaunch& a, uint32_t block, u
             m[c] = mc; v[c] = vc; param[c] = pc;
             if (T.polyak_target) target[c] = rlt_polyak_value(a.polyak, target[c], pc);
         }
-        if (a.source) *reinterpret_cast<f4*>(T.gradient + j) = g;
+        if (from_blocks) *reinterpret_cast<f4*>(T.gradient + j) = g;
         *reinterpret_cast<f4*>(T.first_moment + j) = m; *reinterpret_cast<f4*>(T.second_moment + j) = v; *reinterpret_cast<f4*>(T.parameters + j) = param;
         if (T.polyak_target) *reinterpret_cast<f4*>(T.polyak_target + j) = target;
     }
@@ -165,7 +167,7 @@ __device__ __forceinline__ void adam_body(const AdamLaunch& a, uint32_t block, u
         float m = T.first_moment[j], v = T.second_moment[j], param = T.parameters[j];
         const float target = T.polyak_target ? T.polyak_target[j] : 0.f;
         float g;
-        if (a.source) {
+        if (from_blocks) {
             g = rlt_scaled_sum(sum_of_blocks(source + j, a.groups, a.block_stride), scale, add);
             T.gradient[j] = g;
         } else g = T.gradient[j];

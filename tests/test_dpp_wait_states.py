@@ -12,6 +12,7 @@ import subprocess
 import sys
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+TOOLS = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin")
 
 
 def _registers(operand):
@@ -112,10 +113,10 @@ def lane_control_violations(lines):
     return found, controlled
 
 
-def disassembly(library, scratch):
-    """The lines of a built library's device code: each translation unit's offload bundle (magic, number of entries, then offset, size and name of each) holds one code object for gfx950."""
-    tools, bundles = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin"), scratch / "bundles"
-    subprocess.run([os.path.join(tools, "llvm-objcopy"), "--dump-section", f".hip_fatbin={bundles}", library, "/dev/null"], check=True)
+def code_objects(library, scratch):
+    """The gfx950 code objects of a built library, one after the other in a file: each translation unit's offload bundle is its magic, the number of entries, then offset, size and name of each."""
+    bundles = scratch / "bundles"
+    subprocess.run([os.path.join(TOOLS, "llvm-objcopy"), "--dump-section", f".hip_fatbin={bundles}", library, "/dev/null"], check=True)
     data = bundles.read_bytes()
     for bundle in re.finditer(b"__CLANG_OFFLOAD_BUNDLE__", data):
         at = bundle.end() + 8
@@ -124,9 +125,21 @@ def disassembly(library, scratch):
             target, at = data[at + 24:at + 24 + length], at + 24 + length
             if b"gfx950" in target:
                 (scratch / "code").write_bytes(data[bundle.start() + offset:bundle.start() + offset + size])
-                with subprocess.Popen([os.path.join(tools, "llvm-objdump"), "-d", "--no-show-raw-insn", scratch / "code"], stdout=subprocess.PIPE, text=True) as dump:
-                    yield from dump.stdout
-                assert dump.returncode == 0
+                yield scratch / "code"
+
+
+def disassembly(library, scratch):
+    for code in code_objects(library, scratch):
+        with subprocess.Popen([os.path.join(TOOLS, "llvm-objdump"), "-d", "--no-show-raw-insn", code], stdout=subprocess.PIPE, text=True) as dump:
+            yield from dump.stdout
+        assert dump.returncode == 0
+
+
+def built_library():
+    library = os.path.join(ROOT, "rl-tools_amd", "librlt_rocm.so")
+    if not os.path.exists(library):
+        subprocess.run([sys.executable, os.path.join(ROOT, "rl-tools_amd", "build.py")], check=True, capture_output=True)
+    return library
 
 
 def test_the_check_sees_what_the_rules_forbid():
@@ -142,8 +155,5 @@ def test_the_check_sees_what_the_rules_forbid():
 
 
 def test_lane_controls_of_the_built_library_keep_their_distances(tmp_path):
-    library = os.path.join(ROOT, "rl-tools_amd", "librlt_rocm.so")
-    if not os.path.exists(library):
-        subprocess.run([sys.executable, os.path.join(ROOT, "rl-tools_amd", "build.py")], check=True, capture_output=True)
-    found, controlled = lane_control_violations(disassembly(library, tmp_path))
+    found, controlled = lane_control_violations(disassembly(built_library(), tmp_path))
     assert controlled > 10000 and not found, (len(found), found[:5])
