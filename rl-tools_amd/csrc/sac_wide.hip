@@ -1471,7 +1471,10 @@ static int mlp_wide_launch(rlt_rocm_device* device, const rlt_dense_layer* L, in
         partial = (float*)scratch + trained_floats(hid, batch) + copy_floats;
         set_rows(net, a.kept, in_place ? a.copy_x : x, in_place ? IN : ldx);
     }
-    const bool direct = !blocks && hid == MAX_H && aligned16(a.net.W2) && DIRECT_LDS_FLOATS * sizeof(float) <= (size_t)device->lds_bytes;
+    // (forward + backward of 33 to 64 inputs on tiles of eight rows, whose four chunks of the first layer lie in registers beside the second's values, from the copies: 32.9 / 34.4 us at 1,500 rows of 33
+    // inputs, copies / direct, 36.3 / 38.1 at 2,048 of 64)
+    const bool crowded = pass == MLP_FORWARD_BACKWARD && rows == 8 && IN > 32 && IN <= 64;
+    const bool direct = !blocks && !crowded && hid == MAX_H && aligned16(a.net.W2) && DIRECT_LDS_FLOATS * sizeof(float) <= (size_t)device->lds_bytes;
     if (!direct) {
         if ((rc = rlt_mlp_wide_reserve(device))) return rc;
         Copies copies((float*)device->copy_scratch);

@@ -247,7 +247,7 @@ def test_an_infinite_weight_that_the_activation_saturates_leaves_finite_gradient
     assert rel_err(got[0], ref[0]) <= TOL and rel_err(got[1], ref[1]) <= TOL
 
 
-@pytest.mark.parametrize("B, I", [(1, 1), (3, 16), (5, 33), (1024, 128), (1025, 64), (2047, 17), (2049, 36), (4095, 3)])
+@pytest.mark.parametrize("B, I", [(1, 1), (3, 16), (5, 33), (1024, 128), (1025, 64), (2047, 17), (2048, 33), (2049, 36), (4095, 3)])
 def test_second_layers_of_256_units_wherever_they_lie(oracle, rocm, B, I):
     """256 units: a second layer on 16 bytes is read as it lies, one that is not from copies. Forward + backward in one call and as calls of their own, tiles of four, eight and sixteen rows, the first
     layer in one to eight chunks of sixteen columns."""
