@@ -1475,8 +1475,9 @@ static int mlp_wide_launch(rlt_rocm_device* device, const rlt_dense_layer* L, in
     // inputs, copies / direct, 36.3 / 38.1 at 2,048 of 64)
     const bool crowded = pass == MLP_FORWARD_BACKWARD && rows == 8 && IN > 32 && IN <= 64;
     const bool direct = !blocks && !crowded && hid == MAX_H && aligned16(a.net.W2) && DIRECT_LDS_FLOATS * sizeof(float) <= (size_t)device->lds_bytes;
+    // (a pass that needs no copies asks for their buffer too, unless the stream records a graph: the program may record one that does)
+    if ((!direct || !device->capturing) && (rc = rlt_mlp_wide_reserve(device))) return rc;
     if (!direct) {
-        if ((rc = rlt_mlp_wide_reserve(device))) return rc;
         Copies copies((float*)device->copy_scratch);
         if (!backward_only) copies.forward(a.net);
         if (!forward_only) copies.backward(a.net);

@@ -3,6 +3,8 @@ sixteen wavefronts per tile, the weight gradients over the whole batch by a seco
 call (RLT_MLP_WIDE=0), through the C ABI.
 
 fp32 tolerance: 1e-5 relative to the largest magnitude of the tensor compared (the contraction order differs from the checker's)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -275,3 +277,46 @@ def test_second_layers_of_256_units_wherever_they_lie(oracle, rocm, B, I):
             assert rel_err(y, ref[0]) <= TOL, (shift, separate)
             for off, nw, nb in ref[2]:
                 assert rel_err(grads[off:off + nw], ref[1][off:off + nw]) <= TOL and rel_err(grads[off + nw:off + nw + nb], ref[1][off + nw:off + nw + nb]) <= TOL, (shift, separate, off)
+
+
+@pytest.mark.parametrize("dims, shift", [([17, 128, 128, 6], 0), ([17, 256, 256, 6], 1)])
+def test_passes_that_need_copies_of_the_weights_are_recorded_after_one_that_needs_none(dims, shift):
+    """A handle whose only pass so far, of 256 units on 16 bytes, read its layers as they lie: one of another width, or whose second layer lies elsewhere, is recorded all the same, and every replay
+    leaves what the call by itself leaves, bit for bit."""
+    be, graph, B = helpers.RocmBackend(), C.c_void_p(), 64
+    rng = np.random.default_rng(dims[1])
+    try:
+        def network(dims, shift):
+            params = helpers.random_params(rng, dims)
+            net = Mlp(be, dims, params, B, "tanh", "identity")
+            off, nw, _ = net.offsets[1]
+            net.second = be.array(np.concatenate([np.zeros(shift, np.float32), params[off:off + nw]]))
+            net.layers[1].weights = net.second.offset(shift)
+            return net
+        x, y, dy = be.array(rng.standard_normal((B, 17)).astype(np.float32)), be.zeros((B, 6)), be.array(rng.standard_normal((B, 6)).astype(np.float32))
+
+        def step(net):
+            ws, wsn = net.workspace()
+            be.call("mlp_zero_gradient", net.layers, net.n)
+            return be.device.lib.rlt_rocm_mlp_forward_backward(be.device.handle, net.layers, net.n, x.ptr, 17, y.ptr, 6, dy.ptr, 6, None, 0, 0.0, B, ws, wsn)
+        assert step(network([17, 256, 256, 6], 0)) == 0
+        net = network(dims, shift)
+        be.sync()
+        be.call("graph_begin_capture")
+        try:
+            rc = step(net)
+        finally:
+            be.call("graph_end_capture", C.byref(graph))
+        assert rc == 0
+        replays = []
+        for _ in range(3):
+            be.call("graph_launch", graph)
+            be.sync()
+            replays.append((y.numpy(), net.grads.numpy()))
+        assert step(net) == 0
+        be.sync()
+        for got in replays:
+            assert got[1].any() and np.array_equal(got[0], y.numpy()) and np.array_equal(got[1], net.grads.numpy())
+        be.call("graph_destroy", graph)
+    finally:
+        be.close()
