@@ -1274,10 +1274,6 @@ bool inputs_beside(const rlt_rocm_device* device, const rlt_gru_layer* L, const 
     const double launch = by_rows ? 3750.0 : I <= 32 ? 5800.0 : I % 4 == 0 ? 2400.0 : I % 2 == 0 ? 2600.0 : 3200.0;
     return (by_rows ? 27.2 : 23.8) * 4 * rlt_div_up(S, 4) * even_sixteens(I) + by_row <= launch + ((by_rows ? 0.143 : 0.185) + 0.0017 * I) * rows;
 }
-bool weights_beside(const rlt_rocm_device* device, const rlt_gru_layer* L, int S, int B, size_t room) {      // room: bytes of the caller's workspace that nothing else is kept in
-    if (!one_group_per_unit(device, L, B) || L->input_dim > GW_INPUTS || rlt_div_up(B, GM_ROWS) * gru_gradient_block(L->input_dim) * sizeof(float) > room) return false;
-    return S * (54.0 + 46.0 * even_sixteens(L->input_dim)) + (rows_backward(device, 64, S, B) ? 110.0 * S - (B <= compute_units(device) ? 1500.0 : 2000.0) : 0.0) <= 3400.0 + (0.35 + 0.0037 * L->input_dim) * S * B;
-}
 // The weight gradients of gru_gradients_kernel: pairs of column tiles, shares of the rows (workgroups for the whole chip, but at least eight steps of four rows to a wavefront; once, twice ... so many that no sum is longer than
 // 256 steps, for its error's sake), blocks of sums
 struct GradientShape { int columns, shares, blocks; };
@@ -1287,6 +1283,7 @@ GradientShape gradient_shape(const rlt_rocm_device* device, const rlt_gru_layer*
     const int shares = most < chip ? most : chip * rlt_div_up(rows, 4 * 256 * parts * chip);
     return {columns, shares, shares * parts};
 }
+size_t gradient_shares_bytes(const rlt_rocm_device* device, const rlt_gru_layer* L, int rows) { return gradient_shape(device, L, rows).blocks * gradient_block(L->hidden_dim, L->input_dim) * sizeof(float); }
 // Where they are (widths 16, 32, 64): not where width 64 meets 65,536 rows and more of 66 to 160 inputs, an even number, which wgrad_wide_kernel (gemm.hip) reads once. us of the backward pass
 // with contractions and sums per gradient / this, width 64: 146 inputs 16 steps 4,000 rows 141 / 127, 64 steps 2,048 rows 230 / 249, 16 steps 8,192 rows 247 / 303; 33 inputs 64 steps 2,048 rows 200 / 179,
 // 170 inputs 64 steps 1,024 rows 167 / 143, 300 inputs 64 rows 65.9 / 52.5, 1,024 rows 212 / 189, 1,000 inputs 64 rows 78.7 / 66.5, 1,024 rows 503 / 436; width 32, 500 inputs 64 rows 84.4 / 54.0, 1,000 inputs 1,024 rows
@@ -1295,6 +1292,13 @@ GradientShape gradient_shape(const rlt_rocm_device* device, const rlt_gru_layer*
 bool gradients_in_one(const rlt_gru_layer* L, int S, int B) {
     const int H = L->hidden_dim, I = L->input_dim;
     return (H == 16 || H == 32 || H == 64) && I <= 1024 && !(H == 64 && (size_t)S * B >= 65536 && I > 64 && I <= 160 && I % 2 == 0);
+}
+// (A stream that records a graph takes no launches for whose shares the handle's scratch memory has no room: a workgroup per row is then no reason for them.)
+bool weights_beside(const rlt_rocm_device* device, const rlt_gru_layer* L, int S, int B, size_t room) {      // room: bytes of the caller's workspace that nothing else is kept in
+    if (!one_group_per_unit(device, L, B) || L->input_dim > GW_INPUTS || rlt_div_up(B, GM_ROWS) * gru_gradient_block(L->input_dim) * sizeof(float) > room) return false;
+    const bool by_launches = !device->capturing || (gradients_in_one(L, S, B) && rlt_scratch_reaches(device, gradient_shares_bytes(device, L, S * B)));
+    const double by_row = !by_launches || !rows_backward(device, 64, S, B) ? 0.0 : 110.0 * S - (B <= compute_units(device) ? 1500.0 : 2000.0);      // what the recurrence of its own has from a workgroup per row
+    return S * (54.0 + 46.0 * even_sixteens(L->input_dim)) + by_row <= 3400.0 + (0.35 + 0.0037 * L->input_dim) * S * B;
 }
 int finish_gradients(rlt_rocm_device* device, const rlt_gru_layer* L, const float* blocks, int n, size_t stride, const float* hidden, int n_hidden, size_t hidden_stride) {
     const int H = L->hidden_dim, I = L->input_dim;
@@ -1415,7 +1419,7 @@ int rlt_rocm_gru_backward(rlt_rocm_device* device, const rlt_gru_layer* L, const
     int rc = rlt_launch_status(device);
     if (rc) return rc;
     const GradientShape shape = gradient_shape(device, L, rows);
-    const size_t shares_bytes = shape.blocks * gradient_block(H, I) * sizeof(float);
+    const size_t shares_bytes = gradient_shares_bytes(device, L, rows);
     if (want_weight_gradients && gradients_in_one(L, S, B) && rlt_scratch_reaches(device, shares_bytes)) {
         float* shares = nullptr;
         if ((rc = rlt_scratch(device, shares_bytes, (void**)&shares))) return rc;

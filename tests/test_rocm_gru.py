@@ -257,3 +257,40 @@ def test_a_backward_pass_is_recorded_with_the_scratch_memory_of_a_shorter_one(ro
         be.call("graph_destroy", graph)
     finally:
         be.close()
+
+
+@pytest.mark.parametrize("case", [(48, 256, 3), (64, 256, 16), (20, 512, 16), (33, 257, 32)])
+def test_a_backward_pass_is_recorded_without_scratch_memory(rocm, case):
+    """A handle on which nothing has run but forward passes: few enough rows for a workgroup each, whose weight gradients, as launches of their own, want scratch memory that a recording stream cannot ask for, and
+    which the pass with the gradients beside the recurrence does without (steps * (54 + 92) <= 3,400 + (0.35 + 0.0037 inputs) * steps * sequences for these inputs: beyond that line, as with 128
+    sequences of 64 steps of 3 inputs, a recording has always needed it). Every replay leaves the gradients of the call on a handle that may allocate, to the file's tolerance."""
+    print("case", case, flush=True)
+    (S, B, I), H, rng = case, 64, np.random.default_rng(4)
+    params, x, dy, reset = helpers.gru_random_case(rng, S, B, I, H, True)
+    want = helpers.GruOnBackend(rocm, S, B, I, H, params)
+    want.forward(x, reset)
+    want.backward(dy)
+    rocm.sync()
+    want, be, graph = want.results(), helpers.RocmBackend(), C.c_void_p()
+    try:
+        g = helpers.GruOnBackend(be, S, B, I, H, params)
+        g.forward(x, reset)
+        g.dy, g.dx = be.array(dy), be.zeros((S, B, I))
+        be.sync()
+        be.call("graph_begin_capture")
+        try:
+            rc = be.device.lib.rlt_rocm_gru_backward(be.device.handle, C.byref(g.c), g.x.ptr, g.dy.ptr, g.dx.ptr, g.reset.ptr, S, B, 1, g.ws, g.wsn)
+        finally:
+            be.call("graph_end_capture", C.byref(graph))
+        assert rc == 0
+        for _ in range(3):
+            g.dy.upload(dy)
+            be.call("fill_f32", g.grads.ptr, 1, g.grads.shape[0], g.grads.shape[0], 0.0)
+            be.call("graph_launch", graph)
+            be.sync()
+            got = g.results()
+            for k in KEYS:
+                assert rel_err(got[k], want[k]) <= TOL, k
+        be.call("graph_destroy", graph)
+    finally:
+        be.close()
