@@ -718,8 +718,10 @@ int rlt_gemm_rows_forward(rlt_rocm_device* device, const float* x, int ldx, cons
         ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(W)) & 7u) != 0) return RLT_E_UNSUPPORTED;
     const RowsForward a = {x, ldx, W, bias, y, ldy, batch, out_dim, in_dim};
     const int blocks = rlt_div_up(batch, RF_ROWS), grid = blocks < device->compute_units ? blocks : device->compute_units;
+    // (a workgroup with all of the columns has read its rows before it writes any: outputs may lie where the inputs do)
+    const bool apart = (uintptr_t)y >= (uintptr_t)(x + (size_t)(batch - 1) * ldx + in_dim) || (uintptr_t)x >= (uintptr_t)(y + (size_t)(batch - 1) * ldy + out_dim);
     auto launch = [&](auto all, auto part) {
-        if (2 * blocks <= device->compute_units) hipLaunchKernelGGL(part, dim3(blocks, rlt_div_up(out_dim, 64)), dim3(RF_THREADS), 0, device->stream, a);
+        if (apart && 2 * blocks <= device->compute_units) hipLaunchKernelGGL(part, dim3(blocks, rlt_div_up(out_dim, 64)), dim3(RF_THREADS), 0, device->stream, a);
         else hipLaunchKernelGGL(all, dim3(grid), dim3(RF_THREADS), 0, device->stream, a);
     };
     if (in_dim <= 64) launch(rows_forward_kernel<4, 3>, rows_forward_kernel<4, 1>);

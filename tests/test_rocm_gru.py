@@ -222,6 +222,25 @@ def test_gru_states_may_replace_the_inputs(rocm, case):
         assert want.any() and rel_err(got, want) <= TOL
 
 
+@pytest.mark.parametrize("case", [(32, 64, 44), (64, 64, 52), (33, 65, 48)])
+def test_gru_gates_may_replace_as_many_inputs(rocm, case):
+    """A forward pass whose inputs, 3 H to a row, lie where it leaves the gates: the results of the call with memory of its own, bit for bit (2,048 to 4,096 rows, the layer of whose input gates is shared out by
+    columns where inputs and gates are apart)."""
+    S, B, H = case
+    params, x, _, reset = helpers.gru_random_case(np.random.default_rng(S + H), S, B, 3 * H, H, True)
+    results = []
+    for apart in (True, False):
+        g = helpers.GruOnBackend(rocm, S, B, 3 * H, H, params)
+        flags, xd = rocm.array(reset), rocm.array(x)
+        if not apart:
+            g.post.upload(x)
+        rocm.call("gru_forward", C.byref(g.c), xd.ptr if apart else g.post.ptr, flags.ptr, S, B, g.ws, g.wsn)
+        rocm.sync()
+        results.append([g.out.numpy(), g.post.numpy(), g.npp.numpy()])
+    for want, got in zip(*results):
+        assert want.any() and np.array_equal(got, want)
+
+
 def test_a_backward_pass_is_recorded_with_the_scratch_memory_of_a_shorter_one(rocm):
     """A handle whose scratch memory a call of a few steps has sized: a longer backward pass is recorded all the same (its shares of the rows want 1.3 MB, contractions less), and every replay
     leaves the gradients of the call on a handle that may allocate, to the file's tolerance."""
