@@ -6,8 +6,9 @@
 //   * W_i x + b_i for ALL steps is one contraction over sequence*batch rows (gemm.hip), written straight into post_activation (at hidden width 64 and up to a thousand rows mostly
 //     formed beside the recurrence, inputs_beside);
 //   * the recurrence runs in ONE launch: batch rows are independent, so no grid-wide synchronisation is needed. At hidden width 64 a
-//     workgroup carries four rows through the sequence on the matrix cores at 16 and 32 a wavefront 64 / width rows, both with W_h in registers, and up to a few rows per compute unit a workgroup one row on the vector units; at other widths a workgroup owns a few
-//     rows and keeps W_h and its rows' hidden state in LDS;
+//     workgroup carries four rows through the sequence on the matrix cores, at 16 and 32 a wavefront 64 / width rows on the vector units, both with W_h in registers; where there are few rows for the
+//     compute units (two to five each, backward from a number of steps on: rows_forward(), rows_backward()) a workgroup carries one row on the vector units at all three widths; at other
+//     widths a workgroup owns a few rows and keeps W_h and its rows' hidden state in LDS;
 //   * backward does the same in reverse and stores, per step, the gradient at the gate pre-activations (one copy as the input path sees
 //     it, one as the hidden path sees it, which differs in the n gate by the factor r) and the previous hidden state; the weight
 //     gradients and d_input are then three contractions over sequence*batch rows (the weight gradients, too, mostly beside the recurrence where that is one workgroup per compute unit,

@@ -20,7 +20,8 @@
 //   P6  dW2 += d_pre2^T h1 ; d_h1 = d_pre2 W2       K = 64 rows / K = 256
 //   P7  d_pre1 = d_h1 * act'(h1)  in place of h1
 //   P8  dW1 += d_pre1^T x
-// The weight-gradient accumulators (128 + 16 + 8 registers per lane) live in registers for the whole launch; at the end every
+// The weight-gradient accumulators (128 + 16 + 8 registers per lane) live in registers for the whole launch (64 bytes a lane of other values go to scratch
+// memory, 32 in the pass from kept activations); at the end every
 // workgroup writes its partial gradients and a second kernel sums them in a fixed order into the layers' gradients (beta = 1).
 // act' is taken from the layer output, which relu / tanh / fast_tanh / sigmoid / identity allow.
 //

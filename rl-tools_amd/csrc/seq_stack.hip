@@ -152,8 +152,8 @@ __device__ __forceinline__ float product_sum3(const Weights3<H>& R, float x, flo
 
 // A stage: `before` ticks until its first step is there, one per step, `after` ticks for the stages behind it. The steps are unrolled U at a time with their number in the
 // group as a constant (slots and queues are indexed by it). Whole groups are straight-line code: with an exit before every step, or a request under a condition, the compiler waits where the paths
-// meet, once in a group, for everything that is under way (100 sequences of 100 steps, with four steps ahead instead of six, whose queue fits 128 registers,
-// 354 -> 341 us a set, 1,000 sequences 1,584 -> 1,480). What was requested before the first step is waited for in front of it,
+// meet, once in a group, for everything that is under way (100 sequences of 100 steps, with four steps ahead instead of six, whose queue fits 128 registers but for
+// 16 bytes a lane in scratch memory, 354 -> 341 us a set, 1,000 sequences 1,584 -> 1,480). What was requested before the first step is waited for in front of it,
 // so that a step waits for its own values and not for the last ones.
 template <class F, int... D>
 __device__ __forceinline__ void stage_group(int i, F& step, std::integer_sequence<int, D...>) {

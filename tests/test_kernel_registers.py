@@ -15,5 +15,10 @@ def test_all_workgroups_of_an_optimisers_launch_are_resident(tmp_path, kernel):
     used = []
     for code in code_objects(built_library(), tmp_path):
         notes = subprocess.run([os.path.join(TOOLS, "llvm-readelf"), "--notes", code], check=True, capture_output=True, text=True).stdout
-        used += [int(n) for name, n in re.findall(r"\.name:\s+(\S+)\n(?:(?!\.name:).*\n)*?\s+\.vgpr_count:\s+(\d+)", notes) if kernel in name]
+        name = ""
+        for field in re.findall(r"\.(name|vgpr_count):\s+(\S+)", notes):      # in this order for each kernel
+            if field[0] == "name":
+                name = field[1]
+            elif kernel in name:
+                used.append(int(field[1]))
     assert len(used) == 1 and -(-used[0] // 8) * 8 * 5 <= 512, used
